@@ -48,6 +48,37 @@ AttnWorkspace carve_attn(void* base, int64_t B, int64_t H, int64_t KVH, int64_t 
     return w;
 }
 
+// scratch of the dense operator on the matrix cores: as above, the scores in their final form instead of sums to be
+// reduced, and the key order
+struct DenseWorkspace {
+    void *qr, *kr, *vc;
+    unsigned long long* tile_vis;
+    float *lse, *lse2, *w_ema, *w_new, *part_o, *part_l2;
+    int *key_order, *n_visible;
+    int64_t bytes;
+};
+
+DenseWorkspace carve_dense(void* base, int64_t B, int64_t H, int64_t n_ctx, int64_t n_kv, int64_t D) {
+    const int64_t n_pad = mfma_n_pad(n_kv), rows = B * H * n_ctx;
+    Carver c(base);
+    DenseWorkspace w;
+    w.qr = c.take((rows + kColSlack) * D * 2);
+    w.kr = c.take(B * H * n_pad * D * 2);
+    w.vc = c.take(B * H * n_pad * D * 2);
+    w.tile_vis = (unsigned long long*)c.take(n_pad / 64 * 8);
+    w.lse = (float*)c.take(rows * 4);
+    w.lse2 = (float*)c.take((rows + kColSlack) * 4);
+    w.w_ema = (float*)c.take((n_ctx + kColSlack) * 4);
+    w.w_new = (float*)c.take(n_ctx * 4);
+    w.key_order = (int*)c.take(n_kv * 4);
+    w.n_visible = (int*)c.take(4);
+    const int splits = mfma_fwd_splits_for_workspace(B, H, H, n_ctx, n_kv);
+    w.part_o = splits > 1 ? (float*)c.take(splits * rows * D * 4) : nullptr;
+    w.part_l2 = splits > 1 ? (float*)c.take(splits * rows * 4) : nullptr;
+    w.bytes = c.off;
+    return w;
+}
+
 void contiguous_strides(int64_t* st, int64_t d1, int64_t d2, int64_t d3) {
     st[0] = d1 * d2 * d3;
     st[1] = d2 * d3;
@@ -96,7 +127,7 @@ extern "C" int ckv_attn(const ckv_attn_args* args, void* stream_) {
         rc = launch_weights(w.w_ema, w.w_new, a.Q, a.beta, a.dtype, stream);
         if (rc) return rc;
     }
-    const bool use_mfma = mfma_supported(a.dtype, a.D, a.H, a.KVH, a.Q) && a.Q > 1 && mfma_fits(N);
+    const bool use_mfma = mfma_supported(a.dtype, a.D, a.H, a.KVH, a.Q) && a.Q > 1 && mfma_fits(N, a.D);
     if (use_mfma) {
         MfmaProblem mp;
         mp.seg[0] = MfmaSegment{a.sink_k, a.sink_v, {a.sink_stride[0], a.sink_stride[1], a.sink_stride[2], a.sink_stride[3]},
@@ -123,7 +154,7 @@ extern "C" int ckv_attn(const ckv_attn_args* args, void* stream_) {
         mp.w_ema = w.w_ema; mp.w_new = w.w_new;
         mp.beta = a.beta;
         mp.new_mode = 1;
-        mp.B = a.B; mp.H = a.H; mp.KVH = a.KVH; mp.Q = a.Q; mp.n = N; mp.n_pad = mfma_n_pad(N);
+        mp.B = a.B; mp.H = a.H; mp.KVH = a.KVH; mp.Q = a.Q; mp.D = a.D; mp.n = N; mp.n_pad = mfma_n_pad(N);
         mp.scale = a.scale;
         mp.key_scale = sqrtf(a.scale);
         mp.dtype = a.dtype;
@@ -179,9 +210,9 @@ extern "C" int ckv_attn(const ckv_attn_args* args, void* stream_) {
 }
 
 namespace ckv {
-// 16-bit, head_dim 128, more than one query row: the dense operator runs on the MFMA kernels too
+// 16-bit, head_dim 64 or 128, more than one query row: the dense operator runs on the MFMA kernels too
 static bool dense_uses_mfma(int dtype, int64_t D, int64_t H, int64_t n_ctx, int64_t n_kv) {
-    return n_ctx > 1 && mfma_supported(dtype, D, H, H, n_ctx) && mfma_fits(n_kv);
+    return n_ctx > 1 && mfma_supported(dtype, D, H, H, n_ctx) && mfma_fits(n_kv, D);
 }
 }  // namespace ckv
 
@@ -190,7 +221,7 @@ extern "C" int64_t ckv_dense_workspace_bytes(int64_t B, int64_t H, int64_t n_ctx
     if (B <= 0 || H <= 0 || n_ctx <= 0 || n_kv < n_ctx) return 0;
     using ckv::align_up;
     if (ckv::dense_uses_mfma(dtype, D, H, n_ctx, n_kv))  // staged Q / K / V^T and the column pass's scratch
-        return ckv::carve_attn(nullptr, B, H, H, n_ctx, D, 0, n_kv - n_ctx, dtype).bytes;
+        return ckv::carve_dense(nullptr, B, H, n_ctx, n_kv, D).bytes;
     return align_up(B * H * n_ctx * 4, 256) + align_up(B * H * n_kv * 4, 256) + 2 * align_up((n_ctx + ckv::kColSlack) * 4, 256);
 }
 
@@ -207,23 +238,21 @@ extern "C" int ckv_attn_dense(const ckv_dense_args* args, void* stream_) {
     const int64_t need = ckv_dense_workspace_bytes(a.B, a.H, a.n_ctx, a.n_kv, a.D, a.dtype);
     if (!a.workspace || a.workspace_bytes < need) return CKV_ERR_WORKSPACE;
     if (dense_uses_mfma(a.dtype, a.D, a.H, a.n_ctx, a.n_kv)) {
-        // keys and queries arrive rotated (no position ids); every head is its own kv head
+        // Keys and queries arrive rotated (no position ids); every head is its own kv head.  The mask is the same for
+        // every head, so its keys are sorted once, the visible ones in front, and no kernel behind the staging ever
+        // touches a masked one: half the keys masked at random is half the work.
         const int64_t n_cache = a.n_kv - a.n_ctx;
-        AttnWorkspace w = carve_attn(a.workspace, a.B, a.H, a.H, a.n_ctx, a.D, 0, n_cache, a.dtype);
-        int rc;
-        if (a.scores) {
-            rc = launch_weights(w.w_ema, w.w_new, a.n_ctx, a.beta, a.dtype, stream);
-            if (rc) return rc;
-        }
-        const int64_t es = a.dtype == CKV_F32 ? 4 : 2;
+        DenseWorkspace w = carve_dense(a.workspace, a.B, a.H, a.n_ctx, a.n_kv, a.D);
+        int rc = launch_dense_prologue(a.mask, n_cache, a.n_ctx, w.key_order, w.n_visible, a.scores ? w.w_ema : nullptr, w.w_new,
+                                       a.beta, a.dtype, stream);
+        if (rc) return rc;
         MfmaProblem mp;
         const MfmaSegment none{nullptr, nullptr, {0, 0, 0, 0}, nullptr, {0, 0}, 0, nullptr, 0};
         mp.seg[0] = MfmaSegment{a.k, a.v, {a.kv_stride[0], a.kv_stride[1], a.kv_stride[2], a.kv_stride[3]},
-                                nullptr, {0, 0}, 0, n_cache > 0 ? a.mask : nullptr, n_cache};
-        mp.seg[1] = none;
-        mp.seg[2] = MfmaSegment{(const char*)a.k + n_cache * a.kv_stride[2] * es, (const char*)a.v + n_cache * a.kv_stride[2] * es,
-                                {a.kv_stride[0], a.kv_stride[1], a.kv_stride[2], a.kv_stride[3]},
-                                nullptr, {0, 0}, 0, nullptr, a.n_ctx};
+                                nullptr, {0, 0}, 0, nullptr, a.n_kv};
+        mp.seg[1] = mp.seg[2] = none;
+        mp.key_order = w.key_order;
+        mp.n_visible = w.n_visible;
         mp.q = a.q;
         for (int i = 0; i < 4; i++) { mp.q_stride[i] = a.q_stride[i]; mp.out_stride[i] = a.out_stride[i]; }
         mp.q_pos = nullptr;
@@ -232,27 +261,20 @@ extern "C" int ckv_attn_dense(const ckv_dense_args* args, void* stream_) {
         mp.shared_pos = 1;
         mp.qr = w.qr; mp.kr = w.kr; mp.vt = w.vc; mp.tile_vis = w.tile_vis;
         mp.out = a.out;
-        mp.lse = w.lse;
+        mp.lse = a.lse ? a.lse : w.lse;
         mp.lse2 = w.lse2;
-        mp.colsum = a.scores ? w.colsum : nullptr;
+        mp.colsum = nullptr;
+        mp.scores = a.scores;
+        for (int i = 0; i < 3; i++) mp.scores_stride[i] = a.scores_stride[i];
         mp.part_o = w.part_o; mp.part_l2 = w.part_l2;
         mp.w_ema = w.w_ema; mp.w_new = w.w_new;
         mp.beta = a.beta;
         mp.new_mode = 0;  // every key is weighted by the query row alone (flash_attention.py:73-77)
-        mp.B = a.B; mp.H = a.H; mp.KVH = a.H; mp.Q = a.n_ctx; mp.n = a.n_kv; mp.n_pad = mfma_n_pad(a.n_kv);
+        mp.B = a.B; mp.H = a.H; mp.KVH = a.H; mp.Q = a.n_ctx; mp.D = a.D; mp.n = a.n_kv; mp.n_pad = mfma_n_pad(a.n_kv);
         mp.scale = a.scale;
         mp.key_scale = 1.f;
         mp.dtype = a.dtype;
-        rc = launch_mfma(mp, stream);
-        if (rc) return rc;
-        if (a.scores) {
-            rc = launch_cast_scores(w.colsum, a.scores, a.scores_stride, a.B, a.H, a.n_kv, a.dtype, stream);
-            if (rc) return rc;
-        }
-        if (a.lse) {
-            CKV_HIP_TRY(hipMemcpyAsync(a.lse, w.lse, a.B * a.H * a.n_ctx * sizeof(float), hipMemcpyDeviceToDevice, stream));
-        }
-        return CKV_OK;
+        return launch_mfma(mp, stream);
     }
     Carver c(a.workspace);
     float* lse = (float*)c.take(a.B * a.H * a.n_ctx * 4);

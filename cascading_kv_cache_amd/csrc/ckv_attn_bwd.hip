@@ -2,7 +2,7 @@
 // dq, dk, dv of  out = softmax(scale * q k^T + masks) v  with the cache mask on the first n_kv - n_ctx keys
 // and the causal mask on the last n_ctx.  Only training reaches it (the inference path never differentiates).
 // The kernels in this file are plain fp32-math kernels for every dtype and head size up to 192, tiled through
-// LDS; 16-bit tensors with head_dim 128 go to the matrix-core kernels of ckv_attn_bwd_mfma.hip after the delta
+// LDS; 16-bit tensors with head_dim 64 or 128 go to the matrix-core kernels of ckv_attn_bwd_mfma.hip after the delta
 // kernel.  The probabilities are recomputed from the row normalisers the forward pass returns.
 //
 //   delta   delta[m] = sum_d out[m, d] * dout[m, d]                      (flash_attention.py:279-294)
@@ -23,14 +23,21 @@ constexpr int kThreads = 256;
 struct BwdParams {
     ckv_dense_bwd_args a;
     float* delta;  // (B, H, n_ctx)
+    int* key_order;  // the matrix-core kernels' key order (see launch_dense_prologue); null: none is wanted
+    int* n_visible;
 };
 
 template <typename T>
 __global__ void __launch_bounds__(kThreads) bwd_delta_kernel(BwdParams p) {
     const ckv_dense_bwd_args& a = p.a;
+    int64_t blk = blockIdx.x;
+    if (p.key_order && blk-- == 0) {  // the first workgroup sorts the keys
+        key_order_block<kThreads>(a.mask, a.n_kv - a.n_ctx, a.n_ctx, p.key_order, p.n_visible);
+        return;
+    }
     const int wave = threadIdx.x / CKV_WAVE, lane = threadIdx.x % CKV_WAVE;
     const int64_t rows = a.B * a.H * a.n_ctx;
-    const int64_t row = (int64_t)blockIdx.x * (kThreads / CKV_WAVE) + wave;
+    const int64_t row = blk * (kThreads / CKV_WAVE) + wave;
     if (row >= rows) return;
     const int64_t m = row % a.n_ctx, h = (row / a.n_ctx) % a.H, b = row / (a.n_ctx * a.H);
     const T* o = (const T*)a.out + b * a.out_stride[0] + h * a.out_stride[1] + m * a.out_stride[2];
@@ -236,9 +243,12 @@ int run_bwd(const BwdParams& p, hipStream_t stream) {
         if (int rc = current_device_info(&di)) return rc;
         if (lds_dq > (size_t)di.lds_max || lds_kv_ > (size_t)di.lds_max) return CKV_ERR_UNSUPPORTED;
     }
-    hipLaunchKernelGGL(bwd_delta_kernel<T>, dim3((unsigned)((rows + 3) / 4)), dim3(kThreads), 0, stream, p);
+    const bool mfma = bwd_mfma_supported(a);
+    BwdParams pd = p;
+    if (!mfma) pd.key_order = nullptr;
+    hipLaunchKernelGGL(bwd_delta_kernel<T>, dim3((unsigned)((rows + 3) / 4 + (pd.key_order ? 1 : 0))), dim3(kThreads), 0, stream, pd);
     CKV_HIP_TRY(hipGetLastError());
-    if (bwd_mfma_supported(a)) return launch_bwd_mfma(a, p.delta, stream);
+    if (mfma) return launch_bwd_mfma(a, p.delta, p.key_order, p.n_visible, stream);
     if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(bwd_dq_kernel<T>), (int)lds_dq)) return rc;
     hipLaunchKernelGGL(bwd_dq_kernel<T>, dim3((unsigned)((a.n_ctx + kOwn - 1) / kOwn), (unsigned)(a.B * a.H)), dim3(kThreads),
                        lds_dq, stream, p);
@@ -260,6 +270,8 @@ extern "C" int64_t ckv_dense_bwd_workspace_bytes(int64_t B, int64_t H, int64_t n
     return ckv::align_up(B * H * n_ctx * (int64_t)sizeof(float), 256);
 }
 
+extern "C" int64_t ckv_dense_bwd_key_order_bytes(int64_t n_kv) { return n_kv > 0 ? ckv::align_up((n_kv + 1) * (int64_t)sizeof(int), 256) : 0; }
+
 extern "C" int ckv_attn_dense_bwd(const ckv_dense_bwd_args* args, void* stream_) {
     using namespace ckv;
     if (!args) return CKV_ERR_NULL;
@@ -276,6 +288,12 @@ extern "C" int ckv_attn_dense_bwd(const ckv_dense_bwd_args* args, void* stream_)
     BwdParams p;
     p.a = a;
     p.delta = reinterpret_cast<float*>(a.workspace);
+    p.key_order = p.n_visible = nullptr;
+    const int64_t need = ckv_dense_bwd_workspace_bytes(a.B, a.H, a.n_ctx);
+    if (a.workspace_bytes >= need + ckv_dense_bwd_key_order_bytes(a.n_kv)) {
+        p.n_visible = reinterpret_cast<int*>((char*)a.workspace + need);
+        p.key_order = p.n_visible + 1;
+    }
     switch (a.dtype) {
         case CKV_F32: return run_bwd<float>(p, stream);
         case CKV_F16: return run_bwd<__half>(p, stream);

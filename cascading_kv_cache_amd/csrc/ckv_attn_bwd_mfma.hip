@@ -1,5 +1,5 @@
 // Backward of the dense-input attention operator on the matrix cores (cascade/models/flash_attention.py:279-537):
-// bf16 / fp16, head_dim 128, v_mfma_f32_32x32x16.  Two kernels, as in the reference (_attn_bwd_dq, _attn_bwd_dkdv),
+// bf16 / fp16, head_dim 64 or 128 (template parameter kHD), v_mfma_f32_32x32x16.  Two kernels, as in the reference (_attn_bwd_dq, _attn_bwd_dkdv),
 // so that no gradient is accumulated with atomics; both recompute the probabilities from the row normalisers of
 // the forward pass and take delta[m] = sum_d out[m, d] dout[m, d] from the caller.
 //
@@ -13,9 +13,13 @@
 // The A operands K^T, Q^T and dO^T are read from the row-major tiles in LDS with the transposing read
 // ds_read_b64_tr_b16: lane i of a 16-lane group receives element [4e + i/4][i%4] (e = 0..3) of the 16 x 4 matrix
 // whose row r is the 8 bytes lane r points at; with lane r pointing at dims 4 (r%4) .. +3 of row r/4 of a
-// 4-row group, lane i receives dim i of the four rows.  Rows are 256 bytes; the 16-byte piece c of row r sits in
-// slot c ^ (((r & 3) << 2) | ((r >> 2) & 3)), which keeps both the 16-byte row reads (32 rows, one piece) and the
-// transposing reads (4 rows x 64 bytes) off each other's banks.
+// 4-row group, lane i receives dim i of the four rows.  The 16-byte piece c of row r sits in slot c ^ f(r) of its row
+// (swz), with f chosen so that both the 16-byte row reads (32 rows, one piece) and the transposing reads (4 rows x 64
+// bytes) stay off each other's banks.
+//
+// Masked keys: the caller sorts the keys, the visible ones first (launch_dense_prologue), and both kernels take key
+// block i from the rows key_order names, so a masked key costs no work at all; the dk/dv kernel writes its zeros.
+// Without an order (a caller whose workspace has no room for it) the keys are taken as they lie and masked one by one.
 #include "ckv_attn_internal.h"
 
 namespace ckv {
@@ -29,18 +33,21 @@ typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef short s16x4_t __attribute__((ext_vector_type(4)));
 
-constexpr int kHD = 128;              // head dim
 constexpr int kBlk = 32;              // rows of a streamed block
 constexpr int kWaves = 4;             // wavefronts of a workgroup, 32 stationary rows each
 constexpr int kThreads = kWaves * CKV_WAVE;
 constexpr int kOwn = kWaves * 32;     // stationary rows of a workgroup
-constexpr int kRowBytes = kHD * 2;    // 256
-constexpr int kTile = kBlk * kRowBytes;  // 8 KiB
 constexpr float kLog2e = 1.4426950408889634f;
-// dynamic LDS of the dk/dv kernel: two stages of (Q, dO) tiles, the per-row scalars of both stages, V^T operands
-constexpr int kDkdvRowv = 2 * 2 * kTile;
-constexpr int kDkdvV = kDkdvRowv + 2 * 2 * kBlk * (int)sizeof(float);
-constexpr int kDkdvLds = kDkdvV + kWaves * (kHD / 16) * CKV_WAVE * 16;
+template <int kHD>
+struct Geo {
+    static constexpr int kRowBytes = kHD * 2;
+    static constexpr int kTile = kBlk * kRowBytes;  // 8 KiB with 128 dims
+    static constexpr int kPieces = kHD / 8;         // 16-byte pieces of a row
+    // dynamic LDS of the dk/dv kernel: two stages of (Q, dO) tiles, the per-row scalars of both stages, V^T operands
+    static constexpr int kDkdvRowv = 2 * 2 * kTile;
+    static constexpr int kDkdvV = kDkdvRowv + 2 * 2 * kBlk * (int)sizeof(float);
+    static constexpr int kDkdvLds = kDkdvV + kWaves * (kHD / 16) * CKV_WAVE * 16;
+};
 
 template <typename T>
 struct Mma;
@@ -70,41 +77,87 @@ struct Mma<__half> {
 struct BwdMfmaParams {
     ckv_dense_bwd_args a;
     const float* delta;  // (B, H, n_ctx)
+    const int* key_order;  // null: keys as they lie
+    const int* n_visible;
 };
 
-__device__ inline int swz(int row, int piece) { return piece ^ (((row & 3) << 2) | ((row >> 2) & 3)); }
+// 128 dims: a row is all 64 banks, so 16 consecutive rows need 16 different slots for one piece, and the four rows of a
+// transposing read different 64-byte quarters.  64 dims: two rows share the banks, eight slots each, and rows r, r + 2 of
+// a transposing read need different halves.
+template <int kHD>
+__device__ inline int swz(int row, int piece) {
+    if constexpr (kHD == 128) return piece ^ (((row & 3) << 2) | ((row >> 2) & 3));
+    else return piece ^ ((((row >> 1) & 1) << 2) | ((row >> 2) & 3));
+}
 
-// A 32-row block of a (rows, 128) tensor into a tile, global -> LDS without registers: wavefront w copies rows
-// 8 w .. 8 w + 7 with two instructions of 64 x 16 bytes; lane i fills slot i % 16 of row 4 (2 w + j) + i / 16 with
-// the piece that belongs there.  Rows at or past `limit` repeat row limit - 1 (finite values; whatever is
-// computed from them is masked).  The caller waits with vmcnt(0) before the barrier that publishes the tile.
+// The keys of a launch: `n` of them can be seen (cached ones first), position i is row row_of(i) of K and V.
+struct Keys {
+    const int* order;
+    const uint8_t* mask;
+    int64_t n_cached;   // cached keys in front of the chunk keys
+    int64_t n_seen;     // positions below it hold keys some query may see
+    int64_t n_kv;
+    __device__ Keys(const BwdMfmaParams& p) {
+        const int64_t nc = p.a.n_kv - p.a.n_ctx;
+        order = p.key_order;
+        mask = p.a.mask;
+        n_cached = order ? *p.n_visible : nc;
+        n_seen = n_cached + p.a.n_ctx;
+        n_kv = p.a.n_kv;
+    }
+    __device__ int64_t row_of(int64_t i) const { return order ? order[i] : i; }
+    __device__ bool visible(int64_t i) const { return i < n_seen && (order || i >= n_cached || mask[i] == 0); }
+};
+
+// A 32-row block of a (rows, kHD) tensor into a tile, global -> LDS without registers, 1 KiB per instruction; a
+// wavefront copies kRowBytes / 128 of them, lane i of copy j one slot of row block_row(wave, lane, j).  Rows at or past
+// `limit` repeat row limit - 1 (finite values; whatever is computed from them is masked).  The caller waits with vmcnt(0)
+// before the barrier that publishes the tile.
+template <int kHD>
+__device__ inline int block_row(int wave, int lane, int j) {
+    constexpr int kPer = CKV_WAVE / Geo<kHD>::kPieces;   // rows per instruction
+    return kPer * (kHD / 64 * wave + j) + lane / Geo<kHD>::kPieces;
+}
+template <int kHD>
 __device__ inline void copy_block(const char* base, int64_t row_bytes, int64_t first, int64_t limit, uint32_t tile_lds,
                                   int wave, int lane) {
     const char* blk = base + first * row_bytes;  // uniform
 #pragma unroll
-    for (int j = 0; j < 2; j++) {
-        const int row = 4 * (2 * wave + j) + (lane >> 4);
+    for (int j = 0; j < kHD / 64; j++) {
+        const int row = block_row<kHD>(wave, lane, j);
         int64_t rr = row;
         if (first + rr > limit - 1) rr = limit - 1 - first;
-        const uint32_t voff = (uint32_t)(rr * row_bytes) + (uint32_t)(swz(row, lane & 15) << 4);
-        async_copy16(blk, voff, tile_lds + (uint32_t)(4 * (2 * wave + j) * kRowBytes));
+        const uint32_t voff = (uint32_t)(rr * row_bytes) + (uint32_t)(swz<kHD>(row, lane % Geo<kHD>::kPieces) << 4);
+        async_copy16(blk, voff, tile_lds + (uint32_t)((kHD / 64 * wave + j) * 1024));
+    }
+}
+// The same for rows given by number (one per copy of this lane).
+template <int kHD>
+__device__ inline void copy_rows(const char* base, uint32_t row_bytes, const uint32_t (&rows)[kHD / 64], uint32_t tile_lds, int wave,
+                                 int lane) {
+#pragma unroll
+    for (int j = 0; j < kHD / 64; j++) {
+        const uint32_t voff = rows[j] * row_bytes + (uint32_t)(swz<kHD>(block_row<kHD>(wave, lane, j), lane % Geo<kHD>::kPieces) << 4);
+        async_copy16(base, voff, tile_lds + (uint32_t)((kHD / 64 * wave + j) * 1024));
     }
 }
 
 // A operand of a product that contracts over the head dims: row lane%32 of the tile, dims 16 ds + 8 (lane/32) .. +7
+template <int kHD>
 __device__ inline uint4 row_operand(const unsigned char* tile, int lane, int ds) {
     const int row = lane & 31;
-    return *reinterpret_cast<const uint4*>(tile + row * kRowBytes + swz(row, 2 * ds + (lane >> 5)) * 16);
+    return *reinterpret_cast<const uint4*>(tile + row * Geo<kHD>::kRowBytes + swz<kHD>(row, 2 * ds + (lane >> 5)) * 16);
 }
 
 // A operand of a product that contracts over the rows of the tile: dim 32 db + lane%32 of rows
 // 16 s + 8 a + 4 (lane/32) + e (elements 4 a + e), the order in which the packed B operand holds them.
 // `tr_base[a]` is the lane's address for db = 0, s = 0; blocks of 32 dims flip bits 2-3 of the slot.
+template <int kHD>
 __device__ inline uint4 col_operand(uint32_t tile_lds, const int (&tr_base)[2], int s, int db) {
     uint4 r;
 #pragma unroll
     for (int a = 0; a < 2; a++) {
-        const uint32_t addr = tile_lds + (uint32_t)((tr_base[a] ^ (db << 6)) + s * 16 * kRowBytes);
+        const uint32_t addr = tile_lds + (uint32_t)((tr_base[a] ^ (db << 6)) + s * 16 * Geo<kHD>::kRowBytes);
         const s16x4_t v =
             __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_t*)(uintptr_t)addr);
         const uint2 u = __builtin_bit_cast(uint2, v);
@@ -119,13 +172,14 @@ __device__ inline uint4 col_operand(uint32_t tile_lds, const int (&tr_base)[2], 
     return r;
 }
 
+template <int kHD>
 __device__ inline void col_operand_setup(int lane, int (&tr_base)[2]) {
     const int h = lane >> 5, g16 = (lane >> 4) & 1, rl = lane & 15;
 #pragma unroll
     for (int a = 0; a < 2; a++) {
         const int row = 8 * a + 4 * h + (rl >> 2);             // + 16 s
         const int piece = 2 * g16 + ((rl & 3) >> 1);           // + 4 db
-        tr_base[a] = row * kRowBytes + swz(row, piece) * 16 + 8 * (rl & 1);
+        tr_base[a] = row * Geo<kHD>::kRowBytes + swz<kHD>(row, piece) * 16 + 8 * (rl & 1);
     }
 }
 
@@ -154,12 +208,14 @@ __device__ inline f32x16 zero16() {
 // ---------------------------------------------------------------------------------------------
 // dq
 // ---------------------------------------------------------------------------------------------
-template <typename T>
+template <typename T, int kHD>
 __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dq_kernel(BwdMfmaParams p) {
+    constexpr int kTile = Geo<kHD>::kTile;
     __shared__ __attribute__((aligned(16))) unsigned char smem[2][2][kTile];  // [stage][K, V]
     const ckv_dense_bwd_args& a = p.a;
     const int tid = threadIdx.x, wave = tid / CKV_WAVE, lane = tid % CKV_WAVE, h = lane >> 5;
-    const int64_t n_ctx = a.n_ctx, n_kv = a.n_kv, n_cached = n_kv - n_ctx;
+    const Keys keys(p);
+    const int64_t n_ctx = a.n_ctx, n_cached = keys.n_cached;
     const int64_t bh = blockIdx.y, b = bh / a.H, hd = bh % a.H;
     const int64_t m_wg = (int64_t)blockIdx.x * kOwn;
     const int64_t m_lane = m_wg + wave * 32 + (lane & 31);  // this lane's query
@@ -189,7 +245,7 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dq_kernel(BwdMfmaParams 
     const float c2 = a.scale * kLog2e;
 
     int tr_base[2];
-    col_operand_setup(lane, tr_base);
+    col_operand_setup<kHD>(lane, tr_base);
     const uint32_t lds0 = lds_address(&smem[0][0][0]);
 
     f32x16 dq[kHD / 32];
@@ -202,27 +258,39 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dq_kernel(BwdMfmaParams 
     const int64_t n_end = n_cached + m_last + 1;
     const int nblk = (int)((n_end + kBlk - 1) / kBlk);
 
-    // which keys of a block any query may see: inside the tensor, and not masked if cached.  The mask byte of the
-    // block after this one is requested before that block's copies and looked at after this block's work, so
-    // that nothing in between waits for memory.
-    auto mask_byte = [&](int64_t n0) -> uint32_t {
-        const int64_t n = n0 + (lane & 31);
-        return n < n_kv ? (n < n_cached ? (uint32_t)a.mask[n] : 0u) : 1u;
+    // Which keys of a block any query may see, and the rows this lane copies.  Both are requested a block before the
+    // copies that need them and looked at after this block's work, so that nothing in between waits for memory.
+    auto key_bit = [&](int64_t n0) -> uint32_t { return keys.visible(n0 + (lane & 31)) ? 1u : 0u; };
+    auto rows_of = [&](int64_t n0, uint32_t(&r)[kHD / 64]) {
+#pragma unroll
+        for (int j = 0; j < kHD / 64; j++) {
+            int64_t i = n0 + block_row<kHD>(wave, lane, j);
+            if (i > keys.n_seen - 1) i = keys.n_seen - 1;  // a chunk key: finite values, and no query looks at this copy
+            r[j] = (uint32_t)keys.row_of(i);
+        }
     };
-    uint32_t vis = (uint32_t)__ballot(mask_byte(0) == 0u);
-    copy_block(kb, kv_row, 0, n_kv, lds0, wave, lane);
-    copy_block(vb, kv_row, 0, n_kv, lds0 + kTile, wave, lane);
+    const uint32_t row_bytes = (uint32_t)kv_row;
+    uint32_t rows_next[kHD / 64];
+    rows_of(0, rows_next);
+    uint32_t vis = (uint32_t)__ballot(key_bit(0) != 0u);
+    copy_rows<kHD>(kb, row_bytes, rows_next, lds0, wave, lane);
+    copy_rows<kHD>(vb, row_bytes, rows_next, lds0 + kTile, wave, lane);
+    rows_of(kBlk, rows_next);
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
     __syncthreads();
     for (int blk = 0; blk < nblk; blk++) {
         const int st = blk & 1;
         const int64_t n0 = (int64_t)blk * kBlk;
-        uint32_t mb_next = 1u;
+        uint32_t kb_next = 0u;
         if (blk + 1 < nblk) {  // the other stage was last read before the barrier that ended the step before
-            mb_next = mask_byte(n0 + kBlk);
+            uint32_t rows_now[kHD / 64];
+#pragma unroll
+            for (int j = 0; j < kHD / 64; j++) rows_now[j] = rows_next[j];
+            kb_next = key_bit(n0 + kBlk);
+            rows_of(n0 + 2 * kBlk, rows_next);
             __builtin_amdgcn_sched_barrier(0);
-            copy_block(kb, kv_row, n0 + kBlk, n_kv, lds0 + (uint32_t)((st ^ 1) * 2 * kTile), wave, lane);
-            copy_block(vb, kv_row, n0 + kBlk, n_kv, lds0 + (uint32_t)((st ^ 1) * 2 * kTile + kTile), wave, lane);
+            copy_rows<kHD>(kb, row_bytes, rows_now, lds0 + (uint32_t)((st ^ 1) * 2 * kTile), wave, lane);
+            copy_rows<kHD>(vb, row_bytes, rows_now, lds0 + (uint32_t)((st ^ 1) * 2 * kTile + kTile), wave, lane);
         }
         __builtin_amdgcn_sched_barrier(0);
         // keys of this block that are chunk keys past this wavefront's last row: nothing to do for it
@@ -241,12 +309,12 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dq_kernel(BwdMfmaParams 
             f32x16 s = zero16(), dp = zero16();
 #pragma unroll
             for (int ds = 0; ds < kHD / 16; ds++) {
-                s = Mma<T>::mma(row_operand(kt, lane, ds), qreg[ds], s);
+                s = Mma<T>::mma(row_operand<kHD>(kt, lane, ds), qreg[ds], s);
                 if ((ds & 3) == 3) __builtin_amdgcn_sched_barrier(0);
             }
 #pragma unroll
             for (int ds = 0; ds < kHD / 16; ds++) {
-                dp = Mma<T>::mma(row_operand(vt, lane, ds), greg[ds], dp);
+                dp = Mma<T>::mma(row_operand<kHD>(vt, lane, ds), greg[ds], dp);
                 if ((ds & 3) == 3) __builtin_amdgcn_sched_barrier(0);
             }
             // A lane is a query: a row past the end spoils only its own accumulators, which are never stored, so
@@ -272,14 +340,14 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dq_kernel(BwdMfmaParams 
                 const uint4 bop = pack8<T>(dsv, s2);
 #pragma unroll
                 for (int db = 0; db < kHD / 32; db++) {
-                    dq[db] = Mma<T>::mma(col_operand(kt_lds, tr_base, s2, db), bop, dq[db]);
+                    dq[db] = Mma<T>::mma(col_operand<kHD>(kt_lds, tr_base, s2, db), bop, dq[db]);
                     if (db & 1) __builtin_amdgcn_sched_barrier(0);
                 }
             }
         }
         __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wavefront's copies of the next block have landed
-        vis = (uint32_t)__ballot(mb_next == 0u);
+        vis = (uint32_t)__ballot(kb_next != 0u);
         __syncthreads();
     }
     if (row_ok) {
@@ -299,21 +367,24 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dq_kernel(BwdMfmaParams 
 // ---------------------------------------------------------------------------------------------
 // dk, dv
 // ---------------------------------------------------------------------------------------------
-template <typename T>
+template <typename T, int kHD>
 __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dkdv_kernel(BwdMfmaParams p) {
+    constexpr int kTile = Geo<kHD>::kTile;
     extern __shared__ __attribute__((aligned(16))) unsigned char dyn_smem[];
     typedef unsigned char (*TilePtr)[2][kTile];
     typedef float (*RowPtr)[2][kBlk];
     TilePtr smem = reinterpret_cast<TilePtr>(dyn_smem);                                  // [stage][Q, dO]
-    RowPtr rowv = reinterpret_cast<RowPtr>(dyn_smem + kDkdvRowv);                        // [stage][-lse log2 e, delta]
+    RowPtr rowv = reinterpret_cast<RowPtr>(dyn_smem + Geo<kHD>::kDkdvRowv);                        // [stage][-lse log2 e, delta]
     // the V^T operands of a wavefront's 32 keys, in operand order: [wave][ds][lane] 16 bytes each
-    uint4* vstat = reinterpret_cast<uint4*>(dyn_smem + kDkdvV) + (threadIdx.x / CKV_WAVE) * (kHD / 16) * CKV_WAVE;
+    uint4* vstat = reinterpret_cast<uint4*>(dyn_smem + Geo<kHD>::kDkdvV) + (threadIdx.x / CKV_WAVE) * (kHD / 16) * CKV_WAVE;
     const ckv_dense_bwd_args& a = p.a;
     const int tid = threadIdx.x, wave = tid / CKV_WAVE, lane = tid % CKV_WAVE, h = lane >> 5;
-    const int64_t n_ctx = a.n_ctx, n_kv = a.n_kv, n_cached = n_kv - n_ctx;
+    const Keys keys(p);
+    const int64_t n_ctx = a.n_ctx, n_kv = a.n_kv, n_cached = keys.n_cached;
     const int64_t bh = blockIdx.y, b = bh / a.H, hd = bh % a.H;
     const int64_t n_wg = (int64_t)blockIdx.x * kOwn;
     const int64_t n_lane = n_wg + wave * 32 + (lane & 31);  // this lane's key
+    const bool key_ok = keys.visible(n_lane);
     const char* qb = reinterpret_cast<const char*>(a.q) + (b * a.q_stride[0] + hd * a.q_stride[1]) * 2;
     const char* gb = reinterpret_cast<const char*>(a.dout) + (b * a.dout_stride[0] + hd * a.dout_stride[1]) * 2;
     const int64_t q_row = a.q_stride[2] * 2, g_row = a.dout_stride[2] * 2;
@@ -323,27 +394,25 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dkdv_kernel(BwdMfmaParam
     // stationary B operands: K^T of this lane's key in registers, V^T in LDS (the registers go to the accumulators)
     uint4 kreg[kHD / 16];
     {
-        const int64_t off = (b * a.kv_stride[0] + hd * a.kv_stride[1] + n_lane * a.kv_stride[2]) * 2;
+        const int64_t off = (b * a.kv_stride[0] + hd * a.kv_stride[1] + (key_ok ? keys.row_of(n_lane) : 0) * a.kv_stride[2]) * 2;
         const char* krow = reinterpret_cast<const char*>(a.k) + off;
         const char* vrow = reinterpret_cast<const char*>(a.v) + off;
 #pragma unroll
         for (int ds = 0; ds < kHD / 16; ds++) {
             kreg[ds] = make_uint4(0u, 0u, 0u, 0u);
             uint4 vv = make_uint4(0u, 0u, 0u, 0u);
-            if (n_lane < n_kv) {
+            if (key_ok) {
                 kreg[ds] = *reinterpret_cast<const uint4*>(krow + (16 * ds + 8 * h) * 2);
                 vv = *reinterpret_cast<const uint4*>(vrow + (16 * ds + 8 * h) * 2);
             }
             vstat[ds * CKV_WAVE + lane] = vv;
         }
     }
-    bool key_ok = n_lane < n_kv;
-    if (key_ok && n_lane < n_cached) key_ok = a.mask[n_lane] == 0;
     const int64_t first_row = n_lane < n_cached ? 0 : n_lane - n_cached;  // the first query that sees this key
     const float c2 = a.scale * kLog2e;
 
     int tr_base[2];
-    col_operand_setup(lane, tr_base);
+    col_operand_setup<kHD>(lane, tr_base);
     const uint32_t lds0 = lds_address(dyn_smem);
 
     f32x16 dk[kHD / 32], dv[kHD / 32];
@@ -353,7 +422,8 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dkdv_kernel(BwdMfmaParam
     // the first query block any key of the workgroup can be seen from
     const int64_t m_first = n_wg < n_cached ? 0 : n_wg - n_cached;
     const int blk0 = (int)(m_first / kBlk);
-    const int nblk = (int)((n_ctx + kBlk - 1) / kBlk);
+    // keys sorted behind the visible ones: nothing but the zeros at the end
+    const int nblk = n_wg < keys.n_seen ? (int)((n_ctx + kBlk - 1) / kBlk) : 0;
     // does any key of this wavefront exist and pass its mask?
     const bool wave_alive = __ballot(key_ok) != 0ull;
     const int64_t wave_first_key = n_wg + wave * 32;
@@ -367,8 +437,8 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dkdv_kernel(BwdMfmaParam
         }
     };
     if (blk0 < nblk) {
-        copy_block(qb, q_row, (int64_t)blk0 * kBlk, n_ctx, lds0 + (uint32_t)((blk0 & 1) * 2 * kTile), wave, lane);
-        copy_block(gb, g_row, (int64_t)blk0 * kBlk, n_ctx, lds0 + (uint32_t)((blk0 & 1) * 2 * kTile + kTile), wave, lane);
+        copy_block<kHD>(qb, q_row, (int64_t)blk0 * kBlk, n_ctx, lds0 + (uint32_t)((blk0 & 1) * 2 * kTile), wave, lane);
+        copy_block<kHD>(gb, g_row, (int64_t)blk0 * kBlk, n_ctx, lds0 + (uint32_t)((blk0 & 1) * 2 * kTile + kTile), wave, lane);
         load_rowv(blk0 & 1, (int64_t)blk0 * kBlk);
     }
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
@@ -384,8 +454,8 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dkdv_kernel(BwdMfmaParam
                 if (m < n_ctx) rv_next = tid < kBlk ? lse[m] : dl[m];
             }
             __builtin_amdgcn_sched_barrier(0);
-            copy_block(qb, q_row, m0 + kBlk, n_ctx, lds0 + (uint32_t)((st ^ 1) * 2 * kTile), wave, lane);
-            copy_block(gb, g_row, m0 + kBlk, n_ctx, lds0 + (uint32_t)((st ^ 1) * 2 * kTile + kTile), wave, lane);
+            copy_block<kHD>(qb, q_row, m0 + kBlk, n_ctx, lds0 + (uint32_t)((st ^ 1) * 2 * kTile), wave, lane);
+            copy_block<kHD>(gb, g_row, m0 + kBlk, n_ctx, lds0 + (uint32_t)((st ^ 1) * 2 * kTile + kTile), wave, lane);
         }
         // rows before the first chunk key of the wavefront's keys see none of them when all its keys are chunk keys
         const bool dead = !wave_alive || (wave_first_key >= n_cached && wave_first_key - n_cached > m0 + kBlk - 1);
@@ -407,7 +477,7 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dkdv_kernel(BwdMfmaParam
             f32x16 pv = zero16();
 #pragma unroll
             for (int ds = 0; ds < kHD / 16; ds++) {
-                pv = Mma<T>::mma(row_operand(qt, lane, ds), kreg[ds], pv);
+                pv = Mma<T>::mma(row_operand<kHD>(qt, lane, ds), kreg[ds], pv);
                 if ((ds & 3) == 3) __builtin_amdgcn_sched_barrier(0);
             }
 #pragma unroll
@@ -427,14 +497,14 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dkdv_kernel(BwdMfmaParam
                 const uint4 pb = pack8<T>(pv, s2);
 #pragma unroll
                 for (int db = 0; db < kHD / 32; db++) {
-                    dv[db] = Mma<T>::mma(col_operand(gt_lds, tr_base, s2, db), pb, dv[db]);
+                    dv[db] = Mma<T>::mma(col_operand<kHD>(gt_lds, tr_base, s2, db), pb, dv[db]);
                     if (db & 1) __builtin_amdgcn_sched_barrier(0);
                 }
             }
             f32x16 dp = zero16();
 #pragma unroll
             for (int ds = 0; ds < kHD / 16; ds++) {
-                dp = Mma<T>::mma(row_operand(gt, lane, ds), vstat[ds * CKV_WAVE + lane], dp);
+                dp = Mma<T>::mma(row_operand<kHD>(gt, lane, ds), vstat[ds * CKV_WAVE + lane], dp);
                 if (ds & 1) __builtin_amdgcn_sched_barrier(0);
             }
 #pragma unroll
@@ -453,7 +523,7 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dkdv_kernel(BwdMfmaParam
                 const uint4 db_ = pack8<T>(dp, s2);
 #pragma unroll
                 for (int db = 0; db < kHD / 32; db++) {
-                    dk[db] = Mma<T>::mma(col_operand(qt_lds, tr_base, s2, db), db_, dk[db]);
+                    dk[db] = Mma<T>::mma(col_operand<kHD>(qt_lds, tr_base, s2, db), db_, dk[db]);
                     if (db & 1) __builtin_amdgcn_sched_barrier(0);
                 }
             }
@@ -468,7 +538,7 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dkdv_kernel(BwdMfmaParam
         for (int db = 0; db < kHD / 32; db++) dk[db] = dv[db] = zero16();
     }
     if (n_lane < n_kv) {
-        const int64_t off = (b * a.dkv_stride[0] + hd * a.dkv_stride[1] + n_lane * a.dkv_stride[2]) * 2;
+        const int64_t off = (b * a.dkv_stride[0] + hd * a.dkv_stride[1] + keys.row_of(n_lane) * a.dkv_stride[2]) * 2;
         char* ok_ = reinterpret_cast<char*>(a.dk) + off;
         char* ov_ = reinterpret_cast<char*>(a.dv) + off;
 #pragma unroll
@@ -491,15 +561,15 @@ inline bool rows_ok(const int64_t* st) {
     return st[3] == 1 && st[2] % 8 == 0 && st[1] % 8 == 0 && st[0] % 8 == 0 && st[2] > 0 && st[2] < (1 << 24);
 }
 
-template <typename T>
+template <typename T, int kHD>
 int run(const BwdMfmaParams& p, hipStream_t stream) {
     const ckv_dense_bwd_args& a = p.a;
-    hipLaunchKernelGGL(bwd_mfma_dq_kernel<T>, dim3((unsigned)((a.n_ctx + kOwn - 1) / kOwn), (unsigned)(a.B * a.H)),
+    hipLaunchKernelGGL((bwd_mfma_dq_kernel<T, kHD>), dim3((unsigned)((a.n_ctx + kOwn - 1) / kOwn), (unsigned)(a.B * a.H)),
                        dim3(kThreads), 0, stream, p);
     CKV_HIP_TRY(hipGetLastError());
-    if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(bwd_mfma_dkdv_kernel<T>), kDkdvLds)) return rc;
-    hipLaunchKernelGGL(bwd_mfma_dkdv_kernel<T>, dim3((unsigned)((a.n_kv + kOwn - 1) / kOwn), (unsigned)(a.B * a.H)),
-                       dim3(kThreads), kDkdvLds, stream, p);
+    if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(bwd_mfma_dkdv_kernel<T, kHD>), Geo<kHD>::kDkdvLds)) return rc;
+    hipLaunchKernelGGL((bwd_mfma_dkdv_kernel<T, kHD>), dim3((unsigned)((a.n_kv + kOwn - 1) / kOwn), (unsigned)(a.B * a.H)),
+                       dim3(kThreads), Geo<kHD>::kDkdvLds, stream, p);
     CKV_HIP_TRY(hipGetLastError());
     return CKV_OK;
 }
@@ -508,7 +578,8 @@ int run(const BwdMfmaParams& p, hipStream_t stream) {
 
 bool bwd_mfma_supported(const ckv_dense_bwd_args& a) {
     if (a.dtype != CKV_F16 && a.dtype != CKV_BF16) return false;
-    if (a.D != kHD) return false;
+    if (a.D != 64 && a.D != 128) return false;
+    if (a.n_kv * a.kv_stride[2] * 2 >= (int64_t)1 << 32) return false;  // 32-bit byte offsets inside a head
     if (!rows_ok(a.q_stride) || !rows_ok(a.kv_stride) || !rows_ok(a.dout_stride) || !rows_ok(a.dq_stride) ||
         !rows_ok(a.dkv_stride))
         return false;
@@ -516,11 +587,14 @@ bool bwd_mfma_supported(const ckv_dense_bwd_args& a) {
            aligned16(a.dk) && aligned16(a.dv);
 }
 
-int launch_bwd_mfma(const ckv_dense_bwd_args& a, const float* delta, hipStream_t stream) {
+int launch_bwd_mfma(const ckv_dense_bwd_args& a, const float* delta, const int* key_order, const int* n_visible, hipStream_t stream) {
     BwdMfmaParams p;
     p.a = a;
     p.delta = delta;
-    return a.dtype == CKV_F16 ? run<__half>(p, stream) : run<__hip_bfloat16>(p, stream);
+    p.key_order = key_order;
+    p.n_visible = n_visible;
+    if (a.D == 64) return a.dtype == CKV_F16 ? run<__half, 64>(p, stream) : run<__hip_bfloat16, 64>(p, stream);
+    return a.dtype == CKV_F16 ? run<__half, 128>(p, stream) : run<__hip_bfloat16, 128>(p, stream);
 }
 
 }  // namespace ckv

@@ -16,8 +16,7 @@ __device__ inline float round_t(float v) {
 //          w_new[k] = (1-beta) * beta^k built in the tensor dtype (cascade_attention.py:270-276)
 // ---------------------------------------------------------------------------------------------
 template <typename T>
-__global__ void weights_kernel(float* w_ema, float* w_new, int64_t Q, double beta) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+__device__ inline void weights_at(float* w_ema, float* w_new, int64_t Q, double beta, int64_t i) {
     if (i >= Q + kColSlack) return;
     if (i >= Q) {  // slack read (and multiplied by zero) by the MFMA column pass
         w_ema[i] = 0.f;
@@ -29,6 +28,20 @@ __global__ void weights_kernel(float* w_ema, float* w_new, int64_t Q, double bet
     const float bt = round_t<T>(b32);
     const float pw = round_t<T>(powf(bt, round_t<T>((float)i)));
     w_new[i] = round_t<T>(__fmul_rn(omb, pw));
+}
+
+template <typename T>
+__global__ void weights_kernel(float* w_ema, float* w_new, int64_t Q, double beta) {
+    weights_at<T>(w_ema, w_new, Q, beta, (int64_t)blockIdx.x * blockDim.x + threadIdx.x);
+}
+
+// The first workgroup sorts the keys, the others write the weights.  One workgroup is enough: 16 K mask bytes are one
+// 16-byte load per thread and a scan.
+template <typename T>
+__global__ void __launch_bounds__(1024) dense_prologue_kernel(const uint8_t* mask, int64_t n_cached, int64_t n_ctx, int* key_order,
+                                                              int* n_visible, float* w_ema, float* w_new, double beta) {
+    if (blockIdx.x == 0) key_order_block<1024>(mask, n_cached, n_ctx, key_order, n_visible);
+    else weights_at<T>(w_ema, w_new, n_ctx, beta, (int64_t)(blockIdx.x - 1) * blockDim.x + threadIdx.x);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -665,6 +678,21 @@ int launch_weights(float* w_ema, float* w_new, int64_t Q, double beta, int dtype
             break;
         default: return CKV_ERR_DTYPE;
     }
+    CKV_HIP_TRY(hipGetLastError());
+    return CKV_OK;
+}
+
+int launch_dense_prologue(const uint8_t* mask, int64_t n_cached, int64_t n_ctx, int* key_order, int* n_visible, float* w_ema,
+                          float* w_new, double beta, int dtype, hipStream_t stream) {
+    const dim3 grid(1 + (w_ema ? (unsigned)((n_ctx + kColSlack + 1023) / 1024) : 0)), block(1024);
+    if (dtype == CKV_F16)
+        hipLaunchKernelGGL(dense_prologue_kernel<__half>, grid, block, 0, stream, mask, n_cached, n_ctx, key_order, n_visible,
+                           w_ema, w_new, beta);
+    else if (dtype == CKV_BF16)
+        hipLaunchKernelGGL(dense_prologue_kernel<__hip_bfloat16>, grid, block, 0, stream, mask, n_cached, n_ctx, key_order,
+                           n_visible, w_ema, w_new, beta);
+    else
+        return CKV_ERR_DTYPE;
     CKV_HIP_TRY(hipGetLastError());
     return CKV_OK;
 }

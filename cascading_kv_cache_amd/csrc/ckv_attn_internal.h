@@ -38,6 +38,12 @@ int launch_core_generic(const CoreProblem& p, hipStream_t stream);
 // w_ema gets 64 trailing zeros (slack read by the MFMA column pass)
 int launch_weights(float* w_ema, float* w_new, int64_t Q, double beta, int dtype, hipStream_t stream);
 
+// The dense operator's prologue in one launch: the weights of the score sums (w_ema null: none), and the key order: the
+// rows of the cached keys that are not masked, in ascending order, then the n_ctx chunk keys, then the masked ones.
+// mask (n_cached) 1 = masked; key_order (n_cached + n_ctx); n_visible: how many cached keys are not masked.
+int launch_dense_prologue(const uint8_t* mask, int64_t n_cached, int64_t n_ctx, int* key_order, int* n_visible, float* w_ema,
+                          float* w_new, double beta, int dtype, hipStream_t stream);
+
 int launch_cast_scores(const float* colsum, void* scores, const int64_t* stride, int64_t B, int64_t H, int64_t N,
                        int dtype, hipStream_t stream);
 
@@ -67,7 +73,56 @@ int launch_finish(const FinishProblem& p, hipStream_t stream);
 // tiles of this many query rows
 constexpr int64_t kColSlack = 128;
 
-// ---- bf16/fp16 MFMA family (head_dim 128) ----
+// The key order of launch_dense_prologue, worked out by one workgroup of kThreads threads (64 .. 1024, a multiple of 64).
+template <int kThreads>
+__device__ inline void key_order_block(const uint8_t* mask, int64_t n_cached, int64_t n_ctx, int* key_order, int* n_visible) {
+    constexpr int kPer = 16, kWaves = kThreads / CKV_WAVE;
+    __shared__ int wave_sum[2][kWaves];
+    const int tid = threadIdx.x, lane = tid % CKV_WAVE, wave = tid / CKV_WAVE;
+    const int64_t n_kv = n_cached + n_ctx;
+    const bool vec = (reinterpret_cast<uintptr_t>(mask) & 15) == 0;
+    int seen = 0, round = 0;  // visible keys in the stretches before
+    for (int64_t base = 0; base < n_cached; base += kThreads * kPer, round ^= 1) {
+        // this thread's 16 keys as a word of bits, one per visible key
+        const int64_t first = base + (int64_t)tid * kPer;
+        uint32_t bits = 0;
+        if (vec && first + kPer <= n_cached) {
+            const uint4 m = *reinterpret_cast<const uint4*>(mask + first);
+            const uint32_t w[4] = {m.x, m.y, m.z, m.w};
+#pragma unroll
+            for (int i = 0; i < kPer; i++) bits |= (((w[i >> 2] >> (8 * (i & 3))) & 0xffu) == 0u ? 1u : 0u) << i;
+        } else {
+            for (int i = 0; i < kPer; i++)
+                if (first + i < n_cached && mask[first + i] == 0) bits |= 1u << i;
+        }
+        const int mine = __popc(bits);
+        int incl = mine;
+        for (int off = 1; off < CKV_WAVE; off <<= 1) {
+            const int v = __shfl_up(incl, off);
+            if (lane >= off) incl += v;
+        }
+        if (lane == CKV_WAVE - 1) wave_sum[round][wave] = incl;
+        __syncthreads();  // the sums of the next stretch go to the other half
+        int before = seen, total = seen;
+        for (int w = 0; w < kWaves; w++) {
+            const int v = wave_sum[round][w];
+            before += w < wave ? v : 0;
+            total += v;
+        }
+        int vis = before + incl - mine;                              // visible keys before this thread's first one
+        int64_t hid = n_kv - 1 - (first - vis);                      // masked ones fill the end backwards
+        for (int i = 0; i < kPer; i++) {
+            if (first + i >= n_cached) break;
+            if ((bits >> i) & 1u) key_order[vis++] = (int)(first + i);
+            else key_order[hid--] = (int)(first + i);
+        }
+        seen = total;
+    }
+    for (int64_t i = tid; i < n_ctx; i += kThreads) key_order[seen + i] = (int)(n_cached + i);
+    if (tid == 0) *n_visible = seen;
+}
+
+// ---- bf16/fp16 MFMA family (head_dim 64 and 128) ----
 struct MfmaSegment {
     const void* k;
     const void* v;
@@ -94,13 +149,18 @@ struct MfmaProblem {
     float* lse;            // (B, H, Q) natural log
     float* lse2;           // (B*H*Q + kColSlack) scratch: minus the log2-domain normaliser, for the column pass
     float* colsum;         // (B, H, n) or null
+    void* scores = nullptr;  // takes colsum's place: (B, H, n) in the tensor dtype, at the row each key came from
+    int64_t scores_stride[3] = {0, 0, 0};
+    // keys in another order than they lie in memory (launch_dense_prologue): seg[0] then holds all keys
+    const int* key_order = nullptr;
+    const int* n_visible = nullptr;
     float* part_o;         // (mfma_fwd_splits, B*H*Q, D) and
     float* part_l2;        // (mfma_fwd_splits, B*H*Q): the forward kernel's shares, when it splits the keys
     const float* w_ema;
     const float* w_new;
     double beta;           // the EMA factor the weights were built from
     int new_mode;
-    int64_t B, H, KVH, Q, n, n_pad;
+    int64_t B, H, KVH, Q, D, n, n_pad;
     float scale;
     float key_scale;       // keys with position ids are multiplied by this after rotation and rounded again, the
                            // queries carry scale / key_scale: sqrt(scale) for the cascade path, which follows the
@@ -114,12 +174,13 @@ int64_t mfma_n_pad(int64_t n);
 int mfma_fwd_splits(int64_t B, int64_t H, int64_t KVH, int64_t Q, int64_t n, int cus);
 int mfma_fwd_splits_for_workspace(int64_t B, int64_t H, int64_t KVH, int64_t Q, int64_t n);
 int mfma_device_cus();  // compute units of the current device (256 where none can be asked)
-bool mfma_fits(int64_t n);  // the per-tile bookkeeping of n keys fits in LDS
+bool mfma_fits(int64_t n, int64_t D);  // the per-tile bookkeeping of n keys fits in LDS
 int launch_mfma(const MfmaProblem& p, hipStream_t stream);
 
-// ---- backward of the dense operator on the matrix cores (16-bit, head_dim 128, 16-byte addressable rows) ----
+// ---- backward of the dense operator on the matrix cores (16-bit, head_dim 64 and 128, 16-byte addressable rows) ----
+// key_order / n_visible: see launch_dense_prologue; both null when the caller's workspace has no room for them
 bool bwd_mfma_supported(const ckv_dense_bwd_args& a);
-int launch_bwd_mfma(const ckv_dense_bwd_args& a, const float* delta, hipStream_t stream);  // delta: (B, H, n_ctx)
+int launch_bwd_mfma(const ckv_dense_bwd_args& a, const float* delta, const int* key_order, const int* n_visible, hipStream_t stream);  // delta: (B, H, n_ctx)
 
 // ---- single-token decode family (Q == 1, head_dim 128) ----
 bool decode_supported(const ckv_attn_args& a);

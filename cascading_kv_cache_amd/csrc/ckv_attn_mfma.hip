@@ -1,4 +1,4 @@
-// bf16 / fp16 MFMA attention for head_dim 128 on gfx950 (CDNA4, wave64, v_mfma_f32_32x32x16).
+// bf16 / fp16 MFMA attention for head_dim 64 and 128 on gfx950 (CDNA4, wave64, v_mfma_f32_32x32x16).
 //
 // Stages (all stream-ordered):
 //   stage_keys   rotate K on the way into a padded row-major buffer Kr, transpose V into 64-key
@@ -31,7 +31,7 @@ typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 
-constexpr int kD = 128;    // head dim
+// Kernels take the head dim as a template parameter kD: 64 or 128.
 constexpr int kBN = 64;    // keys per tile
 
 constexpr int kRows = 256;    // (head, position) rows per forward workgroup
@@ -110,6 +110,11 @@ struct StageParams {
     void* vt;                // (B*KVH, n_pad/64) V^T tile images, see v_image_off
     unsigned long long* tile_vis;  // (n_pad/64,)
     int64_t B, KVH, n, n_pad;
+    // Keys in another order than they lie in memory, the visible ones first (see key_order_block): staged key i is row
+    // key_order[i] of segment 0, for i < *n_visible + n_chunk; null: keys in order of the segments.
+    const int* key_order;
+    const int* n_visible;
+    int64_t n_chunk;
 };
 
 __device__ inline int find_segment(const StageParams& p, int64_t n, int64_t& local) {
@@ -120,34 +125,49 @@ __device__ inline int find_segment(const StageParams& p, int64_t n, int64_t& loc
     return 2;
 }
 
-// The staged K and V of one 64-key tile are 16 KiB images in exactly the order the forward kernel
+// The staged K and V of one 64-key tile are images of kD * 128 bytes in exactly the order the forward kernel
 // keeps them in LDS, so a tile reaches LDS as a straight copy and the 64 lanes of an operand read
 // touch 1 KiB made of two contiguous halves (no bank conflicts, one base address per lane):
 //   K image:   16-byte piece c (elements 8c .. 8c+7) of key row r at  (c/2)*2048 + (c%2)*1024 + r*16
-//   V^T image: 16-byte piece c (key slots 8c .. 8c+7) of dim row d at (c/2)*4096 + (c%2)*2048 + d*16
+//   V^T image: 16-byte piece c (key slots 8c .. 8c+7) of dim row d at (c/2)*32 kD + (c%2)*16 kD + d*16
 // Key slot 16s + 8h + 4a + e of a V^T row holds key 16s + 8a + 4h + e of the tile: the order in
 // which the logits leave the matrix pipe.
 __device__ __host__ inline int k_image_off(int r, int c) { return (c >> 1) * 2048 + (c & 1) * 1024 + r * 16; }
-__device__ __host__ inline int v_image_off(int d, int c) { return (c >> 1) * 4096 + (c & 1) * 2048 + d * 16; }
+template <int kD>
+__device__ __host__ inline int v_image_off(int d, int c) { return (c >> 1) * (32 * kD) + (c & 1) * (16 * kD) + d * 16; }
 
 // One block of 256 threads stages key tile `tile_i` for the (b, kvh) units split_i, split_i + n_split, ...:
-// thread = (key = tid/4, quarter = tid%4) owns rotation pairs j = 8q .. 8q+7 and 32+8q .. 32+8q+7, i.e. the
-// 16-byte pieces q, 4+q, 8+q and 12+q of its row: the four threads of a row read (and, for queries, write)
-// 64 contiguous bytes per instruction.
+// thread = (key = tid/4, quarter = tid%4) owns rotation pairs j = 8q .. 8q+7 (and, with 128 dims, 32+8q .. 32+8q+7),
+// i.e. the 16-byte pieces q, 4+q (, 8+q and 12+q) of its row: the four threads of a row read (and, for queries,
+// write) 64 contiguous bytes per instruction.
 __device__ inline int stage_pair(int quarter, int i) { return i < 8 ? 8 * quarter + i : 24 + 8 * quarter + i; }
-template <typename T>
+template <typename T, int kD>
 __device__ inline void stage_keys_block(const StageParams& p, int tile_i, int split_i, int n_split, uint32_t (*v_lds)[kD / 2 + 1]) {
+    constexpr int kPieces = kD / 64;     // 16-byte pieces of each half of the row
+    constexpr int kPairs = kD / 8;       // rotation pairs of a thread
     const int tid = threadIdx.x;
     const int key = tid >> 2, quarter = tid & 3;
     const int64_t tile = tile_i;
     const int64_t n = tile * kBN + key;
     int64_t local = 0;
-    const int sidx = n < p.n ? find_segment(p, n, local) : -1;
+    int sidx = -1;
+    int64_t n_all = p.n;
+    if (p.key_order) {
+        // visible keys first: what lies behind them is read by nobody.  The order indexes segment 0, which holds all keys.
+        n_all = *p.n_visible + p.n_chunk;
+        if (tile * kBN >= n_all) return;
+        if (n < n_all) {
+            local = p.key_order[n];
+            sidx = 0;
+        }
+    } else if (n < p.n) {
+        sidx = find_segment(p, n, local);
+    }
 
     if (split_i == 0 && tid < kBN) {  // visibility word of this tile
         const int64_t nn = tile * kBN + tid;
-        bool vis = nn < p.n;
-        if (vis) {
+        bool vis = nn < n_all;
+        if (vis && !p.key_order) {
             int64_t loc;
             const int si = find_segment(p, nn, loc);
             if (p.seg[si].masked) vis = p.seg[si].masked[loc] == 0;
@@ -156,11 +176,11 @@ __device__ inline void stage_keys_block(const StageParams& p, int tile_i, int sp
         if (tid == 0) p.tile_vis[tile] = bal;
     }
 
-    // cos / sin of this thread's 16 rotation pairs, two per word, rounded to the tensor dtype (see RopeWord)
-    RopeWord<T> rw[8];
+    // cos / sin of this thread's rotation pairs, two per word, rounded to the tensor dtype (see RopeWord)
+    RopeWord<T> rw[kPairs / 2];
     auto trig_at = [&](int64_t pos) {
 #pragma unroll
-        for (int k = 0; k < 8; k++) {
+        for (int k = 0; k < kPairs / 2; k++) {
             float sn[2], cs[2];
 #pragma unroll
             for (int e = 0; e < 2; e++) {
@@ -175,12 +195,13 @@ __device__ inline void stage_keys_block(const StageParams& p, int tile_i, int sp
     if (rotate && p.shared_pos) trig_at(p.seg[sidx].pos[local] + p.seg[sidx].pos_shift);
     const bool key_scaled = p.key_scale != 1.0f;
     const int64_t nbh = p.B * p.KVH;
-    // the rows of unit bh as this thread's eight 16-byte pieces (zeros past the last key)
+    // the rows of unit bh as this thread's 16-byte pieces (zeros past the last key)
     struct Rows {
-        uint4 lo[2], hi[2], vlo[2], vhi[2];
+        uint4 lo[kPieces], hi[kPieces], vlo[kPieces], vhi[kPieces];
     };
     auto load_rows = [&](int64_t bh, Rows& r) {
-        r.lo[0] = r.lo[1] = r.hi[0] = r.hi[1] = r.vlo[0] = r.vlo[1] = r.vhi[0] = r.vhi[1] = make_uint4(0, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < kPieces; i++) r.lo[i] = r.hi[i] = r.vlo[i] = r.vhi[i] = make_uint4(0, 0, 0, 0);
         if (sidx < 0 || bh >= nbh) return;
         const int64_t b = bh / p.KVH, kvh = bh % p.KVH;
         const KeySegment& sg = p.seg[sidx];
@@ -188,24 +209,23 @@ __device__ inline void stage_keys_block(const StageParams& p, int tile_i, int sp
         const T* kp = (const T*)sg.k + off;
         const T* vp = (const T*)sg.v + off;
         if (sg.stride[3] == 1 && ((reinterpret_cast<uintptr_t>(kp) | reinterpret_cast<uintptr_t>(vp)) & 15) == 0) {
-            r.lo[0] = *reinterpret_cast<const uint4*>(kp + 8 * quarter);
-            r.lo[1] = *reinterpret_cast<const uint4*>(kp + 32 + 8 * quarter);
-            r.hi[0] = *reinterpret_cast<const uint4*>(kp + 64 + 8 * quarter);
-            r.hi[1] = *reinterpret_cast<const uint4*>(kp + 96 + 8 * quarter);
-            r.vlo[0] = *reinterpret_cast<const uint4*>(vp + 8 * quarter);
-            r.vlo[1] = *reinterpret_cast<const uint4*>(vp + 32 + 8 * quarter);
-            r.vhi[0] = *reinterpret_cast<const uint4*>(vp + 64 + 8 * quarter);
-            r.vhi[1] = *reinterpret_cast<const uint4*>(vp + 96 + 8 * quarter);
+#pragma unroll
+            for (int i = 0; i < kPieces; i++) {
+                r.lo[i] = *reinterpret_cast<const uint4*>(kp + 32 * i + 8 * quarter);
+                r.hi[i] = *reinterpret_cast<const uint4*>(kp + kD / 2 + 32 * i + 8 * quarter);
+                r.vlo[i] = *reinterpret_cast<const uint4*>(vp + 32 * i + 8 * quarter);
+                r.vhi[i] = *reinterpret_cast<const uint4*>(vp + kD / 2 + 32 * i + 8 * quarter);
+            }
         } else {
             T* l0 = reinterpret_cast<T*>(r.lo);
             T* h0 = reinterpret_cast<T*>(r.hi);
             T* vl = reinterpret_cast<T*>(r.vlo);
             T* vh = reinterpret_cast<T*>(r.vhi);
-            for (int i = 0; i < 16; i++) {
+            for (int i = 0; i < kPairs; i++) {
                 l0[i] = kp[stage_pair(quarter, i) * sg.stride[3]];
-                h0[i] = kp[(64 + stage_pair(quarter, i)) * sg.stride[3]];
+                h0[i] = kp[(kD / 2 + stage_pair(quarter, i)) * sg.stride[3]];
                 vl[i] = vp[stage_pair(quarter, i) * sg.stride[3]];
-                vh[i] = vp[(64 + stage_pair(quarter, i)) * sg.stride[3]];
+                vh[i] = vp[(kD / 2 + stage_pair(quarter, i)) * sg.stride[3]];
             }
         }
     };
@@ -217,10 +237,10 @@ __device__ inline void stage_keys_block(const StageParams& p, int tile_i, int sp
         const int64_t b = bh / p.KVH, kvh = bh % p.KVH;
         Rows cur = nxt;
         load_rows(bh + n_split, nxt);
-        uint4(&lo)[2] = cur.lo;
-        uint4(&hi)[2] = cur.hi;
-        uint4(&vlo)[2] = cur.vlo;
-        uint4(&vhi)[2] = cur.vhi;
+        uint4(&lo)[kPieces] = cur.lo;
+        uint4(&hi)[kPieces] = cur.hi;
+        uint4(&vlo)[kPieces] = cur.vlo;
+        uint4(&vhi)[kPieces] = cur.vhi;
         if (sidx >= 0) {
             const KeySegment& sg = p.seg[sidx];
             if (rotate) {
@@ -229,48 +249,51 @@ __device__ inline void stage_keys_block(const StageParams& p, int tile_i, int sp
                 uint32_t* lw = reinterpret_cast<uint32_t*>(lo);
                 uint32_t* hw = reinterpret_cast<uint32_t*>(hi);
 #pragma unroll
-                for (int k = 0; k < 8; k++) rw[k].rotate(lw[k], hw[k], p.key_scale, key_scaled, lw[k], hw[k]);
+                for (int k = 0; k < kPairs / 2; k++) rw[k].rotate(lw[k], hw[k], p.key_scale, key_scaled, lw[k], hw[k]);
             }
         }
         char* kimg = (char*)p.kr + (bh * (p.n_pad / kBN) + tile) * (int64_t)(kD * kBN * sizeof(T));
-        *reinterpret_cast<uint4*>(kimg + k_image_off(key, quarter)) = lo[0];
-        *reinterpret_cast<uint4*>(kimg + k_image_off(key, 4 + quarter)) = lo[1];
-        *reinterpret_cast<uint4*>(kimg + k_image_off(key, 8 + quarter)) = hi[0];
-        *reinterpret_cast<uint4*>(kimg + k_image_off(key, 12 + quarter)) = hi[1];
+#pragma unroll
+        for (int i = 0; i < kPieces; i++) {
+            *reinterpret_cast<uint4*>(kimg + k_image_off(key, 4 * i + quarter)) = lo[i];
+            *reinterpret_cast<uint4*>(kimg + k_image_off(key, kD / 16 + 4 * i + quarter)) = hi[i];
+        }
 
-        // V: through LDS into the transposed tile.  A thread holds elements j and j + 64 of its key row for
-        // the same 16 values of j, so the two travel as one dword: 16 four-byte LDS writes per thread, and on
-        // the way out thread (j, group of 16 key slots) reads 16 dwords and owns 32 bytes of dim row j and of
-        // dim row j + 64, which the 64 lanes of a wavefront store as 1 KiB runs of the image.
+        // V: through LDS into the transposed tile.  A thread holds elements j and j + kD/2 of its key row for
+        // the same kPairs values of j, so the two travel as one dword: kPairs four-byte LDS writes per thread, and on
+        // the way out thread (j, group of kD/8 key slots) reads as many dwords and owns kD/4 bytes of dim row j and of
+        // dim row j + kD/2, which neighbouring lanes store as runs of the image.
         __syncthreads();
         {
             const uint16_t* vl = reinterpret_cast<const uint16_t*>(vlo);
             const uint16_t* vh = reinterpret_cast<const uint16_t*>(vhi);
 #pragma unroll
-            for (int i = 0; i < 16; i++) v_lds[key][stage_pair(quarter, i)] = (uint32_t)vl[i] | ((uint32_t)vh[i] << 16);
+            for (int i = 0; i < kPairs; i++) v_lds[key][stage_pair(quarter, i)] = (uint32_t)vl[i] | ((uint32_t)vh[i] << 16);
         }
         __syncthreads();
         char* vimg = (char*)p.vt + (bh * (p.n_pad / kBN) + tile) * (int64_t)(kD * kBN * sizeof(T));
         {
-            const int j = tid & 63, g = tid >> 6;
-            uint32_t w[16];
+            constexpr int kSlotsPer = kD / 8;   // key slots of a thread
+            const int j = tid % (kD / 2), g = tid / (kD / 2);
+            uint32_t w[kSlotsPer];
 #pragma unroll
-            for (int sl = 0; sl < 16; sl++) {
-                // inverse of vt_slot: slot = 16g + 8h + 4a + e  ->  key = 16g + 8a + 4h + e
-                const int h = (sl >> 3) & 1, a = (sl >> 2) & 1, e = sl & 3;
-                w[sl] = v_lds[16 * g + 8 * a + 4 * h + e][j];
+            for (int sl = 0; sl < kSlotsPer; sl++) {
+                // inverse of vt_slot: slot = 16s + 8h + 4a + e  ->  key = 16s + 8a + 4h + e
+                const int slot = kSlotsPer * g + sl;
+                const int h = (slot >> 3) & 1, a = (slot >> 2) & 1, e = slot & 3;
+                w[sl] = v_lds[(slot & ~15) + 8 * a + 4 * h + e][j];
             }
-            uint32_t lo_row[8], hi_row[8];
+            uint32_t lo_row[kSlotsPer / 2], hi_row[kSlotsPer / 2];
 #pragma unroll
-            for (int k = 0; k < 8; k++) {
+            for (int k = 0; k < kSlotsPer / 2; k++) {
                 lo_row[k] = (w[2 * k] & 0xffffu) | (w[2 * k + 1] << 16);
                 hi_row[k] = (w[2 * k] >> 16) | (w[2 * k + 1] & 0xffff0000u);
             }
 #pragma unroll
-            for (int i = 0; i < 2; i++) {
-                *reinterpret_cast<uint4*>(vimg + v_image_off(j, 2 * g + i)) =
+            for (int i = 0; i < kPieces; i++) {
+                *reinterpret_cast<uint4*>(vimg + v_image_off<kD>(j, kPieces * g + i)) =
                     make_uint4(lo_row[4 * i], lo_row[4 * i + 1], lo_row[4 * i + 2], lo_row[4 * i + 3]);
-                *reinterpret_cast<uint4*>(vimg + v_image_off(j + 64, 2 * g + i)) =
+                *reinterpret_cast<uint4*>(vimg + v_image_off<kD>(j + kD / 2, kPieces * g + i)) =
                     make_uint4(hi_row[4 * i], hi_row[4 * i + 1], hi_row[4 * i + 2], hi_row[4 * i + 3]);
             }
         }
@@ -293,17 +316,18 @@ struct StageQParams {
 // thread = (position m, quarter of the rotation pairs); the cos/sin of the position are computed once
 // and reused for the batch x head rows share_i, share_i + n_share, ...; a block of 256 threads covers
 // positions 64 blk .. 64 blk + 63
-template <typename T>
+template <typename T, int kD>
 __device__ inline void stage_q_block(const StageQParams& p, int blk, int share_i, int n_share) {
     const int64_t idx = (int64_t)blk * 256 + threadIdx.x;
     const int64_t m = idx >> 2;
     const int quarter = idx & 3;
     if (m >= p.Q) return;
-    RopeWord<T> rw[8];
+    constexpr int kPieces = kD / 64, kPairs = kD / 8;
+    RopeWord<T> rw[kPairs / 2];
     if (p.q_pos) {
         const int64_t pos = p.q_pos[m];
 #pragma unroll
-        for (int k = 0; k < 8; k++) {
+        for (int k = 0; k < kPairs / 2; k++) {
             float sn[2], cs[2];
 #pragma unroll
             for (int e = 0; e < 2; e++) {
@@ -316,22 +340,23 @@ __device__ inline void stage_q_block(const StageQParams& p, int blk, int share_i
     }
     const int64_t nbh = p.rows / p.Q;
     struct Row {
-        T lo[16], hi[16];
+        T lo[kPairs], hi[kPairs];
     };
     auto load_row = [&](int64_t bh, Row& r) {
         if (bh >= nbh) return;
         const int64_t b = bh / p.H, h = bh % p.H;
         const T* src = (const T*)p.q + b * p.stride[0] + h * p.stride[1] + m * p.stride[2];
         if (p.vec) {  // unit stride and 16-byte aligned rows
-            reinterpret_cast<uint4*>(r.lo)[0] = *reinterpret_cast<const uint4*>(src + 8 * quarter);
-            reinterpret_cast<uint4*>(r.lo)[1] = *reinterpret_cast<const uint4*>(src + 32 + 8 * quarter);
-            reinterpret_cast<uint4*>(r.hi)[0] = *reinterpret_cast<const uint4*>(src + 64 + 8 * quarter);
-            reinterpret_cast<uint4*>(r.hi)[1] = *reinterpret_cast<const uint4*>(src + 96 + 8 * quarter);
+#pragma unroll
+            for (int i = 0; i < kPieces; i++) {
+                reinterpret_cast<uint4*>(r.lo)[i] = *reinterpret_cast<const uint4*>(src + 32 * i + 8 * quarter);
+                reinterpret_cast<uint4*>(r.hi)[i] = *reinterpret_cast<const uint4*>(src + kD / 2 + 32 * i + 8 * quarter);
+            }
         } else {
 #pragma unroll
-            for (int i = 0; i < 16; i++) {
+            for (int i = 0; i < kPairs; i++) {
                 r.lo[i] = src[stage_pair(quarter, i) * p.stride[3]];
-                r.hi[i] = src[(64 + stage_pair(quarter, i)) * p.stride[3]];
+                r.hi[i] = src[(kD / 2 + stage_pair(quarter, i)) * p.stride[3]];
             }
         }
     };
@@ -344,7 +369,7 @@ __device__ inline void stage_q_block(const StageQParams& p, int blk, int share_i
         uint32_t* lw = reinterpret_cast<uint32_t*>(r.lo);
         uint32_t* hw = reinterpret_cast<uint32_t*>(r.hi);
 #pragma unroll
-        for (int k = 0; k < 8; k++) {  // on packed pairs, as in stage_keys_block
+        for (int k = 0; k < kPairs / 2; k++) {  // on packed pairs, as in stage_keys_block
             if (p.q_pos) {
                 rw[k].rotate(lw[k], hw[k], p.qscale, true, lw[k], hw[k]);
             } else {
@@ -353,10 +378,11 @@ __device__ inline void stage_q_block(const StageQParams& p, int blk, int share_i
             }
         }
         T* dst = (T*)p.qr + (bh * p.Q + m) * kD;
-        *reinterpret_cast<uint4*>(dst + 8 * quarter) = reinterpret_cast<uint4*>(r.lo)[0];
-        *reinterpret_cast<uint4*>(dst + 32 + 8 * quarter) = reinterpret_cast<uint4*>(r.lo)[1];
-        *reinterpret_cast<uint4*>(dst + 64 + 8 * quarter) = reinterpret_cast<uint4*>(r.hi)[0];
-        *reinterpret_cast<uint4*>(dst + 96 + 8 * quarter) = reinterpret_cast<uint4*>(r.hi)[1];
+#pragma unroll
+        for (int i = 0; i < kPieces; i++) {
+            *reinterpret_cast<uint4*>(dst + 32 * i + 8 * quarter) = reinterpret_cast<uint4*>(r.lo)[i];
+            *reinterpret_cast<uint4*>(dst + kD / 2 + 32 * i + 8 * quarter) = reinterpret_cast<uint4*>(r.hi)[i];
+        }
     };
     // two rows per trip, both requested before either is rotated: a block is a chain of trips to
     // memory, and this halves it
@@ -374,16 +400,16 @@ __device__ inline void stage_q_block(const StageQParams& p, int blk, int share_i
 struct StageGrid {
     int q_bx, q_by, k_bx, k_by;
 };
-template <typename T>
+template <typename T, int kD>
 __global__ void __launch_bounds__(256) stage_kernel(StageParams sp, StageQParams sq, StageGrid g) {
-    __shared__ uint32_t v_lds[kBN][kD / 2 + 1];  // (d, d + 64) pairs of a key row, odd pitch
+    __shared__ uint32_t v_lds[kBN][kD / 2 + 1];  // (d, d + kD/2) pairs of a key row, odd pitch
     const int nk = g.k_bx * g.k_by;
     int id = blockIdx.x;
     if (id < nk) {
-        stage_keys_block<T>(sp, id % g.k_bx, id / g.k_bx, g.k_by, v_lds);
+        stage_keys_block<T, kD>(sp, id % g.k_bx, id / g.k_bx, g.k_by, v_lds);
     } else {
         id -= nk;
-        stage_q_block<T>(sq, id % g.q_bx, id / g.q_bx, g.q_by);
+        stage_q_block<T, kD>(sq, id % g.q_bx, id / g.q_bx, g.q_by);
     }
 }
 
@@ -409,12 +435,17 @@ struct FwdParams {
     int n_split;
     float* part_o;    // (n_split, B*H*Q, D)
     float* part_l2;   // (n_split, B*H*Q): m_ref + log2(l) of the share, -inf when it holds no visible key
+    const int* n_visible;  // when the keys were staged in key order: the number of cached keys (null: Nc)
 };
 
-// LDS tile of 256-byte rows taken from a row-major matrix (the query tile of the column pass): unpadded
+// LDS tile of rows of 2 kD bytes taken from a row-major matrix (the query tile of the column pass): unpadded
 // (the async copy writes 1 KiB per wavefront contiguously); bank conflicts are avoided by XOR-swizzling
-// the 16-byte piece index with the row: piece c of row r lives at r*256 + ((c ^ (r & 15)) << 4)
-__device__ inline int k_lds_off(int r, int c) { return r * 256 + ((c ^ (r & 15)) << 4); }
+// the 16-byte piece index with the row, so that one piece of 16 consecutive rows covers all 256 bytes of banks:
+// piece c of row r lives at r * 2 kD + ((c ^ row_swizzle(r)) << 4)
+template <int kD>
+__device__ inline int row_swizzle(int r) { return kD == 128 ? (r & 15) : ((r >> 1) & 7); }
+template <int kD>
+__device__ inline int k_lds_off(int r, int c) { return r * (2 * kD) + ((c ^ row_swizzle<kD>(r)) << 4); }
 
 // max over the two lane halves (lane l and lane l ^ 32) without a trip through LDS
 __device__ inline float half_max(float x) {
@@ -429,17 +460,20 @@ __device__ inline float half_max(float x) {
 // tile i+3 and V^T tile i+2, which are first read in iteration i+2: the barrier between two
 // iterations waits only for the copies of the iteration before the last one (those of the last one
 // stay in flight across it), and the first operands of an iteration can be fetched before its barrier.
-constexpr int kPipeStage = 16384;
 constexpr int kKStages = 3, kVStages = 4;
-constexpr int kPipeLds = (kKStages + kVStages) * kPipeStage;   // K0 K1 K2 V0 V1 V2 V3
+__host__ __device__ constexpr int pipe_stages_lds(int head_dim) { return (kKStages + kVStages) * head_dim * 2 * kBN; }   // K0 K1 K2 V0 V1 V2 V3
 // stages, one visibility word and one work-list entry per key tile, the list length
-inline int64_t pipe_lds_bytes(int64_t n_pad) { return kPipeLds + (n_pad / kBN) * 12 + 16; }
+inline int64_t pipe_lds_bytes(int64_t n_pad, int head_dim) { return pipe_stages_lds(head_dim) + (n_pad / kBN) * 12 + 16; }
 constexpr int64_t kLdsLimit = 160 * 1024;
 
-template <typename T>
+template <typename T, int kD>
 __global__ void __launch_bounds__(512) fwd_pipe_kernel(FwdParams p) {
     extern __shared__ __align__(16) unsigned char smem[];
-    constexpr int kThreads = 512, kBlocksPerWave = 2, kAhead = 3;
+    constexpr int kPipeStage = kD * 2 * kBN, kPipeLds = pipe_stages_lds(kD);
+    constexpr int kThreads = 512, kBlocksPerWave = kPipeStage / 8192, kAhead = 3;
+    constexpr int kDB = kD / 32, kKK = kD / 16;          // blocks of 32 dims; contraction steps of the logits
+    constexpr int kPvSlots = 4 * kDB, kQkSlots = 2 * kKK; // matrix instructions of a tile's two products
+    const int Nc = p.n_visible ? *p.n_visible : (int)p.Nc;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col = lane & 31, half = lane >> 5;
@@ -466,7 +500,7 @@ __global__ void __launch_bounds__(512) fwd_pipe_kernel(FwdParams p) {
     const int m0 = qt_i * kRows / p.G;
     int m_hi = (qt_i * kRows + kRows - 1) / p.G;
     if (m_hi > (int)p.Q - 1) m_hi = (int)p.Q - 1;
-    const int n_tiles = (int)((p.Nc + m_hi) / kBN) + 1;
+    const int n_tiles = (Nc + m_hi) / kBN + 1;
     const int tiles_cap = (int)(p.n_pad / kBN);
     unsigned long long* vis_lds = reinterpret_cast<unsigned long long*>(smem + kPipeLds);
     int* list_lds = reinterpret_cast<int*>(smem + kPipeLds + 8 * tiles_cap);
@@ -482,7 +516,7 @@ __global__ void __launch_bounds__(512) fwd_pipe_kernel(FwdParams p) {
             const unsigned long long v = t < n_tiles ? vis_lds[t] : 0ull;
             const unsigned long long bal = __ballot(v != 0ull);
             if (v != 0ull) {
-                const bool partial = (v != ~0ull) || (t * kBN + kBN - 1 - (int)p.Nc > m0);
+                const bool partial = (v != ~0ull) || (t * kBN + kBN - 1 - Nc > m0);
                 list_lds[cnt + __popcll(bal & ((1ull << lane) - 1ull))] = t | (partial ? (int)0x80000000 : 0);
             }
             cnt += __popcll(bal);
@@ -497,7 +531,7 @@ __global__ void __launch_bounds__(512) fwd_pipe_kernel(FwdParams p) {
 
     // ---- the query row this lane owns as MFMA column `col`
     int row_m;
-    uint4 qreg[8];
+    uint4 qreg[kKK];
     {
         const int rf = qt_i * kRows + wave * 32 + col;
         const int g = rf % p.G;
@@ -506,13 +540,13 @@ __global__ void __launch_bounds__(512) fwd_pipe_kernel(FwdParams p) {
         const bool row_ok = row_m < p.Q;
         const T* qrow = (const T*)p.qr + ((b * p.H + row_h) * p.Q + row_m) * kD;
 #pragma unroll
-        for (int kk = 0; kk < 8; kk++) {
+        for (int kk = 0; kk < kKK; kk++) {
             qreg[kk] = row_ok ? *reinterpret_cast<const uint4*>(qrow + 16 * kk + 8 * half) : make_uint4(0, 0, 0, 0);
         }
     }
-    f32x16 oacc[4];
+    f32x16 oacc[kDB];
 #pragma unroll
-    for (int dt = 0; dt < 4; dt++)
+    for (int dt = 0; dt < kDB; dt++)
 #pragma unroll
         for (int v = 0; v < 16; v++) oacc[dt][v] = 0.f;
     // m_ref: the reference the row's logits and sums are relative to; m_run: running maximum relative to it
@@ -528,7 +562,7 @@ __global__ void __launch_bounds__(512) fwd_pipe_kernel(FwdParams p) {
     // k_base: key row `col` of the K stage with the next logits' tile; v_base: dim row `col` of the V^T
     // stage with the tile to multiply.
     int k_base = k_image_off(col, half);
-    int v_base = v_image_off(col, half) + (kKStages + kVStages - 1) * kPipeStage;
+    int v_base = v_image_off<kD>(col, half) + (kKStages + kVStages - 1) * kPipeStage;
     int k_rd = 0, v_rd = kVStages - 1;  // the stages k_base / v_base point at
     auto advance_k = [&]() {
         k_base += k_rd == kKStages - 1 ? -(kKStages - 1) * kPipeStage : kPipeStage;
@@ -540,7 +574,7 @@ __global__ void __launch_bounds__(512) fwd_pipe_kernel(FwdParams p) {
     };
     // K piece (kk, ks): contraction step kk of key rows 32ks ..; V^T piece (s, dt): step s of dim rows 32dt ..
     auto k_piece = [&](int kk, int ks) { return *reinterpret_cast<const uint4*>(smem + k_base + kk * 2048 + ks * 512); };
-    auto v_piece = [&](int s_, int dt) { return *reinterpret_cast<const uint4*>(smem + v_base + s_ * 4096 + dt * 512); };
+    auto v_piece = [&](int s_, int dt) { return *reinterpret_cast<const uint4*>(smem + v_base + s_ * (32 * kD) + dt * 512); };
     const uint32_t copy_off = lane * 16;  // a wavefront copies 1 KiB blocks of an image as they are
     const char* kbase = (const char*)uniform_ptr((const char*)p.kr + bkv * p.n_pad * kD * (int64_t)sizeof(T));
     const char* vbase = (const char*)uniform_ptr((const char*)p.vt + bkv * p.n_pad * kD * (int64_t)sizeof(T));
@@ -562,7 +596,7 @@ __global__ void __launch_bounds__(512) fwd_pipe_kernel(FwdParams p) {
 #pragma unroll
         for (int ks = 0; ks < 2; ks++) s[ks] = cinit;
 #pragma unroll
-        for (int kk = 0; kk < 8; kk++) {
+        for (int kk = 0; kk < kKK; kk++) {
 #pragma unroll
             for (int ks = 0; ks < 2; ks++) {
                 s[ks] = Mma<T>::mma(k_piece(kk, ks), qreg[kk], s[ks]);
@@ -575,7 +609,7 @@ __global__ void __launch_bounds__(512) fwd_pipe_kernel(FwdParams p) {
 #pragma unroll
         for (int s = 0; s < 4; s++) {
 #pragma unroll
-            for (int dt = 0; dt < 4; dt++) {
+            for (int dt = 0; dt < kDB; dt++) {
                 const uint4 a = v_piece(s, dt);
                 const uint4 bq = make_uint4(pk[s][0], pk[s][1], pk[s][2], pk[s][3]);
                 oacc[dt] = Mma<T>::mma(a, bq, oacc[dt]);
@@ -588,9 +622,9 @@ __global__ void __launch_bounds__(512) fwd_pipe_kernel(FwdParams p) {
     auto mask_tile = [&](int entry, f32x16(&s)[2]) {
         const int t = entry & 0x7fffffff;
         unsigned long long allowed = vis_lds[t];
-        const int limit = row_m - (t * kBN - (int)p.Nc);  // last key index of the tile the row may see, if it is a chunk tile
-        if (t * kBN + kBN - 1 >= (int)p.Nc) {             // the tile holds chunk keys
-            const int first_chunk = (int)p.Nc - t * kBN;  // <= 0 when the whole tile is chunk
+        const int limit = row_m - (t * kBN - Nc);  // last key index of the tile the row may see, if it is a chunk tile
+        if (t * kBN + kBN - 1 >= Nc) {             // the tile holds chunk keys
+            const int first_chunk = Nc - t * kBN;  // <= 0 when the whole tile is chunk
             unsigned long long causal = limit >= 63 ? ~0ull : (limit < 0 ? 0ull : ((2ull << limit) - 1ull));
             if (first_chunk > 0) causal |= (1ull << first_chunk) - 1ull;  // cached keys in front of the chunk: always allowed
             allowed &= causal;
@@ -611,15 +645,15 @@ __global__ void __launch_bounds__(512) fwd_pipe_kernel(FwdParams p) {
     auto rescale = [&]() {
         if (__builtin_amdgcn_ballot_w64(alpha != 1.f) != 0ull) {
 #pragma unroll
-            for (int dt = 0; dt < 4; dt++)
+            for (int dt = 0; dt < kDB; dt++)
 #pragma unroll
                 for (int v = 0; v < 16; v++) oacc[dt][v] *= alpha;
         }
     };
 
-    // Iteration i, written in issue order: 32 slots, each one matrix instruction (slots 0..15: P.V of
-    // tile i-1 out of the V^T stage at v_base, slots 16..31: logits of tile i+1 out of the K stage at
-    // k_base), the LDS read of the operand kAhead slots ahead, and a slice of the softmax of tile i.
+    // Iteration i, written in issue order: 32 slots (16 with 64 dims; the figures below are for 128), each one
+    // matrix instruction (slots 0..15: P.V of tile i-1 out of the V^T stage at v_base, slots 16..31: logits of
+    // tile i+1 out of the K stage at k_base), the LDS read of the operand kAhead slots ahead, and a slice of the softmax of tile i.
     // Scheduling barriers keep the slots as written, so matrix and vector instructions alternate
     // inside the wavefront.  The probabilities of tile i overwrite those of tile i-1 piece by piece,
     // each after its last use by the P.V product.  The copies (V^T tile t_v = i+2 into stage v_wr, K
@@ -632,18 +666,18 @@ __global__ void __launch_bounds__(512) fwd_pipe_kernel(FwdParams p) {
     auto iteration = [&](auto with_pv, int entry, int t_v, int t_k, f32x16(&s_cur)[2], f32x16(&s_nxt)[2],
                          uint4(&pre)[kAhead], int fetch_idx, int& fetched) {
         constexpr bool kPV = decltype(with_pv)::value;
-        constexpr int kSlots = kPV ? 32 : 16, kQk0 = kPV ? 16 : 0;
-        constexpr int kCopyStep = kSlots / 4;
+        constexpr int kSlots = kPV ? kPvSlots + kQkSlots : kQkSlots, kQk0 = kPV ? kPvSlots : 0;
+        constexpr int kCopies = 2 * kBlocksPerWave, kCopyStep = kSlots / kCopies;
         const int v_wr = v_rd == 0 ? kVStages - 1 : v_rd - 1;   // (v_rd + 3) % 4
         const int k_wr = k_rd == 0 ? kKStages - 1 : k_rd - 1;   // (k_rd + 2) % 3
         if (entry < 0) mask_tile(entry, s_cur);
         rescale();  // tile i-2 is in the accumulator; tile i-1, scaled for the newer reference, is added below
         auto operand = [&](int k) -> uint4 {
             if (k >= kQk0) {
-                const int j = k - kQk0;  // K piece (kk, ks) = (j % 8, j / 8): one 32-key block after the other
-                return k_piece(j & 7, j >> 3);
+                const int j = k - kQk0;  // K piece (kk, ks) = (j % kKK, j / kKK): one 32-key block after the other
+                return k_piece(j % kKK, j / kKK);
             }
-            return v_piece(k >> 2, k & 3);
+            return v_piece(k / kDB, k % kDB);
         };
         uint4 ops[kSlots];
         if (kPV) {
@@ -656,28 +690,28 @@ __global__ void __launch_bounds__(512) fwd_pipe_kernel(FwdParams p) {
         // pair of probabilities per slot: the first 32-key block of the tile is consumed by slot 15 and the
         // second by slot 23, just before the matrix pipe starts to overwrite them with the next tile's
         // logits (slots 16..23 and 24..31), so one set of logit registers serves both tiles.
-        constexpr int kMaxSlots = kPV ? 8 : 4;             // slots with running maxima
+        constexpr int kMaxSlots = kPV ? kPvSlots / 2 : kQkSlots / 4;  // slots with running maxima
         constexpr int kMaxPer = 32 / kMaxSlots;            // logits per such slot
         constexpr int kExpFirst = kMaxSlots;               // first slot with probabilities
-        constexpr int kExpPer = kPV ? 1 : 2;               // pairs per slot
+        constexpr int kExpPer = 16 / (kPV ? kPvSlots : kQkSlots / 2);  // pairs per slot
         float q0[kExpPer], q1[kExpPer];                    // exponentials of the previous slot, packed one slot later
         int raw_entry = 0;
         bool moved = true;                                 // some row of the wavefront takes a new reference
         auto slot = [&](int k) {
             if (kPV && k + kAhead < kSlots) ops[k + kAhead] = operand(k + kAhead);
             if (k % kCopyStep == 1) {
-                const int q = k / kCopyStep;               // 0, 1: V^T blocks; 2, 3: K blocks
-                if (q < 2) copy_v(t_v, v_wr, q);
-                else copy_k(t_k, k_wr, q - 2);
+                const int q = k / kCopyStep;               // the V^T blocks, then the K blocks
+                if (q < kBlocksPerWave) copy_v(t_v, v_wr, q);
+                else copy_k(t_k, k_wr, q - kBlocksPerWave);
             }
             if (k == 4) raw_entry = list_lds[fetch_idx];
             if (!kPV) {
                 // the first iteration of a workgroup: the next tile's logits follow the slots (below)
             } else if (k >= kQk0) {
                 const int j = k - kQk0;
-                s_nxt[j >> 3] = Mma<T>::mma(ops[k], qreg[j & 7], (j & 7) == 0 ? cinit : s_nxt[j >> 3]);
+                s_nxt[j / kKK] = Mma<T>::mma(ops[k], qreg[j % kKK], j % kKK == 0 ? cinit : s_nxt[j / kKK]);
             } else {
-                const int st = k >> 2, dt = k & 3;
+                const int st = k / kDB, dt = k % kDB;
                 const uint4 bq = make_uint4(pk[st][0], pk[st][1], pk[st][2], pk[st][3]);
                 oacc[dt] = Mma<T>::mma(ops[k], bq, oacc[dt]);
             }
@@ -745,7 +779,7 @@ __global__ void __launch_bounds__(512) fwd_pipe_kernel(FwdParams p) {
         advance_v();
         advance_k();
 #pragma unroll
-        for (int k = 0; k < kAhead; k++) pre[k] = v_piece(k >> 2, k & 3);
+        for (int k = 0; k < kAhead; k++) pre[k] = v_piece(k / kDB, k % kDB);
         // keep the packed probabilities in this region (they are next read after the barrier)
 #pragma unroll
         for (int st = 0; st < 4; st++) asm volatile("" ::"v"(pk[st][0]), "v"(pk[st][1]), "v"(pk[st][2]), "v"(pk[st][3]));
@@ -771,8 +805,8 @@ __global__ void __launch_bounds__(512) fwd_pipe_kernel(FwdParams p) {
         int e0 = work(0), e1 = work(1), e2 = work(2), e3 = work(3), e4 = 0;
         __syncthreads();                     // every wavefront is done with K stage 0
         iteration(std::false_type{}, e0, e2 & 0x7fffffff, e3 & 0x7fffffff, sA, sB, pre, clamp_idx(4), e4);
-        // all copies but the four of the iteration just finished have landed
-        constexpr int kWaitOlder = 0x0F74;   // vmcnt(4)
+        // all copies but those of the iteration just finished have landed
+        constexpr int kWaitOlder = 0x0F70 + 2 * kBlocksPerWave;   // vmcnt
         for (int i = 1; i < n_work; i += 2) {
             e0 = e1; e1 = e2; e2 = e3; e3 = e4;
             __builtin_amdgcn_s_waitcnt(kWaitOlder);
@@ -802,7 +836,7 @@ __global__ void __launch_bounds__(512) fwd_pipe_kernel(FwdParams p) {
             const float inv_p = any ? 1.f / l_tot : 0.f;
             float* po = p.part_o + ((int64_t)split_i * p.B * p.H * p.Q + row_p) * kD;
 #pragma unroll
-            for (int dt = 0; dt < 4; dt++)
+            for (int dt = 0; dt < kDB; dt++)
 #pragma unroll
                 for (int v4 = 0; v4 < 4; v4++)
                     *reinterpret_cast<float4*>(po + 32 * dt + 8 * v4 + 4 * half) =
@@ -820,13 +854,13 @@ __global__ void __launch_bounds__(512) fwd_pipe_kernel(FwdParams p) {
     const bool rows16 = p.out_stride[3] == 1 && (reinterpret_cast<uintptr_t>(p.out) & 15) == 0 && p.out_stride[0] % 8 == 0 &&
                         p.out_stride[1] % 8 == 0 && p.out_stride[2] % 8 == 0;
     if (rows16) {
-        // through LDS, so that a row leaves as 16-byte pieces of 16 neighbouring lanes (a lane's own
+        // through LDS, so that a row leaves as 16-byte pieces of neighbouring lanes (a lane's own
         // 8-byte pieces would reach memory as partly filled 32-byte sectors)
-        constexpr int kRowPitch = 256 + 16;  // bytes; the pad spreads the banks
+        constexpr int kRowPitch = 2 * kD + 16;  // bytes; the pad spreads the banks
         __syncthreads();                      // the tile stages are no longer read
         unsigned char* ow = smem + wave * (32 * kRowPitch);
 #pragma unroll
-        for (int dt = 0; dt < 4; dt++) {
+        for (int dt = 0; dt < kDB; dt++) {
 #pragma unroll
             for (int v4 = 0; v4 < 4; v4++) {
                 uint2 w;
@@ -837,10 +871,11 @@ __global__ void __launch_bounds__(512) fwd_pipe_kernel(FwdParams p) {
         }
         __builtin_amdgcn_s_waitcnt(0xC07F);
         __builtin_amdgcn_wave_barrier();
-        // 4 rows per pass: lane = (row in the pass, 16-byte piece)
+        // lane = (row in the pass, 16-byte piece)
+        constexpr int kPieces = kD / 8, kRowsPass = CKV_WAVE / kPieces;
 #pragma unroll
-        for (int pass = 0; pass < 8; pass++) {
-            const int r = 4 * pass + (lane >> 4), piece = lane & 15;
+        for (int pass = 0; pass < 32 / kRowsPass; pass++) {
+            const int r = kRowsPass * pass + lane / kPieces, piece = lane % kPieces;
             const int rr = qt_i * kRows + wave * 32 + r;
             const int g_r = rr % p.G, m_r = rr / p.G;
             if (m_r < p.Q) {
@@ -852,7 +887,7 @@ __global__ void __launch_bounds__(512) fwd_pipe_kernel(FwdParams p) {
     } else if (row_ok) {
         T* orow = (T*)p.out + b * p.out_stride[0] + row_h * p.out_stride[1] + row_m * p.out_stride[2];
 #pragma unroll
-        for (int dt = 0; dt < 4; dt++) {
+        for (int dt = 0; dt < kDB; dt++) {
 #pragma unroll
             for (int v4 = 0; v4 < 4; v4++) {
                 const int d = 32 * dt + 8 * v4 + 4 * half;
@@ -870,13 +905,14 @@ __global__ void __launch_bounds__(512) fwd_pipe_kernel(FwdParams p) {
     }
 }
 
-// Merge of the forward kernel's shares: one row per 32 lanes (4 dims each), 8 rows per workgroup.
-template <typename T>
+// Merge of the forward kernel's shares: one row per kD / 4 lanes (4 dims each).
+template <typename T, int kD>
 __global__ void __launch_bounds__(256) fwd_combine_kernel(FwdParams p) {
     const int64_t rows = p.B * p.H * p.Q;
-    const int64_t row = (int64_t)blockIdx.x * 8 + threadIdx.x / 32;
+    constexpr int kLanes = kD / 4;
+    const int64_t row = (int64_t)blockIdx.x * (256 / kLanes) + threadIdx.x / kLanes;
     if (row >= rows) return;
-    const int d4 = threadIdx.x % 32;
+    const int d4 = threadIdx.x % kLanes;
     float M = -INFINITY;
     for (int s_ = 0; s_ < p.n_split; s_++) M = fmaxf(M, p.part_l2[s_ * rows + row]);
     float L = 0.f;
@@ -918,22 +954,29 @@ struct ColsumParams {
     int G;
     int new_mode;
     float scale_log2;
-    int nkb, first_chunk_blk, nbkv, xcd_aware, gsplit;  // block order and head split, see the kernel
+    int nkb, nbkv, xcd_aware, gsplit;  // block order and head split, see the kernel
+    const int* n_visible; // when the keys were staged in key order: the number of cached keys (null: Nc), and the
+    const int* key_order; // row each key came from
+    void* scores;         // (B, H, N) in the tensor dtype, at the row each key came from: takes the place of colsum
+    int64_t scores_stride[3];
     int wnew_uniform;     // every entry of w_new has the value wnew_value (beta rounds to one in the tensor dtype)
     float wnew_value;
 };
 
 constexpr int kQT2 = 128;                     // query rows per LDS tile of the column pass
 constexpr int kCsSub = kQT2 / 32;             // 32-row subtiles of a tile
-constexpr int kCsStage = kQT2 * 256 + 2 * kQT2 * 4;   // Q tile + its lse2 + its weights
+__host__ __device__ constexpr int cs_stage(int head_dim) { return kQT2 * 2 * head_dim + 2 * kQT2 * 4; }  // Q tile + its lse2 + its weights
 
 // One workgroup = one kv head x 256 keys (64 per wavefront, held in registers as the B operand of
 // S = Q K^T).  The (head, query-tile) sequence streams through a double-buffered LDS stage filled
 // by asynchronous copies; lane (col, half) owns key column `col` of each 32-key subtile, so the
 // weighted column sums never leave the lane.
-template <typename T>
+template <typename T, int kD>
 __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
     extern __shared__ __align__(16) unsigned char smem[];
+    constexpr int kKK = kD / 16, kRowBytes = 2 * kD, kCsStage = cs_stage(kD);
+    const int Nc = p.n_visible ? *p.n_visible : (int)p.Nc;
+    const int N = p.n_visible ? Nc + (int)p.Q : (int)p.N;   // keys somebody can see; those behind get a zero
     float* wnew_lds = reinterpret_cast<float*>(smem + 2 * kCsStage);
     const uint32_t smem_addr = lds_address(smem);
     const int tid = threadIdx.x, lane = tid & 63;
@@ -948,7 +991,7 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
     int bkv_i, kb_i, g_first;
     const int g_cnt = p.G / p.gsplit;
     {
-        const int nkb = p.nkb * p.gsplit, cb0 = p.first_chunk_blk * p.gsplit, heavy = nkb - cb0;
+        const int nkb = p.nkb * p.gsplit, cb0 = (Nc / 256) * p.gsplit, heavy = nkb - cb0;
         int id = blockIdx.x, nb = p.nbkv, first = 0, stride = 1;
         if (p.xcd_aware) {
             first = id & 7;
@@ -975,7 +1018,7 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
     const int64_t key_blk = (int64_t)kb_i * 256;          // first key of the workgroup
     const int64_t key_w = key_blk + wave * 64;            // first key of this wavefront
 
-    uint4 kreg[2][8];
+    uint4 kreg[2][kKK];
     const char* kbase = (const char*)p.kr + bkv * p.n_pad * kD * (int64_t)sizeof(T);
     bool live[2];
     int nrel[2];
@@ -983,22 +1026,22 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
     for (int ks = 0; ks < 2; ks++) {
         const int64_t n = key_w + 32 * ks + col;
 #pragma unroll
-        for (int kk = 0; kk < 8; kk++) {
+        for (int kk = 0; kk < kKK; kk++) {
             kreg[ks][kk] = n < p.n_pad ? *reinterpret_cast<const uint4*>(kbase + (n / kBN) * (int64_t)(kBN * kD * sizeof(T)) +
                                                                          k_image_off((int)(n % kBN), 2 * kk + half))
                                        : make_uint4(0, 0, 0, 0);
         }
-        live[ks] = n < p.N && ((p.tile_vis[n / kBN] >> (n % kBN)) & 1ull);
-        nrel[ks] = (int)(n - p.Nc);
+        live[ks] = n < N && ((p.tile_vis[n / kBN] >> (n % kBN)) & 1ull);
+        nrel[ks] = (int)(n - Nc);
     }
     // first query tile that can see any key of the workgroup
-    int m_first = (int)(key_blk - p.Nc);
+    int m_first = (int)(key_blk - Nc);
     if (m_first < 0) m_first = 0;
     m_first = m_first / kQT2 * kQT2;
-    const bool chunk_keys = key_blk + 255 >= p.Nc;  // some key of the workgroup belongs to the chunk
-    const int last_nrel = (int)(key_blk + 255 - p.Nc);
+    const bool chunk_keys = key_blk + 255 >= Nc;  // some key of the workgroup belongs to the chunk
+    const int last_nrel = (int)(key_blk + 255 - Nc);
     const bool new_chunk = chunk_keys && p.new_mode;
-    const bool pure_chunk = key_blk >= p.Nc;        // no cached key in the workgroup
+    const bool pure_chunk = key_blk >= Nc;        // no cached key in the workgroup
     // the weights of chunk keys by distance: a table in LDS, unless every entry is the same value (then the
     // launch reserves no LDS for it, and two workgroups fit a compute unit whatever the chunk length)
     if (new_chunk && !p.wnew_uniform) {
@@ -1008,19 +1051,19 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
     const int nmt = (Q - m_first + kQT2 - 1) / kQT2;  // query tiles per head
     const int n_steps = nmt * g_cnt;
 
-    // async copy assignments: the Q tile is kQT2 / 4 blocks of 1 KiB (a quarter per wavefront); wavefront 0
+    // async copy assignments: the Q tile is copied in blocks of 1 KiB (a quarter of them per wavefront); wavefront 0
     // also brings the tile's normalisers, wavefront 1 its weights (kQT2 / 4 lanes x 16 bytes each)
-    constexpr int kQBlocks = kQT2 / 16;   // per wavefront
+    constexpr int kQBlocks = kQT2 * kRowBytes / 4096;   // per wavefront
     uint32_t q_src[kQBlocks];
 #pragma unroll
     for (int j = 0; j < kQBlocks; j++) {
         const int pos = (wave * kQBlocks + j) * 64 + lane;
-        const int r = pos >> 4, c = (pos & 15) ^ (r & 15);
-        q_src[j] = r * 256 + c * 16;
+        const int r = pos / (kD / 8), c = (pos % (kD / 8)) ^ row_swizzle<kD>(r);
+        q_src[j] = r * kRowBytes + c * 16;
     }
-    int q_off[8];  // query row `col` of the tile (+32 rows = +8192 B)
+    int q_off[kKK];  // query row `col` of the tile
 #pragma unroll
-    for (int kk = 0; kk < 8; kk++) q_off[kk] = k_lds_off(col, 2 * kk + half);
+    for (int kk = 0; kk < kKK; kk++) q_off[kk] = k_lds_off<kD>(col, 2 * kk + half);
     const int64_t head_row0 = (b * p.H + kvh * p.G) * p.Q;
     // (head, query tile) of a step are tracked incrementally: integer division per step would
     // cost more scalar instructions than the step's matrix work leaves room for
@@ -1032,15 +1075,23 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
         for (int j = 0; j < kQBlocks; j++) async_copy16(qt, q_src[j], st + (wave * kQBlocks + j) * 1024);
         if (wave < 2 && lane < kQT2 / 4) {
             const char* src = wave ? (const char*)(p.w_ema + mt) : (const char*)(p.lse2 + row0);
-            async_copy16(src, lane * 16, st + kQT2 * 256 + wave * (kQT2 * 4));
+            async_copy16(src, lane * 16, st + kQT2 * kRowBytes + wave * (kQT2 * 4));
         }
     };
 
+    auto store = [&](int64_t h, int64_t n, float v) {
+        if (p.scores) {
+            T* dst = (T*)p.scores + b * p.scores_stride[0] + h * p.scores_stride[1];
+            dst[(p.key_order ? p.key_order[n] : n) * p.scores_stride[2]] = Elem<T>::from_float(v);
+        } else {
+            p.colsum[(b * p.H + h) * p.N + n] = v;
+        }
+    };
     float acc[2] = {0.f, 0.f};
     auto tile_step = [&](auto stage_tag, int g, int mt) {
         constexpr int ST = decltype(stage_tag)::value;
         const unsigned char* q_lds = smem + ST * kCsStage;
-        const float* lse_lds = reinterpret_cast<const float*>(q_lds + kQT2 * 256);
+        const float* lse_lds = reinterpret_cast<const float*>(q_lds + kQT2 * kRowBytes);
         const float* w_lds = lse_lds + kQT2;
         const bool tail = mt + kQT2 > Q;                       // rows past the chunk end
         const bool diag = chunk_keys && mt <= last_nrel;       // tile may cross the diagonal
@@ -1072,7 +1123,7 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
             f32x16 sq[2][2];  // [c & 1][ks]
             sq[0][0] = sq[0][1] = row_init(0);
 #pragma unroll
-            for (int kk = 0; kk < 8; kk++) {
+            for (int kk = 0; kk < kKK; kk++) {
                 const uint4 a = *reinterpret_cast<const uint4*>(q_lds + q_off[kk]);
                 sq[0][0] = Mma<T>::mma(a, kreg[0][kk], sq[0][0]);
                 sq[0][1] = Mma<T>::mma(a, kreg[1][kk], sq[0][1]);
@@ -1080,39 +1131,40 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
 #pragma unroll
             for (int c = 1; c < kCsSub; c++) {
                 sq[c & 1][0] = sq[c & 1][1] = row_init(c);
-                uint4 a1[8];
+                uint4 a1[kKK];
 #pragma unroll
-                for (int kk = 0; kk < 8; kk++) a1[kk] = *reinterpret_cast<const uint4*>(q_lds + q_off[kk] + c * 8192);
+                for (int kk = 0; kk < kKK; kk++) a1[kk] = *reinterpret_cast<const uint4*>(q_lds + q_off[kk] + c * (32 * kRowBytes));
                 float ws[16];
                 load_weights(c - 1, ws);
                 __builtin_amdgcn_sched_barrier(0);
                 // an exponential is consumed one slot after it was issued, so no wavefront waits for the
                 // transcendental unit
-                float pe_prev[2] = {0.f, 0.f};
+                constexpr int kPer = 32 / (2 * kKK);   // exponentials per matrix instruction
+                float pe_prev[kPer];
 #pragma unroll
-                for (int slot = 0; slot < 16; slot++) {
+                for (int slot = 0; slot < 2 * kKK; slot++) {
                     const int kk = slot >> 1, ks = slot & 1;
                     sq[c & 1][ks] = Mma<T>::mma(a1[kk], kreg[ks][kk], sq[c & 1][ks]);
-                    float pe[2];
+                    float pe[kPer];
 #pragma unroll
-                    for (int r = 0; r < 2; r++) {
-                        const int j = 2 * slot + r, ksv = j >> 4, v = j & 15;
+                    for (int r = 0; r < kPer; r++) {
+                        const int j = kPer * slot + r, ksv = j >> 4, v = j & 15;
                         pe[r] = __builtin_amdgcn_exp2f(sq[(c - 1) & 1][ksv][v]);
                     }
                     if (slot > 0) {
 #pragma unroll
-                        for (int r = 0; r < 2; r++) {
-                            const int j = 2 * (slot - 1) + r, ksv = j >> 4, v = j & 15;
+                        for (int r = 0; r < kPer; r++) {
+                            const int j = kPer * (slot - 1) + r, ksv = j >> 4, v = j & 15;
                             acc[ksv] = fmaf(ws[v], pe_prev[r], acc[ksv]);
                         }
                     }
-                    pe_prev[0] = pe[0];
-                    pe_prev[1] = pe[1];
+#pragma unroll
+                    for (int r = 0; r < kPer; r++) pe_prev[r] = pe[r];
                     __builtin_amdgcn_sched_barrier(0);
                 }
 #pragma unroll
-                for (int r = 0; r < 2; r++) {
-                    const int j = 30 + r, ksv = j >> 4, v = j & 15;
+                for (int r = 0; r < kPer; r++) {
+                    const int j = 32 - kPer + r, ksv = j >> 4, v = j & 15;
                     acc[ksv] = fmaf(ws[v], pe_prev[r], acc[ksv]);
                 }
             }
@@ -1144,8 +1196,8 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
                 f32x16 sacc[2];
                 sacc[0] = sacc[1] = row_init(c);
 #pragma unroll
-                for (int kk = 0; kk < 8; kk++) {
-                    const uint4 a = *reinterpret_cast<const uint4*>(q_lds + q_off[kk] + c * 8192);
+                for (int kk = 0; kk < kKK; kk++) {
+                    const uint4 a = *reinterpret_cast<const uint4*>(q_lds + q_off[kk] + c * (32 * kRowBytes));
                     sacc[0] = Mma<T>::mma(a, kreg[0][kk], sacc[0]);
                     sacc[1] = Mma<T>::mma(a, kreg[1][kk], sacc[1]);
                 }
@@ -1214,7 +1266,7 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
             for (int ks = 0; ks < 2; ks++) {
                 const float tot = acc[ks] + __shfl_xor(acc[ks], 32);
                 const int64_t n = key_w + 32 * ks + col;
-                if (half == 0 && n < p.N) p.colsum[(b * p.H + h) * p.N + n] = live[ks] ? tot : 0.f;
+                if (half == 0 && n < p.N) store(h, n, live[ks] ? tot : 0.f);
                 acc[ks] = 0.f;
             }
         }
@@ -1248,17 +1300,17 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
             mt_cur = mt_n2;
         }
     }
-    if (n_steps == 0) {  // no query can see these keys (only possible for padding blocks)
+    if (n_steps <= 0) {  // no query can see these keys (padding blocks, and hidden keys sorted behind the visible ones)
         for (int g = g_first; g < g_first + g_cnt; g++)
 #pragma unroll
             for (int ks = 0; ks < 2; ks++) {
                 const int64_t n = key_w + 32 * ks + col;
-                if (half == 0 && n < p.N) p.colsum[(b * p.H + kvh * p.G + g) * p.N + n] = 0.f;
+                if (half == 0 && n < p.N) store(kvh * p.G + g, n, 0.f);
             }
     }
 }
 
-template <typename T>
+template <typename T, int kD>
 int run_mfma(const MfmaProblem& mp, hipStream_t stream) {
     const int64_t n = mp.n, n_pad = mp.n_pad;
     const float scale_log2 = mp.scale * 1.4426950408889634f;
@@ -1285,6 +1337,7 @@ int run_mfma(const MfmaProblem& mp, hipStream_t stream) {
         sp.vt = mp.vt;
         sp.tile_vis = mp.tile_vis;
         sp.B = mp.B; sp.KVH = mp.KVH; sp.n = n; sp.n_pad = n_pad;
+        sp.key_order = mp.key_order; sp.n_visible = mp.n_visible; sp.n_chunk = mp.Q;
         const int64_t nbh = mp.B * mp.KVH;
         // shared positions: a block walks several (b, kvh) units with one set of cos/sin, the next unit's rows
         // always on their way
@@ -1319,7 +1372,7 @@ int run_mfma(const MfmaProblem& mp, hipStream_t stream) {
             g.q_bx = (int)bx; g.q_by = (int)by; g.k_bx = (int)(n_pad / kBN); g.k_by = (int)splits;
             const int64_t blocks = bx * by + (n_pad / kBN) * splits;
             if (blocks > 0x7fffffff) return CKV_ERR_UNSUPPORTED;
-            hipLaunchKernelGGL(stage_kernel<T>, dim3((unsigned)blocks), dim3(256), 0, stream, sp, sq, g);
+            hipLaunchKernelGGL((stage_kernel<T, kD>), dim3((unsigned)blocks), dim3(256), 0, stream, sp, sq, g);
         }
         CKV_HIP_TRY(hipGetLastError());
     }
@@ -1339,29 +1392,34 @@ int run_mfma(const MfmaProblem& mp, hipStream_t stream) {
         fp.n_split = mfma_fwd_splits(mp.B, mp.H, mp.KVH, mp.Q, n, cus);
         fp.part_o = mp.part_o;
         fp.part_l2 = mp.part_l2;
+        fp.n_visible = mp.n_visible;
         if (fp.n_split > 1 && (!fp.part_o || !fp.part_l2)) return CKV_ERR_WORKSPACE;
         const dim3 grid((unsigned)(fp.n_qt * fp.n_split), (unsigned)(mp.B * mp.KVH));
-        const int lds = pipe_lds_bytes(n_pad);
-        if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(fwd_pipe_kernel<T>), lds)) return rc;
+        const int lds = (int)pipe_lds_bytes(n_pad, kD);
+        if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(fwd_pipe_kernel<T, kD>), lds)) return rc;
         fp.xcd_aware = grid.y % 8 == 0;
         hipEvent_t ev0, ev1;
         prof_kernel_events(CKV_STAGE_FWD, &ev0, &ev1);
         const dim3 launch_grid = fp.xcd_aware ? dim3(grid.x * grid.y) : grid;
-        if (ev0) hipExtLaunchKernelGGL(fwd_pipe_kernel<T>, launch_grid, dim3(512), (uint32_t)lds, stream, ev0, ev1, 0u, fp);
-        else hipLaunchKernelGGL(fwd_pipe_kernel<T>, launch_grid, dim3(512), lds, stream, fp);
+        if (ev0) hipExtLaunchKernelGGL((fwd_pipe_kernel<T, kD>), launch_grid, dim3(512), (uint32_t)lds, stream, ev0, ev1, 0u, fp);
+        else hipLaunchKernelGGL((fwd_pipe_kernel<T, kD>), launch_grid, dim3(512), lds, stream, fp);
         CKV_HIP_TRY(hipGetLastError());
         if (fp.n_split > 1) {
             const int64_t rows = mp.B * mp.H * mp.Q;
-            hipLaunchKernelGGL(fwd_combine_kernel<T>, dim3((unsigned)((rows + 7) / 8)), dim3(256), 0, stream, fp);
+            constexpr int per = 256 / (kD / 4);
+            hipLaunchKernelGGL((fwd_combine_kernel<T, kD>), dim3((unsigned)((rows + per - 1) / per)), dim3(256), 0, stream, fp);
             CKV_HIP_TRY(hipGetLastError());
         }
     }
-    if (mp.colsum) {
+    if (mp.colsum || mp.scores) {
         StageScope sc(CKV_STAGE_SCORES, stream);
         ColsumParams cp;
         cp.qr = mp.qr; cp.kr = mp.kr; cp.tile_vis = mp.tile_vis; cp.lse2 = mp.lse2;
         cp.w_ema = mp.w_ema; cp.w_new = mp.w_new; cp.colsum = mp.colsum;
         cp.B = mp.B; cp.H = mp.H; cp.KVH = mp.KVH; cp.Q = mp.Q; cp.N = n; cp.Nc = n - mp.Q; cp.n_pad = n_pad;
+        cp.n_visible = mp.n_visible; cp.key_order = mp.key_order;
+        cp.scores = mp.scores;
+        for (int j = 0; j < 3; j++) cp.scores_stride[j] = mp.scores_stride[j];
         cp.G = G;
         cp.new_mode = mp.new_mode;
         {
@@ -1382,16 +1440,15 @@ int run_mfma(const MfmaProblem& mp, hipStream_t stream) {
         }
         cp.scale_log2 = 1.f;  // already on the staged queries
         cp.nkb = (int)((n + 255) / 256);
-        cp.first_chunk_blk = (int)(cp.Nc / 256);
         cp.nbkv = (int)(mp.B * mp.KVH);
         cp.xcd_aware = cp.nbkv % 8 == 0;
         // two heads per workgroup where the group allows it: the keys a workgroup holds in registers and its
         // pipeline start serve twice the work, and the units stay small enough for an even last round
         cp.gsplit = (G % 2 == 0 && G >= 4) ? G / 2 : G;
         const dim3 grid((unsigned)(cp.nkb * cp.nbkv * cp.gsplit));
-        const int lds = 2 * kCsStage + (cp.wnew_uniform ? 0 : (int)mp.Q * 4);
-        if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(colsum_mfma_kernel<T>), lds)) return rc;
-        hipLaunchKernelGGL(colsum_mfma_kernel<T>, grid, dim3(256), lds, stream, cp);
+        const int lds = 2 * cs_stage(kD) + (cp.wnew_uniform ? 0 : (int)mp.Q * 4);
+        if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(colsum_mfma_kernel<T, kD>), lds)) return rc;
+        hipLaunchKernelGGL((colsum_mfma_kernel<T, kD>), grid, dim3(256), lds, stream, cp);
         CKV_HIP_TRY(hipGetLastError());
     }
     return CKV_OK;
@@ -1401,7 +1458,7 @@ int run_mfma(const MfmaProblem& mp, hipStream_t stream) {
 
 bool mfma_supported(int dtype, int64_t D, int64_t H, int64_t KVH, int64_t Q) {
     if (dtype != CKV_BF16 && dtype != CKV_F16) return false;
-    if (D != kD) return false;
+    if (D != 64 && D != 128) return false;
     if (Q > 16384) return false;  // the column pass keeps a Q-long weight table in LDS beside its two stages
     const int64_t G = H / KVH;
     return G >= 1 && G <= kRows / 32;  // at least 32 positions per workgroup
@@ -1439,12 +1496,12 @@ int mfma_fwd_splits_for_workspace(int64_t B, int64_t H, int64_t KVH, int64_t Q, 
 }
 
 // the forward kernel keeps per-tile bookkeeping of all N keys in LDS
-bool mfma_fits(int64_t n) { return pipe_lds_bytes(mfma_n_pad(n)) <= kLdsLimit; }
+bool mfma_fits(int64_t n, int64_t D) { return pipe_lds_bytes(mfma_n_pad(n), (int)D) <= kLdsLimit; }
 
 
 int launch_mfma(const MfmaProblem& mp, hipStream_t stream) {
-    if (mp.dtype == CKV_BF16) return run_mfma<__hip_bfloat16>(mp, stream);
-    if (mp.dtype == CKV_F16) return run_mfma<__half>(mp, stream);
+    if (mp.dtype == CKV_BF16) return mp.D == 64 ? run_mfma<__hip_bfloat16, 64>(mp, stream) : run_mfma<__hip_bfloat16, 128>(mp, stream);
+    if (mp.dtype == CKV_F16) return mp.D == 64 ? run_mfma<__half, 64>(mp, stream) : run_mfma<__half, 128>(mp, stream);
     return CKV_ERR_DTYPE;
 }
 

@@ -85,7 +85,7 @@ def _backward(q, k, v, o, lse, mask, do, sm_scale):
     a.B, a.H, a.n_ctx, a.n_kv, a.D = B, H, n_ctx, n_kv, D
     a.scale = float(sm_scale)
     a.dtype = _abi.dtype_code(q.dtype)
-    need = lib.ckv_dense_bwd_workspace_bytes(B, H, n_ctx)
+    need = lib.ckv_dense_bwd_workspace_bytes(B, H, n_ctx) + lib.ckv_dense_bwd_key_order_bytes(n_kv)
     with torch.cuda.device(q.device):
         stream = torch.cuda.current_stream(q.device).cuda_stream
         ws = workspace(q.device, need, stream)

@@ -620,3 +620,44 @@ def test_filled_slots_hint_changes_nothing(dtype, H, KVH):
             a, b = getattr(with_hint, name)[0], getattr(without, name)[0]
             assert torch.equal(a.view(torch.uint8) if a.dtype.is_floating_point else a,
                                b.view(torch.uint8) if b.dtype.is_floating_point else b), f"step {step}: {name}"
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("Z,H,N_CTX,N_CACHED", [
+    (1, 2, 2, 0), (1, 3, 33, 1), (2, 1, 63, 65), (1, 2, 256, 64), (1, 8, 129, 1023), (1, 1, 257, 20000),
+])
+@pytest.mark.parametrize("masking", ["random", "none", "all", "tail", "last"])
+def test_dense_operator_with_sorted_keys(D, Z, H, N_CTX, N_CACHED, masking):
+    """The 16-bit dense operator sorts the masked keys out before it works (stretches of 16384 keys, 64-key tiles):
+    no cached key at all, none / all masked, a masked end, only the last key visible; sizes around a tile; masked rows
+    hold infinities and NaN, which must reach nothing.  Output, scores and gradients against the float32 formula on
+    inputs of the tensor dtype, with the bounds of the tests above."""
+    from cascading_kv_cache_amd.flash_attention import attention
+
+    dtype = torch.float16 if D == 64 else torch.bfloat16
+    torch.manual_seed(23)
+    N_KV = N_CACHED + N_CTX
+    q, k, v = (torch.empty((Z, n, H, D), device="cuda").normal_(std=0.5).to(dtype).transpose(1, 2) for n in (N_CTX, N_KV, N_KV))
+    at = torch.arange(N_CACHED, device="cuda")
+    mask = {"random": torch.rand(N_CACHED, device="cuda") > 0.5, "none": at < 0, "all": at >= 0,
+            "tail": at >= N_CACHED * 3 // 4, "last": at < N_CACHED - 1}[masking]
+    dout = torch.randn(Z, H, N_CTX, D, device="cuda").to(dtype)
+    rq, rk, rv = (t.float().requires_grad_() for t in (q, k, v))
+    ref, p = dense_reference(rq, rk, rv, mask, D ** -0.5)
+    ref.backward(dout.float())
+    hidden = torch.cat((mask, torch.zeros(N_CTX, dtype=torch.bool, device="cuda")))
+    k[:, :, hidden], v[:, :, hidden] = float("inf"), float("nan")
+    for t in (q, k, v):
+        t.requires_grad_()
+    out, scores = attention(q, k, v, True, D ** -0.5, mask, 0.9999)
+    got = torch.autograd.grad(out, (q, k, v), dout)
+    assert (out.float() - ref).abs().max().item() <= 1e-2
+    w = (1 - 0.9999) * 0.9999 ** torch.arange(N_CTX - 1, -1, -1, device="cuda", dtype=torch.float64)
+    assert_scores_close(scores, (p.detach().double() * w[None, None, :, None]).sum(dim=2), dtype, "dense scores")
+    assert scores[:, :, hidden].abs().sum().item() == 0
+    # P and dS enter the products rounded to the dtype (2^-9 / 2^-12 relative each), a gradient sums up to N_CTX of them
+    rel = 2.0 ** -6 if dtype == torch.bfloat16 else 2.0 ** -9
+    for name, g, want in zip(("dq", "dk", "dv"), got, (rq.grad, rk.grad, rv.grad)):
+        err = (g.float() - want).norm().item() / want.norm().item()
+        assert err <= rel, f"{name}: relative error {err:.3e}"
+    assert got[1][:, :, hidden].abs().sum().item() == 0 and got[2][:, :, hidden].abs().sum().item() == 0
