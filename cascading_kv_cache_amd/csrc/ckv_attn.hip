@@ -41,7 +41,8 @@ AttnWorkspace carve_attn(void* base, int64_t B, int64_t H, int64_t KVH, int64_t 
     w.w_ema = (float*)c.take((Q + kColSlack) * 4);
     w.w_new = (float*)c.take(Q * 4);
     // shares of the forward kernel when few query rows would leave the chip idle
-    const int splits = mfma_supported(dtype, D, H, KVH, Q) && Q > 1 ? mfma_fwd_splits_for_workspace(B, H, KVH, Q, N) : 1;
+    int splits = mfma_supported(dtype, D, H, KVH, Q) && Q > 1 ? mfma_fwd_splits_for_workspace(B, H, KVH, Q, N) : 1;
+    if (dtype == CKV_F32 && (D == 64 || D == 128)) splits = f32_mfma_splits(B, H, KVH, Q, N, mfma_device_cus());
     w.part_o = splits > 1 ? (float*)c.take(splits * B * H * Q * D * 4) : nullptr;
     w.part_l2 = splits > 1 ? (float*)c.take(splits * B * H * Q * 4) : nullptr;
     w.bytes = c.off;
@@ -182,7 +183,7 @@ extern "C" int ckv_attn(const ckv_attn_args* args, void* stream_) {
         cp.B = a.B; cp.H = a.H; cp.KVH = a.KVH; cp.Q = a.Q; cp.N = N; cp.D = a.D;
         cp.scale = 1.f;  // the staged queries and keys each carry sqrt(scale), rounded in as the eager path does
         cp.dtype = a.dtype;
-        rc = launch_core_generic(cp, stream);
+        rc = f32_mfma_supported(cp) ? launch_f32_mfma(cp, w.part_o, w.part_l2, stream) : launch_core_generic(cp, stream);
         if (rc) return rc;
     }
     if (a.lse) {
@@ -306,7 +307,7 @@ extern "C" int ckv_attn_dense(const ckv_dense_args* args, void* stream_) {
     cp.B = a.B; cp.H = a.H; cp.KVH = a.H; cp.Q = a.n_ctx; cp.N = a.n_kv; cp.D = a.D;
     cp.scale = a.scale;
     cp.dtype = a.dtype;
-    rc = launch_core_generic(cp, stream);
+    rc = f32_mfma_supported(cp) ? launch_f32_mfma(cp, nullptr, nullptr, stream) : launch_core_generic(cp, stream);
     if (rc) return rc;
     if (a.scores) {
         rc = launch_cast_scores(colsum, a.scores, a.scores_stride, a.B, a.H, a.n_kv, a.dtype, stream);

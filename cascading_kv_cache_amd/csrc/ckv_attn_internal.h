@@ -34,6 +34,12 @@ struct CoreProblem {
 // and the fallback for shapes the MFMA kernels do not cover.
 int launch_core_generic(const CoreProblem& p, hipStream_t stream);
 
+// The same in float32 on the matrix cores: head_dim 64 and 128, rows of 16-byte pieces, lse wanted.  part_o / part_l:
+// f32_mfma_splits shares of (B*H*Q, D) / (B*H*Q) floats, or null (then the keys of a row tile are not shared out).
+bool f32_mfma_supported(const CoreProblem& p);
+int f32_mfma_splits(int64_t B, int64_t H, int64_t KVH, int64_t Q, int64_t n, int cus);
+int launch_f32_mfma(const CoreProblem& p, float* part_o, float* part_l, hipStream_t stream);
+
 // weights of the score sums (cascade_attention.py:270-282, 315-317), rounded like the eager path
 // w_ema gets 64 trailing zeros (slack read by the MFMA column pass)
 int launch_weights(float* w_ema, float* w_new, int64_t Q, double beta, int dtype, hipStream_t stream);

@@ -661,3 +661,14 @@ def test_dense_operator_with_sorted_keys(D, Z, H, N_CTX, N_CACHED, masking):
         err = (g.float() - want).norm().item() / want.norm().item()
         assert err <= rel, f"{name}: relative error {err:.3e}"
     assert got[1][:, :, hidden].abs().sum().item() == 0 and got[2][:, :, hidden].abs().sum().item() == 0
+
+
+@pytest.mark.parametrize("D,H,KVH,W,C,steps", [
+    (128, 8, 2, 32, 4, [5, 33, 130, 2, 31]),      # fewer key blocks than wavefronts, ragged rows, a cache that is filling
+    (64, 7, 1, 257, 2, [40, 700, 3, 257]),         # seven heads per kv head, key blocks shared out over workgroups
+    (128, 3, 3, 64, 1, [64, 65, 2]),               # one head per kv head
+])
+def test_float32_on_the_matrix_cores(D, H, KVH, W, C, steps):
+    """float32 chunks of head sizes 64 and 128 take the float32 matrix instructions: 32-row and 32-key blocks, shared
+    out over eight wavefronts and, with few rows, over workgroups.  Against the oracle with the float32 tolerances."""
+    run_teacher_forced(B=2, H=H, KVH=KVH, D=D, NS=4, W=W, C=C, Q=0, chunks=0, dtype=torch.float32, seed=41, steps=steps)
