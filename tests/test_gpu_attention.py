@@ -664,11 +664,35 @@ def test_dense_operator_with_sorted_keys(D, Z, H, N_CTX, N_CACHED, masking):
 
 
 @pytest.mark.parametrize("D,H,KVH,W,C,steps", [
-    (128, 8, 2, 32, 4, [5, 33, 130, 2, 31]),      # fewer key blocks than wavefronts, ragged rows, a cache that is filling
-    (64, 7, 1, 257, 2, [40, 700, 3, 257]),         # seven heads per kv head, key blocks shared out over workgroups
-    (128, 3, 3, 64, 1, [64, 65, 2]),               # one head per kv head
+    # (the first chunk is the longest: the reference's position ids of later chunks are a prefix of the first one's)
+    (128, 8, 2, 32, 4, [130, 5, 33, 2, 31]),      # fewer key blocks than wavefronts, ragged rows, a cache that is filling
+    (64, 7, 1, 257, 2, [700, 40, 3, 257]),         # seven heads per kv head, key blocks shared out over workgroups
+    (128, 3, 3, 64, 1, [65, 64, 2]),               # one head per kv head
 ])
 def test_float32_on_the_matrix_cores(D, H, KVH, W, C, steps):
     """float32 chunks of head sizes 64 and 128 take the float32 matrix instructions: 32-row and 32-key blocks, shared
     out over eight wavefronts and, with few rows, over workgroups.  Against the oracle with the float32 tolerances."""
     run_teacher_forced(B=2, H=H, KVH=KVH, D=D, NS=4, W=W, C=C, Q=0, chunks=0, dtype=torch.float32, seed=41, steps=steps)
+
+
+@pytest.mark.parametrize("H,KVH,dtype", [(8, 2, torch.bfloat16), (3, 1, torch.float16), (7, 1, torch.bfloat16)])
+def test_score_sums_of_ragged_chunks(H, KVH, dtype):
+    """The score kernel takes 128 query rows at a time in subtiles of 32: lengths around both, over a cache that fills
+    (whole blocks of 256 hidden keys) and then evicts.  Against the oracle with the stream tests' bounds."""
+    run_teacher_forced(B=1, H=H, KVH=KVH, D=128, NS=4, W=128, C=8, Q=0, chunks=0, dtype=dtype, seed=43, std=0.7,
+                       steps=[300, 129, 127, 128, 2, 97, 33, 289, 31])
+
+
+def test_score_sums_of_a_ragged_chunk_keep_to_their_head():
+    """The last tile of a head is topped up with rows that are not its own; what the next head's rows hold reaches nothing."""
+    from cascading_kv_cache_amd.flash_attention import attention
+
+    torch.manual_seed(5)
+    q = torch.randn(1, 2, 77, 128, device="cuda", dtype=torch.bfloat16)
+    k = torch.randn(1, 2, 400, 128, device="cuda", dtype=torch.bfloat16)
+    mask = torch.zeros(323, dtype=torch.bool, device="cuda")
+    _, want = attention(q, k, k, True, 0.1, mask, 0.9999)
+    q[:, 1] = float("nan")
+    _, got = attention(q, k, k, True, 0.1, mask, 0.9999)
+    assert torch.equal(got[:, 0].view(torch.int16), want[:, 0].view(torch.int16))
+    assert torch.isfinite(got[:, 0].float()).all()
