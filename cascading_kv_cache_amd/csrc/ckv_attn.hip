@@ -139,6 +139,10 @@ extern "C" int ckv_attn(const ckv_attn_args* args, void* stream_) {
         mp.seg[2] = MfmaSegment{a.k_new, a.v_new,
                                 {a.kv_new_stride[0], a.kv_new_stride[1], a.kv_new_stride[2], a.kv_new_stride[3]},
                                 a.q_pos, {0, 0}, 0, nullptr, a.Q};
+        if (a.filled_slots > 0 && a.filled_slots < a.S) {
+            mp.empty_from = a.num_sink + a.filled_slots;
+            mp.empty_to = a.num_sink + a.S;
+        }
         mp.q = a.q;
         for (int i = 0; i < 4; i++) { mp.q_stride[i] = a.q_stride[i]; mp.out_stride[i] = a.out_stride[i]; }
         mp.q_pos = a.q_pos;

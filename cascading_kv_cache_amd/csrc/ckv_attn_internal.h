@@ -167,6 +167,7 @@ struct MfmaProblem {
     double beta;           // the EMA factor the weights were built from
     int new_mode;
     int64_t B, H, KVH, Q, D, n, n_pad;
+    int64_t empty_from = 0, empty_to = 0;  // keys whose slots cannot hold a token yet
     float scale;
     float key_scale;       // keys with position ids are multiplied by this after rotation and rounded again, the
                            // queries carry scale / key_scale: sqrt(scale) for the cascade path, which follows the

@@ -115,6 +115,7 @@ struct StageParams {
     const int* key_order;
     const int* n_visible;
     int64_t n_chunk;
+    int64_t empty_from, empty_to;  // keys no query can see because their slots are still empty (none: both 0)
 };
 
 __device__ inline int find_segment(const StageParams& p, int64_t n, int64_t& local) {
@@ -164,6 +165,14 @@ __device__ inline void stage_keys_block(const StageParams& p, int tile_i, int sp
         sidx = find_segment(p, n, local);
     }
 
+    // A tile of slots that cannot hold a token yet is read by nobody: the forward kernel leaves it out, the score kernel
+    // zeroes its sums.  A cache that is still filling is mostly such tiles (1000 of 16384 slots, 488-token chunk: the
+    // launch takes 31 us instead of 50).  The bound comes from the host's counter: looking at the mask first costs a
+    // full cache 4 us of 43.
+    if (tile * kBN >= p.empty_from && (tile + 1) * kBN <= p.empty_to) {
+        if (split_i == 0 && tid == 0) p.tile_vis[tile] = 0ull;
+        return;
+    }
     if (split_i == 0 && tid < kBN) {  // visibility word of this tile
         const int64_t nn = tile * kBN + tid;
         bool vis = nn < n_all;
@@ -1015,6 +1024,7 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
     const int64_t bkv = bkv_i;
     const int64_t b = bkv / p.KVH, kvh = bkv % p.KVH;
     const int Q = (int)p.Q;
+    static_assert(4 * kBN == 256, "a workgroup's keys are four visibility words");
     const int64_t key_blk = (int64_t)kb_i * 256;          // first key of the workgroup
     const int64_t key_w = key_blk + wave * 64;            // first key of this wavefront
 
@@ -1049,7 +1059,11 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
     }
     auto wnew_at = [&](int i) -> float { return p.wnew_uniform ? p.wnew_value : wnew_lds[i]; };
     const int nmt = (Q - m_first + kQT2 - 1) / kQT2;  // query tiles per head
-    const int n_steps = nmt * g_cnt;
+    // A block without a single visible key (the empty part of a cache that is still filling) has nothing but zeros to
+    // write: with 1000 of 16384 slots filled and a 488-token chunk that is 63 of 67 blocks.
+    const unsigned long long* vis = p.tile_vis + key_blk / kBN;
+    const bool hidden = p.n_visible ? key_blk >= N : (vis[0] | vis[1] | vis[2] | vis[3]) == 0ull;
+    const int n_steps = hidden ? 0 : nmt * g_cnt;
 
     // async copy assignments: the Q tile is copied in blocks of 1 KiB (a quarter of them per wavefront); wavefront 0
     // also brings the tile's normalisers, wavefront 1 its weights (kQT2 / 4 lanes x 16 bytes each)
@@ -1071,8 +1085,19 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
         const int64_t row0 = head_row0 + (int64_t)g * p.Q + mt;
         const char* qt = (const char*)p.qr + row0 * (kD * (int64_t)sizeof(T));
         const uint32_t st = smem_addr + stage * kCsStage;
+        if (mt + kQT2 > Q) {  // rows past the chunk end repeat its last row
+            const uint32_t last = (uint32_t)(Q - 1 - mt) * kRowBytes;
 #pragma unroll
-        for (int j = 0; j < kQBlocks; j++) async_copy16(qt, q_src[j], st + (wave * kQBlocks + j) * 1024);
+            for (int j = 0; j < kQBlocks; j++) {
+                uint32_t src = q_src[j];
+                asm("" : "+v"(src));   // worked out here, not kept in registers for the whole kernel
+                const uint32_t piece = src % kRowBytes, row = src - piece;
+                async_copy16(qt, (row < last ? row : last) + piece, st + (wave * kQBlocks + j) * 1024);
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < kQBlocks; j++) async_copy16(qt, q_src[j], st + (wave * kQBlocks + j) * 1024);
+        }
         if (wave < 2 && lane < kQT2 / 4) {
             const char* src = wave ? (const char*)(p.w_ema + mt) : (const char*)(p.lse2 + row0);
             async_copy16(src, lane * 16, st + kQT2 * kRowBytes + wave * (kQT2 * 4));
@@ -1093,8 +1118,6 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
         const unsigned char* q_lds = smem + ST * kCsStage;
         const float* lse_lds = reinterpret_cast<const float*>(q_lds + kQT2 * kRowBytes);
         const float* w_lds = lse_lds + kQT2;
-        const bool tail = mt + kQT2 > Q;                       // rows past the chunk end
-        const bool diag = chunk_keys && mt <= last_nrel;       // tile may cross the diagonal
         // Accumulators start from minus the row normaliser, so the matrix pipe hands back log2 P (the
         // softmax scale is already on the staged queries).  Element (c, v) of a 32-row subtile c:
         // query row mt + 32c + 8(v/4) + 4half + v%4, key column of this lane.
@@ -1117,7 +1140,9 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
                 ws[4 * v4] = w4.x; ws[4 * v4 + 1] = w4.y; ws[4 * v4 + 2] = w4.z; ws[4 * v4 + 3] = w4.w;
             }
         };
-        if (!tail && !diag && !new_chunk) {
+        // Cached keys, or chunk keys with the row's weight (dense operator) that every row of the tile sees.  The last
+        // tile of a head comes here too: with 509 rows it is one tile in four.
+        if (!new_chunk && !(chunk_keys && mt <= last_nrel)) {
             // The common case, written in issue order: the logits of subtile c go through the matrix
             // pipe while the vector ALU turns subtile c-1 into weighted probabilities.
             f32x16 sq[2][2];  // [c & 1][ks]
@@ -1182,7 +1207,6 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
             }
         } else {
             // special cases, one 32-row subtile at a time
-            const bool fast_new = !tail && !diag;   // new_chunk holds: every row is later than every key of the block
             bool chunk_lane[2];
 #pragma unroll
             for (int ks = 0; ks < 2; ks++) chunk_lane[ks] = nrel[ks] >= 0;
@@ -1193,6 +1217,12 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
             };
 #pragma unroll 1
             for (int c = 0; c < kCsSub; c++) {
+                const int row0 = mt + 32 * c;
+                const int nrel_w = (int)(key_w - Nc);   // this wavefront's first key among the chunk keys (negative: cached)
+                if (row0 >= Q) break;
+                if (row0 + 31 < nrel_w) continue;       // before every key of the wavefront
+                const bool plain = row0 + 31 < Q && row0 >= nrel_w + 63;   // every row sees every key of the wavefront
+                const bool fast_new = plain && new_chunk;
                 f32x16 sacc[2];
                 sacc[0] = sacc[1] = row_init(c);
 #pragma unroll
@@ -1272,6 +1302,16 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
         }
     };
 
+    // Called by every wavefront once its copies of a step have landed, before the barrier that publishes them.  Rows past
+    // the chunk end are copies of its last row, whose normaliser is somebody else's: starting from this value their
+    // probability is zero (if the last row is not finite it has spoiled the sums already).  In LDS and not at the
+    // accumulators: selects there cost 41 spilled registers, and the whole kernel a quarter of its speed.
+    auto hide_rows = [&](int mt, int stage) {
+        if (mt + kQT2 <= Q || wave != 0) return;
+        float* lse_lds = reinterpret_cast<float*>(smem + stage * kCsStage + kQT2 * kRowBytes);
+        for (int r = lane; r < kQT2; r += 64)
+            if (mt + r >= Q) lse_lds[r] = -3e38f;
+    };
     // two steps per trip: while stage s is consumed the copy of the next step fills stage s^1
     int g_cur = g_first, mt_cur = m_first;    // step being consumed
     auto advance = [&](int& g, int& mt) {
@@ -1286,6 +1326,7 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
         int g_n = g_cur, mt_n = mt_cur;
         advance(g_n, mt_n);
         __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+        hide_rows(mt_cur, 0);
         __syncthreads();
         if (step + 1 < n_steps) issue(g_n, mt_n, 1);
         tile_step(std::integral_constant<int, 0>{}, g_cur, mt_cur);
@@ -1293,6 +1334,7 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
             int g_n2 = g_n, mt_n2 = mt_n;
             advance(g_n2, mt_n2);
             __builtin_amdgcn_s_waitcnt(0x0F70);
+            hide_rows(mt_n, 1);
             __syncthreads();
             if (step + 2 < n_steps) issue(g_n2, mt_n2, 0);
             tile_step(std::integral_constant<int, 1>{}, g_n, mt_n);
@@ -1336,6 +1378,7 @@ int run_mfma(const MfmaProblem& mp, hipStream_t stream) {
         sp.kr = mp.kr;
         sp.vt = mp.vt;
         sp.tile_vis = mp.tile_vis;
+        sp.empty_from = mp.empty_from; sp.empty_to = mp.empty_to;
         sp.B = mp.B; sp.KVH = mp.KVH; sp.n = n; sp.n_pad = n_pad;
         sp.key_order = mp.key_order; sp.n_visible = mp.n_visible; sp.n_chunk = mp.Q;
         const int64_t nbh = mp.B * mp.KVH;
@@ -1442,9 +1485,12 @@ int run_mfma(const MfmaProblem& mp, hipStream_t stream) {
         cp.nkb = (int)((n + 255) / 256);
         cp.nbkv = (int)(mp.B * mp.KVH);
         cp.xcd_aware = cp.nbkv % 8 == 0;
-        // two heads per workgroup where the group allows it: the keys a workgroup holds in registers and its
-        // pipeline start serve twice the work, and the units stay small enough for an even last round
-        cp.gsplit = (G % 2 == 0 && G >= 4) ? G / 2 : G;
+        // Two heads per workgroup where the group allows it: the keys a workgroup holds in registers and its pipeline
+        // start serve twice the work.  With short chunks that matters less than an even last round (509 rows x 16 K
+        // keys x 8 kv heads: 1072 workgroups of two heads on 512 places 136 us, 2144 of one head 95 us; 488 rows over a
+        // cache that holds 1000 tokens 90 -> 52 us); 2048 rows x 16 K keys x 16 kv heads are level (563 and 559 us), and
+        // with longer chunks two heads are 1.4 % ahead.
+        cp.gsplit = (mp.Q >= 2048 && G % 2 == 0 && G >= 4) ? G / 2 : G;
         const dim3 grid((unsigned)(cp.nkb * cp.nbkv * cp.gsplit));
         const int lds = 2 * cs_stage(kD) + (cp.wnew_uniform ? 0 : (int)mp.Q * 4);
         if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(colsum_mfma_kernel<T, kD>), lds)) return rc;
