@@ -242,6 +242,8 @@ def lib():
         L.ckv_dense_bwd_workspace_bytes.restype = I64
         L.ckv_dense_bwd_key_order_bytes.argtypes = [I64]
         L.ckv_dense_bwd_key_order_bytes.restype = I64
+        L.ckv_dense_bwd_split_bytes.argtypes = [I64, I64, I64, I64, I64, C.c_int32]
+        L.ckv_dense_bwd_split_bytes.restype = I64
         L.ckv_chunk_positions.argtypes = [C.c_void_p, I64, I64, C.c_void_p, I64, I64, C.c_void_p, C.c_void_p]
         L.ckv_chunk_positions.restype = C.c_int
         L.ckv_profile_enable.argtypes = [C.c_int]

@@ -25,6 +25,8 @@ struct BwdParams {
     float* delta;  // (B, H, n_ctx)
     int* key_order;  // the matrix-core kernels' key order (see launch_dense_prologue); null: none is wanted
     int* n_visible;
+    float* part_dq;  // the matrix-core dq kernel's shares of the keys (bwd_mfma_dq_splits); null: one share
+    int n_split;
 };
 
 template <typename T>
@@ -248,7 +250,7 @@ int run_bwd(const BwdParams& p, hipStream_t stream) {
     if (!mfma) pd.key_order = nullptr;
     hipLaunchKernelGGL(bwd_delta_kernel<T>, dim3((unsigned)((rows + 3) / 4 + (pd.key_order ? 1 : 0))), dim3(kThreads), 0, stream, pd);
     CKV_HIP_TRY(hipGetLastError());
-    if (mfma) return launch_bwd_mfma(a, p.delta, p.key_order, p.n_visible, stream);
+    if (mfma) return launch_bwd_mfma(a, p.delta, p.key_order, p.n_visible, p.part_dq, p.n_split, stream);
     if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(bwd_dq_kernel<T>), (int)lds_dq)) return rc;
     hipLaunchKernelGGL(bwd_dq_kernel<T>, dim3((unsigned)((a.n_ctx + kOwn - 1) / kOwn), (unsigned)(a.B * a.H)), dim3(kThreads),
                        lds_dq, stream, p);
@@ -272,6 +274,12 @@ extern "C" int64_t ckv_dense_bwd_workspace_bytes(int64_t B, int64_t H, int64_t n
 
 extern "C" int64_t ckv_dense_bwd_key_order_bytes(int64_t n_kv) { return n_kv > 0 ? ckv::align_up((n_kv + 1) * (int64_t)sizeof(int), 256) : 0; }
 
+extern "C" int64_t ckv_dense_bwd_split_bytes(int64_t B, int64_t H, int64_t n_ctx, int64_t n_kv, int64_t D, int32_t dtype) {
+    if (B <= 0 || H <= 0 || n_ctx <= 0 || n_kv < n_ctx || (D != 64 && D != 128) || dtype == CKV_F32) return 0;
+    const int splits = ckv::bwd_mfma_dq_splits(B, H, n_ctx, n_kv, ckv::mfma_device_cus());
+    return splits > 1 ? ckv::align_up(splits * B * H * n_ctx * D * (int64_t)sizeof(float), 256) : 0;
+}
+
 extern "C" int ckv_attn_dense_bwd(const ckv_dense_bwd_args* args, void* stream_) {
     using namespace ckv;
     if (!args) return CKV_ERR_NULL;
@@ -289,10 +297,18 @@ extern "C" int ckv_attn_dense_bwd(const ckv_dense_bwd_args* args, void* stream_)
     p.a = a;
     p.delta = reinterpret_cast<float*>(a.workspace);
     p.key_order = p.n_visible = nullptr;
+    p.part_dq = nullptr;
+    p.n_split = 1;
     const int64_t need = ckv_dense_bwd_workspace_bytes(a.B, a.H, a.n_ctx);
     if (a.workspace_bytes >= need + ckv_dense_bwd_key_order_bytes(a.n_kv)) {
         p.n_visible = reinterpret_cast<int*>((char*)a.workspace + need);
         p.key_order = p.n_visible + 1;
+        const int64_t split_bytes = ckv_dense_bwd_split_bytes(a.B, a.H, a.n_ctx, a.n_kv, a.D, a.dtype);
+        const int64_t split_off = need + ckv_dense_bwd_key_order_bytes(a.n_kv);
+        if (split_bytes > 0 && a.workspace_bytes >= split_off + split_bytes) {
+            p.part_dq = reinterpret_cast<float*>((char*)a.workspace + split_off);
+            p.n_split = bwd_mfma_dq_splits(a.B, a.H, a.n_ctx, a.n_kv, mfma_device_cus());
+        }
     }
     switch (a.dtype) {
         case CKV_F32: return run_bwd<float>(p, stream);

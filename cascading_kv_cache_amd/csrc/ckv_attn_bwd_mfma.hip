@@ -79,6 +79,8 @@ struct BwdMfmaParams {
     const float* delta;  // (B, H, n_ctx)
     const int* key_order;  // null: keys as they lie
     const int* n_visible;
+    float* part_dq;      // dq in shares of the keys, see dq_splits; null with one share
+    int n_split;
 };
 
 // 128 dims: a row is all 64 banks, so 16 consecutive rows need 16 different slots for one piece, and the four rows of a
@@ -217,7 +219,8 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dq_kernel(BwdMfmaParams 
     const Keys keys(p);
     const int64_t n_ctx = a.n_ctx, n_cached = keys.n_cached;
     const int64_t bh = blockIdx.y, b = bh / a.H, hd = bh % a.H;
-    const int64_t m_wg = (int64_t)blockIdx.x * kOwn;
+    const int share = (int)blockIdx.x % p.n_split;
+    const int64_t m_wg = (int64_t)(blockIdx.x / p.n_split) * kOwn;
     const int64_t m_lane = m_wg + wave * 32 + (lane & 31);  // this lane's query
     const char* kb = reinterpret_cast<const char*>(a.k) + (b * a.kv_stride[0] + hd * a.kv_stride[1]) * 2;
     const char* vb = reinterpret_cast<const char*>(a.v) + (b * a.kv_stride[0] + hd * a.kv_stride[1]) * 2;
@@ -256,7 +259,10 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dq_kernel(BwdMfmaParams 
     int64_t m_last = m_wg + kOwn - 1;
     if (m_last > n_ctx - 1) m_last = n_ctx - 1;
     const int64_t n_end = n_cached + m_last + 1;
-    const int nblk = (int)((n_end + kBlk - 1) / kBlk);
+    const int nblk_all = (int)((n_end + kBlk - 1) / kBlk);
+    // this workgroup's share of them: an equal stretch (an empty one leaves zeros)
+    const int per_share = (nblk_all + p.n_split - 1) / p.n_split;
+    const int blk0 = share * per_share, nblk = blk0 + per_share < nblk_all ? blk0 + per_share : nblk_all;
 
     // Which keys of a block any query may see, and the rows this lane copies.  Both are requested a block before the
     // copies that need them and looked at after this block's work, so that nothing in between waits for memory.
@@ -271,14 +277,14 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dq_kernel(BwdMfmaParams 
     };
     const uint32_t row_bytes = (uint32_t)kv_row;
     uint32_t rows_next[kHD / 64];
-    rows_of(0, rows_next);
-    uint32_t vis = (uint32_t)__ballot(key_bit(0) != 0u);
-    copy_rows<kHD>(kb, row_bytes, rows_next, lds0, wave, lane);
-    copy_rows<kHD>(vb, row_bytes, rows_next, lds0 + kTile, wave, lane);
-    rows_of(kBlk, rows_next);
+    rows_of((int64_t)blk0 * kBlk, rows_next);
+    uint32_t vis = (uint32_t)__ballot(key_bit((int64_t)blk0 * kBlk) != 0u);
+    copy_rows<kHD>(kb, row_bytes, rows_next, lds0 + (uint32_t)((blk0 & 1) * 2 * kTile), wave, lane);
+    copy_rows<kHD>(vb, row_bytes, rows_next, lds0 + (uint32_t)((blk0 & 1) * 2 * kTile + kTile), wave, lane);
+    rows_of((int64_t)(blk0 + 1) * kBlk, rows_next);
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
     __syncthreads();
-    for (int blk = 0; blk < nblk; blk++) {
+    for (int blk = blk0; blk < nblk; blk++) {
         const int st = blk & 1;
         const int64_t n0 = (int64_t)blk * kBlk;
         uint32_t kb_next = 0u;
@@ -350,7 +356,15 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dq_kernel(BwdMfmaParams 
         vis = (uint32_t)__ballot(kb_next != 0u);
         __syncthreads();
     }
-    if (row_ok) {
+    if (row_ok && p.n_split > 1) {
+        float* out = p.part_dq + ((int64_t)share * a.B * a.H * n_ctx + bh * n_ctx + m_lane) * kHD;
+#pragma unroll
+        for (int db = 0; db < kHD / 32; db++)
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                *reinterpret_cast<float4*>(out + 32 * db + 8 * j + 4 * h) =
+                    make_float4(dq[db][4 * j], dq[db][4 * j + 1], dq[db][4 * j + 2], dq[db][4 * j + 3]);
+    } else if (row_ok) {
         char* out = reinterpret_cast<char*>(a.dq) + (b * a.dq_stride[0] + hd * a.dq_stride[1] + m_lane * a.dq_stride[2]) * 2;
 #pragma unroll
         for (int db = 0; db < kHD / 32; db++) {
@@ -362,6 +376,24 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dq_kernel(BwdMfmaParams 
             }
         }
     }
+}
+
+// the shares of dq added up in order and rounded once; a thread takes four dims of a row
+template <typename T, int kHD>
+__global__ void __launch_bounds__(kThreads) bwd_dq_sum_kernel(BwdMfmaParams p) {
+    const ckv_dense_bwd_args& a = p.a;
+    const int64_t rows = a.B * a.H * a.n_ctx, i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+    const int64_t row = i / (kHD / 4);
+    const int d = (int)(i % (kHD / 4)) * 4;
+    if (row >= rows) return;
+    float4 sum = *reinterpret_cast<const float4*>(p.part_dq + row * kHD + d);
+    for (int s = 1; s < p.n_split; s++) {
+        const float4 v = *reinterpret_cast<const float4*>(p.part_dq + (s * rows + row) * kHD + d);
+        sum.x += v.x; sum.y += v.y; sum.z += v.z; sum.w += v.w;
+    }
+    const int64_t bh = row / a.n_ctx, m = row % a.n_ctx, b = bh / a.H, hd = bh % a.H;
+    char* out = reinterpret_cast<char*>(a.dq) + (b * a.dq_stride[0] + hd * a.dq_stride[1] + m * a.dq_stride[2] + d) * 2;
+    *reinterpret_cast<uint2*>(out) = make_uint2(Mma<T>::pack2(sum.x, sum.y), Mma<T>::pack2(sum.z, sum.w));
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -564,9 +596,15 @@ inline bool rows_ok(const int64_t* st) {
 template <typename T, int kHD>
 int run(const BwdMfmaParams& p, hipStream_t stream) {
     const ckv_dense_bwd_args& a = p.a;
-    hipLaunchKernelGGL((bwd_mfma_dq_kernel<T, kHD>), dim3((unsigned)((a.n_ctx + kOwn - 1) / kOwn), (unsigned)(a.B * a.H)),
+    hipLaunchKernelGGL((bwd_mfma_dq_kernel<T, kHD>), dim3((unsigned)((a.n_ctx + kOwn - 1) / kOwn * p.n_split), (unsigned)(a.B * a.H)),
                        dim3(kThreads), 0, stream, p);
     CKV_HIP_TRY(hipGetLastError());
+    if (p.n_split > 1) {
+        const int64_t threads = a.B * a.H * a.n_ctx * (kHD / 4);
+        hipLaunchKernelGGL((bwd_dq_sum_kernel<T, kHD>), dim3((unsigned)((threads + kThreads - 1) / kThreads)), dim3(kThreads), 0,
+                           stream, p);
+        CKV_HIP_TRY(hipGetLastError());
+    }
     if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(bwd_mfma_dkdv_kernel<T, kHD>), Geo<kHD>::kDkdvLds)) return rc;
     hipLaunchKernelGGL((bwd_mfma_dkdv_kernel<T, kHD>), dim3((unsigned)((a.n_kv + kOwn - 1) / kOwn), (unsigned)(a.B * a.H)),
                        dim3(kThreads), Geo<kHD>::kDkdvLds, stream, p);
@@ -587,8 +625,24 @@ bool bwd_mfma_supported(const ckv_dense_bwd_args& a) {
            aligned16(a.dk) && aligned16(a.dv);
 }
 
-int launch_bwd_mfma(const ckv_dense_bwd_args& a, const float* delta, const int* key_order, const int* n_visible, hipStream_t stream) {
+// Shares of the keys for dq (1: no sharing).  A launch has one workgroup per 128 rows of a head, two of which fit a compute
+// unit: with fewer than one per compute unit the keys are dealt out over up to 8 of them, at least 8 blocks of 32 keys each,
+// about two workgroups per compute unit in all, and the shares (float32) are added up by a kernel behind.  8 heads x 1000
+// rows are 64 workgroups, a quarter of the chip.
+int bwd_mfma_dq_splits(int64_t B, int64_t H, int64_t n_ctx, int64_t n_kv, int cus) {
+    const int64_t wgs = (n_ctx + kOwn - 1) / kOwn * B * H, blocks = (n_kv + kBlk - 1) / kBlk;
+    if (wgs >= cus) return 1;
+    int64_t s = 2 * (int64_t)cus / wgs;
+    if (s > blocks / 8) s = blocks / 8;
+    if (s > 8) s = 8;
+    return s < 1 ? 1 : (int)s;
+}
+
+int launch_bwd_mfma(const ckv_dense_bwd_args& a, const float* delta, const int* key_order, const int* n_visible, float* part_dq,
+                    int n_split, hipStream_t stream) {
     BwdMfmaParams p;
+    p.part_dq = part_dq;
+    p.n_split = part_dq ? n_split : 1;
     p.a = a;
     p.delta = delta;
     p.key_order = key_order;

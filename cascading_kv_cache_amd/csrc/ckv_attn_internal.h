@@ -187,7 +187,10 @@ int launch_mfma(const MfmaProblem& p, hipStream_t stream);
 // ---- backward of the dense operator on the matrix cores (16-bit, head_dim 64 and 128, 16-byte addressable rows) ----
 // key_order / n_visible: see launch_dense_prologue; both null when the caller's workspace has no room for them
 bool bwd_mfma_supported(const ckv_dense_bwd_args& a);
-int launch_bwd_mfma(const ckv_dense_bwd_args& a, const float* delta, const int* key_order, const int* n_visible, hipStream_t stream);  // delta: (B, H, n_ctx)
+int bwd_mfma_dq_splits(int64_t B, int64_t H, int64_t n_ctx, int64_t n_kv, int cus);
+// delta: (B, H, n_ctx); part_dq: bwd_mfma_dq_splits shares of (B, H, n_ctx, D) floats, or null (then dq is not shared out)
+int launch_bwd_mfma(const ckv_dense_bwd_args& a, const float* delta, const int* key_order, const int* n_visible, float* part_dq,
+                    int n_split, hipStream_t stream);
 
 // ---- single-token decode family (Q == 1, head_dim 128) ----
 bool decode_supported(const ckv_attn_args& a);

@@ -86,6 +86,7 @@ def _backward(q, k, v, o, lse, mask, do, sm_scale):
     a.scale = float(sm_scale)
     a.dtype = _abi.dtype_code(q.dtype)
     need = lib.ckv_dense_bwd_workspace_bytes(B, H, n_ctx) + lib.ckv_dense_bwd_key_order_bytes(n_kv)
+    need += lib.ckv_dense_bwd_split_bytes(B, H, n_ctx, n_kv, D, a.dtype)
     with torch.cuda.device(q.device):
         stream = torch.cuda.current_stream(q.device).cuda_stream
         ws = workspace(q.device, need, stream)

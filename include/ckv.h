@@ -283,6 +283,9 @@ int64_t ckv_dense_bwd_workspace_bytes(int64_t B, int64_t H, int64_t n_ctx);
 /* Room for the order of the keys behind those bytes (optional): with a workspace of both sizes the 16-bit kernels of
  * head_dim 64 and 128 sort the masked keys out once and spend no work on them; with the first alone they test every key. */
 int64_t ckv_dense_bwd_key_order_bytes(int64_t n_kv);
+/* Room behind both (optional): with it a 16-bit backward pass of few query rows shares dq's keys out over several
+ * workgroups.  0 where that would not help. */
+int64_t ckv_dense_bwd_split_bytes(int64_t B, int64_t H, int64_t n_ctx, int64_t n_kv, int64_t D, int32_t dtype);
 
 int ckv_attn_dense_bwd(const ckv_dense_bwd_args* args, void* stream);
 
