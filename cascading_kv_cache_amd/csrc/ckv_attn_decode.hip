@@ -1451,12 +1451,13 @@ __global__ void __launch_bounds__(512) decode_tail_kernel(DecodeParams p) {
 // 513 tiles (a 64K cache) are two batches per group, 257 tiles one.
 constexpr int kTailBatch = 9;
 
+struct TailLds {
+    float m[32], l[32];
+    float o[32][kD];
+};
 template <typename T>
-__global__ void __launch_bounds__(512) decode_tail_stream_kernel(DecodeParams p) {
-    __shared__ float sh_m[32], sh_l[32];
-    __shared__ float sh_o[32][kD];
+__device__ inline void tail_stream_row(const DecodeParams& p, int64_t row, TailLds& sh) {  // row: b * H + h
     const ckv_attn_args& a = p.a;
-    const int64_t row = blockIdx.x;  // b * H + h
     const int tid = threadIdx.x, d8 = tid & 15, grp = tid >> 4;
     const int n_vis = p.n_vis;  // the items are numbered over the tiles that can hold a visible key
     const int64_t nbh = a.B * a.KVH, total = (int64_t)n_vis * nbh;
@@ -1509,23 +1510,23 @@ __global__ void __launch_bounds__(512) decode_tail_stream_kernel(DecodeParams p)
         }
     }
 #pragma unroll
-    for (int e = 0; e < 8; e++) sh_o[grp][d8 * 8 + e] = o[e];
+    for (int e = 0; e < 8; e++) sh.o[grp][d8 * 8 + e] = o[e];
     if (d8 == 0) {
-        sh_m[grp] = M;
-        sh_l[grp] = L;
+        sh.m[grp] = M;
+        sh.l[grp] = L;
     }
     __syncthreads();
     if (tid >= kD) return;
     float Mx = -INFINITY;
 #pragma unroll
-    for (int k = 0; k < 32; k++) Mx = fmaxf(Mx, sh_m[k]);
+    for (int k = 0; k < 32; k++) Mx = fmaxf(Mx, sh.m[k]);
     float od = 0.f;
     L = 0.f;
 #pragma unroll
     for (int k = 0; k < 32; k++) {
-        const float f = sh_m[k] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(sh_m[k] - Mx);
-        od = fmaf(sh_o[k][tid], f, od);
-        L = fmaf(sh_l[k], f, L);
+        const float f = sh.m[k] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(sh.m[k] - Mx);
+        od = fmaf(sh.o[k][tid], f, od);
+        L = fmaf(sh.l[k], f, L);
     }
     const int64_t b = row / a.H, h = row % a.H;
     T* out = (T*)a.out + b * a.out_stride[0] + h * a.out_stride[1];
@@ -1535,6 +1536,12 @@ __global__ void __launch_bounds__(512) decode_tail_stream_kernel(DecodeParams p)
         p.lse2[row] = l2;
         if (a.lse) a.lse[row] = l2 * 0.6931471805599453f;
     }
+}
+
+template <typename T>
+__global__ void __launch_bounds__(512) decode_tail_stream_kernel(DecodeParams p) {
+    __shared__ TailLds sh;
+    tail_stream_row<T>(p, blockIdx.x, sh);
 }
 
 template <typename T, int G>
@@ -1637,13 +1644,10 @@ __global__ void __launch_bounds__(256) decode_scores_kernel(DecodeParams p, floa
 
 // The same after the streaming kernel, per kv head: one thread per (b, kvh, 8 consecutive keys), which are one
 // 16-byte piece of each head's fp16 probabilities and share the tile maximum.
-template <typename T, int G>
-__global__ void __launch_bounds__(256) decode_scores_probs_kernel(DecodeParams p, float w_one, float beta_pow) {
+template <typename T, int G, typename Lse>
+__device__ inline void scores_of_group(const DecodeParams& p, int64_t n0, int64_t b, int64_t kvh, float w_one, float beta_pow,
+                                       Lse lse_of) {  // lse_of(g): the log2-domain normaliser of head g of the kv head
     const ckv_attn_args& a = p.a;
-    const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t per = p.Np / 8;
-    if (idx >= a.B * a.KVH * per) return;
-    const int64_t n0 = (idx % per) * 8, kvh = (idx / per) % a.KVH, b = idx / (per * a.KVH);
     if (n0 + 8 <= a.num_sink || n0 >= p.N) return;  // sinks keep no score; padding
     float pr[G][8];
     const int jt = stream_rank_of(p, (int)(n0 / kSK));  // -1: no key of the tile is visible, all probabilities are 0
@@ -1652,12 +1656,11 @@ __global__ void __launch_bounds__(256) decode_scores_probs_kernel(DecodeParams p
     const unsigned char* chunk = p.chunks + ck * (G * (kSK + kD) * 2);
 #pragma unroll
     for (int g = 0; g < G; g++) {
-        const int64_t row = b * a.H + kvh * G + g;
         uint4 raw = make_uint4(0u, 0u, 0u, 0u);
         float c = 0.f;
         if (jt >= 0) {
             raw = *reinterpret_cast<const uint4*>(chunk + (g * kSK + n0 % kSK) * 2);
-            c = __builtin_amdgcn_exp2f(p.part_ml[(ck * G + g) * 2] - p.lse2[row]);
+            c = __builtin_amdgcn_exp2f(p.part_ml[(ck * G + g) * 2] - lse_of(g));
         }
         const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
 #pragma unroll
@@ -1726,6 +1729,70 @@ __global__ void __launch_bounds__(256) decode_scores_probs_kernel(DecodeParams p
             *c1 = Elem<T>::from_float(__fadd_rn(decayed, red[k]));
         }
     }
+}
+
+template <typename T, int G>
+__global__ void __launch_bounds__(256) decode_scores_probs_kernel(DecodeParams p, float w_one, float beta_pow) {
+    const ckv_attn_args& a = p.a;
+    const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t per = p.Np / 8;
+    if (idx >= a.B * a.KVH * per) return;
+    const int64_t kvh = (idx / per) % a.KVH, b = idx / (per * a.KVH);
+    scores_of_group<T, G>(p, (idx % per) * 8, b, kvh, w_one, beta_pow, [&](int g) { return p.lse2[b * a.H + kvh * G + g]; });
+}
+
+// Tail and scores in one launch: the first B * H workgroups combine a row each, the others work out the scores of 4096
+// keys of one (b, kvh), for which they first merge the (maximum, sum) pairs of its G heads themselves.  That costs a
+// score workgroup two trips to memory before its own work (with more workgroups than the chip holds at once, 16 streams
+// x 257 tiles, 40 us against 30 us for two launches); when all of them run side by side it is hidden behind the rows:
+// with one stream the step is a chain of short launches, and this takes one out (host and device: about 4 us each).
+template <typename T, int G>
+__global__ void __launch_bounds__(512) decode_finish_kernel(DecodeParams p, float w_one, float beta_pow, int per_unit) {
+    __shared__ TailLds sh;
+    const ckv_attn_args& a = p.a;
+    const int rows = (int)(a.B * a.H), tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    if ((int)blockIdx.x < rows) {
+        tail_stream_row<T>(p, blockIdx.x, sh);
+        return;
+    }
+    static_assert(G <= 8, "a wavefront per head merges the pairs");
+    const int id = (int)blockIdx.x - rows, unit = id / per_unit;
+    const int64_t nbh = a.B * a.KVH, total = (int64_t)p.n_vis * nbh;
+    float* sh_lse = &sh.m[0];
+    if (wave < G) {
+        float M = -INFINITY, L = 0.f;
+        constexpr int kBatch = 4;   // tiles of a lane on their way at once
+        for (int t0 = lane; t0 < p.n_vis; t0 += 64 * kBatch) {
+            float2 w[kBatch];
+#pragma unroll
+            for (int u = 0; u < kBatch; u++) {
+                const int t = t0 + 64 * u;
+                w[u] = make_float2(-INFINITY, 0.f);
+                if (t < p.n_vis) {
+                    const int64_t ck = stream_chunk_of((int64_t)t * nbh + unit, total, p.stream_wgs);
+                    w[u] = *reinterpret_cast<const float2*>(p.part_ml + (ck * G + wave) * 2);
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < kBatch; u++) {
+                const float m = fmaxf(M, w[u].x);
+                if (m == -INFINITY) continue;
+                L = L * __builtin_amdgcn_exp2f(M - m) + w[u].y * __builtin_amdgcn_exp2f(w[u].x - m);
+                M = m;
+            }
+        }
+        float Mx = M;
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) Mx = fmaxf(Mx, __shfl_xor(Mx, off));
+        L = M == -INFINITY ? 0.f : L * __builtin_amdgcn_exp2f(M - Mx);
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) L += __shfl_xor(L, off);
+        if (lane == 0) sh_lse[wave] = Mx + __builtin_amdgcn_logf(L);
+    }
+    __syncthreads();
+    const int64_t n0 = ((int64_t)(id % per_unit) * 512 + tid) * 8;
+    if (n0 >= p.Np) return;
+    scores_of_group<T, G>(p, n0, unit / a.KVH, unit % a.KVH, w_one, beta_pow, [&](int g) { return sh_lse[g]; });
 }
 
 // All heads reduced together (cascade_attention.py:240-242) after a streaming kernel: one thread per (batch, key),
@@ -1882,6 +1949,15 @@ int run_decode(const DecodeParams& p_in, hipStream_t stream) {
         StageScope sc(CKV_STAGE_DECODE_TAIL, stream);
         bool launched = false;
         if constexpr (G <= 8 && !std::is_same<T, float>::value) {
+            DeviceInfo di;
+            if (int rc = current_device_info(&di)) return rc;
+            const int64_t per_unit = (p.Np / 8 + 511) / 512, blocks = a.B * a.H + a.B * a.KVH * per_unit;
+            if (use_stream && !a.homogeneous_heads && (a.cache_s || a.new_scores) && blocks <= 2 * (int64_t)di.cus) {
+                hipLaunchKernelGGL((decode_finish_kernel<T, G>), dim3((unsigned)blocks), dim3(512), 0, stream, p,
+                                   (float)(1.0 - a.beta), (float)a.beta, (int)per_unit);
+                CKV_HIP_TRY(hipGetLastError());
+                return CKV_OK;
+            }
             if (use_stream) {
                 hipLaunchKernelGGL(decode_tail_stream_kernel<T>, dim3((unsigned)(a.B * a.H)), dim3(512), 0, stream, p);
                 launched = true;

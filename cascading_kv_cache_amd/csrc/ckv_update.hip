@@ -799,6 +799,11 @@ constexpr int kOneThreads = 1024, kOneWaves = kOneThreads / CKV_WAVE;
 // path spreads them over the chip and is faster while the units are few (8 units of 64K slots: 9.4 + a launch gap
 // against 13.4 us; 128 units of 32K slots: 18 against 12.5 us).
 constexpr int kOneMinUnits = 32;
+// ... unless the slots are few too: from 8 units (one stream of eight kv heads) with up to this many slots each the ids are
+// written in less time than a second launch takes (8 units of 2K slots: 10.1 us for plan and
+// apply, 7.3 in one launch; of 16K slots: 9.8 and 8.0; of 64K slots the two launches are ahead, see above).
+constexpr int kOneFewUnits = 8;
+constexpr int64_t kOneMaxSlots = 16384;
 
 __global__ void __launch_bounds__(kOneThreads) ckv_update_one_kernel(UpdateParams p) {
     __shared__ int sh_chain[kOneWaves];
@@ -1192,7 +1197,8 @@ int run_update(const ckv_update_args& A, void* workspace, hipStream_t stream) {
     p.k_sub = 0;
     p.do_pos = 0;
     p.apply_blocks = 0;
-    if (A.K == 1 && vec && A.cascades <= kOneWaves && A.HID * es / 16 <= CKV_WAVE && A.N * A.H >= kOneMinUnits) {
+    if (A.K == 1 && vec && A.cascades <= kOneWaves && A.HID * es / 16 <= CKV_WAVE &&
+        (A.N * A.H >= kOneMinUnits || (A.N * A.H >= kOneFewUnits && A.max_seq_len <= kOneMaxSlots))) {
         // the decode step of many streams: plan, moves and position ids of a unit by one workgroup, one launch
         launch_timed(CKV_STAGE_APPLY, ckv_update_one_kernel, dim3((unsigned)(A.N * A.H)), dim3(kOneThreads), 0, stream, p);
         CKV_HIP_TRY(hipGetLastError());
