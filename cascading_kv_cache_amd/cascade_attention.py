@@ -203,10 +203,10 @@ def cascade_attention(query_states, key_states, value_states, cache: CascadingKV
         a.k_new, a.v_new = key_states.data_ptr(), value_states.data_ptr()
         a.q_pos = q_pos.data_ptr()
         a.pos_shift = 0 if do_og_pos else cache.pos_shift(L)
-        # the cache fills from slot 0 up and holds at most the tokens seen past the sinks: single-token steps skip
-        # the empty part of a cache that is still filling
-        filled = int(cache._seen_host[L]) - cache.num_sink_tokens
-        a.filled_slots = filled if not replayable and 0 < filled < cache.max_seq_len[L] else 0
+        # the cache fills from slot 0 up and holds at most the tokens seen past the sinks: the kernels skip the empty
+        # part of a cache that is still filling (at least one slot is claimed: 0 would mean no bound)
+        filled = max(int(cache._seen_host[L]) - cache.num_sink_tokens, 1)
+        a.filled_slots = filled if not replayable and filled < cache.max_seq_len[L] else 0
         a.out = out.data_ptr()
         a.new_scores = new_scores.data_ptr()
         ws = workspace(dev, a._need, stream)

@@ -18,6 +18,7 @@
 //                inside a lane (S = Q K^T orientation).
 #include "ckv_attn_internal.h"
 
+#include <algorithm>
 #include <cstring>
 #include <type_traits>
 
@@ -167,8 +168,7 @@ __device__ inline void stage_keys_block(const StageParams& p, int tile_i, int sp
 
     // A tile of slots that cannot hold a token yet is read by nobody: the forward kernel leaves it out, the score kernel
     // zeroes its sums.  A cache that is still filling is mostly such tiles (1000 of 16384 slots, 488-token chunk: the
-    // launch takes 31 us instead of 50).  The bound comes from the host's counter: looking at the mask first costs a
-    // full cache 4 us of 43.
+    // launch takes 31 us instead of 50).  The bound comes from the host's counter, so that nothing waits for the mask.
     if (tile * kBN >= p.empty_from && (tile + 1) * kBN <= p.empty_to) {
         if (split_i == 0 && tid == 0) p.tile_vis[tile] = 0ull;
         return;
@@ -404,8 +404,9 @@ __device__ inline void stage_q_block(const StageQParams& p, int blk, int share_i
     }
 }
 
-// One launch stages queries and keys: the two are independent.  1-D grid: the key blocks (k_bx x k_by)
-// first, then the query blocks (q_bx x q_by), which are short and fill the ragged end of the key blocks.
+// One launch stages queries and keys and writes the weights of the score sums: the three are independent.  1-D grid: the
+// key blocks (k_bx x k_by) first, then the query blocks (q_bx x q_by), which are short and fill the ragged end of the key
+// blocks, then the blocks with weights (a launch of their own took 5 us of 305 with 509 rows over 16 K slots).
 struct StageGrid {
     int q_bx, q_by, k_bx, k_by;
 };
@@ -922,17 +923,34 @@ __global__ void __launch_bounds__(256) fwd_combine_kernel(FwdParams p) {
     const int64_t row = (int64_t)blockIdx.x * (256 / kLanes) + threadIdx.x / kLanes;
     if (row >= rows) return;
     const int d4 = threadIdx.x % kLanes;
+    // with few rows a thread's loads are the whole kernel: all normalisers first, then the rows, eight on their way at once
+    constexpr int kBatch = 8;
     float M = -INFINITY;
-    for (int s_ = 0; s_ < p.n_split; s_++) M = fmaxf(M, p.part_l2[s_ * rows + row]);
+    for (int s0 = 0; s0 < p.n_split; s0 += kBatch) {
+        float l2[kBatch];
+#pragma unroll
+        for (int u = 0; u < kBatch; u++) l2[u] = s0 + u < p.n_split ? p.part_l2[(s0 + u) * rows + row] : -INFINITY;
+#pragma unroll
+        for (int u = 0; u < kBatch; u++) M = fmaxf(M, l2[u]);
+    }
     float L = 0.f;
     float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int s_ = 0; s_ < p.n_split; s_++) {
-        const float l2 = p.part_l2[s_ * rows + row];
-        if (l2 == -INFINITY) continue;
-        const float w = __builtin_amdgcn_exp2f(l2 - M);
-        const float4 v = *reinterpret_cast<const float4*>(p.part_o + (s_ * rows + row) * kD + 4 * d4);
-        L += w;
-        o.x = fmaf(v.x, w, o.x); o.y = fmaf(v.y, w, o.y); o.z = fmaf(v.z, w, o.z); o.w = fmaf(v.w, w, o.w);
+    for (int s0 = 0; s0 < p.n_split; s0 += kBatch) {
+        float l2[kBatch];
+        float4 v[kBatch];
+#pragma unroll
+        for (int u = 0; u < kBatch; u++) {
+            const int s_ = s0 + u < p.n_split ? s0 + u : s0;
+            l2[u] = s0 + u < p.n_split ? p.part_l2[s_ * rows + row] : -INFINITY;
+            v[u] = *reinterpret_cast<const float4*>(p.part_o + (s_ * rows + row) * kD + 4 * d4);
+        }
+#pragma unroll
+        for (int u = 0; u < kBatch; u++) {
+            if (l2[u] == -INFINITY) continue;
+            const float w = __builtin_amdgcn_exp2f(l2[u] - M);
+            L += w;
+            o.x = fmaf(v[u].x, w, o.x); o.y = fmaf(v[u].y, w, o.y); o.z = fmaf(v[u].z, w, o.z); o.w = fmaf(v[u].w, w, o.w);
+        }
     }
     const float inv = 1.f / L;
     const int64_t m = row % p.Q, h = (row / p.Q) % p.H, b = row / (p.Q * p.H);
@@ -1432,7 +1450,7 @@ int run_mfma(const MfmaProblem& mp, hipStream_t stream) {
         fp.G = G;
         fp.scale_log2 = 1.f;  // already on the staged queries
         fp.n_qt = (int)((mp.Q * G + kRows - 1) / kRows);
-        fp.n_split = mfma_fwd_splits(mp.B, mp.H, mp.KVH, mp.Q, n, cus);
+        fp.n_split = mfma_fwd_splits(mp.B, mp.H, mp.KVH, mp.Q, n, cus, mp.empty_to > mp.empty_from);
         fp.part_o = mp.part_o;
         fp.part_l2 = mp.part_l2;
         fp.n_visible = mp.n_visible;
@@ -1512,17 +1530,43 @@ bool mfma_supported(int dtype, int64_t D, int64_t H, int64_t KVH, int64_t Q) {
 
 int64_t mfma_n_pad(int64_t n) { return align_up(n, 256); }
 
-// Shares of a query tile's key tiles (1: no splitting) on a chip of `cus` compute units, each of which holds one
-// workgroup of the forward kernel at a time: launches with fewer workgroups than that are topped up to about two per
-// compute unit, with at least 16 key tiles per share and at most 8 shares.
-int mfma_fwd_splits(int64_t B, int64_t H, int64_t KVH, int64_t Q, int64_t n, int cus) {
+// Shares of a query tile's key tiles (1: no splitting) on a chip of `cus` compute units, each of which holds one workgroup
+// of the forward kernel at a time.  The launch takes whole rounds of workgroups, a round as long as a workgroup: about
+// 1.6 us per key tile with every unit busy and 16 us to start and finish (the work list, the first copies, the rows' way
+// out).  Shares shorten a workgroup, fill a round that is mostly empty, and cost the merge kernel 6 us and its traffic
+// (float32 rows written and read, 256 rows of 512 bytes per workgroup: 0.058 us).  The cheapest number of shares by that
+// count, at least 8 key tiles each.  32 heads on 8 kv heads, forward + merge (before: about two workgroups per unit, at
+// most 8 shares): 509 rows x 16 K keys 162 -> 141 us, 128 x 64 K 203 -> 149, 32 x 64 K 168 -> 93, 1000 x 16 K 271 -> 259,
+// 300 x 2 K 40 -> 34.
+// `filling`: most slots of the cache are known to be empty.  The tiles that are left make shares of a few tiles by either
+// count; those streams keep the count they have always had (about two workgroups per unit, at least 16 tiles by the
+// cache's size, at most 8 shares), so that a decoder's sums are added in the same order as before: four random layers
+// turn one changed rounding of a hidden state into a percent of the logits.
+int mfma_fwd_splits(int64_t B, int64_t H, int64_t KVH, int64_t Q, int64_t n, int cus, bool filling) {
+    constexpr double kTileUs = 1.6, kStartUs = 16.0, kMergeUs = 6.0, kMergeWgUs = 0.058;
+    constexpr int64_t kMaxShares = 32, kMaxShareBytes = (int64_t)256 << 20, kMinTiles = 8;
     const int64_t G = H / KVH;
     const int64_t wgs = ((Q * G + kRows - 1) / kRows) * B * KVH, tiles = (n + kBN - 1) / kBN;
-    if (wgs >= cus) return 1;
-    int64_t s_ = 2 * (int64_t)cus / wgs;
-    if (s_ > tiles / 16) s_ = tiles / 16;
-    if (s_ > 8) s_ = 8;
-    return s_ < 1 ? 1 : (int)s_;
+    if (filling) {
+        if (wgs >= cus) return 1;
+        const int64_t by_size = tiles / 16 < 8 ? tiles / 16 : 8, by_units = 2 * (int64_t)cus / wgs;
+        const int64_t s_ = by_units < by_size ? by_units : by_size;
+        return s_ < 1 ? 1 : (int)s_;
+    }
+    if (wgs >= 4 * (int64_t)cus) return 1;   // at most an eighth of the launch can be an empty round
+    int best = 1;
+    double best_us = 0.0;
+    for (int64_t s_ = 1; s_ <= kMaxShares && (s_ == 1 || tiles / s_ >= kMinTiles); s_++) {
+        if (s_ > 1 && s_ * wgs * kRows * 512 > kMaxShareBytes) break;
+        const double rounds = (double)((wgs * s_ + cus - 1) / cus);
+        const double us = rounds * ((double)tiles / (double)s_ * kTileUs + kStartUs) +
+                          (s_ > 1 ? kMergeUs + kMergeWgUs * (double)(wgs * s_) : 0.0);
+        if (s_ == 1 || us < best_us) {
+            best = (int)s_;
+            best_us = us;
+        }
+    }
+    return best;
 }
 
 // compute units of the current device; 256 (one MI355X) where no device can be asked, e.g. when a workspace is
@@ -1536,9 +1580,10 @@ int mfma_device_cus() {
 // what a workspace is sized for: the shares the current device would use, and never fewer than a 256-unit chip's,
 // so that a size computed where no device is visible also serves the launch
 int mfma_fwd_splits_for_workspace(int64_t B, int64_t H, int64_t KVH, int64_t Q, int64_t n) {
-    const int here = mfma_fwd_splits(B, H, KVH, Q, n, mfma_device_cus());
-    const int base = mfma_fwd_splits(B, H, KVH, Q, n, 256);
-    return here > base ? here : base;
+    int most = 1;
+    for (const int cus : {mfma_device_cus(), 256})
+        for (const bool filling : {false, true}) most = std::max(most, mfma_fwd_splits(B, H, KVH, Q, n, cus, filling));
+    return most;
 }
 
 // the forward kernel keeps per-tile bookkeeping of all N keys in LDS

@@ -195,8 +195,10 @@ typedef struct ckv_attn_args {
                                       cascading_cache.py:381-726, so the tokens stored so far bound it); 0 = no
                                       promise.  Kernels may then skip such slots without reading `mask` (the 16-bit
                                       single-token kernels skip whole 128-key tiles of a cache that is still
-                                      filling) or ignore the hint altogether; visibility is decided by `mask` alone,
-                                      so with a hint that keeps its promise the results do not depend on it, and a
+                                      filling, chunks leave whole 64-key tiles out) or ignore the hint altogether;
+                                      visibility is decided by `mask` alone, so with a hint that keeps its promise the
+                                      results do not depend on it (a chunk's float32 sums may be added up in another
+                                      order), and a
                                       hint that contradicts `mask` gives unspecified results for the slots it
                                       covers. */
 
