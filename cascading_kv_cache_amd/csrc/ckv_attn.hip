@@ -124,11 +124,11 @@ extern "C" int ckv_attn(const ckv_attn_args* args, void* stream_) {
     const int64_t N = a.num_sink + a.S + a.Q;
     const bool want_scores = a.cache_s || a.new_scores;
     int rc;
-    if (want_scores) {
+    const bool use_mfma = mfma_supported(a.dtype, a.D, a.H, a.KVH, a.Q) && a.Q > 1 && mfma_fits(N, a.D);
+    if (want_scores && !use_mfma) {
         rc = launch_weights(w.w_ema, w.w_new, a.Q, a.beta, a.dtype, stream);
         if (rc) return rc;
     }
-    const bool use_mfma = mfma_supported(a.dtype, a.D, a.H, a.KVH, a.Q) && a.Q > 1 && mfma_fits(N, a.D);
     if (use_mfma) {
         MfmaProblem mp;
         mp.seg[0] = MfmaSegment{a.sink_k, a.sink_v, {a.sink_stride[0], a.sink_stride[1], a.sink_stride[2], a.sink_stride[3]},
@@ -158,6 +158,7 @@ extern "C" int ckv_attn(const ckv_attn_args* args, void* stream_) {
         mp.part_o = w.part_o; mp.part_l2 = w.part_l2;
         mp.w_ema = w.w_ema; mp.w_new = w.w_new;
         mp.beta = a.beta;
+        mp.make_weights = want_scores;
         mp.new_mode = 1;
         mp.B = a.B; mp.H = a.H; mp.KVH = a.KVH; mp.Q = a.Q; mp.D = a.D; mp.n = N; mp.n_pad = mfma_n_pad(N);
         mp.scale = a.scale;

@@ -11,25 +11,6 @@ __device__ inline float round_t(float v) {
     return Elem<T>::to_float(Elem<T>::from_float(v));
 }
 
-// ---------------------------------------------------------------------------------------------
-// weights: w_ema[m] = (1-beta) * beta^(Q-1-m) as fp32 (cascade_attention.py:315-317);
-//          w_new[k] = (1-beta) * beta^k built in the tensor dtype (cascade_attention.py:270-276)
-// ---------------------------------------------------------------------------------------------
-template <typename T>
-__device__ inline void weights_at(float* w_ema, float* w_new, int64_t Q, double beta, int64_t i) {
-    if (i >= Q + kColSlack) return;
-    if (i >= Q) {  // slack read (and multiplied by zero) by the MFMA column pass
-        w_ema[i] = 0.f;
-        return;
-    }
-    const float omb = (float)(1.0 - beta);
-    const float b32 = (float)beta;
-    w_ema[i] = __fmul_rn(omb, powf(b32, (float)(Q - 1 - i)));
-    const float bt = round_t<T>(b32);
-    const float pw = round_t<T>(powf(bt, round_t<T>((float)i)));
-    w_new[i] = round_t<T>(__fmul_rn(omb, pw));
-}
-
 template <typename T>
 __global__ void weights_kernel(float* w_ema, float* w_new, int64_t Q, double beta) {
     weights_at<T>(w_ema, w_new, Q, beta, (int64_t)blockIdx.x * blockDim.x + threadIdx.x);

@@ -79,6 +79,24 @@ int launch_finish(const FinishProblem& p, hipStream_t stream);
 // tiles of this many query rows
 constexpr int64_t kColSlack = 128;
 
+// weights: w_ema[m] = (1-beta) * beta^(Q-1-m) as fp32 (cascade_attention.py:315-317);
+//          w_new[k] = (1-beta) * beta^k built in the tensor dtype (cascade_attention.py:270-276)
+template <typename T>
+__device__ inline void weights_at(float* w_ema, float* w_new, int64_t Q, double beta, int64_t i) {
+    auto round_t = [](float v) { return Elem<T>::to_float(Elem<T>::from_float(v)); };
+    if (i >= Q + kColSlack) return;
+    if (i >= Q) {  // slack read (and multiplied by zero) by the MFMA column pass
+        w_ema[i] = 0.f;
+        return;
+    }
+    const float omb = (float)(1.0 - beta);
+    const float b32 = (float)beta;
+    w_ema[i] = __fmul_rn(omb, powf(b32, (float)(Q - 1 - i)));
+    const float bt = round_t(b32);
+    const float pw = round_t(powf(bt, round_t((float)i)));
+    w_new[i] = round_t(__fmul_rn(omb, pw));
+}
+
 // The key order of launch_dense_prologue, worked out by one workgroup of kThreads threads (64 .. 1024, a multiple of 64).
 template <int kThreads>
 __device__ inline void key_order_block(const uint8_t* mask, int64_t n_cached, int64_t n_ctx, int* key_order, int* n_visible) {
@@ -162,9 +180,10 @@ struct MfmaProblem {
     const int* n_visible = nullptr;
     float* part_o;         // (mfma_fwd_splits, B*H*Q, D) and
     float* part_l2;        // (mfma_fwd_splits, B*H*Q): the forward kernel's shares, when it splits the keys
-    const float* w_ema;
-    const float* w_new;
-    double beta;           // the EMA factor the weights were built from
+    float* w_ema;
+    float* w_new;
+    double beta;           // the EMA factor of the weights
+    int make_weights = 0;  // the staging launch writes w_ema and w_new too
     int new_mode;
     int64_t B, H, KVH, Q, D, n, n_pad;
     int64_t empty_from = 0, empty_to = 0;  // keys whose slots cannot hold a token yet

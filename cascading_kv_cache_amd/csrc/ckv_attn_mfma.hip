@@ -410,8 +410,12 @@ __device__ inline void stage_q_block(const StageQParams& p, int blk, int share_i
 struct StageGrid {
     int q_bx, q_by, k_bx, k_by;
 };
+struct StageWeights {
+    float *w_ema, *w_new;
+    double beta;
+};
 template <typename T, int kD>
-__global__ void __launch_bounds__(256) stage_kernel(StageParams sp, StageQParams sq, StageGrid g) {
+__global__ void __launch_bounds__(256) stage_kernel(StageParams sp, StageQParams sq, StageGrid g, StageWeights sw) {
     __shared__ uint32_t v_lds[kBN][kD / 2 + 1];  // (d, d + kD/2) pairs of a key row, odd pitch
     const int nk = g.k_bx * g.k_by;
     int id = blockIdx.x;
@@ -419,7 +423,8 @@ __global__ void __launch_bounds__(256) stage_kernel(StageParams sp, StageQParams
         stage_keys_block<T, kD>(sp, id % g.k_bx, id / g.k_bx, g.k_by, v_lds);
     } else {
         id -= nk;
-        stage_q_block<T, kD>(sq, id % g.q_bx, id / g.q_bx, g.q_by);
+        if (id < g.q_bx * g.q_by) stage_q_block<T, kD>(sq, id % g.q_bx, id / g.q_bx, g.q_by);
+        else weights_at<T>(sw.w_ema, sw.w_new, sq.Q, sw.beta, (int64_t)(id - g.q_bx * g.q_by) * 256 + threadIdx.x);
     }
 }
 
@@ -1431,9 +1436,11 @@ int run_mfma(const MfmaProblem& mp, hipStream_t stream) {
             if (by < 1) by = 1;
             StageGrid g;
             g.q_bx = (int)bx; g.q_by = (int)by; g.k_bx = (int)(n_pad / kBN); g.k_by = (int)splits;
-            const int64_t blocks = bx * by + (n_pad / kBN) * splits;
+            const StageWeights sw{mp.w_ema, mp.w_new, mp.beta};
+            const int64_t w_blocks = mp.make_weights ? (mp.Q + kColSlack + 255) / 256 : 0;
+            const int64_t blocks = bx * by + (n_pad / kBN) * splits + w_blocks;
             if (blocks > 0x7fffffff) return CKV_ERR_UNSUPPORTED;
-            hipLaunchKernelGGL((stage_kernel<T, kD>), dim3((unsigned)blocks), dim3(256), 0, stream, sp, sq, g);
+            hipLaunchKernelGGL((stage_kernel<T, kD>), dim3((unsigned)blocks), dim3(256), 0, stream, sp, sq, g, sw);
         }
         CKV_HIP_TRY(hipGetLastError());
     }
