@@ -22,6 +22,8 @@
 // Without an order (a caller whose workspace has no room for it) the keys are taken as they lie and masked one by one.
 #include "ckv_attn_internal.h"
 
+#include <type_traits>
+
 namespace ckv {
 namespace {
 
@@ -37,6 +39,7 @@ constexpr int kBlk = 32;              // rows of a streamed block
 constexpr int kWaves = 4;             // wavefronts of a workgroup, 32 stationary rows each
 constexpr int kThreads = kWaves * CKV_WAVE;
 constexpr int kOwn = kWaves * 32;     // stationary rows of a workgroup
+constexpr int kAhead = 3, kKvAhead = 2;  // matrix instructions between an operand's read from LDS and its use
 constexpr float kLog2e = 1.4426950408889634f;
 template <int kHD>
 struct Geo {
@@ -81,7 +84,23 @@ struct BwdMfmaParams {
     const int* n_visible;
     float* part_dq;      // dq in shares of the keys, see dq_splits; null with one share
     int n_split;
+    int per_head;        // workgroups of a (batch, head); > 0: 1-D grid, see unit_of
 };
+
+// Workgroup ids go round the 8 XCDs, each with an L2 of its own.  With 8 | B * H all workgroups of a head can run on one
+// XCD, so that the rows they all stream (K and V for dq, Q and dO for dk / dv) are fetched into one L2 instead of eight.
+// dq always does (64 heads x 1024 rows x 8704 visible keys x 128: 555 -> 529 us); dk / dv only while the launch is one round
+// of workgroups (8 heads x 5095 keys x 64: 45.5 -> 39 us; 64 heads x 17408 keys, seventeen rounds: 760 -> 988 us, all compute
+// units of an XCD on the same few rows).
+struct Unit {
+    int x;          // workgroup of the head
+    int64_t bh;
+};
+__device__ inline Unit unit_of(const BwdMfmaParams& p) {
+    if (p.per_head == 0) return Unit{(int)blockIdx.x, (int64_t)blockIdx.y};
+    const int j = (int)blockIdx.x >> 3;
+    return Unit{j % p.per_head, (int64_t)((int)blockIdx.x & 7) + 8 * (j / p.per_head)};
+}
 
 // 128 dims: a row is all 64 banks, so 16 consecutive rows need 16 different slots for one piece, and the four rows of a
 // transposing read different 64-byte quarters.  64 dims: two rows share the banks, eight slots each, and rows r, r + 2 of
@@ -218,9 +237,10 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dq_kernel(BwdMfmaParams 
     const int tid = threadIdx.x, wave = tid / CKV_WAVE, lane = tid % CKV_WAVE, h = lane >> 5;
     const Keys keys(p);
     const int64_t n_ctx = a.n_ctx, n_cached = keys.n_cached;
-    const int64_t bh = blockIdx.y, b = bh / a.H, hd = bh % a.H;
-    const int share = (int)blockIdx.x % p.n_split;
-    const int64_t m_wg = (int64_t)(blockIdx.x / p.n_split) * kOwn;
+    const Unit unit = unit_of(p);
+    const int64_t bh = unit.bh, b = bh / a.H, hd = bh % a.H;
+    const int share = unit.x % p.n_split;
+    const int64_t m_wg = (int64_t)(unit.x / p.n_split) * kOwn;
     const int64_t m_lane = m_wg + wave * 32 + (lane & 31);  // this lane's query
     const char* kb = reinterpret_cast<const char*>(a.k) + (b * a.kv_stride[0] + hd * a.kv_stride[1]) * 2;
     const char* vb = reinterpret_cast<const char*>(a.v) + (b * a.kv_stride[0] + hd * a.kv_stride[1]) * 2;
@@ -312,44 +332,54 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dq_kernel(BwdMfmaParams 
         if (!dead) {
             const unsigned char* kt = smem[st][0];
             const unsigned char* vt = smem[st][1];
+            // Written in issue order: an operand is read from LDS kAhead matrix instructions before the one that takes it
+            // (one operand at a time beside a matrix instruction, instead of four read and waited for; dk / dv 821 -> 760 us, dq level
+            // with 128 dims and 6 % with 64), and the second half of the exponentials runs beside the products of the first.
+            constexpr int kRow = kHD / 16, kDB = kHD / 32;
+            const uint32_t kt_lds = lds0 + (uint32_t)(st * 2 * kTile);
             f32x16 s = zero16(), dp = zero16();
+            uint4 ops[2 * kRow], cops[2 * kDB];
+            auto row_op = [&](int k) { return row_operand<kHD>(k & 1 ? vt : kt, lane, k >> 1); };
+            auto col_op = [&](int k) { return col_operand<kHD>(kt_lds, tr_base, k / kDB, k % kDB); };
 #pragma unroll
-            for (int ds = 0; ds < kHD / 16; ds++) {
-                s = Mma<T>::mma(row_operand<kHD>(kt, lane, ds), qreg[ds], s);
-                if ((ds & 3) == 3) __builtin_amdgcn_sched_barrier(0);
-            }
+            for (int k = 0; k < kAhead; k++) ops[k] = row_op(k);
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int ds = 0; ds < kHD / 16; ds++) {
-                dp = Mma<T>::mma(row_operand<kHD>(vt, lane, ds), greg[ds], dp);
-                if ((ds & 3) == 3) __builtin_amdgcn_sched_barrier(0);
+            for (int k = 0; k < 2 * kRow; k++) {
+                if (k + kAhead < 2 * kRow) ops[k + kAhead] = row_op(k + kAhead);
+                else cops[k + kAhead - 2 * kRow] = col_op(k + kAhead - 2 * kRow);
+                if (k & 1) dp = Mma<T>::mma(ops[k], greg[k >> 1], dp);
+                else s = Mma<T>::mma(ops[k], qreg[k >> 1], s);
+                __builtin_amdgcn_sched_barrier(0);
             }
             // A lane is a query: a row past the end spoils only its own accumulators, which are never stored, so
             // no element tests its row.  A cached block with every key visible tests nothing at all.
-            f32x16 dsv;
-            if (vis == 0xffffffffu && !chunk_part) {
-#pragma unroll
-                for (int i = 0; i < 16; i++) dsv[i] = __builtin_amdgcn_exp2f(fmaf(s[i], c2, nlse2)) * (dp[i] - delta) * a.scale;
-            } else {
-                // bit r of `allow`: key r of the block is visible to this lane's query
-                uint32_t allow = vis;
-                if (chunk_part) allow &= low_bits(r_cached) | low_bits(r_last + 1);
-                allow >>= 4 * h;  // element i looks at key 8 (i / 4) + 4 h + i % 4
-#pragma unroll
-                for (int i = 0; i < 16; i++) {
-                    const float pe = keep_if_bit(__builtin_amdgcn_exp2f(fmaf(s[i], c2, nlse2)), allow, 8 * (i / 4) + (i % 4));
+            auto products = [&](auto masked, uint32_t allow) {
+                f32x16 dsv;
+                auto element = [&](int i) {
+                    float pe = __builtin_amdgcn_exp2f(fmaf(s[i], c2, nlse2));
+                    if constexpr (decltype(masked)::value) pe = keep_if_bit(pe, allow, 8 * (i / 4) + (i % 4));
                     dsv[i] = pe * (dp[i] - delta) * a.scale;
-                }
-            }
-            const uint32_t kt_lds = lds0 + (uint32_t)(st * 2 * kTile);
+                };
 #pragma unroll
-            for (int s2 = 0; s2 < 2; s2++) {
-                const uint4 bop = pack8<T>(dsv, s2);
+                for (int i = 0; i < 8; i++) element(i);
+                uint4 bop = pack8<T>(dsv, 0);
+                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int db = 0; db < kHD / 32; db++) {
-                    dq[db] = Mma<T>::mma(col_operand<kHD>(kt_lds, tr_base, s2, db), bop, dq[db]);
-                    if (db & 1) __builtin_amdgcn_sched_barrier(0);
+                for (int k = 0; k < 2 * kDB; k++) {
+                    if (k + kAhead < 2 * kDB) cops[k + kAhead] = col_op(k + kAhead);
+                    dq[k % kDB] = Mma<T>::mma(cops[k], bop, dq[k % kDB]);
+                    if (k < kDB) {
+#pragma unroll
+                        for (int i = 8 + k * (8 / kDB); i < 8 + (k + 1) * (8 / kDB); i++) element(i);
+                    }
+                    if (k == kDB - 1) bop = pack8<T>(dsv, 1);
+                    __builtin_amdgcn_sched_barrier(0);
                 }
-            }
+            };
+            uint32_t allow = vis;
+            if (chunk_part) allow &= low_bits(r_cached) | low_bits(r_last + 1);
+            products(std::true_type{}, allow >> (4 * h));
         }
         __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wavefront's copies of the next block have landed
@@ -413,8 +443,9 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dkdv_kernel(BwdMfmaParam
     const int tid = threadIdx.x, wave = tid / CKV_WAVE, lane = tid % CKV_WAVE, h = lane >> 5;
     const Keys keys(p);
     const int64_t n_ctx = a.n_ctx, n_kv = a.n_kv, n_cached = keys.n_cached;
-    const int64_t bh = blockIdx.y, b = bh / a.H, hd = bh % a.H;
-    const int64_t n_wg = (int64_t)blockIdx.x * kOwn;
+    const Unit unit = unit_of(p);
+    const int64_t bh = unit.bh, b = bh / a.H, hd = bh % a.H;
+    const int64_t n_wg = (int64_t)unit.x * kOwn;
     const int64_t n_lane = n_wg + wave * 32 + (lane & 31);  // this lane's key
     const bool key_ok = keys.visible(n_lane);
     const char* qb = reinterpret_cast<const char*>(a.q) + (b * a.q_stride[0] + hd * a.q_stride[1]) * 2;
@@ -505,12 +536,23 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dkdv_kernel(BwdMfmaParam
             // bit r of `allow`: row r of the block sees this lane's key; element i looks at row 8 (i / 4) + 4 h + i % 4
             const uint32_t allow = (low_bits(r_hi) & ~low_bits(r_lo)) >> (4 * h);
             const uint32_t qt_lds = lds0 + (uint32_t)(st * 2 * kTile), gt_lds = qt_lds + kTile;
-            // The phases are fenced so that the compiler keeps their registers apart: P, then dV, then dP and dS, then dK.
+            // Phases P, dV, dP with dS, dK, each in issue order: an operand is read from LDS kKvAhead matrix instructions
+            // before the one that takes it, the first ones of a phase in the phase before (more than that, or dP beside the
+            // exponentials, does not fit the registers beside two 32 x 128 accumulators).
+            constexpr int kRow = kHD / 16, kDB = kHD / 32;
+            uint4 qops[kRow], gops[2 * kDB], rops[kRow], vops[kRow], cops[2 * kDB];
+            auto g_col = [&](int k) { return col_operand<kHD>(gt_lds, tr_base, k / kDB, k % kDB); };
+            auto q_col = [&](int k) { return col_operand<kHD>(qt_lds, tr_base, k / kDB, k % kDB); };
             f32x16 pv = zero16();
 #pragma unroll
-            for (int ds = 0; ds < kHD / 16; ds++) {
-                pv = Mma<T>::mma(row_operand<kHD>(qt, lane, ds), kreg[ds], pv);
-                if ((ds & 3) == 3) __builtin_amdgcn_sched_barrier(0);
+            for (int k = 0; k < kKvAhead; k++) qops[k] = row_operand<kHD>(qt, lane, k);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int k = 0; k < kRow; k++) {
+                if (k + kKvAhead < kRow) qops[k + kKvAhead] = row_operand<kHD>(qt, lane, k + kKvAhead);
+                else gops[k + kKvAhead - kRow] = g_col(k + kKvAhead - kRow);
+                pv = Mma<T>::mma(qops[k], kreg[k], pv);
+                __builtin_amdgcn_sched_barrier(0);
             }
 #pragma unroll
             for (int j = 0; j < 4; j++) {
@@ -525,19 +567,26 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dkdv_kernel(BwdMfmaParam
             }
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int s2 = 0; s2 < 2; s2++) {
-                const uint4 pb = pack8<T>(pv, s2);
-#pragma unroll
-                for (int db = 0; db < kHD / 32; db++) {
-                    dv[db] = Mma<T>::mma(col_operand<kHD>(gt_lds, tr_base, s2, db), pb, dv[db]);
-                    if (db & 1) __builtin_amdgcn_sched_barrier(0);
+            for (int k = 0; k < 2 * kDB; k++) {
+                if (k + kKvAhead < 2 * kDB) {
+                    gops[k + kKvAhead] = g_col(k + kKvAhead);
+                } else if (k == 2 * kDB - 1) {
+                    rops[0] = row_operand<kHD>(gt, lane, 0);
+                    vops[0] = vstat[lane];
                 }
+                dv[k % kDB] = Mma<T>::mma(gops[k], pack8<T>(pv, k / kDB), dv[k % kDB]);
+                __builtin_amdgcn_sched_barrier(0);
             }
             f32x16 dp = zero16();
 #pragma unroll
-            for (int ds = 0; ds < kHD / 16; ds++) {
-                dp = Mma<T>::mma(row_operand<kHD>(gt, lane, ds), vstat[ds * CKV_WAVE + lane], dp);
-                if (ds & 1) __builtin_amdgcn_sched_barrier(0);
+            for (int k = 0; k < kRow; k++) {
+                if (k + 1 < kRow) {
+                    rops[k + 1] = row_operand<kHD>(gt, lane, k + 1);
+                    vops[k + 1] = vstat[(k + 1) * CKV_WAVE + lane];
+                }
+                if (k >= kRow - kKvAhead) cops[k + kKvAhead - kRow] = q_col(k + kKvAhead - kRow);
+                dp = Mma<T>::mma(rops[k], vops[k], dp);
+                __builtin_amdgcn_sched_barrier(0);
             }
 #pragma unroll
             for (int j = 0; j < 4; j++) {
@@ -549,15 +598,13 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dkdv_kernel(BwdMfmaParam
                     dp[i] = pv[i] * (dp[i] - des[e]) * a.scale;
                 }
             }
+            const uint4 db_[2] = {pack8<T>(dp, 0), pack8<T>(dp, 1)};
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int s2 = 0; s2 < 2; s2++) {
-                const uint4 db_ = pack8<T>(dp, s2);
-#pragma unroll
-                for (int db = 0; db < kHD / 32; db++) {
-                    dk[db] = Mma<T>::mma(col_operand<kHD>(qt_lds, tr_base, s2, db), db_, dk[db]);
-                    if (db & 1) __builtin_amdgcn_sched_barrier(0);
-                }
+            for (int k = 0; k < 2 * kDB; k++) {
+                if (k + kKvAhead < 2 * kDB) cops[k + kKvAhead] = q_col(k + kKvAhead);
+                dk[k % kDB] = Mma<T>::mma(cops[k], db_[k / kDB], dk[k % kDB]);
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -594,10 +641,17 @@ inline bool rows_ok(const int64_t* st) {
 }
 
 template <typename T, int kHD>
-int run(const BwdMfmaParams& p, hipStream_t stream) {
+int run(const BwdMfmaParams& p_in, hipStream_t stream) {
+    BwdMfmaParams p = p_in;
     const ckv_dense_bwd_args& a = p.a;
-    hipLaunchKernelGGL((bwd_mfma_dq_kernel<T, kHD>), dim3((unsigned)((a.n_ctx + kOwn - 1) / kOwn * p.n_split), (unsigned)(a.B * a.H)),
-                       dim3(kThreads), 0, stream, p);
+    auto grid_of = [&](int64_t per_head, int64_t most) {
+        const int64_t heads = a.B * a.H;
+        const bool by_xcd = heads % 8 == 0 && heads * per_head <= most;
+        p.per_head = by_xcd ? (int)per_head : 0;
+        return by_xcd ? dim3((unsigned)(heads * per_head)) : dim3((unsigned)per_head, (unsigned)heads);
+    };
+    const dim3 grid_dq = grid_of((a.n_ctx + kOwn - 1) / kOwn * p.n_split, 0x7fffffff);
+    hipLaunchKernelGGL((bwd_mfma_dq_kernel<T, kHD>), grid_dq, dim3(kThreads), 0, stream, p);
     CKV_HIP_TRY(hipGetLastError());
     if (p.n_split > 1) {
         const int64_t threads = a.B * a.H * a.n_ctx * (kHD / 4);
@@ -606,8 +660,8 @@ int run(const BwdMfmaParams& p, hipStream_t stream) {
         CKV_HIP_TRY(hipGetLastError());
     }
     if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(bwd_mfma_dkdv_kernel<T, kHD>), Geo<kHD>::kDkdvLds)) return rc;
-    hipLaunchKernelGGL((bwd_mfma_dkdv_kernel<T, kHD>), dim3((unsigned)((a.n_kv + kOwn - 1) / kOwn), (unsigned)(a.B * a.H)),
-                       dim3(kThreads), Geo<kHD>::kDkdvLds, stream, p);
+    const dim3 grid_dkdv = grid_of((a.n_kv + kOwn - 1) / kOwn, 2 * (int64_t)mfma_device_cus());
+    hipLaunchKernelGGL((bwd_mfma_dkdv_kernel<T, kHD>), grid_dkdv, dim3(kThreads), Geo<kHD>::kDkdvLds, stream, p);
     CKV_HIP_TRY(hipGetLastError());
     return CKV_OK;
 }
@@ -641,6 +695,7 @@ int bwd_mfma_dq_splits(int64_t B, int64_t H, int64_t n_ctx, int64_t n_kv, int cu
 int launch_bwd_mfma(const ckv_dense_bwd_args& a, const float* delta, const int* key_order, const int* n_visible, float* part_dq,
                     int n_split, hipStream_t stream) {
     BwdMfmaParams p;
+    p.per_head = 0;
     p.part_dq = part_dq;
     p.n_split = part_dq ? n_split : 1;
     p.a = a;
