@@ -125,10 +125,6 @@ extern "C" int ckv_attn(const ckv_attn_args* args, void* stream_) {
     const bool want_scores = a.cache_s || a.new_scores;
     int rc;
     const bool use_mfma = mfma_supported(a.dtype, a.D, a.H, a.KVH, a.Q) && a.Q > 1 && mfma_fits(N, a.D);
-    if (want_scores && !use_mfma) {
-        rc = launch_weights(w.w_ema, w.w_new, a.Q, a.beta, a.dtype, stream);
-        if (rc) return rc;
-    }
     if (use_mfma) {
         MfmaProblem mp;
         mp.seg[0] = MfmaSegment{a.sink_k, a.sink_v, {a.sink_stride[0], a.sink_stride[1], a.sink_stride[2], a.sink_stride[3]},
@@ -167,7 +163,7 @@ extern "C" int ckv_attn(const ckv_attn_args* args, void* stream_) {
         rc = launch_mfma(mp, stream);
         if (rc) return rc;
     } else {
-        PrepProblem pp{&a, w.qr, w.kr, w.vc, w.kmasked};
+        PrepProblem pp{&a, w.qr, w.kr, w.vc, w.kmasked, want_scores ? w.w_ema : nullptr, w.w_new};
         rc = launch_prep_generic(pp, stream);
         if (rc) return rc;
 

@@ -59,6 +59,7 @@ struct PrepProblem {
     void* kr;        // (B, KVH, N, D) rotated keys, [sink | cache | chunk]
     void* vc;        // (B, KVH, N, D) values in the same order
     uint8_t* kmasked;  // (num_sink + S,)
+    float *w_ema, *w_new;  // the weights of the score sums, see launch_weights; null: none are wanted
 };
 int launch_prep_generic(const PrepProblem& p, hipStream_t stream);
 
