@@ -125,6 +125,19 @@ def test_single_token_calls(B, H, D, NS, W, C, dtype, func, eager, mode):
     run_stream(gpu, cpu, NS + 3 * W * C + 40, lambda: 1, gen, dtype, mode)
 
 
+@pytest.mark.parametrize("B,H", [(1, 7), (1, 8), (2, 4)])
+@pytest.mark.parametrize("W,C", [(33, 3), (16, 16), (64, 17), (16384, 1), (16386, 1)])
+def test_single_token_calls_around_the_one_launch_rule(B, H, W, C):
+    """A single token of few units takes the one-launch kernel from 8 units on, up to 16384 slots and 16 cascades: both
+    sides of each line, from the state a long chunk leaves, bit-exact against the oracle after every call."""
+    dtype = torch.bfloat16
+    gpu, cpu = make_pair(B, H, 8, 2, W, C, dtype)
+    gen = torch.Generator().manual_seed(H * W + C)
+    fill = min(W * C + 2, 2000)
+    lengths = iter([fill] + [1] * 12)
+    run_stream(gpu, cpu, fill + 12, lambda: next(lengths), gen, dtype, "ties")
+
+
 def test_call_larger_than_one_launch():
     """More tokens than one planning launch holds in LDS: the call is split internally."""
     gpu, cpu = make_pair(1, 2, 16, 4, 64, 4, torch.float32, eager=False)
