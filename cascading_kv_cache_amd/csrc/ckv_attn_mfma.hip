@@ -5,7 +5,7 @@
 //                tiles Vt[tile][d][key'] (key' = the order the PV MFMA consumes), build one 64-bit
 //                visibility word per key tile.  cos/sin are computed once per key and reused for
 //                every (batch, kv-head) that shares the position row.
-//   stage_q      rotate Q and fold the softmax scale (times log2 e) in.
+//   stage_q      rotate Q and, with 128 dims, fold the softmax scale (times log2 e) in.
 //   fwd          flash forward, software pipelined.  One workgroup = one kv head x 256 (head,
 //                position) rows, so the G query heads of a group share every K/V tile staged in
 //                LDS.  S^T = K Q^T keeps a query in one lane pair: the row max / sum need a single
@@ -16,9 +16,18 @@
 //                queries stream through LDS, the accumulators start from minus the final
 //                normaliser so the matrix pipe returns log2 P, and the weighted column sums stay
 //                inside a lane (S = Q K^T orientation).
+//
+// Precision.  With 128 dims the scale rides on the 16-bit queries and the probabilities enter P.V rounded to the tensor
+// dtype.  With 64 dims nothing but the operands themselves is held in 16 bits (kExact): the logits of the queries as the
+// eager path rounds them are scaled in float32, and a probability enters P.V as three 16-bit terms that add up to its
+// float32 value (one matrix instruction each, all into the same float32 accumulator), so the result is that of float32
+// arithmetic.  8 heads x 1000 rows x 5095 keys in float16: forward 20 -> 28 us, scores 31.5 -> 34 (the vector
+// kernels, to the same error: 2300 and 521); 32 heads on 8 kv heads, 4096 rows x 16 K slots, the whole call: 1.41 -> 2.02 ms
+// (59).  The vector ALU bounds the forward: seven instructions more per pair of probabilities.
 #include "ckv_attn_internal.h"
 
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <type_traits>
 
@@ -33,6 +42,9 @@ typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 
 // Kernels take the head dim as a template parameter kD: 64 or 128.
+template <int kD>
+constexpr bool kExact = kD == 64;
+constexpr float kLog2e = 1.4426950408889634f;
 constexpr int kBN = 64;    // keys per tile
 
 constexpr int kRows = 256;    // (head, position) rows per forward workgroup
@@ -138,6 +150,13 @@ __device__ __host__ inline int k_image_off(int r, int c) { return (c >> 1) * 204
 template <int kD>
 __device__ __host__ inline int v_image_off(int d, int c) { return (c >> 1) * (32 * kD) + (c & 1) * (16 * kD) + d * 16; }
 
+// cos / sin of a rotation angle before their rounding to the tensor dtype: where nothing else is rounded, to the last bit
+template <int kD>
+__device__ inline void stage_sincos(float x, float* sn, float* cs) {
+    if constexpr (kExact<kD>) sincosf(x, sn, cs);
+    else fast_sincos(x, sn, cs);
+}
+
 // One block of 256 threads stages key tile `tile_i` for the (b, kvh) units split_i, split_i + n_split, ...:
 // thread = (key = tid/4, quarter = tid%4) owns rotation pairs j = 8q .. 8q+7 (and, with 128 dims, 32+8q .. 32+8q+7),
 // i.e. the 16-byte pieces q, 4+q (, 8+q and 12+q) of its row: the four threads of a row read (and, for queries,
@@ -195,7 +214,7 @@ __device__ inline void stage_keys_block(const StageParams& p, int tile_i, int sp
             for (int e = 0; e < 2; e++) {
                 const int j = stage_pair(quarter, 2 * k + e);
                 const float f = p.inv_freq ? p.inv_freq[j] : 1.0f / powf(p.theta, (float)(2 * j) / (float)kD);
-                fast_sincos(__fmul_rn((float)pos, f), &sn[e], &cs[e]);
+                stage_sincos<kD>(__fmul_rn((float)pos, f), &sn[e], &cs[e]);
             }
             rw[k] = RopeWord<T>::make(cs[0], sn[0], cs[1], sn[1]);
         }
@@ -318,7 +337,8 @@ struct StageQParams {
     void* qr;                // (B*H, Q, D) contiguous
     int64_t rows;            // B*H*Q
     int64_t H, Q;
-    float qscale;            // folded into the staged queries: softmax scale * log2(e), over the factor the keys carry
+    float qscale;            // folded into the staged queries: softmax scale * log2(e), over the factor the keys carry; with
+                             // 64 dims the factor of the eager path, or the sign of the scale
     int vec;                 // source rows can be read 16 bytes at a time
 };
 
@@ -342,7 +362,7 @@ __device__ inline void stage_q_block(const StageQParams& p, int blk, int share_i
             for (int e = 0; e < 2; e++) {
                 const int j = stage_pair(quarter, 2 * k + e);
                 const float f = p.inv_freq ? p.inv_freq[j] : 1.0f / powf(p.theta, (float)(2 * j) / (float)kD);
-                fast_sincos(__fmul_rn((float)pos, f), &sn[e], &cs[e]);
+                stage_sincos<kD>(__fmul_rn((float)pos, f), &sn[e], &cs[e]);
             }
             rw[k] = RopeWord<T>::make(cs[0], sn[0], cs[1], sn[1]);
         }
@@ -369,7 +389,7 @@ __device__ inline void stage_q_block(const StageQParams& p, int blk, int share_i
             }
         }
     };
-    // the softmax scale (times log2 e) rides on the staged queries, so the attention kernels exponentiate the
+    // 128 dims: the softmax scale (times log2 e) rides on the staged queries, so the attention kernels exponentiate the
     // products as they come out of the matrix pipe: rotated with the eager path's roundings, then one rounding
     // of the product with qscale (the eager path rounds the product with sqrt(scale) there; log2 e has to ride
     // on one of the two operands, and noise on a query averages out over the rows a score sums)
@@ -442,7 +462,7 @@ struct FwdParams {
     float* lse2;      // (B*H, Q) minus the log2-domain normaliser, consumed by the column pass
     int64_t B, H, KVH, Q, N, Nc, n_pad;
     int G;            // heads per kv head: a workgroup takes 256 consecutive rows of the kv head's (position, head) pairs, position-major
-    float scale_log2; // softmax scale * log2(e)
+    float scale_log2; // with 64 dims: a logit's factor on its way to a power of two
     int n_qt, xcd_aware;  // query tiles per kv head; 1-D XCD-aware block order
     // Few query rows (short chunks, one stream) would leave most of the chip idle: the key tiles of a query tile
     // are then dealt out over n_split workgroups, each of which leaves a partial result (its rows normalised by
@@ -486,8 +506,11 @@ __global__ void __launch_bounds__(512) fwd_pipe_kernel(FwdParams p) {
     extern __shared__ __align__(16) unsigned char smem[];
     constexpr int kPipeStage = kD * 2 * kBN, kPipeLds = pipe_stages_lds(kD);
     constexpr int kThreads = 512, kBlocksPerWave = kPipeStage / 8192, kAhead = 3;
+    constexpr bool kEx = kExact<kD>;
+    constexpr int kTerms = kEx ? 3 : 1;                  // 16-bit terms of a probability
     constexpr int kDB = kD / 32, kKK = kD / 16;          // blocks of 32 dims; contraction steps of the logits
-    constexpr int kPvSlots = 4 * kDB, kQkSlots = 2 * kKK; // matrix instructions of a tile's two products
+    constexpr int kPvOps = 4 * kDB, kQkSlots = 2 * kKK;  // V^T pieces of a tile; matrix instructions of its logits
+    constexpr int kPvSlots = kPvOps * kTerms;            // matrix instructions of its P.V product
     const int Nc = p.n_visible ? *p.n_visible : (int)p.Nc;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -567,10 +590,15 @@ __global__ void __launch_bounds__(512) fwd_pipe_kernel(FwdParams p) {
     // m_ref: the reference the row's logits and sums are relative to; m_run: running maximum relative to it
     // (-inf until the row has seen a key); l_run: partial over this lane's keys, halves are added at the end
     float m_ref = 0.f, m_run = -INFINITY, l_run = 0.f;
-    f32x16 cinit;  // -m_ref in every element: what the matrix pipe starts a tile's logits from
+    f32x16 cinit;  // -m_ref in every element: what the matrix pipe starts a tile's logits from (64 dims: zero)
 #pragma unroll
     for (int v = 0; v < 16; v++) cinit[v] = 0.f;
-    constexpr float kShiftAt = 10.f;  // probabilities stay below 2^10 between two moves of the reference
+    // A row's largest probability lies at 2^kHead when its reference is set and stays below 2^kShiftAt until that moves.
+    // 64 dims: high enough that the terms of a probability 2^-26 times that size are float16 numbers of full precision.
+    constexpr float kShiftAt = kEx ? 15.f : 10.f, kHead = kEx ? 12.f : 0.f;
+    const float c2 = p.scale_log2;
+    // a logit as it leaves the matrix pipe, as a power of two
+    auto prob = [&](float x) { return __builtin_amdgcn_exp2f(kEx ? fmaf(x, c2, -m_ref) : x); };
 
     // ---- LDS byte offset of this lane's operand pieces inside the stage being read (pieces of later
     // contraction steps / row blocks are at compile-time distances); moved from stage to stage in place.
@@ -618,7 +646,23 @@ __global__ void __launch_bounds__(512) fwd_pipe_kernel(FwdParams p) {
             }
         }
     };
-    uint32_t pk[4][4];  // P^T of one tile as the B operands of the four P.V contraction steps
+    uint32_t pk[kTerms][4][4];  // P^T of one tile as the B operands of the four P.V contraction steps
+    // the probabilities q0, q1 as pair w of step st, and their sum (of what the product uses)
+    auto put_pair = [&](int st, int w, float q0, float q1, float sum) -> float {
+        uint32_t t = Mma<T>::pack2(q0, q1);
+        pk[0][st][w] = t;
+        if constexpr (!kEx) return Mma<T>::sum2(t, sum);
+        sum += q0 + q1;
+#pragma unroll
+        for (int i = 1; i < kTerms; i++) {
+            q0 -= Mma<T>::lo_f(t);
+            q1 -= Mma<T>::hi_f(t);
+            t = Mma<T>::pack2(q0, q1);
+            pk[i][st][w] = t;
+        }
+        return sum;
+    };
+    auto p_operand = [&](int term, int st) { return make_uint4(pk[term][st][0], pk[term][st][1], pk[term][st][2], pk[term][st][3]); };
     // O^T += V^T P^T with the V^T tile v_base points at
     auto pv = [&]() {
 #pragma unroll
@@ -626,8 +670,8 @@ __global__ void __launch_bounds__(512) fwd_pipe_kernel(FwdParams p) {
 #pragma unroll
             for (int dt = 0; dt < kDB; dt++) {
                 const uint4 a = v_piece(s, dt);
-                const uint4 bq = make_uint4(pk[s][0], pk[s][1], pk[s][2], pk[s][3]);
-                oacc[dt] = Mma<T>::mma(a, bq, oacc[dt]);
+#pragma unroll
+                for (int i = 0; i < kTerms; i++) oacc[dt] = Mma<T>::mma(a, p_operand(i, s), oacc[dt]);
             }
         }
     };
@@ -666,9 +710,10 @@ __global__ void __launch_bounds__(512) fwd_pipe_kernel(FwdParams p) {
         }
     };
 
-    // Iteration i, written in issue order: 32 slots (16 with 64 dims; the figures below are for 128), each one
-    // matrix instruction (slots 0..15: P.V of tile i-1 out of the V^T stage at v_base, slots 16..31: logits of
-    // tile i+1 out of the K stage at k_base), the LDS read of the operand kAhead slots ahead, and a slice of the softmax of tile i.
+    // Iteration i, written in issue order: 32 slots, each one matrix instruction (slots 0..15: P.V of tile i-1 out of the
+    // V^T stage at v_base, slots 16..31: logits of tile i+1 out of the K stage at k_base; with 64 dims 24 slots of P.V, three
+    // terms after another with each operand, and 8 of logits), the LDS read of the operand kAhead operands ahead, and a
+    // slice of the softmax of tile i.
     // Scheduling barriers keep the slots as written, so matrix and vector instructions alternate
     // inside the wavefront.  The probabilities of tile i overwrite those of tile i-1 piece by piece,
     // each after its last use by the P.V product.  The copies (V^T tile t_v = i+2 into stage v_wr, K
@@ -687,14 +732,15 @@ __global__ void __launch_bounds__(512) fwd_pipe_kernel(FwdParams p) {
         const int k_wr = k_rd == 0 ? kKStages - 1 : k_rd - 1;   // (k_rd + 2) % 3
         if (entry < 0) mask_tile(entry, s_cur);
         rescale();  // tile i-2 is in the accumulator; tile i-1, scaled for the newer reference, is added below
+        constexpr int kOps = (kPV ? kPvOps : 0) + kQkSlots, kQkOp0 = kPV ? kPvOps : 0;
         auto operand = [&](int k) -> uint4 {
-            if (k >= kQk0) {
-                const int j = k - kQk0;  // K piece (kk, ks) = (j % kKK, j / kKK): one 32-key block after the other
+            if (k >= kQkOp0) {
+                const int j = k - kQkOp0;  // K piece (kk, ks) = (j % kKK, j / kKK): one 32-key block after the other
                 return k_piece(j % kKK, j / kKK);
             }
             return v_piece(k / kDB, k % kDB);
         };
-        uint4 ops[kSlots];
+        uint4 ops[kOps];
         if (kPV) {
 #pragma unroll
             for (int k = 0; k < kAhead; k++) ops[k] = pre[k];
@@ -705,15 +751,19 @@ __global__ void __launch_bounds__(512) fwd_pipe_kernel(FwdParams p) {
         // pair of probabilities per slot: the first 32-key block of the tile is consumed by slot 15 and the
         // second by slot 23, just before the matrix pipe starts to overwrite them with the next tile's
         // logits (slots 16..23 and 24..31), so one set of logit registers serves both tiles.
-        constexpr int kMaxSlots = kPV ? kPvSlots / 2 : kQkSlots / 4;  // slots with running maxima
+        // Three terms: maxima in slots 0..7, probabilities in slots 12..27, so that a pair is stored (slots 13..28) after
+        // the last of the six slots that use the one before it (step st: slots 6 st .. 6 st + 5).
+        constexpr int kMaxSlots = kPV ? (kEx ? 8 : kPvSlots / 2) : kQkSlots / 4;  // slots with running maxima
         constexpr int kMaxPer = 32 / kMaxSlots;            // logits per such slot
-        constexpr int kExpFirst = kMaxSlots;               // first slot with probabilities
-        constexpr int kExpPer = 16 / (kPV ? kPvSlots : kQkSlots / 2);  // pairs per slot
+        constexpr int kExpFirst = kPV && kEx ? kPvSlots / 2 : kMaxSlots;  // first slot with probabilities
+        constexpr int kExpPer = kPV && kEx ? 1 : 16 / (kPV ? kPvSlots : kQkSlots / 2);  // pairs per slot
+        static_assert(kExpFirst + 16 / kExpPer < kSlots, "the last pair is stored a slot after its exponentials");
         float q0[kExpPer], q1[kExpPer];                    // exponentials of the previous slot, packed one slot later
         int raw_entry = 0;
         bool moved = true;                                 // some row of the wavefront takes a new reference
         auto slot = [&](int k) {
-            if (kPV && k + kAhead < kSlots) ops[k + kAhead] = operand(k + kAhead);
+            const int op = kPV && k < kQk0 ? k / kTerms : kQkOp0 + k - kQk0;
+            if (kPV && op + kAhead < kOps && (k >= kQk0 || k % kTerms == 0)) ops[op + kAhead] = operand(op + kAhead);
             if (k % kCopyStep == 1) {
                 const int q = k / kCopyStep;               // the V^T blocks, then the K blocks
                 if (q < kBlocksPerWave) copy_v(t_v, v_wr, q);
@@ -724,11 +774,10 @@ __global__ void __launch_bounds__(512) fwd_pipe_kernel(FwdParams p) {
                 // the first iteration of a workgroup: the next tile's logits follow the slots (below)
             } else if (k >= kQk0) {
                 const int j = k - kQk0;
-                s_nxt[j / kKK] = Mma<T>::mma(ops[k], qreg[j % kKK], j % kKK == 0 ? cinit : s_nxt[j / kKK]);
+                s_nxt[j / kKK] = Mma<T>::mma(ops[op], qreg[j % kKK], j % kKK == 0 ? cinit : s_nxt[j / kKK]);
             } else {
-                const int st = k / kDB, dt = k % kDB;
-                const uint4 bq = make_uint4(pk[st][0], pk[st][1], pk[st][2], pk[st][3]);
-                oacc[dt] = Mma<T>::mma(ops[k], bq, oacc[dt]);
+                const int st = op / kDB, dt = op % kDB;
+                oacc[dt] = Mma<T>::mma(ops[op], p_operand(k % kTerms, st), oacc[dt]);
             }
             if (k < kMaxSlots) {
 #pragma unroll
@@ -743,11 +792,12 @@ __global__ void __launch_bounds__(512) fwd_pipe_kernel(FwdParams p) {
                     // first visible key of a row; until then a probability is a bare exponential.
                     float m = fmaxf(fmaxf(mx[0], mx[1]), fmaxf(mx[2], mx[3]));
                     m = half_max(m);
+                    if constexpr (kEx) m = fmaf(m, c2, -m_ref);
                     const float m_new = fmaxf(m_run, m);
                     const bool first = m_run == -INFINITY && m != -INFINITY;
                     const bool sh = first || m_new > kShiftAt;
                     moved = __builtin_amdgcn_ballot_w64(sh) != 0ull;
-                    shift = sh ? m_new : 0.f;
+                    shift = sh ? m_new - kHead : 0.f;
                     alpha = sh ? (first ? 0.f : __builtin_amdgcn_exp2f(-shift)) : 1.f;
                     m_run = m_new - shift;
                     m_ref += shift;
@@ -758,15 +808,13 @@ __global__ void __launch_bounds__(512) fwd_pipe_kernel(FwdParams p) {
                     const int prev = (k - 1 - kExpFirst) * kExpPer + r;  // pair computed one slot ago
                     if (prev >= 0 && prev < 16) {
                         const int ks = prev >> 3, v = 2 * (prev & 7);
-                        const uint32_t w = Mma<T>::pack2(q0[r], q1[r]);
-                        rs = Mma<T>::sum2(w, rs);              // the row sum takes the rounded values the product uses
-                        pk[2 * ks + (v >> 3)][(v & 7) >> 1] = w;
+                        rs = put_pair(2 * ks + (v >> 3), (v & 7) >> 1, q0[r], q1[r], rs);
                     }
                     const int pair = (k - kExpFirst) * kExpPer + r;      // (ks, v) = (pair / 8, 2 * (pair % 8))
                     if (pair < 16) {
                         const int ks = pair >> 3, v = 2 * (pair & 7);
-                        q0[r] = __builtin_amdgcn_exp2f(s_cur[ks][v]);
-                        q1[r] = __builtin_amdgcn_exp2f(s_cur[ks][v + 1]);
+                        q0[r] = prob(s_cur[ks][v]);
+                        q1[r] = prob(s_cur[ks][v + 1]);
                     }
                 }
             }
@@ -774,7 +822,7 @@ __global__ void __launch_bounds__(512) fwd_pipe_kernel(FwdParams p) {
         };
 #pragma unroll
         for (int k = 0; k < kMaxSlots; k++) slot(k);
-        if (moved) {
+        if (!kEx && moved) {
             // rare after the first tiles: this tile's logits come down to the new reference here, the later
             // ones through the accumulator initialisation
 #pragma unroll
@@ -797,7 +845,12 @@ __global__ void __launch_bounds__(512) fwd_pipe_kernel(FwdParams p) {
         for (int k = 0; k < kAhead; k++) pre[k] = v_piece(k / kDB, k % kDB);
         // keep the packed probabilities in this region (they are next read after the barrier)
 #pragma unroll
-        for (int st = 0; st < 4; st++) asm volatile("" ::"v"(pk[st][0]), "v"(pk[st][1]), "v"(pk[st][2]), "v"(pk[st][3]));
+        for (int i = 0; i < kTerms; i++)
+#pragma unroll
+            for (int st = 0; st < 4; st++) {
+                const uint4 w = p_operand(i, st);
+                asm volatile("" ::"v"(w.x), "v"(w.y), "v"(w.z), "v"(w.w));
+            }
     };
 
     f32x16 sA[2], sB[2];
@@ -985,7 +1038,7 @@ struct ColsumParams {
     int64_t B, H, KVH, Q, N, Nc, n_pad;
     int G;
     int new_mode;
-    float scale_log2;
+    float scale_log2;     // as in FwdParams
     int nkb, nbkv, xcd_aware, gsplit;  // block order and head split, see the kernel
     const int* n_visible; // when the keys were staged in key order: the number of cached keys (null: Nc), and the
     const int* key_order; // row each key came from
@@ -1142,9 +1195,10 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
         const float* lse_lds = reinterpret_cast<const float*>(q_lds + kQT2 * kRowBytes);
         const float* w_lds = lse_lds + kQT2;
         // Accumulators start from minus the row normaliser, so the matrix pipe hands back log2 P (the
-        // softmax scale is already on the staged queries).  Element (c, v) of a 32-row subtile c:
+        // softmax scale is already on the staged queries); with 64 dims they start from zero, and the scale and the
+        // normaliser join in float32 (`nl`: the subtile's normalisers).  Element (c, v) of a 32-row subtile c:
         // query row mt + 32c + 8(v/4) + 4half + v%4, key column of this lane.
-        auto row_init = [&](int c) {
+        auto row_norms = [&](int c) {
             f32x16 init;
 #pragma unroll
             for (int v4 = 0; v4 < 4; v4++) {
@@ -1155,6 +1209,21 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
                 init[4 * v4 + 3] = l4.w;
             }
             return init;
+        };
+        auto row_init = [&](int c) {
+            if constexpr (!kExact<kD>) return row_norms(c);
+            f32x16 z;
+#pragma unroll
+            for (int v = 0; v < 16; v++) z[v] = 0.f;
+            return z;
+        };
+        auto norms_of = [&](int c) {
+            if constexpr (kExact<kD>) return row_norms(c);
+            else return 0;
+        };
+        auto prob = [&](float x, const auto& nl, int v) {
+            if constexpr (kExact<kD>) return __builtin_amdgcn_exp2f(fmaf(x, p.scale_log2, nl[v]));
+            else return __builtin_amdgcn_exp2f(x);
         };
         auto load_weights = [&](int c, float(&ws)[16]) {
 #pragma unroll
@@ -1184,6 +1253,7 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
                 for (int kk = 0; kk < kKK; kk++) a1[kk] = *reinterpret_cast<const uint4*>(q_lds + q_off[kk] + c * (32 * kRowBytes));
                 float ws[16];
                 load_weights(c - 1, ws);
+                const auto nl = norms_of(c - 1);
                 __builtin_amdgcn_sched_barrier(0);
                 // an exponential is consumed one slot after it was issued, so no wavefront waits for the
                 // transcendental unit
@@ -1197,7 +1267,7 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
 #pragma unroll
                     for (int r = 0; r < kPer; r++) {
                         const int j = kPer * slot + r, ksv = j >> 4, v = j & 15;
-                        pe[r] = __builtin_amdgcn_exp2f(sq[(c - 1) & 1][ksv][v]);
+                        pe[r] = prob(sq[(c - 1) & 1][ksv][v], nl, v);
                     }
                     if (slot > 0) {
 #pragma unroll
@@ -1219,11 +1289,12 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
             {
                 float ws[16];
                 load_weights(kCsSub - 1, ws);
+                const auto nl = norms_of(kCsSub - 1);
 #pragma unroll
                 for (int v = 0; v < 16; v++) {
 #pragma unroll
                     for (int ks = 0; ks < 2; ks++) {
-                        const float pe = __builtin_amdgcn_exp2f(sq[(kCsSub - 1) & 1][ks][v]);
+                        const float pe = prob(sq[(kCsSub - 1) & 1][ks][v], nl, v);
                         acc[ks] = fmaf(ws[v], pe, acc[ks]);
                     }
                 }
@@ -1248,6 +1319,7 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
                 const bool fast_new = plain && new_chunk;
                 f32x16 sacc[2];
                 sacc[0] = sacc[1] = row_init(c);
+                const auto nl = norms_of(c);
 #pragma unroll
                 for (int kk = 0; kk < kKK; kk++) {
                     const uint4 a = *reinterpret_cast<const uint4*>(q_lds + q_off[kk] + c * (32 * kRowBytes));
@@ -1263,8 +1335,7 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
                     for (int v = 0; v < 16; v += 2) {
 #pragma unroll
                         for (int ks = 0; ks < 2; ks++) {
-                            const uint32_t u = Mma<T>::pack2(__builtin_amdgcn_exp2f(sacc[ks][v]),
-                                                             __builtin_amdgcn_exp2f(sacc[ks][v + 1]));
+                            const uint32_t u = Mma<T>::pack2(prob(sacc[ks][v], nl, v), prob(sacc[ks][v + 1], nl, v + 1));
                             acc[ks] = Mma<T>::sum2(Mma<T>::pack2(Mma<T>::lo_f(u) * wu, Mma<T>::hi_f(u) * wu), acc[ks]);
                         }
                     }
@@ -1277,7 +1348,7 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
                         for (int e = 0; e < 4; e++) {
 #pragma unroll
                             for (int ks = 0; ks < 2; ks++) {
-                                const float pe = __builtin_amdgcn_exp2f(sacc[ks][4 * v4 + e]);
+                                const float pe = prob(sacc[ks][4 * v4 + e], nl, 4 * v4 + e);
                                 const float w = weight_of(ks, r0 + e);
                                 if (pure_chunk) {
                                     acc[ks] += Mma<T>::round1(Mma<T>::round1(pe) * w);
@@ -1297,7 +1368,7 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
                         const float we = w_lds[r];
 #pragma unroll
                         for (int ks = 0; ks < 2; ks++) {
-                            float pe = __builtin_amdgcn_exp2f(sacc[ks][v]);
+                            float pe = prob(sacc[ks][v], nl, v);
                             const bool is_chunk = nrel[ks] >= 0;
                             const bool vis = row_in && (!is_chunk || m >= nrel[ks]);
                             pe = vis ? pe : 0.f;
@@ -1378,7 +1449,15 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
 template <typename T, int kD>
 int run_mfma(const MfmaProblem& mp, hipStream_t stream) {
     const int64_t n = mp.n, n_pad = mp.n_pad;
-    const float scale_log2 = mp.scale * 1.4426950408889634f;
+    // what the staged queries are multiplied by, and the factor the kernels are left with.  Rotated keys carry key_scale.
+    // 64 dims: rotated queries carry the same (the eager path's sqrt(scale)); those that arrive rotated stay as they are but
+    // for the sign, so that the largest product is the largest logit.
+    const float scale_log2 = mp.scale * kLog2e;
+    float qscale = mp.q_pos ? scale_log2 / mp.key_scale : scale_log2, left = 1.f;
+    if (kExact<kD>) {
+        qscale = mp.q_pos ? mp.key_scale : mp.scale < 0.f ? -1.f : mp.scale == 0.f ? 0.f : 1.f;
+        left = mp.q_pos || mp.scale == 0.f ? kLog2e : fabsf(scale_log2);
+    }
     const int cus = mfma_device_cus();
     {
         StageScope sc(CKV_STAGE_PREP, stream);
@@ -1424,7 +1503,7 @@ int run_mfma(const MfmaProblem& mp, hipStream_t stream) {
         sq.qr = mp.qr;
         sq.rows = mp.B * mp.H * mp.Q;
         sq.H = mp.H; sq.Q = mp.Q;
-        sq.qscale = mp.q_pos ? scale_log2 / mp.key_scale : scale_log2;  // rotated keys carry key_scale
+        sq.qscale = qscale;
         sq.vec = mp.q_stride[3] == 1 && reinterpret_cast<uintptr_t>(mp.q) % 16 == 0 && mp.q_stride[0] % 8 == 0 &&
                  mp.q_stride[1] % 8 == 0 && mp.q_stride[2] % 8 == 0;
         {
@@ -1455,7 +1534,7 @@ int run_mfma(const MfmaProblem& mp, hipStream_t stream) {
         fp.lse2 = mp.lse2;
         fp.B = mp.B; fp.H = mp.H; fp.KVH = mp.KVH; fp.Q = mp.Q; fp.N = n; fp.Nc = n - mp.Q; fp.n_pad = n_pad;
         fp.G = G;
-        fp.scale_log2 = 1.f;  // already on the staged queries
+        fp.scale_log2 = left;
         fp.n_qt = (int)((mp.Q * G + kRows - 1) / kRows);
         fp.n_split = mfma_fwd_splits(mp.B, mp.H, mp.KVH, mp.Q, n, cus, mp.empty_to > mp.empty_from);
         fp.part_o = mp.part_o;
@@ -1506,7 +1585,7 @@ int run_mfma(const MfmaProblem& mp, hipStream_t stream) {
             cp.wnew_uniform = round_t_host((float)mp.beta) == 1.0f ? 1 : 0;
             cp.wnew_value = round_t_host((float)(1.0 - mp.beta));
         }
-        cp.scale_log2 = 1.f;  // already on the staged queries
+        cp.scale_log2 = left;
         cp.nkb = (int)((n + 255) / 256);
         cp.nbkv = (int)(mp.B * mp.KVH);
         cp.xcd_aware = cp.nbkv % 8 == 0;

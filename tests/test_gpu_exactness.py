@@ -1,0 +1,112 @@
+"""What the fp32-math paths owe float64 arithmetic on the same inputs.
+
+Head size 64 in the 16-bit formats holds logits, probabilities and every sum in 32 bits: a result is the exact one
+rounded once to the tensor dtype, up to the noise of its float32 sums.
+
+Cached keys are rotated; with ``inv_freq`` zero the rotation is the identity, so that the staged operands are known to
+the bit: queries and keys times sqrt(softmax scale), rounded to the tensor dtype (cascade_attention.py:284-291).
+"""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+F16, BF16, F32 = torch.float16, torch.bfloat16, torch.float32
+HALF_ULP = {BF16: 2.0 ** -8, F16: 2.0 ** -11, F32: 2.0 ** -24}   # relative, at the bottom of a binade
+
+
+def assert_rounded_once(got, exact, spread, n, what):
+    """``got`` is ``exact`` rounded to its dtype behind float32 sums of ``n`` terms, ``spread`` being the root of the sum
+    of their squares.  Half a unit in the last place; a float32 chain over n random terms is off by about
+    2^-24 sqrt(n) spread and a term itself (a logit of a few units, its exponential) by 2^-22 or so: eight times their
+    sum; what a whole row shares (its normaliser, rounded at a magnitude of ten) by 2^-20 of the result; half the
+    smallest float16 number."""
+    bound = (HALF_ULP[got.dtype] + 2.0 ** -20) * exact.abs() + 2.0 ** -21 * math.sqrt(n) * spread
+    bound = bound + (2.0 ** -25 if got.dtype == F16 else 1e-30)
+    excess = ((got.double() - exact).abs() / bound).max().item()
+    assert excess <= 1.0, f"{what}: {excess:.2f} times the bound"
+
+
+def visible(n_ctx, n_kv, mask):
+    """(n_ctx, n_kv): which key a row sees."""
+    causal = torch.ones(n_ctx, n_ctx, dtype=torch.bool, device=mask.device).tril()
+    return torch.cat((~mask[None, :].expand(n_ctx, -1), causal), dim=-1)
+
+
+def exact_attention(q, k, v, see, scale):
+    """out, P, row normalisers and the spread of out, in float64 (every head its own kv head)."""
+    s = torch.matmul(q.double(), k.double().transpose(2, 3).contiguous()) * scale
+    s = s.masked_fill(~see, float("-inf"))
+    p = torch.softmax(s, dim=-1)
+    vd = v.double()
+    return torch.matmul(p, vd), p, torch.logsumexp(s, dim=-1), torch.matmul(p * p, vd * vd).sqrt()
+
+
+DENSE = [(1, 2, 128, 128), (1, 3, 33, 1 + 33), (2, 4, 200, 1000 + 200), (1, 2, 500, 2048 + 64 + 500), (1, 1, 700, 5000 + 700)]
+
+
+def dense_case(Z, H, n_ctx, n_kv, D, dtype, std=0.7):
+    g = torch.Generator(device="cuda").manual_seed(100 + n_kv)
+    q, k, v = ((torch.randn(Z, n, H, D, device="cuda", generator=g) * std).to(dtype).transpose(1, 2) for n in (n_ctx, n_kv, n_kv))
+    mask = torch.rand(n_kv - n_ctx, device="cuda", generator=g) > 0.5
+    return q, k, v, mask, torch.randn(Z, H, n_ctx, D, device="cuda", generator=g).to(dtype)
+
+
+@pytest.mark.parametrize("dtype", [BF16, F16])
+@pytest.mark.parametrize("Z,H,n_ctx,n_kv", DENSE)
+def test_dense_forward_of_head_size_64_is_rounded_once(Z, H, n_ctx, n_kv, dtype):
+    from cascading_kv_cache_amd import flash_attention as fa
+
+    q, k, v, mask, _ = dense_case(Z, H, n_ctx, n_kv, 64, dtype)
+    out, scores, lse, _ = fa._forward(q, k, v, True, 0.5, mask, 0.9, True)
+    ref, p, ref_lse, spread = exact_attention(q, k, v, visible(n_ctx, n_kv, mask), 0.5)
+    assert (lse.double() - ref_lse).abs().max().item() <= 4e-6      # float32 logits and sums, normalisers of up to ten
+    assert_rounded_once(out, ref, spread, n_kv, "out")
+    w = (0.1 * 0.9 ** torch.arange(n_ctx - 1, -1, -1, device="cuda", dtype=torch.float64))[None, None, :, None]
+    assert_rounded_once(scores, (w * p).sum(2), (w * p).square().sum(2).sqrt(), n_ctx, "scores")
+
+
+def one_layer(B, KVH, D, NS, W, C, dtype):
+    from cascading_kv_cache_amd.cascading_cache import CascadingKVCache
+
+    return CascadingKVCache(window_length=W, num_sink_tokens=NS, max_batch_size=B, heads=KVH, dim=D, max_seq_len=W * C,
+                            device="cuda:0", dtype=dtype, layers=1, verbose=False)
+
+
+def cascade_case(B, H, KVH, D, NS, W, C, filled, Q, dtype, std=0.7):
+    """A cache that holds ``filled`` random tokens, and a chunk; no rotation (inv_freq zero)."""
+    g = torch.Generator(device="cuda").manual_seed(7)
+    cache = one_layer(B, KVH, D, NS, W, C, dtype)
+    rows = lambda h, n: (torch.randn(B, n, h, D, device="cuda", generator=g) * std).to(dtype).transpose(1, 2)
+    if filled:
+        cache.update(rows(KVH, filled), rows(KVH, filled), 0, torch.rand(B, KVH, filled, device="cuda", generator=g).to(dtype))
+    return cache, rows(H, Q), rows(KVH, Q), rows(KVH, Q), torch.zeros(D // 2, device="cuda")
+
+
+def staged(cache, q, k, v):
+    """The operands as the kernels stage them, expanded to the query heads, and the mask of the cached keys."""
+    G, rs = q.size(1) // k.size(1), math.sqrt(1 / math.sqrt(q.size(-1)))
+    scaled = lambda t: (t.float() * rs).to(t.dtype)
+    keys = torch.cat((cache.sink_keys[0], cache.key_cache[0], k), dim=2)
+    vals = torch.cat((cache.sink_values[0], cache.value_cache[0], v), dim=2)
+    mask = torch.cat((cache.sink_mask[0].reshape(-1, cache.sink_keys[0].size(2))[0], cache.mask[0].reshape(-1, cache.key_cache[0].size(2))[0]))
+    return scaled(q), scaled(keys).repeat_interleave(G, 1), vals.repeat_interleave(G, 1), mask.bool()
+
+
+CASCADE = [
+    # B, H, KVH, D, NS, W, C, filled, Q, dtype
+    (1, 8, 2, 64, 4, 64, 4, 1000, 96, BF16), (2, 14, 2, 64, 4, 128, 2, 200, 77, F16), (1, 3, 3, 64, 64, 256, 8, 4000, 300, BF16),
+]
+
+
+@pytest.mark.parametrize("B,H,KVH,D,NS,W,C,filled,Q,dtype", CASCADE)
+def test_cascade_forward_is_rounded_once(B, H, KVH, D, NS, W, C, filled, Q, dtype):
+    from cascading_kv_cache_amd.cascade_attention import cascade_attention
+
+    cache, q, k, v, inv_freq = cascade_case(B, H, KVH, D, NS, W, C, filled, Q, dtype)
+    qs, ks, vs, mask = staged(cache, q, k, v)
+    ref, p, _, spread = exact_attention(qs, ks, vs, visible(Q, ks.size(2), mask), 1.0)
+    out, _ = cascade_attention(q, k, v, cache, 0, inv_freq, update_cache=False)
+    assert_rounded_once(out, ref, spread, ks.size(2), "out")
