@@ -10,6 +10,15 @@
 //          S = Q K^T and dP = dO V^T keep a key in one lane; P and dS are the B operands of
 //          dV^T += dO^T P and dK^T += Q^T dS.
 //
+// Precision.  With 128 dims P and dS enter those products rounded to the tensor dtype.  With 64 dims they stay float32:
+// the products run on v_mfma_f32_32x32x2, whose B operand is an accumulator register as it stands and whose A operand is
+// the same transposed read, widened to float32.  16-bit terms that add up to the float32 value, as the forward kernel takes,
+// would need a scale of their own for dS, which has no largest value, and would turn an infinite gradient into NaN.
+// 8 heads x 1000 rows x 5095 keys in float16: dq 32 -> 61 us, dk/dv 40 -> 101 (the vector kernels, to the same error: 2520
+// and 1838).  These products bound both kernels: 2048 and 4096 of the 2304 and 4352 cycles of matrix work per 32 x 32 block,
+// and unlike the 16-bit instructions they do not run beside vector instructions (matrix pipe 43 and 50 % busy, 0 % of the
+// time together with the vector ALU).
+//
 // The A operands K^T, Q^T and dO^T are read from the row-major tiles in LDS with the transposing read
 // ds_read_b64_tr_b16: lane i of a 16-lane group receives element [4e + i/4][i%4] (e = 0..3) of the 16 x 4 matrix
 // whose row r is the 8 bytes lane r points at; with lane r pointing at dims 4 (r%4) .. +3 of row r/4 of a
@@ -64,6 +73,9 @@ struct Mma<__hip_bfloat16> {
         f32x2 f = {lo, hi};
         return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, bf16x2));
     }
+    // the two elements of a packed pair as floats
+    __device__ static float lo_f(uint32_t w) { return __uint_as_float(w << 16); }
+    __device__ static float hi_f(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
 };
 template <>
 struct Mma<__half> {
@@ -75,6 +87,8 @@ struct Mma<__half> {
         f32x2 f = {lo, hi};
         return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, f16x2));
     }
+    __device__ static float lo_f(uint32_t w) { return (float)__builtin_bit_cast(f16x2, w)[0]; }
+    __device__ static float hi_f(uint32_t w) { return (float)__builtin_bit_cast(f16x2, w)[1]; }
 };
 
 struct BwdMfmaParams {
@@ -209,6 +223,47 @@ __device__ inline uint4 pack8(const f32x16& v, int s) {
     return make_uint4(Mma<T>::pack2(v[8 * s + 0], v[8 * s + 1]), Mma<T>::pack2(v[8 * s + 2], v[8 * s + 3]),
                       Mma<T>::pack2(v[8 * s + 4], v[8 * s + 5]), Mma<T>::pack2(v[8 * s + 6], v[8 * s + 7]));
 }
+
+// The B operand of the two products that contract over a block's 32 rows, element 8 s + i of `v` belonging to step s: packed
+// in the tensor dtype (128 dims) or as it is, and the product of a step with the A operand of col_operand.  Element 4 a + e
+// of that holds rows 16 s + 8 a + 4 (lane/32) + e, the row of accumulator register 8 s + 4 a + e in the same lane half.
+// `accumulate` is matrix instruction k of such a product, step k / kDB into accumulator k % kDB with A operand ops[k]; with
+// 64 dims the first one of a step brings the step's float32 instructions, the two accumulators in turn (both operands are
+// there: they are read at least two ahead), all operands widened first (dk/dv 101 us; one before each instruction 113).
+template <typename T, int kHD>
+struct Weights {
+    static constexpr int kDB = kHD / 32;
+    uint4 w[2];
+    __device__ void set(const f32x16& v, int s) { w[s] = pack8<T>(v, s); }
+    __device__ void accumulate(const uint4 (&ops)[2 * kDB], int k, f32x16 (&c)[kDB]) const { c[k % kDB] = Mma<T>::mma(ops[k], w[k / kDB], c[k % kDB]); }
+    __device__ static void accumulate(const uint4 (&ops)[2 * kDB], const f32x16& v, int k, f32x16 (&c)[kDB]) {
+        c[k % kDB] = Mma<T>::mma(ops[k], pack8<T>(v, k / kDB), c[k % kDB]);
+    }
+};
+template <typename T>
+struct Weights<T, 64> {
+    f32x16 w;
+    __device__ void set(const f32x16& v, int s) {
+#pragma unroll
+        for (int i = 8 * s; i < 8 * s + 8; i++) w[i] = v[i];
+    }
+    __device__ void accumulate(const uint4 (&ops)[4], int k, f32x16 (&c)[2]) const { accumulate(ops, w, k, c); }
+    __device__ static void accumulate(const uint4 (&ops)[4], const f32x16& v, int k, f32x16 (&c)[2]) {
+        if (k % 2 != 0) return;
+        float a[2][8];
+#pragma unroll
+        for (int db = 0; db < 2; db++) {
+            const uint32_t p[4] = {ops[k + db].x, ops[k + db].y, ops[k + db].z, ops[k + db].w};
+#pragma unroll
+            for (int i = 0; i < 8; i++) a[db][i] = i & 1 ? Mma<T>::hi_f(p[i >> 1]) : Mma<T>::lo_f(p[i >> 1]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+#pragma unroll
+            for (int db = 0; db < 2; db++) c[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[db][i], v[8 * (k / 2) + i], c[db], 0, 0, 0);
+    }
+};
 
 // bits [0, n) set, for 0 <= n <= 32
 __device__ inline uint32_t low_bits(int n) { return n >= 32 ? 0xffffffffu : ((1u << n) - 1u); }
@@ -363,17 +418,18 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dq_kernel(BwdMfmaParams 
                 };
 #pragma unroll
                 for (int i = 0; i < 8; i++) element(i);
-                uint4 bop = pack8<T>(dsv, 0);
+                Weights<T, kHD> bop;
+                bop.set(dsv, 0);
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int k = 0; k < 2 * kDB; k++) {
                     if (k + kAhead < 2 * kDB) cops[k + kAhead] = col_op(k + kAhead);
-                    dq[k % kDB] = Mma<T>::mma(cops[k], bop, dq[k % kDB]);
+                    bop.accumulate(cops, k, dq);
                     if (k < kDB) {
 #pragma unroll
                         for (int i = 8 + k * (8 / kDB); i < 8 + (k + 1) * (8 / kDB); i++) element(i);
                     }
-                    if (k == kDB - 1) bop = pack8<T>(dsv, 1);
+                    if (k == kDB - 1) bop.set(dsv, 1);
                     __builtin_amdgcn_sched_barrier(0);
                 }
             };
@@ -574,7 +630,7 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dkdv_kernel(BwdMfmaParam
                     rops[0] = row_operand<kHD>(gt, lane, 0);
                     vops[0] = vstat[lane];
                 }
-                dv[k % kDB] = Mma<T>::mma(gops[k], pack8<T>(pv, k / kDB), dv[k % kDB]);
+                Weights<T, kHD>::accumulate(gops, pv, k, dv);
                 __builtin_amdgcn_sched_barrier(0);
             }
             f32x16 dp = zero16();
@@ -598,12 +654,14 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dkdv_kernel(BwdMfmaParam
                     dp[i] = pv[i] * (dp[i] - des[e]) * a.scale;
                 }
             }
-            const uint4 db_[2] = {pack8<T>(dp, 0), pack8<T>(dp, 1)};
+            Weights<T, kHD> dw;
+            dw.set(dp, 0);
+            dw.set(dp, 1);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int k = 0; k < 2 * kDB; k++) {
                 if (k + kKvAhead < 2 * kDB) cops[k + kKvAhead] = q_col(k + kKvAhead);
-                dk[k % kDB] = Mma<T>::mma(cops[k], db_[k / kDB], dk[k % kDB]);
+                dw.accumulate(cops, k, dk);
                 __builtin_amdgcn_sched_barrier(0);
             }
         }

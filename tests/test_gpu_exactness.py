@@ -1,7 +1,7 @@
 """What the fp32-math paths owe float64 arithmetic on the same inputs.
 
-Head size 64 in the 16-bit formats holds logits, probabilities and every sum in 32 bits: a result is the exact one
-rounded once to the tensor dtype, up to the noise of its float32 sums.
+Head size 64 in the 16-bit formats holds logits, probabilities, dS and every sum in 32 bits: a result is the exact
+one rounded once to the tensor dtype, up to the noise of its float32 sums.
 
 Cached keys are rotated; with ``inv_freq`` zero the rotation is the identity, so that the staged operands are known to
 the bit: queries and keys times sqrt(softmax scale), rounded to the tensor dtype (cascade_attention.py:284-291).
@@ -66,6 +66,31 @@ def test_dense_forward_of_head_size_64_is_rounded_once(Z, H, n_ctx, n_kv, dtype)
     assert_rounded_once(out, ref, spread, n_kv, "out")
     w = (0.1 * 0.9 ** torch.arange(n_ctx - 1, -1, -1, device="cuda", dtype=torch.float64))[None, None, :, None]
     assert_rounded_once(scores, (w * p).sum(2), (w * p).square().sum(2).sqrt(), n_ctx, "scores")
+
+
+@pytest.mark.parametrize("dtype", [BF16, F16])
+@pytest.mark.parametrize("grad_scale", [1.0, 2.0 ** 12])   # P dP far past float16's largest number is no overflow of dS
+@pytest.mark.parametrize("Z,H,n_ctx,n_kv", DENSE)
+def test_dense_backward_of_head_size_64_is_rounded_once(Z, H, n_ctx, n_kv, grad_scale, dtype):
+    """Against the formula in float64 on what the kernels are given: the forward's output as it was rounded."""
+    from cascading_kv_cache_amd import flash_attention as fa
+
+    scale = 0.5
+    q, k, v, mask, do = dense_case(Z, H, n_ctx, n_kv, 64, dtype)
+    do = (do.float() * grad_scale).to(dtype)
+    out, _, lse, m = fa._forward(q, k, v, True, scale, mask, 0.9, True)
+    dq, dk, dv = fa._backward(q, k, v, out, lse, m, do, scale)
+    _, p, _, _ = exact_attention(q, k, v, visible(n_ctx, n_kv, mask), scale)
+    qd, kd, vd, g = q.double(), k.double(), v.double(), do.double()
+    dp, delta = torch.matmul(g, vd.transpose(2, 3).contiguous()), (out.double() * g).sum(-1, keepdim=True)
+    ds, ds_size = p * (dp - delta) * scale, p * (dp.abs() + delta.abs() + grad_scale) * scale
+    pt, dst, ds2t = (t.transpose(2, 3).contiguous() for t in (p, ds, ds_size.square()))
+    if grad_scale == 1.0 or dtype == BF16:   # float16 gradients of that size are infinite themselves where they pass 65504
+        assert_rounded_once(dv, torch.matmul(pt, g), torch.matmul(pt.square(), g.square()).sqrt(), n_ctx, "dv")
+        assert_rounded_once(dk, torch.matmul(dst, qd), torch.matmul(ds2t, qd.square()).sqrt(), n_ctx, "dk")
+    want, spread = torch.matmul(ds, kd), torch.matmul(ds_size.square(), kd.square()).sqrt()
+    fits = want.abs() < 6e4 if dtype == F16 else torch.ones_like(want, dtype=torch.bool)
+    assert_rounded_once(dq[fits], want[fits], spread[fits], n_kv, "dq")
 
 
 def one_layer(B, KVH, D, NS, W, C, dtype):
