@@ -13,6 +13,12 @@
 //   colsum   one workgroup = one head x 32 keys, held in registers; its four wavefronts take the 32-row query tiles in
 //            turn.  S = Q K^T keeps a key in one lane pair, so a weighted sum stays in its lane until the end.
 //
+// A matrix instruction multiplies every row of a tile by every value, and zero times infinity or NaN is NaN, while a value
+// whose key has probability zero counts for nothing, whatever it holds (the vector kernels do not touch it).  So a wavefront
+// whose accumulators come out finite is done: nothing else can have been multiplied.  Otherwise it goes over its keys once
+// more with the normalisers it has found, finite values through the matrix pipe and the others where their probability is
+// above zero.
+//
 // A contraction over the head dim may take the dims in any order as long as both operands do: step 4 c + e multiplies
 // dims 8 c + e (lanes 0..31) and 8 c + 4 + e (lanes 32..63), so that an operand is a 16-byte load per four steps.
 #include "ckv_attn_internal.h"
@@ -94,28 +100,10 @@ __global__ void __launch_bounds__(kFwdWaves* CKV_WAVE) fwd_f32_mfma_kernel(F32Fw
     int m_hi = (rt * kRows + kRows - 1) / G;
     if (m_hi > Q - 1) m_hi = Q - 1;
     const int nblk = (Nc + m_hi) / kKeys + 1;            // blocks some row of the tile may see
-    f32x16 o[DB];
-#pragma unroll
-    for (int db = 0; db < DB; db++) o[db] = zero16();
-    float m_run = -INFINITY, l_run = 0.f;
-    for (int blk = split * kFwdWaves + wave; blk < nblk; blk += kFwdWaves * f.n_split) {
-        const int n0 = blk * kKeys;
-        const int n = n0 + col;
-        const uint32_t vis = (uint32_t)__ballot(n < Nc ? !(p.kmasked && p.kmasked[n]) : n < N);
-        if (vis == 0u) continue;
-        float4 kf[NP];
-        {
-            const float* kr = kb + (int64_t)(n < N ? n : N - 1) * p.kv_stride[2] + 4 * half;
-#pragma unroll
-            for (int c = 0; c < NP; c++) kf[c] = *reinterpret_cast<const float4*>(kr + 8 * c);
-        }
-        // values of the lane's half of the keys, dims DB col .. DB col + DB - 1: accumulator db holds dims DB m + db
-        Vec<DB> vf[16];
-#pragma unroll
-        for (int v = 0; v < 16; v++) {
-            const int nv = n0 + acc_row(v, half);
-            vf[v] = *reinterpret_cast<const Vec<DB>*>(vb + (int64_t)(nv < N ? nv : N - 1) * p.kv_stride[2] + DB * col);
-        }
+    // bit r: key r of the block is there and not masked
+    auto visible_keys = [&](int n) { return (uint32_t)__ballot(n < Nc ? !(p.kmasked && p.kmasked[n]) : n < N); };
+    // the logits of a block's keys (lane = its query), and the keys this lane's query sees
+    auto logits = [&](const float4(&kf)[NP]) {
         f32x16 s = zero16();
 #pragma unroll
         for (int c = 0; c < NP; c++) {
@@ -125,13 +113,41 @@ __global__ void __launch_bounds__(kFwdWaves* CKV_WAVE) fwd_f32_mfma_kernel(F32Fw
             s = mma(kf[c].z, q4.z, s);
             s = mma(kf[c].w, q4.w, s);
         }
-        // bit r of `allow`: key r of the block is visible to this lane's query
-        uint32_t allow = vis;
-        if (n0 + kKeys - 1 >= Nc) {
-            const int last = Nc + row_m - n0;   // last key of the block the row may see
-            const uint32_t seen = last >= 31 ? ~0u : (last < 0 ? 0u : (2u << last) - 1u);
-            allow &= seen;                      // cached keys lie in front of the chunk keys: row_m >= 0 lets them all through
+        return s;
+    };
+    auto seen_keys = [&](uint32_t vis, int n0) {
+        if (n0 + kKeys - 1 < Nc) return vis;
+        const int last = Nc + row_m - n0;   // last key of the block the row may see
+        return vis & (last >= 31 ? ~0u : (last < 0 ? 0u : (2u << last) - 1u));   // cached keys lie in front of the chunk keys: row_m >= 0 lets them all through
+    };
+    auto load_keys = [&](int n, float4(&kf)[NP]) {
+        const float* kr = kb + (int64_t)(n < N ? n : N - 1) * p.kv_stride[2] + 4 * half;
+#pragma unroll
+        for (int c = 0; c < NP; c++) kf[c] = *reinterpret_cast<const float4*>(kr + 8 * c);
+    };
+    // values of the lane's half of the keys, dims DB col .. DB col + DB - 1: accumulator db holds dims DB m + db
+    auto load_values = [&](int n0, Vec<DB>(&vf)[16]) {
+#pragma unroll
+        for (int v = 0; v < 16; v++) {
+            const int nv = n0 + acc_row(v, half);
+            vf[v] = *reinterpret_cast<const Vec<DB>*>(vb + (int64_t)(nv < N ? nv : N - 1) * p.kv_stride[2] + DB * col);
         }
+    };
+    f32x16 o[DB];
+#pragma unroll
+    for (int db = 0; db < DB; db++) o[db] = zero16();
+    float m_run = -INFINITY, l_run = 0.f;
+    for (int blk = split * kFwdWaves + wave; blk < nblk; blk += kFwdWaves * f.n_split) {
+        const int n0 = blk * kKeys;
+        const int n = n0 + col;
+        const uint32_t vis = visible_keys(n);
+        if (vis == 0u) continue;
+        float4 kf[NP];
+        load_keys(n, kf);
+        Vec<DB> vf[16];
+        load_values(n0, vf);
+        f32x16 s = logits(kf);
+        const uint32_t allow = seen_keys(vis, n0);   // bit r: key r of the block is visible to this lane's query
         const bool whole = __ballot(allow != ~0u) == 0ull;
         float mx = -INFINITY;
 #pragma unroll
@@ -170,7 +186,55 @@ __global__ void __launch_bounds__(kFwdWaves* CKV_WAVE) fwd_f32_mfma_kernel(F32Fw
             for (int db = 0; db < DB; db++) o[db] = mma(vf[v].v[db], s[v], o[db]);
     }
 
-    // merge: every wavefront scales its share to the common maximum
+    float zero = 0.f;   // or NaN
+#pragma unroll
+    for (int db = 0; db < DB; db++)
+#pragma unroll
+        for (int v = 0; v < 16; v++) zero = fmaf(o[db][v], 0.f, zero);
+    if (__ballot(zero != 0.f) != 0ull) {
+#pragma unroll
+        for (int db = 0; db < DB; db++) o[db] = zero16();
+        for (int blk = split * kFwdWaves + wave; blk < nblk; blk += kFwdWaves * f.n_split) {
+            const int n0 = blk * kKeys;
+            const uint32_t vis = visible_keys(n0 + col);
+            if (vis == 0u) continue;
+            f32x16 s;
+            {
+                float4 kf[NP];
+                load_keys(n0 + col, kf);
+                s = logits(kf);
+            }
+            const uint32_t allow = seen_keys(vis, n0);
+#pragma unroll
+            for (int v = 0; v < 16; v++) s[v] = (allow >> acc_row(v, half)) & 1u ? expf(s[v] * p.scale - m_run) : 0.f;
+            Vec<DB> vf[16];
+            load_values(n0, vf);
+            bool odd = false;
+#pragma unroll
+            for (int v = 0; v < 16; v++)
+#pragma unroll
+                for (int db = 0; db < DB; db++) {
+                    const float x = vf[v].v[db];
+                    odd = odd || !isfinite(x);
+                    o[db] = mma(isfinite(x) ? x : 0.f, s[v], o[db]);
+                }
+            if (__ballot(odd) == 0ull) continue;
+#pragma unroll
+            for (int db = 0; db < DB; db++) {
+                f32x16 up = zero16(), down = zero16();   // how many infinities of either sign a sum holds, a NaN being both
+#pragma unroll
+                for (int v = 0; v < 16; v++) {
+                    const float x = vf[v].v[db], counts = s[v] > 0.f ? 1.f : 0.f;
+                    up = mma(x == INFINITY || isnan(x) ? 1.f : 0.f, counts, up);
+                    down = mma(x == -INFINITY || isnan(x) ? 1.f : 0.f, counts, down);
+                }
+#pragma unroll
+                for (int v = 0; v < 16; v++) o[db][v] += (up[v] > 0.f ? INFINITY : 0.f) + (down[v] > 0.f ? -INFINITY : 0.f);
+            }
+        }
+    }
+
+    // merge: every wavefront scales its share to the common maximum (a share that has come down to nothing is left out)
     l_run += __shfl_xor(l_run, 32);
     if (half == 0) {
         ml_lds[wave * kRows + col] = m_run;
@@ -187,7 +251,7 @@ __global__ void __launch_bounds__(kFwdWaves* CKV_WAVE) fwd_f32_mfma_kernel(F32Fw
         for (int v = 0; v < 16; v++) {
             Vec<DB> t;
 #pragma unroll
-            for (int db = 0; db < DB; db++) t.v[db] = o[db][v] * sc;
+            for (int db = 0; db < DB; db++) t.v[db] = sc == 0.f ? 0.f : o[db][v] * sc;
             *reinterpret_cast<Vec<DB>*>(ow + DB * acc_row(v, half)) = t;
         }
     }
@@ -243,6 +307,7 @@ __global__ void __launch_bounds__(256) fwd_f32_combine_kernel(F32Fwd f) {
         const float l = f.part_l[s * rows + row];
         if (l == -INFINITY) continue;
         const float w = expf(l - M);
+        if (w == 0.f) continue;
         const float4 v = *reinterpret_cast<const float4*>(f.part_o + (s * rows + row) * D + 4 * d4);
         L += w;
         o.x = fmaf(v.x, w, o.x); o.y = fmaf(v.y, w, o.y); o.z = fmaf(v.z, w, o.z); o.w = fmaf(v.w, w, o.w);

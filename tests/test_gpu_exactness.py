@@ -1,7 +1,8 @@
 """What the fp32-math paths owe float64 arithmetic on the same inputs.
 
 Head size 64 in the 16-bit formats holds logits, probabilities, dS and every sum in 32 bits: a result is the exact
-one rounded once to the tensor dtype, up to the noise of its float32 sums.
+one rounded once to the tensor dtype, up to the noise of its float32 sums.  In float32 a value row of a key with
+probability zero is never touched, whatever it holds.
 
 Cached keys are rotated; with ``inv_freq`` zero the rotation is the identity, so that the staged operands are known to
 the bit: queries and keys times sqrt(softmax scale), rounded to the tensor dtype (cascade_attention.py:284-291).
@@ -135,3 +136,73 @@ def test_cascade_forward_is_rounded_once(B, H, KVH, D, NS, W, C, filled, Q, dtyp
     ref, p, _, spread = exact_attention(qs, ks, vs, visible(Q, ks.size(2), mask), 1.0)
     out, _ = cascade_attention(q, k, v, cache, 0, inv_freq, update_cache=False)
     assert_rounded_once(out, ref, spread, ks.size(2), "out")
+
+
+NAN, INF = float("nan"), float("inf")
+
+
+def poison(v, at):
+    """Rows of the chunk that hold what a product with zero does not survive: NaN, both infinities, and one dim with an
+    infinity of each sign from two tokens."""
+    v[:, :, at, 3], v[:, :, at, 5], v[:, :, at, 7] = NAN, INF, -INF
+    v[:, :, at, 9], v[:, :, at + 2, 9] = INF, -INF
+
+
+def check_classes(out, p, v, what):
+    """Finite, infinite and NaN where the sum over the keys with a probability above zero is, and its value where finite."""
+    pd, vd = p.float() > 0, v.double()
+    finite = torch.where(torch.isfinite(vd), vd, 0.0)
+    want = torch.matmul(p, finite)
+    hit = lambda sel: torch.matmul(pd.double(), sel.double()) > 0
+    up, down, bad = hit(vd == INF), hit(vd == -INF), hit(torch.isnan(vd))
+    bad = bad | (up & down)
+    assert torch.equal(torch.isnan(out), bad), f"{what}: {(torch.isnan(out) != bad).sum().item()} values NaN or not"
+    assert torch.equal(out == INF, up & ~bad) and torch.equal(out == -INF, down & ~bad), f"{what}: infinities"
+    fine = ~(up | down | bad)
+    err = (out.double() - want)[fine].abs().max().item()
+    assert err <= (1e-5 if out.dtype == F32 else 1e-2), f"{what}: {err:.2e}"
+
+
+@pytest.mark.parametrize("D,dtype", [(64, F32), (128, F32)])
+@pytest.mark.parametrize("n_ctx,n_kv,at", [(96, 96, 37), (300, 1000 + 300, 130), (64, 64, 0), (40, 3000 + 40, 33)])
+def test_values_of_later_tokens_reach_no_earlier_row(D, dtype, n_ctx, n_kv, at):
+    from cascading_kv_cache_amd.flash_attention import attention
+
+    q, k, v, mask, _ = dense_case(1, 2, n_ctx, n_kv, D, dtype)
+    poison(v, n_kv - n_ctx + at)
+    out, _ = attention(q, k, v, True, 0.3, mask, 0.9)
+    _, p, _, _ = exact_attention(q, k, torch.zeros_like(v), visible(n_ctx, n_kv, mask), 0.3)
+    check_classes(out, p, v, "dense")
+    assert torch.isfinite(out[:, :, :at].float()).all()
+
+
+@pytest.mark.parametrize("D,dtype", [(64, F32), (128, F32)])
+def test_values_of_keys_with_probability_zero_are_not_touched(D, dtype):
+    """A logit so far below the row's largest that its probability is zero in float32: the value row does not count."""
+    from cascading_kv_cache_amd.flash_attention import attention
+
+    q, k, v, mask, _ = dense_case(1, 2, 70, 400 + 70, D, dtype)
+    q[..., 0], k[..., 0] = 8.0, 0.0
+    k[:, :, 11, 0], k[:, :, 410, 0] = -256.0, -256.0     # logits 600 below the others
+    mask[11] = False
+    k[:, :, 224:256, 0] = -256.0                          # and a block of them that nobody else shares
+    mask[224:256] = False
+    poison(v, 11)
+    v[:, :, 410], v[:, :, 224:256] = NAN, INF
+    mask[13] = True                                       # poison()'s second row
+    out, _ = attention(q, k, v, True, 0.3, mask, 0.9)
+    assert torch.isfinite(out.float()).all()
+
+
+@pytest.mark.parametrize("D,dtype,W,C,filled,Q", [
+    (128, F32, 512, 4, 4000, 40), (64, F32, 64, 2, 300, 40)])
+def test_later_values_of_a_chunk_reach_no_earlier_row(D, dtype, W, C, filled, Q):
+    """The same over a cache, with the keys shared out over workgroups (512 x 4) and not."""
+    from cascading_kv_cache_amd.cascade_attention import cascade_attention
+
+    cache, q, k, v, inv_freq = cascade_case(1, 8, 2, D, 4, W, C, filled, Q, dtype)
+    poison(v, 21)
+    qs, ks, vs, mask = staged(cache, q, k, v)
+    _, p, _, _ = exact_attention(qs, ks, torch.zeros_like(vs), visible(Q, ks.size(2), mask), 1.0)
+    out, _ = cascade_attention(q, k, v, cache, 0, inv_freq, update_cache=False)
+    check_classes(out, p, vs, "cascade")
