@@ -893,6 +893,61 @@ __global__ void __launch_bounds__(512) fwd_pipe_kernel(FwdParams p) {
         __builtin_amdgcn_s_waitcnt(0x0F70);
     }
 
+    if constexpr (kEx) {
+        // The matrix pipe multiplies every row by every value, and zero times infinity or NaN is NaN; a value whose key has
+        // probability zero counts for nothing, whatever it holds.  A wavefront whose accumulators come out finite has met no
+        // such value.  Otherwise it goes over its tiles once more, straight from memory, with the references it has found:
+        // finite values times float32 probabilities, the others where the probability is above zero.
+        float zero = 0.f;   // or NaN
+#pragma unroll
+        for (int dt = 0; dt < kDB; dt++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) zero = fmaf(oacc[dt][v], 0.f, zero);
+        if (__builtin_amdgcn_ballot_w64(zero != 0.f) != 0ull) {
+            f32x16 none;
+#pragma unroll
+            for (int v = 0; v < 16; v++) none[v] = 0.f;
+#pragma unroll
+            for (int dt = 0; dt < kDB; dt++) oacc[dt] = none;
+            for (int j = 0; j < n_work; j++) {
+                const int entry = work(j);
+                const char* kt = kbase + (int64_t)(entry & 0x7fffffff) * kTileBytes + k_image_off(col, half);
+                const char* vt = vbase + (int64_t)(entry & 0x7fffffff) * kTileBytes + v_image_off<kD>(col, half);
+                f32x16 s[2] = {none, none};
+#pragma unroll
+                for (int kk = 0; kk < kKK; kk++)
+#pragma unroll
+                    for (int ks = 0; ks < 2; ks++)
+                        s[ks] = Mma<T>::mma(*reinterpret_cast<const uint4*>(kt + kk * 2048 + ks * 512), qreg[kk], s[ks]);
+                if (entry < 0) mask_tile(entry, s);
+#pragma unroll
+                for (int ks = 0; ks < 2; ks++)
+#pragma unroll
+                    for (int v = 0; v < 16; v++) s[ks][v] = prob(s[ks][v]);
+#pragma unroll
+                for (int dt = 0; dt < kDB; dt++) {
+                    f32x16 up = none, down = none;   // how many infinities of either sign a sum holds, a NaN being both
+#pragma unroll
+                    for (int st = 0; st < 4; st++) {
+                        const uint4 a = *reinterpret_cast<const uint4*>(vt + st * (32 * kD) + dt * 512);
+                        const uint32_t w[4] = {a.x, a.y, a.z, a.w};
+#pragma unroll
+                        for (int e = 0; e < 8; e++) {   // key 16 st + 8 (e / 4) + 4 half + e % 4
+                            const float x = e & 1 ? Mma<T>::hi_f(w[e >> 1]) : Mma<T>::lo_f(w[e >> 1]);
+                            const float pe = s[st >> 1][8 * (st & 1) + e], counts = pe > 0.f ? 1.f : 0.f;
+                            auto f32 = [](float x_, float y_, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x2f32(x_, y_, c, 0, 0, 0); };
+                            oacc[dt] = f32(isfinite(x) ? x : 0.f, pe, oacc[dt]);
+                            up = f32(x == INFINITY || isnan(x) ? 1.f : 0.f, counts, up);
+                            down = f32(x == -INFINITY || isnan(x) ? 1.f : 0.f, counts, down);
+                        }
+                    }
+#pragma unroll
+                    for (int v = 0; v < 16; v++) oacc[dt][v] += (up[v] > 0.f ? INFINITY : 0.f) + (down[v] > 0.f ? -INFINITY : 0.f);
+                }
+            }
+        }
+    }
+
     // epilogue: lane owns d = 32dt + 8(v/4) + 4half + v%4 of its query row
     const float l_tot = l_run + __shfl_xor(l_run, 32);
     if (p.n_split > 1) {
@@ -1006,6 +1061,7 @@ __global__ void __launch_bounds__(256) fwd_combine_kernel(FwdParams p) {
         for (int u = 0; u < kBatch; u++) {
             if (l2[u] == -INFINITY) continue;
             const float w = __builtin_amdgcn_exp2f(l2[u] - M);
+            if (kExact<kD> && w == 0.f) continue;   // a share that has come down to nothing, whatever it holds
             L += w;
             o.x = fmaf(v[u].x, w, o.x); o.y = fmaf(v[u].y, w, o.y); o.z = fmaf(v[u].z, w, o.z); o.w = fmaf(v[u].w, w, o.w);
         }

@@ -1,8 +1,8 @@
 """What the fp32-math paths owe float64 arithmetic on the same inputs.
 
 Head size 64 in the 16-bit formats holds logits, probabilities, dS and every sum in 32 bits: a result is the exact
-one rounded once to the tensor dtype, up to the noise of its float32 sums.  In float32 a value row of a key with
-probability zero is never touched, whatever it holds.
+one rounded once to the tensor dtype, up to the noise of its float32 sums.  There and in float32 a value row of a key
+with probability zero is never touched, whatever it holds.
 
 Cached keys are rotated; with ``inv_freq`` zero the rotation is the identity, so that the staged operands are known to
 the bit: queries and keys times sqrt(softmax scale), rounded to the tensor dtype (cascade_attention.py:284-291).
@@ -163,7 +163,7 @@ def check_classes(out, p, v, what):
     assert err <= (1e-5 if out.dtype == F32 else 1e-2), f"{what}: {err:.2e}"
 
 
-@pytest.mark.parametrize("D,dtype", [(64, F32), (128, F32)])
+@pytest.mark.parametrize("D,dtype", [(64, F32), (128, F32), (64, BF16), (64, F16)])
 @pytest.mark.parametrize("n_ctx,n_kv,at", [(96, 96, 37), (300, 1000 + 300, 130), (64, 64, 0), (40, 3000 + 40, 33)])
 def test_values_of_later_tokens_reach_no_earlier_row(D, dtype, n_ctx, n_kv, at):
     from cascading_kv_cache_amd.flash_attention import attention
@@ -176,7 +176,7 @@ def test_values_of_later_tokens_reach_no_earlier_row(D, dtype, n_ctx, n_kv, at):
     assert torch.isfinite(out[:, :, :at].float()).all()
 
 
-@pytest.mark.parametrize("D,dtype", [(64, F32), (128, F32)])
+@pytest.mark.parametrize("D,dtype", [(64, F32), (128, F32), (64, BF16), (64, F16)])
 def test_values_of_keys_with_probability_zero_are_not_touched(D, dtype):
     """A logit so far below the row's largest that its probability is zero in float32: the value row does not count."""
     from cascading_kv_cache_amd.flash_attention import attention
@@ -195,7 +195,7 @@ def test_values_of_keys_with_probability_zero_are_not_touched(D, dtype):
 
 
 @pytest.mark.parametrize("D,dtype,W,C,filled,Q", [
-    (128, F32, 512, 4, 4000, 40), (64, F32, 64, 2, 300, 40)])
+    (128, F32, 512, 4, 4000, 40), (64, F32, 64, 2, 300, 40), (64, BF16, 512, 4, 4000, 40), (64, F16, 64, 2, 300, 100)])
 def test_later_values_of_a_chunk_reach_no_earlier_row(D, dtype, W, C, filled, Q):
     """The same over a cache, with the keys shared out over workgroups (512 x 4) and not."""
     from cascading_kv_cache_amd.cascade_attention import cascade_attention
