@@ -266,8 +266,8 @@ __global__ void __launch_bounds__(kFwdWaves* CKV_WAVE) fwd_f32_mfma_kernel(F32Fw
     for (int w = 0; w < kFwdWaves; w++) M = fmaxf(M, ml_lds[w * kRows + r]);
 #pragma unroll
     for (int w = 0; w < kFwdWaves; w++) {
-        const float mw = ml_lds[w * kRows + r];
-        if (mw != -INFINITY) L = fmaf(ml_lds[(kFwdWaves + w) * kRows + r], expf(mw - M), L);
+        const float mw = ml_lds[w * kRows + r], lw = ml_lds[(kFwdWaves + w) * kRows + r];
+        if (lw != 0.f) L = fmaf(lw, mw == -INFINITY ? 1.f : expf(mw - M), L);   // no largest logit but a sum: a NaN
     }
     float acc[kPer];
 #pragma unroll
@@ -276,13 +276,15 @@ __global__ void __launch_bounds__(kFwdWaves* CKV_WAVE) fwd_f32_mfma_kernel(F32Fw
     for (int w = 0; w < kFwdWaves; w++)
 #pragma unroll
         for (int i = 0; i < kPer; i++) acc[i] += o_lds[(w * kRows + r) * G_::kPitch + d0 + i];
-    const float inv = L > 0.f ? 1.f / L : 0.f;
+    // A row without a probability above zero (all its logits overflowed) or with a NaN among them is NaN, however many
+    // shares its keys are in; a share without one says so by -inf, a NaN has to reach the merge.
+    const float inv = 1.f / L;
     const int64_t row = (b * p.H + kvh * G + g) * p.Q + m, rows = p.B * p.H * p.Q;
     if (f.n_split > 1) {
         float* po = f.part_o + (split * rows + row) * D + d0;
 #pragma unroll
-        for (int i = 0; i < kPer; i++) po[i] = acc[i] * inv;
-        if (d0 == 0) f.part_l[split * rows + row] = L > 0.f ? M + logf(L) : -INFINITY;
+        for (int i = 0; i < kPer; i++) po[i] = L == 0.f ? 0.f : acc[i] * inv;
+        if (d0 == 0) f.part_l[split * rows + row] = L == 0.f ? -INFINITY : M + logf(L);
         return;
     }
     float* orow = (float*)p.out + b * p.out_stride[0] + (kvh * G + g) * p.out_stride[1] + m * p.out_stride[2];

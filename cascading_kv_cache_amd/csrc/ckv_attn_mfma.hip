@@ -955,7 +955,7 @@ __global__ void __launch_bounds__(512) fwd_pipe_kernel(FwdParams p) {
         const int rf_p = qt_i * kRows + wave * 32 + col;
         const int64_t row_p = (b * p.H + kvh * p.G + rf_p % p.G) * p.Q + row_m;
         if (row_m < p.Q) {
-            const bool any = l_tot > 0.f;
+            const bool any = l_tot != 0.f;   // a NaN is not nothing: it has to reach the merge
             const float inv_p = any ? 1.f / l_tot : 0.f;
             float* po = p.part_o + ((int64_t)split_i * p.B * p.H * p.Q + row_p) * kD;
 #pragma unroll

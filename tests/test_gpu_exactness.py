@@ -2,7 +2,8 @@
 
 Head size 64 in the 16-bit formats holds logits, probabilities, dS and every sum in 32 bits: a result is the exact
 one rounded once to the tensor dtype, up to the noise of its float32 sums.  There and in float32 a value row of a key
-with probability zero is never touched, whatever it holds.
+with probability zero is never touched, whatever it holds, and the number of workgroups that share a row's keys changes
+nothing but the order of sums.
 
 Cached keys are rotated; with ``inv_freq`` zero the rotation is the identity, so that the staged operands are known to
 the bit: queries and keys times sqrt(softmax scale), rounded to the tensor dtype (cascade_attention.py:284-291).
@@ -206,3 +207,29 @@ def test_later_values_of_a_chunk_reach_no_earlier_row(D, dtype, W, C, filled, Q)
     _, p, _, _ = exact_attention(qs, ks, torch.zeros_like(vs), visible(Q, ks.size(2), mask), 1.0)
     out, _ = cascade_attention(q, k, v, cache, 0, inv_freq, update_cache=False)
     check_classes(out, p, vs, "cascade")
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("W,C,filled", [(64, 1, 100), (512, 4, 4000)])   # one share of the keys, and four
+def test_a_row_whose_logits_all_overflow_is_nan_however_its_keys_are_shared(D, W, C, filled):
+    from cascading_kv_cache_amd.cascade_attention import cascade_attention
+
+    cache, q, k, v, inv_freq = cascade_case(1, 8, 2, D, 4, W, C, filled, 40, F32)
+    for t, x in ((q, 1e20), (k, -1e20), (cache.key_cache[0], -1e20), (cache.sink_keys[0], -1e20)):
+        t.zero_()
+        t[..., 0] = x
+    q[:, :, 7] = 0.0          # a row with logits of zero among them
+    out, _ = cascade_attention(q, k, v, cache, 0, inv_freq, update_cache=False)
+    rows = torch.arange(40, device="cuda") != 7
+    assert torch.isnan(out[:, :, rows]).all() and torch.isfinite(out[:, :, 7]).all()
+
+
+@pytest.mark.parametrize("D,dtype", [(64, F32), (128, F32), (64, BF16), (64, F16), (128, BF16), (128, F16)])
+@pytest.mark.parametrize("W,C,filled", [(64, 1, 100), (512, 4, 4000)])   # one share of the keys, and several
+def test_a_key_that_is_nan_makes_every_row_that_sees_it_nan_however_its_keys_are_shared(D, dtype, W, C, filled):
+    from cascading_kv_cache_amd.cascade_attention import cascade_attention
+
+    cache, q, k, v, inv_freq = cascade_case(1, 8, 2, D, 4, W, C, filled, 40, dtype)
+    cache.key_cache[0][:, 1, 11] = NAN
+    out, _ = cascade_attention(q, k, v, cache, 0, inv_freq, update_cache=False)
+    assert torch.isnan(out[:, 4:]).all() and torch.isfinite(out[:, :4].float()).all()
