@@ -41,7 +41,7 @@ AttnWorkspace carve_attn(void* base, int64_t B, int64_t H, int64_t KVH, int64_t 
     w.w_ema = (float*)c.take((Q + kColSlack) * 4);
     w.w_new = (float*)c.take(Q * 4);
     // shares of the forward kernel when few query rows would leave the chip idle
-    int splits = mfma_supported(dtype, D, H, KVH, Q) && Q > 1 ? mfma_fwd_splits_for_workspace(B, H, KVH, Q, N) : 1;
+    int splits = mfma_supported(dtype, D, H, KVH, Q) && Q > 1 ? mfma_fwd_splits_for_workspace(B, H, KVH, Q, N, false) : 1;
     if (dtype == CKV_F32 && (D == 64 || D == 128)) splits = f32_mfma_splits(B, H, KVH, Q, N, mfma_device_cus());
     w.part_o = splits > 1 ? (float*)c.take(splits * B * H * Q * D * 4) : nullptr;
     w.part_l2 = splits > 1 ? (float*)c.take(splits * B * H * Q * 4) : nullptr;
@@ -73,7 +73,7 @@ DenseWorkspace carve_dense(void* base, int64_t B, int64_t H, int64_t n_ctx, int6
     w.w_new = (float*)c.take(n_ctx * 4);
     w.key_order = (int*)c.take(n_kv * 4);
     w.n_visible = (int*)c.take(4);
-    const int splits = mfma_fwd_splits_for_workspace(B, H, H, n_ctx, n_kv);
+    const int splits = mfma_fwd_splits_for_workspace(B, H, H, n_ctx, n_kv, true);
     w.part_o = splits > 1 ? (float*)c.take(splits * rows * D * 4) : nullptr;
     w.part_l2 = splits > 1 ? (float*)c.take(splits * rows * 4) : nullptr;
     w.bytes = c.off;

@@ -1592,7 +1592,7 @@ int run_mfma(const MfmaProblem& mp, hipStream_t stream) {
         fp.G = G;
         fp.scale_log2 = left;
         fp.n_qt = (int)((mp.Q * G + kRows - 1) / kRows);
-        fp.n_split = mfma_fwd_splits(mp.B, mp.H, mp.KVH, mp.Q, n, cus, mp.empty_to > mp.empty_from);
+        fp.n_split = mfma_fwd_splits(mp.B, mp.H, mp.KVH, mp.Q, n, cus, mp.key_order != nullptr);
         fp.part_o = mp.part_o;
         fp.part_l2 = mp.part_l2;
         fp.n_visible = mp.n_visible;
@@ -1673,42 +1673,49 @@ bool mfma_supported(int dtype, int64_t D, int64_t H, int64_t KVH, int64_t Q) {
 int64_t mfma_n_pad(int64_t n) { return align_up(n, 256); }
 
 // Shares of a query tile's key tiles (1: no splitting) on a chip of `cus` compute units, each of which holds one workgroup
-// of the forward kernel at a time.  The launch takes whole rounds of workgroups, a round as long as a workgroup: about
-// 1.6 us per key tile with every unit busy and 16 us to start and finish (the work list, the first copies, the rows' way
-// out).  Shares shorten a workgroup, fill a round that is mostly empty, and cost the merge kernel 6 us and its traffic
-// (float32 rows written and read, 256 rows of 512 bytes per workgroup: 0.058 us).  The cheapest number of shares by that
-// count, at least 8 key tiles each.  32 heads on 8 kv heads, forward + merge (before: about two workgroups per unit, at
-// most 8 shares): 509 rows x 16 K keys 162 -> 141 us, 128 x 64 K 203 -> 149, 32 x 64 K 168 -> 93, 1000 x 16 K 271 -> 259,
-// 300 x 2 K 40 -> 34.
-// `filling`: most slots of the cache are known to be empty.  The tiles that are left make shares of a few tiles by either
-// count; those streams keep the count they have always had (about two workgroups per unit, at least 16 tiles by the
-// cache's size, at most 8 shares), so that a decoder's sums are added in the same order as before: four random layers
-// turn one changed rounding of a hidden state into a percent of the logits.
-int mfma_fwd_splits(int64_t B, int64_t H, int64_t KVH, int64_t Q, int64_t n, int cus, bool filling) {
+// of the forward kernel at a time.  The count is a matter of sizes alone, never of how many slots hold a token: it sets the
+// order in which a row's sums are added, so a hint about the filled slots would otherwise change results.
+//
+// `dense`: the dense operator, which takes the cheapest count throughout (the last paragraph).  A chunk over a cache:
+//
+// Fewer workgroups than units: about two per unit, at least 16 tiles each, at most 8 shares; where 8 shares would be of
+// more than 32 tiles, the cheapest count from 8 to 32 by the estimate below.  Forward + merge in us, 32 heads on 8 kv heads,
+// by shares:     509 rows x 16 K  4: 141  8: 155    488 x 16 K, 1000 slots filled  4: 34  8: 47    300 x 2 K  2: 44  4: 35
+//   128 x 64 K   8: 175  16: 134  32: 160        32 x 64 K  8: 162  16: 95  32: 90      509 x 32 K  4: 237  8: 250
+// Up to 16 K slots half the shares would be some 10 % cheaper; they stay, because a decoder of random weights turns the
+// changed rounding of one hidden state into a percent of its logits.
+//
+// More: the launch takes whole rounds of workgroups, a round as long as a workgroup: about 1.6 us per key tile with every
+// unit busy and 16 us to start and finish (the work list, the first copies, the rows' way out).  Shares fill a round that is
+// mostly empty, and cost the merge kernel 6 us and its traffic (float32 rows written and read, 256 rows of 512 bytes per
+// workgroup: 0.058 us).  The cheapest count by that estimate, at least 8 tiles each: 2300 x 8 K  1: 391  3: 353  8: 416.
+// (64 dims: 1: 503  3: 398  6: 382; masked keys of the dense operator, which cost nothing, count like the others.)
+int mfma_fwd_splits(int64_t B, int64_t H, int64_t KVH, int64_t Q, int64_t n, int cus, bool dense) {
     constexpr double kTileUs = 1.6, kStartUs = 16.0, kMergeUs = 6.0, kMergeWgUs = 0.058;
-    constexpr int64_t kMaxShares = 32, kMaxShareBytes = (int64_t)256 << 20, kMinTiles = 8;
+    constexpr int64_t kMaxShares = 32, kMaxShareBytes = (int64_t)256 << 20, kFew = 8, kMinTiles = 8, kMinTilesFew = 16, kMinTilesMany = 32;
     const int64_t G = H / KVH;
     const int64_t wgs = ((Q * G + kRows - 1) / kRows) * B * KVH, tiles = (n + kBN - 1) / kBN;
-    if (filling) {
-        if (wgs >= cus) return 1;
-        const int64_t by_size = tiles / 16 < 8 ? tiles / 16 : 8, by_units = 2 * (int64_t)cus / wgs;
-        const int64_t s_ = by_units < by_size ? by_units : by_size;
-        return s_ < 1 ? 1 : (int)s_;
-    }
     if (wgs >= 4 * (int64_t)cus) return 1;   // at most an eighth of the launch can be an empty round
-    int best = 1;
+    int64_t first = 1, min_tiles = kMinTiles;
+    if (wgs < cus && !dense) {
+        const int64_t few = std::max<int64_t>(1, std::min({2 * (int64_t)cus / wgs, tiles / kMinTilesFew, kFew}));
+        if (few < kFew || tiles / kMinTilesMany <= kFew) return (int)few;
+        first = kFew;
+        min_tiles = kMinTilesMany;
+    }
+    int64_t best = first;
     double best_us = 0.0;
-    for (int64_t s_ = 1; s_ <= kMaxShares && (s_ == 1 || tiles / s_ >= kMinTiles); s_++) {
-        if (s_ > 1 && s_ * wgs * kRows * 512 > kMaxShareBytes) break;
+    for (int64_t s_ = first; s_ <= kMaxShares && (s_ == first || tiles / s_ >= min_tiles); s_++) {
+        if (s_ > first && s_ * wgs * kRows * 512 > kMaxShareBytes) break;
         const double rounds = (double)((wgs * s_ + cus - 1) / cus);
         const double us = rounds * ((double)tiles / (double)s_ * kTileUs + kStartUs) +
                           (s_ > 1 ? kMergeUs + kMergeWgUs * (double)(wgs * s_) : 0.0);
-        if (s_ == 1 || us < best_us) {
-            best = (int)s_;
+        if (s_ == first || us < best_us) {
+            best = s_;
             best_us = us;
         }
     }
-    return best;
+    return (int)best;
 }
 
 // compute units of the current device; 256 (one MI355X) where no device can be asked, e.g. when a workspace is
@@ -1721,11 +1728,8 @@ int mfma_device_cus() {
 
 // what a workspace is sized for: the shares the current device would use, and never fewer than a 256-unit chip's,
 // so that a size computed where no device is visible also serves the launch
-int mfma_fwd_splits_for_workspace(int64_t B, int64_t H, int64_t KVH, int64_t Q, int64_t n) {
-    int most = 1;
-    for (const int cus : {mfma_device_cus(), 256})
-        for (const bool filling : {false, true}) most = std::max(most, mfma_fwd_splits(B, H, KVH, Q, n, cus, filling));
-    return most;
+int mfma_fwd_splits_for_workspace(int64_t B, int64_t H, int64_t KVH, int64_t Q, int64_t n, bool dense) {
+    return std::max(mfma_fwd_splits(B, H, KVH, Q, n, mfma_device_cus(), dense), mfma_fwd_splits(B, H, KVH, Q, n, 256, dense));
 }
 
 // the forward kernel keeps per-tile bookkeeping of all N keys in LDS

@@ -197,8 +197,7 @@ typedef struct ckv_attn_args {
                                       single-token kernels skip whole 128-key tiles of a cache that is still
                                       filling, chunks leave whole 64-key tiles out) or ignore the hint altogether;
                                       visibility is decided by `mask` alone, so with a hint that keeps its promise the
-                                      results do not depend on it (a chunk's float32 sums may be added up in another
-                                      order), and a
+                                      results do not depend on it, to the bit, and a
                                       hint that contradicts `mask` gives unspecified results for the slots it
                                       covers. */
 

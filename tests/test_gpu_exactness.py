@@ -233,3 +233,22 @@ def test_a_key_that_is_nan_makes_every_row_that_sees_it_nan_however_its_keys_are
     cache.key_cache[0][:, 1, 11] = NAN
     out, _ = cascade_attention(q, k, v, cache, 0, inv_freq, update_cache=False)
     assert torch.isnan(out[:, 4:]).all() and torch.isfinite(out[:, :4].float()).all()
+
+
+@pytest.mark.parametrize("D,dtype", [(128, BF16), (128, F16), (64, F16), (128, F32)])
+@pytest.mark.parametrize("H,KVH,W,C,filled,Q", [(8, 2, 1024, 4, 1000, 128), (32, 8, 1024, 4, 4095, 300), (8, 2, 2048, 8, 3000, 33),
+                                                (7, 1, 64, 2, 90, 40)])
+def test_the_filled_slots_hint_changes_no_bit_of_a_chunk(D, dtype, H, KVH, W, C, filled, Q):
+    """Chunks over a cache that is filling, with the hint (from the host's token counter) and without (``replayable``):
+    the number of workgroups that share a row's keys is a matter of sizes, not of how many slots hold a token."""
+    from cascading_kv_cache_amd.cascade_attention import cascade_attention
+
+    cache, q, k, v, inv_freq = cascade_case(1, H, KVH, D, 4, W, C, filled, Q, dtype)
+    before = cache.score_cache[0].clone()
+    results = []
+    for replayable in (False, True):
+        cache.score_cache[0].copy_(before)
+        out, new_scores = cascade_attention(q, k, v, cache, 0, inv_freq, update_cache=False, replayable=replayable)
+        results.append([t.clone().view(torch.uint8) for t in (out, new_scores, cache.score_cache[0])])
+    for a, b in zip(*results):
+        assert torch.equal(a, b)
