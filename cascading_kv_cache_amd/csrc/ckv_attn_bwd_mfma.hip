@@ -166,14 +166,16 @@ __device__ inline void copy_block(const char* base, int64_t row_bytes, int64_t f
         async_copy16(blk, voff, tile_lds + (uint32_t)((kHD / 64 * wave + j) * 1024));
     }
 }
-// The same for rows given by number (one per copy of this lane).
-template <int kHD>
+// The same for rows given by number (one per copy of this lane).  kWide: the rows of a head span 4 GiB or more.
+template <int kHD, bool kWide>
 __device__ inline void copy_rows(const char* base, uint32_t row_bytes, const uint32_t (&rows)[kHD / 64], uint32_t tile_lds, int wave,
                                  int lane) {
 #pragma unroll
     for (int j = 0; j < kHD / 64; j++) {
-        const uint32_t voff = rows[j] * row_bytes + (uint32_t)(swz<kHD>(block_row<kHD>(wave, lane, j), lane % Geo<kHD>::kPieces) << 4);
-        async_copy16(base, voff, tile_lds + (uint32_t)((kHD / 64 * wave + j) * 1024));
+        const uint32_t piece = (uint32_t)(swz<kHD>(block_row<kHD>(wave, lane, j), lane % Geo<kHD>::kPieces) << 4);
+        const uint32_t to = tile_lds + (uint32_t)((kHD / 64 * wave + j) * 1024);
+        if constexpr (kWide) async_copy16_from(base + (uint64_t)rows[j] * row_bytes + piece, to);
+        else async_copy16(base, rows[j] * row_bytes + piece, to);
     }
 }
 
@@ -284,7 +286,7 @@ __device__ inline f32x16 zero16() {
 // ---------------------------------------------------------------------------------------------
 // dq
 // ---------------------------------------------------------------------------------------------
-template <typename T, int kHD>
+template <typename T, int kHD, bool kWide>
 __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dq_kernel(BwdMfmaParams p) {
     constexpr int kTile = Geo<kHD>::kTile;
     __shared__ __attribute__((aligned(16))) unsigned char smem[2][2][kTile];  // [stage][K, V]
@@ -354,8 +356,8 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dq_kernel(BwdMfmaParams 
     uint32_t rows_next[kHD / 64];
     rows_of((int64_t)blk0 * kBlk, rows_next);
     uint32_t vis = (uint32_t)__ballot(key_bit((int64_t)blk0 * kBlk) != 0u);
-    copy_rows<kHD>(kb, row_bytes, rows_next, lds0 + (uint32_t)((blk0 & 1) * 2 * kTile), wave, lane);
-    copy_rows<kHD>(vb, row_bytes, rows_next, lds0 + (uint32_t)((blk0 & 1) * 2 * kTile + kTile), wave, lane);
+    copy_rows<kHD, kWide>(kb, row_bytes, rows_next, lds0 + (uint32_t)((blk0 & 1) * 2 * kTile), wave, lane);
+    copy_rows<kHD, kWide>(vb, row_bytes, rows_next, lds0 + (uint32_t)((blk0 & 1) * 2 * kTile + kTile), wave, lane);
     rows_of((int64_t)(blk0 + 1) * kBlk, rows_next);
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
     __syncthreads();
@@ -370,8 +372,8 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dq_kernel(BwdMfmaParams 
             kb_next = key_bit(n0 + kBlk);
             rows_of(n0 + 2 * kBlk, rows_next);
             __builtin_amdgcn_sched_barrier(0);
-            copy_rows<kHD>(kb, row_bytes, rows_now, lds0 + (uint32_t)((st ^ 1) * 2 * kTile), wave, lane);
-            copy_rows<kHD>(vb, row_bytes, rows_now, lds0 + (uint32_t)((st ^ 1) * 2 * kTile + kTile), wave, lane);
+            copy_rows<kHD, kWide>(kb, row_bytes, rows_now, lds0 + (uint32_t)((st ^ 1) * 2 * kTile), wave, lane);
+            copy_rows<kHD, kWide>(vb, row_bytes, rows_now, lds0 + (uint32_t)((st ^ 1) * 2 * kTile + kTile), wave, lane);
         }
         __builtin_amdgcn_sched_barrier(0);
         // keys of this block that are chunk keys past this wavefront's last row: nothing to do for it
@@ -709,7 +711,8 @@ int run(const BwdMfmaParams& p_in, hipStream_t stream) {
         return by_xcd ? dim3((unsigned)(heads * per_head)) : dim3((unsigned)per_head, (unsigned)heads);
     };
     const dim3 grid_dq = grid_of((a.n_ctx + kOwn - 1) / kOwn * p.n_split, 0x7fffffff);
-    hipLaunchKernelGGL((bwd_mfma_dq_kernel<T, kHD>), grid_dq, dim3(kThreads), 0, stream, p);
+    if (a.n_kv * a.kv_stride[2] * 2 < (int64_t)1 << 32) hipLaunchKernelGGL((bwd_mfma_dq_kernel<T, kHD, false>), grid_dq, dim3(kThreads), 0, stream, p);
+    else hipLaunchKernelGGL((bwd_mfma_dq_kernel<T, kHD, true>), grid_dq, dim3(kThreads), 0, stream, p);
     CKV_HIP_TRY(hipGetLastError());
     if (p.n_split > 1) {
         const int64_t threads = a.B * a.H * a.n_ctx * (kHD / 4);
@@ -729,7 +732,6 @@ int run(const BwdMfmaParams& p_in, hipStream_t stream) {
 bool bwd_mfma_supported(const ckv_dense_bwd_args& a) {
     if (a.dtype != CKV_F16 && a.dtype != CKV_BF16) return false;
     if (a.D != 64 && a.D != 128) return false;
-    if (a.n_kv * a.kv_stride[2] * 2 >= (int64_t)1 << 32) return false;  // 32-bit byte offsets inside a head
     if (!rows_ok(a.q_stride) || !rows_ok(a.kv_stride) || !rows_ok(a.dout_stride) || !rows_ok(a.dq_stride) ||
         !rows_ok(a.dkv_stride))
         return false;

@@ -206,6 +206,14 @@ __device__ inline void async_copy16(const void* sbase, uint32_t voff, uint32_t l
                  : "memory");
 }
 
+// The same from an address of the lane's own, for sources more than 4 GiB apart.
+__device__ inline void async_copy16_from(const void* src, uint32_t lds_wave_base) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+                 :
+                 : "s"(__builtin_amdgcn_readfirstlane(lds_wave_base)), "v"(src)
+                 : "memory");
+}
+
 __device__ inline uint32_t lds_address(const void* p) {
     return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
 }

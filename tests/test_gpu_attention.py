@@ -696,3 +696,26 @@ def test_score_sums_of_a_ragged_chunk_keep_to_their_head():
     _, got = attention(q, k, k, True, 0.1, mask, 0.9999)
     assert torch.equal(got[:, 0].view(torch.int16), want[:, 0].view(torch.int16))
     assert torch.isfinite(got[:, 0].float()).all()
+
+
+@pytest.mark.parametrize("D,dtype", [(128, torch.bfloat16), (64, torch.float16)])
+def test_backward_of_rows_that_span_four_gibibytes(D, dtype):
+    """Rows of a head up to 2^24 elements apart (a view into a larger buffer): byte offsets inside a head past 32 bits, the
+    same result to the bit as over rows that lie together."""
+    from cascading_kv_cache_amd import flash_attention as fa
+
+    torch.manual_seed(29)
+    n_ctx, n_kv, stride = 40, 40 + 100, (1 << 24) - 8
+    buffer = torch.empty((n_kv - 1) * stride + 4 * D, dtype=dtype, device="cuda")   # 4.7 GB; only its rows are written
+    assert n_kv * stride * 2 > 1 << 32
+    k, v = (buffer.as_strided((1, 2, n_kv, D), (0, D, stride, 1), off) for off in (0, 2 * D))
+    for t in (k, v):
+        t.copy_(torch.empty((1, 2, n_kv, D), device="cuda").normal_(std=0.5))
+    q, do = (torch.empty((1, 2, n_ctx, D), device="cuda").normal_(std=0.5).to(dtype) for _ in range(2))
+    mask = torch.rand(n_kv - n_ctx, device="cuda") > 0.5
+    results = []
+    for kk, vv in ((k, v), (k.contiguous(), v.contiguous())):
+        out, _, lse, m = fa._forward(q, kk, vv, True, 0.5, mask, 0.9, True)
+        results.append((out, lse) + fa._backward(q, kk, vv, out, lse, m, do, 0.5))
+    for name, a, b in zip(("out", "lse", "dq", "dk", "dv"), *results):
+        assert torch.equal(a, b), name
