@@ -55,8 +55,8 @@ def _forward(q, k, v, causal, sm_scale, mask, beta, want_lse):
     a.causal = int(bool(causal))
     a.dtype = _abi.dtype_code(q.dtype)
     a.lse = lse.data_ptr() if want_lse else None
-    need = lib.ckv_dense_workspace_bytes(B, H, n_ctx, n_kv, D, a.dtype)
     with torch.cuda.device(q.device):
+        need = lib.ckv_dense_workspace_bytes(B, H, n_ctx, n_kv, D, a.dtype)
         stream = torch.cuda.current_stream(q.device).cuda_stream
         ws = workspace(q.device, need, stream)
         a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
@@ -85,9 +85,9 @@ def _backward(q, k, v, o, lse, mask, do, sm_scale):
     a.B, a.H, a.n_ctx, a.n_kv, a.D = B, H, n_ctx, n_kv, D
     a.scale = float(sm_scale)
     a.dtype = _abi.dtype_code(q.dtype)
-    need = lib.ckv_dense_bwd_workspace_bytes(B, H, n_ctx) + lib.ckv_dense_bwd_key_order_bytes(n_kv)
-    need += lib.ckv_dense_bwd_split_bytes(B, H, n_ctx, n_kv, D, a.dtype)
     with torch.cuda.device(q.device):
+        need = lib.ckv_dense_bwd_workspace_bytes(B, H, n_ctx) + lib.ckv_dense_bwd_key_order_bytes(n_kv)
+        need += lib.ckv_dense_bwd_split_bytes(B, H, n_ctx, n_kv, D, a.dtype)   # depends on the device's compute units
         stream = torch.cuda.current_stream(q.device).cuda_stream
         ws = workspace(q.device, need, stream)
         a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()

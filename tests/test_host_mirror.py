@@ -177,3 +177,41 @@ def test_rope_flavours_agree_and_match_the_complex_rotation():
     # tables handed back are reused
     again, _, _ = layers[1].rope(x, pos, cos=cos_b, sin=layers[1].rope(x, pos)[2])
     assert torch.equal(again, b)
+
+
+def test_dense_operator_asks_for_scratch_sizes_on_the_tensors_device(monkeypatch):
+    """A size may depend on the device's compute units, so it is asked with the tensors' device current, in both
+    directions (several devices per process; no kernel is launched here)."""
+    from types import SimpleNamespace
+
+    from cascading_kv_cache_amd import flash_attention as fa
+
+    current, asked = [None], {}
+
+    class Device:
+        def __init__(self, device):
+            self.device = device
+
+        def __enter__(self):
+            self.before, current[0] = current[0], self.device
+
+        def __exit__(self, *_):
+            current[0] = self.before
+
+    class Lib:
+        def __getattr__(self, name):
+            def call(*_):
+                asked[name] = current[0]
+                return 0 if name in ("ckv_attn_dense", "ckv_attn_dense_bwd") else 256
+            return call
+
+    monkeypatch.setattr(torch.cuda, "device", Device)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda _: SimpleNamespace(cuda_stream=0))
+    monkeypatch.setattr(fa, "_require_device", lambda *_: None)
+    monkeypatch.setattr(fa, "workspace", lambda device, n, stream: torch.empty(n, dtype=torch.uint8))
+    monkeypatch.setattr(_abi, "lib", Lib)
+    q, k = torch.zeros(1, 2, 8, 64), torch.zeros(1, 2, 12, 64)
+    out, _, lse, mask = fa._forward(q, k, k, True, 1.0, torch.zeros(4, dtype=torch.bool), 0.9, True)
+    fa._backward(q, k, k, out, lse, mask, out, 1.0)
+    assert {"ckv_dense_workspace_bytes", "ckv_dense_bwd_split_bytes", "ckv_attn_dense", "ckv_attn_dense_bwd"} <= set(asked)
+    assert set(asked.values()) == {q.device}, asked
