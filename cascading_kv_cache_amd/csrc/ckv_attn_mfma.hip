@@ -1646,11 +1646,14 @@ int run_mfma(const MfmaProblem& mp, hipStream_t stream) {
         cp.nbkv = (int)(mp.B * mp.KVH);
         cp.xcd_aware = cp.nbkv % 8 == 0;
         // Two heads per workgroup where the group allows it: the keys a workgroup holds in registers and its pipeline
-        // start serve twice the work.  With short chunks that matters less than an even last round (509 rows x 16 K
-        // keys x 8 kv heads: 1072 workgroups of two heads on 512 places 136 us, 2144 of one head 95 us; 488 rows over a
-        // cache that holds 1000 tokens 90 -> 52 us); 2048 rows x 16 K keys x 16 kv heads are level (563 and 559 us), and
-        // with longer chunks two heads are 1.4 % ahead.
-        cp.gsplit = (mp.Q >= 2048 && G % 2 == 0 && G >= 4) ? G / 2 : G;
+        // start serve twice the work.  That pays once the launch has rounds enough for an uneven last one to cost little; a
+        // round is two workgroups per compute unit, and the line is at four rounds of such workgroups.  Score kernel in us
+        // with one and two heads, 32 heads on 8 kv heads, B streams x rows x slots, by rounds of two heads:
+        //   0.5 (1 x 2048 x 2 K)  173  332     2.1 (1 x 509 x 16 K)  77  103     2.5 (1 x 4096 x 16 K)  550  767
+        //   4.2 (2 x 509 x 16 K) 134  134      4.6 (2 x 2048 x 16 K) 510  508    8.0 (1 x 128 x 64 K)  92  75
+        //   8.5 (1 x 4096 x 64 K) 1815 1814    16 (2 x 33 x 64 K) 190  145       16 (2 x 1500 x 64 K) 1394 1363
+        const int64_t of_two = (int64_t)cp.nkb * cp.nbkv * (G / 2);
+        cp.gsplit = (G % 2 == 0 && G >= 4 && of_two >= 4 * 2 * (int64_t)cus) ? G / 2 : G;
         const dim3 grid((unsigned)(cp.nkb * cp.nbkv * cp.gsplit));
         const int lds = 2 * cs_stage(kD) + (cp.wnew_uniform ? 0 : (int)mp.Q * 4);
         if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(colsum_mfma_kernel<T, kD>), lds)) return rc;

@@ -800,8 +800,9 @@ constexpr int kOneThreads = 1024, kOneWaves = kOneThreads / CKV_WAVE;
 // against 13.4 us; 128 units of 32K slots: 18 against 12.5 us).
 constexpr int kOneMinUnits = 32;
 // ... unless the slots are few too: from 8 units (one stream of eight kv heads) with up to this many slots each the ids are
-// written in less time than a second launch takes (8 units of 2K slots: 10.1 us for plan and
-// apply, 7.3 in one launch; of 16K slots: 9.8 and 8.0; of 64K slots the two launches are ahead, see above).
+// written in less time than a second launch takes.  A step in two launches and in one, us, 8 / 16 / 28 units: 2 K slots
+// 10.5 / 10.5 / 10.5 and 8.4 / 8.4 / 8.5; 16 K 10.3 / 10.5 / 10.7 and 9.4 / 9.6 / 9.7; 32 K 10.5 / 10.6 / 11.4 and
+// 10.8 / 10.9 / 11.4; 64 K 10.7 / 11.7 / 13.0 and 13.2 / 13.8 / 14.8.
 constexpr int kOneFewUnits = 8;
 constexpr int64_t kOneMaxSlots = 16384;
 
