@@ -666,13 +666,33 @@ def test_dense_operator_with_sorted_keys(D, Z, H, N_CTX, N_CACHED, masking):
 @pytest.mark.parametrize("D,H,KVH,W,C,steps", [
     # (the first chunk is the longest: the reference's position ids of later chunks are a prefix of the first one's)
     (128, 8, 2, 32, 4, [130, 5, 33, 2, 31]),      # fewer key blocks than wavefronts, ragged rows, a cache that is filling
-    (64, 7, 1, 257, 2, [700, 40, 3, 257]),         # seven heads per kv head, key blocks shared out over workgroups
+    (64, 7, 1, 257, 2, [700, 40, 3, 257]),         # seven heads per kv head, one share of the keys throughout
+    (128, 8, 2, 512, 4, [600, 40, 33, 500, 500, 500, 2]),   # from the second chunk on four shares, two thirds empty at first
+    (64, 4, 4, 512, 4, [600, 300, 40, 600, 600, 600, 17]),  # two to four shares, one head per kv head
     (128, 3, 3, 64, 1, [65, 64, 2]),               # one head per kv head
 ])
 def test_float32_on_the_matrix_cores(D, H, KVH, W, C, steps):
     """float32 chunks of head sizes 64 and 128 take the float32 matrix instructions: 32-row and 32-key blocks, shared
-    out over eight wavefronts and, with few rows, over workgroups.  Against the oracle with the float32 tolerances."""
+    out over eight wavefronts and, with fewer row tiles than compute units and at least 16 key blocks a share, over
+    workgroups (the first three rows stay below that, the others do not).  Against the oracle with the float32 tolerances."""
     run_teacher_forced(B=2, H=H, KVH=KVH, D=D, NS=4, W=W, C=C, Q=0, chunks=0, dtype=torch.float32, seed=41, steps=steps)
+
+
+@pytest.mark.parametrize("H,KVH,W,C,NS,eager,og,dtype,reduction,homogeneous,steps", [
+    (8, 2, 64, 4, 64, True, False, torch.bfloat16, "mean", False, [300, 129, 31, 2, 200, 64]),    # G = 4, fills and evicts
+    (14, 2, 128, 4, 4, False, False, torch.float16, "max", False, [260, 96, 96, 200, 59, 96]),    # G = 7, lazy fill
+    (4, 4, 64, 2, 8, True, False, torch.bfloat16, "median", True, [200, 33, 200, 7]),              # G = 1, homogeneous heads
+    (16, 2, 32, 8, 64, False, True, torch.float16, "mean", False, [150, 64, 64, 90, 27]),          # G = 8, original positions
+    (8, 2, 1024, 4, 4, True, False, torch.bfloat16, "mean", False, [320, 320, 309, 2000, 1500, 320]),   # keys in shares
+])
+def test_sixteen_bit_chunks_of_head_size_64(H, KVH, W, C, NS, eager, og, dtype, reduction, homogeneous, steps):
+    """16-bit chunks of head size 64 on the matrix cores: staging with rotation, groups of 1 to 8 heads, position ids per
+    (batch, kv head), sinks, chunk-key weights.  Streams against the oracle with the bounds of the streams above."""
+    big = steps.index(max(steps))   # the first chunk is the longest: the oracle's position ids of later ones are a prefix of its
+    steps = [steps[big]] + steps[:big] + steps[big + 1:]
+    led = run_teacher_forced(2, H, KVH, 64, NS, W, C, 0, 0, dtype, seed=47, eager=eager, std=0.7, steps=steps, reduction=reduction,
+                             homogeneous=homogeneous, do_og_pos=og)
+    assert og or led.flips <= flip_bound(led), led.summary()
 
 
 @pytest.mark.parametrize("H,KVH,dtype", [(8, 2, torch.bfloat16), (3, 1, torch.float16), (7, 1, torch.bfloat16)])

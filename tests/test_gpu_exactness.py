@@ -125,6 +125,10 @@ def staged(cache, q, k, v):
 CASCADE = [
     # B, H, KVH, D, NS, W, C, filled, Q, dtype
     (1, 8, 2, 64, 4, 64, 4, 1000, 96, BF16), (2, 14, 2, 64, 4, 128, 2, 200, 77, F16), (1, 3, 3, 64, 64, 256, 8, 4000, 300, BF16),
+    # float32 with fewer row tiles (32 rows each) than compute units and at least 16 key blocks (32 keys each) a share: the
+    # keys of a tile are shared out over 4, 2 (the cache half empty) and 8 workgroups
+    (1, 8, 2, 128, 4, 512, 4, 4000, 40, F32), (1, 7, 1, 64, 4, 1024, 1, 500, 33, F32), (1, 4, 1, 128, 4, 1024, 4, 3000, 100, F32),
+    (1, 32, 8, 128, 4, 128, 4, 1000, 256, F32),   # one share
 ]
 
 
