@@ -95,6 +95,24 @@ def test_dense_backward_of_head_size_64_is_rounded_once(Z, H, n_ctx, n_kv, grad_
     assert_rounded_once(dq[fits], want[fits], spread[fits], n_kv, "dq")
 
 
+@pytest.mark.parametrize("dtype", [BF16, F16])
+@pytest.mark.parametrize("scale", [-0.5, 0.0, 1e-3, 3.0])
+def test_any_softmax_scale_of_head_size_64(scale, dtype):
+    """The scale joins in float32 behind the logits: negative, zero (every visible key weighs the same), small and large."""
+    from cascading_kv_cache_amd import flash_attention as fa
+
+    q, k, v, mask, do = dense_case(1, 3, 150, 700 + 150, 64, dtype)
+    out, scores, lse, m = fa._forward(q, k, v, True, scale, mask, 0.9, True)
+    ref, p, ref_lse, spread = exact_attention(q, k, v, visible(150, 850, mask), scale)
+    assert (lse.double() - ref_lse).abs().max().item() <= 4e-6 * max(1.0, abs(scale) * 8)    # logits of up to thirty
+    assert_rounded_once(out, ref, spread * max(1.0, abs(scale) * 4), 850, "out")
+    dq, dk, dv = fa._backward(q, k, v, out, lse, m, do, scale)
+    dp, delta = torch.matmul(do.double(), v.double().transpose(2, 3).contiguous()), (out.double() * do.double()).sum(-1, keepdim=True)
+    ds = p * (dp - delta) * scale
+    size = (p * (dp.abs() + delta.abs() + 1.0) * scale).square() * max(1.0, abs(scale) * 4) ** 2
+    assert_rounded_once(dq, torch.matmul(ds, k.double()), torch.matmul(size, k.double().square()).sqrt(), 850, "dq")
+
+
 def one_layer(B, KVH, D, NS, W, C, dtype):
     from cascading_kv_cache_amd.cascading_cache import CascadingKVCache
 
