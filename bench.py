@@ -592,7 +592,7 @@ def run_cpu_config1():
 
 def run_gpu_config1(device):
     """Config 1 on the device, beside `cpu_config1`: the same float32 stream (B=1, 32q/8kv heads, head_dim 128,
-    sink 4, window 512 in 4 cascades, 4096 tokens in 16 chunks of 256) through the library's fp32-math kernels."""
+    sink 4, window 512 in 4 cascades, 4096 tokens in 16 chunks of 256) through the library's float32 kernels on the matrix cores."""
     from cascading_kv_cache_amd.cascade_attention import cascade_attention, default_inv_freq
     from cascading_kv_cache_amd.cascading_cache import CascadingKVCache
 
@@ -615,8 +615,8 @@ def run_gpu_config1(device):
     dt = min(stream() for _ in range(3))
     assert cache._seen_host[0] == 4096 and not bool(cache.mask[0].any())
     return dict(value=4096 / dt, unit="tokens/s", seconds=dt, dtype="f32",
-                sample="config 1 in full on the device: 4096 tokens in 16 chunks of 256, float32 (fp32-math kernels, "
-                       "no matrix cores); best of 3 streams")
+                sample="config 1 in full on the device: 4096 tokens in 16 chunks of 256, float32 (float32 "
+                       "matrix instructions); best of 3 streams")
 
 
 def run_short_strides(cache, dtype, device):

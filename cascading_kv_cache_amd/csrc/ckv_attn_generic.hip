@@ -1,5 +1,5 @@
-// fp32-math attention kernels for every dtype: the parity path for float32 caches and the
-// fallback for shapes the MFMA kernels do not take.  Also the small shared stages: score-sum
+// fp32-math attention kernels on the vector ALU for every dtype: the fallback for shapes the kernels on the matrix cores
+// (16-bit and float32) do not take.  Also the small shared stages: score-sum
 // weights, the rotate+gather prologue, and the head-reduction / EMA epilogue.
 #include "ckv_attn_internal.h"
 

@@ -30,8 +30,8 @@ struct CoreProblem {
     int dtype;
 };
 
-// fp32-math kernels for every dtype and head size (<= 256): the parity path for float32 caches
-// and the fallback for shapes the MFMA kernels do not cover.
+// fp32-math kernels on the vector ALU for every dtype and head size (<= 256): the fallback for shapes the kernels on the
+// matrix cores (16-bit and float32) do not cover.
 int launch_core_generic(const CoreProblem& p, hipStream_t stream);
 
 // The same in float32 on the matrix cores: head_dim 64 and 128, rows of 16-byte pieces, lse wanted.  part_o / part_l:

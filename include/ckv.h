@@ -205,6 +205,8 @@ typedef struct ckv_attn_args {
     int64_t workspace_bytes;
 } ckv_attn_args;
 
+/* Scratch of a call on the current device.  Where few query rows would leave the chip idle this includes float32 partial
+ * results of the shares their keys are dealt out in: up to 256 MiB beyond the staged operands. */
 int64_t ckv_attn_workspace_bytes(int64_t B, int64_t H, int64_t KVH, int64_t Q, int64_t D,
                                  int64_t num_sink, int64_t S, int32_t dtype);
 
@@ -240,6 +242,7 @@ typedef struct ckv_dense_args {
                                       backward pass needs (the reference keeps M, flash_attention.py:272-276) */
 } ckv_dense_args;
 
+/* as ckv_attn_workspace_bytes */
 int64_t ckv_dense_workspace_bytes(int64_t B, int64_t H, int64_t n_ctx, int64_t n_kv, int64_t D,
                                   int32_t dtype);
 
