@@ -14,10 +14,18 @@
 // the products run on v_mfma_f32_32x32x2, whose B operand is an accumulator register as it stands and whose A operand is
 // the same transposed read, widened to float32.  16-bit terms that add up to the float32 value, as the forward kernel takes,
 // would need a scale of their own for dS, which has no largest value, and would turn an infinite gradient into NaN.
-// 8 heads x 1000 rows x 5095 keys in float16: dq 32 -> 61 us, dk/dv 40 -> 101 (the vector kernels, to the same error: 2520
+// 8 heads x 1000 rows x 5095 keys in float16: dq 32 -> 55 us, dk/dv 40 -> 91 (the vector kernels, to the same error: 2520
 // and 1838).  These products bound both kernels: 2048 and 4096 of the 2304 and 4352 cycles of matrix work per 32 x 32 block,
 // and unlike the 16-bit instructions they do not run beside vector instructions (matrix pipe 43 and 50 % busy, 0 % of the
 // time together with the vector ALU).
+//
+// What bounds them (64 heads x 1024 rows x 8704 visible keys, 128 dims, bf16: dq 548 -> 440 us, dk/dv 770 -> 620).  Vector work
+// beside the matrix work: both take most of a block's time and overlap only where a wavefront alternates them, so an
+// element costs one fused multiply-add, one exponential, one multiplication and half a conversion per product (no
+// subtraction of delta, no scale, no mask in a block that every row sees, no addresses), where it was twice that.  The
+// copies: 100 to 170 cycles each at the issue, whatever else the wavefront does (let out one by one between matrix
+// instructions: dq 514 us, dk/dv level); dq has them two blocks ahead.  At 2.1 GHz and 56 % matrix work dq is within reach
+// of the clock's power limit.  Reads from LDS are not it: 4 instead of 2 matrix instructions ahead, dk/dv level.
 //
 // The A operands K^T, Q^T and dO^T are read from the row-major tiles in LDS with the transposing read
 // ds_read_b64_tr_b16: lane i of a 16-lane group receives element [4e + i/4][i%4] (e = 0..3) of the 16 x 4 matrix
@@ -42,6 +50,7 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef short s16x4_t __attribute__((ext_vector_type(4)));
 
 constexpr int kBlk = 32;              // rows of a streamed block
@@ -49,6 +58,7 @@ constexpr int kWaves = 4;             // wavefronts of a workgroup, 32 stationar
 constexpr int kThreads = kWaves * CKV_WAVE;
 constexpr int kOwn = kWaves * 32;     // stationary rows of a workgroup
 constexpr int kAhead = 3, kKvAhead = 2;  // matrix instructions between an operand's read from LDS and its use
+constexpr int kDqStages = 3;          // stages of K and V blocks of the dq kernel: copies two blocks ahead
 constexpr float kLog2e = 1.4426950408889634f;
 template <int kHD>
 struct Geo {
@@ -58,7 +68,8 @@ struct Geo {
     // dynamic LDS of the dk/dv kernel: two stages of (Q, dO) tiles, the per-row scalars of both stages, V^T operands
     static constexpr int kDkdvRowv = 2 * 2 * kTile;
     static constexpr int kDkdvV = kDkdvRowv + 2 * 2 * kBlk * (int)sizeof(float);
-    static constexpr int kDkdvLds = kDkdvV + kWaves * (kHD / 16) * CKV_WAVE * 16;
+    static constexpr int kParked = kHD == 128 ? 2 : 0;   // K^T operands that are kept there too: 8 registers that would spill
+    static constexpr int kDkdvLds = kDkdvV + kWaves * (kHD / 16 + kParked) * CKV_WAVE * 16;
 };
 
 template <typename T>
@@ -145,8 +156,8 @@ struct Keys {
 };
 
 // A 32-row block of a (rows, kHD) tensor into a tile, global -> LDS without registers, 1 KiB per instruction; a
-// wavefront copies kRowBytes / 128 of them, lane i of copy j one slot of row block_row(wave, lane, j).  Rows at or past
-// `limit` repeat row limit - 1 (finite values; whatever is computed from them is masked).  The caller waits with vmcnt(0)
+// wavefront copies kRowBytes / 128 of them, lane i of copy j one slot of row block_row(wave, lane, j).  Rows past row `last`
+// of the block repeat it (finite values; whatever is computed from them is masked).  The caller waits with vmcnt(0)
 // before the barrier that publishes the tile.
 template <int kHD>
 __device__ inline int block_row(int wave, int lane, int j) {
@@ -154,15 +165,11 @@ __device__ inline int block_row(int wave, int lane, int j) {
     return kPer * (kHD / 64 * wave + j) + lane / Geo<kHD>::kPieces;
 }
 template <int kHD>
-__device__ inline void copy_block(const char* base, int64_t row_bytes, int64_t first, int64_t limit, uint32_t tile_lds,
-                                  int wave, int lane) {
-    const char* blk = base + first * row_bytes;  // uniform
+__device__ inline void copy_block(const char* blk, uint32_t row_bytes, int last, uint32_t tile_lds, int wave, int lane) {
 #pragma unroll
     for (int j = 0; j < kHD / 64; j++) {
-        const int row = block_row<kHD>(wave, lane, j);
-        int64_t rr = row;
-        if (first + rr > limit - 1) rr = limit - 1 - first;
-        const uint32_t voff = (uint32_t)(rr * row_bytes) + (uint32_t)(swz<kHD>(row, lane % Geo<kHD>::kPieces) << 4);
+        const int row = block_row<kHD>(wave, lane, j), rr = row < last ? row : last;
+        const uint32_t voff = (uint32_t)rr * row_bytes + (uint32_t)(swz<kHD>(row, lane % Geo<kHD>::kPieces) << 4);
         async_copy16(blk, voff, tile_lds + (uint32_t)((kHD / 64 * wave + j) * 1024));
     }
 }
@@ -179,46 +186,48 @@ __device__ inline void copy_rows(const char* base, uint32_t row_bytes, const uin
     }
 }
 
-// A operand of a product that contracts over the head dims: row lane%32 of the tile, dims 16 ds + 8 (lane/32) .. +7
-template <int kHD>
-__device__ inline uint4 row_operand(const unsigned char* tile, int lane, int ds) {
-    const int row = lane & 31;
-    return *reinterpret_cast<const uint4*>(tile + row * Geo<kHD>::kRowBytes + swz<kHD>(row, 2 * ds + (lane >> 5)) * 16);
-}
-
-// A operand of a product that contracts over the rows of the tile: dim 32 db + lane%32 of rows
-// 16 s + 8 a + 4 (lane/32) + e (elements 4 a + e), the order in which the packed B operand holds them.
-// `tr_base[a]` is the lane's address for db = 0, s = 0; blocks of 32 dims flip bits 2-3 of the slot.
-template <int kHD>
-__device__ inline uint4 col_operand(uint32_t tile_lds, const int (&tr_base)[2], int s, int db) {
-    uint4 r;
+// Where a lane's operands lie inside a tile; the tile itself is a constant offset of the instruction, so that a read costs no
+// address arithmetic (an addition per read was a seventh of the vector work of a block).
+//   row[ds]    A operand of a product that contracts over the head dims: row lane%32, dims 16 ds + 8 (lane/32) .. +7
+//   col[db][a] A operand of a product that contracts over the rows of the tile: dim 32 db + lane%32 of rows
+//              16 s + 8 a + 4 (lane/32) + e (elements 4 a + e), the order in which the packed B operand holds them;
+//              blocks of 32 dims flip bits 2-3 of the slot, step s is 16 rows further
+// kTight: registers are kept for 64 dims of columns only, those of the other 64 are worked out at the read.
+template <int kHD, bool kTight>
+struct Operands {
+    static constexpr int kCols = kTight && kHD == 128 ? 2 : kHD / 32;
+    uint32_t row[kHD / 16], col[kCols][2];
+    __device__ Operands(uint32_t lds0, int lane) {
+        const int r = lane & 31, h = lane >> 5, g16 = (lane >> 4) & 1, rl = lane & 15;
 #pragma unroll
-    for (int a = 0; a < 2; a++) {
-        const uint32_t addr = tile_lds + (uint32_t)((tr_base[a] ^ (db << 6)) + s * 16 * Geo<kHD>::kRowBytes);
-        const s16x4_t v =
-            __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_t*)(uintptr_t)addr);
-        const uint2 u = __builtin_bit_cast(uint2, v);
-        if (a == 0) {
-            r.x = u.x;
-            r.y = u.y;
-        } else {
-            r.z = u.x;
-            r.w = u.y;
+        for (int ds = 0; ds < kHD / 16; ds++) row[ds] = lds0 + (uint32_t)(r * Geo<kHD>::kRowBytes + swz<kHD>(r, 2 * ds + h) * 16);
+#pragma unroll
+        for (int a = 0; a < 2; a++) {
+            const int cr = 8 * a + 4 * h + (rl >> 2);              // + 16 s
+            const int piece = 2 * g16 + ((rl & 3) >> 1);           // + 4 db
+            const uint32_t base = (uint32_t)(cr * Geo<kHD>::kRowBytes + swz<kHD>(cr, piece) * 16 + 8 * (rl & 1));
+#pragma unroll
+            for (int db = 0; db < kCols; db++) col[db][a] = lds0 + (base ^ (uint32_t)(db << 6));
         }
-    }
-    return r;
-}
-
-template <int kHD>
-__device__ inline void col_operand_setup(int lane, int (&tr_base)[2]) {
-    const int h = lane >> 5, g16 = (lane >> 4) & 1, rl = lane & 15;
 #pragma unroll
-    for (int a = 0; a < 2; a++) {
-        const int row = 8 * a + 4 * h + (rl >> 2);             // + 16 s
-        const int piece = 2 * g16 + ((rl & 3) >> 1);           // + 4 db
-        tr_base[a] = row * Geo<kHD>::kRowBytes + swz<kHD>(row, piece) * 16 + 8 * (rl & 1);
+        for (int ds = 0; ds < kHD / 16; ds++) asm("" : "+v"(row[ds]));   // kept, not worked out again at every read
+#pragma unroll
+        for (int db = 0; db < kCols; db++) asm("" : "+v"(col[db][0]), "+v"(col[db][1]));
     }
-}
+    __device__ uint4 row_op(uint32_t tile, int ds) const { const u32x4 v = *(const __attribute__((address_space(3))) u32x4*)(uintptr_t)(row[ds] + tile);
+        return make_uint4(v[0], v[1], v[2], v[3]); }
+    __device__ uint4 col_op(uint32_t tile, int s, int db) const {
+        uint2 u[2];
+#pragma unroll
+        for (int a = 0; a < 2; a++) {
+            uint32_t at = col[db % kCols][a];
+            if (db >= kCols) asm volatile("v_xor_b32 %0, 0x80, %1" : "=v"(at) : "v"(at));   // volatile: not kept in a register
+            u[a] = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_t*)(uintptr_t)(
+                                                 at + tile + (uint32_t)(s * 16 * Geo<kHD>::kRowBytes))));
+        }
+        return make_uint4(u[0].x, u[0].y, u[1].x, u[1].y);
+    }
+};
 
 template <typename T>
 __device__ inline uint4 pack8(const f32x16& v, int s) {
@@ -270,9 +279,13 @@ struct Weights<T, 64> {
 // bits [0, n) set, for 0 <= n <= 32
 __device__ inline uint32_t low_bits(int n) { return n >= 32 ? 0xffffffffu : ((1u << n) - 1u); }
 
+// dk: the softmax scale multiplies dS, so that float16 dS stays in range as it always has, or the finished sum
+template <typename T, int kHD>
+constexpr bool kScaleInside = kHD == 128 && std::is_same<T, __half>::value;
+
 // v if bit `bit` of `word` is set, else +0: a sign-extended one-bit field and a bitwise and
 __device__ inline float keep_if_bit(float v, uint32_t word, int bit) {
-    const int32_t m = (int32_t)(word << (31 - bit)) >> 31;
+    const int32_t m = __builtin_amdgcn_sbfe((int32_t)word, bit, 1);
     return __uint_as_float(__float_as_uint(v) & (uint32_t)m);
 }
 
@@ -288,20 +301,23 @@ __device__ inline f32x16 zero16() {
 // ---------------------------------------------------------------------------------------------
 template <typename T, int kHD, bool kWide>
 __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dq_kernel(BwdMfmaParams p) {
-    constexpr int kTile = Geo<kHD>::kTile;
-    __shared__ __attribute__((aligned(16))) unsigned char smem[2][2][kTile];  // [stage][K, V]
+    constexpr int kTile = Geo<kHD>::kTile, kStage = 2 * kTile;   // K, V
+    constexpr int kCopies = 2 * (kHD / 64);                      // of a wavefront and block
+    constexpr int kMine = kBlk / kWaves;                         // rows of a block that a wavefront copies
+    __shared__ __attribute__((aligned(16))) unsigned char smem[kDqStages * (kStage + kBlk * (int)sizeof(int))];
     const ckv_dense_bwd_args& a = p.a;
-    const int tid = threadIdx.x, wave = tid / CKV_WAVE, lane = tid % CKV_WAVE, h = lane >> 5;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / CKV_WAVE), lane = tid % CKV_WAVE, h = lane >> 5;
     const Keys keys(p);
-    const int64_t n_ctx = a.n_ctx, n_cached = keys.n_cached;
+    const int64_t n_ctx = a.n_ctx;
+    const int n_cached = (int)keys.n_cached, n_seen = (int)keys.n_seen;   // below 2^31, see bwd_mfma_supported
     const Unit unit = unit_of(p);
     const int64_t bh = unit.bh, b = bh / a.H, hd = bh % a.H;
     const int share = unit.x % p.n_split;
-    const int64_t m_wg = (int64_t)(unit.x / p.n_split) * kOwn;
-    const int64_t m_lane = m_wg + wave * 32 + (lane & 31);  // this lane's query
+    const int m_wg = unit.x / p.n_split * kOwn;
+    const int m_lane = m_wg + wave * 32 + (lane & 31);  // this lane's query
     const char* kb = reinterpret_cast<const char*>(a.k) + (b * a.kv_stride[0] + hd * a.kv_stride[1]) * 2;
     const char* vb = reinterpret_cast<const char*>(a.v) + (b * a.kv_stride[0] + hd * a.kv_stride[1]) * 2;
-    const int64_t kv_row = a.kv_stride[2] * 2;
+    const uint32_t row_bytes = (uint32_t)(a.kv_stride[2] * 2);
 
     // stationary B operands: Q^T and dO^T of this lane's query, dims 16 ds + 8 h .. +7
     uint4 qreg[kHD / 16], greg[kHD / 16];
@@ -320,84 +336,94 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dq_kernel(BwdMfmaParams 
         }
     }
     const bool row_ok = m_lane < n_ctx;
-    const float nlse2 = row_ok ? -a.lse[bh * n_ctx + m_lane] * kLog2e : 0.f;
-    const float delta = row_ok ? p.delta[bh * n_ctx + m_lane] : 0.f;
+    // The magnitude of the softmax scale rides on the exponent (nothing here needs P without it), its sign on the result;
+    // the products of V and dO start from -delta.  That leaves one multiplication per element beside the exponential.
+    const float nl = row_ok ? fmaf(-a.lse[bh * n_ctx + m_lane], kLog2e, __builtin_amdgcn_logf(fabsf(a.scale))) : 0.f;
     const float c2 = a.scale * kLog2e;
+    f32x16 neg_delta;
+    {
+        const float d = row_ok ? -p.delta[bh * n_ctx + m_lane] : 0.f;
+#pragma unroll
+        for (int i = 0; i < 16; i++) neg_delta[i] = d;
+        asm volatile("" : "+v"(neg_delta));   // 16 registers to start from, not 16 moves a block
+    }
 
-    int tr_base[2];
-    col_operand_setup<kHD>(lane, tr_base);
-    const uint32_t lds0 = lds_address(&smem[0][0][0]);
+    const uint32_t lds0 = lds_address(smem);
+    const Operands<kHD, false> op(lds0, lane);
 
     f32x16 dq[kHD / 32];
 #pragma unroll
     for (int db = 0; db < kHD / 32; db++) dq[db] = zero16();
 
     // keys past the diagonal of the workgroup's last row are visible to none of its rows
-    int64_t m_last = m_wg + kOwn - 1;
-    if (m_last > n_ctx - 1) m_last = n_ctx - 1;
-    const int64_t n_end = n_cached + m_last + 1;
-    const int nblk_all = (int)((n_end + kBlk - 1) / kBlk);
+    int m_last = m_wg + kOwn - 1;
+    if (m_last > (int)n_ctx - 1) m_last = (int)n_ctx - 1;
+    const int nblk_all = (int)(((int64_t)n_cached + m_last + kBlk) / kBlk);
     // this workgroup's share of them: an equal stretch (an empty one leaves zeros)
     const int per_share = (nblk_all + p.n_split - 1) / p.n_split;
     const int blk0 = share * per_share, nblk = blk0 + per_share < nblk_all ? blk0 + per_share : nblk_all;
 
-    // Which keys of a block any query may see, and the rows this lane copies.  Both are requested a block before the
-    // copies that need them and looked at after this block's work, so that nothing in between waits for memory.
-    auto key_bit = [&](int64_t n0) -> uint32_t { return keys.visible(n0 + (lane & 31)) ? 1u : 0u; };
-    auto rows_of = [&](int64_t n0, uint32_t(&r)[kHD / 64]) {
-#pragma unroll
-        for (int j = 0; j < kHD / 64; j++) {
-            int64_t i = n0 + block_row<kHD>(wave, lane, j);
-            if (i > keys.n_seen - 1) i = keys.n_seen - 1;  // a chunk key: finite values, and no query looks at this copy
-            r[j] = (uint32_t)keys.row_of(i);
-        }
+    // Blocks are copied two ahead into three stages.  With an order the row numbers of a wavefront's eight rows of a block
+    // come to LDS the same way, three blocks ahead, so that no load in the loop is one whose result the compiler would
+    // wait for together with the copies behind it.
+    const uint32_t mine = lds0 + (uint32_t)(kDqStages * kStage + wave * kMine * (int)sizeof(int));
+    constexpr uint32_t kSlot = kBlk * sizeof(int);
+    const int mine_lane = kHD == 128 ? lane / 16 : lane / 8;   // of copy 0; copy j takes row 4 j + this one
+    auto clamped = [&](int i) { return i < n_seen ? i : n_seen - 1; };   // a chunk key: finite values, and no query looks at this copy
+    auto request_rows = [&](int blk, int slot) {
+        if (keys.order && lane < kMine)
+            async_copy4(keys.order, (uint32_t)clamped(blk * kBlk + wave * kMine + lane) * 4u, mine + (uint32_t)slot * kSlot);
     };
-    const uint32_t row_bytes = (uint32_t)kv_row;
-    uint32_t rows_next[kHD / 64];
-    rows_of((int64_t)blk0 * kBlk, rows_next);
-    uint32_t vis = (uint32_t)__ballot(key_bit((int64_t)blk0 * kBlk) != 0u);
-    copy_rows<kHD, kWide>(kb, row_bytes, rows_next, lds0 + (uint32_t)((blk0 & 1) * 2 * kTile), wave, lane);
-    copy_rows<kHD, kWide>(vb, row_bytes, rows_next, lds0 + (uint32_t)((blk0 & 1) * 2 * kTile + kTile), wave, lane);
-    rows_of((int64_t)(blk0 + 1) * kBlk, rows_next);
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-    __syncthreads();
-    for (int blk = blk0; blk < nblk; blk++) {
-        const int st = blk & 1;
-        const int64_t n0 = (int64_t)blk * kBlk;
-        uint32_t kb_next = 0u;
-        if (blk + 1 < nblk) {  // the other stage was last read before the barrier that ended the step before
-            uint32_t rows_now[kHD / 64];
+    auto rows_of = [&](int blk, int slot, uint32_t(&r)[kHD / 64]) {
 #pragma unroll
-            for (int j = 0; j < kHD / 64; j++) rows_now[j] = rows_next[j];
-            kb_next = key_bit(n0 + kBlk);
-            rows_of(n0 + 2 * kBlk, rows_next);
-            __builtin_amdgcn_sched_barrier(0);
-            copy_rows<kHD, kWide>(kb, row_bytes, rows_now, lds0 + (uint32_t)((st ^ 1) * 2 * kTile), wave, lane);
-            copy_rows<kHD, kWide>(vb, row_bytes, rows_now, lds0 + (uint32_t)((st ^ 1) * 2 * kTile + kTile), wave, lane);
+        for (int j = 0; j < kHD / 64; j++)
+            r[j] = keys.order ? *(const __attribute__((address_space(3))) uint32_t*)(uintptr_t)(mine + (uint32_t)slot * kSlot + (uint32_t)(4 * j + mine_lane) * 4u)
+                              : (uint32_t)clamped(blk * kBlk + wave * kMine + 4 * j + mine_lane);
+    };
+    auto copy = [&](const uint32_t(&r)[kHD / 64], int st) {
+        copy_rows<kHD, kWide>(kb, row_bytes, r, lds0 + (uint32_t)(st * kStage), wave, lane);
+        copy_rows<kHD, kWide>(vb, row_bytes, r, lds0 + (uint32_t)(st * kStage + kTile), wave, lane);
+    };
+    uint32_t rows_next[kHD / 64];   // of the block that is copied next
+    if (blk0 < nblk) {
+#pragma unroll
+        for (int i = 0; i < kDqStages; i++) request_rows(blk0 + i, i);
+        wait_copies<0>();
+        rows_of(blk0, 0, rows_next);
+        copy(rows_next, 0);
+        rows_of(blk0 + 1, 1, rows_next);
+        if (blk0 + 1 < nblk) copy(rows_next, 1);
+        rows_of(blk0 + 2, 2, rows_next);
+        if (blk0 + 1 < nblk) wait_copies<kCopies>();
+        else wait_copies<0>();
+    }
+    __syncthreads();
+    auto step = [&](auto stage_tag, int blk) {
+        constexpr int st = decltype(stage_tag)::value;
+        constexpr uint32_t kt = st * kStage, vt = kt + kTile;
+        const int n0 = blk * kBlk;
+        const bool more = blk + 2 < nblk;
+        if (more) {  // the stage was last read before the barrier that ended the step before
+            request_rows(blk + 3, st);
+            copy(rows_next, (st + 2) % kDqStages);
         }
+        // Which keys of the block any query may see: all of them in front of the chunk when they were sorted.
+        uint32_t vis = 0xffffffffu;
+        if (!keys.order) vis = (uint32_t)__ballot(keys.visible(n0 + (lane & 31)));
         __builtin_amdgcn_sched_barrier(0);
         // keys of this block that are chunk keys past this wavefront's last row: nothing to do for it
-        const bool chunk_part = n0 + kBlk > n_cached;
-        // chunk key r of the block is visible to this lane's query iff r <= r_last (every r when the block is cached)
-        int64_t r_last64 = m_lane + n_cached - n0;
-        if (r_last64 > kBlk) r_last64 = kBlk;
-        if (r_last64 < -1) r_last64 = -1;
-        const int r_last = (int)r_last64;
-        const int r_cached = n_cached - n0 >= kBlk ? kBlk : (n_cached > n0 ? (int)(n_cached - n0) : 0);  // r < r_cached: cached
-        const int64_t wave_last = m_wg + wave * 32 + 31;
-        const bool dead = vis == 0u || (n0 >= n_cached && n0 - n_cached > wave_last);
+        const bool dead = vis == 0u || (n0 >= n_cached && n0 - n_cached > m_wg + wave * 32 + 31);
+        // Written in issue order: an operand is read from LDS kAhead matrix instructions before the one that takes it, the
+        // exponentials run beside the products of V and dO, the second half of dS beside the products of the first.
+        constexpr int kRow = kHD / 16, kDB = kHD / 32;
         if (!dead) {
-            const unsigned char* kt = smem[st][0];
-            const unsigned char* vt = smem[st][1];
-            // Written in issue order: an operand is read from LDS kAhead matrix instructions before the one that takes it
-            // (one operand at a time beside a matrix instruction, instead of four read and waited for; dk / dv 821 -> 760 us, dq level
-            // with 128 dims and 6 % with 64), and the second half of the exponentials runs beside the products of the first.
-            constexpr int kRow = kHD / 16, kDB = kHD / 32;
-            const uint32_t kt_lds = lds0 + (uint32_t)(st * 2 * kTile);
-            f32x16 s = zero16(), dp = zero16();
+            f32x16 s = zero16(), dp = neg_delta;
             uint4 ops[2 * kRow], cops[2 * kDB];
-            auto row_op = [&](int k) { return row_operand<kHD>(k & 1 ? vt : kt, lane, k >> 1); };
-            auto col_op = [&](int k) { return col_operand<kHD>(kt_lds, tr_base, k / kDB, k % kDB); };
+            auto row_op = [&](int k) { return op.row_op(k < kRow ? kt : vt, k % kRow); };
+            auto col_op = [&](int k) { return op.col_op(kt, k / kDB, k % kDB); };
+            auto weight = [&](int i) {
+                s[i] = __builtin_amdgcn_exp2f(fmaf(s[i], c2, nl));
+            };
 #pragma unroll
             for (int k = 0; k < kAhead; k++) ops[k] = row_op(k);
             __builtin_amdgcn_sched_barrier(0);
@@ -405,44 +431,61 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dq_kernel(BwdMfmaParams 
             for (int k = 0; k < 2 * kRow; k++) {
                 if (k + kAhead < 2 * kRow) ops[k + kAhead] = row_op(k + kAhead);
                 else cops[k + kAhead - 2 * kRow] = col_op(k + kAhead - 2 * kRow);
-                if (k & 1) dp = Mma<T>::mma(ops[k], greg[k >> 1], dp);
-                else s = Mma<T>::mma(ops[k], qreg[k >> 1], s);
+                if (k < kRow) s = Mma<T>::mma(ops[k], qreg[k], s);
+                else dp = Mma<T>::mma(ops[k], greg[k - kRow], dp);
+                if (k > kRow) {   // not beside the first, which the last logits are only just behind
+                    constexpr int kPer = (16 + kRow - 2) / (kRow - 1);
+#pragma unroll
+                    for (int i = (k - kRow - 1) * kPer; i < (k - kRow) * kPer && i < 16; i++) weight(i);
+                }
                 __builtin_amdgcn_sched_barrier(0);
             }
-            // A lane is a query: a row past the end spoils only its own accumulators, which are never stored, so
-            // no element tests its row.  A cached block with every key visible tests nothing at all.
-            auto products = [&](auto masked, uint32_t allow) {
-                f32x16 dsv;
-                auto element = [&](int i) {
-                    float pe = __builtin_amdgcn_exp2f(fmaf(s[i], c2, nlse2));
-                    if constexpr (decltype(masked)::value) pe = keep_if_bit(pe, allow, 8 * (i / 4) + (i % 4));
-                    dsv[i] = pe * (dp[i] - delta) * a.scale;
-                };
+            // A cached block with every key visible tests nothing.  A lane is a query: a row past the end spoils only its own
+            // accumulators, which are never stored, so no element tests its row.
+            if (vis != 0xffffffffu || n0 + kBlk > n_cached) {
+                // cached key r of the block is visible to all, chunk key r to this lane's query iff it is no later
+                const int cached = n_cached - n0, seen = cached + m_lane + 1;
+                const uint32_t allow = (vis & (low_bits(cached > 0 ? cached : 0) | low_bits(seen > 0 ? seen : 0))) >> (4 * h);
 #pragma unroll
-                for (int i = 0; i < 8; i++) element(i);
-                Weights<T, kHD> bop;
-                bop.set(dsv, 0);
-                __builtin_amdgcn_sched_barrier(0);
+                for (int i = 0; i < 16; i++) s[i] = keep_if_bit(s[i], allow, 8 * (i / 4) + (i % 4));
+            }
+            f32x16 dsv;
 #pragma unroll
-                for (int k = 0; k < 2 * kDB; k++) {
-                    if (k + kAhead < 2 * kDB) cops[k + kAhead] = col_op(k + kAhead);
-                    bop.accumulate(cops, k, dq);
-                    if (k < kDB) {
+            for (int i = 0; i < 8; i++) dsv[i] = s[i] * dp[i];
+            Weights<T, kHD> bop;
+            bop.set(dsv, 0);
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                        for (int i = 8 + k * (8 / kDB); i < 8 + (k + 1) * (8 / kDB); i++) element(i);
-                    }
-                    if (k == kDB - 1) bop.set(dsv, 1);
-                    __builtin_amdgcn_sched_barrier(0);
+            for (int k = 0; k < 2 * kDB; k++) {
+                if (k + kAhead < 2 * kDB) cops[k + kAhead] = col_op(k + kAhead);
+                bop.accumulate(cops, k, dq);
+                if (k < kDB) {
+#pragma unroll
+                    for (int i = 8 + k * (8 / kDB); i < 8 + (k + 1) * (8 / kDB); i++) dsv[i] = s[i] * dp[i];
                 }
-            };
-            uint32_t allow = vis;
-            if (chunk_part) allow &= low_bits(r_cached) | low_bits(r_last + 1);
-            products(std::true_type{}, allow >> (4 * h));
+                if (k == kDB - 1) bop.set(dsv, 1);
+                __builtin_amdgcn_sched_barrier(0);
+            }
         }
         __builtin_amdgcn_sched_barrier(0);
-        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wavefront's copies of the next block have landed
-        vis = (uint32_t)__ballot(kb_next != 0u);
+        if (more) {   // this wavefront's copies of the next block have landed, and the row numbers requested above
+            wait_copies<kCopies>();
+            rows_of(blk + 3, st, rows_next);
+        } else {
+            wait_copies<0>();
+        }
         __syncthreads();
+    };
+    for (int blk = blk0; blk < nblk; blk += kDqStages) {
+        step(std::integral_constant<int, 0>{}, blk);
+        if (blk + 1 < nblk) step(std::integral_constant<int, 1>{}, blk + 1);
+        if (blk + 2 < nblk) step(std::integral_constant<int, 2>{}, blk + 2);
+    }
+    if (a.scale < 0.f) {
+#pragma unroll
+        for (int db = 0; db < kHD / 32; db++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) dq[db][i] = -dq[db][i];
     }
     if (row_ok && p.n_split > 1) {
         float* out = p.part_dq + ((int64_t)share * a.B * a.H * n_ctx + bh * n_ctx + m_lane) * kHD;
@@ -491,20 +534,18 @@ template <typename T, int kHD>
 __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dkdv_kernel(BwdMfmaParams p) {
     constexpr int kTile = Geo<kHD>::kTile;
     extern __shared__ __attribute__((aligned(16))) unsigned char dyn_smem[];
-    typedef unsigned char (*TilePtr)[2][kTile];
     typedef float (*RowPtr)[2][kBlk];
-    TilePtr smem = reinterpret_cast<TilePtr>(dyn_smem);                                  // [stage][Q, dO]
-    RowPtr rowv = reinterpret_cast<RowPtr>(dyn_smem + Geo<kHD>::kDkdvRowv);                        // [stage][-lse log2 e, delta]
-    // the V^T operands of a wavefront's 32 keys, in operand order: [wave][ds][lane] 16 bytes each
-    uint4* vstat = reinterpret_cast<uint4*>(dyn_smem + Geo<kHD>::kDkdvV) + (threadIdx.x / CKV_WAVE) * (kHD / 16) * CKV_WAVE;
+    RowPtr rowv = reinterpret_cast<RowPtr>(dyn_smem + Geo<kHD>::kDkdvRowv);                        // [stage][-lse log2 e, -delta]
+    // the V^T operands of a wavefront's 32 keys and the first of K^T, in operand order: [wave][ds][lane] 16 bytes each
+    uint4* vstat = reinterpret_cast<uint4*>(dyn_smem + Geo<kHD>::kDkdvV) + __builtin_amdgcn_readfirstlane(threadIdx.x / CKV_WAVE) * (kHD / 16 + Geo<kHD>::kParked) * CKV_WAVE;
     const ckv_dense_bwd_args& a = p.a;
-    const int tid = threadIdx.x, wave = tid / CKV_WAVE, lane = tid % CKV_WAVE, h = lane >> 5;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / CKV_WAVE), lane = tid % CKV_WAVE, h = lane >> 5;
     const Keys keys(p);
-    const int64_t n_ctx = a.n_ctx, n_kv = a.n_kv, n_cached = keys.n_cached;
+    const int n_ctx = (int)a.n_ctx, n_cached = (int)keys.n_cached;   // below 2^31, see bwd_mfma_supported
     const Unit unit = unit_of(p);
     const int64_t bh = unit.bh, b = bh / a.H, hd = bh % a.H;
-    const int64_t n_wg = (int64_t)unit.x * kOwn;
-    const int64_t n_lane = n_wg + wave * 32 + (lane & 31);  // this lane's key
+    const int n_wg = unit.x * kOwn;
+    const int n_lane = n_wg + wave * 32 + (lane & 31);  // this lane's key
     const bool key_ok = keys.visible(n_lane);
     const char* qb = reinterpret_cast<const char*>(a.q) + (b * a.q_stride[0] + hd * a.q_stride[1]) * 2;
     const char* gb = reinterpret_cast<const char*>(a.dout) + (b * a.dout_stride[0] + hd * a.dout_stride[1]) * 2;
@@ -512,154 +553,148 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dkdv_kernel(BwdMfmaParam
     const float* lse = a.lse + bh * n_ctx;
     const float* dl = p.delta + bh * n_ctx;
 
-    // stationary B operands: K^T of this lane's key in registers, V^T in LDS (the registers go to the accumulators)
-    uint4 kreg[kHD / 16];
+    // stationary B operands: K^T of this lane's key in registers but for what is parked in LDS, V^T in LDS (the registers go to the accumulators)
+    constexpr int kParked = Geo<kHD>::kParked;
+    uint4 kreg[kHD / 16 - kParked];   // of ds >= kParked
     {
         const int64_t off = (b * a.kv_stride[0] + hd * a.kv_stride[1] + (key_ok ? keys.row_of(n_lane) : 0) * a.kv_stride[2]) * 2;
         const char* krow = reinterpret_cast<const char*>(a.k) + off;
         const char* vrow = reinterpret_cast<const char*>(a.v) + off;
 #pragma unroll
         for (int ds = 0; ds < kHD / 16; ds++) {
-            kreg[ds] = make_uint4(0u, 0u, 0u, 0u);
-            uint4 vv = make_uint4(0u, 0u, 0u, 0u);
+            uint4 kk = make_uint4(0u, 0u, 0u, 0u), vv = kk;
             if (key_ok) {
-                kreg[ds] = *reinterpret_cast<const uint4*>(krow + (16 * ds + 8 * h) * 2);
+                kk = *reinterpret_cast<const uint4*>(krow + (16 * ds + 8 * h) * 2);
                 vv = *reinterpret_cast<const uint4*>(vrow + (16 * ds + 8 * h) * 2);
             }
             vstat[ds * CKV_WAVE + lane] = vv;
+            if (ds < kParked) vstat[(kHD / 16 + ds) * CKV_WAVE + lane] = kk;
+            else kreg[ds - kParked] = kk;
         }
     }
-    const int64_t first_row = n_lane < n_cached ? 0 : n_lane - n_cached;  // the first query that sees this key
+    const int first_row = n_lane < n_cached ? 0 : n_lane - n_cached;  // the first query that sees this key
     const float c2 = a.scale * kLog2e;
 
-    int tr_base[2];
-    col_operand_setup<kHD>(lane, tr_base);
     const uint32_t lds0 = lds_address(dyn_smem);
+    const Operands<kHD, true> op(lds0, lane);
 
     f32x16 dk[kHD / 32], dv[kHD / 32];
 #pragma unroll
     for (int db = 0; db < kHD / 32; db++) dk[db] = dv[db] = zero16();
 
     // the first query block any key of the workgroup can be seen from
-    const int64_t m_first = n_wg < n_cached ? 0 : n_wg - n_cached;
-    const int blk0 = (int)(m_first / kBlk);
+    const int blk0 = (n_wg < n_cached ? 0 : n_wg - n_cached) / kBlk;
     // keys sorted behind the visible ones: nothing but the zeros at the end
-    const int nblk = n_wg < keys.n_seen ? (int)((n_ctx + kBlk - 1) / kBlk) : 0;
+    const int nblk = n_wg < keys.n_seen ? (n_ctx + kBlk - 1) / kBlk : 0;
     // does any key of this wavefront exist and pass its mask?
     const bool wave_alive = __ballot(key_ok) != 0ull;
-    const int64_t wave_first_key = n_wg + wave * 32;
+    const int wave_first_key = n_wg + wave * 32;
 
-    auto load_rowv = [&](int st, int64_t m0) {
-        if (tid < 2 * kBlk) {
-            const int64_t m = m0 + (tid & (kBlk - 1));
-            float v = 0.f;
-            if (m < n_ctx) v = tid < kBlk ? -lse[m] * kLog2e : dl[m];
-            rowv[st][tid / kBlk][tid & (kBlk - 1)] = v;
-        }
+    // the copies of block m0 / 32 into a stage; rows past the end repeat the last one
+    auto copy = [&](int m0, int st) {
+        copy_block<kHD>(qb + m0 * q_row, (uint32_t)q_row, n_ctx - 1 - m0, lds0 + (uint32_t)(st * 2 * kTile), wave, lane);
+        copy_block<kHD>(gb + m0 * g_row, (uint32_t)g_row, n_ctx - 1 - m0, lds0 + (uint32_t)(st * 2 * kTile + kTile), wave, lane);
+    };
+    // per-row scalars of a block, one per lane of wavefront 0
+    auto row_scalar = [&](int m0) {
+        const int m = m0 + (lane & 31);
+        return m < n_ctx ? (h ? dl[m] : lse[m]) : 0.f;
     };
     if (blk0 < nblk) {
-        copy_block<kHD>(qb, q_row, (int64_t)blk0 * kBlk, n_ctx, lds0 + (uint32_t)((blk0 & 1) * 2 * kTile), wave, lane);
-        copy_block<kHD>(gb, g_row, (int64_t)blk0 * kBlk, n_ctx, lds0 + (uint32_t)((blk0 & 1) * 2 * kTile + kTile), wave, lane);
-        load_rowv(blk0 & 1, (int64_t)blk0 * kBlk);
+        copy(blk0 * kBlk, 0);
+        if (wave == 0) { const float v = row_scalar(blk0 * kBlk); rowv[0][h][lane & 31] = h ? -v : -v * kLog2e; }
     }
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
     __syncthreads();
-    for (int blk = blk0; blk < nblk; blk++) {
-        const int st = blk & 1;
-        const int64_t m0 = (int64_t)blk * kBlk;
+    auto step = [&](auto stage_tag, int blk) {
+        constexpr int st = decltype(stage_tag)::value;
+        constexpr uint32_t qt = st * 2 * kTile, gt = qt + kTile;
+        const int m0 = blk * kBlk;
         const bool more = blk + 1 < nblk;
-        float rv_next = 0.f;  // this thread's per-row scalar of the next block: requested first, parked in LDS last
+        float rv_next = 0.f;  // a per-row scalar of the next block: requested first, parked in LDS last
         if (more) {  // the other stage was last read before the barrier that ended the step before
-            if (tid < 2 * kBlk) {
-                const int64_t m = m0 + kBlk + (tid & (kBlk - 1));
-                if (m < n_ctx) rv_next = tid < kBlk ? lse[m] : dl[m];
-            }
+            if (wave == 0) rv_next = row_scalar(m0 + kBlk);
             __builtin_amdgcn_sched_barrier(0);
-            copy_block<kHD>(qb, q_row, m0 + kBlk, n_ctx, lds0 + (uint32_t)((st ^ 1) * 2 * kTile), wave, lane);
-            copy_block<kHD>(gb, g_row, m0 + kBlk, n_ctx, lds0 + (uint32_t)((st ^ 1) * 2 * kTile + kTile), wave, lane);
+            copy(m0 + kBlk, st ^ 1);
         }
         // rows before the first chunk key of the wavefront's keys see none of them when all its keys are chunk keys
         const bool dead = !wave_alive || (wave_first_key >= n_cached && wave_first_key - n_cached > m0 + kBlk - 1);
         if (!dead) {
-            const unsigned char* qt = smem[st][0];
-            const unsigned char* gt = smem[st][1];
-            // rows r of the block with r_lo <= r < r_hi see this lane's key
-            int64_t lo64 = first_row - m0, hi64 = n_ctx - m0;
-            if (lo64 < 0) lo64 = 0;
-            if (lo64 > kBlk) lo64 = kBlk;
-            if (hi64 > kBlk) hi64 = kBlk;
-            // A lane is a key: a masked or absent key spoils only its own accumulators, which are stored as zeros.
-            const int r_lo = (int)lo64, r_hi = (int)hi64;
+            // Rows r of the block with r_lo <= r < r_hi see this lane's key.  A lane is a key: a masked or absent key spoils only
+            // its own accumulators, which are stored as zeros.
+            const int r_lo = first_row - m0 < 0 ? 0 : first_row - m0 > kBlk ? kBlk : first_row - m0;
+            const int r_hi = n_ctx - m0 > kBlk ? kBlk : n_ctx - m0;
             const bool plain = __ballot(r_lo > 0) == 0ull && r_hi == kBlk;  // every row of the block sees every key
             // bit r of `allow`: row r of the block sees this lane's key; element i looks at row 8 (i / 4) + 4 h + i % 4
             const uint32_t allow = (low_bits(r_hi) & ~low_bits(r_lo)) >> (4 * h);
-            const uint32_t qt_lds = lds0 + (uint32_t)(st * 2 * kTile), gt_lds = qt_lds + kTile;
-            // Phases P, dV, dP with dS, dK, each in issue order: an operand is read from LDS kKvAhead matrix instructions
-            // before the one that takes it, the first ones of a phase in the phase before (more than that, or dP beside the
-            // exponentials, does not fit the registers beside two 32 x 128 accumulators).
+            // Phases S, dP with P, dV with dS, dK, each in issue order: an operand is read from LDS kKvAhead matrix
+            // instructions before the one that takes it, the first ones of a phase in the phase before.
             constexpr int kRow = kHD / 16, kDB = kHD / 32;
-            uint4 qops[kRow], gops[2 * kDB], rops[kRow], vops[kRow], cops[2 * kDB];
-            auto g_col = [&](int k) { return col_operand<kHD>(gt_lds, tr_base, k / kDB, k % kDB); };
-            auto q_col = [&](int k) { return col_operand<kHD>(qt_lds, tr_base, k / kDB, k % kDB); };
-            f32x16 pv = zero16();
+            static_assert(kParked <= kKvAhead, "parked operands are read with the first ones");
+            uint4 kops[kKvAhead], qops[kRow], gops[2 * kDB], rops[kRow], vops[kRow], cops[2 * kDB];
+            auto g_col = [&](int k) { return op.col_op(gt, k / kDB, k % kDB); };
+            auto q_col = [&](int k) { return op.col_op(qt, k / kDB, k % kDB); };
+            f32x16 pv = zero16(), dp;
+            float nls[16];
+            auto row_scalars = [&](int which, int j, auto& to) {
+                const float4 v = *reinterpret_cast<const float4*>(&rowv[st][which][8 * j + 4 * h]);
+                to[4 * j] = v.x; to[4 * j + 1] = v.y; to[4 * j + 2] = v.z; to[4 * j + 3] = v.w;
+            };
 #pragma unroll
-            for (int k = 0; k < kKvAhead; k++) qops[k] = row_operand<kHD>(qt, lane, k);
+            for (int k = 0; k < kKvAhead; k++) {
+                qops[k] = op.row_op(qt, k);
+                if (k < kParked) kops[k] = vstat[(kRow + k) * CKV_WAVE + lane];
+            }
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int k = 0; k < kRow; k++) {
-                if (k + kKvAhead < kRow) qops[k + kKvAhead] = row_operand<kHD>(qt, lane, k + kKvAhead);
-                else gops[k + kKvAhead - kRow] = g_col(k + kKvAhead - kRow);
-                pv = Mma<T>::mma(qops[k], kreg[k], pv);
+                if (k + kKvAhead < kRow) qops[k + kKvAhead] = op.row_op(qt, k + kKvAhead);
+                else if (k == kRow - 1) {
+                    rops[0] = op.row_op(gt, 0);
+                    vops[0] = vstat[lane];
+                }
+                if (k >= kRow - 4) row_scalars(1, k - (kRow - 4), dp);
+                pv = Mma<T>::mma(qops[k], k < kParked ? kops[k] : kreg[k - kParked], pv);
                 __builtin_amdgcn_sched_barrier(0);
             }
+            constexpr int kPer = (16 + kRow - 2) / (kRow - 1);   // exponentials beside a matrix instruction
+            auto weight = [&](int i) { pv[i] = __builtin_amdgcn_exp2f(fmaf(pv[i], c2, nls[i])); };
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const float4 nl = *reinterpret_cast<const float4*>(&rowv[st][0][8 * j + 4 * h]);
-                const float nls[4] = {nl.x, nl.y, nl.z, nl.w};
+            for (int k = 0; k < kRow; k++) {
+                if (k + 1 < kRow) {
+                    rops[k + 1] = op.row_op(gt, k + 1);
+                    vops[k + 1] = vstat[(k + 1) * CKV_WAVE + lane];
+                }
+                if (k >= kRow - kKvAhead) gops[k + kKvAhead - kRow] = g_col(k + kKvAhead - kRow);
 #pragma unroll
-                for (int e = 0; e < 4; e++) pv[4 * j + e] = __builtin_amdgcn_exp2f(fmaf(pv[4 * j + e], c2, nls[e]));
+                for (int j = 0; j < 4; j++)
+                    if (k == 4 * j / kPer) row_scalars(0, j, nls);   // a slot before the first exponential that takes one
+                dp = Mma<T>::mma(rops[k], vops[k], dp);
+                if (k > 0) {   // not beside the first, which the last logits are only just behind
+#pragma unroll
+                    for (int i = (k - 1) * kPer; i < k * kPer && i < 16; i++) weight(i);
+                }
+                __builtin_amdgcn_sched_barrier(0);
             }
             if (!plain) {
 #pragma unroll
                 for (int i = 0; i < 16; i++) pv[i] = keep_if_bit(pv[i], allow, 8 * (i / 4) + (i % 4));
             }
+            Weights<T, kHD> pw, dw;
+            pw.set(pv, 0);
+            pw.set(pv, 1);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int k = 0; k < 2 * kDB; k++) {
-                if (k + kKvAhead < 2 * kDB) {
-                    gops[k + kKvAhead] = g_col(k + kKvAhead);
-                } else if (k == 2 * kDB - 1) {
-                    rops[0] = row_operand<kHD>(gt, lane, 0);
-                    vops[0] = vstat[lane];
-                }
-                Weights<T, kHD>::accumulate(gops, pv, k, dv);
+                if (k + kKvAhead < 2 * kDB) gops[k + kKvAhead] = g_col(k + kKvAhead);
+                else cops[k + kKvAhead - 2 * kDB] = q_col(k + kKvAhead - 2 * kDB);
+                pw.accumulate(gops, k, dv);
+#pragma unroll
+                for (int i = k * (8 / kDB); i < (k + 1) * (8 / kDB); i++) dp[i] = kScaleInside<T, kHD> ? pv[i] * dp[i] * a.scale : pv[i] * dp[i];
+                if (k == kDB - 1) dw.set(dp, 0);
                 __builtin_amdgcn_sched_barrier(0);
             }
-            f32x16 dp = zero16();
-#pragma unroll
-            for (int k = 0; k < kRow; k++) {
-                if (k + 1 < kRow) {
-                    rops[k + 1] = row_operand<kHD>(gt, lane, k + 1);
-                    vops[k + 1] = vstat[(k + 1) * CKV_WAVE + lane];
-                }
-                if (k >= kRow - kKvAhead) cops[k + kKvAhead - kRow] = q_col(k + kKvAhead - kRow);
-                dp = Mma<T>::mma(rops[k], vops[k], dp);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const float4 de = *reinterpret_cast<const float4*>(&rowv[st][1][8 * j + 4 * h]);
-                const float des[4] = {de.x, de.y, de.z, de.w};
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    const int i = 4 * j + e;
-                    dp[i] = pv[i] * (dp[i] - des[e]) * a.scale;
-                }
-            }
-            Weights<T, kHD> dw;
-            dw.set(dp, 0);
             dw.set(dp, 1);
-            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int k = 0; k < 2 * kDB; k++) {
                 if (k + kKvAhead < 2 * kDB) cops[k + kKvAhead] = q_col(k + kKvAhead);
@@ -669,29 +704,50 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dkdv_kernel(BwdMfmaParam
         }
         __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wavefront's copies of the next block have landed
-        if (more && tid < 2 * kBlk) rowv[st ^ 1][tid / kBlk][tid & (kBlk - 1)] = tid < kBlk ? -rv_next * kLog2e : rv_next;
+        if (more && wave == 0) rowv[st ^ 1][h][lane & 31] = h ? -rv_next : -rv_next * kLog2e;
         __syncthreads();
+    };
+    for (int blk = blk0; blk < nblk; blk += 2) {
+        step(std::integral_constant<int, 0>{}, blk);
+        if (blk + 1 < nblk) step(std::integral_constant<int, 1>{}, blk + 1);
+    }
+    if constexpr (!kScaleInside<T, kHD>) {
+#pragma unroll
+        for (int db = 0; db < kHD / 32; db++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) dk[db][i] *= a.scale;
     }
     if (!key_ok) {
 #pragma unroll
         for (int db = 0; db < kHD / 32; db++) dk[db] = dv[db] = zero16();
     }
-    if (n_lane < n_kv) {
-        const int64_t off = (b * a.dkv_stride[0] + hd * a.dkv_stride[1] + keys.row_of(n_lane) * a.dkv_stride[2]) * 2;
-        char* ok_ = reinterpret_cast<char*>(a.dk) + off;
-        char* ov_ = reinterpret_cast<char*>(a.dv) + off;
+    // The rows leave through LDS (the stages: nobody reads them any more), so that a store is whole rows of 16-byte pieces, 1 KiB
+    // an instruction; 8-byte pieces of 32 rows apiece cost a workgroup of 32 blocks an eighth of its time.
+    constexpr int kPieces = Geo<kHD>::kPieces, kPer = CKV_WAVE / kPieces, kOut = 32 / kPer;   // rows of a store, stores of a tensor
+    unsigned char* mine = dyn_smem + wave * 32 * Geo<kHD>::kRowBytes;
+    int64_t out_off[kOut];
+#pragma unroll
+    for (int i = 0; i < kOut; i++) {
+        const int64_t n = n_wg + wave * 32 + kPer * i + lane / kPieces;
+        out_off[i] = n < a.n_kv ? (b * a.dkv_stride[0] + hd * a.dkv_stride[1] + keys.row_of(n) * a.dkv_stride[2]) * 2 + (lane % kPieces) * 16 : -1;
+    }
+    auto store = [&](const f32x16(&acc)[kHD / 32], void* to) {
 #pragma unroll
         for (int db = 0; db < kHD / 32; db++) {
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const int d = 32 * db + 8 * j + 4 * h;
-                *reinterpret_cast<uint2*>(ok_ + d * 2) = make_uint2(Mma<T>::pack2(dk[db][4 * j], dk[db][4 * j + 1]),
-                                                                    Mma<T>::pack2(dk[db][4 * j + 2], dk[db][4 * j + 3]));
-                *reinterpret_cast<uint2*>(ov_ + d * 2) = make_uint2(Mma<T>::pack2(dv[db][4 * j], dv[db][4 * j + 1]),
-                                                                    Mma<T>::pack2(dv[db][4 * j + 2], dv[db][4 * j + 3]));
-            }
+            for (int j = 0; j < 4; j++)   // dims 32 db + 8 j + 4 h .. +3 of this lane's key
+                *reinterpret_cast<uint2*>(mine + (lane & 31) * Geo<kHD>::kRowBytes + (((4 * db + j) ^ (lane & (kPieces - 1))) << 4) + 8 * h) =
+                    make_uint2(Mma<T>::pack2(acc[db][4 * j], acc[db][4 * j + 1]), Mma<T>::pack2(acc[db][4 * j + 2], acc[db][4 * j + 3]));
         }
-    }
+#pragma unroll
+        for (int i = 0; i < kOut; i++) {
+            const int row = kPer * i + lane / kPieces, piece = lane % kPieces;
+            const uint4 v = *reinterpret_cast<const uint4*>(mine + row * Geo<kHD>::kRowBytes + ((piece ^ (row & (kPieces - 1))) << 4));
+            if (out_off[i] >= 0) *reinterpret_cast<uint4*>(reinterpret_cast<char*>(to) + out_off[i]) = v;
+        }
+    };
+    store(dk, a.dk);
+    store(dv, a.dv);
 }
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
@@ -732,6 +788,7 @@ int run(const BwdMfmaParams& p_in, hipStream_t stream) {
 bool bwd_mfma_supported(const ckv_dense_bwd_args& a) {
     if (a.dtype != CKV_F16 && a.dtype != CKV_BF16) return false;
     if (a.D != 64 && a.D != 128) return false;
+    if (a.n_kv > 0x7fffff00) return false;   // keys and rows are numbered in 32 bits
     if (!rows_ok(a.q_stride) || !rows_ok(a.kv_stride) || !rows_ok(a.dout_stride) || !rows_ok(a.dq_stride) ||
         !rows_ok(a.dkv_stride))
         return false;

@@ -206,6 +206,22 @@ __device__ inline void async_copy16(const void* sbase, uint32_t voff, uint32_t l
                  : "memory");
 }
 
+// One 4-byte piece per lane, lane i at +4*i; lanes that are switched off leave their piece alone.
+__device__ inline void async_copy4(const void* sbase, uint32_t voff, uint32_t lds_wave_base) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
+                 :
+                 : "s"(__builtin_amdgcn_readfirstlane(lds_wave_base)), "v"(voff), "s"(uniform_ptr(sbase))
+                 : "memory");
+}
+
+// Waits until at most kLeft of this wavefront's copies (and other vector memory operations) are on their way.  Reads of what
+// landed may follow at once where the wavefront copied it itself.
+template <int kLeft>
+__device__ inline void wait_copies() {
+    static_assert(kLeft < 64, "vmcnt has six bits");
+    asm volatile("s_waitcnt vmcnt(%0)" : : "n"(kLeft) : "memory");
+}
+
 // The same from an address of the lane's own, for sources more than 4 GiB apart.
 __device__ inline void async_copy16_from(const void* src, uint32_t lds_wave_base) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"

@@ -536,6 +536,22 @@ def test_reference_mixin_surface(flavour):
         assert_scores_close(torch.where(same, sh, sf), sf, dtype, f"chunk {c}: score cache")
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("N_CTX,N_KV,sm_scale", [
+    (5, 5, 0.5), (20, 20 + 13, 0.5), (32, 32 + 64, -0.25), (3, 3 + 125, 0.0), (40, 40 + 120, 1.25), (130, 130 + 60, -1.0),
+])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_backward_of_few_key_blocks_and_any_scale(D, N_CTX, N_KV, sm_scale, dtype):
+    """One to six blocks of 32 keys, fewer and more than dq's three stages, and the softmax scale that rides on its
+    exponentials by magnitude and on the result by sign (dk: on the finished sum).  Tolerance as in
+    ``test_dense_operator_backward``, whose dq and dk are products of sm_scale, a row of v and a row of k or q, 0.5 ** 3 in
+    the mean: here at most 1.25 * 0.3 ** 2, which is less."""
+    torch.manual_seed(23)
+    q, k, v = (torch.empty((1, 2, n, D), dtype=dtype, device="cuda").normal_(mean=0.0, std=0.3).requires_grad_()
+               for n in (N_CTX, N_KV, N_KV))
+    check_backward_against_autograd(q, k, v, torch.rand(N_KV - N_CTX, device="cuda") > 0.7, dtype, sm_scale)
+
+
 def test_backward_is_refused_up_front_for_head_sizes_it_does_not_tile():
     """head_dim 256 runs forward (the reference operator's set is 16 .. 256) but the backward kernels stage fp32
     rows of at most 192 columns: asking for gradients raises at the call, not later inside ``.backward()``; head
