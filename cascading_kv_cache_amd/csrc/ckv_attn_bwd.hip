@@ -29,25 +29,40 @@ struct BwdParams {
     int n_split;
 };
 
+// delta[row] = sum over the head dims of out times dout.  16-bit rows of up to 512 contiguous dims, 16-byte addressable (`lanes`
+// > 0): a row is D / 8 lanes, one 16-byte piece of each tensor apiece; other rows a wavefront, element by element.  The first
+// workgroup sorts the keys beside them, and with 256 threads it was what the launch waited for: 65536 rows of 128 dims and
+// 16384 keys 23 -> 15 us with 1024.
+constexpr int kDeltaThreads = 1024;
 template <typename T>
-__global__ void __launch_bounds__(kThreads) bwd_delta_kernel(BwdParams p) {
+__global__ void __launch_bounds__(kDeltaThreads) bwd_delta_kernel(BwdParams p, int lanes) {
     const ckv_dense_bwd_args& a = p.a;
     int64_t blk = blockIdx.x;
     if (p.key_order && blk-- == 0) {  // the first workgroup sorts the keys
-        key_order_block<kThreads>(a.mask, a.n_kv - a.n_ctx, a.n_ctx, p.key_order, p.n_visible);
+        key_order_block<kDeltaThreads>(a.mask, a.n_kv - a.n_ctx, a.n_ctx, p.key_order, p.n_visible);
         return;
     }
-    const int wave = threadIdx.x / CKV_WAVE, lane = threadIdx.x % CKV_WAVE;
+    const int per_row = lanes > 0 ? lanes : CKV_WAVE, lane = threadIdx.x % per_row;
     const int64_t rows = a.B * a.H * a.n_ctx;
-    const int64_t row = blk * (kThreads / CKV_WAVE) + wave;
-    if (row >= rows) return;
+    const int64_t row = blk * (kDeltaThreads / per_row) + threadIdx.x / per_row;
+    if (row >= rows) return;   // all lanes of a row at once
     const int64_t m = row % a.n_ctx, h = (row / a.n_ctx) % a.H, b = row / (a.n_ctx * a.H);
     const T* o = (const T*)a.out + b * a.out_stride[0] + h * a.out_stride[1] + m * a.out_stride[2];
     const T* g = (const T*)a.dout + b * a.dout_stride[0] + h * a.dout_stride[1] + m * a.dout_stride[2];
     float acc = 0.f;
-    for (int64_t d = lane; d < a.D; d += CKV_WAVE)
-        acc = fmaf(Elem<T>::to_float(o[d * a.out_stride[3]]), Elem<T>::to_float(g[d * a.dout_stride[3]]), acc);
-    for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off);
+    if (lanes > 0) {
+        if constexpr (sizeof(T) == 2) {
+            const uint4 ov = *reinterpret_cast<const uint4*>(o + 8 * lane), gv = *reinterpret_cast<const uint4*>(g + 8 * lane);
+            const T* oe = reinterpret_cast<const T*>(&ov);
+            const T* ge = reinterpret_cast<const T*>(&gv);
+#pragma unroll
+            for (int i = 0; i < 8; i++) acc = fmaf(Elem<T>::to_float(oe[i]), Elem<T>::to_float(ge[i]), acc);
+        }
+    } else {
+        for (int64_t d = lane; d < a.D; d += CKV_WAVE)
+            acc = fmaf(Elem<T>::to_float(o[d * a.out_stride[3]]), Elem<T>::to_float(g[d * a.dout_stride[3]]), acc);
+    }
+    for (int off = per_row / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off);
     if (lane == 0) p.delta[row] = acc;
 }
 
@@ -248,7 +263,16 @@ int run_bwd(const BwdParams& p, hipStream_t stream) {
     const bool mfma = bwd_mfma_supported(a);
     BwdParams pd = p;
     if (!mfma) pd.key_order = nullptr;
-    hipLaunchKernelGGL(bwd_delta_kernel<T>, dim3((unsigned)((rows + 3) / 4 + (pd.key_order ? 1 : 0))), dim3(kThreads), 0, stream, pd);
+    auto in_pieces = [](const void* base, const int64_t* st) {
+        return reinterpret_cast<uintptr_t>(base) % 16 == 0 && st[3] == 1 && st[0] % 8 == 0 && st[1] % 8 == 0 && st[2] % 8 == 0;
+    };
+    const int64_t pieces = a.D / 8;
+    const bool vec = sizeof(T) == 2 && pieces <= CKV_WAVE && (pieces & (pieces - 1)) == 0 && in_pieces(a.out, a.out_stride) &&
+                     in_pieces(a.dout, a.dout_stride);
+    const int lanes = vec ? (int)pieces : 0;
+    const int64_t rows_per = kDeltaThreads / (lanes > 0 ? lanes : CKV_WAVE);
+    hipLaunchKernelGGL(bwd_delta_kernel<T>, dim3((unsigned)((rows + rows_per - 1) / rows_per + (pd.key_order ? 1 : 0))),
+                       dim3(kDeltaThreads), 0, stream, pd, lanes);
     CKV_HIP_TRY(hipGetLastError());
     if (mfma) return launch_bwd_mfma(a, p.delta, p.key_order, p.n_visible, p.part_dq, p.n_split, stream);
     if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(bwd_dq_kernel<T>), (int)lds_dq)) return rc;

@@ -1543,9 +1543,12 @@ int run_mfma(const MfmaProblem& mp, hipStream_t stream) {
         // shared positions: a block walks several (b, kvh) units with one set of cos/sin, the next unit's rows
         // always on their way
         int64_t splits = nbh;
-        if (mp.shared_pos) {  // about two workgroups per compute unit
+        if (mp.shared_pos) {
+            // About two workgroups per compute unit; eight where the keys are gathered by an order: those are not rotated, so
+            // there is nothing to reuse from unit to unit, and the tiles of masked keys leave at once (64 heads x 17408 keys,
+            // half of them masked: 164 us with two, 139 with eight, 152 with sixteen).
             const int64_t tiles = n_pad / kBN;
-            splits = (2 * cus + tiles - 1) / tiles;
+            splits = ((mp.key_order ? 8 : 2) * cus + tiles - 1) / tiles;
             if (splits < 2) splits = 2;
             if (splits > nbh) splits = nbh;
         }
