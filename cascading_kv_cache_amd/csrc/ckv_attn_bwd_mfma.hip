@@ -10,14 +10,14 @@
 //          S = Q K^T and dP = dO V^T keep a key in one lane; P and dS are the B operands of
 //          dV^T += dO^T P and dK^T += Q^T dS.
 //
-// Precision.  With 128 dims P and dS enter those products rounded to the tensor dtype.  With 64 dims they stay float32:
-// the products run on v_mfma_f32_32x32x2, whose B operand is an accumulator register as it stands and whose A operand is
-// the same transposed read, widened to float32.  16-bit terms that add up to the float32 value, as the forward kernel takes,
-// would need a scale of their own for dS, which has no largest value, and would turn an infinite gradient into NaN.
-// 8 heads x 1000 rows x 5095 keys in float16: dq 32 -> 55 us, dk/dv 40 -> 91 (the vector kernels, to the same error: 2520
-// and 1838).  These products bound both kernels: 2048 and 4096 of the 2304 and 4352 cycles of matrix work per 32 x 32 block,
-// and unlike the 16-bit instructions they do not run beside vector instructions (matrix pipe 43 and 50 % busy, 0 % of the
-// time together with the vector ALU).
+// Precision.  With 128 dims P and dS enter those products rounded to the tensor dtype.  With 64 dims nothing but the operands
+// is held in 16 bits: P and dS enter as three terms of the tensor dtype that add up to the float32 value, one matrix
+// instruction each (Weights), float16 terms of dS times a power of two that keeps them in range (Range); blocks that the
+// terms cannot hold, infinite gradients among them, take v_mfma_f32_32x32x2 on the values themselves.  That instruction for
+// every block, which is four times the matrix work of three terms and never runs beside a vector instruction, took 8 heads x
+// 1000 rows x 5095 keys in float16 dq 55 and dk/dv 91 us instead of 35 and 49 (the vector kernels 2520 and 1838); against
+// float64 over 16 random shapes the terms are level or closer (dq 2.0999e-4 against 2.1000e-4, dk 2.0808e-4 and 2.0808e-4,
+// dv 2.0778e-4 and 2.0778e-4 relative, float16: the rounding of the result).
 //
 // What bounds them (64 heads x 1024 rows x 8704 visible keys, 128 dims, bf16: dq 548 -> 440 us, dk/dv 770 -> 620).  Vector work
 // beside the matrix work: both take most of a block's time and overlap only where a wavefront alternates them, so an
@@ -57,7 +57,7 @@ constexpr int kBlk = 32;              // rows of a streamed block
 constexpr int kWaves = 4;             // wavefronts of a workgroup, 32 stationary rows each
 constexpr int kThreads = kWaves * CKV_WAVE;
 constexpr int kOwn = kWaves * 32;     // stationary rows of a workgroup
-constexpr int kAhead = 3, kKvAhead = 2;  // matrix instructions between an operand's read from LDS and its use
+constexpr int kAhead = 3, kKvAhead = 3;  // matrix instructions between an operand's read from LDS and its use
 constexpr int kDqStages = 3;          // stages of K and V blocks of the dq kernel: copies two blocks ahead
 constexpr float kLog2e = 1.4426950408889634f;
 template <int kHD>
@@ -67,8 +67,9 @@ struct Geo {
     static constexpr int kPieces = kHD / 8;         // 16-byte pieces of a row
     // dynamic LDS of the dk/dv kernel: two stages of (Q, dO) tiles, the per-row scalars of both stages, V^T operands
     static constexpr int kDkdvRowv = 2 * 2 * kTile;
-    static constexpr int kDkdvV = kDkdvRowv + 2 * 2 * kBlk * (int)sizeof(float);
-    static constexpr int kParked = kHD == 128 ? 2 : 0;   // K^T operands that are kept there too: 8 registers that would spill
+    static constexpr int kDkdvOdd = kDkdvRowv + 2 * 2 * kBlk * (int)sizeof(float);   // 64 dims: a word per stage
+    static constexpr int kDkdvV = kDkdvOdd + (kHD == 64 ? 16 : 0);
+    static constexpr int kParked = kHD == 128 ? 3 : 0;   // K^T operands that are kept there too: 12 registers that would spill
     static constexpr int kDkdvLds = kDkdvV + kWaves * (kHD / 16 + kParked) * CKV_WAVE * 16;
 };
 
@@ -87,6 +88,9 @@ struct Mma<__hip_bfloat16> {
     // the two elements of a packed pair as floats
     __device__ static float lo_f(uint32_t w) { return __uint_as_float(w << 16); }
     __device__ static float hi_f(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
+    // x less an element of a packed pair, exact where the element is x rounded
+    __device__ static float less_lo(float x, uint32_t w) { return x - lo_f(w); }
+    __device__ static float less_hi(float x, uint32_t w) { return x - hi_f(w); }
 };
 template <>
 struct Mma<__half> {
@@ -100,6 +104,17 @@ struct Mma<__half> {
     }
     __device__ static float lo_f(uint32_t w) { return (float)__builtin_bit_cast(f16x2, w)[0]; }
     __device__ static float hi_f(uint32_t w) { return (float)__builtin_bit_cast(f16x2, w)[1]; }
+    // one instruction that widens and subtracts, where the compiler makes two (half the vector work of a set of terms)
+    __device__ static float less_lo(float x, uint32_t w) {
+        float r;
+        asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(w), "v"(x));
+        return r;
+    }
+    __device__ static float less_hi(float x, uint32_t w) {
+        float r;
+        asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(w), "v"(x));
+        return r;
+    }
 };
 
 struct BwdMfmaParams {
@@ -235,44 +250,89 @@ __device__ inline uint4 pack8(const f32x16& v, int s) {
                       Mma<T>::pack2(v[8 * s + 4], v[8 * s + 5]), Mma<T>::pack2(v[8 * s + 6], v[8 * s + 7]));
 }
 
-// The B operand of the two products that contract over a block's 32 rows, element 8 s + i of `v` belonging to step s: packed
-// in the tensor dtype (128 dims) or as it is, and the product of a step with the A operand of col_operand.  Element 4 a + e
-// of that holds rows 16 s + 8 a + 4 (lane/32) + e, the row of accumulator register 8 s + 4 a + e in the same lane half.
-// `accumulate` is matrix instruction k of such a product, step k / kDB into accumulator k % kDB with A operand ops[k]; with
-// 64 dims the first one of a step brings the step's float32 instructions, the two accumulators in turn (both operands are
-// there: they are read at least two ahead), all operands widened first (dk/dv 101 us; one before each instruction 113).
+// The B operand of the two products that contract over a block's 32 rows, element 8 s + i of `v` belonging to step s, and the
+// product of a step with the A operand of Operands::col_op.  Element 4 a + e of that holds rows 16 s + 8 a + 4 (lane/32) + e,
+// the row of accumulator register 8 s + 4 a + e in the same lane half.  `accumulate` is product k, step k / kDB into
+// accumulator k % kDB with A operand ops[k].  128 dims: packed in the tensor dtype; 64 dims: three terms of it that add up to
+// the float32 value, one matrix instruction each.
 template <typename T, int kHD>
 struct Weights {
-    static constexpr int kDB = kHD / 32;
-    uint4 w[2];
-    __device__ void set(const f32x16& v, int s) { w[s] = pack8<T>(v, s); }
-    __device__ void accumulate(const uint4 (&ops)[2 * kDB], int k, f32x16 (&c)[kDB]) const { c[k % kDB] = Mma<T>::mma(ops[k], w[k / kDB], c[k % kDB]); }
-    __device__ static void accumulate(const uint4 (&ops)[2 * kDB], const f32x16& v, int k, f32x16 (&c)[kDB]) {
-        c[k % kDB] = Mma<T>::mma(ops[k], pack8<T>(v, k / kDB), c[k % kDB]);
+    static constexpr int kDB = kHD / 32, kTerms = kHD == 64 ? 3 : 1;
+    uint4 w[kTerms][2];
+    __device__ void set(const f32x16& v, int s) {
+        w[0][s] = pack8<T>(v, s);
+        if constexpr (kTerms == 3) {
+            f32x16 rest = v;
+#pragma unroll
+            for (int t = 1; t < 3; t++) {
+                const uint32_t p[4] = {w[t - 1][s].x, w[t - 1][s].y, w[t - 1][s].z, w[t - 1][s].w};
+#pragma unroll
+                for (int i = 0; i < 8; i++) rest[8 * s + i] = i & 1 ? Mma<T>::less_hi(rest[8 * s + i], p[i >> 1]) : Mma<T>::less_lo(rest[8 * s + i], p[i >> 1]);
+                w[t][s] = pack8<T>(rest, s);
+            }
+        }
+    }
+    __device__ void accumulate(const uint4 (&ops)[2 * kDB], int k, f32x16 (&c)[kDB]) const {
+#pragma unroll
+        for (int t = 0; t < kTerms; t++) c[k % kDB] = Mma<T>::mma(ops[k], w[t][k / kDB], c[k % kDB]);
     }
 };
+
+// The same product with the float32 values themselves, all of it (64 dims): v_mfma_f32_32x32x2, whose B operand is an
+// accumulator register as it stands and whose A operand is the same transposed read, widened.  For what the terms cannot
+// hold: infinity less its first term is NaN.
 template <typename T>
-struct Weights<T, 64> {
-    f32x16 w;
-    __device__ void set(const f32x16& v, int s) {
+__device__ inline void accumulate_f32(const uint4 (&ops)[4], const f32x16& v, f32x16 (&c)[2]) {
 #pragma unroll
-        for (int i = 8 * s; i < 8 * s + 8; i++) w[i] = v[i];
-    }
-    __device__ void accumulate(const uint4 (&ops)[4], int k, f32x16 (&c)[2]) const { accumulate(ops, w, k, c); }
-    __device__ static void accumulate(const uint4 (&ops)[4], const f32x16& v, int k, f32x16 (&c)[2]) {
-        if (k % 2 != 0) return;
+    for (int s = 0; s < 2; s++) {
         float a[2][8];
 #pragma unroll
         for (int db = 0; db < 2; db++) {
-            const uint32_t p[4] = {ops[k + db].x, ops[k + db].y, ops[k + db].z, ops[k + db].w};
+            const uint4& o = ops[2 * s + db];
+            const uint32_t p[4] = {o.x, o.y, o.z, o.w};
 #pragma unroll
             for (int i = 0; i < 8; i++) a[db][i] = i & 1 ? Mma<T>::hi_f(p[i >> 1]) : Mma<T>::lo_f(p[i >> 1]);
         }
-        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int i = 0; i < 8; i++)
 #pragma unroll
-            for (int db = 0; db < 2; db++) c[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[db][i], v[8 * (k / 2) + i], c[db], 0, 0, 0);
+            for (int db = 0; db < 2; db++) c[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[db][i], v[8 * s + i], c[db], 0, 0, 0);
+    }
+}
+
+// 64 dims: whether three terms hold the dS of a block.  bfloat16 has float32's range, so that they do unless dS is out of all
+// range.  float16 terms hold 33 bits of a number of 2^-2 and more and resolve 2^-24: the dS of a lane (a query or a key: one
+// column of the accumulators) are held times a power of two that takes the largest to about 2^12.  It is set by the first
+// block that is not all zero and moves when a block outgrows 2^15; what is smaller than the largest by 2^-15 loses bits below
+// 2^-36 of that, which float32 sums of the two would lose as well.  2^40 at most: smaller dS are below every float16 result.
+template <typename T>
+struct Range {
+    static constexpr bool kMoves = std::is_same<T, __half>::value;
+    float limit = kMoves ? 0.f : 0x1p120f;
+    int total = 0;   // dS and accumulators are held times 2^total
+    // true: the block does not go into terms; `factor`: what later blocks are to be multiplied by on top
+    __device__ bool outside(f32x16& ds, f32x16 (&acc)[2], float* factor) {
+        *factor = 1.f;
+        float m = 0.f;
+#pragma unroll
+        for (int i = 0; i < 16; i++) m = fmaxf(m, fabsf(ds[i]));
+        if constexpr (kMoves) m = half_max(m);
+        if (__ballot(m > limit) == 0ull) return false;
+        if (!kMoves || __ballot(m > 0x1p100f) != 0ull) return true;
+        if (m > limit) {
+            int up = 12 - __builtin_amdgcn_frexp_expf(m);
+            if (up > 40 - total) up = 40 - total;
+            total += up;
+            limit = 32768.f;
+            *factor = __builtin_amdgcn_ldexpf(1.f, up);
+        }
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            ds[i] *= *factor;
+            acc[0][i] *= *factor;
+            acc[1][i] *= *factor;
+        }
+        return false;
     }
 };
 
@@ -338,7 +398,7 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dq_kernel(BwdMfmaParams 
     const bool row_ok = m_lane < n_ctx;
     // The magnitude of the softmax scale rides on the exponent (nothing here needs P without it), its sign on the result;
     // the products of V and dO start from -delta.  That leaves one multiplication per element beside the exponential.
-    const float nl = row_ok ? fmaf(-a.lse[bh * n_ctx + m_lane], kLog2e, __builtin_amdgcn_logf(fabsf(a.scale))) : 0.f;
+    float nl = row_ok ? fmaf(-a.lse[bh * n_ctx + m_lane], kLog2e, __builtin_amdgcn_logf(fabsf(a.scale))) : 0.f;
     const float c2 = a.scale * kLog2e;
     f32x16 neg_delta;
     {
@@ -354,6 +414,7 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dq_kernel(BwdMfmaParams 
     f32x16 dq[kHD / 32];
 #pragma unroll
     for (int db = 0; db < kHD / 32; db++) dq[db] = zero16();
+    Range<T> range;   // 64 dims
 
     // keys past the diagonal of the workgroup's last row are visible to none of its rows
     int m_last = m_wg + kOwn - 1;
@@ -450,21 +511,35 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dq_kernel(BwdMfmaParams 
                 for (int i = 0; i < 16; i++) s[i] = keep_if_bit(s[i], allow, 8 * (i / 4) + (i % 4));
             }
             f32x16 dsv;
+            bool outside = false;
 #pragma unroll
-            for (int i = 0; i < 8; i++) dsv[i] = s[i] * dp[i];
-            Weights<T, kHD> bop;
-            bop.set(dsv, 0);
-            __builtin_amdgcn_sched_barrier(0);
+            for (int i = 0; i < (kHD == 64 ? 16 : 8); i++) dsv[i] = s[i] * dp[i];
+            if constexpr (kHD == 64) {
+                float factor;
+                outside = range.outside(dsv, dq, &factor);
+                nl += __builtin_amdgcn_logf(factor);   // a power of two: whole
+                if (outside) {
 #pragma unroll
-            for (int k = 0; k < 2 * kDB; k++) {
-                if (k + kAhead < 2 * kDB) cops[k + kAhead] = col_op(k + kAhead);
-                bop.accumulate(cops, k, dq);
-                if (k < kDB) {
-#pragma unroll
-                    for (int i = 8 + k * (8 / kDB); i < 8 + (k + 1) * (8 / kDB); i++) dsv[i] = s[i] * dp[i];
+                    for (int k = kAhead; k < 2 * kDB; k++) cops[k] = col_op(k);
+                    accumulate_f32<T>(cops, dsv, dq);
                 }
-                if (k == kDB - 1) bop.set(dsv, 1);
+                asm volatile("");
+            }
+            if (!outside) {
+                Weights<T, kHD> bop;
+                bop.set(dsv, 0);
                 __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int k = 0; k < 2 * kDB; k++) {
+                    if (k + kAhead < 2 * kDB) cops[k + kAhead] = col_op(k + kAhead);
+                    bop.accumulate(cops, k, dq);
+                    if (kHD == 128 && k < kDB) {
+#pragma unroll
+                        for (int i = 8 + k * (8 / kDB); i < 8 + (k + 1) * (8 / kDB); i++) dsv[i] = s[i] * dp[i];
+                    }
+                    if (k == (kHD == 128 ? kDB - 1 : 0)) bop.set(dsv, 1);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
             }
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -486,6 +561,12 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dq_kernel(BwdMfmaParams 
         for (int db = 0; db < kHD / 32; db++)
 #pragma unroll
             for (int i = 0; i < 16; i++) dq[db][i] = -dq[db][i];
+    }
+    if constexpr (kHD == 64 && Range<T>::kMoves) {
+#pragma unroll
+        for (int db = 0; db < kHD / 32; db++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) dq[db][i] = __builtin_amdgcn_ldexpf(dq[db][i], -range.total);
     }
     if (row_ok && p.n_split > 1) {
         float* out = p.part_dq + ((int64_t)share * a.B * a.H * n_ctx + bh * n_ctx + m_lane) * kHD;
@@ -536,6 +617,7 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dkdv_kernel(BwdMfmaParam
     extern __shared__ __attribute__((aligned(16))) unsigned char dyn_smem[];
     typedef float (*RowPtr)[2][kBlk];
     RowPtr rowv = reinterpret_cast<RowPtr>(dyn_smem + Geo<kHD>::kDkdvRowv);                        // [stage][-lse log2 e, -delta]
+    int* odd_rows = reinterpret_cast<int*>(dyn_smem + Geo<kHD>::kDkdvOdd);               // [stage] some row's delta is not finite
     // the V^T operands of a wavefront's 32 keys and the first of K^T, in operand order: [wave][ds][lane] 16 bytes each
     uint4* vstat = reinterpret_cast<uint4*>(dyn_smem + Geo<kHD>::kDkdvV) + __builtin_amdgcn_readfirstlane(threadIdx.x / CKV_WAVE) * (kHD / 16 + Geo<kHD>::kParked) * CKV_WAVE;
     const ckv_dense_bwd_args& a = p.a;
@@ -595,14 +677,27 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dkdv_kernel(BwdMfmaParam
         copy_block<kHD>(qb + m0 * q_row, (uint32_t)q_row, n_ctx - 1 - m0, lds0 + (uint32_t)(st * 2 * kTile), wave, lane);
         copy_block<kHD>(gb + m0 * g_row, (uint32_t)g_row, n_ctx - 1 - m0, lds0 + (uint32_t)(st * 2 * kTile + kTile), wave, lane);
     };
-    // per-row scalars of a block, one per lane of wavefront 0
+    // Per-row scalars of a block, one per lane of wavefront 0.  Rows of dout that are not finite show in their delta (a sum of
+    // products with out): in their blocks the products with 64 dims take P and dS as they are, zero terms times infinity are NaN.
+    // float16 with 64 dims: P is held times 2^15, so that its terms resolve 2^-39, and dk and dv are brought back at the end.
+    constexpr bool kTerms = kHD == 64;
+    constexpr float kHead = kTerms && Range<T>::kMoves ? 15.f : 0.f;
     auto row_scalar = [&](int m0) {
         const int m = m0 + (lane & 31);
         return m < n_ctx ? (h ? dl[m] : lse[m]) : 0.f;
     };
+    auto park = [&](float v, int st) {
+        rowv[st][h][lane & 31] = h ? -v : fmaf(-v, kLog2e, kHead);
+        if constexpr (kTerms) {
+            const bool odd = __ballot(h && !(fabsf(v) < INFINITY)) != 0ull;
+            if (lane == 0) odd_rows[st] = odd ? 1 : 0;
+        }
+    };
+    Range<T> range;                                                   // 64 dims
+    float dscale = kHead > 0.f ? 0x1p-15f : 1.f;                       // of dS, by the lane
     if (blk0 < nblk) {
         copy(blk0 * kBlk, 0);
-        if (wave == 0) { const float v = row_scalar(blk0 * kBlk); rowv[0][h][lane & 31] = h ? -v : -v * kLog2e; }
+        if (wave == 0) park(row_scalar(blk0 * kBlk), 0);
     }
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
     __syncthreads();
@@ -680,31 +775,87 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dkdv_kernel(BwdMfmaParam
 #pragma unroll
                 for (int i = 0; i < 16; i++) pv[i] = keep_if_bit(pv[i], allow, 8 * (i / 4) + (i % 4));
             }
-            Weights<T, kHD> pw, dw;
-            pw.set(pv, 0);
-            pw.set(pv, 1);
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int k = 0; k < 2 * kDB; k++) {
-                if (k + kKvAhead < 2 * kDB) gops[k + kKvAhead] = g_col(k + kKvAhead);
-                else cops[k + kKvAhead - 2 * kDB] = q_col(k + kKvAhead - 2 * kDB);
-                pw.accumulate(gops, k, dv);
-#pragma unroll
-                for (int i = k * (8 / kDB); i < (k + 1) * (8 / kDB); i++) dp[i] = kScaleInside<T, kHD> ? pv[i] * dp[i] * a.scale : pv[i] * dp[i];
-                if (k == kDB - 1) dw.set(dp, 0);
+            auto ds_of = [&](int i) {
+                dp[i] = pv[i] * dp[i];
+                if constexpr (kHead > 0.f) dp[i] *= dscale;
+            };
+            if constexpr (!kTerms) {
+                Weights<T, kHD> pw, dw;
+                pw.set(pv, 0);
+                pw.set(pv, 1);
                 __builtin_amdgcn_sched_barrier(0);
-            }
-            dw.set(dp, 1);
 #pragma unroll
-            for (int k = 0; k < 2 * kDB; k++) {
-                if (k + kKvAhead < 2 * kDB) cops[k + kKvAhead] = q_col(k + kKvAhead);
-                dw.accumulate(cops, k, dk);
-                __builtin_amdgcn_sched_barrier(0);
+                for (int k = 0; k < 2 * kDB; k++) {
+                    if (k + kKvAhead < 2 * kDB) gops[k + kKvAhead] = g_col(k + kKvAhead);
+                    else cops[k + kKvAhead - 2 * kDB] = q_col(k + kKvAhead - 2 * kDB);
+                    pw.accumulate(gops, k, dv);
+#pragma unroll
+                    for (int i = k * (8 / kDB); i < (k + 1) * (8 / kDB); i++) dp[i] = kScaleInside<T, kHD> ? pv[i] * dp[i] * a.scale : pv[i] * dp[i];
+                    if (k == kDB - 1) dw.set(dp, 0);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                dw.set(dp, 1);
+#pragma unroll
+                for (int k = 0; k < 2 * kDB; k++) {
+                    if (k + kKvAhead < 2 * kDB) cops[k + kKvAhead] = q_col(k + kKvAhead);
+                    dw.accumulate(cops, k, dk);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            } else {
+                // the rare sides are branches of their own: as the other sides of one they spill registers of the common one
+                const bool odd = __builtin_amdgcn_readfirstlane(odd_rows[st]) != 0;
+                auto dk_f32 = [&]() {
+#pragma unroll
+                    for (int k = 0; k < 2 * kDB; k++) cops[k] = q_col(k);
+                    accumulate_f32<T>(cops, dp, dk);
+                };
+                if (odd) {
+#pragma unroll
+                    for (int k = 0; k < 2 * kDB; k++) gops[k] = g_col(k);
+                    accumulate_f32<T>(gops, pv, dv);
+#pragma unroll
+                    for (int i = 0; i < 16; i++) ds_of(i);
+                    dk_f32();
+                }
+                asm volatile("");
+                if (!odd) {
+                    Weights<T, kHD> w;
+                    w.set(pv, 0);
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int k = 0; k < 2 * kDB; k++) {
+                        if (k + kKvAhead < 2 * kDB) gops[k + kKvAhead] = g_col(k + kKvAhead);
+                        else cops[k + kKvAhead - 2 * kDB] = q_col(k + kKvAhead - 2 * kDB);
+                        w.accumulate(gops, k, dv);
+                        if (k == 0) w.set(pv, 1);
+                        if (k > 0) {
+#pragma unroll
+                            for (int i = (k - 1) * 6; i < k * 6 && i < 16; i++) ds_of(i);
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                    float factor;
+                    const bool outside = range.outside(dp, dk, &factor);
+                    dscale *= factor;
+                    if (outside) dk_f32();
+                    asm volatile("");
+                    if (!outside) {
+                        w.set(dp, 0);
+                        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                        for (int k = 0; k < 2 * kDB; k++) {
+                            if (k + kKvAhead < 2 * kDB) cops[k + kKvAhead] = q_col(k + kKvAhead);
+                            w.accumulate(cops, k, dk);
+                            if (k == 0) w.set(dp, 1);
+                            __builtin_amdgcn_sched_barrier(0);
+                        }
+                    }
+                }
             }
         }
         __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wavefront's copies of the next block have landed
-        if (more && wave == 0) rowv[st ^ 1][h][lane & 31] = h ? -rv_next : -rv_next * kLog2e;
+        if (more && wave == 0) park(rv_next, st ^ 1);
         __syncthreads();
     };
     for (int blk = blk0; blk < nblk; blk += 2) {
@@ -716,6 +867,15 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dkdv_kernel(BwdMfmaParam
         for (int db = 0; db < kHD / 32; db++)
 #pragma unroll
             for (int i = 0; i < 16; i++) dk[db][i] *= a.scale;
+    }
+    if constexpr (kHead > 0.f) {
+#pragma unroll
+        for (int db = 0; db < kHD / 32; db++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                dk[db][i] = __builtin_amdgcn_ldexpf(dk[db][i], -range.total);
+                dv[db][i] *= 0x1p-15f;
+            }
     }
     if (!key_ok) {
 #pragma unroll

@@ -5,6 +5,12 @@
 
 namespace ckv {
 
+// max over the two lane halves (lane l and lane l ^ 32) without a trip through LDS
+__device__ inline float half_max(float x) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
 // Attention over keys that are already rotated and laid out as [cached | chunk]:
 //   out[b,h,m]  = softmax_n(scale * q[b,h,m] . k[b,h/G,n] + mask) v[b,h/G,n]
 //   cached key n < n_cached is masked iff kmasked[n]; chunk key n is visible iff n-n_cached <= m

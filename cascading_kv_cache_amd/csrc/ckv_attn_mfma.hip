@@ -482,12 +482,6 @@ __device__ inline int row_swizzle(int r) { return kD == 128 ? (r & 15) : ((r >> 
 template <int kD>
 __device__ inline int k_lds_off(int r, int c) { return r * (2 * kD) + ((c ^ row_swizzle<kD>(r)) << 4); }
 
-// max over the two lane halves (lane l and lane l ^ 32) without a trip through LDS
-__device__ inline float half_max(float x) {
-    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-
 // Software-pipelined forward: eight wavefronts, 32 (head, position) rows each.  Iteration i runs
 // the softmax of tile i on the vector ALU while the matrix pipe adds the P.V product of tile i-1
 // and computes the logits of tile i+1; neither depends on the softmax in flight, so the two pipes

@@ -96,6 +96,54 @@ def test_dense_backward_of_head_size_64_is_rounded_once(Z, H, n_ctx, n_kv, grad_
 
 
 @pytest.mark.parametrize("dtype", [BF16, F16])
+@pytest.mark.parametrize("octaves", [-24, 24])
+def test_dense_backward_of_head_size_64_over_many_octaves(octaves, dtype):
+    """dS whose size falls or rises by 2^24 from the first block to the last, along the keys and along the rows: float16
+    holds them by terms times a power of two that the first block sets and later ones move."""
+    from cascading_kv_cache_amd import flash_attention as fa
+
+    n_ctx, n_kv, scale = 300, 900, 0.5
+    q, k, v, mask, do = dense_case(1, 2, n_ctx, n_kv, 64, dtype)
+    ramp = lambda n: 2.0 ** (octaves * (torch.arange(n, device="cuda") / (n - 1) - 0.5) / 2)
+    v = (v.float() * ramp(n_kv)[:, None]).to(dtype)
+    do = (do.float() * ramp(n_ctx)[:, None]).to(dtype)
+    out, _, lse, m = fa._forward(q, k, v, True, scale, mask, 0.9, True)
+    dq, dk, dv = fa._backward(q, k, v, out, lse, m, do, scale)
+    _, p, _, _ = exact_attention(q, k, v, visible(n_ctx, n_kv, mask), scale)
+    dp, delta = torch.matmul(do.double(), v.double().transpose(2, 3).contiguous()), (out.double() * do.double()).sum(-1, keepdim=True)
+    # delta and dP are float32 sums of 64 products each, rounded at the size of their largest terms
+    size = torch.matmul(do.double().abs(), v.double().abs().transpose(2, 3).contiguous()) + (out.double() * do.double()).abs().sum(-1, keepdim=True)
+    ds, ds2 = p * (dp - delta) * scale, (p * size * scale).square()
+    pt, dst, ds2t = (t.transpose(2, 3).contiguous() for t in (p, ds, ds2))
+    assert_rounded_once(dv, torch.matmul(pt, do.double()), torch.matmul(pt.square(), do.double().square()).sqrt(), n_ctx, "dv")
+    assert_rounded_once(dk, torch.matmul(dst, q.double()), torch.matmul(ds2t, q.double().square()).sqrt(), n_ctx, "dk")
+    assert_rounded_once(dq, torch.matmul(ds, k.double()), torch.matmul(ds2, k.double().square()).sqrt(), n_kv, "dq")
+
+
+@pytest.mark.parametrize("dtype", [BF16, F16])
+def test_dense_backward_of_head_size_64_with_an_infinite_gradient(dtype):
+    """An infinite element of dout is infinite in dv of every key its row sees and of no head but its own, and a key's other
+    dims are what they were: its block takes float32 products (zero terms times infinity would be NaN)."""
+    from cascading_kv_cache_amd import flash_attention as fa
+
+    n_ctx, n_kv, row, dim = 150, 450, 70, 7
+    q, k, v, mask, do = dense_case(1, 2, n_ctx, n_kv, 64, dtype)
+    out, _, lse, m = fa._forward(q, k, v, True, 0.5, mask, 0.9, True)
+    clean = fa._backward(q, k, v, out, lse, m, do, 0.5)
+    do[0, 0, row, dim] = float("inf")
+    dq, dk, dv = fa._backward(q, k, v, out, lse, m, do, 0.5)
+    for got, want in zip((dq, dk, dv), clean):
+        assert torch.equal(got[0, 1], want[0, 1])
+    seen = torch.cat((~mask, torch.arange(n_ctx, device="cuda") <= row))
+    assert torch.equal(dv[0, 0, seen, dim], torch.full_like(dv[0, 0, seen, dim], float("inf")))
+    others = [d for d in range(64) if d != dim]
+    err = (dv[0, 0, seen][:, others].double() - clean[2][0, 0, seen][:, others].double()).abs()
+    assert (err <= 2 * HALF_ULP[dtype] * clean[2][0, 0, seen][:, others].double().abs() + 2.0 ** -24).all()   # one rounding each
+    assert dv[0, 0, :n_kv - n_ctx][mask].abs().max().item() == 0.0
+    assert dk[0, 0, seen].isfinite().sum().item() == 0
+
+
+@pytest.mark.parametrize("dtype", [BF16, F16])
 @pytest.mark.parametrize("scale", [-0.5, 0.0, 1e-3, 3.0])
 def test_any_softmax_scale_of_head_size_64(scale, dtype):
     """The scale joins in float32 behind the logits: negative, zero (every visible key weighs the same), small and large."""
