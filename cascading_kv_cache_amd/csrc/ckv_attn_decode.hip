@@ -98,6 +98,8 @@ struct DecodeParams {
     unsigned char* chunks;
     int64_t Np;        // the keys rounded up to whole tiles of the streaming kernel
     int stream_wgs;    // workgroups of the streaming kernel
+    int nbh;           // B * KVH, the items of a tile
+    int run_q, run_r;  // items / stream_wgs and what is left: see stream_first_item
     float* part_ml;    // (B, H, tiles, 2); after the streaming kernel (chunk, G, 2)
     float* part_o;     // (B, H, tiles, 128)
     float* lse2;       // (B, H)
@@ -119,18 +121,16 @@ __device__ inline int stream_rank_of(const DecodeParams& p, int tile) {
     return tile < p.tiles_pre ? tile : (tile == p.tiles - 1 ? p.n_vis - 1 : -1);
 }
 
-// Items (tile-major: item = tile * B * KVH + b * KVH + kvh) are dealt out in equal contiguous runs:
-// workgroup w takes [total * w / wgs, total * (w + 1) / wgs).  Chunk index of an item.
-__device__ inline int64_t stream_chunk_of(int64_t item, int64_t total, int64_t wgs) {
-    int64_t w, first;
-    if ((total + 1) * wgs < ((int64_t)1 << 32)) {  // 32-bit division: a fraction of the cost
-        w = (int64_t)(((uint32_t)(item + 1) * (uint32_t)wgs - 1u) / (uint32_t)total);
-        first = (int64_t)((uint32_t)total * (uint32_t)w / (uint32_t)wgs);
-    } else {
-        w = ((item + 1) * wgs - 1) / total;
-        first = total * w / wgs;
-    }
-    return (item - first) * wgs + w;
+// Items (tile-major: item = tile * B * KVH + b * KVH + kvh) are dealt out in contiguous runs, the first run_r workgroups
+// one item more than the others.  First item of a workgroup, and the chunk of an item.  All of it in 32 bits: a 64-bit
+// division is a routine of a hundred dependent instructions, and the two that found a workgroup's run and the two that
+// found its tile were 6 of the 17 us that the streaming kernel took for one item a workgroup.
+__device__ inline int stream_first_item(const DecodeParams& p, int w) { return w * p.run_q + (w < p.run_r ? w : p.run_r); }
+__device__ inline int64_t stream_chunk_of(const DecodeParams& p, int item) {
+    const uint32_t cut = (uint32_t)p.run_r * (uint32_t)(p.run_q + 1);   // items of the longer runs
+    const bool longer = (uint32_t)item < cut;
+    const uint32_t w = ((uint32_t)item - (longer ? 0u : cut)) / (uint32_t)(longer ? p.run_q + 1 : p.run_q) + (longer ? 0u : (uint32_t)p.run_r);
+    return (int64_t)(item - stream_first_item(p, (int)w)) * p.stream_wgs + w;
 }
 
 template <typename T>
@@ -138,7 +138,7 @@ __global__ void decode_q_kernel(DecodeParams p) {
     const ckv_attn_args& a = p.a;
     const int64_t row = blockIdx.x;  // b * H + h
     const int j = threadIdx.x;       // 0..63: rotation pair
-    const int64_t b = row / a.H, h = row % a.H;
+    const int64_t b = blockIdx.x / (uint32_t)a.H, h = blockIdx.x - (uint32_t)b * (uint32_t)a.H;
     const T* q = (const T*)a.q + b * a.q_stride[0] + h * a.q_stride[1];
     const float f = a.inv_freq ? a.inv_freq[j] : 1.0f / powf(a.rope_theta, (float)(2 * j) / (float)kD);
     float sn, cs;
@@ -658,7 +658,8 @@ constexpr int kStreamStage = 2 * kSK * 256;       // K rows then V rows of one t
 // two stages | two 1 KiB query blocks | two [4 heads][kSK keys] logit planes | per wavefront [4][kSK] probabilities
 constexpr int kStreamQ = 2 * kStreamStage, kStreamS = kStreamQ + 2 * 1024, kStreamP = kStreamS + 2 * 4 * kSK * 4;
 constexpr int kStreamPPitch = kSK * 2 + 32;        // bytes per head row of the probabilities: the pad puts the four heads on different banks
-constexpr int kStreamLds = kStreamP + kStreamWaves * 4 * kStreamPPitch;
+constexpr int kStreamFreq = kStreamP + kStreamWaves * 4 * kStreamPPitch;   // the 64 rotation frequencies
+constexpr int kStreamLds = kStreamFreq + 64 * 4;
 
 // sum / max over the four 16-lane rows of a wavefront (lanes l, l^16, l^32, l^48)
 __device__ inline float rows4_sum(float x) {
@@ -685,6 +686,10 @@ __device__ inline float mod4_sum(float l) {
     return rows4_sum(l);
 }
 
+__device__ inline void stage_freqs(const ckv_attn_args& a, float* freqs, int tid) {
+    if (tid < kD / 2) freqs[tid] = a.inv_freq ? a.inv_freq[tid] : 1.0f / powf(a.rope_theta, (float)(2 * tid) / (float)kD);
+}
+
 // the byte offsets of the rows inside a (b, kvh) slab must fit the 32-bit lane offsets of the copies
 inline bool stream_offsets_fit(const ckv_attn_args& a) {
     const int64_t lim = (int64_t)1 << 31, es = 2;
@@ -705,8 +710,8 @@ __global__ void __launch_bounds__(kStreamThreads, kStreamWgPerCu) decode_stream_
     const int key16 = lane & 15, kq = lane >> 4;  // logits: MFMA column (key) and k-quarter
     const int pg = lane & 3, kgrp = lane >> 2;    // softmax: head and group of kKpl keys
     constexpr int kKpl = kSK / 16, kDb = kStreamDimBlocks;
-    const int64_t nbh = a.B * a.KVH, total = (int64_t)p.n_vis * nbh;
-    const int64_t item0 = total * blockIdx.x / gridDim.x, item1 = total * (blockIdx.x + 1) / gridDim.x;
+    const int nbh = p.nbh;
+    const int item0 = stream_first_item(p, (int)blockIdx.x), item1 = stream_first_item(p, (int)blockIdx.x + 1);
     const int64_t NS = a.num_sink, S = a.S;
     const int KVH = (int)a.KVH;
     constexpr int kEs = (int)sizeof(T);
@@ -739,32 +744,26 @@ __global__ void __launch_bounds__(kStreamThreads, kStreamWgPerCu) decode_stream_
     float* s_all = reinterpret_cast<float*>(smem + kStreamS);                                   // [2][4][kSK]
     unsigned char* p_wave = smem + kStreamP + wave * (4 * kStreamPPitch);                       // [4][kSK] 16-bit, padded rows
 
-    for (int64_t item = item0; item < item1;) {
-        const int64_t jt = item / nbh, bh0 = item % nbh;  // jt: the tile's rank among the visible ones
-        const int64_t tile = stream_tile_of(p, (int)jt);
-        const int64_t bh1 = (jt + 1) * nbh > item1 ? item1 - jt * nbh : nbh;
+    float* freqs = reinterpret_cast<float*>(smem + kStreamFreq);
+    stage_freqs(a, freqs, tid);
+    __syncthreads();
+    int jt = (int)((uint32_t)item0 / (uint32_t)nbh), bh0 = item0 - jt * nbh;  // jt: the tile's rank among the visible ones
+    for (int item = item0; item < item1; jt++, bh0 = 0) {
+        const int64_t tile = stream_tile_of(p, jt);
+        const int bh1 = (jt + 1) * nbh > item1 ? item1 - jt * nbh : nbh;
         item = jt * nbh + bh1;
         const int64_t n_wave = tile * kSK + wave * 16;  // first key of this wavefront
 
         // ---- per-tile constants (the same for every (b, kvh): positions are shared)
         bool vis1 = false;
-        RopeWord<T> rw[2][4];  // [ks][word]: dims 32 ks + 8 kq + 2 w, + 1 and their partners 64 further
+        int64_t pos = 0;
         {
             const int64_t n = n_wave + key16;
-            int64_t pos = 0;
             if (n < NS) { vis1 = a.sink_mask[n] == 0; pos = a.sink_pos[n]; }
             else if (n < NS + S) { vis1 = a.mask[n - NS] == 0; pos = a.pos[n - NS] + a.pos_shift; }
             else if (n < p.N) { vis1 = true; pos = a.q_pos[0]; }
-#pragma unroll
-            for (int ks = 0; ks < 2; ks++)
-#pragma unroll
-                for (int w = 0; w < 4; w++) {
-                    const int f = 32 * ks + 8 * kq + 2 * w;
-                    const float f0 = a.inv_freq ? a.inv_freq[f] : 1.0f / powf(a.rope_theta, (float)(2 * f) / (float)kD);
-                    const float f1 = a.inv_freq ? a.inv_freq[f + 1] : 1.0f / powf(a.rope_theta, (float)(2 * f + 2) / (float)kD);
-                    rw[ks][w] = rope_word_at<T>(__fmul_rn((float)pos, f0), __fmul_rn((float)pos, f1));
-                }
         }
+        float fpos = (float)pos;
         // Rows of hidden slots may hold anything (their probability is zero, but 0 * NaN is not), so
         // they are zeroed on the way into the P.V product: masks of this lane's operand keys
         // 16 ks + 4 kq .. + 3, two 16-bit values per word.
@@ -803,6 +802,7 @@ __global__ void __launch_bounds__(kStreamThreads, kStreamWgPerCu) decode_stream_
             relv[jb] = (uint32_t)(row_off * kEs) + ((((uint32_t)lane & 15u) ^ (((uint32_t)r & 7u) << 1)) << 4);
             cache_only[jb] = __builtin_amdgcn_ballot_w64(seg_c[jb] == 1) == ~0ull;
         }
+        asm volatile("" : "+v"(fpos));   // the loads above have come back: a wait for them behind the copies would be one for those
         // slab pointers of (b, kvh)
         auto slabs = [&](int b, int kvh, const char* (&kb)[3], const char* (&vb)[3]) {
             const int64_t o0 = ((int64_t)b * a.sink_stride[0] + (int64_t)kvh * a.sink_stride[1]) * kEs;
@@ -846,7 +846,7 @@ __global__ void __launch_bounds__(kStreamThreads, kStreamWgPerCu) decode_stream_
             copy_rows(vb, relv, lds_base + st * kStreamStage + kSK * 256 + wave * 4096);
         };
 
-        int b = (int)(bh0 / KVH), kvh = (int)(bh0 % KVH);
+        int b = (int)((uint32_t)bh0 / (uint32_t)KVH), kvh = bh0 - b * KVH;
         // results of the previous item, stored at the top of the next one
         bool pending = false;
         int pend_b = 0, pend_kvh = 0;
@@ -860,8 +860,8 @@ __global__ void __launch_bounds__(kStreamThreads, kStreamWgPerCu) decode_stream_
         // of them (two wavefronts one more each), and none before the first item of a run has results.
         auto flush = [&]() {
             if (!pending) return;
-            const int64_t pend_item = jt * nbh + (int64_t)pend_b * KVH + pend_kvh;
-            const int64_t chunk_i = (pend_item - item0) * gridDim.x + blockIdx.x;
+            const int pend_item = jt * nbh + pend_b * KVH + pend_kvh;
+            const int64_t chunk_i = (int64_t)(pend_item - item0) * gridDim.x + blockIdx.x;
             unsigned char* chunk = p.chunks + chunk_i * (G * (kSK + kD) * 2);
             if (wave == kStreamProbWave && pg < G)  // every wavefront holds all of them: one stores, 16 bytes a lane
                 *reinterpret_cast<uint4*>(chunk + (pg * kSK + kKpl * kgrp) * 2) = pend_e;
@@ -880,6 +880,19 @@ __global__ void __launch_bounds__(kStreamThreads, kStreamWgPerCu) decode_stream_
         // one (kDb and up, once there is one), V rows of the next item (4).
         copy_kq(b, kvh, 0);
         copy_v(b, kvh, 0);
+        // cos and sin while the first rows are on their way
+        RopeWord<T> rw[2][4];  // [ks][word]: dims 32 ks + 8 kq + 2 w, + 1 and their partners 64 further
+#pragma unroll
+        for (int ks = 0; ks < 2; ks++) {
+            float f[8];
+#pragma unroll
+            for (int e = 0; e < 8; e += 4) {
+                const float4 f4 = *reinterpret_cast<const float4*>(freqs + 32 * ks + 8 * kq + e);
+                f[e] = f4.x; f[e + 1] = f4.y; f[e + 2] = f4.z; f[e + 3] = f4.w;
+            }
+#pragma unroll
+            for (int w = 0; w < 4; w++) rw[ks][w] = rope_word_at<T>(__fmul_rn(fpos, f[2 * w]), __fmul_rn(fpos, f[2 * w + 1]));
+        }
         // the first query block of the run must have landed for every wavefront (younger: the four V copies)
         __builtin_amdgcn_s_waitcnt(0x0F74);
         __builtin_amdgcn_s_barrier();
@@ -909,7 +922,7 @@ __global__ void __launch_bounds__(kStreamThreads, kStreamWgPerCu) decode_stream_
             }
         };
         static_assert(kDb <= 2, "wait_copies covers up to kDb + 2 stores");
-        for (int64_t bh = bh0; bh < bh1; bh++) {
+        for (int bh = bh0; bh < bh1; bh++) {
             int b_nx = b, kvh_nx = kvh;
             if (bh + 1 < bh1) {  // the last item of a run copies itself again: cheaper than a different path
                 kvh_nx = kvh + 1 == KVH ? 0 : kvh + 1;
@@ -1056,7 +1069,8 @@ __global__ void __launch_bounds__(kStreamThreads, kStreamWgPerCu) decode_stream_
 constexpr int kWideQ = 2 * kStreamStage;            // two query blocks [8 heads][256 bytes]
 constexpr int kWideS = kWideQ + 2 * 2048;           // two [8 heads] logit planes, rows of kWidePitch floats
 constexpr int kWidePitch = kSK + 16;                // the pad spreads the heads over the banks
-constexpr int kWideLds = kWideS + 2 * 8 * kWidePitch * 4;
+constexpr int kWideFreq = kWideS + 2 * 8 * kWidePitch * 4;
+constexpr int kWideLds = kWideFreq + 64 * 4;
 
 __device__ inline void wait_vm(int n, bool lds_too) {  // s_waitcnt vmcnt(n) [lgkmcnt(0)]: the count is an immediate
     if (lds_too) {
@@ -1088,8 +1102,8 @@ __global__ void __launch_bounds__(kStreamThreads, kStreamWgPerCu) decode_stream_
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int key16 = lane & 15, kq = lane >> 4;  // logits: MFMA column (key) and k-quarter; softmax and P.V: head and key quarter
     constexpr int kPv = kSK / 16, kDb = kStreamDimBlocks;   // contraction steps of 16 keys
-    const int64_t nbh = a.B * a.KVH, total = (int64_t)p.n_vis * nbh;
-    const int64_t item0 = total * blockIdx.x / gridDim.x, item1 = total * (blockIdx.x + 1) / gridDim.x;
+    const int nbh = p.nbh;
+    const int item0 = stream_first_item(p, (int)blockIdx.x), item1 = stream_first_item(p, (int)blockIdx.x + 1);
     const int64_t NS = a.num_sink, S = a.S;
     const int KVH = (int)a.KVH;
     constexpr int kEs = (int)sizeof(T);
@@ -1114,32 +1128,26 @@ __global__ void __launch_bounds__(kStreamThreads, kStreamWgPerCu) decode_stream_
     float* s_all = reinterpret_cast<float*>(smem + kWideS);  // [2][8][kWidePitch]
     const bool head_ok = key16 < G;
 
-    for (int64_t item = item0; item < item1;) {
-        const int64_t jt = item / nbh, bh0 = item % nbh;  // jt: the tile's rank among those with items
-        const int64_t tile = stream_tile_of(p, (int)jt);
-        const int64_t bh1 = (jt + 1) * nbh > item1 ? item1 - jt * nbh : nbh;
+    float* freqs = reinterpret_cast<float*>(smem + kWideFreq);
+    stage_freqs(a, freqs, tid);
+    __syncthreads();
+    int jt = (int)((uint32_t)item0 / (uint32_t)nbh), bh0 = item0 - jt * nbh;  // jt: the tile's rank among those with items
+    for (int item = item0; item < item1; jt++, bh0 = 0) {
+        const int64_t tile = stream_tile_of(p, jt);
+        const int bh1 = (jt + 1) * nbh > item1 ? item1 - jt * nbh : nbh;
         item = jt * nbh + bh1;
         const int64_t n_wave = tile * kSK + wave * 16;  // first key of this wavefront
 
         // ---- per-tile constants (the same for every (b, kvh): positions are shared)
         bool vis1 = false;
-        RopeWord<T> rw[2][4];  // [ks][word]: dims 32 ks + 8 kq + 2 w, + 1 and their partners 64 further
+        int64_t pos = 0;
         {
             const int64_t n = n_wave + key16;
-            int64_t pos = 0;
             if (n < NS) { vis1 = a.sink_mask[n] == 0; pos = a.sink_pos[n]; }
             else if (n < NS + S) { vis1 = a.mask[n - NS] == 0; pos = a.pos[n - NS] + a.pos_shift; }
             else if (n < p.N) { vis1 = true; pos = a.q_pos[0]; }
-#pragma unroll
-            for (int ks = 0; ks < 2; ks++)
-#pragma unroll
-                for (int w = 0; w < 4; w++) {
-                    const int f = 32 * ks + 8 * kq + 2 * w;
-                    const float f0 = a.inv_freq ? a.inv_freq[f] : 1.0f / powf(a.rope_theta, (float)(2 * f) / (float)kD);
-                    const float f1 = a.inv_freq ? a.inv_freq[f + 1] : 1.0f / powf(a.rope_theta, (float)(2 * f + 2) / (float)kD);
-                    rw[ks][w] = rope_word_at<T>(__fmul_rn((float)pos, f0), __fmul_rn((float)pos, f1));
-                }
         }
+        float fpos = (float)pos;
         // rows of hidden slots are zeroed on the way into the P.V product (0 * NaN): masks of this lane's
         // operand keys 16 ks + 4 kq .. + 3, two 16-bit values per word
         uint32_t m01[kPv], m23[kPv];
@@ -1175,6 +1183,7 @@ __global__ void __launch_bounds__(kStreamThreads, kStreamWgPerCu) decode_stream_
             relv[jb] = (uint32_t)(row_off * kEs) + ((((uint32_t)lane & 15u) ^ (((uint32_t)r & 7u) << 1)) << 4);
             cache_only[jb] = __builtin_amdgcn_ballot_w64(seg_c[jb] == 1) == ~0ull;
         }
+        asm volatile("" : "+v"(fpos));   // as in the kernel above
         auto slabs = [&](int b, int kvh, const char* (&kb)[3], const char* (&vb)[3]) {
             const int64_t o0 = ((int64_t)b * a.sink_stride[0] + (int64_t)kvh * a.sink_stride[1]) * kEs;
             const int64_t o1 = ((int64_t)b * a.cache_stride[0] + (int64_t)kvh * a.cache_stride[1]) * kEs;
@@ -1214,7 +1223,7 @@ __global__ void __launch_bounds__(kStreamThreads, kStreamWgPerCu) decode_stream_
             copy_rows(vb, relv, lds_base + st * kStreamStage + kSK * 256 + wave * 4096);
         };
 
-        int b = (int)(bh0 / KVH), kvh = (int)(bh0 % KVH);
+        int b = (int)((uint32_t)bh0 / (uint32_t)KVH), kvh = bh0 - b * KVH;
         // results of the previous item, stored at the top of the next one
         bool pending = false;
         int pend_b = 0, pend_kvh = 0;
@@ -1225,8 +1234,8 @@ __global__ void __launch_bounds__(kStreamThreads, kStreamWgPerCu) decode_stream_
         for (int b2 = 0; b2 < kDb; b2++) pend_o[b2] = make_uint2(0u, 0u);
         auto flush = [&]() {
             if (!pending) return;
-            const int64_t pend_item = jt * nbh + (int64_t)pend_b * KVH + pend_kvh;
-            const int64_t chunk_i = (pend_item - item0) * gridDim.x + blockIdx.x;
+            const int pend_item = jt * nbh + pend_b * KVH + pend_kvh;
+            const int64_t chunk_i = (int64_t)(pend_item - item0) * gridDim.x + blockIdx.x;
             unsigned char* chunk = p.chunks + chunk_i * (G * (kSK + kD) * 2);
             if (head_ok) {
                 *reinterpret_cast<uint2*>(chunk + (key16 * kSK + 16 * wave + 4 * kq) * 2) = pend_e;
@@ -1244,11 +1253,24 @@ __global__ void __launch_bounds__(kStreamThreads, kStreamWgPerCu) decode_stream_
         int stored = 0;
         copy_kq(b, kvh, 0);
         copy_v(b, kvh, 0);
+        // cos and sin while the first rows are on their way
+        RopeWord<T> rw[2][4];  // [ks][word]: dims 32 ks + 8 kq + 2 w, + 1 and their partners 64 further
+#pragma unroll
+        for (int ks = 0; ks < 2; ks++) {
+            float f[8];
+#pragma unroll
+            for (int e = 0; e < 8; e += 4) {
+                const float4 f4 = *reinterpret_cast<const float4*>(freqs + 32 * ks + 8 * kq + e);
+                f[e] = f4.x; f[e + 1] = f4.y; f[e + 2] = f4.z; f[e + 3] = f4.w;
+            }
+#pragma unroll
+            for (int w = 0; w < 4; w++) rw[ks][w] = rope_word_at<T>(__fmul_rn(fpos, f[2 * w]), __fmul_rn(fpos, f[2 * w + 1]));
+        }
         // the first query block of the run must have landed for every wavefront (younger: the four V copies)
         __builtin_amdgcn_s_waitcnt(0x0F74);
         __builtin_amdgcn_s_barrier();
         int st = 0;
-        for (int64_t bh = bh0; bh < bh1; bh++) {
+        for (int bh = bh0; bh < bh1; bh++) {
             int b_nx = b, kvh_nx = kvh;
             if (bh + 1 < bh1) {  // the last item of a run copies itself again: cheaper than a different path
                 kvh_nx = kvh + 1 == KVH ? 0 : kvh + 1;
@@ -1456,13 +1478,13 @@ struct TailLds {
     float o[32][kD];
 };
 template <typename T>
-__device__ inline void tail_stream_row(const DecodeParams& p, int64_t row, TailLds& sh) {  // row: b * H + h
+__device__ inline void tail_stream_row(const DecodeParams& p, int row, TailLds& sh) {  // row: b * H + h
     const ckv_attn_args& a = p.a;
     const int tid = threadIdx.x, d8 = tid & 15, grp = tid >> 4;
     const int n_vis = p.n_vis;  // the items are numbered over the tiles that can hold a visible key
-    const int64_t nbh = a.B * a.KVH, total = (int64_t)n_vis * nbh;
-    const int G = (int)(a.H / a.KVH), g = (int)((row % a.H) % G);
-    const int64_t bh = (row / a.H) * a.KVH + (row % a.H) / G;
+    const int nbh = p.nbh, H = (int)a.H, KVH = (int)a.KVH;
+    const int G = (int)((uint32_t)H / (uint32_t)KVH), b = (int)((uint32_t)row / (uint32_t)H), h = row - b * H;
+    const int kvh = (int)((uint32_t)h / (uint32_t)G), g = h - kvh * G, bh = b * KVH + kvh;
     const int64_t chunk_bytes = (int64_t)G * (kSK + kD) * 2;
     const int64_t in_chunk = ((int64_t)G * kSK + g * kD) * 2 + d8 * 16;
     float M = -INFINITY, L = 0.f;
@@ -1474,7 +1496,7 @@ __device__ inline void tail_stream_row(const DecodeParams& p, int64_t row, TailL
         int64_t ck_mine = 0;
         {
             const int t = t0 + 32 * d8;
-            if (d8 < kTailBatch && t < n_vis) ck_mine = stream_chunk_of((int64_t)t * nbh + bh, total, p.stream_wgs);
+            if (d8 < kTailBatch && t < n_vis) ck_mine = stream_chunk_of(p, t * nbh + bh);
         }
         uint4 v[kTailBatch];
         float2 w[kTailBatch];
@@ -1528,7 +1550,6 @@ __device__ inline void tail_stream_row(const DecodeParams& p, int64_t row, TailL
         od = fmaf(sh.o[k][tid], f, od);
         L = fmaf(sh.l[k], f, L);
     }
-    const int64_t b = row / a.H, h = row % a.H;
     T* out = (T*)a.out + b * a.out_stride[0] + h * a.out_stride[1];
     out[tid * a.out_stride[3]] = Elem<T>::from_float(od / L);
     if (tid == 0) {
@@ -1541,7 +1562,7 @@ __device__ inline void tail_stream_row(const DecodeParams& p, int64_t row, TailL
 template <typename T>
 __global__ void __launch_bounds__(512) decode_tail_stream_kernel(DecodeParams p) {
     __shared__ TailLds sh;
-    tail_stream_row<T>(p, blockIdx.x, sh);
+    tail_stream_row<T>(p, (int)blockIdx.x, sh);
 }
 
 template <typename T, int G>
@@ -1594,8 +1615,7 @@ __global__ void __launch_bounds__(256) decode_scores_kernel(DecodeParams p, floa
                 const int jt = stream_rank_of(p, (int)(n / kSK));  // -1: no key of the tile is visible
                 pt = 0.f;
                 if (jt >= 0) {
-                    const int64_t ck = stream_chunk_of((int64_t)jt * (a.B * a.KVH) + b * a.KVH + kv,
-                                                       (int64_t)p.n_vis * (a.B * a.KVH), p.stream_wgs);
+                    const int64_t ck = stream_chunk_of(p, jt * p.nbh + (int)(b * a.KVH + kv));
                     const float e = (float)reinterpret_cast<const _Float16*>(p.chunks + ck * (G * (kSK + kD) * 2))[g * kSK + n % kSK];
                     const float m = p.part_ml[(ck * G + g) * 2];
                     pt = e == 0.f ? 0.f : round_t<T>(e * __builtin_amdgcn_exp2f(m - p.lse2[row]));
@@ -1651,8 +1671,7 @@ __device__ inline void scores_of_group(const DecodeParams& p, int64_t n0, int64_
     if (n0 + 8 <= a.num_sink || n0 >= p.N) return;  // sinks keep no score; padding
     float pr[G][8];
     const int jt = stream_rank_of(p, (int)(n0 / kSK));  // -1: no key of the tile is visible, all probabilities are 0
-    const int64_t ck = jt < 0 ? 0 : stream_chunk_of((int64_t)jt * (a.B * a.KVH) + b * a.KVH + kvh,
-                                                    (int64_t)p.n_vis * (a.B * a.KVH), p.stream_wgs);
+    const int64_t ck = jt < 0 ? 0 : stream_chunk_of(p, jt * p.nbh + (int)(b * a.KVH + kvh));
     const unsigned char* chunk = p.chunks + ck * (G * (kSK + kD) * 2);
 #pragma unroll
     for (int g = 0; g < G; g++) {
@@ -1734,11 +1753,11 @@ __device__ inline void scores_of_group(const DecodeParams& p, int64_t n0, int64_
 template <typename T, int G>
 __global__ void __launch_bounds__(256) decode_scores_probs_kernel(DecodeParams p, float w_one, float beta_pow) {
     const ckv_attn_args& a = p.a;
-    const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t per = p.Np / 8;
-    if (idx >= a.B * a.KVH * per) return;
-    const int64_t kvh = (idx / per) % a.KVH, b = idx / (per * a.KVH);
-    scores_of_group<T, G>(p, (idx % per) * 8, b, kvh, w_one, beta_pow, [&](int g) { return p.lse2[b * a.H + kvh * G + g]; });
+    const uint32_t idx = blockIdx.x * 256u + threadIdx.x, per = (uint32_t)p.Np / 8u;   // eighths of the items' keys: below 2^32
+    const uint32_t unit = idx / per;
+    if (unit >= (uint32_t)p.nbh) return;
+    const int b = (int)(unit / (uint32_t)a.KVH), kvh = (int)(unit - (uint32_t)b * (uint32_t)a.KVH);
+    scores_of_group<T, G>(p, (int64_t)(idx - unit * per) * 8, b, kvh, w_one, beta_pow, [&](int g) { return p.lse2[b * a.H + kvh * G + g]; });
 }
 
 // Tail and scores in one launch: the first B * H workgroups combine a row each, the others work out the scores of 4096
@@ -1752,12 +1771,11 @@ __global__ void __launch_bounds__(512) decode_finish_kernel(DecodeParams p, floa
     const ckv_attn_args& a = p.a;
     const int rows = (int)(a.B * a.H), tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     if ((int)blockIdx.x < rows) {
-        tail_stream_row<T>(p, blockIdx.x, sh);
+        tail_stream_row<T>(p, (int)blockIdx.x, sh);
         return;
     }
     static_assert(G <= 8, "a wavefront per head merges the pairs");
-    const int id = (int)blockIdx.x - rows, unit = id / per_unit;
-    const int64_t nbh = a.B * a.KVH, total = (int64_t)p.n_vis * nbh;
+    const int id = (int)blockIdx.x - rows, unit = (int)((uint32_t)id / (uint32_t)per_unit), KVH = (int)a.KVH;
     float* sh_lse = &sh.m[0];
     if (wave < G) {
         float M = -INFINITY, L = 0.f;
@@ -1769,7 +1787,7 @@ __global__ void __launch_bounds__(512) decode_finish_kernel(DecodeParams p, floa
                 const int t = t0 + 64 * u;
                 w[u] = make_float2(-INFINITY, 0.f);
                 if (t < p.n_vis) {
-                    const int64_t ck = stream_chunk_of((int64_t)t * nbh + unit, total, p.stream_wgs);
+                    const int64_t ck = stream_chunk_of(p, t * p.nbh + unit);
                     w[u] = *reinterpret_cast<const float2*>(p.part_ml + (ck * G + wave) * 2);
                 }
             }
@@ -1790,9 +1808,10 @@ __global__ void __launch_bounds__(512) decode_finish_kernel(DecodeParams p, floa
         if (lane == 0) sh_lse[wave] = Mx + __builtin_amdgcn_logf(L);
     }
     __syncthreads();
-    const int64_t n0 = ((int64_t)(id % per_unit) * 512 + tid) * 8;
+    const int64_t n0 = ((int64_t)(id - unit * per_unit) * 512 + tid) * 8;
     if (n0 >= p.Np) return;
-    scores_of_group<T, G>(p, n0, unit / a.KVH, unit % a.KVH, w_one, beta_pow, [&](int g) { return sh_lse[g]; });
+    const int b = (int)((uint32_t)unit / (uint32_t)KVH);
+    scores_of_group<T, G>(p, n0, b, unit - b * KVH, w_one, beta_pow, [&](int g) { return sh_lse[g]; });
 }
 
 // All heads reduced together (cascade_attention.py:240-242) after a streaming kernel: one thread per (batch, key),
@@ -1816,8 +1835,7 @@ __global__ void __launch_bounds__(kSK) decode_scores_homo_kernel(DecodeParams p,
         const int kv = tid / G, g = tid % G;
         float c = 0.f;
         if (jt >= 0) {
-            const int64_t ck = stream_chunk_of((int64_t)jt * (a.B * KVH) + (int64_t)b * KVH + kv, (int64_t)p.n_vis * (a.B * KVH),
-                                               p.stream_wgs);
+            const int64_t ck = stream_chunk_of(p, jt * p.nbh + b * KVH + kv);
             c = __builtin_amdgcn_exp2f(p.part_ml[(ck * G + g) * 2] - p.lse2[(int64_t)b * H + tid]);
             if (g == 0) sh_ck[kv] = ck;
         }
@@ -1880,7 +1898,8 @@ int run_decode(const DecodeParams& p_in, hipStream_t stream) {
     DecodeParams p = p_in;
     const ckv_attn_args& a = p.a;
     const bool use_stream =
-        !std::is_same<T, float>::value && G <= 8 && p.shared_pos && stream_offsets_fit(a);
+        !std::is_same<T, float>::value && G <= 8 && p.shared_pos && stream_offsets_fit(a) &&
+        (p.N + kSK) * a.B * a.KVH < (int64_t)1 << 34;   // items and eighths of their keys are numbered in 32 bits
     if (use_stream) {
         p.tiles = (int)((p.N + kSK - 1) / kSK);  // the streaming kernel has its own tile size
         // keys that can be visible: the sinks, the leading `filled_slots` cache slots (all S when the caller gives
@@ -1921,6 +1940,8 @@ int run_decode(const DecodeParams& p_in, hipStream_t stream) {
                 if (wgs > kStreamMaxWgs) wgs = kStreamMaxWgs;
                 if (wgs > p.n_vis * nbh) wgs = p.n_vis * nbh;
                 p.stream_wgs = (int)wgs;
+                p.run_q = (int)(p.n_vis * nbh / wgs);
+                p.run_r = (int)(p.n_vis * nbh % wgs);
                 hipEvent_t ev0, ev1;
                 prof_kernel_events(CKV_STAGE_DECODE, &ev0, &ev1);
                 if constexpr (G <= 4) {
@@ -2060,7 +2081,8 @@ int launch_decode(const ckv_attn_args& a, hipStream_t stream) {
     p.qrot_t = w; w += align_up(a.B * a.H * kD * 4, 256);
     p.logits = reinterpret_cast<float*>(w);
     p.chunks = reinterpret_cast<unsigned char*>(w);
-    p.stream_wgs = 0;
+    p.stream_wgs = p.run_q = p.run_r = 0;
+    p.nbh = (int)(a.B * a.KVH);
     p.tiles_pre = 0;
     p.n_vis = 0;
     w += logits_area_bytes(a.B, a.H, a.KVH, p.N);
