@@ -100,6 +100,8 @@ struct DecodeParams {
     int stream_wgs;    // workgroups of the streaming kernel
     int nbh;           // B * KVH, the items of a tile
     int run_q, run_r;  // items / stream_wgs and what is left: see stream_first_item
+    int own_q;         // every workgroup of the streaming kernel rotates the queries itself, see SharedQueries
+    uint32_t inv_h;    // 2^16 / H, rounded up
     float* part_ml;    // (B, H, tiles, 2); after the streaming kernel (chunk, G, 2)
     float* part_o;     // (B, H, tiles, 128)
     float* lse2;       // (B, H)
@@ -133,23 +135,33 @@ __device__ inline int64_t stream_chunk_of(const DecodeParams& p, int item) {
     return (int64_t)(item - stream_first_item(p, (int)w)) * p.stream_wgs + w;
 }
 
+__device__ inline float pair_freq(const ckv_attn_args& a, int j) {   // of rotation pair j
+    return a.inv_freq ? a.inv_freq[j] : 1.0f / powf(a.rope_theta, (float)(2 * j) / (float)kD);
+}
+// Elements j and j + 64 of a query row.  From the elements as they are stored, wherever they were read: the compiler forms the
+// same instructions of the tensor dtype (fused ones among them) from the same expression, so that both callers agree to the bit.
+template <typename T>
+__device__ inline void rotate_query(T x1, T x2, float cs, float sn, float post, float& r1, float& r2) {
+    rope_ref<T>(Elem<T>::to_float(x1), Elem<T>::to_float(x2), round_t<T>(cs), round_t<T>(sn), post, r1, r2);
+}
+template <typename T>
+__device__ inline const T* query_row(const ckv_attn_args& a, uint32_t row) {   // row: b * H + h
+    const int64_t b = row / (uint32_t)a.H, h = row - (uint32_t)b * (uint32_t)a.H;
+    return (const T*)a.q + b * a.q_stride[0] + h * a.q_stride[1];
+}
+
 template <typename T>
 __global__ void decode_q_kernel(DecodeParams p) {
-    const ckv_attn_args& a = p.a;
-    const int64_t row = blockIdx.x;  // b * H + h
-    const int j = threadIdx.x;       // 0..63: rotation pair
-    const int64_t b = blockIdx.x / (uint32_t)a.H, h = blockIdx.x - (uint32_t)b * (uint32_t)a.H;
-    const T* q = (const T*)a.q + b * a.q_stride[0] + h * a.q_stride[1];
-    const float f = a.inv_freq ? a.inv_freq[j] : 1.0f / powf(a.rope_theta, (float)(2 * j) / (float)kD);
-    float sn, cs;
-    sincosf(__fmul_rn((float)a.q_pos[0], f), &sn, &cs);
-    const float x1 = Elem<T>::to_float(q[j * a.q_stride[3]]), x2 = Elem<T>::to_float(q[(j + 64) * a.q_stride[3]]);
-    float r1, r2;
-    rope_ref<T>(x1, x2, round_t<T>(cs), round_t<T>(sn), p.key_scale, r1, r2);
-    p.qrot[row * kD + j] = r1 * p.scale_log2;
-    p.qrot[row * kD + 64 + j] = r2 * p.scale_log2;
-    ((T*)p.qrot_t)[row * kD + j] = Elem<T>::from_float(r1);
-    ((T*)p.qrot_t)[row * kD + 64 + j] = Elem<T>::from_float(r2);
+    const uint32_t row = blockIdx.x;  // b * H + h
+    const int j = threadIdx.x;        // 0..63: rotation pair
+    const T* q = query_row<T>(p.a, row);
+    float sn, cs, r1, r2;
+    sincosf(__fmul_rn((float)p.a.q_pos[0], pair_freq(p.a, j)), &sn, &cs);
+    rotate_query<T>(q[j * p.a.q_stride[3]], q[(j + 64) * p.a.q_stride[3]], cs, sn, p.key_scale, r1, r2);
+    p.qrot[(int64_t)row * kD + j] = r1 * p.scale_log2;
+    p.qrot[(int64_t)row * kD + 64 + j] = r2 * p.scale_log2;
+    ((T*)p.qrot_t)[(int64_t)row * kD + j] = Elem<T>::from_float(r1);
+    ((T*)p.qrot_t)[(int64_t)row * kD + 64 + j] = Elem<T>::from_float(r2);
 }
 
 // source row of key n: sink, cache slot or the new token
@@ -652,6 +664,7 @@ __global__ void __launch_bounds__(256, 2) decode_main_mfma_kernel(DecodeParams p
 // path.
 // ---------------------------------------------------------------------------------------------
 constexpr int kStreamThreads = 64 * kStreamWaves;
+constexpr int kOwnQRows = 64;                     // query rows (batch x heads) a workgroup of the streaming kernel rotates itself
 constexpr int kStreamWgPerCu = 8 / kStreamWaves;  // eight wavefronts per CU
 constexpr int kStreamDimBlocks = 8 / kStreamWaves;  // 16-dim blocks of the output a wavefront owns
 constexpr int kStreamStage = 2 * kSK * 256;       // K rows then V rows of one tile (16-bit, 256 B per row)
@@ -659,7 +672,9 @@ constexpr int kStreamStage = 2 * kSK * 256;       // K rows then V rows of one t
 constexpr int kStreamQ = 2 * kStreamStage, kStreamS = kStreamQ + 2 * 1024, kStreamP = kStreamS + 2 * 4 * kSK * 4;
 constexpr int kStreamPPitch = kSK * 2 + 32;        // bytes per head row of the probabilities: the pad puts the four heads on different banks
 constexpr int kStreamFreq = kStreamP + kStreamWaves * 4 * kStreamPPitch;   // the 64 rotation frequencies
-constexpr int kStreamLds = kStreamFreq + 64 * 4;
+constexpr int kStreamOwnQ = kStreamFreq + 64 * 4;   // the rotated queries of every head, where the workgroup rotates them itself
+constexpr int kStreamLds = kStreamOwnQ + kOwnQRows * 256;
+static_assert(kStreamLds <= 160 * 1024, "one workgroup per compute unit");
 
 // sum / max over the four 16-lane rows of a wavefront (lanes l, l^16, l^32, l^48)
 __device__ inline float rows4_sum(float x) {
@@ -686,9 +701,63 @@ __device__ inline float mod4_sum(float l) {
     return rows4_sum(l);
 }
 
-__device__ inline void stage_freqs(const ckv_attn_args& a, float* freqs, int tid) {
-    if (tid < kD / 2) freqs[tid] = a.inv_freq ? a.inv_freq[tid] : 1.0f / powf(a.rope_theta, (float)(2 * tid) / (float)kD);
-}
+// What the workgroups of a streaming kernel share, by all its threads: the 64 frequencies in LDS and, with few query rows (own_q),
+// all of them rotated there, head g of a kv head with its 16-byte piece c in slot c ^ g.  The rows are a kernel of their own
+// otherwise, whose launch costs a step of one stream 4 us on the device and 3 on the host.  Requested at the start, worked out
+// while the first rows of the cache are on their way.
+template <typename T, int G>
+struct SharedQueries {
+    static constexpr int kRows = kOwnQRows / kStreamWaves;   // of a thread: its wavefront's number and every eighth from there
+    float f = 0.f, pos = 0.f;
+    uint32_t x1[kRows] = {}, x2[kRows] = {};   // elements j and j + 64 of the rows, as they lie in memory
+    __device__ void request(const DecodeParams& p, int tid, uint32_t wave) {
+        const ckv_attn_args& a = p.a;
+        const int j = tid & 63;
+        f = pair_freq(a, j);
+        if (!p.own_q) return;
+        pos = (float)a.q_pos[0];
+#pragma unroll
+        for (int i = 0; i < kRows; i++) {
+            const uint32_t row = wave + kStreamWaves * i;
+            if (row < (uint32_t)(p.nbh * G)) {
+                const uint32_t b = row * p.inv_h >> 16, h = row - b * (uint32_t)a.H;   // row / H, both below 64
+                const T* q = (const T*)a.q + b * a.q_stride[0] + h * a.q_stride[1];
+                x1[i] = __builtin_bit_cast(uint16_t, q[j * a.q_stride[3]]);
+                x2[i] = __builtin_bit_cast(uint16_t, q[(j + 64) * a.q_stride[3]]);
+            }
+        }
+    }
+    // called before the first copies go out: a wait for these loads behind them would be one for the copies too
+    __device__ void arrived() {
+        asm volatile("" : "+v"(f), "+v"(pos));
+#pragma unroll
+        for (int i = 0; i < kRows; i++) asm volatile("" : "+v"(x1[i]), "+v"(x2[i]));
+    }
+    __device__ void finish(const DecodeParams& p, float* freqs, unsigned char* own_q, int tid, uint32_t wave) {
+        const uint32_t j = tid & 63;
+        if (tid < 64) freqs[tid] = f;
+        if (p.own_q) {
+            float sn, cs;
+            sincosf(__fmul_rn(pos, f), &sn, &cs);
+#pragma unroll
+            for (int i = 0; i < kRows; i++) {
+                const uint32_t row = wave + kStreamWaves * i;
+                if (row < (uint32_t)(p.nbh * G)) {
+                    float r1, r2;
+                    rotate_query<T>(__builtin_bit_cast(T, (uint16_t)x1[i]), __builtin_bit_cast(T, (uint16_t)x2[i]), cs, sn, p.key_scale, r1, r2);
+                    unsigned char* at = own_q + row * 256 + (j % 8) * 2;
+                    const uint32_t g = row % (uint32_t)G;
+                    *reinterpret_cast<T*>(at + (((j / 8) ^ g) << 4)) = Elem<T>::from_float(r1);
+                    *reinterpret_cast<T*>(at + (((j / 8 + 8) ^ g) << 4)) = Elem<T>::from_float(r2);
+                }
+            }
+        }
+        // in LDS for every wavefront; a barrier of the language would also wait for the copies
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    }
+};
 
 // the byte offsets of the rows inside a (b, kvh) slab must fit the 32-bit lane offsets of the copies
 inline bool stream_offsets_fit(const ckv_attn_args& a) {
@@ -740,13 +809,14 @@ __global__ void __launch_bounds__(kStreamThreads, kStreamWgPerCu) decode_stream_
     // query block of an item: head g at g * 256, its 16-byte piece c in slot c ^ g (the heads' rows would
     // otherwise sit on the same banks); lanes of idle MFMA rows read head 0 (their results are not used)
     const int q_row = key16 < G ? key16 : 0;
-    const int q_off = kStreamQ + q_row * 256 + ((kq ^ q_row) << 4);
+    const int q_off = q_row * 256 + ((kq ^ q_row) << 4);
     float* s_all = reinterpret_cast<float*>(smem + kStreamS);                                   // [2][4][kSK]
     unsigned char* p_wave = smem + kStreamP + wave * (4 * kStreamPPitch);                       // [4][kSK] 16-bit, padded rows
 
     float* freqs = reinterpret_cast<float*>(smem + kStreamFreq);
-    stage_freqs(a, freqs, tid);
-    __syncthreads();
+    SharedQueries<T, G> shared;
+    shared.request(p, tid, wave);
+    bool first_tile = true;
     int jt = (int)((uint32_t)item0 / (uint32_t)nbh), bh0 = item0 - jt * nbh;  // jt: the tile's rank among the visible ones
     for (int item = item0; item < item1; jt++, bh0 = 0) {
         const int64_t tile = stream_tile_of(p, jt);
@@ -802,7 +872,9 @@ __global__ void __launch_bounds__(kStreamThreads, kStreamWgPerCu) decode_stream_
             relv[jb] = (uint32_t)(row_off * kEs) + ((((uint32_t)lane & 15u) ^ (((uint32_t)r & 7u) << 1)) << 4);
             cache_only[jb] = __builtin_amdgcn_ballot_w64(seg_c[jb] == 1) == ~0ull;
         }
-        asm volatile("" : "+v"(fpos));   // the loads above have come back: a wait for them behind the copies would be one for those
+        // the loads above have come back: a wait for them behind the copies would be one for those
+        asm volatile("" : "+v"(fpos));
+        if (first_tile) shared.arrived();
         // slab pointers of (b, kvh)
         auto slabs = [&](int b, int kvh, const char* (&kb)[3], const char* (&vb)[3]) {
             const int64_t o0 = ((int64_t)b * a.sink_stride[0] + (int64_t)kvh * a.sink_stride[1]) * kEs;
@@ -830,7 +902,7 @@ __global__ void __launch_bounds__(kStreamThreads, kStreamWgPerCu) decode_stream_
         // goes first: whoever waits for the four K copies behind it has waited for it too, and the item's barrier
         // makes it visible to the other wavefronts.
         auto copy_kq = [&](int b, int kvh, int st) {
-            if (wave == 0) {
+            if (wave == 0 && !p.own_q) {
                 const char* qsrc = (const char*)p.qrot_t + ((int64_t)b * a.H + (int64_t)kvh * G) * (kD * kEs);
                 if ((lane >> 4) < G)
                     async_copy16(qsrc, (lane >> 4) * 256 + (((lane & 15) ^ (lane >> 4)) << 4), lds_base + kStreamQ + st * 1024);
@@ -880,6 +952,8 @@ __global__ void __launch_bounds__(kStreamThreads, kStreamWgPerCu) decode_stream_
         // one (kDb and up, once there is one), V rows of the next item (4).
         copy_kq(b, kvh, 0);
         copy_v(b, kvh, 0);
+        if (first_tile) shared.finish(p, freqs, smem + kStreamOwnQ, tid, wave);
+        first_tile = false;
         // cos and sin while the first rows are on their way
         RopeWord<T> rw[2][4];  // [ks][word]: dims 32 ks + 8 kq + 2 w, + 1 and their partners 64 further
 #pragma unroll
@@ -935,6 +1009,7 @@ __global__ void __launch_bounds__(kStreamThreads, kStreamWgPerCu) decode_stream_
             stored = pending ? my_stores : 0;
             flush();
             const unsigned char* stage = smem + st * kStreamStage;
+            const int q_at = p.own_q ? kStreamOwnQ + (b * KVH + kvh) * (G * 256) : kStreamQ + st * 1024;
 
             // ---- rotate K in registers, logits by MFMA, shared through LDS
             {
@@ -942,7 +1017,7 @@ __global__ void __launch_bounds__(kStreamThreads, kStreamWgPerCu) decode_stream_
 #pragma unroll
                 for (int ks = 0; ks < 4; ks++) kraw[ks] = *reinterpret_cast<const uint4*>(stage + kaddr[ks]);
 #pragma unroll
-                for (int ks = 0; ks < 4; ks++) qop[ks] = *reinterpret_cast<const uint4*>(smem + q_off + st * 1024 + ks * 64);
+                for (int ks = 0; ks < 4; ks++) qop[ks] = *reinterpret_cast<const uint4*>(smem + q_at + q_off + ks * 64);
                 uint4 kop[4];
 #pragma unroll
                 for (int ks = 0; ks < 2; ks++) {
@@ -1070,7 +1145,9 @@ constexpr int kWideQ = 2 * kStreamStage;            // two query blocks [8 heads
 constexpr int kWideS = kWideQ + 2 * 2048;           // two [8 heads] logit planes, rows of kWidePitch floats
 constexpr int kWidePitch = kSK + 16;                // the pad spreads the heads over the banks
 constexpr int kWideFreq = kWideS + 2 * 8 * kWidePitch * 4;
-constexpr int kWideLds = kWideFreq + 64 * 4;
+constexpr int kWideOwnQ = kWideFreq + 64 * 4;
+constexpr int kWideLds = kWideOwnQ + kOwnQRows * 256;
+static_assert(kWideLds <= 160 * 1024, "one workgroup per compute unit");
 
 __device__ inline void wait_vm(int n, bool lds_too) {  // s_waitcnt vmcnt(n) [lgkmcnt(0)]: the count is an immediate
     if (lds_too) {
@@ -1124,13 +1201,14 @@ __global__ void __launch_bounds__(kStreamThreads, kStreamWgPerCu) decode_stream_
     const int q_row = key16 < G ? key16 : 0;
     int q_off[4];
 #pragma unroll
-    for (int ks = 0; ks < 4; ks++) q_off[ks] = kWideQ + q_row * 256 + (((4 * ks + kq) ^ q_row) << 4);
+    for (int ks = 0; ks < 4; ks++) q_off[ks] = q_row * 256 + (((4 * ks + kq) ^ q_row) << 4);
     float* s_all = reinterpret_cast<float*>(smem + kWideS);  // [2][8][kWidePitch]
     const bool head_ok = key16 < G;
 
     float* freqs = reinterpret_cast<float*>(smem + kWideFreq);
-    stage_freqs(a, freqs, tid);
-    __syncthreads();
+    SharedQueries<T, G> shared;
+    shared.request(p, tid, wave);
+    bool first_tile = true;
     int jt = (int)((uint32_t)item0 / (uint32_t)nbh), bh0 = item0 - jt * nbh;  // jt: the tile's rank among those with items
     for (int item = item0; item < item1; jt++, bh0 = 0) {
         const int64_t tile = stream_tile_of(p, jt);
@@ -1184,6 +1262,7 @@ __global__ void __launch_bounds__(kStreamThreads, kStreamWgPerCu) decode_stream_
             cache_only[jb] = __builtin_amdgcn_ballot_w64(seg_c[jb] == 1) == ~0ull;
         }
         asm volatile("" : "+v"(fpos));   // as in the kernel above
+        if (first_tile) shared.arrived();
         auto slabs = [&](int b, int kvh, const char* (&kb)[3], const char* (&vb)[3]) {
             const int64_t o0 = ((int64_t)b * a.sink_stride[0] + (int64_t)kvh * a.sink_stride[1]) * kEs;
             const int64_t o1 = ((int64_t)b * a.cache_stride[0] + (int64_t)kvh * a.cache_stride[1]) * kEs;
@@ -1208,7 +1287,7 @@ __global__ void __launch_bounds__(kStreamThreads, kStreamWgPerCu) decode_stream_
         // i % 16 of head 4 wave + i / 16 with the piece that belongs there), then this wavefront's K rows.  The
         // query copy goes first: whoever waits for the four K copies behind it has waited for it too.
         auto copy_kq = [&](int b, int kvh, int st) {
-            if (wave < 2) {
+            if (wave < 2 && !p.own_q) {
                 const char* qsrc = (const char*)p.qrot_t + ((int64_t)b * a.H + (int64_t)kvh * G) * (kD * kEs);
                 const int h = 4 * wave + (lane >> 4);
                 if (h < G) async_copy16(qsrc, h * 256 + (((lane & 15) ^ h) << 4), lds_base + kWideQ + st * 2048 + wave * 1024);
@@ -1253,6 +1332,8 @@ __global__ void __launch_bounds__(kStreamThreads, kStreamWgPerCu) decode_stream_
         int stored = 0;
         copy_kq(b, kvh, 0);
         copy_v(b, kvh, 0);
+        if (first_tile) shared.finish(p, freqs, smem + kWideOwnQ, tid, wave);
+        first_tile = false;
         // cos and sin while the first rows are on their way
         RopeWord<T> rw[2][4];  // [ks][word]: dims 32 ks + 8 kq + 2 w, + 1 and their partners 64 further
 #pragma unroll
@@ -1286,11 +1367,12 @@ __global__ void __launch_bounds__(kStreamThreads, kStreamWgPerCu) decode_stream_
 
             // ---- rotate K in registers, logits by MFMA, shared through LDS
             {
+                const int q_at = p.own_q ? kWideOwnQ + (b * KVH + kvh) * (G * 256) : kWideQ + st * 2048;
                 uint4 kraw[4], qop[4];
 #pragma unroll
                 for (int ks = 0; ks < 4; ks++) kraw[ks] = *reinterpret_cast<const uint4*>(stage + kaddr[ks]);
 #pragma unroll
-                for (int ks = 0; ks < 4; ks++) qop[ks] = *reinterpret_cast<const uint4*>(smem + q_off[ks] + st * 2048);
+                for (int ks = 0; ks < 4; ks++) qop[ks] = *reinterpret_cast<const uint4*>(smem + q_at + q_off[ks]);
                 uint4 kop[4];
 #pragma unroll
                 for (int ks = 0; ks < 2; ks++) {
@@ -1909,7 +1991,9 @@ int run_decode(const DecodeParams& p_in, hipStream_t stream) {
         p.n_vis = p.tiles_pre < p.tiles ? p.tiles_pre + 1 : p.tiles_pre;
     }
     p.Np = (int64_t)p.tiles * kSK;
-    {
+    p.own_q = use_stream && a.B * a.H <= kOwnQRows;
+    p.inv_h = (uint32_t)((65536 + a.H - 1) / a.H);
+    if (!p.own_q) {
         StageScope sc(CKV_STAGE_PREP, stream);
         hipLaunchKernelGGL(decode_q_kernel<T>, dim3((unsigned)(a.B * a.H)), dim3(64), 0, stream, p);
         CKV_HIP_TRY(hipGetLastError());
@@ -2081,7 +2165,8 @@ int launch_decode(const ckv_attn_args& a, hipStream_t stream) {
     p.qrot_t = w; w += align_up(a.B * a.H * kD * 4, 256);
     p.logits = reinterpret_cast<float*>(w);
     p.chunks = reinterpret_cast<unsigned char*>(w);
-    p.stream_wgs = p.run_q = p.run_r = 0;
+    p.stream_wgs = p.run_q = p.run_r = p.own_q = 0;
+    p.inv_h = 0;
     p.nbh = (int)(a.B * a.KVH);
     p.tiles_pre = 0;
     p.n_vis = 0;
