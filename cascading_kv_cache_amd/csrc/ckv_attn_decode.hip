@@ -769,6 +769,124 @@ constexpr int kStreamMaxWgs = 1024;  // the result chunks are sized for at most 
 constexpr int kStreamProbWave = 1;  // the wavefront that stores the tile's probabilities (wavefront 0 stores maximum and sum)
 static_assert(kSK / 16 == 8, "a lane's probabilities of a tile are stored as one 16-byte piece");
 
+// What a wavefront of the two streaming kernels keeps of the tile it works on, and the copies of its 16 rows of the
+// tile it copies.  The two are different tiles at the last item of a tile: that item copies the first rows of the
+// next one, as any item copies the next item's, so a run goes from tile to tile without draining its copies.  The
+// positions and masks of the next tile are requested at the first item of a tile and have long arrived by then;
+// what is left between two tiles is their cos and sin.  With the copies drained and a barrier between two tiles,
+// and the positions fetched after it, 65601 keys x 8 kv heads (about 16 items and 3 tiles a workgroup) took 72 us
+// instead of 63.5, x 4 kv heads of 7 query heads each 48.5 instead of 42.8.  Every workgroup has at least one item.
+// (A copy per segment under an exec mask instead of one from lane addresses took 32 KiB of code and spilled scalars:
+// 16 x 8 x 32833 keys 450 us instead of 438.)
+template <typename T>
+struct StreamRows {
+    static constexpr int kEs = (int)sizeof(T);
+    static constexpr int kSteps = kSK / 16;  // contraction steps of 16 keys
+    const DecodeParams& p;
+    const int wave, lane, key16, kq;
+    // the tile that is worked on
+    bool visible = false;          // key key16 of the wavefront's 16
+    uint32_t m01[kSteps], m23[kSteps];  // masks of this lane's P.V operand keys 16 ks + 4 kq .. + 3, two 16-bit values per word:
+                                        // rows of hidden slots may hold anything (their probability is zero, but 0 * NaN is not)
+    RopeWord<T> rw[2][4];          // [ks][word]: dims 32 ks + 8 kq + 2 w, + 1 and their partners 64 further
+    // the requested tile
+    int64_t pos = 0, shift = 0;    // of key key16: position id, and what is added to it
+    int hid = 1, hid64[kSK / 64];  // hidden or not: key key16; keys 64 i + lane
+    float fpos = 0.f;
+    unsigned long long vis64[kSK / 64];
+    // the tile that is copied.  Segments: 0 sink, 1 cache, 2 the new token (rows past the end repeat it and stay hidden)
+    int64_t first = 0;             // its first key of this wavefront
+    bool all_cache = false;        // every one of its rows is a cache slot
+    uint32_t relk[4], relv[4];     // byte offsets inside the (b, kvh) slab of the row's segment
+
+    __device__ __forceinline__ StreamRows(const DecodeParams& p_, int wave_, int lane_)
+        : p(p_), wave(wave_), lane(lane_), key16(lane_ & 15), kq(lane_ >> 4) {}
+    __device__ __forceinline__ int segment_of(int64_t n) const {
+        const int64_t NS = p.a.num_sink;
+        return n < NS ? 0 : n < NS + p.a.S ? 1 : 2;
+    }
+    __device__ __forceinline__ int hidden(int64_t n) const {
+        const ckv_attn_args& a = p.a;
+        const int sg = segment_of(n);
+        return sg == 0 ? (int)a.sink_mask[n] : sg == 1 ? (int)a.mask[n - a.num_sink] : n < p.N ? 0 : 1;
+    }
+    __device__ __forceinline__ void request(int jt) {  // the loads
+        const ckv_attn_args& a = p.a;
+        const int64_t tile = stream_tile_of(p, jt), n = tile * kSK + wave * 16 + key16;
+        const int sg = segment_of(n);
+        pos = sg == 0 ? a.sink_pos[n] : sg == 1 ? a.pos[n - a.num_sink] : n < p.N ? a.q_pos[0] : 0;
+        shift = sg == 1 ? a.pos_shift : 0;
+        hid = hidden(n);
+#pragma unroll
+        for (int i = 0; i < kSK / 64; i++) hid64[i] = hidden(tile * kSK + 64 * i + lane);
+    }
+    __device__ __forceinline__ void arrived() {  // before the next copies: a wait behind them would be one for those too
+        asm volatile("" : "+v"(pos), "+v"(hid));
+        fpos = (float)(pos + shift);
+#pragma unroll
+        for (int i = 0; i < kSK / 64; i++) vis64[i] = __builtin_amdgcn_ballot_w64(hid64[i] == 0);
+    }
+    __device__ __forceinline__ void take(const float* freqs) {  // the requested tile is worked on from here
+        visible = hid == 0;
+#pragma unroll
+        for (int ks = 0; ks < kSteps; ks++) {
+            const uint32_t vk = (uint32_t)(vis64[ks / 4] >> (16 * (ks % 4) + 4 * kq)) & 0xfu;
+            m01[ks] = ((vk & 1u) ? 0x0000ffffu : 0u) | ((vk & 2u) ? 0xffff0000u : 0u);
+            m23[ks] = ((vk & 4u) ? 0x0000ffffu : 0u) | ((vk & 8u) ? 0xffff0000u : 0u);
+        }
+#pragma unroll
+        for (int ks = 0; ks < 2; ks++) {
+            float f[8];
+#pragma unroll
+            for (int e = 0; e < 8; e += 4) {
+                const float4 f4 = *reinterpret_cast<const float4*>(freqs + 32 * ks + 8 * kq + e);
+                f[e] = f4.x; f[e + 1] = f4.y; f[e + 2] = f4.z; f[e + 3] = f4.w;
+            }
+#pragma unroll
+            for (int w = 0; w < 4; w++) rw[ks][w] = rope_word_at<T>(__fmul_rn(fpos, f[2 * w]), __fmul_rn(fpos, f[2 * w + 1]));
+        }
+    }
+    // Block jb of a wavefront brings rows 4 jb .. 4 jb + 3 of its 16 (1 KiB: lane i lands at + 16 i, i.e. row
+    // 4 jb + i / 16, slot i % 16, and fetches the source piece that belongs there).
+    __device__ __forceinline__ void copy_from(int jt) {
+        const ckv_attn_args& a = p.a;
+        first = (int64_t)stream_tile_of(p, jt) * kSK + wave * 16;
+        all_cache = first >= a.num_sink && first + 16 <= a.num_sink + a.S;
+#pragma unroll
+        for (int jb = 0; jb < 4; jb++) {
+            const uint32_t r = 4 * jb + (lane >> 4), piece = (uint32_t)lane & 15u;
+            const int64_t n = first + r;
+            const int sg = segment_of(n);
+            const uint32_t row_off = (uint32_t)((sg == 0 ? n * a.sink_stride[2] : sg == 1 ? (n - a.num_sink) * a.cache_stride[2] : 0) * kEs);
+            relk[jb] = row_off + ((piece ^ (r & 15u)) << 4);
+            relv[jb] = row_off + ((piece ^ ((r & 7u) << 1)) << 4);
+        }
+    }
+    // four copies, whatever the segments (the waits count on that)
+    template <bool kV>
+    __device__ __forceinline__ void copy(int b, int kvh, uint32_t dst) const {
+        const ckv_attn_args& a = p.a;
+        auto slab = [&](int sg) -> const char* {
+            const int64_t* st = sg == 0 ? a.sink_stride : sg == 1 ? a.cache_stride : a.kv_new_stride;
+            const void* base = sg == 0 ? (kV ? a.sink_v : a.sink_k) : sg == 1 ? (kV ? a.cache_v : a.cache_k) : (kV ? a.v_new : a.k_new);
+            return (const char*)base + ((int64_t)b * st[0] + (int64_t)kvh * st[1]) * kEs;
+        };
+        const uint32_t(&rel)[4] = kV ? relv : relk;
+        if (all_cache) {
+            const char* base = slab(1);
+#pragma unroll
+            for (int jb = 0; jb < 4; jb++) async_copy16(base, rel[jb], dst + jb * 1024);
+        } else {  // few tiles: the first, the last and those around the ring's ends
+            const char *sink = slab(0), *cache = slab(1), *token = slab(2);
+#pragma unroll
+            for (int jb = 0; jb < 4; jb++) {
+                const int sg = segment_of(first + 4 * jb + (lane >> 4));
+                async_copy16_from((sg == 0 ? sink : sg == 1 ? cache : token) + rel[jb], dst + jb * 1024);
+            }
+        }
+    }
+};
+
 template <typename T, int G>
 __global__ void __launch_bounds__(kStreamThreads, kStreamWgPerCu) decode_stream_kernel(DecodeParams p) {
     extern __shared__ __align__(16) unsigned char smem[];
@@ -781,7 +899,6 @@ __global__ void __launch_bounds__(kStreamThreads, kStreamWgPerCu) decode_stream_
     constexpr int kKpl = kSK / 16, kDb = kStreamDimBlocks;
     const int nbh = p.nbh;
     const int item0 = stream_first_item(p, (int)blockIdx.x), item1 = stream_first_item(p, (int)blockIdx.x + 1);
-    const int64_t NS = a.num_sink, S = a.S;
     const int KVH = (int)a.KVH;
     constexpr int kEs = (int)sizeof(T);
 
@@ -814,323 +931,239 @@ __global__ void __launch_bounds__(kStreamThreads, kStreamWgPerCu) decode_stream_
     unsigned char* p_wave = smem + kStreamP + wave * (4 * kStreamPPitch);                       // [4][kSK] 16-bit, padded rows
 
     float* freqs = reinterpret_cast<float*>(smem + kStreamFreq);
+    StreamRows<T> rows(p, wave, lane);
+    // the query block of (b, kvh) into stage `st` (one per workgroup, copied by wavefront 0: lane i fills slot
+    // i % 16 of head i / 16 with the piece that belongs there), then this wavefront's K rows.  The query copy
+    // goes first: whoever waits for the four K copies behind it has waited for it too, and the item's barrier
+    // makes it visible to the other wavefronts.
+    auto copy_kq = [&](int b, int kvh, int st) {
+        if (wave == 0 && !p.own_q) {
+            const char* qsrc = (const char*)p.qrot_t + ((int64_t)b * a.H + (int64_t)kvh * G) * (kD * kEs);
+            if ((lane >> 4) < G)
+                async_copy16(qsrc, (lane >> 4) * 256 + (((lane & 15) ^ (lane >> 4)) << 4), lds_base + kStreamQ + st * 1024);
+        }
+        rows.template copy<false>(b, kvh, lds_base + st * kStreamStage + wave * 4096);
+    };
+    // V rows: four copies
+    auto copy_v = [&](int b, int kvh, int st) { rows.template copy<true>(b, kvh, lds_base + st * kStreamStage + kSK * 256 + wave * 4096); };
+
+    // results of the previous item, stored at the top of the next one
+    int pend_item = -1;
+    uint2 pend_o[kDb];  // the tile's weighted V average (sum / l) of this lane's four dims, in the tensor dtype
+    float pend_m = 0.f, pend_l = 0.f;
+    uint4 pend_e = make_uint4(0u, 0u, 0u, 0u);  // the storing wavefront's probabilities: head pg, keys kKpl kgrp ..
+#pragma unroll
+    for (int b2 = 0; b2 < kDb; b2++) pend_o[b2] = make_uint2(0u, 0u);
+    // Stores share the counter of the copies and retire in order with them.  All stores of an item are
+    // issued together, right after the copies of the next item's K rows; every wavefront issues kDb
+    // of them (two wavefronts one more each), and none before the first item of a run has results.
+    auto flush = [&]() {
+        if (pend_item < 0) return;
+        const int64_t chunk_i = (int64_t)(pend_item - item0) * gridDim.x + blockIdx.x;
+        unsigned char* chunk = p.chunks + chunk_i * (G * (kSK + kD) * 2);
+        if (wave == kStreamProbWave && pg < G)  // every wavefront holds all of them: one stores, 16 bytes a lane
+            *reinterpret_cast<uint4*>(chunk + (pg * kSK + kKpl * kgrp) * 2) = pend_e;
+        if (key16 < G) {
+#pragma unroll
+            for (int b2 = 0; b2 < kDb; b2++)
+                *reinterpret_cast<uint2*>(chunk + (G * kSK + key16 * kD + 16 * (kDb * wave + b2) + 4 * kq) * 2) = pend_o[b2];
+        }
+        if (wave == 0 && kgrp == 0 && pg < G)  // maximum and sum: G pairs per chunk, in chunk order
+            *reinterpret_cast<float2*>(p.part_ml + (chunk_i * G + pg) * 2) = make_float2(pend_m, pend_l);
+    };
+    auto wait_copies = [&](int younger, bool lds_too) {  // vmcnt(younger) [, lgkmcnt(0)]: the count is an immediate
+        if (lds_too) {
+            switch (younger) {
+                case 4: __builtin_amdgcn_s_waitcnt(0x0074); break;
+                case 5: __builtin_amdgcn_s_waitcnt(0x0075); break;
+                case 6: __builtin_amdgcn_s_waitcnt(0x0076); break;
+                case 7: __builtin_amdgcn_s_waitcnt(0x0077); break;
+                case 8: __builtin_amdgcn_s_waitcnt(0x0078); break;
+                default: __builtin_amdgcn_s_waitcnt(0x0070); break;
+            }
+        } else {
+            switch (younger) {
+                case 4: __builtin_amdgcn_s_waitcnt(0x0F74); break;
+                case 5: __builtin_amdgcn_s_waitcnt(0x0F75); break;
+                case 6: __builtin_amdgcn_s_waitcnt(0x0F76); break;
+                case 7: __builtin_amdgcn_s_waitcnt(0x0F77); break;
+                default: __builtin_amdgcn_s_waitcnt(0x0F70); break;
+            }
+        }
+    };
+    static_assert(kDb <= 2, "wait_copies covers up to kDb + 2 stores");
+
+    // ---- start: what the first item needs is requested in one go, then its rows, and the rest is worked out while they travel
+    int jt = (int)((uint32_t)item0 / (uint32_t)nbh);  // the tile's rank among the visible ones
+    int b, kvh;
+    {
+        const int bh = item0 - jt * nbh;
+        b = (int)((uint32_t)bh / (uint32_t)KVH);
+        kvh = bh - b * KVH;
+    }
     SharedQueries<T, G> shared;
     shared.request(p, tid, wave);
-    bool first_tile = true;
-    int jt = (int)((uint32_t)item0 / (uint32_t)nbh), bh0 = item0 - jt * nbh;  // jt: the tile's rank among the visible ones
-    for (int item = item0; item < item1; jt++, bh0 = 0) {
-        const int64_t tile = stream_tile_of(p, jt);
-        const int bh1 = (jt + 1) * nbh > item1 ? item1 - jt * nbh : nbh;
-        item = jt * nbh + bh1;
-        const int64_t n_wave = tile * kSK + wave * 16;  // first key of this wavefront
-
-        // ---- per-tile constants (the same for every (b, kvh): positions are shared)
-        bool vis1 = false;
-        int64_t pos = 0;
-        {
-            const int64_t n = n_wave + key16;
-            if (n < NS) { vis1 = a.sink_mask[n] == 0; pos = a.sink_pos[n]; }
-            else if (n < NS + S) { vis1 = a.mask[n - NS] == 0; pos = a.pos[n - NS] + a.pos_shift; }
-            else if (n < p.N) { vis1 = true; pos = a.q_pos[0]; }
+    rows.request(jt);
+    rows.copy_from(jt);
+    rows.arrived();
+    shared.arrived();
+    copy_kq(b, kvh, 0);
+    copy_v(b, kvh, 0);
+    shared.finish(p, freqs, smem + kStreamOwnQ, tid, wave);
+    rows.take(freqs);
+    bool request = (jt + 1) * nbh < item1;
+    // Loads and stores retire in issue order, so "at most n operations outstanding" with n younger ones issued after the
+    // wanted copies means the wanted ones are done (and more younger ones than counted only wait for more).  Per item
+    // the order is [wavefront 0: the query block of the next item,] K rows of the next item (4), stores of the previous
+    // one (kDb and up, once there is one), V rows of the next item (4).
+    // The first query block of the run must have landed for every wavefront (younger: the four V copies).
+    __builtin_amdgcn_s_waitcnt(0x0F74);
+    __builtin_amdgcn_s_barrier();
+    int st = 0;
+    // stores this wavefront issued in the latest flush(): kDb partial averages, the probabilities
+    // from one wavefront, maximum and sum from another
+    const int my_stores = kDb + (wave == kStreamProbWave ? 1 : 0) + (wave == 0 ? 1 : 0);
+    int stored = 0;
+    for (int item = item0; item < item1; item++) {
+        const bool more = item + 1 < item1, next_tile = more && item + 1 == (jt + 1) * nbh;
+        // this wavefront's K rows of the item are in LDS (younger: the stores issued after them and the four V
+        // copies of this item); the item's query block was complete before the previous barrier
+        wait_copies(4 + stored, false);
+        int b_nx = b, kvh_nx = kvh + 1;
+        if (kvh_nx == KVH) { kvh_nx = 0; b_nx = b + 1; }
+        if (request) {
+            rows.request(jt + 1);
+            request = false;
         }
-        float fpos = (float)pos;
-        // Rows of hidden slots may hold anything (their probability is zero, but 0 * NaN is not), so
-        // they are zeroed on the way into the P.V product: masks of this lane's operand keys
-        // 16 ks + 4 kq .. + 3, two 16-bit values per word.
-        uint32_t m01[kKpl], m23[kKpl];
-#pragma unroll
-        for (int half = 0; half < kSK / 64; half++) {
-            const int64_t n = tile * kSK + 64 * half + lane;
-            bool v = false;
-            if (n < NS) v = a.sink_mask[n] == 0;
-            else if (n < NS + S) v = a.mask[n - NS] == 0;
-            else if (n < p.N) v = true;
-            const unsigned long long vis64 = __builtin_amdgcn_ballot_w64(v);
-#pragma unroll
-            for (int k4 = 0; k4 < 4; k4++) {
-                const int ks = 4 * half + k4;
-                const uint32_t vk = (uint32_t)(vis64 >> (16 * k4 + 4 * kq)) & 0xfu;
-                m01[ks] = ((vk & 1u) ? 0x0000ffffu : 0u) | ((vk & 2u) ? 0xffff0000u : 0u);
-                m23[ks] = ((vk & 4u) ? 0x0000ffffu : 0u) | ((vk & 8u) ? 0xffff0000u : 0u);
-            }
+        if (next_tile) {
+            rows.arrived();
+            rows.copy_from(jt + 1);
+            b_nx = 0;
         }
-        // Copies: block jb of a wavefront brings rows 4 jb .. 4 jb + 3 of its 16 (1 KiB: lane i lands at
-        // +16 i, i.e. row 4 jb + i / 16, slot i % 16, and fetches the source piece that belongs there).
-        // seg: 0 sink, 1 cache, 2 the new token (rows past the end repeat it and stay hidden).
-        int seg_c[4];
-        uint32_t relk[4], relv[4];  // byte offsets inside the (b, kvh) slab of the row's segment
-        bool cache_only[4];         // every row of the block is a cache slot: one copy with the slab as base
-#pragma unroll
-        for (int jb = 0; jb < 4; jb++) {
-            const int r = 4 * jb + (lane >> 4);
-            const int64_t n = n_wave + r;
-            int64_t row_off;
-            if (n < NS) { seg_c[jb] = 0; row_off = n * a.sink_stride[2]; }
-            else if (n < NS + S) { seg_c[jb] = 1; row_off = (n - NS) * a.cache_stride[2]; }
-            else { seg_c[jb] = 2; row_off = 0; }
-            relk[jb] = (uint32_t)(row_off * kEs) + ((((uint32_t)lane & 15u) ^ ((uint32_t)r & 15u)) << 4);
-            relv[jb] = (uint32_t)(row_off * kEs) + ((((uint32_t)lane & 15u) ^ (((uint32_t)r & 7u) << 1)) << 4);
-            cache_only[jb] = __builtin_amdgcn_ballot_w64(seg_c[jb] == 1) == ~0ull;
-        }
-        // the loads above have come back: a wait for them behind the copies would be one for those
-        asm volatile("" : "+v"(fpos));
-        if (first_tile) shared.arrived();
-        // slab pointers of (b, kvh)
-        auto slabs = [&](int b, int kvh, const char* (&kb)[3], const char* (&vb)[3]) {
-            const int64_t o0 = ((int64_t)b * a.sink_stride[0] + (int64_t)kvh * a.sink_stride[1]) * kEs;
-            const int64_t o1 = ((int64_t)b * a.cache_stride[0] + (int64_t)kvh * a.cache_stride[1]) * kEs;
-            const int64_t o2 = ((int64_t)b * a.kv_new_stride[0] + (int64_t)kvh * a.kv_new_stride[1]) * kEs;
-            kb[0] = (const char*)a.sink_k + o0; vb[0] = (const char*)a.sink_v + o0;
-            kb[1] = (const char*)a.cache_k + o1; vb[1] = (const char*)a.cache_v + o1;
-            kb[2] = (const char*)a.k_new + o2; vb[2] = (const char*)a.v_new + o2;
-        };
-        // four copies, at least one per block whatever the segments (the waits below count on that)
-        auto copy_rows = [&](const char* (&base)[3], const uint32_t(&rel)[4], uint32_t dst) {
-#pragma unroll
-            for (int jb = 0; jb < 4; jb++) {
-                if (cache_only[jb]) {
-                    async_copy16(base[1], rel[jb], dst + jb * 1024);
-                } else {
-#pragma unroll
-                    for (int sgm = 0; sgm < 3; sgm++)
-                        if (seg_c[jb] == sgm) async_copy16(base[sgm], rel[jb], dst + jb * 1024);
-                }
-            }
-        };
-        // the query block of (b, kvh) into stage `st` (one per workgroup, copied by wavefront 0: lane i fills slot
-        // i % 16 of head i / 16 with the piece that belongs there), then this wavefront's K rows.  The query copy
-        // goes first: whoever waits for the four K copies behind it has waited for it too, and the item's barrier
-        // makes it visible to the other wavefronts.
-        auto copy_kq = [&](int b, int kvh, int st) {
-            if (wave == 0 && !p.own_q) {
-                const char* qsrc = (const char*)p.qrot_t + ((int64_t)b * a.H + (int64_t)kvh * G) * (kD * kEs);
-                if ((lane >> 4) < G)
-                    async_copy16(qsrc, (lane >> 4) * 256 + (((lane & 15) ^ (lane >> 4)) << 4), lds_base + kStreamQ + st * 1024);
-            }
-            const char *kb[3], *vb[3];
-            slabs(b, kvh, kb, vb);
-            copy_rows(kb, relk, lds_base + st * kStreamStage + wave * 4096);
-        };
-        // V rows: four copies
-        auto copy_v = [&](int b, int kvh, int st) {
-            const char *kb[3], *vb[3];
-            slabs(b, kvh, kb, vb);
-            copy_rows(vb, relv, lds_base + st * kStreamStage + kSK * 256 + wave * 4096);
-        };
-
-        int b = (int)((uint32_t)bh0 / (uint32_t)KVH), kvh = bh0 - b * KVH;
-        // results of the previous item, stored at the top of the next one
-        bool pending = false;
-        int pend_b = 0, pend_kvh = 0;
-        uint2 pend_o[kDb];  // the tile's weighted V average (sum / l) of this lane's four dims, in the tensor dtype
-        float pend_m = 0.f, pend_l = 0.f;
-        uint4 pend_e = make_uint4(0u, 0u, 0u, 0u);  // the storing wavefront's probabilities: head pg, keys kKpl kgrp ..
-#pragma unroll
-        for (int b2 = 0; b2 < kDb; b2++) pend_o[b2] = make_uint2(0u, 0u);
-        // Stores share the counter of the copies and retire in order with them.  All stores of an item are
-        // issued together, right after the copies of the next item's K rows; every wavefront issues kDb
-        // of them (two wavefronts one more each), and none before the first item of a run has results.
-        auto flush = [&]() {
-            if (!pending) return;
-            const int pend_item = jt * nbh + pend_b * KVH + pend_kvh;
-            const int64_t chunk_i = (int64_t)(pend_item - item0) * gridDim.x + blockIdx.x;
-            unsigned char* chunk = p.chunks + chunk_i * (G * (kSK + kD) * 2);
-            if (wave == kStreamProbWave && pg < G)  // every wavefront holds all of them: one stores, 16 bytes a lane
-                *reinterpret_cast<uint4*>(chunk + (pg * kSK + kKpl * kgrp) * 2) = pend_e;
-            if (key16 < G) {
-#pragma unroll
-                for (int b2 = 0; b2 < kDb; b2++)
-                    *reinterpret_cast<uint2*>(chunk + (G * kSK + key16 * kD + 16 * (kDb * wave + b2) + 4 * kq) * 2) = pend_o[b2];
-            }
-            if (wave == 0 && kgrp == 0 && pg < G)  // maximum and sum: G pairs per chunk, in chunk order
-                *reinterpret_cast<float2*>(p.part_ml + (chunk_i * G + pg) * 2) = make_float2(pend_m, pend_l);
-        };
-
-        // Loads and stores retire in issue order, so "at most n operations outstanding" with n younger
-        // ones issued after the wanted copies means the wanted ones are done.  Per item the order is
-        // [wavefront 0: the query block of the next item,] K rows of the next item (4), stores of the previous
-        // one (kDb and up, once there is one), V rows of the next item (4).
-        copy_kq(b, kvh, 0);
-        copy_v(b, kvh, 0);
-        if (first_tile) shared.finish(p, freqs, smem + kStreamOwnQ, tid, wave);
-        first_tile = false;
-        // cos and sin while the first rows are on their way
-        RopeWord<T> rw[2][4];  // [ks][word]: dims 32 ks + 8 kq + 2 w, + 1 and their partners 64 further
-#pragma unroll
-        for (int ks = 0; ks < 2; ks++) {
-            float f[8];
-#pragma unroll
-            for (int e = 0; e < 8; e += 4) {
-                const float4 f4 = *reinterpret_cast<const float4*>(freqs + 32 * ks + 8 * kq + e);
-                f[e] = f4.x; f[e + 1] = f4.y; f[e + 2] = f4.z; f[e + 3] = f4.w;
-            }
-#pragma unroll
-            for (int w = 0; w < 4; w++) rw[ks][w] = rope_word_at<T>(__fmul_rn(fpos, f[2 * w]), __fmul_rn(fpos, f[2 * w + 1]));
-        }
-        // the first query block of the run must have landed for every wavefront (younger: the four V copies)
-        __builtin_amdgcn_s_waitcnt(0x0F74);
-        __builtin_amdgcn_s_barrier();
-        int st = 0;
-        // stores this wavefront issued in the latest flush(): kDb partial averages, the probabilities
-        // from one wavefront, maximum and sum from another
-        const int my_stores = kDb + (wave == kStreamProbWave ? 1 : 0) + (wave == 0 ? 1 : 0);
-        int stored = 0;
-        auto wait_copies = [&](int younger, bool lds_too) {  // vmcnt(younger) [, lgkmcnt(0)]: the count is an immediate
-            if (lds_too) {
-                switch (younger) {
-                    case 4: __builtin_amdgcn_s_waitcnt(0x0074); break;
-                    case 5: __builtin_amdgcn_s_waitcnt(0x0075); break;
-                    case 6: __builtin_amdgcn_s_waitcnt(0x0076); break;
-                    case 7: __builtin_amdgcn_s_waitcnt(0x0077); break;
-                    case 8: __builtin_amdgcn_s_waitcnt(0x0078); break;
-                    default: __builtin_amdgcn_s_waitcnt(0x0070); break;
-                }
-            } else {
-                switch (younger) {
-                    case 4: __builtin_amdgcn_s_waitcnt(0x0F74); break;
-                    case 5: __builtin_amdgcn_s_waitcnt(0x0F75); break;
-                    case 6: __builtin_amdgcn_s_waitcnt(0x0F76); break;
-                    case 7: __builtin_amdgcn_s_waitcnt(0x0F77); break;
-                    default: __builtin_amdgcn_s_waitcnt(0x0F70); break;
-                }
-            }
-        };
-        static_assert(kDb <= 2, "wait_copies covers up to kDb + 2 stores");
-        for (int bh = bh0; bh < bh1; bh++) {
-            int b_nx = b, kvh_nx = kvh;
-            if (bh + 1 < bh1) {  // the last item of a run copies itself again: cheaper than a different path
-                kvh_nx = kvh + 1 == KVH ? 0 : kvh + 1;
-                b_nx = kvh + 1 == KVH ? b + 1 : b;
-            }
-            // this wavefront's K rows of the item are in LDS (younger: the stores issued after them and the four V
-            // copies of this item); the item's query block was complete before the previous barrier
-            wait_copies(4 + stored, false);
-            copy_kq(b_nx, kvh_nx, st ^ 1);
-            stored = pending ? my_stores : 0;
-            flush();
-            const unsigned char* stage = smem + st * kStreamStage;
-            const int q_at = p.own_q ? kStreamOwnQ + (b * KVH + kvh) * (G * 256) : kStreamQ + st * 1024;
-
-            // ---- rotate K in registers, logits by MFMA, shared through LDS
-            {
-                uint4 kraw[4], qop[4];
-#pragma unroll
-                for (int ks = 0; ks < 4; ks++) kraw[ks] = *reinterpret_cast<const uint4*>(stage + kaddr[ks]);
-#pragma unroll
-                for (int ks = 0; ks < 4; ks++) qop[ks] = *reinterpret_cast<const uint4*>(smem + q_at + q_off + ks * 64);
-                uint4 kop[4];
-#pragma unroll
-                for (int ks = 0; ks < 2; ks++) {
-                    const uint32_t* w1 = reinterpret_cast<const uint32_t*>(&kraw[ks]);
-                    const uint32_t* w2 = reinterpret_cast<const uint32_t*>(&kraw[ks + 2]);
-                    uint32_t o1[4], o2[4];
-#pragma unroll
-                    for (int w = 0; w < 4; w++) {
-                        rw[ks][w].rotate(w1[w], w2[w], p.key_scale, true, o1[w], o2[w]);
-                    }
-                    kop[ks] = make_uint4(o1[0], o1[1], o1[2], o1[3]);
-                    kop[ks + 2] = make_uint4(o2[0], o2[1], o2[2], o2[3]);
-                }
-                f32x4 sacc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int ks = 0; ks < 4; ks++) sacc = Mma16<T>::mma(qop[ks], kop[ks], sacc);
-                // lane holds heads 4 kq + v of key key16: with G <= 4 only the lanes of kq == 0 hold heads
-                if (kq == 0) {
-#pragma unroll
-                    for (int v = 0; v < G; v++)
-                        s_all[(st * 4 + v) * kSK + wave * 16 + key16] = vis1 ? sacc[v] * p.scale_log2 : -INFINITY;
-                }
-            }
-            // this wavefront's V rows of the item and (wavefront 0) the next query block have landed (younger: the
-            // four K copies of the next item and the stores of flush()); its logits are in LDS
-            wait_copies(4 + stored, true);
-            __builtin_amdgcn_s_barrier();
-            // every wavefront is past the previous item: its V stage can be refilled
-            copy_v(b_nx, kvh_nx, st ^ 1);
-
-            // ---- softmax over the tile's keys, done by every wavefront: lane = (head, kKpl keys)
-            float m_t, l_t;
-            uint4 e_half = make_uint4(0u, 0u, 0u, 0u);
-            {
-                float x[kKpl];
-#pragma unroll
-                for (int e = 0; e < kKpl; e += 4) {
-                    float4 x4 = make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
-                    if (pg < G) x4 = *reinterpret_cast<const float4*>(s_all + (st * 4 + pg) * kSK + kKpl * kgrp + e);
-                    x[e] = x4.x; x[e + 1] = x4.y; x[e + 2] = x4.z; x[e + 3] = x4.w;
-                }
-                float mloc = x[0];
-#pragma unroll
-                for (int e = 1; e < kKpl; e++) mloc = fmaxf(mloc, x[e]);
-                const float m = mod4_max(mloc);
-                const float ms = m == -INFINITY ? 0.f : m;
-                float lloc = 0.f;
-#pragma unroll
-                for (int e = 0; e < kKpl; e += 4) {
-                    const float e0 = __builtin_amdgcn_exp2f(x[e] - ms), e1 = __builtin_amdgcn_exp2f(x[e + 1] - ms);
-                    const float e2 = __builtin_amdgcn_exp2f(x[e + 2] - ms), e3 = __builtin_amdgcn_exp2f(x[e + 3] - ms);
-                    lloc += (e0 + e1) + (e2 + e3);
-                    // probabilities in the tensor dtype, [head][kSK keys] (hidden keys and idle lanes: 0)
-                    const uint2 pk = make_uint2(Mma16<T>::pack2(e0, e1), Mma16<T>::pack2(e2, e3));
-                    *reinterpret_cast<uint2*>(p_wave + pg * kStreamPPitch + (kKpl * kgrp + e) * 2) = pk;
-                    // the copy that goes to memory for the score kernel is fp16 whatever the tensor dtype
-                    uint2 hk = pk;
-                    if constexpr (!std::is_same<T, __half>::value) {
-                        if (wave == kStreamProbWave) hk = make_uint2(Mma16<__half>::pack2(e0, e1), Mma16<__half>::pack2(e2, e3));
-                    }
-                    if (e == 0) { e_half.x = hk.x; e_half.y = hk.y; } else { e_half.z = hk.x; e_half.w = hk.y; }
-                }
-                m_t = m;
-                l_t = mod4_sum(lloc);
-            }
-            __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
-            __builtin_amdgcn_wave_barrier();
-            // ---- weighted V sum on the matrix pipe: this wavefront's dims over all keys of the tile.  Lane
-            //      16 q + g (g < G) ends up with dims 16 (kDb wave + b2) + 4 q .. + 3 of head g.
-            f32x4 acc[kDb];
-#pragma unroll
-            for (int b2 = 0; b2 < kDb; b2++) acc[b2] = f32x4{0.f, 0.f, 0.f, 0.f};
-            {
-                const uint32_t vbase = lds_base + st * kStreamStage;
-#pragma unroll
-                for (int ks = 0; ks < kKpl; ks++) {
-                    uint2 pb = make_uint2(0u, 0u);
-                    if (key16 < G) pb = *reinterpret_cast<const uint2*>(p_wave + key16 * kStreamPPitch + ks * 32 + kq * 8);
-#pragma unroll
-                    for (int b2 = 0; b2 < kDb; b2++) {
-                        const s16x4_t va = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                            (__attribute__((address_space(3))) s16x4_t*)(uintptr_t)(vbase + vt_addr[b2] + ks * 4096));
-                        uint2 av = __builtin_bit_cast(uint2, va);
-                        av.x &= m01[ks];
-                        av.y &= m23[ks];
-                        acc[b2] = Mma16<T>::mma_k16(av, pb, acc[b2]);
-                    }
-                }
-            }
-            {
-                // lanes 16 q + g hold head g, and g == pg there: l_t is that head's sum (0: the tile is hidden)
-                const float inv_l = l_t > 0.f ? 1.0f / l_t : 0.f;
-#pragma unroll
-                for (int b2 = 0; b2 < kDb; b2++)
-                    pend_o[b2] = make_uint2(Mma16<T>::pack2(acc[b2][0] * inv_l, acc[b2][1] * inv_l),
-                                            Mma16<T>::pack2(acc[b2][2] * inv_l, acc[b2][3] * inv_l));
-            }
-            pend_m = m_t;
-            pend_l = l_t;
-            pend_e = e_half;
-            pending = true;
-            pend_b = b;
-            pend_kvh = kvh;
-            b = b_nx;
-            kvh = kvh_nx;
-            st ^= 1;
-        }
+        if (more) copy_kq(b_nx, kvh_nx, st ^ 1);
+        stored = pend_item >= 0 ? my_stores : 0;
         flush();
-        // the repeated copies of the last item must land, and every wavefront be done with the stages,
-        // before the next run of items refills them
-        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+        const unsigned char* stage = smem + st * kStreamStage;
+        const int q_at = p.own_q ? kStreamOwnQ + (b * KVH + kvh) * (G * 256) : kStreamQ + st * 1024;
+
+        // ---- rotate K in registers, logits by MFMA, shared through LDS
+        {
+            uint4 kraw[4], qop[4];
+#pragma unroll
+            for (int ks = 0; ks < 4; ks++) kraw[ks] = *reinterpret_cast<const uint4*>(stage + kaddr[ks]);
+#pragma unroll
+            for (int ks = 0; ks < 4; ks++) qop[ks] = *reinterpret_cast<const uint4*>(smem + q_at + q_off + ks * 64);
+            uint4 kop[4];
+#pragma unroll
+            for (int ks = 0; ks < 2; ks++) {
+                const uint32_t* w1 = reinterpret_cast<const uint32_t*>(&kraw[ks]);
+                const uint32_t* w2 = reinterpret_cast<const uint32_t*>(&kraw[ks + 2]);
+                uint32_t o1[4], o2[4];
+#pragma unroll
+                for (int w = 0; w < 4; w++) {
+                    rows.rw[ks][w].rotate(w1[w], w2[w], p.key_scale, true, o1[w], o2[w]);
+                }
+                kop[ks] = make_uint4(o1[0], o1[1], o1[2], o1[3]);
+                kop[ks + 2] = make_uint4(o2[0], o2[1], o2[2], o2[3]);
+            }
+            f32x4 sacc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int ks = 0; ks < 4; ks++) sacc = Mma16<T>::mma(qop[ks], kop[ks], sacc);
+            // lane holds heads 4 kq + v of key key16: with G <= 4 only the lanes of kq == 0 hold heads
+            if (kq == 0) {
+#pragma unroll
+                for (int v = 0; v < G; v++)
+                    s_all[(st * 4 + v) * kSK + wave * 16 + key16] = rows.visible ? sacc[v] * p.scale_log2 : -INFINITY;
+            }
+        }
+        // this wavefront's V rows of the item and (wavefront 0) the next query block have landed (younger: the
+        // four K copies of the next item and the stores of flush()); its logits are in LDS
+        wait_copies(more ? 4 + stored : 0, true);
         __builtin_amdgcn_s_barrier();
+        // every wavefront is past the previous item: its V stage can be refilled
+        if (more) copy_v(b_nx, kvh_nx, st ^ 1);
+
+        // ---- softmax over the tile's keys, done by every wavefront: lane = (head, kKpl keys)
+        float m_t, l_t;
+        uint4 e_half = make_uint4(0u, 0u, 0u, 0u);
+        {
+            float x[kKpl];
+#pragma unroll
+            for (int e = 0; e < kKpl; e += 4) {
+                float4 x4 = make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
+                if (pg < G) x4 = *reinterpret_cast<const float4*>(s_all + (st * 4 + pg) * kSK + kKpl * kgrp + e);
+                x[e] = x4.x; x[e + 1] = x4.y; x[e + 2] = x4.z; x[e + 3] = x4.w;
+            }
+            float mloc = x[0];
+#pragma unroll
+            for (int e = 1; e < kKpl; e++) mloc = fmaxf(mloc, x[e]);
+            const float m = mod4_max(mloc);
+            const float ms = m == -INFINITY ? 0.f : m;
+            float lloc = 0.f;
+#pragma unroll
+            for (int e = 0; e < kKpl; e += 4) {
+                const float e0 = __builtin_amdgcn_exp2f(x[e] - ms), e1 = __builtin_amdgcn_exp2f(x[e + 1] - ms);
+                const float e2 = __builtin_amdgcn_exp2f(x[e + 2] - ms), e3 = __builtin_amdgcn_exp2f(x[e + 3] - ms);
+                lloc += (e0 + e1) + (e2 + e3);
+                // probabilities in the tensor dtype, [head][kSK keys] (hidden keys and idle lanes: 0)
+                const uint2 pk = make_uint2(Mma16<T>::pack2(e0, e1), Mma16<T>::pack2(e2, e3));
+                *reinterpret_cast<uint2*>(p_wave + pg * kStreamPPitch + (kKpl * kgrp + e) * 2) = pk;
+                // the copy that goes to memory for the score kernel is fp16 whatever the tensor dtype
+                uint2 hk = pk;
+                if constexpr (!std::is_same<T, __half>::value) {
+                    if (wave == kStreamProbWave) hk = make_uint2(Mma16<__half>::pack2(e0, e1), Mma16<__half>::pack2(e2, e3));
+                }
+                if (e == 0) { e_half.x = hk.x; e_half.y = hk.y; } else { e_half.z = hk.x; e_half.w = hk.y; }
+            }
+            m_t = m;
+            l_t = mod4_sum(lloc);
+        }
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+        __builtin_amdgcn_wave_barrier();
+        // ---- weighted V sum on the matrix pipe: this wavefront's dims over all keys of the tile.  Lane
+        //      16 q + g (g < G) ends up with dims 16 (kDb wave + b2) + 4 q .. + 3 of head g.
+        f32x4 acc[kDb];
+#pragma unroll
+        for (int b2 = 0; b2 < kDb; b2++) acc[b2] = f32x4{0.f, 0.f, 0.f, 0.f};
+        {
+            const uint32_t vbase = lds_base + st * kStreamStage;
+#pragma unroll
+            for (int ks = 0; ks < kKpl; ks++) {
+                uint2 pb = make_uint2(0u, 0u);
+                if (key16 < G) pb = *reinterpret_cast<const uint2*>(p_wave + key16 * kStreamPPitch + ks * 32 + kq * 8);
+#pragma unroll
+                for (int b2 = 0; b2 < kDb; b2++) {
+                    const s16x4_t va = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                        (__attribute__((address_space(3))) s16x4_t*)(uintptr_t)(vbase + vt_addr[b2] + ks * 4096));
+                    uint2 av = __builtin_bit_cast(uint2, va);
+                    av.x &= rows.m01[ks];
+                    av.y &= rows.m23[ks];
+                    acc[b2] = Mma16<T>::mma_k16(av, pb, acc[b2]);
+                }
+            }
+        }
+        {
+            // lanes 16 q + g hold head g, and g == pg there: l_t is that head's sum (0: the tile is hidden)
+            const float inv_l = l_t > 0.f ? 1.0f / l_t : 0.f;
+#pragma unroll
+            for (int b2 = 0; b2 < kDb; b2++)
+                pend_o[b2] = make_uint2(Mma16<T>::pack2(acc[b2][0] * inv_l, acc[b2][1] * inv_l),
+                                        Mma16<T>::pack2(acc[b2][2] * inv_l, acc[b2][3] * inv_l));
+        }
+        pend_m = m_t;
+        pend_l = l_t;
+        pend_e = e_half;
+        pend_item = item;
+        b = b_nx;
+        kvh = kvh_nx;
+        st ^= 1;
+        if (next_tile) {
+            jt++;
+            rows.take(freqs);
+            request = (jt + 1) * nbh < item1;
+        }
     }
+    flush();
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1181,7 +1214,6 @@ __global__ void __launch_bounds__(kStreamThreads, kStreamWgPerCu) decode_stream_
     constexpr int kPv = kSK / 16, kDb = kStreamDimBlocks;   // contraction steps of 16 keys
     const int nbh = p.nbh;
     const int item0 = stream_first_item(p, (int)blockIdx.x), item1 = stream_first_item(p, (int)blockIdx.x + 1);
-    const int64_t NS = a.num_sink, S = a.S;
     const int KVH = (int)a.KVH;
     constexpr int kEs = (int)sizeof(T);
 
@@ -1206,279 +1238,201 @@ __global__ void __launch_bounds__(kStreamThreads, kStreamWgPerCu) decode_stream_
     const bool head_ok = key16 < G;
 
     float* freqs = reinterpret_cast<float*>(smem + kWideFreq);
+    StreamRows<T> rows(p, wave, lane);
+    // the query block of (b, kvh) into stage `st` (wavefronts 0 and 1, four heads each: lane i fills slot
+    // i % 16 of head 4 wave + i / 16 with the piece that belongs there), then this wavefront's K rows.  The
+    // query copy goes first: whoever waits for the four K copies behind it has waited for it too.
+    auto copy_kq = [&](int b, int kvh, int st) {
+        if (wave < 2 && !p.own_q) {
+            const char* qsrc = (const char*)p.qrot_t + ((int64_t)b * a.H + (int64_t)kvh * G) * (kD * kEs);
+            const int h = 4 * wave + (lane >> 4);
+            if (h < G) async_copy16(qsrc, h * 256 + (((lane & 15) ^ h) << 4), lds_base + kWideQ + st * 2048 + wave * 1024);
+        }
+        rows.template copy<false>(b, kvh, lds_base + st * kStreamStage + wave * 4096);
+    };
+    auto copy_v = [&](int b, int kvh, int st) { rows.template copy<true>(b, kvh, lds_base + st * kStreamStage + kSK * 256 + wave * 4096); };
+
+    // results of the previous item, stored at the top of the next one
+    int pend_item = -1;
+    uint2 pend_o[kDb];
+    float pend_m = 0.f, pend_l = 0.f;
+    uint2 pend_e = make_uint2(0u, 0u);  // fp16 probabilities of head key16, keys 16 wave + 4 kq .. + 3
+#pragma unroll
+    for (int b2 = 0; b2 < kDb; b2++) pend_o[b2] = make_uint2(0u, 0u);
+    auto flush = [&]() {
+        if (pend_item < 0) return;
+        const int64_t chunk_i = (int64_t)(pend_item - item0) * gridDim.x + blockIdx.x;
+        unsigned char* chunk = p.chunks + chunk_i * (G * (kSK + kD) * 2);
+        if (head_ok) {
+            *reinterpret_cast<uint2*>(chunk + (key16 * kSK + 16 * wave + 4 * kq) * 2) = pend_e;
+#pragma unroll
+            for (int b2 = 0; b2 < kDb; b2++)
+                *reinterpret_cast<uint2*>(chunk + (G * kSK + key16 * kD + 16 * (kDb * wave + b2) + 4 * kq) * 2) = pend_o[b2];
+        }
+        if (wave == 0 && kq == 0 && head_ok)  // maximum and sum: G pairs per chunk, in chunk order
+            *reinterpret_cast<float2*>(p.part_ml + (chunk_i * G + key16) * 2) = make_float2(pend_m, pend_l);
+    };
+    // ---- start, as in the kernel above
+    int jt = (int)((uint32_t)item0 / (uint32_t)nbh);  // the tile's rank among those with items
+    int b, kvh;
+    {
+        const int bh = item0 - jt * nbh;
+        b = (int)((uint32_t)bh / (uint32_t)KVH);
+        kvh = bh - b * KVH;
+    }
     SharedQueries<T, G> shared;
     shared.request(p, tid, wave);
-    bool first_tile = true;
-    int jt = (int)((uint32_t)item0 / (uint32_t)nbh), bh0 = item0 - jt * nbh;  // jt: the tile's rank among those with items
-    for (int item = item0; item < item1; jt++, bh0 = 0) {
-        const int64_t tile = stream_tile_of(p, jt);
-        const int bh1 = (jt + 1) * nbh > item1 ? item1 - jt * nbh : nbh;
-        item = jt * nbh + bh1;
-        const int64_t n_wave = tile * kSK + wave * 16;  // first key of this wavefront
-
-        // ---- per-tile constants (the same for every (b, kvh): positions are shared)
-        bool vis1 = false;
-        int64_t pos = 0;
-        {
-            const int64_t n = n_wave + key16;
-            if (n < NS) { vis1 = a.sink_mask[n] == 0; pos = a.sink_pos[n]; }
-            else if (n < NS + S) { vis1 = a.mask[n - NS] == 0; pos = a.pos[n - NS] + a.pos_shift; }
-            else if (n < p.N) { vis1 = true; pos = a.q_pos[0]; }
+    rows.request(jt);
+    rows.copy_from(jt);
+    rows.arrived();
+    shared.arrived();
+    copy_kq(b, kvh, 0);
+    copy_v(b, kvh, 0);
+    shared.finish(p, freqs, smem + kWideOwnQ, tid, wave);
+    rows.take(freqs);
+    bool request = (jt + 1) * nbh < item1;
+    // Per item a wavefront issues, in this order: [the query copy of the next item,] four K copies of the
+    // next item, the stores of the previous item's results, and after the barrier four V copies of the next
+    // item.  Loads and stores retire in issue order.
+    const int my_stores = kDb + 1 + (wave == 0 ? 1 : 0);
+    int stored = 0;
+    // the first query block of the run must have landed for every wavefront (younger: the four V copies)
+    __builtin_amdgcn_s_waitcnt(0x0F74);
+    __builtin_amdgcn_s_barrier();
+    int st = 0;
+    for (int item = item0; item < item1; item++) {
+        const bool more = item + 1 < item1, next_tile = more && item + 1 == (jt + 1) * nbh;
+        // this wavefront's K rows of the item are in LDS (younger: the stores issued after them and the four V
+        // copies of this item); its query block was complete before the previous barrier
+        wait_vm(4 + stored, false);
+        int b_nx = b, kvh_nx = kvh + 1;
+        if (kvh_nx == KVH) { kvh_nx = 0; b_nx = b + 1; }
+        if (request) {
+            rows.request(jt + 1);
+            request = false;
         }
-        float fpos = (float)pos;
-        // rows of hidden slots are zeroed on the way into the P.V product (0 * NaN): masks of this lane's
-        // operand keys 16 ks + 4 kq .. + 3, two 16-bit values per word
-        uint32_t m01[kPv], m23[kPv];
-#pragma unroll
-        for (int half = 0; half < kSK / 64; half++) {
-            const int64_t n = tile * kSK + 64 * half + lane;
-            bool v = false;
-            if (n < NS) v = a.sink_mask[n] == 0;
-            else if (n < NS + S) v = a.mask[n - NS] == 0;
-            else if (n < p.N) v = true;
-            const unsigned long long vis64 = __builtin_amdgcn_ballot_w64(v);
-#pragma unroll
-            for (int k4 = 0; k4 < 4; k4++) {
-                const int ks = 4 * half + k4;
-                const uint32_t vk = (uint32_t)(vis64 >> (16 * k4 + 4 * kq)) & 0xfu;
-                m01[ks] = ((vk & 1u) ? 0x0000ffffu : 0u) | ((vk & 2u) ? 0xffff0000u : 0u);
-                m23[ks] = ((vk & 4u) ? 0x0000ffffu : 0u) | ((vk & 8u) ? 0xffff0000u : 0u);
-            }
+        if (next_tile) {
+            rows.arrived();
+            rows.copy_from(jt + 1);
+            b_nx = 0;
         }
-        // copies: block jb of a wavefront brings rows 4 jb .. 4 jb + 3 of its 16; seg: 0 sink, 1 cache, 2 the new token
-        int seg_c[4];
-        uint32_t relk[4], relv[4];
-        bool cache_only[4];
-#pragma unroll
-        for (int jb = 0; jb < 4; jb++) {
-            const int r = 4 * jb + (lane >> 4);
-            const int64_t n = n_wave + r;
-            int64_t row_off;
-            if (n < NS) { seg_c[jb] = 0; row_off = n * a.sink_stride[2]; }
-            else if (n < NS + S) { seg_c[jb] = 1; row_off = (n - NS) * a.cache_stride[2]; }
-            else { seg_c[jb] = 2; row_off = 0; }
-            relk[jb] = (uint32_t)(row_off * kEs) + ((((uint32_t)lane & 15u) ^ ((uint32_t)r & 15u)) << 4);
-            relv[jb] = (uint32_t)(row_off * kEs) + ((((uint32_t)lane & 15u) ^ (((uint32_t)r & 7u) << 1)) << 4);
-            cache_only[jb] = __builtin_amdgcn_ballot_w64(seg_c[jb] == 1) == ~0ull;
-        }
-        asm volatile("" : "+v"(fpos));   // as in the kernel above
-        if (first_tile) shared.arrived();
-        auto slabs = [&](int b, int kvh, const char* (&kb)[3], const char* (&vb)[3]) {
-            const int64_t o0 = ((int64_t)b * a.sink_stride[0] + (int64_t)kvh * a.sink_stride[1]) * kEs;
-            const int64_t o1 = ((int64_t)b * a.cache_stride[0] + (int64_t)kvh * a.cache_stride[1]) * kEs;
-            const int64_t o2 = ((int64_t)b * a.kv_new_stride[0] + (int64_t)kvh * a.kv_new_stride[1]) * kEs;
-            kb[0] = (const char*)a.sink_k + o0; vb[0] = (const char*)a.sink_v + o0;
-            kb[1] = (const char*)a.cache_k + o1; vb[1] = (const char*)a.cache_v + o1;
-            kb[2] = (const char*)a.k_new + o2; vb[2] = (const char*)a.v_new + o2;
-        };
-        auto copy_rows = [&](const char* (&base)[3], const uint32_t(&rel)[4], uint32_t dst) {  // four copies
-#pragma unroll
-            for (int jb = 0; jb < 4; jb++) {
-                if (cache_only[jb]) {
-                    async_copy16(base[1], rel[jb], dst + jb * 1024);
-                } else {
-#pragma unroll
-                    for (int sgm = 0; sgm < 3; sgm++)
-                        if (seg_c[jb] == sgm) async_copy16(base[sgm], rel[jb], dst + jb * 1024);
-                }
-            }
-        };
-        // the query block of (b, kvh) into stage `st` (wavefronts 0 and 1, four heads each: lane i fills slot
-        // i % 16 of head 4 wave + i / 16 with the piece that belongs there), then this wavefront's K rows.  The
-        // query copy goes first: whoever waits for the four K copies behind it has waited for it too.
-        auto copy_kq = [&](int b, int kvh, int st) {
-            if (wave < 2 && !p.own_q) {
-                const char* qsrc = (const char*)p.qrot_t + ((int64_t)b * a.H + (int64_t)kvh * G) * (kD * kEs);
-                const int h = 4 * wave + (lane >> 4);
-                if (h < G) async_copy16(qsrc, h * 256 + (((lane & 15) ^ h) << 4), lds_base + kWideQ + st * 2048 + wave * 1024);
-            }
-            const char *kb[3], *vb[3];
-            slabs(b, kvh, kb, vb);
-            copy_rows(kb, relk, lds_base + st * kStreamStage + wave * 4096);
-        };
-        auto copy_v = [&](int b, int kvh, int st) {
-            const char *kb[3], *vb[3];
-            slabs(b, kvh, kb, vb);
-            copy_rows(vb, relv, lds_base + st * kStreamStage + kSK * 256 + wave * 4096);
-        };
-
-        int b = (int)((uint32_t)bh0 / (uint32_t)KVH), kvh = bh0 - b * KVH;
-        // results of the previous item, stored at the top of the next one
-        bool pending = false;
-        int pend_b = 0, pend_kvh = 0;
-        uint2 pend_o[kDb];
-        float pend_m = 0.f, pend_l = 0.f;
-        uint2 pend_e = make_uint2(0u, 0u);  // fp16 probabilities of head key16, keys 16 wave + 4 kq .. + 3
-#pragma unroll
-        for (int b2 = 0; b2 < kDb; b2++) pend_o[b2] = make_uint2(0u, 0u);
-        auto flush = [&]() {
-            if (!pending) return;
-            const int pend_item = jt * nbh + pend_b * KVH + pend_kvh;
-            const int64_t chunk_i = (int64_t)(pend_item - item0) * gridDim.x + blockIdx.x;
-            unsigned char* chunk = p.chunks + chunk_i * (G * (kSK + kD) * 2);
-            if (head_ok) {
-                *reinterpret_cast<uint2*>(chunk + (key16 * kSK + 16 * wave + 4 * kq) * 2) = pend_e;
-#pragma unroll
-                for (int b2 = 0; b2 < kDb; b2++)
-                    *reinterpret_cast<uint2*>(chunk + (G * kSK + key16 * kD + 16 * (kDb * wave + b2) + 4 * kq) * 2) = pend_o[b2];
-            }
-            if (wave == 0 && kq == 0 && head_ok)  // maximum and sum: G pairs per chunk, in chunk order
-                *reinterpret_cast<float2*>(p.part_ml + (chunk_i * G + key16) * 2) = make_float2(pend_m, pend_l);
-        };
-        // Per item a wavefront issues, in this order: [the query copy of the next item,] four K copies of the
-        // next item, the stores of the previous item's results, and after the barrier four V copies of the next
-        // item.  Loads and stores retire in issue order.
-        const int my_stores = kDb + 1 + (wave == 0 ? 1 : 0);
-        int stored = 0;
-        copy_kq(b, kvh, 0);
-        copy_v(b, kvh, 0);
-        if (first_tile) shared.finish(p, freqs, smem + kWideOwnQ, tid, wave);
-        first_tile = false;
-        // cos and sin while the first rows are on their way
-        RopeWord<T> rw[2][4];  // [ks][word]: dims 32 ks + 8 kq + 2 w, + 1 and their partners 64 further
-#pragma unroll
-        for (int ks = 0; ks < 2; ks++) {
-            float f[8];
-#pragma unroll
-            for (int e = 0; e < 8; e += 4) {
-                const float4 f4 = *reinterpret_cast<const float4*>(freqs + 32 * ks + 8 * kq + e);
-                f[e] = f4.x; f[e + 1] = f4.y; f[e + 2] = f4.z; f[e + 3] = f4.w;
-            }
-#pragma unroll
-            for (int w = 0; w < 4; w++) rw[ks][w] = rope_word_at<T>(__fmul_rn(fpos, f[2 * w]), __fmul_rn(fpos, f[2 * w + 1]));
-        }
-        // the first query block of the run must have landed for every wavefront (younger: the four V copies)
-        __builtin_amdgcn_s_waitcnt(0x0F74);
-        __builtin_amdgcn_s_barrier();
-        int st = 0;
-        for (int bh = bh0; bh < bh1; bh++) {
-            int b_nx = b, kvh_nx = kvh;
-            if (bh + 1 < bh1) {  // the last item of a run copies itself again: cheaper than a different path
-                kvh_nx = kvh + 1 == KVH ? 0 : kvh + 1;
-                b_nx = kvh + 1 == KVH ? b + 1 : b;
-            }
-            // this wavefront's K rows of the item are in LDS (younger: the stores issued after them and the four V
-            // copies of this item); its query block was complete before the previous barrier
-            wait_vm(4 + stored, false);
-            copy_kq(b_nx, kvh_nx, st ^ 1);
-            stored = pending ? my_stores : 0;
-            flush();
-            const unsigned char* stage = smem + st * kStreamStage;
-
-            // ---- rotate K in registers, logits by MFMA, shared through LDS
-            {
-                const int q_at = p.own_q ? kWideOwnQ + (b * KVH + kvh) * (G * 256) : kWideQ + st * 2048;
-                uint4 kraw[4], qop[4];
-#pragma unroll
-                for (int ks = 0; ks < 4; ks++) kraw[ks] = *reinterpret_cast<const uint4*>(stage + kaddr[ks]);
-#pragma unroll
-                for (int ks = 0; ks < 4; ks++) qop[ks] = *reinterpret_cast<const uint4*>(smem + q_at + q_off[ks]);
-                uint4 kop[4];
-#pragma unroll
-                for (int ks = 0; ks < 2; ks++) {
-                    const uint32_t* w1 = reinterpret_cast<const uint32_t*>(&kraw[ks]);
-                    const uint32_t* w2 = reinterpret_cast<const uint32_t*>(&kraw[ks + 2]);
-                    uint32_t o1[4], o2[4];
-#pragma unroll
-                    for (int w = 0; w < 4; w++) {
-                        rw[ks][w].rotate(w1[w], w2[w], p.key_scale, true, o1[w], o2[w]);
-                    }
-                    kop[ks] = make_uint4(o1[0], o1[1], o1[2], o1[3]);
-                    kop[ks + 2] = make_uint4(o2[0], o2[1], o2[2], o2[3]);
-                }
-                f32x4 sacc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int ks = 0; ks < 4; ks++) sacc = Mma16<T>::mma(qop[ks], kop[ks], sacc);
-                // lane holds heads 4 kq + v of key key16
-                if (kq < 2) {
-#pragma unroll
-                    for (int v = 0; v < 4; v++)
-                        if (4 * kq + v < G)
-                            s_all[(st * 8 + 4 * kq + v) * kWidePitch + wave * 16 + key16] = vis1 ? sacc[v] * p.scale_log2 : -INFINITY;
-                }
-            }
-            // this wavefront's V rows of the item and (wavefronts 0, 1) its part of the next query block have landed
-            // (younger: the four K copies of the next item and the stores of flush()); its logits are in LDS
-            wait_vm(4 + stored, true);
-            __builtin_amdgcn_s_barrier();
-            // every wavefront is past the previous item: its V stage can be refilled
-            copy_v(b_nx, kvh_nx, st ^ 1);
-
-            // ---- softmax of head key16 over the tile, by every wavefront, in the layout of the P.V operand:
-            //      this lane holds keys 16 ks + 4 kq .. + 3 (ks = 0 .. 7); lanes l, l ^ 16, l ^ 32, l ^ 48 share a head
-            float m_t, l_t;
-            uint2 pb[kPv];
-            uint2 e_mine = make_uint2(0u, 0u);
-            {
-                float x[kPv][4];
-                float mloc = -INFINITY;
-#pragma unroll
-                for (int ks = 0; ks < kPv; ks++) {
-                    float4 x4 = make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
-                    if (head_ok) x4 = *reinterpret_cast<const float4*>(s_all + (st * 8 + key16) * kWidePitch + 16 * ks + 4 * kq);
-                    x[ks][0] = x4.x; x[ks][1] = x4.y; x[ks][2] = x4.z; x[ks][3] = x4.w;
-                    mloc = fmaxf(fmaxf(mloc, fmaxf(x4.x, x4.y)), fmaxf(x4.z, x4.w));
-                }
-                const float m = rows4_max(mloc);
-                const float ms = m == -INFINITY ? 0.f : m;
-                float lloc = 0.f;
-#pragma unroll
-                for (int ks = 0; ks < kPv; ks++) {
-                    const float e0 = __builtin_amdgcn_exp2f(x[ks][0] - ms), e1 = __builtin_amdgcn_exp2f(x[ks][1] - ms);
-                    const float e2 = __builtin_amdgcn_exp2f(x[ks][2] - ms), e3 = __builtin_amdgcn_exp2f(x[ks][3] - ms);
-                    lloc += (e0 + e1) + (e2 + e3);
-                    pb[ks] = make_uint2(Mma16<T>::pack2(e0, e1), Mma16<T>::pack2(e2, e3));  // hidden keys and idle rows: 0
-                    if (ks == wave) {  // the piece this wavefront hands to the score kernel, fp16 whatever the tensor dtype
-                        e_mine = make_uint2(Mma16<__half>::pack2(e0, e1), Mma16<__half>::pack2(e2, e3));
-                    }
-                }
-                m_t = m;
-                l_t = rows4_sum(lloc);
-            }
-            // ---- weighted V sum on the matrix pipe: this wavefront's dims over all keys of the tile.  Lane
-            //      16 q + g (g < G) ends up with dims 16 (kDb wave + b2) + 4 q .. + 3 of head g.
-            f32x4 acc[kDb];
-#pragma unroll
-            for (int b2 = 0; b2 < kDb; b2++) acc[b2] = f32x4{0.f, 0.f, 0.f, 0.f};
-            {
-                const uint32_t vbase = lds_base + st * kStreamStage;
-#pragma unroll
-                for (int ks = 0; ks < kPv; ks++) {
-#pragma unroll
-                    for (int b2 = 0; b2 < kDb; b2++) {
-                        const s16x4_t va = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                            (__attribute__((address_space(3))) s16x4_t*)(uintptr_t)(vbase + vt_addr[b2] + ks * 4096));
-                        uint2 av = __builtin_bit_cast(uint2, va);
-                        av.x &= m01[ks];
-                        av.y &= m23[ks];
-                        acc[b2] = Mma16<T>::mma_k16(av, pb[ks], acc[b2]);
-                    }
-                }
-            }
-            {
-                // lanes 16 q + g hold head g = key16: l_t is that head's sum (0: the tile is hidden)
-                const float inv_l = l_t > 0.f ? 1.0f / l_t : 0.f;
-#pragma unroll
-                for (int b2 = 0; b2 < kDb; b2++)
-                    pend_o[b2] = make_uint2(Mma16<T>::pack2(acc[b2][0] * inv_l, acc[b2][1] * inv_l),
-                                            Mma16<T>::pack2(acc[b2][2] * inv_l, acc[b2][3] * inv_l));
-            }
-            pend_m = m_t;
-            pend_l = l_t;
-            pend_e = e_mine;
-            pending = true;
-            pend_b = b;
-            pend_kvh = kvh;
-            b = b_nx;
-            kvh = kvh_nx;
-            st ^= 1;
-        }
+        if (more) copy_kq(b_nx, kvh_nx, st ^ 1);
+        stored = pend_item >= 0 ? my_stores : 0;
         flush();
-        // the repeated copies of the last item must land, and every wavefront be done with the stages,
-        // before the next run of items refills them
-        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+        const unsigned char* stage = smem + st * kStreamStage;
+
+        // ---- rotate K in registers, logits by MFMA, shared through LDS
+        {
+            const int q_at = p.own_q ? kWideOwnQ + (b * KVH + kvh) * (G * 256) : kWideQ + st * 2048;
+            uint4 kraw[4], qop[4];
+#pragma unroll
+            for (int ks = 0; ks < 4; ks++) kraw[ks] = *reinterpret_cast<const uint4*>(stage + kaddr[ks]);
+#pragma unroll
+            for (int ks = 0; ks < 4; ks++) qop[ks] = *reinterpret_cast<const uint4*>(smem + q_at + q_off[ks]);
+            uint4 kop[4];
+#pragma unroll
+            for (int ks = 0; ks < 2; ks++) {
+                const uint32_t* w1 = reinterpret_cast<const uint32_t*>(&kraw[ks]);
+                const uint32_t* w2 = reinterpret_cast<const uint32_t*>(&kraw[ks + 2]);
+                uint32_t o1[4], o2[4];
+#pragma unroll
+                for (int w = 0; w < 4; w++) {
+                    rows.rw[ks][w].rotate(w1[w], w2[w], p.key_scale, true, o1[w], o2[w]);
+                }
+                kop[ks] = make_uint4(o1[0], o1[1], o1[2], o1[3]);
+                kop[ks + 2] = make_uint4(o2[0], o2[1], o2[2], o2[3]);
+            }
+            f32x4 sacc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int ks = 0; ks < 4; ks++) sacc = Mma16<T>::mma(qop[ks], kop[ks], sacc);
+            // lane holds heads 4 kq + v of key key16
+            if (kq < 2) {
+#pragma unroll
+                for (int v = 0; v < 4; v++)
+                    if (4 * kq + v < G)
+                        s_all[(st * 8 + 4 * kq + v) * kWidePitch + wave * 16 + key16] = rows.visible ? sacc[v] * p.scale_log2 : -INFINITY;
+            }
+        }
+        // this wavefront's V rows of the item and (wavefronts 0, 1) its part of the next query block have landed
+        // (younger: the four K copies of the next item and the stores of flush()); its logits are in LDS
+        wait_vm(more ? 4 + stored : 0, true);
         __builtin_amdgcn_s_barrier();
+        // every wavefront is past the previous item: its V stage can be refilled
+        if (more) copy_v(b_nx, kvh_nx, st ^ 1);
+
+        // ---- softmax of head key16 over the tile, by every wavefront, in the layout of the P.V operand:
+        //      this lane holds keys 16 ks + 4 kq .. + 3 (ks = 0 .. 7); lanes l, l ^ 16, l ^ 32, l ^ 48 share a head
+        float m_t, l_t;
+        uint2 pb[kPv];
+        uint2 e_mine = make_uint2(0u, 0u);
+        {
+            float x[kPv][4];
+            float mloc = -INFINITY;
+#pragma unroll
+            for (int ks = 0; ks < kPv; ks++) {
+                float4 x4 = make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
+                if (head_ok) x4 = *reinterpret_cast<const float4*>(s_all + (st * 8 + key16) * kWidePitch + 16 * ks + 4 * kq);
+                x[ks][0] = x4.x; x[ks][1] = x4.y; x[ks][2] = x4.z; x[ks][3] = x4.w;
+                mloc = fmaxf(fmaxf(mloc, fmaxf(x4.x, x4.y)), fmaxf(x4.z, x4.w));
+            }
+            const float m = rows4_max(mloc);
+            const float ms = m == -INFINITY ? 0.f : m;
+            float lloc = 0.f;
+#pragma unroll
+            for (int ks = 0; ks < kPv; ks++) {
+                const float e0 = __builtin_amdgcn_exp2f(x[ks][0] - ms), e1 = __builtin_amdgcn_exp2f(x[ks][1] - ms);
+                const float e2 = __builtin_amdgcn_exp2f(x[ks][2] - ms), e3 = __builtin_amdgcn_exp2f(x[ks][3] - ms);
+                lloc += (e0 + e1) + (e2 + e3);
+                pb[ks] = make_uint2(Mma16<T>::pack2(e0, e1), Mma16<T>::pack2(e2, e3));  // hidden keys and idle rows: 0
+                if (ks == wave) {  // the piece this wavefront hands to the score kernel, fp16 whatever the tensor dtype
+                    e_mine = make_uint2(Mma16<__half>::pack2(e0, e1), Mma16<__half>::pack2(e2, e3));
+                }
+            }
+            m_t = m;
+            l_t = rows4_sum(lloc);
+        }
+        // ---- weighted V sum on the matrix pipe: this wavefront's dims over all keys of the tile.  Lane
+        //      16 q + g (g < G) ends up with dims 16 (kDb wave + b2) + 4 q .. + 3 of head g.
+        f32x4 acc[kDb];
+#pragma unroll
+        for (int b2 = 0; b2 < kDb; b2++) acc[b2] = f32x4{0.f, 0.f, 0.f, 0.f};
+        {
+            const uint32_t vbase = lds_base + st * kStreamStage;
+#pragma unroll
+            for (int ks = 0; ks < kPv; ks++) {
+#pragma unroll
+                for (int b2 = 0; b2 < kDb; b2++) {
+                    const s16x4_t va = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                        (__attribute__((address_space(3))) s16x4_t*)(uintptr_t)(vbase + vt_addr[b2] + ks * 4096));
+                    uint2 av = __builtin_bit_cast(uint2, va);
+                    av.x &= rows.m01[ks];
+                    av.y &= rows.m23[ks];
+                    acc[b2] = Mma16<T>::mma_k16(av, pb[ks], acc[b2]);
+                }
+            }
+        }
+        {
+            // lanes 16 q + g hold head g = key16: l_t is that head's sum (0: the tile is hidden)
+            const float inv_l = l_t > 0.f ? 1.0f / l_t : 0.f;
+#pragma unroll
+            for (int b2 = 0; b2 < kDb; b2++)
+                pend_o[b2] = make_uint2(Mma16<T>::pack2(acc[b2][0] * inv_l, acc[b2][1] * inv_l),
+                                        Mma16<T>::pack2(acc[b2][2] * inv_l, acc[b2][3] * inv_l));
+        }
+        pend_m = m_t;
+        pend_l = l_t;
+        pend_e = e_mine;
+        pend_item = item;
+        b = b_nx;
+        kvh = kvh_nx;
+        st ^= 1;
+        if (next_tile) {
+            jt++;
+            rows.take(freqs);
+            request = (jt + 1) * nbh < item1;
+        }
     }
+    flush();
 }
 
 // one workgroup per (b, h): 16 groups of 32 threads walk every 16th tile, eight tiles in flight, then merge

@@ -292,6 +292,48 @@ def test_decode_streaming_many_items(H, KVH, dtype, fill):
             assert torch.equal(getattr(gpu, name)[0].cpu(), getattr(cpu, name)), f"step {step}: {name}"
 
 
+@pytest.mark.parametrize("B,H,KVH,W,fill,dtype", [
+    (1, 4, 1, 128, 300, torch.bfloat16),      # fewer items than compute units
+    (1, 4, 1, 10240, 36000, torch.bfloat16),  # one item a tile, one or two tiles a run: every item changes the tile
+    (1, 2, 1, 10240, 36000, torch.float16),
+    (1, 7, 1, 10240, 36000, torch.bfloat16),  # the same in the kernel for 5 to 8 heads
+    (1, 64, 16, 1024, 3500, torch.bfloat16),  # 64 query rows: the most that the workgroups rotate themselves
+    (3, 24, 6, 1024, 3500, torch.bfloat16),   # 72 rows: a launch of their own; runs of two or three items of 18 a tile
+    (5, 13, 13, 512, 1900, torch.float16),    # 65 rows
+    (1, 64, 8, 1024, 3500, torch.float16),    # 64 rows, eight heads per kv head
+    (3, 24, 3, 4096, 12000, torch.bfloat16),  # 72 rows, eight heads per kv head
+])
+def test_decode_runs_from_tile_to_tile(B, H, KVH, W, fill, dtype):
+    """One token over a window of many or few (tile, kv head) items, dealt in runs that rarely divide evenly: tiles that
+    begin and end anywhere in a run, the first with sinks and the last with the new token, and queries rotated by the
+    workgroups or by a launch of their own.  Against the oracle, with the bounds of the tests above; hidden slots hold NaN."""
+    from cascading_kv_cache_amd.cascade_attention import cascade_attention, default_inv_freq
+
+    D, NS = 128, 5
+    gpu, cpu = make_pair(B, KVH, D, NS, W, 4, dtype)
+    gen = torch.Generator().manual_seed(6)
+
+    def some(heads, n):
+        return (torch.randn(B, heads, n, D, generator=gen) * 0.7).to(dtype)
+
+    for lo in range(0, fill, 2048):
+        n = min(2048, fill - lo)
+        cpu.update(some(KVH, n), some(KVH, n), torch.rand(B, KVH, n, generator=gen).to(dtype))
+    layer = OracleCascadeAttention(H, KVH, D, rope_theta=5e5)
+    layer.query_pos = torch.arange(0, 512, dtype=torch.long).view(1, -1)
+    q, k, v = some(H, 1), some(KVH, 1), some(KVH, 1)
+    push_state(gpu, cpu)
+    hidden = gpu.mask[0].bool().expand(gpu.key_cache[0].shape[:-1])
+    gpu.key_cache[0][hidden] = float("nan")
+    gpu.value_cache[0][hidden] = float("nan")
+    out_g, new_g = cascade_attention(q.cuda(), k.cuda(), v.cuda(), gpu, 0, default_inv_freq(D, 5e5, "cuda:0"))
+    out_c = layer.forward(q, k, v, cpu)
+    assert torch.isfinite(out_g.float()).all()
+    err = (out_g.float().cpu() - out_c.float()).abs().max().item()
+    assert err <= tol(dtype), f"out max err {err:.3e}"
+    assert_scores_close(new_g, layer.last_new_scores[:, :KVH], dtype, "new-token scores")
+
+
 @pytest.mark.parametrize("dtype,D,H,KVH,Q,q_last", [
     (torch.float32, 32, 4, 2, 10, 3),       # fp32-math kernels
     (torch.bfloat16, 128, 8, 2, 64, 17),    # matrix-core prefill, key positions per (batch, kv head)
