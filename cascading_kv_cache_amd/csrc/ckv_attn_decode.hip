@@ -1947,9 +1947,10 @@ int run_decode(const DecodeParams& p_in, hipStream_t stream) {
     p.Np = (int64_t)p.tiles * kSK;
     p.own_q = use_stream && a.B * a.H <= kOwnQRows;
     p.inv_h = (uint32_t)((65536 + a.H - 1) / a.H);
-    if (!p.own_q) {
+    {
+        // timed stages: a call has this one either way, empty where the streaming kernel rotates the queries itself
         StageScope sc(CKV_STAGE_PREP, stream);
-        hipLaunchKernelGGL(decode_q_kernel<T>, dim3((unsigned)(a.B * a.H)), dim3(64), 0, stream, p);
+        if (!p.own_q) hipLaunchKernelGGL(decode_q_kernel<T>, dim3((unsigned)(a.B * a.H)), dim3(64), 0, stream, p);
         CKV_HIP_TRY(hipGetLastError());
     }
     {
