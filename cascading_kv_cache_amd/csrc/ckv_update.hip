@@ -3,7 +3,8 @@
 // Replaces the serial per-token Triton program of the reference
 // (cascade/models/cascading_cache.py:145-299 token loop, 302-774 body) with
 //
-//   plan   one workgroup per (batch, kv-head).  Walks the cascades in order; at every cascade
+//   plan   a unit (batch, kv-head) in the steady state is planned from closed forms, its cascades side by side.
+//          Else one workgroup walks the cascades of the unit in order; at every cascade
 //          the arrivals of the whole call are classified (insert / challenger), numbered with a
 //          ballot prefix sum, the challengers of each group are reduced to the group's winner
 //          ("later wins iff score >=", cascading_cache.py:699), and the tokens the cascade evicts
@@ -11,7 +12,7 @@
 //          a forest of disjoint move chains in global memory:
 //              first[t]   = slot the incoming token t finally lands in (-1: dropped)
 //              next_of[d] = slot the OLD content of slot d finally lands in (-1: dropped)
-//          plus the updated trackers.
+//          plus the trackers after the call, which apply commits.
 //   apply  one lane group per incoming token.  Follows the chain of its token from the head,
 //          carrying a whole row (K, V, score, original index) in registers with 16-byte lanes:
 //          read the displaced row, write the carried one, move on.  Chains are vertex-disjoint
@@ -33,6 +34,9 @@ constexpr int kMaxCascades = 64;
 constexpr int kPlanMaxTokens = 8192;   // incoming tokens one plan launch takes at most
 constexpr int kRingPer = 8;            // kPlanMaxTokens / 1024 threads, and enough for 256 tokens on 256 threads
 
+constexpr int32_t kPosChange = 1;      // the call put a token into the cascades, so the position ids change
+constexpr int32_t kPlanned = 2;        // the unit has been planned by the steady-state kernel
+
 struct UpdateParams {
     ckv_update_args a;
     int64_t token_offset;  // first incoming token handled by this launch
@@ -40,10 +44,17 @@ struct UpdateParams {
     int32_t do_pos;        // run the position pass (last launch of a call only)
     int32_t* first;        // [N*H][K]
     int32_t* next_of;      // [N*H][S]
-    int32_t* pos_flag;     // [N*H]: the call put a token into the cascades, so the position ids change
-    int32_t* mode;         // [N*H]: 1 = planned by the steady-state kernel: the new ring starts wait in start_new
-    int32_t* start_new;    // [N*H][cascades]: ring starts after the call, committed by the apply kernel
+    int32_t* flags;        // [N*H]: kPosChange | kPlanned
+    int32_t* sinks_new;    // [N*H]: sinks stored after the call
+    int32_t* trackers;     // [N*H][cascades]: tracker_word of every cascade
     int32_t apply_blocks;  // blocks along x that move rows; the blocks behind them write position ids
+};
+
+// The (batch, kv head) of a workgroup: grid coordinates y and z, so that no workgroup begins with 64-bit divisions (these
+// and the ones of the single-token walk were 0.9 us of the 7.3 that its launch took).
+struct Unit {
+    int64_t n, h, bh;
+    __device__ explicit Unit(const ckv_update_args& A) : n(blockIdx.z), h(blockIdx.y), bh((int64_t)blockIdx.z * A.H + blockIdx.y) {}
 };
 
 // exclusive prefix sum of one flag per thread over the whole workgroup; returns the block total
@@ -75,17 +86,256 @@ __device__ inline void emit_move(int32_t* first, int32_t* next_of, int dst, int 
     }
 }
 
+// ---- Units in the steady state: sinks and every cascade full, no token of the call accepted by the eager-fill rule, and every
+// acceptance period divides the next one (the power schedules).  Which arrivals a cascade sees, which of them are inserted
+// and where is then a closed form of the token counter: the arrivals of cascade i are the tokens whose index is a multiple of
+// period i - 1, every (period i / period i - 1)-th of them is inserted, the n-th insert lands n slots behind the ring start
+// and pushes the n-th oldest entry on to cascade i + 1.  What is left to compute is who wins each group.
+constexpr int kClosedThreads = 512;
+
+struct ClosedCascade {
+    int32_t nA, kf, E;  // arrivals, index of the first inserted arrival, inserts
+    uint32_t r;         // inserts every r-th arrival
+    int32_t sx;         // ring start before the call
+};
+
+// From the token counter (less the sinks) and the periods.  `U`: unsigned type that holds them.  A step or group length past 2^31
+// means at most one arrival or insert: any such value does.
+template <typename U>
+__device__ inline bool closed_cascade(U rel0, U per, U per_prev, int cap, ClosedCascade& c) {
+    if (per % per_prev != 0) return false;
+    const U r = per / per_prev, most = (U)0x7fffffff;
+    const U a0 = rel0 % per_prev ? per_prev - rel0 % per_prev : 0;   // first token that arrives here
+    const U q0 = rel0 / per_prev + (a0 ? 1 : 0);                     // arrival k is inserted iff (q0 + k) % r == 0
+    const U kf = q0 % r ? r - q0 % r : 0;
+    c.nA = a0 < (U)cap ? (int32_t)(((U)cap - a0 + per_prev - 1) / per_prev) : 0;
+    c.E = kf < (U)c.nA ? (int32_t)(((U)c.nA - kf + r - 1) / r) : 0;
+    c.kf = (int32_t)(kf < most ? kf : most);
+    c.r = (uint32_t)(r < most ? r : most);
+    return true;
+}
+
+// Lane j of every wavefront gets cascade j; false: the unit is left to the walk over all arrivals.  `touched`: the cascades that
+// hand on entries which depend on this call's scores -- the newest old entry once arrivals have challenged it, or winners
+// among the call's own tokens.  (Cascade 0 with period 1 inserts every token: there it is the tokens in order.)
+__device__ inline bool closed_forms(const ckv_update_args& A, const Unit& u, int64_t seen, int cap, int lane, ClosedCascade& c,
+                                    unsigned long long& touched) {
+    const int C = A.cascades;
+    const int64_t W = A.window_size, rel0 = seen - A.num_sink;
+    int64_t st = W, per = 1;
+    c = {};
+    if (lane < C) {
+        const int64_t at = u.n * A.tracker_stride[0] + u.h * A.tracker_stride[1] + lane * A.tracker_stride[2];
+        st = A.stored_tokens[at];
+        const int64_t sx = A.start_indices[at];
+        if (sx < 0 || sx >= W) st = -1;
+        c.sx = (int32_t)sx;
+        per = A.do_cache_every_n[lane];
+    }
+    const int64_t sinks0 = A.stored_sinks[u.n * A.stored_sinks_stride[0] + u.h * A.stored_sinks_stride[1]];
+    int64_t per_prev = __shfl_up(per, 1);
+    if (lane == 0) per_prev = 1;
+    bool ok = st == W && per > 0 && W >= 2 && sinks0 >= A.num_sink && rel0 >= 0 && !(A.eager_fill && seen <= A.max_seq_len + A.num_sink);
+    if (__builtin_amdgcn_ballot_w64(ok) != ~0ull) return false;
+    // 32-bit division when everything fits, which it does outside pathological streams
+    if (lane < C) {
+        if (rel0 < (1ll << 31) && __builtin_amdgcn_ballot_w64(per >= (1ll << 30)) == 0) {
+            ok = closed_cascade<uint32_t>((uint32_t)rel0, (uint32_t)per, (uint32_t)per_prev, cap, c);
+        } else {
+            ok = closed_cascade<uint64_t>((uint64_t)rel0, (uint64_t)per, (uint64_t)per_prev, cap, c);
+        }
+    }
+    const int before = __shfl_up(c.E, 1);
+    ok = ok && (lane == 0 || lane >= C || before == c.nA);  // what a full cascade evicts: as many as it inserts
+    touched = __builtin_amdgcn_ballot_w64(lane < C && !(c.E <= W - 1 || (c.E <= W && c.kf == 0) || (lane == 0 && per == 1)));
+    return __builtin_amdgcn_ballot_w64(ok) == ~0ull;
+}
+
+// Workgroup `part` of `parts` plans its share of the inserts of cascade `mine`: a thread per insert folds the arrivals up to the next insert into the group's winner
+// ("later wins iff score >=", cascading_cache.py:699) and writes where every member ends up.  Every chain entry has one
+// writer: cascade i owns the pointers of cascade i's arrivals.  Those are entries of the ring before as it was before the
+// call, so all cascades are planned side by side; where the cascade before is touched, this workgroup first repeats its pass
+// (and that of further touched ones before it) without the pointers, for what they hand on: the old entries, oldest first,
+// the newest of them as its challengers left it, then the call's own winners.
+// Bound by its chain of dependent loads (trackers, scores) and, where the inserts are many, by instructions: one workgroup
+// that walked all cascades took 22 us for 8 units x 4096 tokens x 8 cascades, a workgroup per cascade 10.2, one per 512
+// inserts 7.1 (16 units x 16 rings of 2048: 15.6; with 256 threads 7.2 and 24.1, with 1024 8.3 and 16.2).  Touched cascades
+// used to be left to the walk, to which a call like 256 tokens on rings of 128 or 4096 on rings of 2048 goes at every other
+// alignment: 14.4 and 77 us there, 6.1 and 15.6 here.  A pass that read its arrivals into registers instead of LDS: level.
+__device__ inline void plan_closed(const UpdateParams& p, const Unit& u, const ClosedCascade& forms, unsigned long long touched,
+                                   int mine, int part, int parts, unsigned char* smem) {
+    const ckv_update_args& A = p.a;
+    const int tid = threadIdx.x, T = blockDim.x;
+    const int C = A.cascades, W = (int)A.window_size, cap = p.k_sub;
+    const int64_t cs_base = u.n * A.cache_s_stride[0] + u.h * A.cache_s_stride[1];
+    const int64_t s_base = u.n * A.s_stride[0] + u.h * A.s_stride[1] + p.token_offset * A.s_stride[2];
+    int32_t* first = p.first + u.bh * A.K + p.token_offset;
+    int32_t* next_of = p.next_of + u.bh * A.max_seq_len;
+    int32_t* src[2] = {reinterpret_cast<int32_t*>(smem), reinterpret_cast<int32_t*>(smem) + cap};
+    float* score[2] = {reinterpret_cast<float*>(smem) + 2 * (size_t)cap, reinterpret_cast<float*>(smem) + 3 * (size_t)cap};
+    auto of = [&](int v, int j) -> int { return __builtin_amdgcn_readlane(v, j); };
+    auto slot_of = [&](int i, int sx, int m) -> int {  // the m-th entry from the ring start, m < W
+        const int ring = sx + m;
+        return i * W + (ring >= W ? ring - W : ring);
+    };
+    auto score_of = [&](int from) -> float {
+        return from < 0 ? load_as_float(A.s, s_base + (int64_t)(-1 - from) * A.s_stride[2], A.dtype)
+                        : load_as_float(A.cache_s, cs_base + (int64_t)from * A.cache_s_stride[2], A.dtype);
+    };
+    auto point = [&](int from, int slot) {  // the arrival that came from `from` ends up in `slot` (-1: nowhere)
+        if (from < 0) first[-1 - from] = slot;
+        else next_of[from] = slot;
+    };
+    // this workgroup's inserts (those of a pass that is repeated are all its own)
+    const int E_mine = of(forms.E, mine), share = (E_mine + parts - 1) / parts;
+    const int g_lo = part * share, g_hi = g_lo + share < E_mine ? g_lo + share : E_mine;
+    if (part > 0 && g_lo >= E_mine) return;
+    // the first cascade of the passes: its arrivals are read where they were before the call
+    const unsigned long long below = ~touched & ((1ull << mine) - 1ull);
+    const int from_cascade = below ? 64 - __builtin_clzll(below) : 0;
+    {
+        const int i = from_cascade, nA = of(forms.nA, i), sx_prev = i > 0 ? of(forms.sx, i - 1) : 0;
+        const bool scores = i != mine || of((int)forms.r, i) != 1 || of(forms.kf, i) != 0;   // else nobody is challenged
+        // a workgroup that has its own pass only needs the arrivals of its inserts, the first one those before them too
+        const int r = of((int)forms.r, i), kf = of(forms.kf, i);
+        const int lo = i == mine && part > 0 ? kf + g_lo * r : 0, hi = i == mine && part + 1 < parts ? kf + g_hi * r : nA;
+        for (int k = lo + tid; k < hi; k += T) {
+            // cascade 0 sees every token; past a ring's old entries its own inserts follow, which only cascade 0 hands on untouched
+            const int from = i == 0 ? -1 - k : k >= W ? -1 - (k - W) : slot_of(i - 1, sx_prev, k);
+            src[i & 1][k] = from;
+            if (scores) score[i & 1][k] = score_of(from);
+        }
+    }
+    for (int i = from_cascade; i <= mine; i++) {
+        __syncthreads();
+        const int nA = of(forms.nA, i), kf = of(forms.kf, i), E = of(forms.E, i), sx = of(forms.sx, i);
+        const uint32_t r = (uint32_t)of((int)forms.r, i);
+        const bool writes = i == mine, last = i + 1 >= C;
+        const int32_t* a_src = src[i & 1];
+        const float* a_score = score[i & 1];
+        int32_t* b_src = src[(i & 1) ^ 1];
+        float* b_score = score[(i & 1) ^ 1];
+        // arrivals k0 .. k1 - 1 challenge the holder; who loses ends up nowhere
+        auto challenge = [&](int k0, int k1, int& ws, float& wv, bool& held) {
+            for (int k = k0; k < k1; k++) {
+                const int from = a_src[k];
+                const float v = a_score[k];
+                if (v >= wv) {
+                    if (writes && !held) point(ws, -1);
+                    held = false;
+                    ws = from;
+                    wv = v;
+                } else if (writes) {
+                    point(from, -1);
+                }
+            }
+        };
+        if (tid == T - 1 && (!writes || part == 0) && (kf > 0 || (!writes && E >= W))) {
+            // arrivals before the first insert challenge the newest entry earlier calls left
+            const int p_lead = slot_of(i, sx, W - 1);
+            int ws = p_lead;
+            float wv = score_of(p_lead);
+            bool held = true;  // the old entry still holds the slot
+            challenge(0, kf < nA ? kf : nA, ws, wv, held);
+            if (writes) {
+                if (!held) next_of[p_lead] = -1;  // the old entry is dropped
+                if (!held && E < W) point(ws, p_lead);
+                if (!held && E >= W && last) point(ws, -1);  // insert W - 1 takes the slot again
+            } else if (E >= W) {
+                b_src[W - 1] = ws;
+                b_score[W - 1] = wv;
+            }
+        }
+        const int g_end = writes ? g_hi : E;
+        for (int g = (writes ? g_lo : 0) + tid; g < g_end; g += T) {
+            const int k0 = kf + (int)((uint32_t)g * r);
+            const int k1 = r < (uint32_t)(nA - k0) ? k0 + (int)r : nA;
+            int ws = a_src[k0];
+            float wv = 0.f;
+            bool held = false;
+            if (k1 > k0 + 1 || !writes) {
+                wv = a_score[k0];
+                challenge(k0 + 1, k1, ws, wv, held);
+            }
+            if (!writes) {
+                if (g + W < E) {  // pushed out again within the call
+                    b_src[g + W] = ws;
+                    b_score[g + W] = wv;
+                }
+                if (g < W - 1) {
+                    const int slot = slot_of(i, sx, g);
+                    b_src[g] = slot;
+                    b_score[g] = score_of(slot);
+                }
+            } else if (g + W >= E) {
+                const int slot = i * W + (int)(((uint32_t)sx + (uint32_t)g) % (uint32_t)W);
+                point(ws, slot);
+                if (last) next_of[slot] = -1;  // what the last cascade evicts is dropped
+            } else if (last) {
+                point(ws, -1);
+            }
+        }
+    }
+}
+
+// A cascade's trackers after the call as one word, which the plan leaves in scratch and the apply kernel commits (workgroups
+// of the plan launch still read the old ones): a cascade that is not full after the call has not moved its ring start.
+__device__ inline int32_t tracker_word(int32_t stored, int32_t start, int32_t W) { return stored >= W ? start : -1 - stored; }
+
+// Workgroups of a unit: one per cascade and extra ones for those with more inserts than threads, as far as they go (with
+// periods that double, cascades of a call of K tokens insert at most 2 K between them).
+__global__ void __launch_bounds__(kClosedThreads) ckv_update_plan_steady_kernel(UpdateParams p) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    const ckv_update_args& A = p.a;
+    const Unit u(A);
+    const int tid = threadIdx.x, lane = tid % CKV_WAVE, T = kClosedThreads;
+    const int C = A.cascades, block = (int)blockIdx.x, extra = (int)gridDim.x - C;
+    const int64_t seen = *A.real_token_idx + p.token_offset;  // tokens before token 0 of this launch
+    ClosedCascade forms;
+    unsigned long long touched;
+    const bool closed = closed_forms(A, u, seen, p.k_sub, lane, forms, touched);
+    if (block == 0 && tid == 0) {
+        p.flags[u.bh] = closed ? kPlanned | kPosChange : 0;
+        if (closed) p.sinks_new[u.bh] = (int32_t)A.stored_sinks[u.n * A.stored_sinks_stride[0] + u.h * A.stored_sinks_stride[1]];
+    }
+    if (!closed) return;
+    int mine = block, part = 0;
+    const int want = lane < C && forms.E > T ? (forms.E - 1) / T : 0;
+    int before = want;  // extra workgroups the cascades before this lane's want
+#pragma unroll
+    for (int off = 1; off < CKV_WAVE; off *= 2) {
+        const int v = __shfl_up(before, off);
+        if (lane >= off) before += v;
+    }
+    before -= want;
+    if (block >= C) {
+        const unsigned long long here = __builtin_amdgcn_ballot_w64(before <= block - C && block - C < before + want);
+        if (here == 0) return;
+        mine = __builtin_ctzll(here);
+        part = block - C - __shfl(before, mine) + 1;
+    }
+    const int left = extra - __shfl(before, mine), wanted = __shfl(want, mine);
+    const int parts = 1 + (wanted < left ? wanted : left > 0 ? left : 0);
+    if (part == 0 && tid == mine) {
+        p.trackers[u.bh * C + mine] = (int32_t)(((uint32_t)forms.sx + (uint32_t)forms.E) % (uint32_t)A.window_size);
+    }
+    plan_closed(p, u, forms, touched, mine, part, parts, smem);
+}
+
 __global__ void ckv_update_plan_kernel(UpdateParams p) {
     extern __shared__ __align__(16) unsigned char smem[];
     const ckv_update_args& A = p.a;
     const int tid = threadIdx.x, T = blockDim.x;
-    const int64_t bh = blockIdx.x;
-    if (p.mode[bh]) return;  // the steady-state kernel has planned this unit
-    const int64_t n = bh / A.H, h = bh % A.H;
+    const Unit u(A);
+    const int64_t n = u.n, h = u.h, bh = u.bh;
+    if (p.flags[bh] & kPlanned) return;  // the steady-state kernel has planned this unit
     const int cap = p.k_sub;
     const int C = A.cascades;
     const int64_t W = A.window_size, S = A.max_seq_len, NS = A.num_sink;
+    const int32_t Wi = (int32_t)W;
+    int32_t* trackers = p.trackers + bh * C;
 
+    const int64_t seen = *A.real_token_idx + p.token_offset;  // tokens before token 0 of this launch
     int32_t* a_src[2];
     uint16_t* a_trig[2];   // index of the token whose arrival set the entry moving: below kPlanMaxTokens
     float* a_score[2];
@@ -109,14 +359,13 @@ __global__ void ckv_update_plan_kernel(UpdateParams p) {
         a_trig[i] = reinterpret_cast<uint16_t*>(ptr); ptr += 2 * (size_t)((cap + 1) & ~1);
     }
 
-    int64_t* g_stored = A.stored_tokens + n * A.tracker_stride[0] + h * A.tracker_stride[1];
-    int64_t* g_start = A.start_indices + n * A.tracker_stride[0] + h * A.tracker_stride[1];
-    int64_t* g_sinks = A.stored_sinks + n * A.stored_sinks_stride[0] + h * A.stored_sinks_stride[1];
+    const int64_t* g_stored = A.stored_tokens + n * A.tracker_stride[0] + h * A.tracker_stride[1];
+    const int64_t* g_start = A.start_indices + n * A.tracker_stride[0] + h * A.tracker_stride[1];
+    const int64_t* g_sinks = A.stored_sinks + n * A.stored_sinks_stride[0] + h * A.stored_sinks_stride[1];
     const int64_t cs_base = n * A.cache_s_stride[0] + h * A.cache_s_stride[1];
     int32_t* first = p.first + bh * A.K + p.token_offset;
     int32_t* next_of = p.next_of + bh * S;
 
-    const int64_t seen = *A.real_token_idx + p.token_offset;  // tokens before token 0 of this launch
     const int64_t sinks0 = *g_sinks;
     int64_t room = NS - sinks0;
     if (room < 0) room = 0;
@@ -147,7 +396,8 @@ __global__ void ckv_update_plan_kernel(UpdateParams p) {
         }
     }
     __syncthreads();
-    if (tid == 0 && n_sink_new > 0) *g_sinks = sinks0 + n_sink_new;
+    if (tid == 0) p.sinks_new[bh] = (int32_t)(sinks0 + n_sink_new);
+    for (int i = tid; i < C; i += T) trackers[i] = tracker_word(st_l[i], sx_l[i], Wi);  // of the cascades that no arrival reaches
 
     // 64-bit division per arrival is what this kernel would spend its time on: token indices, periods
     // and the window fit 32 bits in every realistic call, and both divisors are usually powers of two
@@ -278,8 +528,7 @@ __global__ void ckv_update_plan_kernel(UpdateParams p) {
             const int sx_new = mod_w((int64_t)start0 + n_ev);
             st_l[i] = st_new;
             sx_l[i] = sx_new;
-            g_stored[i * A.tracker_stride[2]] = st_new;
-            g_start[i * A.tracker_stride[2]] = sx_new;
+            trackers[i] = tracker_word(st_new, sx_new, Wi);
         }
         nA = has_next ? n_ev : 0;
         cur ^= 1;
@@ -287,363 +536,198 @@ __global__ void ckv_update_plan_kernel(UpdateParams p) {
     __syncthreads();
 
     // the position ids change only when the last token of the call went to the cascades
-    if (p.do_pos && tid == 0) p.pos_flag[bh] = cap > n_sink_new ? 1 : 0;
+    if (tid == 0) p.flags[bh] = cap > n_sink_new ? kPosChange : 0;
 }
 
-// Steady-state plan: every cascade of the unit is full, no token of the call is accepted by the eager-fill rule,
-// and every acceptance period divides the next one (the power schedules).  Then which arrivals a cascade sees,
-// which of them are inserted and where, is a closed form of the token counter: the arrivals of cascade i are
-// the tokens whose index is a multiple of period i-1, every (period i / period i-1)-th of them is inserted,
-// the n-th insert lands n slots behind the ring start and pushes the n-th oldest entry on to cascade i+1.
-// As long as a cascade evicts only entries the call has not touched, its arrivals can be read straight from
-// the cache as it was before the call, so every cascade is planned by workgroups of its own, side by side:
-// one thread per insert folds the arrivals up to the next insert into the group's winner ("later wins iff
-// score >=", cascading_cache.py:699) and writes where every member of the group ends up.  Every chain entry
-// has one writer: the workgroups of cascade i own the pointers of cascade i's arrivals.  The ring starts after
-// the call go to scratch (the neighbours still read the old ones); the apply kernel commits them.
-// A unit that does not meet the conditions is left to the general kernel (mode 0).
-constexpr int kSteadyParts = 4;   // workgroups per cascade and unit
-constexpr int kSteadyThreads = 256;
-
-struct SteadyCascade {
-    int64_t per_prev, r;   // period of the cascade before, inserts every r-th arrival
-    int64_t a0;            // first token of the call that arrives at this cascade
-    int32_t nA, kf, E;     // arrivals, index of the first inserted arrival, inserts
-    int32_t sx;            // ring start before the call
+// The walk of a single incoming token (the decode step), by one wavefront: lane i fetches what cascade i may need (trackers,
+// period, the scores of its oldest and its newest slot) and works out where a row that comes to cascade i would land, so that
+// all cascades' loads travel together and every division is done once.  The token passes through the full cascades that
+// accept it, pushing their oldest entries on, up to the first cascade that is not full or does not accept: a count of
+// trailing ones.  Same semantics as the general kernel (cascading_cache.py:381-726 for one token).
+struct TokenWalk {
+    int count;            // slots of the chain; the token lands in the first, the old content of each in the next, the last's is dropped
+    int slot;             // lane i < count: slot i of the chain
+    int32_t st, sx;       // lane i: trackers of cascade i before the call
+    int32_t st_new, sx_new;  // and after it
+    bool sink;            // the token is a sink: the chain is its slot, S + index
+    int32_t sinks;        // sinks stored before the call
 };
 
-__global__ void __launch_bounds__(kSteadyThreads) ckv_update_plan_steady_kernel(UpdateParams p) {
-    __shared__ SteadyCascade sc[kMaxCascades];
-    __shared__ int64_t st_s[kMaxCascades], sx_s[kMaxCascades], per_s[kMaxCascades], seen_s, sinks_s;
-    __shared__ int fast_s;
-    const ckv_update_args& A = p.a;
-    const int tid = threadIdx.x;
-    const int64_t bh = blockIdx.y;
-    const int i = blockIdx.x / kSteadyParts, part = blockIdx.x % kSteadyParts;
-    const int64_t n = bh / A.H, h = bh % A.H;
+__device__ inline TokenWalk walk_token(const ckv_update_args& A, int64_t n, int64_t h, int64_t token, int lane) {
     const int C = A.cascades;
-    const int64_t W = A.window_size, S = A.max_seq_len, NS = A.num_sink;
-    const int cap = (int)A.K;  // the whole call is planned at once
-    const int64_t* g_stored = A.stored_tokens + n * A.tracker_stride[0] + h * A.tracker_stride[1];
-    const int64_t* g_start = A.start_indices + n * A.tracker_stride[0] + h * A.tracker_stride[1];
-    // the trackers of all cascades travel together; one thread then works out the closed forms
-    if (tid < C) {
-        st_s[tid] = g_stored[tid * A.tracker_stride[2]];
-        sx_s[tid] = g_start[tid * A.tracker_stride[2]];
-        per_s[tid] = A.do_cache_every_n[tid];
-    } else if (tid == kMaxCascades) {
-        seen_s = *A.real_token_idx;
-    } else if (tid == kMaxCascades + 1) {
-        sinks_s = A.stored_sinks[n * A.stored_sinks_stride[0] + h * A.stored_sinks_stride[1]];
-    }
-    __syncthreads();
-    // one thread per cascade works out that cascade's closed forms (they depend on the token counter and the
-    // periods only); 32-bit division when everything fits, which it does outside pathological streams
-    __shared__ int ok_s[kMaxCascades];
-    if (tid < C) {
-        const int j = tid;
-        const int64_t seen = seen_s, sinks0 = sinks_s;
-        const int64_t rel0 = seen - NS;
-        const int64_t per = per_s[j], per_prev = j == 0 ? 1 : per_s[j - 1];
-        const int64_t st = st_s[j], sx = sx_s[j];
-        bool ok = sinks0 >= NS && rel0 >= 0 && !(A.eager_fill && seen <= S + NS) && W >= 2 && W < (1ll << 30) &&
-                  cap < (1 << 30) && per > 0 && per_prev > 0 && st == W && sx >= 0 && sx < W;
-        SteadyCascade c;
-        c.per_prev = per_prev;
-        c.r = 1;
-        c.nA = c.kf = c.E = 0;
-        c.sx = (int32_t)sx;
-        c.a0 = 0;
-        if (ok) {
-            const bool small = rel0 < (1ll << 31) && per < (1ll << 31);
-            auto mod = [&](int64_t x, int64_t y) -> int64_t { return small ? (int64_t)((uint32_t)x % (uint32_t)y) : x % y; };
-            auto div = [&](int64_t x, int64_t y) -> int64_t { return small ? (int64_t)((uint32_t)x / (uint32_t)y) : x / y; };
-            ok = mod(per, per_prev) == 0;
-            if (ok) {
-                c.r = div(per, per_prev);
-                const int64_t a0 = mod(per_prev - mod(rel0, per_prev), per_prev);   // first token that arrives here
-                c.a0 = a0;
-                c.nA = a0 < cap ? (int32_t)div(cap - a0 + per_prev - 1, per_prev) : 0;
-                const int64_t q0 = div(rel0 + a0, per_prev);                       // arrival k is inserted iff (q0 + k) % r == 0
-                c.kf = (int32_t)mod(c.r - mod(q0, c.r), c.r);
-                c.E = c.nA > c.kf ? (int32_t)div((int64_t)c.nA - c.kf + c.r - 1, c.r) : 0;
-                // what the cascade evicts must be entries the call has not touched: at most all but the newest
-                // old entry; or all of them when no arrival challenges that entry before the first insert; cascade
-                // 0 with period 1 has no challengers at all, and what it evicts beyond its old entries are the
-                // call's own tokens in order
-                const bool untouched = c.E <= W - 1 || (c.E <= W && c.kf == 0) || (j == 0 && per == 1);
-                ok = j + 1 < C ? untouched : (c.E <= W || (j == 0 && per == 1));
-            }
-        }
-        sc[j] = c;
-        ok_s[j] = ok ? 1 : 0;
-    }
-    __syncthreads();
-    if (tid == 0) {
-        bool ok = true;
-        for (int j = 0; j < C; j++) {
-            ok = ok && ok_s[j];
-            if (j >= 1 && sc[j - 1].E != sc[j].nA) ok = false;  // evictions of a full cascade = its inserts
-        }
-        fast_s = ok ? 1 : 0;
-    }
-    __syncthreads();
-    const bool fast = fast_s != 0;
-    if (blockIdx.x == 0 && tid == 0) {
-        p.mode[bh] = fast ? 1 : 0;
-        if (fast) p.pos_flag[bh] = 1;
-    }
-    if (!fast) return;
-    const SteadyCascade c = sc[i];
+    const int32_t W = (int32_t)A.window_size;
     const int64_t cs_base = n * A.cache_s_stride[0] + h * A.cache_s_stride[1];
-    int32_t* first = p.first + bh * A.K;
-    int32_t* next_of = p.next_of + bh * S;
-    const int l = (int)((int64_t)i * W);
-    const int Wi = (int)W;
-    const bool prev_passes_tokens = i == 1 && sc[0].per_prev == 1 && sc[0].r == 1;  // cascade 0 has period 1
-    const int sx_prev = i >= 1 ? sc[i - 1].sx : 0;
-    // arrival k of this cascade: where it comes from (-1 - token, or the slot of the cascade before) and its score
-    auto arrival = [&](int k, int& src, float& score) {
-        if (i == 0) {
-            const int64_t t = c.a0 + (int64_t)k * c.per_prev;
-            src = -1 - (int)t;
-            score = load_as_float(A.s, n * A.s_stride[0] + h * A.s_stride[1] + t * A.s_stride[2], A.dtype);
-        } else if (prev_passes_tokens && k >= Wi) {
-            const int t = k - Wi;  // evicted by cascade 0 after it had been placed there in this call
-            src = -1 - t;
-            score = load_as_float(A.s, n * A.s_stride[0] + h * A.s_stride[1] + (int64_t)t * A.s_stride[2], A.dtype);
-        } else {
-            int ring = sx_prev + k;
-            if (ring >= Wi) ring -= Wi;
-            src = l - Wi + ring;
-            score = load_as_float(A.cache_s, cs_base + (int64_t)src * A.cache_s_stride[2], A.dtype);
-        }
-    };
-    auto point = [&](int src, int dst) {  // the arrival that came from `src` ends up in slot dst (-1: nowhere)
-        if (src < 0) first[-1 - src] = dst;
-        else next_of[src] = dst;
-    };
-    if (part == 0 && tid == 0) {
-        int sx_new = c.sx + (int)(c.E % Wi);
-        if (sx_new >= Wi) sx_new -= Wi;
-        p.start_new[bh * C + i] = sx_new;
-        // arrivals before the first insert challenge the newest entry earlier calls left
-        const int lead_n = c.kf < c.nA ? c.kf : c.nA;
-        if (lead_n > 0) {
-            const int p_lead = l + (c.sx == 0 ? Wi - 1 : c.sx - 1);
-            int ws = p_lead;
-            float wv = load_as_float(A.cache_s, cs_base + (int64_t)p_lead * A.cache_s_stride[2], A.dtype);
-            bool held = true;  // the old entry still holds the slot
-            for (int k = 0; k < lead_n; k++) {
-                int src;
-                float score;
-                arrival(k, src, score);
-                if (score >= wv) {
-                    if (!held) point(ws, -1);
-                    held = false;
-                    ws = src;
-                    wv = score;
-                } else {
-                    point(src, -1);
-                }
-            }
-            // with W inserts in the call the slot is taken again by the last of them (only behind the last
-            // cascade: elsewhere such a call is left to the general kernel), and the group's winner is dropped
-            const bool survives = c.E <= Wi - 1;
-            if (!held) {
-                if (survives) {
-                    point(ws, p_lead);
-                    next_of[p_lead] = -1;  // the old entry is dropped
-                } else {
-                    point(ws, -1);
-                }
-            }
+    const int64_t gidx = *A.real_token_idx + token;  // 0-based global index of the token
+    const int64_t sinks0 = A.stored_sinks[n * A.stored_sinks_stride[0] + h * A.stored_sinks_stride[1]];
+    const float tok_score = load_as_float(A.s, n * A.s_stride[0] + h * A.s_stride[1] + token * A.s_stride[2], A.dtype);
+    TokenWalk w;
+    w.st = w.sx = w.count = 0;
+    w.slot = -1;
+    int64_t per = 1;
+    float oldest = 0.f, newest = 0.f;
+    int lead = 0;
+    if (lane < C) {
+        w.st = (int32_t)A.stored_tokens[n * A.tracker_stride[0] + h * A.tracker_stride[1] + lane * A.tracker_stride[2]];
+        w.sx = (int32_t)A.start_indices[n * A.tracker_stride[0] + h * A.tracker_stride[1] + lane * A.tracker_stride[2]];
+        per = A.do_cache_every_n[lane];
+        if (w.st > 0) {
+            lead = lane * W + (w.sx > 0 && w.sx <= w.st ? w.sx - 1 : (w.sx - 1 + w.st) % w.st);
+            oldest = load_as_float(A.cache_s, cs_base + ((int64_t)lane * W + w.sx) * A.cache_s_stride[2], A.dtype);
+            newest = load_as_float(A.cache_s, cs_base + (int64_t)lead * A.cache_s_stride[2], A.dtype);
         }
     }
-    const int drop_before = c.E > Wi ? c.E - Wi : 0;  // inserts whose slot is taken again later in the call
-    for (int g = part * kSteadyThreads + tid; g < c.E; g += kSteadyParts * kSteadyThreads) {
-        const int k0 = c.kf + (int)((int64_t)g * c.r);
-        int k1 = k0 + (int)c.r;
-        if (k1 > c.nA) k1 = c.nA;
-        if (g < drop_before) {
-            // placed and pushed out again within the call: cascade 1 owns the pointer (it sees the token as an
-            // arrival of its own); behind the last cascade the members are dropped
-            if (i + 1 >= C) {
-                for (int k = k0; k < k1; k++) {
-                    int src;
-                    float score;
-                    arrival(k, src, score);
-                    point(src, -1);
-                }
-            }
-            continue;
+    w.st_new = w.st;
+    w.sx_new = w.sx;
+    w.sink = sinks0 < A.num_sink;
+    w.sinks = (int32_t)sinks0;
+    if (w.sink) {  // cascading_cache.py:399-431
+        w.count = 1;
+        w.slot = (int)(A.max_seq_len + sinks0);
+        return w;
+    }
+    const int64_t rel = gidx - A.num_sink;
+    bool on_period;
+    if (rel >= 0 && rel < (1ll << 32) && __builtin_amdgcn_ballot_w64(per <= 0 || per >= (1ll << 32)) == 0) {
+        on_period = (uint32_t)rel % (uint32_t)per == 0;
+    } else {
+        on_period = lane < C && rel % per == 0;
+    }
+    const bool takes = lane < C && ((A.eager_fill && gidx <= A.max_seq_len + A.num_sink) || on_period || w.st == 0);
+    const uint32_t ahead = (uint32_t)w.sx + (uint32_t)w.st;  // W: the ring's slots; both at most W
+    const int phys = lane * W + (int)(ahead < (uint32_t)W ? ahead : ahead < 2u * (uint32_t)W ? ahead - (uint32_t)W : ahead % (uint32_t)W);
+    const unsigned long long stays = ~__builtin_amdgcn_ballot_w64(takes && w.st >= W);
+    const int stop = stays ? __builtin_ctzll(stays) : CKV_WAVE;  // at most C: the lanes past it take nothing
+    w.count = stop;
+    if (lane < stop) {
+        w.slot = phys;
+        w.sx_new = w.sx + 1 < W ? w.sx + 1 : (w.sx + 1) % W;
+    }
+    if (stop < C) {
+        const float carried = stop == 0 ? tok_score : __shfl(oldest, stop > 0 ? stop - 1 : 0);
+        // an append (or the first entry of an empty cascade); else the newest slot keeps its token unless the arrival's
+        // score is at least as large
+        const bool lands = takes || carried >= newest;
+        if (lane == stop && lands) {
+            w.slot = takes ? phys : lead;
+            if (takes) w.st_new = w.st + 1;
         }
-        int ring = c.sx + (g % Wi);
-        if (ring >= Wi) ring -= Wi;
-        const int phys = l + ring;
-        int ws;
-        float wv;
-        arrival(k0, ws, wv);
-        for (int k = k0 + 1; k < k1; k++) {
-            int src;
-            float score;
-            arrival(k, src, score);
-            if (score >= wv) {
-                point(ws, -1);
-                ws = src;
-                wv = score;
-            } else {
-                point(src, -1);
-            }
-        }
-        point(ws, phys);
-        if (i + 1 >= C) next_of[phys] = -1;  // what the last cascade evicts is dropped
+        w.count += (int)(__builtin_amdgcn_ballot_w64(lands) >> stop & 1);
+    }
+    return w;
+}
+
+// lane i: cascade i's trackers, sinks by the last chain slot
+__device__ inline void write_trackers(const ckv_update_args& A, int64_t n, int64_t h, const TokenWalk& w, int lane) {
+    const int64_t at = n * A.tracker_stride[0] + h * A.tracker_stride[1] + lane * A.tracker_stride[2];
+    if (w.sink) {
+        if (lane == 0) A.stored_sinks[n * A.stored_sinks_stride[0] + h * A.stored_sinks_stride[1]] = w.slot - A.max_seq_len + 1;
+    } else if (lane < A.cascades) {
+        if (w.st_new != w.st) A.stored_tokens[at] = w.st_new;
+        if (w.sx_new != w.sx) A.start_indices[at] = w.sx_new;
     }
 }
 
-// The plan of a single incoming token (the decode step): one wavefront per (batch, kv head), no workgroup
-// barriers.  Lane i fetches what cascade i may need (trackers, period, the scores of its oldest and its newest
-// slot) so that all cascades' loads travel together; the walk over the cascades then runs on values handed
-// round by shuffles, identical in every lane, and lane 0 writes the chain.  Same semantics as the general
-// kernel (cascading_cache.py:381-726 for one token).
+// The plan of a single incoming token: one wavefront per (batch, kv head).
 __global__ void __launch_bounds__(CKV_WAVE) ckv_update_plan1_kernel(UpdateParams p) {
     const ckv_update_args& A = p.a;
     const int lane = threadIdx.x;
-    const int64_t bh = blockIdx.x;
-    const int64_t n = bh / A.H, h = bh % A.H;
-    const int C = A.cascades;
-    const int64_t W = A.window_size, S = A.max_seq_len, NS = A.num_sink;
-    int64_t* g_stored = A.stored_tokens + n * A.tracker_stride[0] + h * A.tracker_stride[1];
-    int64_t* g_start = A.start_indices + n * A.tracker_stride[0] + h * A.tracker_stride[1];
-    int64_t* g_sinks = A.stored_sinks + n * A.stored_sinks_stride[0] + h * A.stored_sinks_stride[1];
-    const int64_t cs_base = n * A.cache_s_stride[0] + h * A.cache_s_stride[1];
-    int32_t* first = p.first + bh * A.K + p.token_offset;
-    int32_t* next_of = p.next_of + bh * S;
-
-    const int64_t gidx = *A.real_token_idx + p.token_offset;  // 0-based global index of the token
-    const int64_t sinks0 = *g_sinks;
-    const float tok_score = load_as_float(A.s, n * A.s_stride[0] + h * A.s_stride[1] + p.token_offset * A.s_stride[2], A.dtype);
-    // lane i: cascade i
-    int32_t st = 0, sx = 0;
-    int64_t per = 1;
-    float oldest = 0.f, newest = 0.f;
-    if (lane < C) {
-        st = (int32_t)g_stored[lane * A.tracker_stride[2]];
-        sx = (int32_t)g_start[lane * A.tracker_stride[2]];
-        per = A.do_cache_every_n[lane];
-        const int64_t l = (int64_t)lane * W;
-        if (st > 0) {
-            oldest = load_as_float(A.cache_s, cs_base + (l + sx) * A.cache_s_stride[2], A.dtype);
-            newest = load_as_float(A.cache_s, cs_base + (l + (sx - 1 + st) % st) * A.cache_s_stride[2], A.dtype);
-        }
-    }
-    if (lane == 0) p.mode[bh] = 0;  // the trackers are written here, not left in scratch
-    if (sinks0 < NS) {  // the token is a sink (cascading_cache.py:399-431): no position pass
-        if (lane == 0) {
-            first[0] = (int32_t)(S + sinks0);
-            *g_sinks = sinks0 + 1;
-            if (p.do_pos) p.pos_flag[bh] = 0;
-        }
-        return;
-    }
-    int carry_src = -1;          // -1 - token index, or the slot whose old content is carried
-    float carry_score = tok_score;
-    int32_t first_val = -1;      // where the token lands (-1: dropped)
-    const int64_t rel = gidx - NS;
-    const bool eager = A.eager_fill && gidx <= S + NS;
-    for (int i = 0; i < C; i++) {
-        const int32_t st_i = __shfl(st, i), sx_i = __shfl(sx, i);
-        const int64_t per_i = __shfl(per, i);
-        const int l = (int)((int64_t)i * W);
-        const bool acc = eager || (rel % per_i) == 0;
-        if (acc || st_i == 0) {
-            const int phys = l + (int)(((int64_t)sx_i + st_i) % W);
-            if (st_i < (int32_t)W) {  // append (or the first entry of an empty cascade)
-                if (lane == 0) {
-                    next_of[phys] = -1;
-                    if (carry_src < 0) first_val = phys; else next_of[carry_src] = phys;
-                    g_stored[i * A.tracker_stride[2]] = st_i + 1;
-                }
-                break;
-            }
-            // full: the oldest entry (at the ring start) leaves for the next cascade, or is dropped
-            if (lane == 0) {
-                next_of[phys] = -1;
-                if (carry_src < 0) first_val = phys; else next_of[carry_src] = phys;
-                g_start[i * A.tracker_stride[2]] = (int64_t)((sx_i + 1) % (int32_t)W);
-            }
-            carry_src = phys;
-            carry_score = __shfl(oldest, i);
-            continue;
-        }
-        // not accepted: the newest slot keeps its token unless the arrival's score is at least as large
-        if (carry_score >= __shfl(newest, i)) {
-            const int p_lead = l + (sx_i - 1 + st_i) % st_i;
-            if (lane == 0) {
-                next_of[p_lead] = -1;
-                if (carry_src < 0) first_val = p_lead; else next_of[carry_src] = p_lead;
-            }
-        }
-        break;
-    }
+    const Unit u(A);
+    int32_t* next_of = p.next_of + u.bh * A.max_seq_len;
+    const TokenWalk w = walk_token(A, u.n, u.h, p.token_offset, lane);
+    const int next = __shfl_down(w.slot, 1);
+    if (!w.sink && lane < w.count) next_of[w.slot] = lane + 1 < w.count ? next : -1;
     if (lane == 0) {
-        first[0] = first_val;
-        if (p.do_pos) p.pos_flag[bh] = 1;
+        p.first[u.bh * A.K + p.token_offset] = w.count > 0 ? w.slot : -1;
+        p.flags[u.bh] = w.sink ? 0 : kPosChange;
+        p.sinks_new[u.bh] = w.sink ? (int32_t)(w.slot - A.max_seq_len) + 1 : w.sinks;
     }
+    if (lane < A.cascades) p.trackers[u.bh * A.cascades + lane] = tracker_word(w.st_new, w.sx_new, (int32_t)A.window_size);
 }
 
-// Position pass (cascading_cache.py:728-774, 129-142) after the plan kernel has updated the trackers:
-// slot j of cascade i gets ((j + seg - start) mod seg) + ub - seg, where seg is the number of stored
-// tokens and ub the ids still to hand out (all stored tokens, less a window per earlier cascade).
+// What a cascade's position ids are made of, from the trackers after the call (cascading_cache.py:728-774, 129-142): slot j
+// gets ((j + seg - start) mod seg) + ub - seg, where seg is the number of stored tokens and ub the ids still to hand out (all
+// stored tokens, less a window per earlier cascade).  Lane i of a wavefront holds cascade i.
+struct PosRange {
+    bool write;     // every earlier cascade holds tokens and ids are left
+    uint32_t seg, add;
+    int32_t base;
+    __device__ int64_t id_of(uint32_t j) const {
+        uint32_t x = j + add;
+        if (x >= seg) x -= seg;
+        if (x >= seg) x %= seg;  // slots past the stored tokens of a cascade that is not full
+        return (int64_t)((int32_t)x + base);
+    }
+};
+
+__device__ inline PosRange pos_range(int lane, int C, int32_t W, int32_t st, int32_t sx) {   // by every lane: it sums over them
+    int32_t tot = C * W;   // ids are indices below max_seq_len: they fit 32 bits
+    const unsigned long long below = __builtin_amdgcn_ballot_w64(lane < C && st < W);
+    int first_empty = C;
+    if (below) {
+        tot = lane < C ? st : 0;
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1) tot += __shfl_xor(tot, off);
+        const unsigned long long empty = __builtin_amdgcn_ballot_w64(lane < C && st <= 0);
+        if (empty) first_empty = __builtin_ctzll(empty);
+    }
+    const int32_t ub = tot - lane * W;
+    PosRange r;
+    r.seg = (uint32_t)(st < W ? st : W);
+    r.write = lane <= first_empty && (lane == 0 || ub > 0) && r.seg != 0;
+    r.add = r.seg - (uint32_t)sx;  // start < seg or start == 0
+    r.base = ub - (int32_t)r.seg;
+    return r;
+}
+
+// Position pass after the plan kernel has updated the trackers.
 // One 256-thread block per kPosChunk slots of a cascade and (batch, kv head), so the whole chip writes; the
 // blocks ride at the end of the apply kernels' grid (they need the plan's trackers, not the moved rows).
 constexpr int kPosChunk = 2048;
-
-__device__ inline void update_positions_block(const UpdateParams& p, int blk) {
+__device__ inline void update_positions_block(const UpdateParams& p, const Unit& u, int blk) {
     const ckv_update_args& A = p.a;
-    const int64_t bh = blockIdx.y;
-    if (!p.pos_flag[bh]) return;
-    const int64_t n = bh / A.H, h = bh % A.H;
-    const int C = A.cascades;
+    const int64_t n = u.n, h = u.h;
+    const int C = A.cascades, tid = threadIdx.x, lane = tid % CKV_WAVE;
     const int W = (int)A.window_size;
     const int per_c = (W + kPosChunk - 1) / kPosChunk;
     const int i = blk / per_c, j0 = (blk % per_c) * kPosChunk;
-    const int64_t* g_stored = A.stored_tokens + n * A.tracker_stride[0] + h * A.tracker_stride[1];
-    const int64_t* g_start = A.start_indices + n * A.tracker_stride[0] + h * A.tracker_stride[1];
-    // a unit planned by the steady-state kernel: every cascade is full, and the ring starts after the call are
-    // still in scratch (this launch commits them, so the trackers themselves are not read here)
-    const bool steady = p.mode[bh] != 0;
-    int64_t ub = 0;
-    for (int c = 0; c < C; c++) ub += steady ? (int64_t)W : g_stored[c * A.tracker_stride[2]];
-    // cascade i is written only if every earlier one holds tokens and ids are left
-    for (int c = 0; c < i; c++) {
-        if (!steady && g_stored[c * A.tracker_stride[2]] <= 0) return;
-        ub -= W;
-        if (ub <= 0) return;
+    const bool wanted = (p.flags[u.bh] & kPosChange) != 0;
+    int32_t st = 0, sx = 0;   // lane: cascade
+    if (lane < C) {
+        // a ring start that the call has not moved is read where it stands: nobody writes another value there
+        const int32_t word = p.trackers[u.bh * C + lane];
+        const int64_t start = A.start_indices[n * A.tracker_stride[0] + h * A.tracker_stride[1] + lane * A.tracker_stride[2]];
+        st = word >= 0 ? W : -1 - word;
+        sx = word >= 0 ? word : (int32_t)start;
     }
-    const int64_t st = steady ? (int64_t)W : g_stored[i * A.tracker_stride[2]];
-    const uint32_t seg = (uint32_t)(st < W ? st : W);
-    if (seg == 0) return;
-    const uint32_t sx_now = steady ? (uint32_t)p.start_new[bh * C + i] : (uint32_t)g_start[i * A.tracker_stride[2]];
-    const uint32_t add = seg - sx_now;  // start < seg or start == 0
-    const int64_t base = ub - seg;
-    auto id_of = [&](int j) -> int64_t {
-        uint32_t x = (uint32_t)j + add;
-        if (x >= seg) x -= seg;
-        if (x >= seg) x %= seg;  // slots past the stored tokens of a cascade that is not full
-        return (int64_t)x + base;
-    };
+    if (!wanted) return;
+    PosRange range = pos_range(lane, C, W, st, sx);
+    auto of = [&](int v) -> int { return __builtin_amdgcn_readlane(v, i); };
+    range.write = of((int)range.write) != 0;
+    range.seg = (uint32_t)of((int)range.seg);
+    range.add = (uint32_t)of((int)range.add);
+    range.base = of(range.base);
+    if (!range.write) return;
     int64_t* pos = A.pos + n * A.pos_stride[0] + h * A.pos_stride[1] + (int64_t)i * W * A.pos_stride[2];
-    const int tid = threadIdx.x;
     if (A.pos_stride[2] == 1 && (reinterpret_cast<uintptr_t>(pos) & 15u) == 0 && (W & 1) == 0) {
 #pragma unroll
         for (int it = 0; it < kPosChunk / 512; it++) {
             const int j = j0 + it * 512 + 2 * tid;
-            if (j < W) *reinterpret_cast<longlong2*>(pos + j) = make_longlong2(id_of(j), id_of(j + 1));
+            if (j < W) *reinterpret_cast<longlong2*>(pos + j) = make_longlong2(range.id_of(j), range.id_of(j + 1));
         }
     } else {
-        for (int j = j0 + tid; j < j0 + kPosChunk && j < W; j += 256) pos[(int64_t)j * A.pos_stride[2]] = id_of(j);
+        for (int j = j0 + tid; j < j0 + kPosChunk && j < W; j += 256) pos[(int64_t)j * A.pos_stride[2]] = range.id_of(j);
     }
+}
+
+// The first workgroup of a unit writes the trackers that the plan left in scratch.
+__device__ inline void commit_trackers(const UpdateParams& p, const Unit& u) {
+    const ckv_update_args& A = p.a;
+    if (blockIdx.x != 0 || (int)threadIdx.x >= A.cascades) return;
+    const int32_t word = p.trackers[u.bh * A.cascades + threadIdx.x];
+    const int64_t at = u.n * A.tracker_stride[0] + u.h * A.tracker_stride[1] + threadIdx.x * A.tracker_stride[2];
+    A.stored_tokens[at] = word >= 0 ? A.window_size : -1 - word;
+    if (word >= 0) A.start_indices[at] = word;
+    if (threadIdx.x == 0) A.stored_sinks[u.n * A.stored_sinks_stride[0] + u.h * A.stored_sinks_stride[1]] = p.sinks_new[u.bh];
 }
 
 // One 16-byte piece of a row per lane.
@@ -655,21 +739,16 @@ template <int LANES>
 __global__ void ckv_update_apply_vec_kernel(UpdateParams p) {
     const ckv_update_args& A = p.a;
     constexpr int kGroups = 256 / LANES;
-    if (blockIdx.x == 0 && p.do_pos && p.mode[blockIdx.y] && (int)threadIdx.x < A.cascades) {
-        // commit the ring starts the steady-state plan left in scratch (nobody reads the trackers in this launch)
-        const int64_t bh_c = blockIdx.y;
-        A.start_indices[(bh_c / A.H) * A.tracker_stride[0] + (bh_c % A.H) * A.tracker_stride[1] +
-                        threadIdx.x * A.tracker_stride[2]] = p.start_new[bh_c * A.cascades + threadIdx.x];
-    }
+    const Unit u(A);
+    commit_trackers(p, u);
     if ((int)blockIdx.x >= p.apply_blocks) {
-        update_positions_block(p, (int)blockIdx.x - p.apply_blocks);
+        update_positions_block(p, u, (int)blockIdx.x - p.apply_blocks);
         return;
     }
     const int g = blockIdx.x * kGroups + threadIdx.x / LANES;
     const int lane = threadIdx.x % LANES;
     if (g >= p.k_sub) return;
-    const int64_t bh = blockIdx.y;
-    const int64_t n = bh / A.H, h = bh % A.H;
+    const int64_t n = u.n, h = u.h, bh = u.bh;
     const int64_t S = A.max_seq_len;
     const int32_t* first = p.first + bh * A.K + p.token_offset;
     const int32_t* next_of = p.next_of + bh * S;
@@ -809,102 +888,25 @@ constexpr int64_t kOneMaxSlots = 16384;
 __global__ void __launch_bounds__(kOneThreads) ckv_update_one_kernel(UpdateParams p) {
     __shared__ int sh_chain[kOneWaves];
     __shared__ int sh_n, sh_pos;
-    __shared__ int sh_write[kOneWaves];                     // position ids of the cascade are written
-    __shared__ unsigned sh_seg[kOneWaves], sh_add[kOneWaves];
-    __shared__ long long sh_base[kOneWaves];
+    __shared__ PosRange sh_range[kOneWaves];
     const ckv_update_args& A = p.a;
     const int tid = threadIdx.x, lane = tid % CKV_WAVE, wave = tid / CKV_WAVE;
-    const int64_t bh = blockIdx.x;
-    const int64_t n = bh / A.H, h = bh % A.H;
+    const Unit u(A);
+    const int64_t n = u.n, h = u.h;
     const int C = A.cascades;
-    const int64_t W = A.window_size, S = A.max_seq_len, NS = A.num_sink;
+    const int64_t W = A.window_size, S = A.max_seq_len;
     const int es = (int)elem_bytes(A.dtype);
 
     if (wave == 0) {
-        int64_t* g_stored = A.stored_tokens + n * A.tracker_stride[0] + h * A.tracker_stride[1];
-        int64_t* g_start = A.start_indices + n * A.tracker_stride[0] + h * A.tracker_stride[1];
-        int64_t* g_sinks = A.stored_sinks + n * A.stored_sinks_stride[0] + h * A.stored_sinks_stride[1];
-        const int64_t cs_base = n * A.cache_s_stride[0] + h * A.cache_s_stride[1];
-        const int64_t gidx = *A.real_token_idx;  // 0-based global index of the token
-        const int64_t sinks0 = *g_sinks;
-        const float tok_score = load_as_float(A.s, n * A.s_stride[0] + h * A.s_stride[1], A.dtype);
-        // lane i: cascade i; all cascades' loads travel together
-        int32_t st = 0, sx = 0;
-        int64_t per = 1;
-        float oldest = 0.f, newest = 0.f;
-        if (lane < C) {
-            st = (int32_t)g_stored[lane * A.tracker_stride[2]];
-            sx = (int32_t)g_start[lane * A.tracker_stride[2]];
-            per = A.do_cache_every_n[lane];
-            const int64_t l = (int64_t)lane * W;
-            if (st > 0) {
-                oldest = load_as_float(A.cache_s, cs_base + (l + sx) * A.cache_s_stride[2], A.dtype);
-                newest = load_as_float(A.cache_s, cs_base + (l + (sx - 1 + st) % st) * A.cache_s_stride[2], A.dtype);
-            }
-        }
-        int n_chain = 0, do_pos = 1;
-        int st_new = st, sx_new = sx;  // lane i: trackers of cascade i after the call
-        if (sinks0 < NS) {  // the token is a sink (cascading_cache.py:399-431): no position pass
-            if (lane == 0) {
-                sh_chain[0] = (int)(S + sinks0);
-                *g_sinks = sinks0 + 1;
-            }
-            n_chain = 1;
-            do_pos = 0;
-        } else {
-            float carry_score = tok_score;
-            const int64_t rel = gidx - NS;
-            const bool eager = A.eager_fill && gidx <= S + NS;
-            for (int i = 0; i < C; i++) {
-                const int32_t st_i = __shfl(st, i), sx_i = __shfl(sx, i);
-                const int64_t per_i = __shfl(per, i);
-                const int l = (int)((int64_t)i * W);
-                const bool acc = eager || (rel % per_i) == 0;
-                if (acc || st_i == 0) {
-                    const int phys = l + (int)(((int64_t)sx_i + st_i) % W);
-                    if (lane == 0) sh_chain[n_chain] = phys;
-                    n_chain++;
-                    if (st_i < (int32_t)W) {  // append (or the first entry of an empty cascade)
-                        if (lane == i) st_new = st_i + 1;
-                        if (lane == 0) g_stored[i * A.tracker_stride[2]] = st_i + 1;
-                        break;
-                    }
-                    // full: the oldest entry (at the ring start) leaves for the next cascade, or is dropped
-                    if (lane == i) sx_new = (sx_i + 1) % (int32_t)W;
-                    if (lane == 0) g_start[i * A.tracker_stride[2]] = (int64_t)((sx_i + 1) % (int32_t)W);
-                    carry_score = __shfl(oldest, i);
-                    continue;
-                }
-                // not accepted: the newest slot keeps its token unless the arrival's score is at least as large
-                if (carry_score >= __shfl(newest, i)) {
-                    if (lane == 0) sh_chain[n_chain] = l + (sx_i - 1 + st_i) % st_i;
-                    n_chain++;
-                }
-                break;
-            }
-        }
-        // ---- parameters of the position ids (cascading_cache.py:728-774, 129-142) from the trackers after the
-        //      call, which lane i holds for cascade i: the same closed form as the position blocks of the apply
-        //      kernel.  Cascade i is written while every earlier cascade holds tokens and ids are left for it.
-        {
-            long long tot = lane < C ? (long long)st_new : 0;
-#pragma unroll
-            for (int off = 32; off >= 1; off >>= 1) tot += __shfl_xor(tot, off);
-            const unsigned long long empty = __builtin_amdgcn_ballot_w64(lane < C && st_new <= 0);
-            const int first_empty = empty ? __builtin_ctzll(empty) : C;
-            if (lane < C) {
-                const long long ub = tot - (long long)lane * W;   // ids still to hand out when cascade `lane` is reached
-                const unsigned seg = (unsigned)((long long)st_new < W ? st_new : (int32_t)W);
-                sh_write[lane] = (lane <= first_empty && (lane == 0 || ub > 0) && seg != 0) ? 1 : 0;
-                sh_seg[lane] = seg;
-                sh_add[lane] = seg - (unsigned)sx_new;  // start < seg or start == 0
-                sh_base[lane] = ub - (long long)seg;
-            }
-        }
+        const TokenWalk w = walk_token(A, n, h, 0, lane);
+        if (lane < w.count) sh_chain[lane] = w.slot;
+        const PosRange range = pos_range(lane, C, (int32_t)W, w.st_new, w.sx_new);
+        if (lane < C) sh_range[lane] = range;
         if (lane == 0) {
-            sh_n = n_chain;
-            sh_pos = do_pos;
+            sh_n = w.count;
+            sh_pos = w.sink ? 0 : 1;
         }
+        write_trackers(A, n, h, w, lane);
     }
     __syncthreads();
     const int n_chain = sh_n;
@@ -950,24 +952,19 @@ __global__ void __launch_bounds__(kOneThreads) ckv_update_one_kernel(UpdateParam
     // ---- position ids: they need the plan alone, so their stores go out while the displaced rows are on their way
     if (do_pos) {
         int64_t* pos = A.pos + n * A.pos_stride[0] + h * A.pos_stride[1];
-        auto id_of = [&](int i, unsigned j) -> int64_t {
-            const unsigned seg = sh_seg[i];
-            unsigned x = j + sh_add[i];
-            if (x >= seg) x -= seg;
-            if (x >= seg) x %= seg;  // slots past the stored tokens of a cascade that is not full
-            return (int64_t)x + sh_base[i];
-        };
         if (A.pos_stride[2] == 1 && (reinterpret_cast<uintptr_t>(pos) & 15u) == 0 && (W & 1) == 0) {
             for (int i = 0; i < C; i++) {
-                if (!sh_write[i]) continue;
+                const PosRange range = sh_range[i];
+                if (!range.write) continue;
                 int64_t* pc = pos + (int64_t)i * W;
                 for (int64_t j = 2 * (int64_t)tid; j < W; j += 2 * kOneThreads)
-                    *reinterpret_cast<longlong2*>(pc + j) = make_longlong2(id_of(i, (unsigned)j), id_of(i, (unsigned)j + 1));
+                    *reinterpret_cast<longlong2*>(pc + j) = make_longlong2(range.id_of((uint32_t)j), range.id_of((uint32_t)j + 1));
             }
         } else {
             for (int i = 0; i < C; i++) {
-                if (!sh_write[i]) continue;
-                for (int64_t j = tid; j < W; j += kOneThreads) pos[((int64_t)i * W + j) * A.pos_stride[2]] = id_of(i, (unsigned)j);
+                const PosRange range = sh_range[i];
+                if (!range.write) continue;
+                for (int64_t j = tid; j < W; j += kOneThreads) pos[((int64_t)i * W + j) * A.pos_stride[2]] = range.id_of((uint32_t)j);
             }
         }
     }
@@ -1007,21 +1004,16 @@ template <typename U>
 __global__ void ckv_update_apply_elem_kernel(UpdateParams p) {
     const ckv_update_args& A = p.a;
     constexpr int kPerLane = 8;
-    if (blockIdx.x == 0 && p.do_pos && p.mode[blockIdx.y] && (int)threadIdx.x < A.cascades) {
-        // commit the ring starts the steady-state plan left in scratch (nobody reads the trackers in this launch)
-        const int64_t bh_c = blockIdx.y;
-        A.start_indices[(bh_c / A.H) * A.tracker_stride[0] + (bh_c % A.H) * A.tracker_stride[1] +
-                        threadIdx.x * A.tracker_stride[2]] = p.start_new[bh_c * A.cascades + threadIdx.x];
-    }
+    const Unit u(A);
+    commit_trackers(p, u);
     if ((int)blockIdx.x >= p.apply_blocks) {
-        update_positions_block(p, (int)blockIdx.x - p.apply_blocks);
+        update_positions_block(p, u, (int)blockIdx.x - p.apply_blocks);
         return;
     }
     const int g = blockIdx.x * (256 / CKV_WAVE) + threadIdx.x / CKV_WAVE;
     const int lane = threadIdx.x % CKV_WAVE;
     if (g >= p.k_sub) return;
-    const int64_t bh = blockIdx.y;
-    const int64_t n = bh / A.H, h = bh % A.H;
+    const int64_t n = u.n, h = u.h, bh = u.bh;
     const int64_t S = A.max_seq_len;
     const int32_t* first = p.first + bh * A.K + p.token_offset;
     const int32_t* next_of = p.next_of + bh * S;
@@ -1119,7 +1111,7 @@ inline size_t plan_lds_bytes(int cap) {
 extern "C" int64_t ckv_update_workspace_bytes(int64_t N, int64_t H, int64_t K, int64_t max_seq_len,
                                               int32_t cascades) {
     if (N <= 0 || H <= 0 || K < 0 || max_seq_len <= 0 || cascades <= 0) return 0;
-    // move chains (first, next_of), then per unit: position flag, plan mode, ring starts after the call
+    // move chains (first, next_of), then per unit: flags, sinks and trackers after the call
     return ckv::align_up(N * H * (K + max_seq_len) * (int64_t)sizeof(int32_t), 256) +
            2 * ckv::align_up(N * H * (int64_t)sizeof(int32_t), 256) +
            ckv::align_up(N * H * cascades * (int64_t)sizeof(int32_t), 256) + 256;
@@ -1190,41 +1182,40 @@ int run_update(const ckv_update_args& A, void* workspace, hipStream_t stream) {
     p.a = A;
     p.first = reinterpret_cast<int32_t*>(workspace);
     p.next_of = p.first + A.N * A.H * A.K;
-    p.pos_flag = reinterpret_cast<int32_t*>(reinterpret_cast<char*>(workspace) +
+    p.flags = reinterpret_cast<int32_t*>(reinterpret_cast<char*>(workspace) +
                                             align_up(A.N * A.H * (A.K + A.max_seq_len) * (int64_t)sizeof(int32_t), 256));
-    p.mode = p.pos_flag + align_up(A.N * A.H * (int64_t)sizeof(int32_t), 256) / 4;
-    p.start_new = p.mode + align_up(A.N * A.H * (int64_t)sizeof(int32_t), 256) / 4;
+    p.sinks_new = p.flags + align_up(A.N * A.H * (int64_t)sizeof(int32_t), 256) / 4;
+    p.trackers = p.sinks_new + align_up(A.N * A.H * (int64_t)sizeof(int32_t), 256) / 4;
     p.token_offset = 0;
     p.k_sub = 0;
     p.do_pos = 0;
     p.apply_blocks = 0;
+    const unsigned H = (unsigned)A.H, N = (unsigned)A.N;
     if (A.K == 1 && vec && A.cascades <= kOneWaves && A.HID * es / 16 <= CKV_WAVE &&
         (A.N * A.H >= kOneMinUnits || (A.N * A.H >= kOneFewUnits && A.max_seq_len <= kOneMaxSlots))) {
         // the decode step of many streams: plan, moves and position ids of a unit by one workgroup, one launch
-        launch_timed(CKV_STAGE_APPLY, ckv_update_one_kernel, dim3((unsigned)(A.N * A.H)), dim3(kOneThreads), 0, stream, p);
+        launch_timed(CKV_STAGE_APPLY, ckv_update_one_kernel, dim3(1, H, N), dim3(kOneThreads), 0, stream, p);
         CKV_HIP_TRY(hipGetLastError());
         return CKV_OK;
     }
-    if (A.K >= 2) {
-        // every unit first gets the chance of the steady-state plan (whole call, all cascades side by side); it
-        // marks the units it has planned, the general kernel below takes the others
-        launch_timed(CKV_STAGE_PLAN, ckv_update_plan_steady_kernel,
-                     dim3((unsigned)(A.cascades * kSteadyParts), (unsigned)(A.N * A.H)), dim3(kSteadyThreads), 0, stream, p);
-        CKV_HIP_TRY(hipGetLastError());
-    }
-
     for (int64_t off = 0; off < A.K; off += qmax) {
         const int ksub = (int)((A.K - off < qmax) ? (A.K - off) : qmax);
         p.token_offset = off;
         p.k_sub = ksub;
         p.do_pos = (off + ksub == A.K) ? 1 : 0;
         if (A.K == 1) {  // the decode step: one wavefront per unit
-            launch_timed(CKV_STAGE_PLAN, ckv_update_plan1_kernel, dim3((unsigned)(A.N * A.H)), dim3(CKV_WAVE), 0, stream, p);
+            launch_timed(CKV_STAGE_PLAN, ckv_update_plan1_kernel, dim3(1, H, N), dim3(CKV_WAVE), 0, stream, p);
         } else {
+            // every unit first gets the chance of the closed forms; the general kernel takes the others
+            const size_t lds_closed = (size_t)ksub * 16;
+            if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(ckv_update_plan_steady_kernel), (int)lds_closed)) return rc;
+            launch_timed(CKV_STAGE_PLAN, ckv_update_plan_steady_kernel, dim3((unsigned)(A.cascades + 2 * ksub / kClosedThreads), H, N),
+                         dim3(kClosedThreads), lds_closed, stream, p);
+            CKV_HIP_TRY(hipGetLastError());
             const int T = ksub <= 256 ? 256 : 1024;  // few tokens: a small block plans them
             const size_t lds = plan_lds_bytes(ksub);
             if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(ckv_update_plan_kernel), (int)lds)) return rc;
-            launch_timed(CKV_STAGE_PLAN, ckv_update_plan_kernel, dim3((unsigned)(A.N * A.H)), dim3(T), lds, stream, p);
+            launch_timed(CKV_STAGE_PLAN, ckv_update_plan_kernel, dim3(1, H, N), dim3(T), lds, stream, p);
         }
         CKV_HIP_TRY(hipGetLastError());
         // the position ids of the last launch of a call are written by extra blocks of the apply grid
@@ -1237,7 +1228,7 @@ int run_update(const ckv_update_args& A, void* workspace, hipStream_t stream) {
             while (lanes < chunks) lanes *= 2;
             const dim3 block(256);
             p.apply_blocks = (ksub + 256 / lanes - 1) / (256 / lanes);
-            const dim3 grid((unsigned)p.apply_blocks + pos_blocks, (unsigned)(A.N * A.H));
+            const dim3 grid((unsigned)p.apply_blocks + pos_blocks, H, N);
             switch (lanes) {
                 case 1: launch_timed(CKV_STAGE_APPLY, ckv_update_apply_vec_kernel<1>, grid, block, 0, stream, p); break;
                 case 2: launch_timed(CKV_STAGE_APPLY, ckv_update_apply_vec_kernel<2>, grid, block, 0, stream, p); break;
@@ -1250,7 +1241,7 @@ int run_update(const ckv_update_args& A, void* workspace, hipStream_t stream) {
         } else {
             const dim3 block(256);
             p.apply_blocks = (ksub + 3) / 4;
-            const dim3 grid((unsigned)p.apply_blocks + pos_blocks, (unsigned)(A.N * A.H));
+            const dim3 grid((unsigned)p.apply_blocks + pos_blocks, H, N);
             if (es == 4) {
                 launch_timed(CKV_STAGE_APPLY, ckv_update_apply_elem_kernel<uint32_t>, grid, block, 0, stream, p);
             } else {

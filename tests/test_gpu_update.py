@@ -138,6 +138,20 @@ def test_single_token_calls_around_the_one_launch_rule(B, H, W, C):
     run_stream(gpu, cpu, fill + 12, lambda: next(lengths), gen, dtype, "ties")
 
 
+@pytest.mark.parametrize("func", ["pow2", "iplus1"])
+@pytest.mark.parametrize("W,C", [(2, 3), (7, 4), (16, 2), (300, 3), (16, 1)])
+def test_calls_that_evict_what_they_brought(W, C, func):
+    """Full caches and calls of about W, 2 W, 4 W tokens at every alignment with the acceptance periods: a cascade hands on
+    all but the newest of its old entries, all of them (the newest as its challengers left it), or entries the call itself
+    brought; with periods that divide each other (``pow2``) and with some that do not.  Bit-exact after every call."""
+    gpu, cpu = make_pair(1, 2, 8, 3, W, C, torch.bfloat16, func, eager=False)
+    gen = torch.Generator().manual_seed(W + C)
+    lengths = [3 + 2 ** C * W * 2] + [m * W + d for m in (1, 2, 4) for d in (-1, 0, 1)] + [2 * W, 2 * W + 1, 1, 2 * W, 4 * W + 3]
+    lengths = [n for n in lengths if n > 0]
+    left = iter(lengths)
+    run_stream(gpu, cpu, sum(lengths), lambda: next(left), gen, torch.bfloat16, "ties")
+
+
 def test_call_larger_than_one_launch():
     """More tokens than one planning launch holds in LDS: the call is split internally."""
     gpu, cpu = make_pair(1, 2, 16, 4, 64, 4, torch.float32, eager=False)
