@@ -77,11 +77,11 @@ __global__ void __launch_bounds__(kFwdWaves* CKV_WAVE) fwd_f32_mfma_kernel(F32Fw
     const int tid = threadIdx.x, lane = tid & 63, col = lane & 31, half = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // kv heads go round the XCDs (when they divide evenly), so a head's keys stay in one L2; heavy row tiles first
-    const int nbkv = (int)(p.B * p.KVH), G = (int)(p.H / p.KVH);
-    const int n_rt = (int)((p.Q * G + kRows - 1) / kRows);
+    const int nbkv = (int)(p.B * p.KVH), KVH = (int)p.KVH, G = (int)p.H / KVH;
+    const int n_rt = (int)(((int)p.Q * G + kRows - 1) / kRows);
     const int bkv = blockIdx.x % nbkv, rest = blockIdx.x / nbkv;
     const int split = rest % f.n_split, rt = n_rt - 1 - rest / f.n_split;
-    const int64_t b = bkv / p.KVH, kvh = bkv % p.KVH;
+    const int64_t b = bkv / KVH, kvh = bkv % KVH;
     const int N = (int)p.N, Q = (int)p.Q, Nc = N - Q;
     const float* kb = (const float*)p.k + b * p.kv_stride[0] + kvh * p.kv_stride[1];
     const float* vb = (const float*)p.v + b * p.kv_stride[0] + kvh * p.kv_stride[1];
@@ -315,7 +315,8 @@ __global__ void __launch_bounds__(256) fwd_f32_combine_kernel(F32Fwd f) {
         o.x = fmaf(v.x, w, o.x); o.y = fmaf(v.y, w, o.y); o.z = fmaf(v.z, w, o.z); o.w = fmaf(v.w, w, o.w);
     }
     const float inv = 1.f / L;
-    const int64_t m = row % p.Q, h = (row / p.Q) % p.H, b = row / (p.Q * p.H);
+    int64_t m, h;
+    const int64_t b = div_index(div_index(row, p.Q, m), p.H, h);
     float* dst = (float*)p.out + b * p.out_stride[0] + h * p.out_stride[1] + m * p.out_stride[2];
     dst[(4 * d4) * p.out_stride[3]] = o.x * inv;
     dst[(4 * d4 + 1) * p.out_stride[3]] = o.y * inv;
@@ -330,13 +331,13 @@ __global__ void __launch_bounds__(kColWaves* CKV_WAVE, 2) colsum_f32_mfma_kernel
     __shared__ float sums[kColWaves][kKeys];
     const int tid = threadIdx.x, lane = tid & 63, col = lane & 31, half = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int nbkv = (int)(p.B * p.KVH), G = (int)(p.H / p.KVH);
+    const int nbkv = (int)(p.B * p.KVH), KVH = (int)p.KVH, G = (int)p.H / KVH;
     const int N = (int)p.N, Q = (int)p.Q, Nc = N - Q, nblk = (N + kKeys - 1) / kKeys;
     // kv heads round the XCDs; blocks of chunk keys see fewer rows and come last
     const int bkv = blockIdx.x % nbkv, rest = blockIdx.x / nbkv;
     const int g = rest % G, blk = rest / G;
     if (blk >= nblk) return;
-    const int64_t b = bkv / p.KVH, kvh = bkv % p.KVH, h = kvh * G + g;
+    const int64_t b = bkv / KVH, kvh = bkv % KVH, h = kvh * G + g;
     const int n0 = blk * kKeys, n = n0 + col, nrel = n - Nc;   // nrel >= 0: a chunk key
     const bool live = n < N && !(n < Nc && p.kmasked && p.kmasked[n]);
     float acc = 0.f;

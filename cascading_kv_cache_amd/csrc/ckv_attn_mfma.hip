@@ -157,13 +157,51 @@ __device__ inline void stage_sincos(float x, float* sn, float* cs) {
     else fast_sincos(x, sn, cs);
 }
 
+// pair i of the threads with `quarter`
+__device__ inline int stage_pair(int quarter, int i) { return i < 8 ? 8 * quarter + i : 24 + 8 * quarter + i; }
+
+// LDS of a block: (d, d + kD/2) pairs of a key row, odd pitch; cos and sin of the threads' pairs while they are computed
+template <int kD>
+struct StageLds {
+    static constexpr int kPitch = kD / 2 + 1;
+    union {
+        uint32_t v[kBN][kPitch];
+        uint2 trig[kD / 16][256];
+    };
+    float freqs[kD / 2];
+};
+
+// frequencies of the rotation pairs into LDS (visible after a barrier)
+template <int kD>
+__device__ inline void stage_freqs(const float* inv_freq, float theta, StageLds<kD>& lds) {
+    const int j = threadIdx.x;
+    if (j < kD / 2) lds.freqs[j] = inv_freq ? inv_freq[j] : 1.0f / powf(theta, (float)(2 * j) / (float)kD);
+}
+
+// cos / sin of a thread's rotation pairs, two per word, rounded to the tensor dtype (see RopeWord).  A loop on purpose, with
+// the words parked in LDS: unrolled 16 times, the range reductions and the power function are 48 KiB of instructions that
+// a launch fetches cold and executes once per workgroup (8 heads x 16897 keys and 509 x 32 queries: 47 us unrolled, 33.5 so;
+// 16 x 18496: 90 and 73; 8 x 69696: 133 and 109, 5.2 TB/s).
+template <typename T, int kD>
+__device__ inline void stage_trig(float pos, int quarter, StageLds<kD>& lds, RopeWord<T> (&rw)[kD / 16]) {
+    const int tid = threadIdx.x;
+#pragma unroll 1
+    for (int k = 0; k < kD / 16; k++) {
+        float sn[2], cs[2];
+#pragma unroll
+        for (int e = 0; e < 2; e++) stage_sincos<kD>(__fmul_rn(pos, lds.freqs[stage_pair(quarter, 2 * k + e)]), &sn[e], &cs[e]);
+        lds.trig[k][tid] = make_uint2(RopeWord<T>::pack2(cs[0], cs[1]), RopeWord<T>::pack2(sn[0], sn[1]));
+    }
+#pragma unroll
+    for (int k = 0; k < kD / 16; k++) rw[k] = RopeWord<T>::of(lds.trig[k][tid]);   // a thread's own words
+}
+
 // One block of 256 threads stages key tile `tile_i` for the (b, kvh) units split_i, split_i + n_split, ...:
 // thread = (key = tid/4, quarter = tid%4) owns rotation pairs j = 8q .. 8q+7 (and, with 128 dims, 32+8q .. 32+8q+7),
 // i.e. the 16-byte pieces q, 4+q (, 8+q and 12+q) of its row: the four threads of a row read (and, for queries,
 // write) 64 contiguous bytes per instruction.
-__device__ inline int stage_pair(int quarter, int i) { return i < 8 ? 8 * quarter + i : 24 + 8 * quarter + i; }
 template <typename T, int kD>
-__device__ inline void stage_keys_block(const StageParams& p, int tile_i, int split_i, int n_split, uint32_t (*v_lds)[kD / 2 + 1]) {
+__device__ inline void stage_keys_block(const StageParams& p, int tile_i, int split_i, int n_split, StageLds<kD>& lds) {
     constexpr int kPieces = kD / 64;     // 16-byte pieces of each half of the row
     constexpr int kPairs = kD / 8;       // rotation pairs of a thread
     const int tid = threadIdx.x;
@@ -204,25 +242,36 @@ __device__ inline void stage_keys_block(const StageParams& p, int tile_i, int sp
         if (tid == 0) p.tile_vis[tile] = bal;
     }
 
-    // cos / sin of this thread's rotation pairs, two per word, rounded to the tensor dtype (see RopeWord)
-    RopeWord<T> rw[kPairs / 2];
-    auto trig_at = [&](int64_t pos) {
-#pragma unroll
-        for (int k = 0; k < kPairs / 2; k++) {
-            float sn[2], cs[2];
-#pragma unroll
-            for (int e = 0; e < 2; e++) {
-                const int j = stage_pair(quarter, 2 * k + e);
-                const float f = p.inv_freq ? p.inv_freq[j] : 1.0f / powf(p.theta, (float)(2 * j) / (float)kD);
-                stage_sincos<kD>(__fmul_rn((float)pos, f), &sn[e], &cs[e]);
-            }
-            rw[k] = RopeWord<T>::make(cs[0], sn[0], cs[1], sn[1]);
-        }
-    };
     const bool rotate = sidx >= 0 && p.seg[sidx].pos != nullptr;
-    if (rotate && p.shared_pos) trig_at(p.seg[sidx].pos[local] + p.seg[sidx].pos_shift);
+    int64_t pos = 0;
+    if (rotate && p.shared_pos) pos = p.seg[sidx].pos[local] + p.seg[sidx].pos_shift;
+    RopeWord<T> rw[kPairs / 2];
     const bool key_scaled = p.key_scale != 1.0f;
     const int64_t nbh = p.B * p.KVH;
+    // units split_i, split_i + n_split, ... as (b, kvh): stepped, not divided
+    const int KVH = (int)p.KVH, step_b = (int)((uint32_t)n_split / (uint32_t)KVH), step_h = n_split - step_b * KVH;
+    struct Unit {
+        int b, kvh;
+    };
+    auto next_unit = [&](Unit& u) {
+        u.b += step_b;
+        u.kvh += step_h;
+        if (u.kvh >= KVH) { u.kvh -= KVH; u.b++; }
+    };
+    Unit ahead;   // of the rows that are requested
+    ahead.b = (int)((uint32_t)split_i / (uint32_t)KVH);
+    ahead.kvh = split_i - ahead.b * KVH;
+    // this thread's row of the segment it lies in
+    const T *k_row = nullptr, *v_row = nullptr;
+    int64_t stride_b = 0, stride_h = 0, stride_d = 0;
+    if (sidx >= 0) {
+        const KeySegment& sg = p.seg[sidx];
+        k_row = (const T*)sg.k + local * sg.stride[2];
+        v_row = (const T*)sg.v + local * sg.stride[2];
+        stride_b = sg.stride[0];
+        stride_h = sg.stride[1];
+        stride_d = sg.stride[3];
+    }
     // the rows of unit bh as this thread's 16-byte pieces (zeros past the last key)
     struct Rows {
         uint4 lo[kPieces], hi[kPieces], vlo[kPieces], vhi[kPieces];
@@ -231,12 +280,10 @@ __device__ inline void stage_keys_block(const StageParams& p, int tile_i, int sp
 #pragma unroll
         for (int i = 0; i < kPieces; i++) r.lo[i] = r.hi[i] = r.vlo[i] = r.vhi[i] = make_uint4(0, 0, 0, 0);
         if (sidx < 0 || bh >= nbh) return;
-        const int64_t b = bh / p.KVH, kvh = bh % p.KVH;
-        const KeySegment& sg = p.seg[sidx];
-        const int64_t off = b * sg.stride[0] + kvh * sg.stride[1] + local * sg.stride[2];
-        const T* kp = (const T*)sg.k + off;
-        const T* vp = (const T*)sg.v + off;
-        if (sg.stride[3] == 1 && ((reinterpret_cast<uintptr_t>(kp) | reinterpret_cast<uintptr_t>(vp)) & 15) == 0) {
+        const int64_t off = ahead.b * stride_b + ahead.kvh * stride_h;
+        const T* kp = k_row + off;
+        const T* vp = v_row + off;
+        if (stride_d == 1 && ((reinterpret_cast<uintptr_t>(kp) | reinterpret_cast<uintptr_t>(vp)) & 15) == 0) {
 #pragma unroll
             for (int i = 0; i < kPieces; i++) {
                 r.lo[i] = *reinterpret_cast<const uint4*>(kp + 32 * i + 8 * quarter);
@@ -250,10 +297,10 @@ __device__ inline void stage_keys_block(const StageParams& p, int tile_i, int sp
             T* vl = reinterpret_cast<T*>(r.vlo);
             T* vh = reinterpret_cast<T*>(r.vhi);
             for (int i = 0; i < kPairs; i++) {
-                l0[i] = kp[stage_pair(quarter, i) * sg.stride[3]];
-                h0[i] = kp[(kD / 2 + stage_pair(quarter, i)) * sg.stride[3]];
-                vl[i] = vp[stage_pair(quarter, i) * sg.stride[3]];
-                vh[i] = vp[(kD / 2 + stage_pair(quarter, i)) * sg.stride[3]];
+                l0[i] = kp[stage_pair(quarter, i) * stride_d];
+                h0[i] = kp[(kD / 2 + stage_pair(quarter, i)) * stride_d];
+                vl[i] = vp[stage_pair(quarter, i) * stride_d];
+                vh[i] = vp[(kD / 2 + stage_pair(quarter, i)) * stride_d];
             }
         }
     };
@@ -261,24 +308,32 @@ __device__ inline void stage_keys_block(const StageParams& p, int tile_i, int sp
     // the workgroup always has loads in flight.
     Rows nxt;
     load_rows(split_i, nxt);
+    // no barrier between a thread's own words here and the first rows in LDS but the one in front of those
+    const bool rotates = p.seg[0].pos || p.seg[1].pos || p.seg[2].pos;
+    if (rotates) {
+        stage_freqs<kD>(p.inv_freq, p.theta, lds);
+        __syncthreads();
+        if (rotate && p.shared_pos) stage_trig<T, kD>((float)pos, quarter, lds, rw);
+    }
     for (int64_t bh = split_i; bh < nbh; bh += n_split) {
-        const int64_t b = bh / p.KVH, kvh = bh % p.KVH;
+        const Unit u = ahead;
         Rows cur = nxt;
+        next_unit(ahead);
         load_rows(bh + n_split, nxt);
         uint4(&lo)[kPieces] = cur.lo;
         uint4(&hi)[kPieces] = cur.hi;
         uint4(&vlo)[kPieces] = cur.vlo;
         uint4(&vhi)[kPieces] = cur.vhi;
-        if (sidx >= 0) {
-            const KeySegment& sg = p.seg[sidx];
-            if (rotate) {
-                if (!p.shared_pos)
-                    trig_at(sg.pos[b * sg.pos_stride[0] + kvh * sg.pos_stride[1] + local] + sg.pos_shift);
-                uint32_t* lw = reinterpret_cast<uint32_t*>(lo);
-                uint32_t* hw = reinterpret_cast<uint32_t*>(hi);
-#pragma unroll
-                for (int k = 0; k < kPairs / 2; k++) rw[k].rotate(lw[k], hw[k], p.key_scale, key_scaled, lw[k], hw[k]);
+        if (rotates && !p.shared_pos) __syncthreads();   // the last unit's rows have been read from LDS
+        if (rotate) {
+            if (!p.shared_pos) {
+                const KeySegment& sg = p.seg[sidx];
+                stage_trig<T, kD>((float)(sg.pos[u.b * sg.pos_stride[0] + u.kvh * sg.pos_stride[1] + local] + sg.pos_shift), quarter, lds, rw);
             }
+            uint32_t* lw = reinterpret_cast<uint32_t*>(lo);
+            uint32_t* hw = reinterpret_cast<uint32_t*>(hi);
+#pragma unroll
+            for (int k = 0; k < kPairs / 2; k++) rw[k].rotate(lw[k], hw[k], p.key_scale, key_scaled, lw[k], hw[k]);
         }
         char* kimg = (char*)p.kr + (bh * (p.n_pad / kBN) + tile) * (int64_t)(kD * kBN * sizeof(T));
 #pragma unroll
@@ -296,7 +351,7 @@ __device__ inline void stage_keys_block(const StageParams& p, int tile_i, int sp
             const uint16_t* vl = reinterpret_cast<const uint16_t*>(vlo);
             const uint16_t* vh = reinterpret_cast<const uint16_t*>(vhi);
 #pragma unroll
-            for (int i = 0; i < kPairs; i++) v_lds[key][stage_pair(quarter, i)] = (uint32_t)vl[i] | ((uint32_t)vh[i] << 16);
+            for (int i = 0; i < kPairs; i++) lds.v[key][stage_pair(quarter, i)] = (uint32_t)vl[i] | ((uint32_t)vh[i] << 16);
         }
         __syncthreads();
         char* vimg = (char*)p.vt + (bh * (p.n_pad / kBN) + tile) * (int64_t)(kD * kBN * sizeof(T));
@@ -309,7 +364,7 @@ __device__ inline void stage_keys_block(const StageParams& p, int tile_i, int sp
                 // inverse of vt_slot: slot = 16s + 8h + 4a + e  ->  key = 16s + 8a + 4h + e
                 const int slot = kSlotsPer * g + sl;
                 const int h = (slot >> 3) & 1, a = (slot >> 2) & 1, e = slot & 3;
-                w[sl] = v_lds[(slot & ~15) + 8 * a + 4 * h + e][j];
+                w[sl] = lds.v[(slot & ~15) + 8 * a + 4 * h + e][j];
             }
             uint32_t lo_row[kSlotsPer / 2], hi_row[kSlotsPer / 2];
 #pragma unroll
@@ -346,34 +401,27 @@ struct StageQParams {
 // and reused for the batch x head rows share_i, share_i + n_share, ...; a block of 256 threads covers
 // positions 64 blk .. 64 blk + 63
 template <typename T, int kD>
-__device__ inline void stage_q_block(const StageQParams& p, int blk, int share_i, int n_share) {
+__device__ inline void stage_q_block(const StageQParams& p, int blk, int share_i, int n_share, StageLds<kD>& lds) {
     const int64_t idx = (int64_t)blk * 256 + threadIdx.x;
     const int64_t m = idx >> 2;
     const int quarter = idx & 3;
-    if (m >= p.Q) return;
     constexpr int kPieces = kD / 64, kPairs = kD / 8;
     RopeWord<T> rw[kPairs / 2];
     if (p.q_pos) {
-        const int64_t pos = p.q_pos[m];
-#pragma unroll
-        for (int k = 0; k < kPairs / 2; k++) {
-            float sn[2], cs[2];
-#pragma unroll
-            for (int e = 0; e < 2; e++) {
-                const int j = stage_pair(quarter, 2 * k + e);
-                const float f = p.inv_freq ? p.inv_freq[j] : 1.0f / powf(p.theta, (float)(2 * j) / (float)kD);
-                stage_sincos<kD>(__fmul_rn((float)pos, f), &sn[e], &cs[e]);
-            }
-            rw[k] = RopeWord<T>::make(cs[0], sn[0], cs[1], sn[1]);
-        }
+        const int64_t pos = m < p.Q ? p.q_pos[m] : 0;
+        stage_freqs<kD>(p.inv_freq, p.theta, lds);
+        __syncthreads();
+        stage_trig<T, kD>((float)pos, quarter, lds, rw);
     }
+    if (m >= p.Q) return;
     const int64_t nbh = p.rows / p.Q;
     struct Row {
         T lo[kPairs], hi[kPairs];
     };
     auto load_row = [&](int64_t bh, Row& r) {
         if (bh >= nbh) return;
-        const int64_t b = bh / p.H, h = bh % p.H;
+        int64_t h;
+        const int64_t b = div_index(bh, p.H, h);
         const T* src = (const T*)p.q + b * p.stride[0] + h * p.stride[1] + m * p.stride[2];
         if (p.vec) {  // unit stride and 16-byte aligned rows
 #pragma unroll
@@ -436,14 +484,14 @@ struct StageWeights {
 };
 template <typename T, int kD>
 __global__ void __launch_bounds__(256) stage_kernel(StageParams sp, StageQParams sq, StageGrid g, StageWeights sw) {
-    __shared__ uint32_t v_lds[kBN][kD / 2 + 1];  // (d, d + kD/2) pairs of a key row, odd pitch
+    __shared__ __align__(16) StageLds<kD> lds;
     const int nk = g.k_bx * g.k_by;
     int id = blockIdx.x;
     if (id < nk) {
-        stage_keys_block<T, kD>(sp, id % g.k_bx, id / g.k_bx, g.k_by, v_lds);
+        stage_keys_block<T, kD>(sp, id % g.k_bx, id / g.k_bx, g.k_by, lds);
     } else {
         id -= nk;
-        if (id < g.q_bx * g.q_by) stage_q_block<T, kD>(sq, id % g.q_bx, id / g.q_bx, g.q_by);
+        if (id < g.q_bx * g.q_by) stage_q_block<T, kD>(sq, id % g.q_bx, id / g.q_bx, g.q_by, lds);
         else weights_at<T>(sw.w_ema, sw.w_new, sq.Q, sw.beta, (int64_t)(id - g.q_bx * g.q_by) * 256 + threadIdx.x);
     }
 }
@@ -525,7 +573,8 @@ __global__ void __launch_bounds__(512) fwd_pipe_kernel(FwdParams p) {
     // light + heavy everywhere instead of heavy + heavy on the slowest unit).
     qt_i = p.n_qt - 1 - qt_i;
     const int64_t bkv = bkv_i;
-    const int64_t b = bkv / p.KVH, kvh = bkv % p.KVH;
+    int64_t kvh;
+    const int64_t b = div_index(bkv, p.KVH, kvh);
     // rows of a kv head are its (position, head) pairs, position-major: row rf = position * G + head.  A workgroup
     // takes 256 consecutive ones whatever G is (7 heads per kv head: 36 4/7 positions), so every wavefront has
     // 32 real rows and the number of workgroups is Q * G / 256, not Q / floor(256 / G).
@@ -1061,7 +1110,8 @@ __global__ void __launch_bounds__(256) fwd_combine_kernel(FwdParams p) {
         }
     }
     const float inv = 1.f / L;
-    const int64_t m = row % p.Q, h = (row / p.Q) % p.H, b = row / (p.Q * p.H);
+    int64_t m, h;
+    const int64_t b = div_index(div_index(row, p.Q, m), p.H, h);
     T* dst = (T*)p.out + b * p.out_stride[0] + h * p.out_stride[1] + m * p.out_stride[2];
     dst[(4 * d4) * p.out_stride[3]] = Elem<T>::from_float(o.x * inv);
     dst[(4 * d4 + 1) * p.out_stride[3]] = Elem<T>::from_float(o.y * inv);
@@ -1148,7 +1198,8 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
         kb_i /= p.gsplit;
     }
     const int64_t bkv = bkv_i;
-    const int64_t b = bkv / p.KVH, kvh = bkv % p.KVH;
+    int64_t kvh;
+    const int64_t b = div_index(bkv, p.KVH, kvh);
     const int Q = (int)p.Q;
     static_assert(4 * kBN == 256, "a workgroup's keys are four visibility words");
     const int64_t key_blk = (int64_t)kb_i * 256;          // first key of the workgroup
@@ -1538,11 +1589,12 @@ int run_mfma(const MfmaProblem& mp, hipStream_t stream) {
         // always on their way
         int64_t splits = nbh;
         if (mp.shared_pos) {
-            // About two workgroups per compute unit; eight where the keys are gathered by an order: those are not rotated, so
+            // About three workgroups per compute unit (two and three, us: 8 heads x 16897 keys 33.9 and 31.0, 16 x 18496 73 and
+            // 68, 8 x 69696 109 and 109); eight where the keys are gathered by an order: those are not rotated, so
             // there is nothing to reuse from unit to unit, and the tiles of masked keys leave at once (64 heads x 17408 keys,
             // half of them masked: 164 us with two, 139 with eight, 152 with sixteen).
             const int64_t tiles = n_pad / kBN;
-            splits = ((mp.key_order ? 8 : 2) * cus + tiles - 1) / tiles;
+            splits = ((mp.key_order ? 8 : 3) * cus + tiles - 1) / tiles;
             if (splits < 2) splits = 2;
             if (splits > nbh) splits = nbh;
         }

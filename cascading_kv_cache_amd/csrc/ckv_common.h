@@ -86,6 +86,17 @@ struct StageScope {
     }
 };
 
+// Quotient and remainder of indices, which nearly always fit 32 bits: 64-bit division is a long chain of instructions.
+__device__ inline int64_t div_index(int64_t x, int64_t y, int64_t& rem) {
+    if ((((uint64_t)x | (uint64_t)y) >> 32) == 0) {
+        const uint32_t q = (uint32_t)x / (uint32_t)y;
+        rem = (int64_t)((uint32_t)x - q * (uint32_t)y);
+        return (int64_t)q;
+    }
+    rem = x % y;
+    return x / y;
+}
+
 inline int64_t align_up(int64_t v, int64_t a) { return (v + a - 1) / a * a; }
 
 // Facts about the current device, asked of the runtime once per device and process.
@@ -143,6 +154,9 @@ struct RopeWord<__hip_bfloat16> {
     __device__ static RopeWord make(float c0, float s0, float c1, float s1) {
         return RopeWord{pack2(c0, 0.f), pack2(0.f, c1), pack2(s0, 0.f), pack2(0.f, s1)};
     }
+    __device__ static RopeWord of(uint2 w) {  // w: pack2(c0, c1), pack2(s0, s1)
+        return RopeWord{w.x & 0xffffu, w.x & 0xffff0000u, w.y & 0xffffu, w.y & 0xffff0000u};
+    }
     __device__ static float dot(uint32_t a, uint32_t b) {
         return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(ckv_bf16x2, a), __builtin_bit_cast(ckv_bf16x2, b), 0.f, false);
     }
@@ -170,6 +184,7 @@ struct RopeWord<__half> {
     __device__ static float lo(uint32_t w) { return (float)__builtin_bit_cast(ckv_f16x2, w)[0]; }
     __device__ static float hi(uint32_t w) { return (float)__builtin_bit_cast(ckv_f16x2, w)[1]; }
     __device__ static RopeWord make(float c0, float s0, float c1, float s1) { return RopeWord{pack2(c0, c1), pack2(s0, s1)}; }
+    __device__ static RopeWord of(uint2 w) { return RopeWord{w.x, w.y}; }  // w: pack2(c0, c1), pack2(s0, s1)
     __device__ void rotate(uint32_t w1, uint32_t w2, float post, bool scaled, uint32_t& o1, uint32_t& o2) const {
 #pragma clang fp contract(off)  // a fused multiply-add would skip the rounding of the product
         const ckv_f16x2 x1 = __builtin_bit_cast(ckv_f16x2, w1), x2 = __builtin_bit_cast(ckv_f16x2, w2);
