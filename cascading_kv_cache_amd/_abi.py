@@ -114,7 +114,7 @@ def set_strides(field, tensor_or_strides):
 def same_layout(a, b) -> bool:
     """Equal shapes and equal strides on every dimension that is actually stepped through
     (the stride of a size-1 dimension is arbitrary in torch)."""
-    return a.shape == b.shape and all(sa == sb for n, sa, sb in zip(a.shape, a.stride(), b.stride()) if n > 1)
+    return a.shape == b.shape and (a.stride() == b.stride() or all(sa == sb for n, sa, sb in zip(a.shape, a.stride(), b.stride()) if n > 1))
 
 
 def fill_update_args(k, v, s, sink_k, sink_v, sink_mask, sink_pos, cache_k, cache_v, cache_s, mask, pos,

@@ -15,7 +15,7 @@ import torch
 from torch import nn
 
 from . import _abi
-from .cascading_cache import CascadingKVCache, _require_device, workspace
+from .cascading_cache import CascadingKVCache, _require_device, on_device, raw_stream, workspace
 
 
 _DEBUG_COUNTERS = os.environ.get("CKV_DEBUG_COUNTERS", "0") not in ("", "0")
@@ -179,8 +179,8 @@ def cascade_attention(query_states, key_states, value_states, cache: CascadingKV
     if scale is None:
         scale = 1 / math.sqrt(D)
 
-    with torch.cuda.device(dev):
-        stream = torch.cuda.current_stream(dev).cuda_stream
+    with on_device(dev):
+        stream = raw_stream(dev)
         q_pos = chunk_positions(cache, L, Q, do_og_pos, _stream=stream, _replayable=replayable)
         out = torch.empty((B, H, Q, D), dtype=dtype, device=dev)
         new_scores = torch.empty((B, KVH, Q), dtype=dtype, device=dev)
@@ -196,6 +196,7 @@ def cascade_attention(query_states, key_states, value_states, cache: CascadingKV
             check_against_cache(query_states, key_states, value_states, cache, L)
             a = _describe_attention(query_states, key_states, value_states, cache, L, inv_freq, reduction,
                                     homogeneous_heads, do_og_pos, scale, out, new_scores)
+            a._update = None
             if len(cache._attn_memo) > 64:
                 cache._attn_memo.clear()
             cache._attn_memo[key] = a
@@ -213,8 +214,10 @@ def cascade_attention(query_states, key_states, value_states, cache: CascadingKV
         a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
         _abi.check(lib.ckv_attn(C.byref(a), C.c_void_p(stream)), "ckv_attn")
         if update_cache:
+            if a._update is None:  # of the layouts and placements that the key above holds
+                a._update = cache._update_args(key_states, value_states, new_scores, L)
             cache.update_state(key_states, value_states, L, score_states=new_scores, _stream=stream,
-                               _device_counter=replayable)
+                               _device_counter=replayable, _args=a._update)
     return out, new_scores
 
 

@@ -6,6 +6,7 @@
 (cascade/models/cascading_cache.py:1031-1348) without depending on ``transformers``.
 There is no CPU path: tensors must live on a HIP device and the library must be built.
 """
+import contextlib
 import ctypes as C
 from typing import List, Optional, Union
 
@@ -44,6 +45,19 @@ def workspace(device: torch.device, nbytes: int, stream: int = 0) -> Tensor:
         buf = torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
         _WORKSPACES[key] = buf
     return buf
+
+
+_SAME_DEVICE = contextlib.nullcontext()
+
+
+def on_device(device: torch.device):
+    """``torch.cuda.device(device)``, which costs a single-token step 1.4 us of host time, where another device is current."""
+    return _SAME_DEVICE if torch.cuda.current_device() == device.index else torch.cuda.device(device)
+
+
+def raw_stream(device: torch.device) -> int:
+    """The handle of the current stream of ``device``, without the stream object (0.1 instead of 1.9 us)."""
+    return torch._C._cuda_getCurrentRawStream(device.index)
 
 
 def _require_device(t: Tensor, what: str):
@@ -365,14 +379,15 @@ class CascadingKVCache:
         return a
 
     def update_state(self, key_states: Tensor, value_states: Tensor, layer_idx: int, score_states: Tensor = None,
-                     _stream: Optional[int] = None, _device_counter: bool = False):
+                     _stream: Optional[int] = None, _device_counter: bool = False, _args=None):
         """``update`` without building the tuple of views it returns (the shifted position row of
         ``get_vals`` is a device operation of its own); for callers that read the state in place.
 
         The argument block of ``ckv_update`` is described once per layer and input layout and reused:
         between two calls of the same shape only the three input pointers change (single-token steps
         at batch 1 are bound by this host code, not by the device).  ``_stream``: raw stream handle when
-        the caller already holds the device context.
+        the caller already holds the device context.  ``_args``: the argument block that ``_update_args`` gave for
+        these layouts, when the caller has looked up by layouts and placements that determine it.
 
         The update reads the number of tokens seen so far from device memory (``real_token_idx``).  The host knows
         that number, so the call points the library at the element of a constant table ``0, 1, 2, ...`` that holds
@@ -386,7 +401,11 @@ class CascadingKVCache:
         if layer_idx == 0:
             self._seen_tokens += key_states.shape[-2]
 
-        a = self._update_args(key_states, value_states, score_states, layer_idx)
+        a = _args
+        if a is None:
+            a = self._update_args(key_states, value_states, score_states, layer_idx)
+        else:
+            a.k, a.v, a.s = key_states.data_ptr(), value_states.data_ptr(), score_states.data_ptr()
         n_new = key_states.shape[-2]
         table = None if _device_counter else _counter_table(key_states.device)
         if table is not None and self._seen_host[layer_idx] < table.numel():
@@ -396,8 +415,8 @@ class CascadingKVCache:
             self._flush_counter()
             a.real_token_idx = a._counter
         if _stream is None:
-            with torch.cuda.device(key_states.device):
-                stream = torch.cuda.current_stream(key_states.device).cuda_stream
+            with on_device(key_states.device):
+                stream = raw_stream(key_states.device)
                 ws = workspace(key_states.device, a._need, stream)
                 a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
                 _abi.check(_abi.lib().ckv_update(C.byref(a), C.c_void_p(stream)), "ckv_update")
