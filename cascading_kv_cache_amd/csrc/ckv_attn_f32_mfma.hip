@@ -3,15 +3,23 @@
 // The float32 matrix instructions multiply and accumulate in float32 (every product enters the accumulator through a
 // fused multiply-add), at twice the rate of the vector ALU and with one operand register per lane instead of LDS reads
 // per product, which is what bounded the vector kernels (ckv_attn_generic.hip keeps them for the shapes that do not
-// fit here).  32 heads x 256 rows x 516 + 256 keys x 128: forward 269 -> 49 us, scores 321 -> 34 us.
+// fit here).  32 heads x 256 rows x 516 + 256 keys x 128: forward 269 -> 45 us, scores 321 -> 31 us.  Both are bound by the
+// products and the vector work together: vector instructions do not run beside these products (a tile's exponentials take
+// 5700 cycles next to the other wavefront's 64 products, which take 4400 alone, and 1700 by themselves), so what is not
+// arithmetic of the attention -- masks of whole blocks, addresses of rows -- is kept off the vector pipe.
 //
 //   forward  one workgroup = one kv head x 32 (position, head) rows; its eight wavefronts take the 32-key blocks in
 //            turn, each with an online softmax of its own, and merge at the end through LDS.  S^T = K Q^T keeps a query
 //            in one lane pair, and register v of S^T is, as it stands, the B operand of step v of O^T += V^T P^T: nothing
-//            is moved between the two products.  Keys and values go from memory straight to the operand registers (no
-//            two wavefronts of a workgroup share any); the queries sit in LDS in operand order.
-//   colsum   one workgroup = one head x 32 keys, held in registers; its four wavefronts take the 32-row query tiles in
-//            turn.  S = Q K^T keeps a key in one lane pair, so a weighted sum stays in its lane until the end.
+//            is moved between the two products.  Values go from memory straight to the operand registers (no two
+//            wavefronts of a workgroup share any), keys through LDS, as operand pieces of 32 rows touch 32 lines of the
+//            first-level cache at a time; the queries sit in LDS in operand order.  With keys straight to registers and
+//            the addresses worked out per lane the forward took 47.7 us.
+//   colsum   one workgroup = one head x four blocks of 32 keys, held in registers (one block where that makes too few
+//            workgroups); two streams of its wavefronts take the 32-row query tiles, which come through LDS, in turn.
+//            S = Q K^T keeps a key in one lane pair, so a weighted sum stays in its lane until the end.  With a block of
+//            keys a workgroup and queries straight to registers the scores took 34 us (28 heads x 2568 keys, 512 rows: 156,
+//            now 130), with a barrier a tile 31.3.
 //
 // A matrix instruction multiplies every row of a tile by every value, and zero times infinity or NaN is NaN, while a value
 // whose key has probability zero counts for nothing, whatever it holds (the vector kernels do not touch it).  So a wavefront
@@ -23,6 +31,8 @@
 // dims 8 c + e (lanes 0..31) and 8 c + 4 + e (lanes 32..63), so that an operand is a 16-byte load per four steps.
 #include "ckv_attn_internal.h"
 
+#include <type_traits>
+
 namespace ckv {
 namespace {
 
@@ -30,7 +40,14 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int kRows = 32;      // query rows of a forward workgroup
 constexpr int kKeys = 32;      // keys of a block
-constexpr int kFwdWaves = 8, kColWaves = 4;
+constexpr int kFwdWaves = 8;
+constexpr int kColSums = 4;    // partial sums of a key, one per query tile mod 4
+// a workgroup of the score sums: blocks of keys it takes, and streams of query tiles, each a wavefront per block of keys
+template <int kGroups>
+struct Col {
+    static constexpr int kStreams = kGroups == 1 ? 4 : 2, kWaves = kGroups * kStreams, kBlockKeys = kGroups * kKeys;
+    static constexpr int kAcc = kColSums / kStreams;   // partial sums of a wavefront
+};
 
 template <int D>
 struct Geo {
@@ -39,6 +56,11 @@ struct Geo {
     static constexpr int kPitch = D + 4;    // floats of a row in the merge area
     static constexpr int kQ = kPieces * CKV_WAVE * 16;
     static constexpr int kFwdLds = kQ + kFwdWaves * kRows * kPitch * 4 + 2 * kFwdWaves * kRows * 4;
+    // 32 rows in LDS as asynchronous copies of 1 KiB bring them: 16-byte piece c of row r in slot c ^ (r mod slots), so that one
+    // piece of 16 consecutive rows covers all banks
+    static constexpr int kSlots = D / 4, kTile = 32 * D * 4, kCopies = kTile / 1024;
+    static_assert(kFwdWaves * kTile <= kFwdWaves * kRows * kPitch * 4, "the key blocks lie where the shares are merged");
+    __device__ static int slot(int r, int c) { return c ^ (r & (kSlots - 1)); }
 };
 
 template <int N>
@@ -86,16 +108,6 @@ __global__ void __launch_bounds__(kFwdWaves* CKV_WAVE) fwd_f32_mfma_kernel(F32Fw
     const float* kb = (const float*)p.k + b * p.kv_stride[0] + kvh * p.kv_stride[1];
     const float* vb = (const float*)p.v + b * p.kv_stride[0] + kvh * p.kv_stride[1];
 
-    for (int i = tid; i < NP * CKV_WAVE; i += kFwdWaves * CKV_WAVE) {
-        const int rf = rt * kRows + (i & 31), m = rf / G, g = rf % G;
-        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (m < Q)
-            v = *reinterpret_cast<const float4*>((const float*)p.q + b * p.q_stride[0] + (kvh * G + g) * p.q_stride[1] +
-                                                 m * p.q_stride[2] + 8 * (i >> 6) + 4 * ((i >> 5) & 1));
-        q_lds[i] = v;
-    }
-    __syncthreads();
-
     const int row_m = (rt * kRows + col) / G;            // this lane's query
     int m_hi = (rt * kRows + kRows - 1) / G;
     if (m_hi > Q - 1) m_hi = Q - 1;
@@ -103,15 +115,16 @@ __global__ void __launch_bounds__(kFwdWaves* CKV_WAVE) fwd_f32_mfma_kernel(F32Fw
     // bit r: key r of the block is there and not masked
     auto visible_keys = [&](int n) { return (uint32_t)__ballot(n < Nc ? !(p.kmasked && p.kmasked[n]) : n < N); };
     // the logits of a block's keys (lane = its query), and the keys this lane's query sees
-    auto logits = [&](const float4(&kf)[NP]) {
+    auto logits = [&](auto&& key_piece) {
         f32x16 s = zero16();
 #pragma unroll
         for (int c = 0; c < NP; c++) {
-            const float4 q4 = q_lds[c * CKV_WAVE + lane];
-            s = mma(kf[c].x, q4.x, s);
-            s = mma(kf[c].y, q4.y, s);
-            s = mma(kf[c].z, q4.z, s);
-            s = mma(kf[c].w, q4.w, s);
+            if (c % 4 == 0) __builtin_amdgcn_sched_barrier(0);   // eight operand reads ahead, not all of them
+            const float4 k4 = key_piece(c), q4 = q_lds[c * CKV_WAVE + lane];
+            s = mma(k4.x, q4.x, s);
+            s = mma(k4.y, q4.y, s);
+            s = mma(k4.z, q4.z, s);
+            s = mma(k4.w, q4.w, s);
         }
         return s;
     };
@@ -120,6 +133,34 @@ __global__ void __launch_bounds__(kFwdWaves* CKV_WAVE) fwd_f32_mfma_kernel(F32Fw
         const int last = Nc + row_m - n0;   // last key of the block the row may see
         return vis & (last >= 31 ? ~0u : (last < 0 ? 0u : (2u << last) - 1u));   // cached keys lie in front of the chunk keys: row_m >= 0 lets them all through
     };
+    const bool near = p.kv_stride[2] >= 0 && p.kv_stride[2] < (1 << 24);   // offsets of a few rows fit 32 bits
+    const uint32_t row_bytes = (uint32_t)p.kv_stride[2] * 4u;
+    // the wavefront's block of keys in LDS
+    unsigned char* k_lds = reinterpret_cast<unsigned char*>(o_lds) + wave * G_::kTile;
+    const uint32_t k_at = lds_address(k_lds);
+    auto copy_keys = [&](int n0) {
+        constexpr int kRowsPer = CKV_WAVE / G_::kSlots;   // rows of a copy
+        const int r0 = lane / G_::kSlots;
+        int c0 = G_::slot(r0, lane % G_::kSlots);
+        asm volatile("" : "+v"(c0));   // worked out again each time: sixteen kept offsets are sixteen registers
+        if (near && n0 + kKeys <= N) {
+            // the block's rows from a uniform address: vector instructions do not run beside float32 products
+            const uint32_t row = (uint32_t)r0 * row_bytes;
+            const float* from = kb + (int64_t)n0 * p.kv_stride[2];
+#pragma unroll
+            for (int j = 0; j < G_::kCopies; j++)
+                async_copy16(from + (int64_t)(j * kRowsPer) * p.kv_stride[2], row + 16u * (uint32_t)G_::slot(j * kRowsPer, c0), k_at + j * 1024);
+        } else {
+#pragma unroll
+            for (int j = 0; j < G_::kCopies; j++) {
+                const int n = n0 + r0 + j * kRowsPer, c = G_::slot(j * kRowsPer, c0);
+                async_copy16_from(kb + (int64_t)(n < N ? n : N - 1) * p.kv_stride[2] + 4 * c, k_at + j * 1024);
+            }
+        }
+    };
+    auto read_keys = [&](int c) {
+        return *reinterpret_cast<const float4*>(k_lds + col * (D * 4) + G_::slot(col, 2 * c + half) * 16);
+    };
     auto load_keys = [&](int n, float4(&kf)[NP]) {
         const float* kr = kb + (int64_t)(n < N ? n : N - 1) * p.kv_stride[2] + 4 * half;
 #pragma unroll
@@ -127,40 +168,115 @@ __global__ void __launch_bounds__(kFwdWaves* CKV_WAVE) fwd_f32_mfma_kernel(F32Fw
     };
     // values of the lane's half of the keys, dims DB col .. DB col + DB - 1: accumulator db holds dims DB m + db
     auto load_values = [&](int n0, Vec<DB>(&vf)[16]) {
+        if (near && n0 + kKeys <= N) {
+            const uint32_t at = (uint32_t)(4 * half) * row_bytes + (uint32_t)(DB * col * 4);
+            const char* from = reinterpret_cast<const char*>(vb + (int64_t)n0 * p.kv_stride[2]);
+#pragma unroll
+            for (int v = 0; v < 16; v++)
+                vf[v] = *reinterpret_cast<const Vec<DB>*>(from + (int64_t)acc_row(v, 0) * p.kv_stride[2] * 4 + at);
+            return;
+        }
 #pragma unroll
         for (int v = 0; v < 16; v++) {
             const int nv = n0 + acc_row(v, half);
             vf[v] = *reinterpret_cast<const Vec<DB>*>(vb + (int64_t)(nv < N ? nv : N - 1) * p.kv_stride[2] + DB * col);
         }
     };
+    // A wavefront's blocks blk, blk + step, ...  The next one with a visible key is requested as soon as this one's place is free:
+    // its keys behind the logits, its values behind the second product.  So a wavefront waits for memory once, at its first
+    // block, which is requested with the queries and before its mask is known (nearly always wanted, and in bounds).
+    // Loads and copies retire in issue order; "at most n outstanding" below counts what was issued behind the wanted ones.
+    const int step = kFwdWaves * f.n_split;
+    auto mask_byte = [&](int n) -> int { return n < Nc ? (p.kmasked ? p.kmasked[n] : 0) : n < N ? 0 : 1; };
+    int blk = split * kFwdWaves + wave;
+    int hidden = blk < nblk ? mask_byte(blk * kKeys + col) : 1;
+    Vec<DB> vf[16];
+    constexpr int kValueLoads = 16;
+    {
+#pragma unroll
+        for (int t = 0; t < NP / kFwdWaves; t++) {
+            const int c = t * kFwdWaves + wave, rf = rt * kRows + col, m = rf / G, g = rf % G;
+            if (m < Q)
+                async_copy16_from((const float*)p.q + b * p.q_stride[0] + (kvh * G + g) * p.q_stride[1] + m * p.q_stride[2] + 8 * c + 4 * half,
+                                  lds_address(q_lds) + c * (CKV_WAVE * 16));
+            else
+                q_lds[c * CKV_WAVE + lane] = make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+        if (blk < nblk) {
+            copy_keys(blk * kKeys);
+            load_values(blk * kKeys, vf);
+            wait_copies<G_::kCopies + kValueLoads>();
+        } else {
+            wait_copies<0>();
+        }
+    }
+    // a barrier of the language would wait for the keys and values too
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
     f32x16 o[DB];
 #pragma unroll
     for (int db = 0; db < DB; db++) o[db] = zero16();
     float m_run = -INFINITY, l_run = 0.f;
-    for (int blk = split * kFwdWaves + wave; blk < nblk; blk += kFwdWaves * f.n_split) {
+    uint32_t vis = (uint32_t)__ballot(hidden == 0);
+    // on to a block with a visible key, if there is one
+    auto skip_hidden = [&]() {
+        while (vis == 0u && blk + step < nblk) {
+            blk += step;
+            vis = visible_keys(blk * kKeys + col);
+        }
+    };
+    if (blk < nblk && vis == 0u) {
+        skip_hidden();
+        wait_copies<0>();   // also where nothing follows: the shares are merged in this LDS
+        if (vis != 0u) {
+            copy_keys(blk * kKeys);
+            load_values(blk * kKeys, vf);
+        }
+    }
+    while (vis != 0u) {
         const int n0 = blk * kKeys;
-        const int n = n0 + col;
-        const uint32_t vis = visible_keys(n);
-        if (vis == 0u) continue;
-        float4 kf[NP];
-        load_keys(n, kf);
-        Vec<DB> vf[16];
-        load_values(n0, vf);
-        f32x16 s = logits(kf);
-        const uint32_t allow = seen_keys(vis, n0);   // bit r: key r of the block is visible to this lane's query
+        const uint32_t vis_now = vis;
+        wait_copies<kValueLoads>();   // the keys are there
+        const bool more = blk + step < nblk;
+        hidden = more ? mask_byte((blk + step) * kKeys + col) : 1;
+        f32x16 s = logits(read_keys);
+        // the values have arrived (under the logits): what the compiler would wait for behind the next copies are those too
+#pragma unroll
+        for (int v = 0; v < 16; v++)
+#pragma unroll
+            for (int db = 0; db < DB; db++) asm volatile("" : "+v"(vf[v].v[db]));
+        vis = (uint32_t)__ballot(hidden == 0);
+        if (more) {
+            blk += step;
+            skip_hidden();
+        }
+        if (vis != 0u) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the keys have been read
+            copy_keys(blk * kKeys);
+        }
+        const uint32_t allow = seen_keys(vis_now, n0);   // bit r: key r of the block is visible to this lane's query
         const bool whole = __ballot(allow != ~0u) == 0ull;
         float mx = -INFINITY;
+        if (whole) {
 #pragma unroll
-        for (int v = 0; v < 16; v++) {
-            const float x = s[v] * p.scale;
-            s[v] = whole || ((allow >> acc_row(v, half)) & 1u) ? x : -INFINITY;
-            mx = fmaxf(mx, s[v]);
+            for (int v = 0; v < 16; v++) {
+                s[v] *= p.scale;
+                mx = fmaxf(mx, s[v]);
+            }
         }
-        if (!whole) {   // the row of a key nobody sees may hold anything
+        asm volatile("");   // two branches, not one with an alternative: the registers of the rare one are not kept for the other
+        if (!whole) {
+#pragma unroll
+            for (int v = 0; v < 16; v++) {
+                s[v] = (allow >> acc_row(v, half)) & 1u ? s[v] * p.scale : -INFINITY;
+                mx = fmaxf(mx, s[v]);
+            }
+            // the row of a key nobody sees may hold anything
 #pragma unroll
             for (int v = 0; v < 16; v++)
 #pragma unroll
-                for (int db = 0; db < DB; db++) vf[v].v[db] = (vis >> acc_row(v, half)) & 1u ? vf[v].v[db] : 0.f;
+                for (int db = 0; db < DB; db++) vf[v].v[db] = (vis_now >> acc_row(v, half)) & 1u ? vf[v].v[db] : 0.f;
         }
         mx = fmaxf(mx, __shfl_xor(mx, 32));
         const float m_new = fmaxf(m_run, mx);
@@ -184,6 +300,10 @@ __global__ void __launch_bounds__(kFwdWaves* CKV_WAVE) fwd_f32_mfma_kernel(F32Fw
         for (int v = 0; v < 16; v++)
 #pragma unroll
             for (int db = 0; db < DB; db++) o[db] = mma(vf[v].v[db], s[v], o[db]);
+        if (vis != 0u) {
+            asm volatile("" ::: "memory");   // behind the copies of the keys
+            load_values(blk * kKeys, vf);
+        }
     }
 
     float zero = 0.f;   // or NaN
@@ -202,7 +322,7 @@ __global__ void __launch_bounds__(kFwdWaves* CKV_WAVE) fwd_f32_mfma_kernel(F32Fw
             {
                 float4 kf[NP];
                 load_keys(n0 + col, kf);
-                s = logits(kf);
+                s = logits([&](int c) { return kf[c]; });
             }
             const uint32_t allow = seen_keys(vis, n0);
 #pragma unroll
@@ -325,69 +445,129 @@ __global__ void __launch_bounds__(256) fwd_f32_combine_kernel(F32Fwd f) {
     if (d4 == 0 && p.lse) p.lse[row] = M + logf(L);
 }
 
-template <int D>
-__global__ void __launch_bounds__(kColWaves* CKV_WAVE, 2) colsum_f32_mfma_kernel(CoreProblem p) {
-    constexpr int NP = Geo<D>::kPieces;
-    __shared__ float sums[kColWaves][kKeys];
+template <int D, int kGroups>
+__global__ void __launch_bounds__(Col<kGroups>::kWaves* CKV_WAVE, 2) colsum_f32_mfma_kernel(CoreProblem p) {
+    constexpr int kColGroups = kGroups, kColStreams = Col<kGroups>::kStreams, kColWaves = Col<kGroups>::kWaves, kColKeys = Col<kGroups>::kBlockKeys;
+    constexpr int kAcc = Col<kGroups>::kAcc;
+    constexpr int NP = Geo<D>::kPieces, kSlots = Geo<D>::kSlots, kTile = Geo<D>::kTile;
+    extern __shared__ __attribute__((aligned(16))) float lds[];   // kColWaves tiles of 32 queries
+    __shared__ float sums[kColSums][kColKeys];
     const int tid = threadIdx.x, lane = tid & 63, col = lane & 31, half = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int group = wave % kColGroups, stream = wave / kColGroups;
     const int nbkv = (int)(p.B * p.KVH), KVH = (int)p.KVH, G = (int)p.H / KVH;
-    const int N = (int)p.N, Q = (int)p.Q, Nc = N - Q, nblk = (N + kKeys - 1) / kKeys;
+    const int N = (int)p.N, Q = (int)p.Q, Nc = N - Q, nblk = (N + kColKeys - 1) / kColKeys;
     // kv heads round the XCDs; blocks of chunk keys see fewer rows and come last
     const int bkv = blockIdx.x % nbkv, rest = blockIdx.x / nbkv;
     const int g = rest % G, blk = rest / G;
     if (blk >= nblk) return;
     const int64_t b = bkv / KVH, kvh = bkv % KVH, h = kvh * G + g;
-    const int n0 = blk * kKeys, n = n0 + col, nrel = n - Nc;   // nrel >= 0: a chunk key
-    const bool live = n < N && !(n < Nc && p.kmasked && p.kmasked[n]);
-    float acc = 0.f;
-    if (__ballot(live) != 0ull) {
-        float4 kf[NP];
+    const int n0 = blk * kColKeys + group * kKeys, n = n0 + col, nrel = n - Nc;   // nrel >= 0: a chunk key
+    const int masked = n < Nc && p.kmasked ? p.kmasked[n] : 0;
+    const float* qb = (const float*)p.q + b * p.q_stride[0] + h * p.q_stride[1];
+    const float* lse = p.lse + (b * p.H + h) * p.Q;
+    const int blk0 = blk * kColKeys;
+    const int t_first = blk0 > Nc ? (blk0 - Nc) / kRows : 0;   // first tile with a row that sees a key of the workgroup
+    const int t_own = n0 > Nc ? (n0 - Nc) / kRows : 0;         // ... of this wavefront
+    const int n_tiles = (Q + kRows - 1) / kRows;
+    // a wavefront copies a tile of the next kColWaves ones
+    const unsigned char* q_lds = reinterpret_cast<const unsigned char*>(lds);
+    auto copy_queries = [&](int t) {
+#pragma unroll
+        for (int j = 0; j < Geo<D>::kCopies; j++) {
+            const int piece = j * CKV_WAVE + lane, r = piece / kSlots, m = t * kRows + r;
+            async_copy16_from(qb + (int64_t)(m < Q ? m : Q - 1) * p.q_stride[2] + 4 * Geo<D>::slot(r, piece % kSlots),
+                              lds_address(lds) + wave * kTile + j * 1024);
+        }
+    };
+    if (t_first + wave < n_tiles) copy_queries(t_first + wave);
+    float4 kf[NP];
+    {
         const float* kr = (const float*)p.k + b * p.kv_stride[0] + kvh * p.kv_stride[1] +
                           (int64_t)(n < N ? n : N - 1) * p.kv_stride[2] + 4 * half;
 #pragma unroll
         for (int c = 0; c < NP; c++) kf[c] = *reinterpret_cast<const float4*>(kr + 8 * c);
-        const float* qb = (const float*)p.q + b * p.q_stride[0] + h * p.q_stride[1];
-        const float* lse = p.lse + (b * p.H + h) * p.Q;
-        const int t0 = n0 > Nc ? (n0 - Nc) / kRows : 0;   // first tile with a row that sees a key of the block
-        for (int mt = (t0 + wave) * kRows; mt < Q; mt += kColWaves * kRows) {
-            float4 qf[NP];
-            const float* qr = qb + (int64_t)(mt + col < Q ? mt + col : Q - 1) * p.q_stride[2] + 4 * half;
+    }
+    const bool live = n < N && masked == 0;
+    const bool wanted = __ballot(live) != 0ull;
+    const bool chunk_keys = n0 + kKeys > Nc, by_distance = nrel >= 0 && p.new_mode;
+    float acc[kAcc] = {};   // of this stream's tiles with the same (t - t_own) mod 4; of a key nobody sees, anything
+    const int t_end = __syncthreads_or(wanted) ? n_tiles : t_first;
+    for (int t0 = t_first; t0 < t_end; t0 += kColWaves) {
+        if (t0 > t_first) {
+            __syncthreads();   // the tiles before have been read
+            if (t0 + wave < n_tiles) copy_queries(t0 + wave);
+        }
+        wait_copies<0>();
+        __syncthreads();
+        // each stream takes every other tile, at its own pace: with a barrier a tile, the vector work of one of the two
+        // wavefronts of a SIMD waits for the products of the other and then has the SIMD to itself
+        for (int t = t0 + stream; t < t0 + kColWaves && t < n_tiles; t += kColStreams) {
+            if (!wanted || t < t_own) continue;
+            // whole tiles of rows that all see the keys: normalisers and weights in 16-byte pieces, and no comparisons (vector
+            // instructions do not run beside float32 products)
+            const bool whole = !chunk_keys && t * kRows + kRows <= Q;
+            Vec<4> ls[4], w[4];
 #pragma unroll
-            for (int c = 0; c < NP; c++) qf[c] = *reinterpret_cast<const float4*>(qr + 8 * c);
-            float ls[16];
+            for (int i4 = 0; i4 < 4; i4++) {
+                const int m0 = t * kRows + 8 * i4 + 4 * half;
+                if (whole) {
+                    ls[i4] = *reinterpret_cast<const Vec<4>*>(lse + m0);
+                    w[i4] = *reinterpret_cast<const Vec<4>*>(p.w_ema + m0);
+                } else {
 #pragma unroll
-            for (int v = 0; v < 16; v++) {
-                const int m = mt + acc_row(v, half);
-                ls[v] = lse[m < Q ? m : Q - 1];
+                    for (int e = 0; e < 4; e++) {
+                        const int m = m0 + e < Q ? m0 + e : Q - 1, d = m - nrel;
+                        ls[i4].v[e] = lse[m];
+                        w[i4].v[e] = by_distance ? p.w_new[d > 0 ? d : 0] : p.w_ema[m];
+                    }
+                }
             }
             f32x16 s = zero16();
+            const unsigned char* tile = q_lds + (t - t0) * kTile + col * (D * 4);
 #pragma unroll
             for (int c = 0; c < NP; c++) {
-                s = mma(qf[c].x, kf[c].x, s);
-                s = mma(qf[c].y, kf[c].y, s);
-                s = mma(qf[c].z, kf[c].z, s);
-                s = mma(qf[c].w, kf[c].w, s);
+                const float4 q4 = *reinterpret_cast<const float4*>(tile + Geo<D>::slot(col, 2 * c + half) * 16);
+                s = mma(q4.x, kf[c].x, s);
+                s = mma(q4.y, kf[c].y, s);
+                s = mma(q4.z, kf[c].z, s);
+                s = mma(q4.w, kf[c].w, s);
             }
-            const bool by_distance = nrel >= 0 && p.new_mode;
+            const bool second = kAcc == 2 && ((t - t_own) & 2);
+            float a = second ? acc[kAcc - 1] : acc[0];
+            if (whole) {
 #pragma unroll
-            for (int v = 0; v < 16; v++) {
-                const int m = mt + acc_row(v, half);
-                const bool seen = live && m < Q && m >= nrel;
-                const int d = m - nrel;
-                const float w = by_distance ? p.w_new[seen ? d : 0] : p.w_ema[m < Q ? m : Q - 1];
-                if (seen) acc = fmaf(w, expf(s[v] * p.scale - ls[v]), acc);
+                for (int v = 0; v < 16; v++) a = fmaf(w[v >> 2].v[v & 3], expf(s[v] * p.scale - ls[v >> 2].v[v & 3]), a);
             }
+            asm volatile("");
+            if (!whole) {
+#pragma unroll
+                for (int v = 0; v < 16; v++) {
+                    const int m = t * kRows + acc_row(v, half);
+                    const float x = fmaf(w[v >> 2].v[v & 3], expf(s[v] * p.scale - ls[v >> 2].v[v & 3]), a);
+                    a = m < Q && m >= nrel ? x : a;
+                }
+            }
+            if (second) acc[kAcc - 1] = a;
+            else acc[0] = a;
         }
     }
-    acc += __shfl_xor(acc, 32);
-    if (half == 0) sums[wave][col] = acc;
+    wait_copies<0>();   // none is on its way to LDS that is somebody else's by then
+    // the sums of tiles t_own + i, + 4, ... for i = 0 .. 3, added in that order
+    const int class0 = (t_first + stream - t_own) & (kColStreams - 1);
+#pragma unroll
+    for (int i = 0; i < kAcc; i++) {
+        acc[i] += __shfl_xor(acc[i], 32);
+        if (!live) acc[i] = 0.f;
+        if (half == 0) sums[class0 + kColStreams * i][group * kKeys + col] = acc[i];
+    }
     __syncthreads();
-    if (tid < kKeys && n < N) {
+    const int nt = blk0 + tid;
+    if (tid < kColKeys && nt < N) {
         float tot = 0.f;
 #pragma unroll
-        for (int w = 0; w < kColWaves; w++) tot += sums[w][tid];
-        p.colsum[(b * p.H + h) * p.N + n] = tot;
+        for (int i = 0; i < kColSums; i++) tot += sums[i][tid];
+        p.colsum[(b * p.H + h) * p.N + nt] = tot;
     }
 }
 
@@ -414,8 +594,21 @@ int run(const CoreProblem& p, float* part_o, float* part_l, hipStream_t stream) 
     }
     if (p.colsum) {
         StageScope sc(CKV_STAGE_SCORES, stream);
-        const int64_t blocks = p.B * p.H * ((p.N + kKeys - 1) / kKeys);
-        hipLaunchKernelGGL(colsum_f32_mfma_kernel<D>, dim3((unsigned)blocks), dim3(kColWaves * CKV_WAVE), 0, stream, p);
+        // Four blocks of keys share their workgroup's query tiles, unless that leaves more than a quarter of the chip idle (28 heads
+        // x 276 and 32 x 360 keys, 16 and 100 rows, 84 and 96 workgroups: 9.6 and 17.5 us against 7.8 and 12.3 with one block each;
+        // 32 x 776 keys, 256 rows, 224 workgroups: 30.7 against 34, 28 x 2568 keys, 512 rows: 130 against 156).
+        auto launch = [&](auto groups) -> int {
+            using C_ = Col<groups.value>;
+            auto kernel = colsum_f32_mfma_kernel<D, groups.value>;
+            const int lds = C_::kWaves * Geo<D>::kTile;
+            if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(kernel), lds)) return rc;
+            const int64_t blocks = p.B * p.H * ((p.N + C_::kBlockKeys - 1) / C_::kBlockKeys);
+            hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(C_::kWaves * CKV_WAVE), lds, stream, p);
+            return CKV_OK;
+        };
+        const int64_t shared = p.B * p.H * ((p.N + Col<4>::kBlockKeys - 1) / Col<4>::kBlockKeys);
+        if (int rc = 4 * shared >= 3 * (int64_t)mfma_device_cus() ? launch(std::integral_constant<int, 4>{})
+                                                                    : launch(std::integral_constant<int, 1>{})) return rc;
         CKV_HIP_TRY(hipGetLastError());
     }
     return CKV_OK;

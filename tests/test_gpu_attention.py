@@ -737,6 +737,17 @@ def test_float32_on_the_matrix_cores(D, H, KVH, W, C, steps):
     run_teacher_forced(B=2, H=H, KVH=KVH, D=D, NS=4, W=W, C=C, Q=0, chunks=0, dtype=torch.float32, seed=41, steps=steps)
 
 
+@pytest.mark.parametrize("D,H,KVH,W,C,steps", [
+    (64, 32, 8, 96, 3, [290, 257, 33, 2]),   # four blocks of 32 keys a workgroup, more than eight tiles of rows, hidden blocks first
+    (128, 28, 4, 96, 3, [97, 31, 64, 3]),    # up to four tiles; keys that end inside a workgroup's blocks
+    (128, 4, 4, 24, 2, [161, 32, 3]),        # one block a workgroup, six tiles of rows by four streams
+])
+def test_float32_score_sums_shared_out(D, H, KVH, W, C, steps):
+    """The float32 score sums take one or four blocks of keys a workgroup, whichever leaves less of the chip idle, and the
+    query tiles by streams that start at the first tile a block's keys can be seen from.  As the test above."""
+    run_teacher_forced(B=2, H=H, KVH=KVH, D=D, NS=5, W=W, C=C, Q=0, chunks=0, dtype=torch.float32, seed=43, steps=steps)
+
+
 @pytest.mark.parametrize("H,KVH,W,C,NS,eager,og,dtype,reduction,homogeneous,steps", [
     (8, 2, 64, 4, 64, True, False, torch.bfloat16, "mean", False, [300, 129, 31, 2, 200, 64]),    # G = 4, fills and evicts
     (14, 2, 128, 4, 4, False, False, torch.float16, "max", False, [260, 96, 96, 200, 59, 96]),    # G = 7, lazy fill
