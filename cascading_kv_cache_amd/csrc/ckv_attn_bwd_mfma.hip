@@ -11,13 +11,15 @@
 //          dV^T += dO^T P and dK^T += Q^T dS.
 //
 // Precision.  With 128 dims P and dS enter those products rounded to the tensor dtype.  With 64 dims nothing but the operands
-// is held in 16 bits: P and dS enter as three terms of the tensor dtype that add up to the float32 value, one matrix
-// instruction each (Weights), float16 terms of dS times a power of two that keeps them in range (Range); blocks that the
-// terms cannot hold, infinite gradients among them, take v_mfma_f32_32x32x2 on the values themselves.  That instruction for
-// every block, which is four times the matrix work of three terms and never runs beside a vector instruction, took 8 heads x
-// 1000 rows x 5095 keys in float16 dq 55 and dk/dv 91 us instead of 35 and 49 (the vector kernels 2520 and 1838); against
-// float64 over 16 random shapes the terms are level or closer (dq 2.0999e-4 against 2.1000e-4, dk 2.0808e-4 and 2.0808e-4,
-// dv 2.0778e-4 and 2.0778e-4 relative, float16: the rounding of the result).
+// is held in 16 bits: P and dS enter as three bfloat16 terms that add up to the float32 value, one matrix instruction each
+// (Weights).  A float16 operand of such a product is two bfloat16 numbers (Halves), so that it takes six.  Float16 terms would
+// need three, but resolve 2^-24 of a value that has to be scaled into their range: a dS 2^-25 times its row's largest would keep
+// half of its bits, and where that row's largest meet zeros in a dim of K or Q the sum is what was lost.  Blocks that no terms
+// hold (infinite dS or gradients) take v_mfma_f32_32x32x2 on the values themselves.  That instruction for every block never runs
+// beside a vector instruction: 8 heads x 1000 rows x 5095 keys in float16 dq 55 and dk/dv 91 us, six products 45 and 74 (three
+// float16 ones 35 and 49; the vector kernels 2520 and 1838).  Against float64 over 50 random shapes dq, dk and dv are 2.0956e-4,
+// 2.0816e-4 and 2.0747e-4 off (relative), which is the rounding of the result; float32 products 2.0956e-4, 2.0816e-4, 2.0747e-4.
+// Before that rounding dq is 2.99e-7 off (8 shapes), bfloat16 3.11e-7; with float32 products 3.69e-7 and 3.61e-7.
 //
 // What bounds them (64 heads x 1024 rows x 8704 visible keys, 128 dims, bf16: dq 548 -> 440 us, dk/dv 770 -> 620).  Vector work
 // beside the matrix work: both take most of a block's time and overlap only where a wavefront alternates them, so an
@@ -60,13 +62,16 @@ constexpr int kOwn = kWaves * 32;     // stationary rows of a workgroup
 constexpr int kAhead = 3, kKvAhead = 3;  // matrix instructions between an operand's read from LDS and its use
 constexpr int kDqStages = 3;          // stages of K and V blocks of the dq kernel: copies two blocks ahead
 constexpr float kLog2e = 1.4426950408889634f;
-template <int kHD>
+// kSplit: the A operands of the products that P and dS enter come from two bfloat16 tiles beside the tile itself, see Halves
+template <int kHD, bool kSplit = false>
 struct Geo {
     static constexpr int kRowBytes = kHD * 2;
     static constexpr int kTile = kBlk * kRowBytes;  // 8 KiB with 128 dims
     static constexpr int kPieces = kHD / 8;         // 16-byte pieces of a row
-    // dynamic LDS of the dk/dv kernel: two stages of (Q, dO) tiles, the per-row scalars of both stages, V^T operands
-    static constexpr int kDkdvRowv = 2 * 2 * kTile;
+    // dynamic LDS of the dk/dv kernel: two stages of (Q, dO) tiles, with kSplit their halves, the per-row scalars of both
+    // stages, V^T operands
+    static constexpr int kDkdvHalves = 2 * 2 * kTile;
+    static constexpr int kDkdvRowv = kDkdvHalves + (kSplit ? 2 * 2 * 2 * kTile : 0);
     static constexpr int kDkdvOdd = kDkdvRowv + 2 * 2 * kBlk * (int)sizeof(float);   // 64 dims: a word per stage
     static constexpr int kDkdvV = kDkdvOdd + (kHD == 64 ? 16 : 0);
     static constexpr int kParked = kHD == 128 ? 3 : 0;   // K^T operands that are kept there too: 12 registers that would spill
@@ -104,17 +109,6 @@ struct Mma<__half> {
     }
     __device__ static float lo_f(uint32_t w) { return (float)__builtin_bit_cast(f16x2, w)[0]; }
     __device__ static float hi_f(uint32_t w) { return (float)__builtin_bit_cast(f16x2, w)[1]; }
-    // one instruction that widens and subtracts, where the compiler makes two (half the vector work of a set of terms)
-    __device__ static float less_lo(float x, uint32_t w) {
-        float r;
-        asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(w), "v"(x));
-        return r;
-    }
-    __device__ static float less_hi(float x, uint32_t w) {
-        float r;
-        asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(w), "v"(x));
-        return r;
-    }
 };
 
 struct BwdMfmaParams {
@@ -244,6 +238,13 @@ struct Operands {
     }
 };
 
+__device__ inline f32x16 zero16() {
+    f32x16 z;
+#pragma unroll
+    for (int i = 0; i < 16; i++) z[i] = 0.f;
+    return z;
+}
+
 template <typename T>
 __device__ inline uint4 pack8(const f32x16& v, int s) {
     return make_uint4(Mma<T>::pack2(v[8 * s + 0], v[8 * s + 1]), Mma<T>::pack2(v[8 * s + 2], v[8 * s + 3]),
@@ -253,28 +254,86 @@ __device__ inline uint4 pack8(const f32x16& v, int s) {
 // The B operand of the two products that contract over a block's 32 rows, element 8 s + i of `v` belonging to step s, and the
 // product of a step with the A operand of Operands::col_op.  Element 4 a + e of that holds rows 16 s + 8 a + 4 (lane/32) + e,
 // the row of accumulator register 8 s + 4 a + e in the same lane half.  `accumulate` is product k, step k / kDB into
-// accumulator k % kDB with A operand ops[k].  128 dims: packed in the tensor dtype; 64 dims: three terms of it that add up to
-// the float32 value, one matrix instruction each.
+// accumulator k % kDB with A operand `op`.  128 dims: packed in the tensor dtype; 64 dims: three bfloat16 terms that add up
+// to the float32 value (24 bits in three times 8, and bfloat16 has float32's range), one matrix instruction each.
 template <typename T, int kHD>
 struct Weights {
     static constexpr int kDB = kHD / 32, kTerms = kHD == 64 ? 3 : 1;
+    typedef typename std::conditional<kHD == 64, __hip_bfloat16, T>::type Term;
+    typedef Mma<Term> M;
     uint4 w[kTerms][2];
     __device__ void set(const f32x16& v, int s) {
-        w[0][s] = pack8<T>(v, s);
+        w[0][s] = pack8<Term>(v, s);
         if constexpr (kTerms == 3) {
             f32x16 rest = v;
 #pragma unroll
             for (int t = 1; t < 3; t++) {
                 const uint32_t p[4] = {w[t - 1][s].x, w[t - 1][s].y, w[t - 1][s].z, w[t - 1][s].w};
 #pragma unroll
-                for (int i = 0; i < 8; i++) rest[8 * s + i] = i & 1 ? Mma<T>::less_hi(rest[8 * s + i], p[i >> 1]) : Mma<T>::less_lo(rest[8 * s + i], p[i >> 1]);
-                w[t][s] = pack8<T>(rest, s);
+                for (int i = 0; i < 8; i++) rest[8 * s + i] -= i & 1 ? M::hi_f(p[i >> 1]) : M::lo_f(p[i >> 1]);   // exact
+                w[t][s] = pack8<Term>(rest, s);
             }
         }
     }
-    __device__ void accumulate(const uint4 (&ops)[2 * kDB], int k, f32x16 (&c)[kDB]) const {
+    __device__ void accumulate(const uint4& op, int k, f32x16 (&c)[kDB]) const {
 #pragma unroll
-        for (int t = 0; t < kTerms; t++) c[k % kDB] = Mma<T>::mma(ops[k], w[t][k / kDB], c[k % kDB]);
+        for (int t = 0; t < kTerms; t++) c[k % kDB] = M::mma(op, w[t][k / kDB], c[k % kDB]);
+    }
+};
+
+// Float16 operands of those products with 64 dims: a float16 number is the sum of two bfloat16 ones, itself rounded to 8 bits
+// and the rest, which has three (infinity: the rest is NaN, but a product of P or dS with an infinite row of K or Q is NaN in
+// any arithmetic, and blocks with an infinite row of dO take float32 products).  Every wavefront splits the rows that it copied
+// itself, its lanes the 16 bytes that they copied, into two tiles laid out like the first (`split`: kTiles of them from byte
+// `tile` on, two each from byte `halves` on).
+template <typename T, int kHD>
+struct Halves {
+    static constexpr bool kSplit = kHD == 64 && std::is_same<T, __half>::value;
+    static constexpr int kOps = kSplit ? 2 : 1;   // A operands of a product
+    // Product k with all of its operands.  Of a split one the instructions are added up from zero in `block`, which joins the
+    // accumulator when the block is done: one rounding of the large sum per block instead of twelve (dq before it is rounded
+    // 2.99e-7 off instead of 3.49e-7, for 1.5 us of 74 in dk/dv and none in dq).
+    __device__ static void accumulate(const Weights<T, kHD>& w, const uint4 (&ops)[kOps][kHD / 16], int k, f32x16 (&c)[kHD / 32], f32x16 (&block)[kHD / 32]) {
+        constexpr int kDB = kHD / 32;
+        if constexpr (kSplit) {
+            if (k < kDB) block[k] = zero16();
+#pragma unroll
+            for (int o = 0; o < kOps; o++) w.accumulate(ops[o][k], k, block);
+            if (k > kDB) join(k - kDB - 1, c, block);   // a product behind its last instruction
+        } else {
+            w.accumulate(ops[0][k], k, c);
+        }
+    }
+    // the last accumulator's, once there is other work to do behind its last instruction
+    __device__ static void finish(f32x16 (&c)[kHD / 32], const f32x16 (&block)[kHD / 32]) {
+        if constexpr (kSplit) join(kHD / 32 - 1, c, block);
+    }
+    __device__ static void join(int db, f32x16 (&c)[kHD / 32], const f32x16 (&block)[kHD / 32]) {
+#pragma unroll
+        for (int i = 0; i < 16; i++) c[db][i] += block[db][i];
+    }
+    template <int kTiles>
+    __device__ static void split(unsigned char* lds, uint32_t tile, uint32_t halves, int wave, int lane) {
+        if constexpr (kSplit) {
+            constexpr int kTile = Geo<kHD>::kTile;
+            const uint32_t at = (uint32_t)(wave * 1024 + lane * 16);
+#pragma unroll
+            for (int i = 0; i < kTiles; i++) {
+                const uint4 v = *reinterpret_cast<const uint4*>(lds + tile + (uint32_t)(i * kTile) + at);
+                const uint32_t in[4] = {v.x, v.y, v.z, v.w};
+                uint32_t hi[4], lo[4];
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    typedef Mma<__hip_bfloat16> M;
+                    const float x0 = Mma<__half>::lo_f(in[j]), x1 = Mma<__half>::hi_f(in[j]);
+                    hi[j] = M::pack2(x0, x1);
+                    lo[j] = M::pack2(x0 - M::lo_f(hi[j]), x1 - M::hi_f(hi[j]));   // exact
+                }
+                unsigned char* to = lds + halves + (uint32_t)(2 * i * kTile) + at;
+                *reinterpret_cast<uint4*>(to) = make_uint4(hi[0], hi[1], hi[2], hi[3]);
+                *reinterpret_cast<uint4*>(to + kTile) = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+            }
+        }
     }
 };
 
@@ -300,41 +359,13 @@ __device__ inline void accumulate_f32(const uint4 (&ops)[4], const f32x16& v, f3
     }
 }
 
-// 64 dims: whether three terms hold the dS of a block.  bfloat16 has float32's range, so that they do unless dS is out of all
-// range.  float16 terms hold 33 bits of a number of 2^-2 and more and resolve 2^-24: the dS of a lane (a query or a key: one
-// column of the accumulators) are held times a power of two that takes the largest to about 2^12.  It is set by the first
-// block that is not all zero and moves when a block outgrows 2^15; what is smaller than the largest by 2^-15 loses bits below
-// 2^-36 of that, which float32 sums of the two would lose as well.  2^40 at most: smaller dS are below every float16 result.
-template <typename T>
-struct Range {
-    static constexpr bool kMoves = std::is_same<T, __half>::value;
-    float limit = kMoves ? 0.f : 0x1p120f;
-    int total = 0;   // dS and accumulators are held times 2^total
-    // true: the block does not go into terms; `factor`: what later blocks are to be multiplied by on top
-    __device__ bool outside(f32x16& ds, f32x16 (&acc)[2], float* factor) {
-        *factor = 1.f;
-        float m = 0.f;
+// 64 dims: some dS of the wavefront's block is infinite or so large that its terms could be
+__device__ inline bool beyond_terms(const f32x16& ds) {
+    float m = 0.f;
 #pragma unroll
-        for (int i = 0; i < 16; i++) m = fmaxf(m, fabsf(ds[i]));
-        if constexpr (kMoves) m = half_max(m);
-        if (__ballot(m > limit) == 0ull) return false;
-        if (!kMoves || __ballot(m > 0x1p100f) != 0ull) return true;
-        if (m > limit) {
-            int up = 12 - __builtin_amdgcn_frexp_expf(m);
-            if (up > 40 - total) up = 40 - total;
-            total += up;
-            limit = 32768.f;
-            *factor = __builtin_amdgcn_ldexpf(1.f, up);
-        }
-#pragma unroll
-        for (int i = 0; i < 16; i++) {
-            ds[i] *= *factor;
-            acc[0][i] *= *factor;
-            acc[1][i] *= *factor;
-        }
-        return false;
-    }
-};
+    for (int i = 0; i < 16; i++) m = fmaxf(m, fabsf(ds[i]));
+    return __ballot(m > 0x1p120f) != 0ull;
+}
 
 // bits [0, n) set, for 0 <= n <= 32
 __device__ inline uint32_t low_bits(int n) { return n >= 32 ? 0xffffffffu : ((1u << n) - 1u); }
@@ -349,13 +380,6 @@ __device__ inline float keep_if_bit(float v, uint32_t word, int bit) {
     return __uint_as_float(__float_as_uint(v) & (uint32_t)m);
 }
 
-__device__ inline f32x16 zero16() {
-    f32x16 z;
-#pragma unroll
-    for (int i = 0; i < 16; i++) z[i] = 0.f;
-    return z;
-}
-
 // ---------------------------------------------------------------------------------------------
 // dq
 // ---------------------------------------------------------------------------------------------
@@ -364,7 +388,9 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dq_kernel(BwdMfmaParams 
     constexpr int kTile = Geo<kHD>::kTile, kStage = 2 * kTile;   // K, V
     constexpr int kCopies = 2 * (kHD / 64);                      // of a wavefront and block
     constexpr int kMine = kBlk / kWaves;                         // rows of a block that a wavefront copies
-    __shared__ __attribute__((aligned(16))) unsigned char smem[kDqStages * (kStage + kBlk * (int)sizeof(int))];
+    typedef Halves<T, kHD> Half;                                 // of K: two tiles per stage
+    constexpr uint32_t kHalves = kDqStages * kStage, kRowNumbers = kHalves + (Half::kSplit ? kDqStages * 2 * kTile : 0);
+    __shared__ __attribute__((aligned(16))) unsigned char smem[kRowNumbers + kDqStages * kBlk * (int)sizeof(int)];
     const ckv_dense_bwd_args& a = p.a;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / CKV_WAVE), lane = tid % CKV_WAVE, h = lane >> 5;
     const Keys keys(p);
@@ -414,7 +440,6 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dq_kernel(BwdMfmaParams 
     f32x16 dq[kHD / 32];
 #pragma unroll
     for (int db = 0; db < kHD / 32; db++) dq[db] = zero16();
-    Range<T> range;   // 64 dims
 
     // keys past the diagonal of the workgroup's last row are visible to none of its rows
     int m_last = m_wg + kOwn - 1;
@@ -427,7 +452,7 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dq_kernel(BwdMfmaParams 
     // Blocks are copied two ahead into three stages.  With an order the row numbers of a wavefront's eight rows of a block
     // come to LDS the same way, three blocks ahead, so that no load in the loop is one whose result the compiler would
     // wait for together with the copies behind it.
-    const uint32_t mine = lds0 + (uint32_t)(kDqStages * kStage + wave * kMine * (int)sizeof(int));
+    const uint32_t mine = lds0 + kRowNumbers + (uint32_t)(wave * kMine * (int)sizeof(int));
     constexpr uint32_t kSlot = kBlk * sizeof(int);
     const int mine_lane = kHD == 128 ? lane / 16 : lane / 8;   // of copy 0; copy j takes row 4 j + this one
     auto clamped = [&](int i) { return i < n_seen ? i : n_seen - 1; };   // a chunk key: finite values, and no query looks at this copy
@@ -457,6 +482,7 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dq_kernel(BwdMfmaParams 
         rows_of(blk0 + 2, 2, rows_next);
         if (blk0 + 1 < nblk) wait_copies<kCopies>();
         else wait_copies<0>();
+        Half::template split<1>(smem, 0, kHalves, wave, lane);
     }
     __syncthreads();
     auto step = [&](auto stage_tag, int blk) {
@@ -479,9 +505,13 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dq_kernel(BwdMfmaParams 
         constexpr int kRow = kHD / 16, kDB = kHD / 32;
         if (!dead) {
             f32x16 s = zero16(), dp = neg_delta;
-            uint4 ops[2 * kRow], cops[2 * kDB];
+            constexpr uint32_t ct = Half::kSplit ? kHalves + st * 2 * kTile : kt;
+            uint4 ops[2 * kRow], cops[Half::kOps][2 * kDB];
             auto row_op = [&](int k) { return op.row_op(k < kRow ? kt : vt, k % kRow); };
-            auto col_op = [&](int k) { return op.col_op(kt, k / kDB, k % kDB); };
+            auto col_op = [&](int k) {
+#pragma unroll
+                for (int o = 0; o < Half::kOps; o++) cops[o][k] = op.col_op(ct + o * kTile, k / kDB, k % kDB);
+            };
             auto weight = [&](int i) {
                 s[i] = __builtin_amdgcn_exp2f(fmaf(s[i], c2, nl));
             };
@@ -491,7 +521,7 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dq_kernel(BwdMfmaParams 
 #pragma unroll
             for (int k = 0; k < 2 * kRow; k++) {
                 if (k + kAhead < 2 * kRow) ops[k + kAhead] = row_op(k + kAhead);
-                else cops[k + kAhead - 2 * kRow] = col_op(k + kAhead - 2 * kRow);
+                else col_op(k + kAhead - 2 * kRow);
                 if (k < kRow) s = Mma<T>::mma(ops[k], qreg[k], s);
                 else dp = Mma<T>::mma(ops[k], greg[k - kRow], dp);
                 if (k > kRow) {   // not beside the first, which the last logits are only just behind
@@ -515,24 +545,24 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dq_kernel(BwdMfmaParams 
 #pragma unroll
             for (int i = 0; i < (kHD == 64 ? 16 : 8); i++) dsv[i] = s[i] * dp[i];
             if constexpr (kHD == 64) {
-                float factor;
-                outside = range.outside(dsv, dq, &factor);
-                nl += __builtin_amdgcn_logf(factor);   // a power of two: whole
+                outside = beyond_terms(dsv);
                 if (outside) {
+                    uint4 kops[2 * kDB];
 #pragma unroll
-                    for (int k = kAhead; k < 2 * kDB; k++) cops[k] = col_op(k);
-                    accumulate_f32<T>(cops, dsv, dq);
+                    for (int k = 0; k < 2 * kDB; k++) kops[k] = op.col_op(kt, k / kDB, k % kDB);
+                    accumulate_f32<T>(kops, dsv, dq);
                 }
                 asm volatile("");
             }
             if (!outside) {
                 Weights<T, kHD> bop;
+                f32x16 block[kDB];
                 bop.set(dsv, 0);
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int k = 0; k < 2 * kDB; k++) {
-                    if (k + kAhead < 2 * kDB) cops[k + kAhead] = col_op(k + kAhead);
-                    bop.accumulate(cops, k, dq);
+                    if (k + kAhead < 2 * kDB) col_op(k + kAhead);
+                    Half::accumulate(bop, cops, k, dq, block);
                     if (kHD == 128 && k < kDB) {
 #pragma unroll
                         for (int i = 8 + k * (8 / kDB); i < 8 + (k + 1) * (8 / kDB); i++) dsv[i] = s[i] * dp[i];
@@ -540,6 +570,7 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dq_kernel(BwdMfmaParams 
                     if (k == (kHD == 128 ? kDB - 1 : 0)) bop.set(dsv, 1);
                     __builtin_amdgcn_sched_barrier(0);
                 }
+                Half::finish(dq, block);
             }
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -549,6 +580,8 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dq_kernel(BwdMfmaParams 
         } else {
             wait_copies<0>();
         }
+        // the halves of a stage were last read two barriers ago
+        if (blk + 1 < nblk) Half::template split<1>(smem, (st + 1) % kDqStages * kStage, kHalves + (st + 1) % kDqStages * 2 * kTile, wave, lane);
         __syncthreads();
     };
     for (int blk = blk0; blk < nblk; blk += kDqStages) {
@@ -561,12 +594,6 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dq_kernel(BwdMfmaParams 
         for (int db = 0; db < kHD / 32; db++)
 #pragma unroll
             for (int i = 0; i < 16; i++) dq[db][i] = -dq[db][i];
-    }
-    if constexpr (kHD == 64 && Range<T>::kMoves) {
-#pragma unroll
-        for (int db = 0; db < kHD / 32; db++)
-#pragma unroll
-            for (int i = 0; i < 16; i++) dq[db][i] = __builtin_amdgcn_ldexpf(dq[db][i], -range.total);
     }
     if (row_ok && p.n_split > 1) {
         float* out = p.part_dq + ((int64_t)share * a.B * a.H * n_ctx + bh * n_ctx + m_lane) * kHD;
@@ -613,13 +640,15 @@ __global__ void __launch_bounds__(kThreads) bwd_dq_sum_kernel(BwdMfmaParams p) {
 // ---------------------------------------------------------------------------------------------
 template <typename T, int kHD>
 __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dkdv_kernel(BwdMfmaParams p) {
-    constexpr int kTile = Geo<kHD>::kTile;
+    typedef Halves<T, kHD> Half;   // of Q and dO
+    typedef Geo<kHD, Half::kSplit> G;
+    constexpr int kTile = G::kTile;
     extern __shared__ __attribute__((aligned(16))) unsigned char dyn_smem[];
     typedef float (*RowPtr)[2][kBlk];
-    RowPtr rowv = reinterpret_cast<RowPtr>(dyn_smem + Geo<kHD>::kDkdvRowv);                        // [stage][-lse log2 e, -delta]
-    int* odd_rows = reinterpret_cast<int*>(dyn_smem + Geo<kHD>::kDkdvOdd);               // [stage] some row's delta is not finite
+    RowPtr rowv = reinterpret_cast<RowPtr>(dyn_smem + G::kDkdvRowv);                        // [stage][-lse log2 e, -delta]
+    int* odd_rows = reinterpret_cast<int*>(dyn_smem + G::kDkdvOdd);               // [stage] some row's delta is not finite
     // the V^T operands of a wavefront's 32 keys and the first of K^T, in operand order: [wave][ds][lane] 16 bytes each
-    uint4* vstat = reinterpret_cast<uint4*>(dyn_smem + Geo<kHD>::kDkdvV) + __builtin_amdgcn_readfirstlane(threadIdx.x / CKV_WAVE) * (kHD / 16 + Geo<kHD>::kParked) * CKV_WAVE;
+    uint4* vstat = reinterpret_cast<uint4*>(dyn_smem + G::kDkdvV) + __builtin_amdgcn_readfirstlane(threadIdx.x / CKV_WAVE) * (kHD / 16 + G::kParked) * CKV_WAVE;
     const ckv_dense_bwd_args& a = p.a;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / CKV_WAVE), lane = tid % CKV_WAVE, h = lane >> 5;
     const Keys keys(p);
@@ -636,7 +665,7 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dkdv_kernel(BwdMfmaParam
     const float* dl = p.delta + bh * n_ctx;
 
     // stationary B operands: K^T of this lane's key in registers but for what is parked in LDS, V^T in LDS (the registers go to the accumulators)
-    constexpr int kParked = Geo<kHD>::kParked;
+    constexpr int kParked = G::kParked;
     uint4 kreg[kHD / 16 - kParked];   // of ds >= kParked
     {
         const int64_t off = (b * a.kv_stride[0] + hd * a.kv_stride[1] + (key_ok ? keys.row_of(n_lane) : 0) * a.kv_stride[2]) * 2;
@@ -679,27 +708,24 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dkdv_kernel(BwdMfmaParam
     };
     // Per-row scalars of a block, one per lane of wavefront 0.  Rows of dout that are not finite show in their delta (a sum of
     // products with out): in their blocks the products with 64 dims take P and dS as they are, zero terms times infinity are NaN.
-    // float16 with 64 dims: P is held times 2^15, so that its terms resolve 2^-39, and dk and dv are brought back at the end.
     constexpr bool kTerms = kHD == 64;
-    constexpr float kHead = kTerms && Range<T>::kMoves ? 15.f : 0.f;
     auto row_scalar = [&](int m0) {
         const int m = m0 + (lane & 31);
         return m < n_ctx ? (h ? dl[m] : lse[m]) : 0.f;
     };
     auto park = [&](float v, int st) {
-        rowv[st][h][lane & 31] = h ? -v : fmaf(-v, kLog2e, kHead);
+        rowv[st][h][lane & 31] = h ? -v : -v * kLog2e;
         if constexpr (kTerms) {
             const bool odd = __ballot(h && !(fabsf(v) < INFINITY)) != 0ull;
             if (lane == 0) odd_rows[st] = odd ? 1 : 0;
         }
     };
-    Range<T> range;                                                   // 64 dims
-    float dscale = kHead > 0.f ? 0x1p-15f : 1.f;                       // of dS, by the lane
     if (blk0 < nblk) {
         copy(blk0 * kBlk, 0);
         if (wave == 0) park(row_scalar(blk0 * kBlk), 0);
     }
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+    wait_copies<0>();
+    if (blk0 < nblk) Half::template split<2>(dyn_smem, 0, G::kDkdvHalves, wave, lane);
     __syncthreads();
     auto step = [&](auto stage_tag, int blk) {
         constexpr int st = decltype(stage_tag)::value;
@@ -726,9 +752,17 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dkdv_kernel(BwdMfmaParam
             // instructions before the one that takes it, the first ones of a phase in the phase before.
             constexpr int kRow = kHD / 16, kDB = kHD / 32;
             static_assert(kParked <= kKvAhead, "parked operands are read with the first ones");
-            uint4 kops[kKvAhead], qops[kRow], gops[2 * kDB], rops[kRow], vops[kRow], cops[2 * kDB];
-            auto g_col = [&](int k) { return op.col_op(gt, k / kDB, k % kDB); };
-            auto q_col = [&](int k) { return op.col_op(qt, k / kDB, k % kDB); };
+            constexpr uint32_t qc = Half::kSplit ? G::kDkdvHalves + st * 4 * kTile : qt, gc = Half::kSplit ? qc + 2 * kTile : gt;
+            uint4 kops[kKvAhead], qops[kRow], gops[Half::kOps][2 * kDB], rops[kRow], vops[kRow], cops[Half::kOps][2 * kDB];
+            auto g_col = [&](int k) {
+#pragma unroll
+                for (int o = 0; o < Half::kOps; o++) gops[o][k] = op.col_op(gc + o * kTile, k / kDB, k % kDB);
+            };
+            auto q_col = [&](int k) {
+#pragma unroll
+                for (int o = 0; o < Half::kOps; o++) cops[o][k] = op.col_op(qc + o * kTile, k / kDB, k % kDB);
+            };
+            f32x16 block[kDB];
             f32x16 pv = zero16(), dp;
             float nls[16];
             auto row_scalars = [&](int which, int j, auto& to) {
@@ -760,7 +794,7 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dkdv_kernel(BwdMfmaParam
                     rops[k + 1] = op.row_op(gt, k + 1);
                     vops[k + 1] = vstat[(k + 1) * CKV_WAVE + lane];
                 }
-                if (k >= kRow - kKvAhead) gops[k + kKvAhead - kRow] = g_col(k + kKvAhead - kRow);
+                if (k >= kRow - kKvAhead) g_col(k + kKvAhead - kRow);
 #pragma unroll
                 for (int j = 0; j < 4; j++)
                     if (k == 4 * j / kPer) row_scalars(0, j, nls);   // a slot before the first exponential that takes one
@@ -775,10 +809,6 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dkdv_kernel(BwdMfmaParam
 #pragma unroll
                 for (int i = 0; i < 16; i++) pv[i] = keep_if_bit(pv[i], allow, 8 * (i / 4) + (i % 4));
             }
-            auto ds_of = [&](int i) {
-                dp[i] = pv[i] * dp[i];
-                if constexpr (kHead > 0.f) dp[i] *= dscale;
-            };
             if constexpr (!kTerms) {
                 Weights<T, kHD> pw, dw;
                 pw.set(pv, 0);
@@ -786,9 +816,9 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dkdv_kernel(BwdMfmaParam
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int k = 0; k < 2 * kDB; k++) {
-                    if (k + kKvAhead < 2 * kDB) gops[k + kKvAhead] = g_col(k + kKvAhead);
-                    else cops[k + kKvAhead - 2 * kDB] = q_col(k + kKvAhead - 2 * kDB);
-                    pw.accumulate(gops, k, dv);
+                    if (k + kKvAhead < 2 * kDB) g_col(k + kKvAhead);
+                    else q_col(k + kKvAhead - 2 * kDB);
+                    Half::accumulate(pw, gops, k, dv, block);
 #pragma unroll
                     for (int i = k * (8 / kDB); i < (k + 1) * (8 / kDB); i++) dp[i] = kScaleInside<T, kHD> ? pv[i] * dp[i] * a.scale : pv[i] * dp[i];
                     if (k == kDB - 1) dw.set(dp, 0);
@@ -797,25 +827,24 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dkdv_kernel(BwdMfmaParam
                 dw.set(dp, 1);
 #pragma unroll
                 for (int k = 0; k < 2 * kDB; k++) {
-                    if (k + kKvAhead < 2 * kDB) cops[k + kKvAhead] = q_col(k + kKvAhead);
-                    dw.accumulate(cops, k, dk);
+                    if (k + kKvAhead < 2 * kDB) q_col(k + kKvAhead);
+                    Half::accumulate(dw, cops, k, dk, block);
                     __builtin_amdgcn_sched_barrier(0);
                 }
             } else {
                 // the rare sides are branches of their own: as the other sides of one they spill registers of the common one
                 const bool odd = __builtin_amdgcn_readfirstlane(odd_rows[st]) != 0;
-                auto dk_f32 = [&]() {
+                auto product_f32 = [&](uint32_t tile, const f32x16& v, f32x16(&c)[kDB]) {
+                    uint4 ops[2 * kDB];
 #pragma unroll
-                    for (int k = 0; k < 2 * kDB; k++) cops[k] = q_col(k);
-                    accumulate_f32<T>(cops, dp, dk);
+                    for (int k = 0; k < 2 * kDB; k++) ops[k] = op.col_op(tile, k / kDB, k % kDB);
+                    accumulate_f32<T>(ops, v, c);
                 };
                 if (odd) {
+                    product_f32(gt, pv, dv);
 #pragma unroll
-                    for (int k = 0; k < 2 * kDB; k++) gops[k] = g_col(k);
-                    accumulate_f32<T>(gops, pv, dv);
-#pragma unroll
-                    for (int i = 0; i < 16; i++) ds_of(i);
-                    dk_f32();
+                    for (int i = 0; i < 16; i++) dp[i] *= pv[i];
+                    product_f32(qt, dp, dk);
                 }
                 asm volatile("");
                 if (!odd) {
@@ -824,38 +853,41 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dkdv_kernel(BwdMfmaParam
                     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                     for (int k = 0; k < 2 * kDB; k++) {
-                        if (k + kKvAhead < 2 * kDB) gops[k + kKvAhead] = g_col(k + kKvAhead);
-                        else cops[k + kKvAhead - 2 * kDB] = q_col(k + kKvAhead - 2 * kDB);
-                        w.accumulate(gops, k, dv);
+                        if (k + kKvAhead < 2 * kDB) g_col(k + kKvAhead);
+                        else q_col(k + kKvAhead - 2 * kDB);
+                        Half::accumulate(w, gops, k, dv, block);
                         if (k == 0) w.set(pv, 1);
                         if (k > 0) {
 #pragma unroll
-                            for (int i = (k - 1) * 6; i < k * 6 && i < 16; i++) ds_of(i);
+                            for (int i = (k - 1) * 6; i < k * 6 && i < 16; i++) dp[i] *= pv[i];
                         }
                         __builtin_amdgcn_sched_barrier(0);
                     }
-                    float factor;
-                    const bool outside = range.outside(dp, dk, &factor);
-                    dscale *= factor;
-                    if (outside) dk_f32();
+                    const bool outside = beyond_terms(dp);
+                    Half::finish(dv, block);
+                    if (outside) product_f32(qt, dp, dk);
                     asm volatile("");
                     if (!outside) {
                         w.set(dp, 0);
                         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                         for (int k = 0; k < 2 * kDB; k++) {
-                            if (k + kKvAhead < 2 * kDB) cops[k + kKvAhead] = q_col(k + kKvAhead);
-                            w.accumulate(cops, k, dk);
+                            if (k + kKvAhead < 2 * kDB) q_col(k + kKvAhead);
+                            Half::accumulate(w, cops, k, dk, block);
                             if (k == 0) w.set(dp, 1);
                             __builtin_amdgcn_sched_barrier(0);
                         }
+                        Half::finish(dk, block);
                     }
                 }
             }
         }
         __builtin_amdgcn_sched_barrier(0);
-        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wavefront's copies of the next block have landed
-        if (more && wave == 0) park(rv_next, st ^ 1);
+        wait_copies<0>();  // this wavefront's copies of the next block have landed
+        if (more) {
+            if (wave == 0) park(rv_next, st ^ 1);
+            Half::template split<2>(dyn_smem, (st ^ 1) * 2 * kTile, G::kDkdvHalves + (st ^ 1) * 4 * kTile, wave, lane);
+        }
         __syncthreads();
     };
     for (int blk = blk0; blk < nblk; blk += 2) {
@@ -868,23 +900,14 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dkdv_kernel(BwdMfmaParam
 #pragma unroll
             for (int i = 0; i < 16; i++) dk[db][i] *= a.scale;
     }
-    if constexpr (kHead > 0.f) {
-#pragma unroll
-        for (int db = 0; db < kHD / 32; db++)
-#pragma unroll
-            for (int i = 0; i < 16; i++) {
-                dk[db][i] = __builtin_amdgcn_ldexpf(dk[db][i], -range.total);
-                dv[db][i] *= 0x1p-15f;
-            }
-    }
     if (!key_ok) {
 #pragma unroll
         for (int db = 0; db < kHD / 32; db++) dk[db] = dv[db] = zero16();
     }
     // The rows leave through LDS (the stages: nobody reads them any more), so that a store is whole rows of 16-byte pieces, 1 KiB
     // an instruction; 8-byte pieces of 32 rows apiece cost a workgroup of 32 blocks an eighth of its time.
-    constexpr int kPieces = Geo<kHD>::kPieces, kPer = CKV_WAVE / kPieces, kOut = 32 / kPer;   // rows of a store, stores of a tensor
-    unsigned char* mine = dyn_smem + wave * 32 * Geo<kHD>::kRowBytes;
+    constexpr int kPieces = G::kPieces, kPer = CKV_WAVE / kPieces, kOut = 32 / kPer;   // rows of a store, stores of a tensor
+    unsigned char* mine = dyn_smem + wave * 32 * G::kRowBytes;
     int64_t out_off[kOut];
 #pragma unroll
     for (int i = 0; i < kOut; i++) {
@@ -896,13 +919,13 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dkdv_kernel(BwdMfmaParam
         for (int db = 0; db < kHD / 32; db++) {
 #pragma unroll
             for (int j = 0; j < 4; j++)   // dims 32 db + 8 j + 4 h .. +3 of this lane's key
-                *reinterpret_cast<uint2*>(mine + (lane & 31) * Geo<kHD>::kRowBytes + (((4 * db + j) ^ (lane & (kPieces - 1))) << 4) + 8 * h) =
+                *reinterpret_cast<uint2*>(mine + (lane & 31) * G::kRowBytes + (((4 * db + j) ^ (lane & (kPieces - 1))) << 4) + 8 * h) =
                     make_uint2(Mma<T>::pack2(acc[db][4 * j], acc[db][4 * j + 1]), Mma<T>::pack2(acc[db][4 * j + 2], acc[db][4 * j + 3]));
         }
 #pragma unroll
         for (int i = 0; i < kOut; i++) {
             const int row = kPer * i + lane / kPieces, piece = lane % kPieces;
-            const uint4 v = *reinterpret_cast<const uint4*>(mine + row * Geo<kHD>::kRowBytes + ((piece ^ (row & (kPieces - 1))) << 4));
+            const uint4 v = *reinterpret_cast<const uint4*>(mine + row * G::kRowBytes + ((piece ^ (row & (kPieces - 1))) << 4));
             if (out_off[i] >= 0) *reinterpret_cast<uint4*>(reinterpret_cast<char*>(to) + out_off[i]) = v;
         }
     };
@@ -936,9 +959,10 @@ int run(const BwdMfmaParams& p_in, hipStream_t stream) {
                            stream, p);
         CKV_HIP_TRY(hipGetLastError());
     }
-    if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(bwd_mfma_dkdv_kernel<T, kHD>), Geo<kHD>::kDkdvLds)) return rc;
+    constexpr int kDkdvLds = Geo<kHD, Halves<T, kHD>::kSplit>::kDkdvLds;
+    if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(bwd_mfma_dkdv_kernel<T, kHD>), kDkdvLds)) return rc;
     const dim3 grid_dkdv = grid_of((a.n_kv + kOwn - 1) / kOwn, 2 * (int64_t)mfma_device_cus());
-    hipLaunchKernelGGL((bwd_mfma_dkdv_kernel<T, kHD>), grid_dkdv, dim3(kThreads), Geo<kHD>::kDkdvLds, stream, p);
+    hipLaunchKernelGGL((bwd_mfma_dkdv_kernel<T, kHD>), grid_dkdv, dim3(kThreads), kDkdvLds, stream, p);
     CKV_HIP_TRY(hipGetLastError());
     return CKV_OK;
 }

@@ -257,7 +257,7 @@ int ckv_attn_dense(const ckv_dense_args* args, void* stream);
  * CKV_ERR_UNSUPPORTED before anything is launched).  bf16 / fp16 tensors with head_dim 64 or 128, unit stride along the
  * head dim, every other stride a multiple of 8 elements and 16-byte aligned base addresses run on the matrix cores,
  * with fp32 accumulation: with head_dim 128 probabilities and dS are rounded to the tensor dtype for the products, with
- * head_dim 64 they stay fp32.  Everything else runs fp32-math kernels.
+ * head_dim 64 they stay fp32 (as three bf16 terms that add up to the value).  Everything else runs fp32-math kernels.
  * ---------------------------------------------------------------------------------------- */
 typedef struct ckv_dense_bwd_args {
     const void* q;                 /* (B, H, n_ctx, D) */

@@ -46,6 +46,18 @@ def exact_attention(q, k, v, see, scale):
     return torch.matmul(p, vd), p, torch.logsumexp(s, dim=-1), torch.matmul(p * p, vd * vd).sqrt()
 
 
+def exact_weights(q, k, v, out, lse, mask, do, scale):
+    """P and dS of the backward pass in float64 from what its kernels are given, the forward's output and row normalisers
+    among it, and the size that dS's float32 sums of 64 or 128 products are rounded at."""
+    see = visible(q.size(2), k.size(2), mask)
+    s = torch.matmul(q.double(), k.double().transpose(2, 3).contiguous()) * scale
+    p = torch.exp(s - lse.double()[..., None]).masked_fill(~see, 0.0)
+    g, vt = do.double(), v.double().transpose(2, 3).contiguous()
+    dp, delta = torch.matmul(g, vt), (out.double() * g).sum(-1, keepdim=True)
+    size = torch.matmul(g.abs(), vt.abs()) + (out.double() * g).abs().sum(-1, keepdim=True)
+    return p, p * (dp - delta) * scale, p * size * abs(scale)
+
+
 DENSE = [(1, 2, 128, 128), (1, 3, 33, 1 + 33), (2, 4, 200, 1000 + 200), (1, 2, 500, 2048 + 64 + 500), (1, 1, 700, 5000 + 700)]
 
 
@@ -98,8 +110,7 @@ def test_dense_backward_of_head_size_64_is_rounded_once(Z, H, n_ctx, n_kv, grad_
 @pytest.mark.parametrize("dtype", [BF16, F16])
 @pytest.mark.parametrize("octaves", [-24, 24])
 def test_dense_backward_of_head_size_64_over_many_octaves(octaves, dtype):
-    """dS whose size falls or rises by 2^24 from the first block to the last, along the keys and along the rows: float16
-    holds them by terms times a power of two that the first block sets and later ones move."""
+    """dS whose size falls or rises by 2^24 from the first block to the last, along the keys and along the rows."""
     from cascading_kv_cache_amd import flash_attention as fa
 
     n_ctx, n_kv, scale = 300, 900, 0.5
@@ -118,6 +129,33 @@ def test_dense_backward_of_head_size_64_over_many_octaves(octaves, dtype):
     assert_rounded_once(dv, torch.matmul(pt, do.double()), torch.matmul(pt.square(), do.double().square()).sqrt(), n_ctx, "dv")
     assert_rounded_once(dk, torch.matmul(dst, q.double()), torch.matmul(ds2t, q.double().square()).sqrt(), n_ctx, "dk")
     assert_rounded_once(dq, torch.matmul(ds, k.double()), torch.matmul(ds2, k.double().square()).sqrt(), n_kv, "dq")
+
+
+@pytest.mark.parametrize("dtype", [BF16, F16])
+def test_small_weights_beside_large_ones_of_head_size_64(dtype):
+    """dS is float32 whatever stands beside it: it is 28 octaves smaller in every other row (for dk) and 36 for every other
+    key (for dq, as P is), and the large ones meet zeros in one dim of the other operand.  There the sum is the small ones
+    alone, to the last bit that the result's format shows."""
+    from cascading_kv_cache_amd import flash_attention as fa
+
+    n_ctx, n_kv, scale = 64, 160, 0.5
+    q, k, v, mask, do = (t.clone() for t in dense_case(1, 2, n_ctx, n_kv, 64, dtype, std=0.3))
+    v = (v.float() * 3).to(dtype)
+    do[:, :, ::2] *= 2.0 ** 10
+    do[:, :, 1::2] *= 2.0 ** -18
+    q[..., 5:8], k[..., 5:8] = 0.0, 0.0
+    q[:, :, 1::2, 5] = 2.0 ** 13           # dk, dim 5: the rows of the small gradients alone
+    k[:, :, 1::2, 6] = 2.0 ** 14           # dq, dim 6: the keys of the small probabilities alone
+    q[..., 7], k[:, :, 1::2, 7] = 8.0, -6.25   # their logits 25 below the others': 2^-36
+    out, _, lse, m = fa._forward(q, k, v, True, scale, mask, 0.9, True)
+    dq, dk, dv = fa._backward(q, k, v, out, lse, m, do, scale)
+    p, ds, size = exact_weights(q, k, v, out, lse, mask, do, scale)
+    pt, dst, sizet = (t.transpose(2, 3).contiguous() for t in (p, ds, size))
+    large, small = ds[0, :, ::2].abs().amax(), ds[0, :, 1::2].abs().amax()
+    assert large > 2.0 ** 24 * small and (dk[0, :, 0, 5] != 0).any() and (dq[0, :, ::2, 6] != 0).any()
+    assert_rounded_once(dv, torch.matmul(pt, do.double()), torch.matmul(pt.square(), do.double().square()).sqrt(), n_ctx, "dv")
+    assert_rounded_once(dk, torch.matmul(dst, q.double()), torch.matmul(sizet.square(), q.double().square()).sqrt(), n_ctx, "dk")
+    assert_rounded_once(dq, torch.matmul(ds, k.double()), torch.matmul(size.square(), k.double().square()).sqrt(), n_kv, "dq")
 
 
 @pytest.mark.parametrize("dtype", [BF16, F16])
