@@ -181,6 +181,47 @@ def test_dense_backward_of_head_size_64_with_an_infinite_gradient(dtype):
     assert dk[0, 0, seen].isfinite().sum().item() == 0
 
 
+def rounding_variance(x, dtype):
+    """of a number rounded to ``dtype``: uniform over a unit in the last place"""
+    bits, least = {BF16: (7, -126), F16: (10, -14)}[dtype]
+    ulp = torch.ldexp(torch.ones_like(x), (torch.frexp(x)[1] - 1).clamp(min=least) - bits)
+    return ulp.square() / 12
+
+
+def assert_rounded(got, exact, variance, what):
+    """``got`` is ``exact`` but for roundings of which ``variance`` is the sum, its own among them.  One bit less in P or dS shows
+    as a root mean square of 1.7 times that, a fault in one place as many deviations there."""
+    off = (got.double() - exact).square() / (variance + rounding_variance(exact, got.dtype))
+    rms, worst = off.mean().sqrt().item(), off.max().sqrt().item()
+    assert rms <= 1.1 and worst <= 8.0, f"{what}: root mean square {rms:.3f}, largest {worst:.2f} of the roundings' deviation"
+
+
+def check_backward(q, k, v, out, lse, mask, do, scale, dq, dk, dv):
+    """Head size 64: float32 but for the result.  Head size 128: P and dS enter the products rounded to the tensor dtype, dS
+    with or without the softmax scale, which no rounding of a mantissa tells apart."""
+    p, ds, size = exact_weights(q, k, v, out, lse, mask, do, scale)
+    n_ctx, n_kv = q.size(2), k.size(2)
+    turned = lambda t: t.transpose(2, 3).contiguous()
+    for what, got, w, weight_size, rows in (("dv", dv, turned(p), turned(p), do), ("dk", dk, turned(ds), turned(size), q), ("dq", dq, ds, size, k)):
+        x = rows.double()
+        exact, spread2 = torch.matmul(w, x), torch.matmul(weight_size.square(), x.square())
+        if q.size(-1) == 64:
+            assert_rounded_once(got, exact, spread2.sqrt(), n_kv if what == "dq" else n_ctx, what)
+        else:
+            assert_rounded(got, exact, torch.matmul(rounding_variance(w, got.dtype) * (w != 0), x.square()) + 2.0 ** -44 * spread2, what)
+
+
+@pytest.mark.parametrize("dtype", [BF16, F16])
+@pytest.mark.parametrize("scale", [0.3, -0.125])
+@pytest.mark.parametrize("Z,H,n_ctx,n_kv", DENSE)
+def test_dense_backward_of_head_size_128_rounds_weights_once(Z, H, n_ctx, n_kv, scale, dtype):
+    from cascading_kv_cache_amd import flash_attention as fa
+
+    q, k, v, mask, do = dense_case(Z, H, n_ctx, n_kv, 128, dtype)
+    out, _, lse, m = fa._forward(q, k, v, True, scale, mask, 0.9, True)
+    check_backward(q, k, v, out, lse, mask, do, scale, *fa._backward(q, k, v, out, lse, m, do, scale))
+
+
 @pytest.mark.parametrize("dtype", [BF16, F16])
 @pytest.mark.parametrize("scale", [-0.5, 0.0, 1e-3, 3.0])
 def test_any_softmax_scale_of_head_size_64(scale, dtype):
