@@ -223,6 +223,34 @@ def test_dense_backward_of_head_size_128_rounds_weights_once(Z, H, n_ctx, n_kv, 
 
 
 @pytest.mark.parametrize("dtype", [BF16, F16])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("room", ["delta", "delta and order"])
+@pytest.mark.parametrize("Z,H,n_ctx,n_kv,masked", [
+    (1, 2, 128, 128, None), (1, 3, 33, 1 + 33, None), (1, 1, 31, 64 + 31, slice(0, 64)),   # no cached key, one, none visible
+    (2, 4, 200, 1000 + 200, None), (1, 8, 129, 1500 + 129, slice(32, 700)),                 # whole blocks of masked keys
+    (1, 1, 300, 95 + 300, slice(0, 33))])
+def test_dense_backward_with_less_room_than_it_could_use(Z, H, n_ctx, n_kv, masked, room, D, dtype):
+    """A workspace without room for the order of the keys (they are taken as they lie and masked one by one), or without room
+    for dq's shares, as ``ckv_dense_bwd_key_order_bytes`` and ``ckv_dense_bwd_split_bytes`` allow."""
+    from cascading_kv_cache_amd import _abi
+    from cascading_kv_cache_amd import flash_attention as fa
+
+    q, k, v, mask, do = dense_case(Z, H, n_ctx, n_kv, D, dtype)
+    if masked is not None:
+        mask[masked] = True
+    out, _, lse, m = fa._forward(q, k, v, True, 0.3, mask, 0.9, True)
+    size = _abi.lib().ckv_dense_bwd_workspace_bytes(Z, H, n_ctx)
+    if room == "delta and order":
+        size += _abi.lib().ckv_dense_bwd_key_order_bytes(n_kv)
+    with pytest.MonkeyPatch.context() as patch:
+        patch.setattr(fa, "workspace", lambda device, need, stream: torch.empty(size, dtype=torch.uint8, device=device))
+        grads = fa._backward(q, k, v, out, lse, m, do, 0.3)
+    check_backward(q, k, v, out, lse, mask, do, 0.3, *grads)
+    hidden = torch.cat((mask, torch.zeros(n_ctx, dtype=torch.bool, device="cuda")))
+    assert (grads[1][:, :, hidden] == 0).all() and (grads[2][:, :, hidden] == 0).all()
+
+
+@pytest.mark.parametrize("dtype", [BF16, F16])
 @pytest.mark.parametrize("scale", [-0.5, 0.0, 1e-3, 3.0])
 def test_any_softmax_scale_of_head_size_64(scale, dtype):
     """The scale joins in float32 behind the logits: negative, zero (every visible key weighs the same), small and large."""
