@@ -215,3 +215,16 @@ def test_dense_operator_asks_for_scratch_sizes_on_the_tensors_device(monkeypatch
     fa._backward(q, k, k, out, lse, mask, out, 1.0)
     assert {"ckv_dense_workspace_bytes", "ckv_dense_bwd_split_bytes", "ckv_attn_dense", "ckv_attn_dense_bwd"} <= set(asked)
     assert set(asked.values()) == {q.device}, asked
+
+
+def test_the_stream_handle_comes_from_the_public_call_where_torch_has_no_other(monkeypatch):
+    from types import SimpleNamespace
+
+    from cascading_kv_cache_amd import cascading_cache as cc
+
+    device = torch.device("cuda", 3)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda d: SimpleNamespace(cuda_stream=100 + d.index))
+    monkeypatch.setattr(cc, "_current_raw_stream", None)
+    assert cc.raw_stream(device) == 103
+    monkeypatch.setattr(cc, "_current_raw_stream", lambda index: 200 + index)
+    assert cc.raw_stream(device) == 203
