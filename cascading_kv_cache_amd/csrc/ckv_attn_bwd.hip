@@ -31,8 +31,9 @@ struct BwdParams {
 
 // delta[row] = sum over the head dims of out times dout.  16-bit rows of up to 512 contiguous dims, 16-byte addressable (`lanes`
 // > 0): a row is D / 8 lanes, one 16-byte piece of each tensor apiece; other rows a wavefront, element by element.  The first
-// workgroup sorts the keys beside them, and with 256 threads it was what the launch waited for: 65536 rows of 128 dims and
-// 16384 keys 23 -> 15 us with 1024.
+// workgroup sorts the keys beside them, and with few threads it is what the launch waits for where the rows are few (256, 512 and
+// 1024 threads, us: 66 rows and 16384 cached keys 11.8 10.4 10.2, 2400 rows and 16384 10.2 8.9 8.2, 16384 rows and 8192 8.2 7.2
+// 6.2; 65536 rows and 16384 keys 15.5 13.1 15.2; 2048 keys or less 4 to 5 with any).
 constexpr int kDeltaThreads = 1024;
 template <typename T>
 __global__ void __launch_bounds__(kDeltaThreads) bwd_delta_kernel(BwdParams p, int lanes) {

@@ -650,21 +650,26 @@ __global__ void __launch_bounds__(256, 2) decode_main_mfma_kernel(DecodeParams p
 // ---------------------------------------------------------------------------------------------
 // Streaming variant of the main kernel (16-bit caches, shared positions, G <= 4).
 //
-// The (64-key tile, batch x kv-head) items are dealt out in equal contiguous runs over as many
-// workgroups as the chip holds at once (two per CU), so the launch has no tail.  A workgroup is four
-// wavefronts; each stages 16 key rows of an item.  The rows travel global -> LDS as asynchronous
-// copies one item ahead (two LDS stages), swizzled on the way by the choice of each lane's source
-// piece, so no register holds data in flight and the loads of the next item overlap the arithmetic
-// of this one.  Per item: (1) every wavefront rotates its 16 K rows in registers (cos / sin of the
-// tile's positions stay in registers for all (b, kvh) of the tile) and gets their logits from the
-// matrix pipe; (2) after the item's only workgroup barrier every wavefront normalises all 64 logits
-// of each head (redundantly: 4 values per lane) and (3) multiplies P by a 32-dim slice of all 64 V
-// rows on the matrix pipe, so the tile's partial result is complete in registers and needs no
+// The (128-key tile, batch x kv-head) items, those of a tile behind one another, are dealt out in
+// equal contiguous runs over as many workgroups as the chip holds at once (one per CU), so the launch
+// has no tail.  A workgroup is eight wavefronts; each stages 16 key rows of an item.  The rows travel
+// global -> LDS as asynchronous copies one item ahead (two LDS stages), from tile to tile too,
+// swizzled on the way by the choice of each lane's source piece, so no register holds data in flight
+// and the loads of the next item overlap the arithmetic of this one.  Per item: (1) every wavefront
+// rotates its 16 K rows in registers (cos / sin of the tile's positions stay in registers for all
+// (b, kvh) of the tile) and gets their logits from the matrix pipe; (2) after the item's only
+// workgroup barrier every wavefront normalises all 128 logits of each head (redundantly: 8 values
+// per lane) and (3) multiplies P by a 16-dim slice of all 128 V rows on the matrix pipe, so the
+// tile's partial result is complete in registers and needs no
 // combination across wavefronts.  It is written out at the top of the next item, off the critical
 // path.
 // ---------------------------------------------------------------------------------------------
 constexpr int kStreamThreads = 64 * kStreamWaves;
-constexpr int kOwnQRows = 64;                     // query rows (batch x heads) a workgroup of the streaming kernel rotates itself
+// Query rows (batch x heads) a workgroup of the streaming kernel rotates itself: as many as fit beside its stages in LDS (67), a
+// multiple of eight.  Below the line it pays at every size measured (us a step, own rows and a launch for them, on 2K, 16K and 64K
+// slots): 32 rows 24.8 37.2 76.5 and 27.5 38.9 79.1, 56 rows of 7 heads a kv head 24.3 42.0 86.8 and 26.6 44.1 89.7, 64 rows 28.2
+// 48.7 133.5 and 30.2 50.5 136.0.
+constexpr int kOwnQRows = 64;
 constexpr int kStreamWgPerCu = 8 / kStreamWaves;  // eight wavefronts per CU
 constexpr int kStreamDimBlocks = 8 / kStreamWaves;  // 16-dim blocks of the output a wavefront owns
 constexpr int kStreamStage = 2 * kSK * 256;       // K rows then V rows of one tile (16-bit, 256 B per row)
@@ -703,7 +708,7 @@ __device__ inline float mod4_sum(float l) {
 
 // What the workgroups of a streaming kernel share, by all its threads: the 64 frequencies in LDS and, with few query rows (own_q),
 // all of them rotated there, head g of a kv head with its 16-byte piece c in slot c ^ g.  The rows are a kernel of their own
-// otherwise, whose launch costs a step of one stream 4 us on the device and 3 on the host.  Requested at the start, worked out
+// otherwise, whose launch costs a step two to three us (kOwnQRows).  Requested at the start, worked out
 // while the first rows of the cache are on their way.
 template <typename T, int G>
 struct SharedQueries {

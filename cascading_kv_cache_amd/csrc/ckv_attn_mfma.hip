@@ -19,9 +19,9 @@
 //
 // Precision.  With 128 dims the scale rides on the 16-bit queries and the probabilities enter P.V rounded to the tensor
 // dtype.  With 64 dims nothing but the operands themselves is held in 16 bits (kExact): the logits of the queries as the
-// eager path rounds them are scaled in float32, and a probability enters P.V as three 16-bit terms that add up to its
-// float32 value (one matrix instruction each, all into the same float32 accumulator), so the result is that of float32
-// arithmetic.  8 heads x 1000 rows x 5095 keys in float16: forward 20 -> 28 us, scores 31.5 -> 34 (the vector
+// eager path rounds them are scaled in float32, and a probability enters P.V as three terms of the tensor dtype that
+// add up to its float32 value (one matrix instruction each, all into the same float32 accumulator; float16: to 2^-37 of the
+// row's largest probability, see kHead), so the result is that of float32 arithmetic.  8 heads x 1000 rows x 5095 keys in float16: forward 20 -> 28 us, scores 31.5 -> 34 (the vector
 // kernels, to the same error: 2300 and 521); 32 heads on 8 kv heads, 4096 rows x 16 K slots, the whole call: 1.41 -> 2.02 ms
 // (59).  The vector ALU bounds the forward: seven instructions more per pair of probabilities.
 #include "ckv_attn_internal.h"
@@ -637,7 +637,10 @@ __global__ void __launch_bounds__(512) fwd_pipe_kernel(FwdParams p) {
 #pragma unroll
     for (int v = 0; v < 16; v++) cinit[v] = 0.f;
     // A row's largest probability lies at 2^kHead when its reference is set and stays below 2^kShiftAt until that moves.
-    // 64 dims: high enough that the terms of a probability 2^-26 times that size are float16 numbers of full precision.
+    // 64 dims: as high as float16 allows.  Three float16 terms hold all 24 bits of a probability down to 2^-12 of the row's
+    // largest and resolve 2^-37 of that, which a float16 result can only show in a dim where the values of the row's largest
+    // keys are zero and others' above 2^12.  (bfloat16 terms, which hold every bit, would need V in two halves and twice the
+    // products.)
     constexpr float kShiftAt = kEx ? 15.f : 10.f, kHead = kEx ? 12.f : 0.f;
     const float c2 = p.scale_log2;
     // a logit as it leaves the matrix pipe, as a power of two
@@ -1591,8 +1594,10 @@ int run_mfma(const MfmaProblem& mp, hipStream_t stream) {
         if (mp.shared_pos) {
             // About three workgroups per compute unit (two and three, us: 8 heads x 16897 keys 33.9 and 31.0, 16 x 18496 73 and
             // 68, 8 x 69696 109 and 109); eight where the keys are gathered by an order: those are not rotated, so
-            // there is nothing to reuse from unit to unit, and the tiles of masked keys leave at once (64 heads x 17408 keys,
-            // half of them masked: 164 us with two, 139 with eight, 152 with sixteen).
+            // there is nothing to reuse from unit to unit, and the tiles of masked keys leave at once (two, four, eight and
+            // sixteen, us, half of the cached keys masked: 64 heads x 17408 keys x 128 dims 148 147 130 135, 32 x 8704 x 128
+            // 35.0 34.0 32.6 30.7, 8 x 16684 x 128 16.6 16.8 17.0 17.0, 64 x 2176 x 64 dims 13.6 12.4 12.4 12.7, 8 x 5095 x 64
+            // 9.8 8.6 8.5 8.6).
             const int64_t tiles = n_pad / kBN;
             splits = ((mp.key_order ? 8 : 3) * cus + tiles - 1) / tiles;
             if (splits < 2) splits = 2;
