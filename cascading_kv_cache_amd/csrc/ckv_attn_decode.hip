@@ -550,8 +550,9 @@ __global__ void __launch_bounds__(256, 2) decode_main_mfma_kernel(DecodeParams p
                 const uint32_t* w2 = reinterpret_cast<const uint32_t*>(&kraw[gi][ks + 2]);
                 uint32_t o1[4], o2[4];
 #pragma unroll
-                for (int w = 0; w < 4; w++) {
-                    rw[gi][ks][w].rotate(w1[w], w2[w], p.key_scale, true, o1[w], o2[w]);
+                for (int w = 0; w < 4; w += 2) {
+                    RopeWord<T>::rotate_scaled2(rw[gi][ks][w], rw[gi][ks][w + 1], w1[w], w2[w], w1[w + 1], w2[w + 1], p.key_scale, o1[w], o2[w],
+                                                o1[w + 1], o2[w + 1]);
                 }
                 kop[ks] = make_uint4(o1[0], o1[1], o1[2], o1[3]);
                 kop[ks + 2] = make_uint4(o2[0], o2[1], o2[2], o2[3]);
@@ -1065,8 +1066,9 @@ __global__ void __launch_bounds__(kStreamThreads, kStreamWgPerCu) decode_stream_
                 const uint32_t* w2 = reinterpret_cast<const uint32_t*>(&kraw[ks + 2]);
                 uint32_t o1[4], o2[4];
 #pragma unroll
-                for (int w = 0; w < 4; w++) {
-                    rows.rw[ks][w].rotate(w1[w], w2[w], p.key_scale, true, o1[w], o2[w]);
+                for (int w = 0; w < 4; w += 2) {
+                    RopeWord<T>::rotate_scaled2(rows.rw[ks][w], rows.rw[ks][w + 1], w1[w], w2[w], w1[w + 1], w2[w + 1], p.key_scale, o1[w], o2[w],
+                                                o1[w + 1], o2[w + 1]);
                 }
                 kop[ks] = make_uint4(o1[0], o1[1], o1[2], o1[3]);
                 kop[ks + 2] = make_uint4(o2[0], o2[1], o2[2], o2[3]);
@@ -1341,8 +1343,9 @@ __global__ void __launch_bounds__(kStreamThreads, kStreamWgPerCu) decode_stream_
                 const uint32_t* w2 = reinterpret_cast<const uint32_t*>(&kraw[ks + 2]);
                 uint32_t o1[4], o2[4];
 #pragma unroll
-                for (int w = 0; w < 4; w++) {
-                    rows.rw[ks][w].rotate(w1[w], w2[w], p.key_scale, true, o1[w], o2[w]);
+                for (int w = 0; w < 4; w += 2) {
+                    RopeWord<T>::rotate_scaled2(rows.rw[ks][w], rows.rw[ks][w + 1], w1[w], w2[w], w1[w + 1], w2[w + 1], p.key_scale, o1[w], o2[w],
+                                                o1[w + 1], o2[w + 1]);
                 }
                 kop[ks] = make_uint4(o1[0], o1[1], o1[2], o1[3]);
                 kop[ks + 2] = make_uint4(o2[0], o2[1], o2[2], o2[3]);
