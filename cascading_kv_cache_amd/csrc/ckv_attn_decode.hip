@@ -881,13 +881,13 @@ struct StreamRows {
         if (all_cache) {
             const char* base = slab(1);
 #pragma unroll
-            for (int jb = 0; jb < 4; jb++) async_copy16(base, rel[jb], dst + jb * 1024);
+            for (int jb = 0; jb < 4; jb++) async_copy16_once(base, rel[jb], dst + jb * 1024);
         } else {  // few tiles: the first, the last and those around the ring's ends
             const char *sink = slab(0), *cache = slab(1), *token = slab(2);
 #pragma unroll
             for (int jb = 0; jb < 4; jb++) {
                 const int sg = segment_of(first + 4 * jb + (lane >> 4));
-                async_copy16_from((sg == 0 ? sink : sg == 1 ? cache : token) + rel[jb], dst + jb * 1024);
+                async_copy16_once_from((sg == 0 ? sink : sg == 1 ? cache : token) + rel[jb], dst + jb * 1024);
             }
         }
     }
