@@ -21,13 +21,15 @@
 // 2.0816e-4 and 2.0747e-4 off (relative), which is the rounding of the result; float32 products 2.0956e-4, 2.0816e-4, 2.0747e-4.
 // Before that rounding dq is 2.99e-7 off (8 shapes), bfloat16 3.11e-7; with float32 products 3.69e-7 and 3.61e-7.
 //
-// What bounds them (64 heads x 1024 rows x 8704 visible keys, 128 dims, bf16: dq 548 -> 440 us, dk/dv 770 -> 620).  Vector work
+// What bounds them (64 heads x 1024 rows x 8704 visible keys, 128 dims, bf16: dq 386 us, dk/dv 590).  Vector work
 // beside the matrix work: both take most of a block's time and overlap only where a wavefront alternates them, so an
 // element costs one fused multiply-add, one exponential, one multiplication and half a conversion per product (no
 // subtraction of delta, no scale, no mask in a block that every row sees, no addresses), where it was twice that.  The
 // copies: 100 to 170 cycles each at the issue, whatever else the wavefront does (let out one by one between matrix
-// instructions: dq 514 us, dk/dv level); dq has them two blocks ahead.  At 2.1 GHz and 56 % matrix work dq is within reach
-// of the clock's power limit.  Reads from LDS are not it: 4 instead of 2 matrix instructions ahead, dk/dv level.
+// instructions: dq 514 us, dk/dv level); dq has them 64 keys ahead.  Waiting for them where the work does not need them yet: the
+// compiler put a wait for everything in flight before the first use of registers loaded in front of the loop (arrived; without
+// it dq 436 us, with it 401, by eight wavefronts 386).  Reads from LDS are not it: operands of dK / dV 4 instead of 2 matrix
+// instructions ahead, and of dP 2 instead of 1, dk/dv level; dk/dv by eight wavefronts and 64 rows a barrier 628 us instead of 590.
 //
 // The A operands K^T, Q^T and dO^T are read from the row-major tiles in LDS with the transposing read
 // ds_read_b64_tr_b16: lane i of a 16-lane group receives element [4e + i/4][i%4] (e = 0..3) of the 16 x 4 matrix
@@ -60,7 +62,13 @@ constexpr int kWaves = 4;             // wavefronts of a workgroup, 32 stationar
 constexpr int kThreads = kWaves * CKV_WAVE;
 constexpr int kOwn = kWaves * 32;     // stationary rows of a workgroup
 constexpr int kAhead = 3, kKvAhead = 3;  // matrix instructions between an operand's read from LDS and its use
-constexpr int kDqStages = 3;          // stages of K and V blocks of the dq kernel: copies two blocks ahead
+// Workgroups of the dq kernel: four wavefronts with a block of keys per barrier, two workgroups on a compute unit, or eight with
+// two blocks, one workgroup (wide_dq).  Either way a wavefront copies as much per barrier, 64 keys ahead of their use.
+template <int kDqWaves>
+struct Team {
+    static constexpr int kThreads = kDqWaves * CKV_WAVE, kOwn = kDqWaves * 32, kPerCu = 8 / kDqWaves;
+    static constexpr int kSub = kDqWaves / 4, kRows = kSub * kBlk, kStages = kSub == 1 ? 3 : 2;   // blocks and keys of a stage, stages
+};
 constexpr float kLog2e = 1.4426950408889634f;
 // kSplit: the A operands of the products that P and dS enter come from two bfloat16 tiles beside the tile itself, see Halves
 template <int kHD, bool kSplit = false>
@@ -164,7 +172,7 @@ struct Keys {
     __device__ bool visible(int64_t i) const { return i < n_seen && (order || i >= n_cached || mask[i] == 0); }
 };
 
-// A 32-row block of a (rows, kHD) tensor into a tile, global -> LDS without registers, 1 KiB per instruction; a
+// A block of a (rows, kHD) tensor, eight rows a wavefront, into a tile, global -> LDS without registers, 1 KiB per instruction; a
 // wavefront copies kRowBytes / 128 of them, lane i of copy j one slot of row block_row(wave, lane, j).  Rows past row `last`
 // of the block repeat it (finite values; whatever is computed from them is masked).  The caller waits with vmcnt(0)
 // before the barrier that publishes the tile.
@@ -237,6 +245,14 @@ struct Operands {
         return make_uint4(u[0].x, u[0].y, u[1].x, u[1].y);
     }
 };
+
+// The loads of these registers end here.  The compiler does not see what wait_copies waits for: to it a load in front of a loop
+// may be in flight in every turn, and it waits at the first use there, for the copies issued since as well.
+template <int kN>
+__device__ inline void arrived(uint4 (&regs)[kN]) {
+#pragma unroll
+    for (int i = 0; i < kN; i++) asm volatile("" : "+v"(regs[i].x), "+v"(regs[i].y), "+v"(regs[i].z), "+v"(regs[i].w));
+}
 
 __device__ inline f32x16 zero16() {
     f32x16 z;
@@ -312,10 +328,9 @@ struct Halves {
 #pragma unroll
         for (int i = 0; i < 16; i++) c[db][i] += block[db][i];
     }
-    template <int kTiles>
+    template <int kTiles, int kTile>
     __device__ static void split(unsigned char* lds, uint32_t tile, uint32_t halves, int wave, int lane) {
         if constexpr (kSplit) {
-            constexpr int kTile = Geo<kHD>::kTile;
             const uint32_t at = (uint32_t)(wave * 1024 + lane * 16);
 #pragma unroll
             for (int i = 0; i < kTiles; i++) {
@@ -385,14 +400,16 @@ __device__ inline float keep_if_bit(float v, uint32_t word, int bit) {
 // ---------------------------------------------------------------------------------------------
 // dq
 // ---------------------------------------------------------------------------------------------
-template <typename T, int kHD, bool kWide>
-__global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dq_kernel(BwdMfmaParams p) {
-    constexpr int kTile = Geo<kHD>::kTile, kStage = 2 * kTile;   // K, V
-    constexpr int kCopies = 2 * (kHD / 64);                      // of a wavefront and block
-    constexpr int kMine = kBlk / kWaves;                         // rows of a block that a wavefront copies
+template <typename T, int kHD, bool kWide, int kWaves>
+__global__ void __launch_bounds__(Team<kWaves>::kThreads, Team<kWaves>::kPerCu) bwd_mfma_dq_kernel(BwdMfmaParams p) {
+    constexpr int kOwn = Team<kWaves>::kOwn, kSub = Team<kWaves>::kSub, kRows = Team<kWaves>::kRows, kDqStages = Team<kWaves>::kStages;
+    constexpr int kBlkBytes = Geo<kHD>::kTile, kTile = kSub * kBlkBytes, kStage = 2 * kTile;   // K, V
+    constexpr int kCopies = 2 * (kHD / 64);                      // of a wavefront and stage
+    constexpr int kMine = kRows / kWaves;                        // rows of a stage that a wavefront copies
     typedef Halves<T, kHD> Half;                                 // of K: two tiles per stage
     constexpr uint32_t kHalves = kDqStages * kStage, kRowNumbers = kHalves + (Half::kSplit ? kDqStages * 2 * kTile : 0);
-    __shared__ __attribute__((aligned(16))) unsigned char smem[kRowNumbers + kDqStages * kBlk * (int)sizeof(int)];
+    extern __shared__ __attribute__((aligned(16))) unsigned char dyn_smem[];   // dq_lds of them
+    unsigned char* const smem = dyn_smem;
     const ckv_dense_bwd_args& a = p.a;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / CKV_WAVE), lane = tid % CKV_WAVE, h = lane >> 5;
     const Keys keys(p);
@@ -423,6 +440,8 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dq_kernel(BwdMfmaParams 
             }
         }
     }
+    arrived(qreg);
+    arrived(greg);
     const bool row_ok = m_lane < n_ctx;
     // The magnitude of the softmax scale rides on the exponent (nothing here needs P without it), its sign on the result;
     // the products of V and dO start from -delta.  That leaves one multiplication per element beside the exponential.
@@ -446,27 +465,27 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dq_kernel(BwdMfmaParams 
     // keys past the diagonal of the workgroup's last row are visible to none of its rows
     int m_last = m_wg + kOwn - 1;
     if (m_last > (int)n_ctx - 1) m_last = (int)n_ctx - 1;
-    const int nblk_all = (int)(((int64_t)n_cached + m_last + kBlk) / kBlk);
+    const int nblk_all = (int)(((int64_t)n_cached + m_last + kRows) / kRows);   // stages of them
     // this workgroup's share of them: an equal stretch (an empty one leaves zeros)
     const int per_share = (nblk_all + p.n_split - 1) / p.n_split;
     const int blk0 = share * per_share, nblk = blk0 + per_share < nblk_all ? blk0 + per_share : nblk_all;
 
-    // Blocks are copied two ahead into three stages.  With an order the row numbers of a wavefront's eight rows of a block
-    // come to LDS the same way, three blocks ahead, so that no load in the loop is one whose result the compiler would
+    // Stages are copied 64 rows ahead.  With an order the row numbers of a wavefront's eight rows of a stage
+    // come to LDS the same way, one stage earlier, so that no load in the loop is one whose result the compiler would
     // wait for together with the copies behind it.
     const uint32_t mine = lds0 + kRowNumbers + (uint32_t)(wave * kMine * (int)sizeof(int));
-    constexpr uint32_t kSlot = kBlk * sizeof(int);
+    constexpr uint32_t kSlot = kRows * sizeof(int);
     const int mine_lane = kHD == 128 ? lane / 16 : lane / 8;   // of copy 0; copy j takes row 4 j + this one
     auto clamped = [&](int i) { return i < n_seen ? i : n_seen - 1; };   // a chunk key: finite values, and no query looks at this copy
     auto request_rows = [&](int blk, int slot) {
         if (keys.order && lane < kMine)
-            async_copy4(keys.order, (uint32_t)clamped(blk * kBlk + wave * kMine + lane) * 4u, mine + (uint32_t)slot * kSlot);
+            async_copy4(keys.order, (uint32_t)clamped(blk * kRows + wave * kMine + lane) * 4u, mine + (uint32_t)slot * kSlot);
     };
     auto rows_of = [&](int blk, int slot, uint32_t(&r)[kHD / 64]) {
 #pragma unroll
         for (int j = 0; j < kHD / 64; j++)
             r[j] = keys.order ? *(const __attribute__((address_space(3))) uint32_t*)(uintptr_t)(mine + (uint32_t)slot * kSlot + (uint32_t)(4 * j + mine_lane) * 4u)
-                              : (uint32_t)clamped(blk * kBlk + wave * kMine + 4 * j + mine_lane);
+                              : (uint32_t)clamped(blk * kRows + wave * kMine + 4 * j + mine_lane);
     };
     auto copy = [&](const uint32_t(&r)[kHD / 64], int st) {
         copy_rows<kHD, kWide>(kb, row_bytes, r, lds0 + (uint32_t)(st * kStage), wave, lane);
@@ -479,23 +498,19 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dq_kernel(BwdMfmaParams 
         wait_copies<0>();
         rows_of(blk0, 0, rows_next);
         copy(rows_next, 0);
-        rows_of(blk0 + 1, 1, rows_next);
-        if (blk0 + 1 < nblk) copy(rows_next, 1);
-        rows_of(blk0 + 2, 2, rows_next);
-        if (blk0 + 1 < nblk) wait_copies<kCopies>();
+        if constexpr (kDqStages == 3) {
+            rows_of(blk0 + 1, 1, rows_next);
+            if (blk0 + 1 < nblk) copy(rows_next, 1);
+        }
+        rows_of(blk0 + kDqStages - 1, kDqStages - 1, rows_next);
+        if (kDqStages == 3 && blk0 + 1 < nblk) wait_copies<kCopies>();
         else wait_copies<0>();
-        Half::template split<1>(smem, 0, kHalves, wave, lane);
+        Half::template split<1, kTile>(smem, 0, kHalves, wave, lane);
     }
     __syncthreads();
-    auto step = [&](auto stage_tag, int blk) {
-        constexpr int st = decltype(stage_tag)::value;
-        constexpr uint32_t kt = st * kStage, vt = kt + kTile;
-        const int n0 = blk * kBlk;
-        const bool more = blk + 2 < nblk;
-        if (more) {  // the stage was last read before the barrier that ended the step before
-            request_rows(blk + 3, st);
-            copy(rows_next, (st + 2) % kDqStages);
-        }
+    // 32 keys from position n0 on, whose tiles begin at byte kt of the stages (K) and vt (V)
+    auto block = [&](auto tile_tag, auto halves_tag, int n0) {
+        constexpr uint32_t kt = decltype(tile_tag)::value, vt = kt + kTile;
         // Which keys of the block any query may see: all of them in front of the chunk when they were sorted.
         uint32_t vis = 0xffffffffu;
         if (!keys.order) vis = (uint32_t)__ballot(keys.visible(n0 + (lane & 31)));
@@ -507,7 +522,7 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dq_kernel(BwdMfmaParams 
         constexpr int kRow = kHD / 16, kDB = kHD / 32;
         if (!dead) {
             f32x16 s = zero16(), dp = neg_delta;
-            constexpr uint32_t ct = Half::kSplit ? kHalves + st * 2 * kTile : kt;
+            constexpr uint32_t ct = Half::kSplit ? decltype(halves_tag)::value : kt;
             uint4 ops[2 * kRow], cops[Half::kOps][2 * kDB];
             auto row_op = [&](int k) { return op.row_op(k < kRow ? kt : vt, k % kRow); };
             auto col_op = [&](int k) {
@@ -558,13 +573,13 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dq_kernel(BwdMfmaParams 
             }
             if (!outside) {
                 Weights<T, kHD> bop;
-                f32x16 block[kDB];
+                f32x16 sums[kDB];
                 bop.set(dsv, 0);
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int k = 0; k < 2 * kDB; k++) {
                     if (k + kAhead < 2 * kDB) col_op(k + kAhead);
-                    Half::accumulate(bop, cops, k, dq, block);
+                    Half::accumulate(bop, cops, k, dq, sums);
                     if (kHD == 128 && k < kDB) {
 #pragma unroll
                         for (int i = 8 + k * (8 / kDB); i < 8 + (k + 1) * (8 / kDB); i++) dsv[i] = s[i] * dp[i];
@@ -572,24 +587,38 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dq_kernel(BwdMfmaParams 
                     if (k == (kHD == 128 ? kDB - 1 : 0)) bop.set(dsv, 1);
                     __builtin_amdgcn_sched_barrier(0);
                 }
-                Half::finish(dq, block);
+                Half::finish(dq, sums);
             }
         }
         __builtin_amdgcn_sched_barrier(0);
+    };
+    auto step = [&](auto stage_tag, int blk) {
+        constexpr int st = decltype(stage_tag)::value;
+        const bool more = blk + kDqStages - 1 < nblk;
+        if (more) {  // the stage was last read before the barrier that ended the step before
+            request_rows(blk + kDqStages, st);
+            copy(rows_next, (st + kDqStages - 1) % kDqStages);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        block(std::integral_constant<uint32_t, st * kStage>{}, std::integral_constant<uint32_t, kHalves + st * 2 * kTile>{}, blk * kRows);
+        if constexpr (kSub == 2)
+            block(std::integral_constant<uint32_t, st * kStage + kBlkBytes>{}, std::integral_constant<uint32_t, kHalves + st * 2 * kTile + kBlkBytes>{},
+                  blk * kRows + kBlk);
         if (more) {   // this wavefront's copies of the next block have landed, and the row numbers requested above
-            wait_copies<kCopies>();
-            rows_of(blk + 3, st, rows_next);
+            wait_copies<(kDqStages - 2) * kCopies>();
+            rows_of(blk + kDqStages, st, rows_next);
         } else {
             wait_copies<0>();
         }
         // the halves of a stage were last read two barriers ago
-        if (blk + 1 < nblk) Half::template split<1>(smem, (st + 1) % kDqStages * kStage, kHalves + (st + 1) % kDqStages * 2 * kTile, wave, lane);
+        if (blk + 1 < nblk) Half::template split<1, kTile>(smem, (st + 1) % kDqStages * kStage, kHalves + (st + 1) % kDqStages * 2 * kTile, wave, lane);
         __syncthreads();
     };
     for (int blk = blk0; blk < nblk; blk += kDqStages) {
         step(std::integral_constant<int, 0>{}, blk);
         if (blk + 1 < nblk) step(std::integral_constant<int, 1>{}, blk + 1);
-        if (blk + 2 < nblk) step(std::integral_constant<int, 2>{}, blk + 2);
+        if constexpr (kDqStages == 3)
+            if (blk + 2 < nblk) step(std::integral_constant<int, 2>{}, blk + 2);
     }
     if (a.scale < 0.f) {
 #pragma unroll
@@ -727,7 +756,7 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dkdv_kernel(BwdMfmaParam
         if (wave == 0) park(row_scalar(blk0 * kBlk), 0);
     }
     wait_copies<0>();
-    if (blk0 < nblk) Half::template split<2>(dyn_smem, 0, G::kDkdvHalves, wave, lane);
+    if (blk0 < nblk) Half::template split<2, kTile>(dyn_smem, 0, G::kDkdvHalves, wave, lane);
     __syncthreads();
     auto step = [&](auto stage_tag, int blk) {
         constexpr int st = decltype(stage_tag)::value;
@@ -888,7 +917,7 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dkdv_kernel(BwdMfmaParam
         wait_copies<0>();  // this wavefront's copies of the next block have landed
         if (more) {
             if (wave == 0) park(rv_next, st ^ 1);
-            Half::template split<2>(dyn_smem, (st ^ 1) * 2 * kTile, G::kDkdvHalves + (st ^ 1) * 4 * kTile, wave, lane);
+            Half::template split<2, kTile>(dyn_smem, (st ^ 1) * 2 * kTile, G::kDkdvHalves + (st ^ 1) * 4 * kTile, wave, lane);
         }
         __syncthreads();
     };
@@ -941,6 +970,22 @@ inline bool rows_ok(const int64_t* st) {
     return st[3] == 1 && st[2] % 8 == 0 && st[1] % 8 == 0 && st[0] % 8 == 0 && st[2] > 0 && st[2] < (1 << 24);
 }
 
+template <typename T, int kHD, int kWaves>
+constexpr int dq_lds() {
+    constexpr int kTile = Team<kWaves>::kSub * Geo<kHD>::kTile;
+    return Team<kWaves>::kStages * (2 * kTile + (Halves<T, kHD>::kSplit ? 2 * kTile : 0) + Team<kWaves>::kRows * (int)sizeof(int));
+}
+
+// Eight wavefronts where their workgroups leave no more rows empty than those of four and there is one for every compute unit.
+// K and V then reach a unit's LDS once instead of once per workgroup of four, and a barrier comes every 64 keys: 64 heads x 1024
+// rows x 8704 visible keys, 128 dims 401 -> 386 us; x 8192 keys, 64 dims, bf16 308 -> 286, float16 436 -> 395; 8 heads x 1000 x
+// 4071 keys, 64 dims, in 8 shares 42.8 -> 41.7; 32 x 512 x 4608 in 4 shares level.  Elsewhere four: 300 rows (a wide workgroup of
+// 256 and one of 44) 45.6 us, wide 76.8; 2 heads x 1024 rows in 8 shares (64 wide workgroups) 27.0, wide 36.6.
+inline bool wide_dq(const ckv_dense_bwd_args& a, int n_split) {
+    const int64_t wide = (a.n_ctx + Team<8>::kOwn - 1) / Team<8>::kOwn, narrow = (a.n_ctx + Team<4>::kOwn - 1) / Team<4>::kOwn;
+    return 2 * wide == narrow && wide * a.B * a.H * n_split >= mfma_device_cus();
+}
+
 template <typename T, int kHD>
 int run(const BwdMfmaParams& p_in, hipStream_t stream) {
     BwdMfmaParams p = p_in;
@@ -951,10 +996,25 @@ int run(const BwdMfmaParams& p_in, hipStream_t stream) {
         p.per_head = by_xcd ? (int)per_head : 0;
         return by_xcd ? dim3((unsigned)(heads * per_head)) : dim3((unsigned)per_head, (unsigned)heads);
     };
-    const dim3 grid_dq = grid_of((a.n_ctx + kOwn - 1) / kOwn * p.n_split, 0x7fffffff);
-    if (a.n_kv * a.kv_stride[2] * 2 < (int64_t)1 << 32) hipLaunchKernelGGL((bwd_mfma_dq_kernel<T, kHD, false>), grid_dq, dim3(kThreads), 0, stream, p);
-    else hipLaunchKernelGGL((bwd_mfma_dq_kernel<T, kHD, true>), grid_dq, dim3(kThreads), 0, stream, p);
-    CKV_HIP_TRY(hipGetLastError());
+    auto launch_dq = [&](auto waves_tag, auto wide_rows_tag) -> int {
+        constexpr int kWaves = decltype(waves_tag)::value, kOwn = Team<kWaves>::kOwn;
+        constexpr int kLds = dq_lds<T, kHD, kWaves>();
+        auto* kernel = bwd_mfma_dq_kernel<T, kHD, decltype(wide_rows_tag)::value, kWaves>;
+        if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(kernel), kLds)) return rc;
+        const dim3 grid = grid_of((a.n_ctx + kOwn - 1) / kOwn * p.n_split, 0x7fffffff);
+        hipLaunchKernelGGL(kernel, grid, dim3(Team<kWaves>::kThreads), kLds, stream, p);
+        CKV_HIP_TRY(hipGetLastError());
+        return CKV_OK;
+    };
+    constexpr std::integral_constant<int, 4> narrow{};
+    constexpr std::integral_constant<int, 8> wide{};
+    if (a.n_kv * a.kv_stride[2] * 2 >= (int64_t)1 << 32) {
+        if (int rc = launch_dq(narrow, std::true_type{})) return rc;
+    } else if (wide_dq(a, p.n_split)) {
+        if (int rc = launch_dq(wide, std::false_type{})) return rc;
+    } else if (int rc = launch_dq(narrow, std::false_type{})) {
+        return rc;
+    }
     if (p.n_split > 1) {
         const int64_t threads = a.B * a.H * a.n_ctx * (kHD / 4);
         hipLaunchKernelGGL((bwd_dq_sum_kernel<T, kHD>), dim3((unsigned)((threads + kThreads - 1) / kThreads)), dim3(kThreads), 0,
@@ -987,7 +1047,8 @@ bool bwd_mfma_supported(const ckv_dense_bwd_args& a) {
 // about two workgroups per compute unit in all, and the shares (float32) are added up by a kernel behind.  8 heads x 1000
 // rows are 64 workgroups, a quarter of the chip.
 int bwd_mfma_dq_splits(int64_t B, int64_t H, int64_t n_ctx, int64_t n_kv, int cus) {
-    const int64_t wgs = (n_ctx + kOwn - 1) / kOwn * B * H, blocks = (n_kv + kBlk - 1) / kBlk;
+    constexpr int kDqRows = Team<4>::kOwn;
+    const int64_t wgs = (n_ctx + kDqRows - 1) / kDqRows * B * H, blocks = (n_kv + kBlk - 1) / kBlk;
     if (wgs >= cus) return 1;
     int64_t s = 2 * (int64_t)cus / wgs;
     if (s > blocks / 8) s = blocks / 8;

@@ -511,6 +511,41 @@ def test_backward_on_the_matrix_cores(Z, H, N_CTX, N_KV, masking, layout, dtype)
     check_backward_against_autograd(q, k, v, mask, dtype)
 
 
+@pytest.mark.parametrize("Z,H,N_CTX,N_KV", [(4, 64, 129, 129 + 95), (4, 64, 250, 250), (2, 32, 256, 1025 + 256), (2, 32, 400, 1190 + 400)])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_backward_dq_by_eight_wavefronts(Z, H, N_CTX, N_KV, D, dtype):
+    """Heads enough for a workgroup of 256 query rows on every compute unit, with and without shares of the keys: the last
+    workgroup short of rows, 64-key stages whose second half lies past the last visible key or on the diagonal.  dq against
+    float64, with the rounded out in delta as the operator defines it: P, dS and the result are rounded at most once each, half a unit (2^-9 or 2^-12) at the most,
+    relative to all rows; for one row relative to it and to the rows' root mean square (a row whose few keys cancel is
+    smaller than what was rounded)."""
+    from cascading_kv_cache_amd.flash_attention import attention
+
+    torch.manual_seed(23)
+
+    def leaf(n):
+        return torch.empty((Z, n, H, D), dtype=dtype, device="cuda").normal_(mean=0.0, std=0.5).transpose(1, 2).requires_grad_()
+
+    q, k, v = leaf(N_CTX), leaf(N_KV), leaf(N_KV)
+    mask = torch.rand(N_KV - N_CTX, device="cuda") > 0.5
+    dout = torch.randn_like(q)
+    out, _ = attention(q, k, v, True, 0.125, mask, 1.0)
+    dq, = torch.autograd.grad(out, (q,), dout)
+    hidden = torch.cat((mask[None, :].expand(N_CTX, -1),
+                        torch.ones(N_CTX, N_CTX, dtype=torch.bool, device="cuda").triu(1)), dim=-1)
+    bound = 3 * (2.0 ** -9 if dtype == torch.bfloat16 else 2.0 ** -12)
+    for z in range(Z):
+        q64, k64, v64, do64 = (t[z].detach().double().contiguous() for t in (q, k, v, dout))
+        p = torch.softmax((q64 @ k64.transpose(1, 2).contiguous() * 0.125).masked_fill(hidden, float("-inf")), dim=-1)
+        dp = do64 @ v64.transpose(1, 2).contiguous()
+        delta = (out[z].detach().double() * do64).sum(-1, keepdim=True)
+        want = (p * (dp - delta) * 0.125) @ k64
+        err, size = (dq[z].double() - want).norm(dim=-1), want.norm(dim=-1)
+        assert (err.norm() / size.norm()).item() <= bound
+        assert (err / (size + size.square().mean().sqrt())).max().item() <= bound
+
+
 @pytest.mark.parametrize("flavour", ["llama", "qwen2"])
 def test_reference_mixin_surface(flavour):
     """A layer written the way the reference's model files use the mixin — ``get_vals``, ``self.rope`` on queries,
