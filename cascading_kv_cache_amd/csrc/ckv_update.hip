@@ -25,6 +25,8 @@
 // slot depends on scores, and that is decided inside the group of arrivals between two inserts.
 #include "ckv_common.h"
 
+#include <type_traits>
+
 #include <mutex>
 
 namespace ckv {
@@ -730,12 +732,33 @@ __device__ inline void commit_trackers(const UpdateParams& p, const Unit& u) {
     if (threadIdx.x == 0) A.stored_sinks[u.n * A.stored_sinks_stride[0] + u.h * A.stored_sinks_stride[1]] = p.sinks_new[u.bh];
 }
 
-// One 16-byte piece of a row per lane.
+// One 16-byte piece of a row per lane.  kOnce: rows are read and written past the L2 (non-temporal).  Nothing here looks at them
+// twice, and the words that do go round in it (chains, position ids, scores) stay: 4096 tokens x 8 units into 64 K slots, the moves
+// 25.0 -> 22.8 us (loads alone 23.5, stores alone 24.3); 2048 x 16 into 16 K 23.1 -> 22.7.  Not for a cache that would stay in the
+// L2 until the next call (kOnceBytes): 256 tokens x 8 units into 512 float32 slots, the next chunk's staging 10.5 -> 11.4.
 struct RowPiece {
     uint4 k, v;
 };
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+template <bool kOnce>
+__device__ inline uint4 load_piece(const char* row, int lane) {
+    if constexpr (!kOnce) return reinterpret_cast<const uint4*>(row)[lane];
+    const u32x4 v = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(row) + lane);
+    return make_uint4(v[0], v[1], v[2], v[3]);
+}
+template <bool kOnce>
+__device__ inline void store_piece(char* row, int lane, const uint4& x) {
+    if constexpr (!kOnce) {
+        reinterpret_cast<uint4*>(row)[lane] = x;
+        return;
+    }
+    const u32x4 v = {x.x, x.y, x.z, x.w};
+    __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(row) + lane);
+}
 
-template <int LANES>
+constexpr int64_t kOnceBytes = 32 << 20;   // of K and V in all slots of the call's units: the eight L2s together
+
+template <int LANES, bool kOnce>
 __global__ void ckv_update_apply_vec_kernel(UpdateParams p) {
     const ckv_update_args& A = p.a;
     constexpr int kGroups = 256 / LANES;
@@ -768,16 +791,16 @@ __global__ void ckv_update_apply_vec_kernel(UpdateParams p) {
     carry.k = make_uint4(0, 0, 0, 0);
     carry.v = make_uint4(0, 0, 0, 0);
     if (active) {
-        carry.k = reinterpret_cast<const uint4*>(kin)[lane];
-        carry.v = reinterpret_cast<const uint4*>(vin)[lane];
+        carry.k = load_piece<kOnce>(kin, lane);
+        carry.v = load_piece<kOnce>(vin, lane);
     }
 
     if (d >= S) {  // sink slot (cascading_cache.py:61-109)
         const int64_t j = d - S;
         const int64_t so = (n * A.sink_stride[0] + h * A.sink_stride[1] + j * A.sink_stride[2]) * es;
         if (active) {
-            reinterpret_cast<uint4*>(reinterpret_cast<char*>(A.sink_k) + so)[lane] = carry.k;
-            reinterpret_cast<uint4*>(reinterpret_cast<char*>(A.sink_v) + so)[lane] = carry.v;
+            store_piece<kOnce>(reinterpret_cast<char*>(A.sink_k) + so, lane, carry.k);
+            store_piece<kOnce>(reinterpret_cast<char*>(A.sink_v) + so, lane, carry.v);
         }
         if (lane == 0) {
             A.sink_pos[n * A.sink_pos_stride[0] + h * A.sink_pos_stride[1] + j * A.sink_pos_stride[2]] = j;
@@ -825,8 +848,8 @@ __global__ void ckv_update_apply_vec_kernel(UpdateParams p) {
             o_og[j] = 0;
             if (sl[j] >= 0 && succ >= 0) {  // the displaced row lives on elsewhere: pick it up
                 if (active) {
-                    old[j].k = reinterpret_cast<const uint4*>(ck + (int64_t)sl[j] * row_bytes)[lane];
-                    old[j].v = reinterpret_cast<const uint4*>(cv + (int64_t)sl[j] * row_bytes)[lane];
+                    old[j].k = load_piece<kOnce>(ck + (int64_t)sl[j] * row_bytes, lane);
+                    old[j].v = load_piece<kOnce>(cv + (int64_t)sl[j] * row_bytes, lane);
                 }
                 if (lane == 0) {
                     const int64_t sidx = cs_base + (int64_t)sl[j] * A.cache_s_stride[2];
@@ -843,8 +866,8 @@ __global__ void ckv_update_apply_vec_kernel(UpdateParams p) {
             const uint32_t w_score = j == 0 ? c_score : o_score[j - 1];
             const int64_t w_og = j == 0 ? c_og : o_og[j - 1];
             if (active) {
-                reinterpret_cast<uint4*>(ck + (int64_t)sl[j] * row_bytes)[lane] = src.k;
-                reinterpret_cast<uint4*>(cv + (int64_t)sl[j] * row_bytes)[lane] = src.v;
+                store_piece<kOnce>(ck + (int64_t)sl[j] * row_bytes, lane, src.k);
+                store_piece<kOnce>(cv + (int64_t)sl[j] * row_bytes, lane, src.v);
             }
             if (lane == 0) {
                 const int64_t sidx = cs_base + (int64_t)sl[j] * A.cache_s_stride[2];
@@ -1229,15 +1252,20 @@ int run_update(const ckv_update_args& A, void* workspace, hipStream_t stream) {
             const dim3 block(256);
             p.apply_blocks = (ksub + 256 / lanes - 1) / (256 / lanes);
             const dim3 grid((unsigned)p.apply_blocks + pos_blocks, H, N);
-            switch (lanes) {
-                case 1: launch_timed(CKV_STAGE_APPLY, ckv_update_apply_vec_kernel<1>, grid, block, 0, stream, p); break;
-                case 2: launch_timed(CKV_STAGE_APPLY, ckv_update_apply_vec_kernel<2>, grid, block, 0, stream, p); break;
-                case 4: launch_timed(CKV_STAGE_APPLY, ckv_update_apply_vec_kernel<4>, grid, block, 0, stream, p); break;
-                case 8: launch_timed(CKV_STAGE_APPLY, ckv_update_apply_vec_kernel<8>, grid, block, 0, stream, p); break;
-                case 16: launch_timed(CKV_STAGE_APPLY, ckv_update_apply_vec_kernel<16>, grid, block, 0, stream, p); break;
-                case 32: launch_timed(CKV_STAGE_APPLY, ckv_update_apply_vec_kernel<32>, grid, block, 0, stream, p); break;
-                default: launch_timed(CKV_STAGE_APPLY, ckv_update_apply_vec_kernel<64>, grid, block, 0, stream, p); break;
-            }
+            auto launch = [&](auto once_tag) {
+                constexpr bool kOnce = decltype(once_tag)::value;
+                switch (lanes) {
+                    case 1: launch_timed(CKV_STAGE_APPLY, ckv_update_apply_vec_kernel<1, kOnce>, grid, block, 0, stream, p); break;
+                    case 2: launch_timed(CKV_STAGE_APPLY, ckv_update_apply_vec_kernel<2, kOnce>, grid, block, 0, stream, p); break;
+                    case 4: launch_timed(CKV_STAGE_APPLY, ckv_update_apply_vec_kernel<4, kOnce>, grid, block, 0, stream, p); break;
+                    case 8: launch_timed(CKV_STAGE_APPLY, ckv_update_apply_vec_kernel<8, kOnce>, grid, block, 0, stream, p); break;
+                    case 16: launch_timed(CKV_STAGE_APPLY, ckv_update_apply_vec_kernel<16, kOnce>, grid, block, 0, stream, p); break;
+                    case 32: launch_timed(CKV_STAGE_APPLY, ckv_update_apply_vec_kernel<32, kOnce>, grid, block, 0, stream, p); break;
+                    default: launch_timed(CKV_STAGE_APPLY, ckv_update_apply_vec_kernel<64, kOnce>, grid, block, 0, stream, p); break;
+                }
+            };
+            if (A.N * A.H * A.max_seq_len * A.HID * es * 2 >= kOnceBytes) launch(std::true_type{});
+            else launch(std::false_type{});
         } else {
             const dim3 block(256);
             p.apply_blocks = (ksub + 3) / 4;
