@@ -587,30 +587,7 @@ __global__ void __launch_bounds__(512) fwd_pipe_kernel(FwdParams p) {
     int* list_lds = reinterpret_cast<int*>(smem + kPipeLds + 8 * tiles_cap);
     const uint32_t smem_addr = lds_address(smem);
 
-    // ---- work list: tiles with at least one visible key; bit 31 marks tiles that need masking
-    for (int i = tid; i < n_tiles; i += kThreads) vis_lds[i] = p.tile_vis[i];
-    __syncthreads();
-    if (wave == 0) {
-        int cnt = 0;
-        for (int base = 0; base < n_tiles; base += 64) {
-            const int t = base + lane;
-            const unsigned long long v = t < n_tiles ? vis_lds[t] : 0ull;
-            const unsigned long long bal = __ballot(v != 0ull);
-            if (v != 0ull) {
-                const bool partial = (v != ~0ull) || (t * kBN + kBN - 1 - Nc > m0);
-                list_lds[cnt + __popcll(bal & ((1ull << lane) - 1ull))] = t | (partial ? (int)0x80000000 : 0);
-            }
-            cnt += __popcll(bal);
-        }
-        if (lane == 0) list_lds[tiles_cap] = cnt;
-    }
-    __syncthreads();
-    const int n_work_all = __builtin_amdgcn_readfirstlane(list_lds[tiles_cap]);
-    const int j_first = n_work_all * split_i / p.n_split;
-    const int n_work = n_work_all * (split_i + 1) / p.n_split - j_first;
-    list_lds += j_first;
-
-    // ---- the query row this lane owns as MFMA column `col`
+    // ---- the query row this lane owns as MFMA column `col`, requested first: its trip to memory is that of the words below
     int row_m;
     uint4 qreg[kKK];
     {
@@ -625,6 +602,47 @@ __global__ void __launch_bounds__(512) fwd_pipe_kernel(FwdParams p) {
             qreg[kk] = row_ok ? *reinterpret_cast<const uint4*>(qrow + 16 * kk + 8 * half) : make_uint4(0, 0, 0, 0);
         }
     }
+    // ---- work list: tiles with at least one visible key; bit 31 marks tiles that need masking.  Every wavefront counts a stretch
+    // of the tiles and then writes its entries behind those of the stretches before it.
+    constexpr int kWaves = kThreads / CKV_WAVE;
+    int* counts = reinterpret_cast<int*>(smem);   // of the wavefronts; no copy is on its way yet
+    const int per_wave = (n_tiles + 64 * kWaves - 1) / (64 * kWaves) * 64;
+    const int t_first = wave * per_wave, t_last = t_first + per_wave < n_tiles ? t_first + per_wave : n_tiles;
+    int mine = 0;
+    for (int base = t_first; base < t_last; base += 64) {
+        const int t = base + lane;
+        const unsigned long long v = t < t_last ? p.tile_vis[t] : 0ull;
+        if (t < t_last) vis_lds[t] = v;
+        mine += __popcll(__ballot(v != 0ull));
+    }
+    if (lane == 0) counts[wave] = mine;
+    __syncthreads();
+    int cnt = 0, n_work_all = 0;
+#pragma unroll
+    for (int w = 0; w < kWaves; w++) {
+        const int c = __builtin_amdgcn_readfirstlane(counts[w]);
+        if (w < wave) cnt += c;
+        n_work_all += c;
+    }
+    for (int base = t_first; base < t_last; base += 64) {
+        const int t = base + lane;
+        const unsigned long long v = t < t_last ? vis_lds[t] : 0ull;
+        const unsigned long long bal = __ballot(v != 0ull);
+        if (v != 0ull) {
+            const bool partial = (v != ~0ull) || (t * kBN + kBN - 1 - Nc > m0);
+            list_lds[cnt + __popcll(bal & ((1ull << lane) - 1ull))] = t | (partial ? (int)0x80000000 : 0);
+        }
+        cnt += __popcll(bal);
+    }
+    __syncthreads();
+    // The query rows are there (the words were behind them): said here, or the compiler waits for them at their first use, where
+    // the copies are on their way too.
+#pragma unroll
+    for (int kk = 0; kk < kKK; kk++) asm volatile("" : "+v"(qreg[kk].x), "+v"(qreg[kk].y), "+v"(qreg[kk].z), "+v"(qreg[kk].w));
+    const int j_first = n_work_all * split_i / p.n_split;
+    const int n_work = n_work_all * (split_i + 1) / p.n_split - j_first;
+    list_lds += j_first;
+
     f32x16 oacc[kDB];
 #pragma unroll
     for (int dt = 0; dt < kDB; dt++)
@@ -903,20 +921,24 @@ __global__ void __launch_bounds__(512) fwd_pipe_kernel(FwdParams p) {
     uint4 pre[kAhead];
     if (n_work > 0) {
 #pragma unroll
+        for (int j = 0; j < kBlocksPerWave; j++) copy_k(work(0) & 0x7fffffff, 0, j);
+#pragma unroll
+        for (int j = 0; j < kBlocksPerWave; j++) copy_k(work(1) & 0x7fffffff, 1, j);
+#pragma unroll
+        for (int j = 0; j < kBlocksPerWave; j++) copy_v(work(0) & 0x7fffffff, 0, j);
+#pragma unroll
         for (int j = 0; j < kBlocksPerWave; j++) {
-            copy_k(work(0) & 0x7fffffff, 0, j);
-            copy_k(work(1) & 0x7fffffff, 1, j);
             copy_k(work(2) & 0x7fffffff, 2, j);
-            copy_v(work(0) & 0x7fffffff, 0, j);
             copy_v(work(1) & 0x7fffffff, 1, j);
         }
-        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+        __builtin_amdgcn_s_waitcnt(0x0F70 + 4 * kBlocksPerWave);  // vmcnt: the first K tile is there
         __syncthreads();
         qk(sA);
         advance_k();
         // iteration 0: nothing to multiply by V yet.  e0 .. e3: work-list entries of tiles i .. i+3
         auto clamp_idx = [&](int j) { return j < n_work ? j : n_work - 1; };
         int e0 = work(0), e1 = work(1), e2 = work(2), e3 = work(3), e4 = 0;
+        __builtin_amdgcn_s_waitcnt(0x0F70 + 2 * kBlocksPerWave);  // the second one and the first V^T tile too
         __syncthreads();                     // every wavefront is done with K stage 0
         iteration(std::false_type{}, e0, e2 & 0x7fffffff, e3 & 0x7fffffff, sA, sB, pre, clamp_idx(4), e4);
         // all copies but those of the iteration just finished have landed
@@ -998,21 +1020,45 @@ __global__ void __launch_bounds__(512) fwd_pipe_kernel(FwdParams p) {
     const float l_tot = l_run + __shfl_xor(l_run, 32);
     if (p.n_split > 1) {
         // a share of the key tiles: the row normalised by the share's own sum, and the share's normaliser
-        const int rf_p = qt_i * kRows + wave * 32 + col;
-        const int64_t row_p = (b * p.H + kvh * p.G + rf_p % p.G) * p.Q + row_m;
-        if (row_m < p.Q) {
-            const bool any = l_tot != 0.f;   // a NaN is not nothing: it has to reach the merge
-            const float inv_p = any ? 1.f / l_tot : 0.f;
-            float* po = p.part_o + ((int64_t)split_i * p.B * p.H * p.Q + row_p) * kD;
+        auto row_of = [&](int r, int& m) {   // of part_o and part_l2: row r of this wavefront's 32, at position m
+            const int rf = qt_i * kRows + wave * 32 + r;
+            m = rf / p.G;
+            return (int64_t)split_i * p.B * p.H * p.Q + (b * p.H + kvh * p.G + rf % p.G) * p.Q + m;
+        };
+        const bool any = l_tot != 0.f;   // a NaN is not nothing: it has to reach the merge
+        const float inv_p = any ? 1.f / l_tot : 0.f;
+        // Through LDS, half of the dims at a time, so that a store is whole stretches of 256 (128) bytes of four (eight) rows: a
+        // lane's own 16 bytes have one neighbour in each of 32 rows (with the start above, 32 heads x 509 rows x 16897 keys in 8
+        // shares: 145.5 -> 142.8 us).
+        constexpr int kStep = kD / 2, kLanes = kStep / 4, kPassRows = CKV_WAVE / kLanes;
+        constexpr int kPitch = 4 * kStep + 16;   // bytes; the pad spreads the banks
+        static_assert(kWaves * 32 * kPitch <= kPipeLds, "fits in the stages");
+        __syncthreads();                      // the tile stages are no longer read
+        unsigned char* ow = smem + wave * (32 * kPitch);
 #pragma unroll
-            for (int dt = 0; dt < kDB; dt++)
+        for (int d0 = 0; d0 < kD; d0 += kStep) {
+#pragma unroll
+            for (int dt = d0 / 32; dt < (d0 + kStep) / 32; dt++)
 #pragma unroll
                 for (int v4 = 0; v4 < 4; v4++)
-                    *reinterpret_cast<float4*>(po + 32 * dt + 8 * v4 + 4 * half) =
+                    *reinterpret_cast<float4*>(ow + col * kPitch + (32 * dt - d0 + 8 * v4 + 4 * half) * 4) =
                         make_float4(oacc[dt][4 * v4] * inv_p, oacc[dt][4 * v4 + 1] * inv_p, oacc[dt][4 * v4 + 2] * inv_p,
                                     oacc[dt][4 * v4 + 3] * inv_p);
-            if (half == 0)
-                p.part_l2[(int64_t)split_i * p.B * p.H * p.Q + row_p] = any ? m_ref + __builtin_amdgcn_logf(l_tot) : -INFINITY;
+            __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0)
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int pass = 0; pass < 32 / kPassRows; pass++) {
+                const int r = kPassRows * pass + lane / kLanes;
+                int m;
+                const int64_t row = row_of(r, m);
+                const float4 v = *reinterpret_cast<const float4*>(ow + r * kPitch + (lane % kLanes) * 16);
+                if (m < p.Q) *reinterpret_cast<float4*>(p.part_o + row * kD + d0 + (lane % kLanes) * 4) = v;
+            }
+            __builtin_amdgcn_wave_barrier();
+        }
+        if (half == 0 && row_m < p.Q) {
+            int m;
+            p.part_l2[row_of(col, m)] = any ? m_ref + __builtin_amdgcn_logf(l_tot) : -INFINITY;
         }
         return;
     }
