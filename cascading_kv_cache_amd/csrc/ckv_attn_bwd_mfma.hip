@@ -424,43 +424,8 @@ __global__ void __launch_bounds__(Team<kWaves>::kThreads, Team<kWaves>::kPerCu) 
     const char* vb = reinterpret_cast<const char*>(a.v) + (b * a.kv_stride[0] + hd * a.kv_stride[1]) * 2;
     const uint32_t row_bytes = (uint32_t)(a.kv_stride[2] * 2);
 
-    // stationary B operands: Q^T and dO^T of this lane's query, dims 16 ds + 8 h .. +7
-    uint4 qreg[kHD / 16], greg[kHD / 16];
-    {
-        const char* qrow = reinterpret_cast<const char*>(a.q) +
-                           (b * a.q_stride[0] + hd * a.q_stride[1] + m_lane * a.q_stride[2]) * 2;
-        const char* grow = reinterpret_cast<const char*>(a.dout) +
-                           (b * a.dout_stride[0] + hd * a.dout_stride[1] + m_lane * a.dout_stride[2]) * 2;
-#pragma unroll
-        for (int ds = 0; ds < kHD / 16; ds++) {
-            qreg[ds] = greg[ds] = make_uint4(0u, 0u, 0u, 0u);
-            if (m_lane < n_ctx) {
-                qreg[ds] = *reinterpret_cast<const uint4*>(qrow + (16 * ds + 8 * h) * 2);
-                greg[ds] = *reinterpret_cast<const uint4*>(grow + (16 * ds + 8 * h) * 2);
-            }
-        }
-    }
-    arrived(qreg);
-    arrived(greg);
-    const bool row_ok = m_lane < n_ctx;
-    // The magnitude of the softmax scale rides on the exponent (nothing here needs P without it), its sign on the result;
-    // the products of V and dO start from -delta.  That leaves one multiplication per element beside the exponential.
-    float nl = row_ok ? fmaf(-a.lse[bh * n_ctx + m_lane], kLog2e, __builtin_amdgcn_logf(fabsf(a.scale))) : 0.f;
-    const float c2 = a.scale * kLog2e;
-    f32x16 neg_delta;
-    {
-        const float d = row_ok ? -p.delta[bh * n_ctx + m_lane] : 0.f;
-#pragma unroll
-        for (int i = 0; i < 16; i++) neg_delta[i] = d;
-        asm volatile("" : "+v"(neg_delta));   // 16 registers to start from, not 16 moves a block
-    }
-
     const uint32_t lds0 = lds_address(smem);
     const Operands<kHD, false> op(lds0, lane);
-
-    f32x16 dq[kHD / 32];
-#pragma unroll
-    for (int db = 0; db < kHD / 32; db++) dq[db] = zero16();
 
     // keys past the diagonal of the workgroup's last row are visible to none of its rows
     int m_last = m_wg + kOwn - 1;
@@ -492,9 +457,49 @@ __global__ void __launch_bounds__(Team<kWaves>::kThreads, Team<kWaves>::kPerCu) 
         copy_rows<kHD, kWide>(vb, row_bytes, r, lds0 + (uint32_t)(st * kStage + kTile), wave, lane);
     };
     uint32_t rows_next[kHD / 64];   // of the block that is copied next
+    // All that does not hang on the row numbers is requested with them, in one go: as loads of one operand at a time, each behind
+    // the last one's, these were four (64 dims) or eight (128) trips to memory in a row and two more for the scalars (64 heads x 1024 rows x
+    // 8704 visible keys, 128 dims: 389 -> 386 us; the same for dk/dv, whose workgroups come in rounds, level).
     if (blk0 < nblk) {
 #pragma unroll
         for (int i = 0; i < kDqStages; i++) request_rows(blk0 + i, i);
+    }
+    // stationary B operands: Q^T and dO^T of this lane's query, dims 16 ds + 8 h .. +7
+    uint4 qreg[kHD / 16], greg[kHD / 16];
+    const bool row_ok = m_lane < n_ctx;
+    float lse = 0.f, delta = 0.f;
+#pragma unroll
+    for (int ds = 0; ds < kHD / 16; ds++) qreg[ds] = greg[ds] = make_uint4(0u, 0u, 0u, 0u);
+    if (row_ok) {
+        const char* qrow = reinterpret_cast<const char*>(a.q) +
+                           (b * a.q_stride[0] + hd * a.q_stride[1] + m_lane * a.q_stride[2]) * 2;
+        const char* grow = reinterpret_cast<const char*>(a.dout) +
+                           (b * a.dout_stride[0] + hd * a.dout_stride[1] + m_lane * a.dout_stride[2]) * 2;
+#pragma unroll
+        for (int ds = 0; ds < kHD / 16; ds++) {
+            qreg[ds] = *reinterpret_cast<const uint4*>(qrow + (16 * ds + 8 * h) * 2);
+            greg[ds] = *reinterpret_cast<const uint4*>(grow + (16 * ds + 8 * h) * 2);
+        }
+        lse = a.lse[bh * n_ctx + m_lane];
+        delta = p.delta[bh * n_ctx + m_lane];
+    }
+    arrived(qreg);
+    arrived(greg);
+    // The magnitude of the softmax scale rides on the exponent (nothing here needs P without it), its sign on the result;
+    // the products of V and dO start from -delta.  That leaves one multiplication per element beside the exponential.
+    float nl = row_ok ? fmaf(-lse, kLog2e, __builtin_amdgcn_logf(fabsf(a.scale))) : 0.f;
+    const float c2 = a.scale * kLog2e;
+    f32x16 neg_delta;
+    {
+        const float d = -delta;
+#pragma unroll
+        for (int i = 0; i < 16; i++) neg_delta[i] = d;
+        asm volatile("" : "+v"(neg_delta));   // 16 registers to start from, not 16 moves a block
+    }
+    f32x16 dq[kHD / 32];
+#pragma unroll
+    for (int db = 0; db < kHD / 32; db++) dq[db] = zero16();
+    if (blk0 < nblk) {
         wait_copies<0>();
         rows_of(blk0, 0, rows_next);
         copy(rows_next, 0);
