@@ -1031,34 +1031,50 @@ __global__ void __launch_bounds__(512) fwd_pipe_kernel(FwdParams p) {
         };
         const bool any = l_tot != 0.f;   // a NaN is not nothing: it has to reach the merge
         const float inv_p = any ? 1.f / l_tot : 0.f;
-        // Through LDS, half of the dims at a time, so that a store is whole stretches of 256 (128) bytes of four (eight) rows: a
-        // lane's own 16 bytes have one neighbour in each of 32 rows (with the start above, 32 heads x 509 rows x 16897 keys in 8
-        // shares: 145.5 -> 142.8 us).
-        constexpr int kStep = kD / 2, kLanes = kStep / 4, kPassRows = CKV_WAVE / kLanes;
-        constexpr int kPitch = 4 * kStep + 16;   // bytes; the pad spreads the banks
-        static_assert(kWaves * 32 * kPitch <= kPipeLds, "fits in the stages");
-        __syncthreads();                      // the tile stages are no longer read
-        unsigned char* ow = smem + wave * (32 * kPitch);
-#pragma unroll
-        for (int d0 = 0; d0 < kD; d0 += kStep) {
-#pragma unroll
-            for (int dt = d0 / 32; dt < (d0 + kStep) / 32; dt++)
-#pragma unroll
-                for (int v4 = 0; v4 < 4; v4++)
-                    *reinterpret_cast<float4*>(ow + col * kPitch + (32 * dt - d0 + 8 * v4 + 4 * half) * 4) =
-                        make_float4(oacc[dt][4 * v4] * inv_p, oacc[dt][4 * v4 + 1] * inv_p, oacc[dt][4 * v4 + 2] * inv_p,
-                                    oacc[dt][4 * v4 + 3] * inv_p);
-            __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0)
-            __builtin_amdgcn_wave_barrier();
-#pragma unroll
-            for (int pass = 0; pass < 32 / kPassRows; pass++) {
-                const int r = kPassRows * pass + lane / kLanes;
+        if constexpr (kD == 64) {
+            // A row is 256 bytes and half of it all that the stages have room for: stretches of 128 bytes, which do not pay for the
+            // way through LDS (8 heads x 148 rows x 5236 keys in shares: 23.9 us that way, 23.1 so; 16 x 700 x 2200: 27.0, 26.6).
+            if (row_m < p.Q) {
                 int m;
-                const int64_t row = row_of(r, m);
-                const float4 v = *reinterpret_cast<const float4*>(ow + r * kPitch + (lane % kLanes) * 16);
-                if (m < p.Q) *reinterpret_cast<float4*>(p.part_o + row * kD + d0 + (lane % kLanes) * 4) = v;
+                float* po = p.part_o + row_of(col, m) * kD + 4 * half;
+#pragma unroll
+                for (int dt = 0; dt < kDB; dt++)
+#pragma unroll
+                    for (int v4 = 0; v4 < 4; v4++)
+                        *reinterpret_cast<float4*>(po + 32 * dt + 8 * v4) =
+                            make_float4(oacc[dt][4 * v4] * inv_p, oacc[dt][4 * v4 + 1] * inv_p, oacc[dt][4 * v4 + 2] * inv_p,
+                                        oacc[dt][4 * v4 + 3] * inv_p);
             }
-            __builtin_amdgcn_wave_barrier();
+        } else {
+            // Through LDS, half of the dims at a time, so that a store is whole stretches of 256 bytes of four rows: a lane's own
+            // 16 bytes have one neighbour in each of 32 rows (with the start above, 32 heads x 509 rows x 16897 keys in 8 shares:
+            // 145.5 -> 142.8 us).
+            constexpr int kStep = kD / 2, kLanes = kStep / 4, kPassRows = CKV_WAVE / kLanes;
+            constexpr int kPitch = 4 * kStep + 16;   // bytes; the pad spreads the banks
+            static_assert(kWaves * 32 * kPitch <= kPipeLds, "fits in the stages");
+            __syncthreads();                      // the tile stages are no longer read
+            unsigned char* ow = smem + wave * (32 * kPitch);
+#pragma unroll
+            for (int d0 = 0; d0 < kD; d0 += kStep) {
+#pragma unroll
+                for (int dt = d0 / 32; dt < (d0 + kStep) / 32; dt++)
+#pragma unroll
+                    for (int v4 = 0; v4 < 4; v4++)
+                        *reinterpret_cast<float4*>(ow + col * kPitch + (32 * dt - d0 + 8 * v4 + 4 * half) * 4) =
+                            make_float4(oacc[dt][4 * v4] * inv_p, oacc[dt][4 * v4 + 1] * inv_p, oacc[dt][4 * v4 + 2] * inv_p,
+                                        oacc[dt][4 * v4 + 3] * inv_p);
+                __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0)
+                __builtin_amdgcn_wave_barrier();
+#pragma unroll
+                for (int pass = 0; pass < 32 / kPassRows; pass++) {
+                    const int r = kPassRows * pass + lane / kLanes;
+                    int m;
+                    const int64_t row = row_of(r, m);
+                    const float4 v = *reinterpret_cast<const float4*>(ow + r * kPitch + (lane % kLanes) * 16);
+                    if (m < p.Q) *reinterpret_cast<float4*>(p.part_o + row * kD + d0 + (lane % kLanes) * 4) = v;
+                }
+                __builtin_amdgcn_wave_barrier();
+            }
         }
         if (half == 0 && row_m < p.Q) {
             int m;
