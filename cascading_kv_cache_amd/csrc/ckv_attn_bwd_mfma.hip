@@ -981,14 +981,22 @@ constexpr int dq_lds() {
     return Team<kWaves>::kStages * (2 * kTile + (Halves<T, kHD>::kSplit ? 2 * kTile : 0) + Team<kWaves>::kRows * (int)sizeof(int));
 }
 
-// Eight wavefronts where their workgroups leave no more rows empty than those of four and there is one for every compute unit.
-// K and V then reach a unit's LDS once instead of once per workgroup of four, and a barrier comes every 64 keys: 64 heads x 1024
-// rows x 8704 visible keys, 128 dims 401 -> 386 us; x 8192 keys, 64 dims, bf16 308 -> 286, float16 436 -> 395; 8 heads x 1000 x
-// 4071 keys, 64 dims, in 8 shares 42.8 -> 41.7; 32 x 512 x 4608 in 4 shares level.  Elsewhere four: 300 rows (a wide workgroup of
-// 256 and one of 44) 45.6 us, wide 76.8; 2 heads x 1024 rows in 8 shares (64 wide workgroups) 27.0, wide 36.6.
-inline bool wide_dq(const ckv_dense_bwd_args& a, int n_split) {
-    const int64_t wide = (a.n_ctx + Team<8>::kOwn - 1) / Team<8>::kOwn, narrow = (a.n_ctx + Team<4>::kOwn - 1) / Team<4>::kOwn;
-    return 2 * wide == narrow && wide * a.B * a.H * n_split >= mfma_device_cus();
+// Eight wavefronts where their workgroups leave no more rows empty than those of four, run all at once, and those of four would
+// share compute units two by two.  K and V then reach a unit's LDS once instead of twice, and a barrier comes every 64 keys.
+// units: heads of the batch x shares of the keys.  Time of the wide kernel over that of the narrow one, by the number of wide
+// workgroups on 256 compute units (1024 rows x 1536 visible cached keys; 128 dims bf16 / 64 dims f16 / 64 dims bf16):
+//   128 (a narrow one has a unit to itself)   1.25 / 1.17 / 1.20
+//   144 to 248   0.92 to 0.95 / 0.88 to 0.91 / 0.88 to 0.91        256   0.96 / 0.91 / 0.92   (114, 150 and 107 us)
+//   272   1.14 / 1.11 / 1.34     384   1.08 / 1.06 / 1.26     512   0.97 / 0.95 / 0.98
+//   576   1.18 / 1.17 / 1.32     768   1.00 / 0.96 / 1.04    1536   1.03 / 1.03 / 1.12
+// Past one round a unit stands idle while a wide workgroup ends or fetches its first keys, and a last round of few takes as long
+// as a full one; two full rounds still gain here and lose elsewhere (1000 rows of chunk keys alone 1.00 / 0.95 / 1.15, 2048
+// rows 1.13 / 1.08 / 1.33).  Within one round the other shapes are 0.88 to 1.00 too (256 rows x 768 cached keys, chunk keys
+// alone, 512 rows x 3072 in shares), 2048 rows of chunk keys in 128 dims 0.95 to 1.02, and the launches of shares at few heads (32
+// or 40 workgroups in 8 or 6 shares) 0.93 to 1.03.
+inline bool wide_dq(int64_t n_ctx, int64_t units, int64_t cus) {
+    const int64_t wide = (n_ctx + Team<8>::kOwn - 1) / Team<8>::kOwn, narrow = (n_ctx + Team<4>::kOwn - 1) / Team<4>::kOwn;
+    return 2 * wide == narrow && wide * units <= cus && narrow * units > cus;
 }
 
 template <typename T, int kHD>
@@ -1015,7 +1023,7 @@ int run(const BwdMfmaParams& p_in, hipStream_t stream) {
     constexpr std::integral_constant<int, 8> wide{};
     if (a.n_kv * a.kv_stride[2] * 2 >= (int64_t)1 << 32) {
         if (int rc = launch_dq(narrow, std::true_type{})) return rc;
-    } else if (wide_dq(a, p.n_split)) {
+    } else if (wide_dq(a.n_ctx, a.B * a.H * p.n_split, mfma_device_cus())) {
         if (int rc = launch_dq(wide, std::false_type{})) return rc;
     } else if (int rc = launch_dq(narrow, std::false_type{})) {
         return rc;
@@ -1076,3 +1084,8 @@ int launch_bwd_mfma(const ckv_dense_bwd_args& a, const float* delta, const int* 
 }
 
 }  // namespace ckv
+
+// wavefronts of dq's workgroups for rows addressed in 32 bits (cus 0: the current device's), for tests that aim at one kernel
+extern "C" int ckv_dense_bwd_dq_wavefronts(int64_t n_ctx, int64_t units, int64_t cus) {
+    return ckv::wide_dq(n_ctx, units, cus > 0 ? cus : ckv::mfma_device_cus()) ? 8 : 4;
+}

@@ -300,3 +300,15 @@ def test_oracle_result_does_not_depend_on_the_layout(dtype):
         for n in _ORDER[3:]:
             assert torch.equal(t[n], flat[n]), (call, n)
     assert not t["mask"].all() and t["stored_sinks"].eq(sc["num_sink"]).all()
+
+
+@pytest.mark.parametrize("n_ctx,units,wavefronts", [
+    (1024, 64, 8), (1024, 62, 8), (1024, 33, 8), (1024, 32, 4),              # one round; one narrow workgroup a compute unit
+    (1024, 65, 4), (1024, 72, 4), (1024, 96, 4), (1024, 128, 4), (1024, 320, 4),   # more than one round, full or not
+    (1000, 8 * 8, 8), (1000, 8, 4), (256, 256, 8), (256, 257, 4), (129, 256, 8), (129, 129, 8), (128, 256, 4),
+    (300, 85, 4), (2200, 28, 8), (2100, 28, 4),                              # an odd number of 128-row tiles: half of a wide one empty
+])
+def test_dq_by_eight_wavefronts_where_all_run_at_once(lib, n_ctx, units, wavefronts):
+    """The dense operator's dq on 256 compute units: workgroups of eight wavefronts where each has a unit of its own and those
+    of four would share them.  With a round and a bit of them (65 heads of 1000 rows) the kernel took a third longer."""
+    assert C.CDLL(_abi.LIB_PATH).ckv_dense_bwd_dq_wavefronts(C.c_int64(n_ctx), C.c_int64(units), C.c_int64(256)) == wavefronts
