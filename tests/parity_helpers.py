@@ -10,6 +10,7 @@ each other.  ``check_update_against_replay`` proves the first half (the oracle's
 library's scores reproduces the library's state bit for bit); ``flip_margins`` measures the second.
 """
 import copy
+import ctypes
 
 import torch
 
@@ -132,3 +133,13 @@ def flip_bound(ledger):
 
 def clone_oracle(cpu):
     return copy.deepcopy(cpu)
+
+
+def dq_wavefronts(Z, H, n_ctx, n_kv, D, dtype, shared=True):
+    """of the workgroups that the dense operator's dq runs in on this device; ``shared``: given room for shares of the keys"""
+    from cascading_kv_cache_amd import _abi
+
+    size = _abi.lib().ckv_dense_bwd_split_bytes(Z, H, n_ctx, n_kv, D, _abi.dtype_code(dtype)) if shared else 0
+    shares = max(1, size // (Z * H * n_ctx * D * 4))
+    rule = ctypes.CDLL(_abi.LIB_PATH).ckv_dense_bwd_dq_wavefronts
+    return rule(ctypes.c_int64(n_ctx), ctypes.c_int64(Z * H * shares), ctypes.c_int64(0))

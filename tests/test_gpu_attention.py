@@ -16,7 +16,7 @@ from oracle.update import OracleCache
 pytestmark = pytest.mark.gpu
 
 from parity_helpers import (META, STATE, FlipLedger, assert_scores_close, check_update_against_replay, clone_oracle,
-                            flip_bound, flip_margins, push_state, tol)
+                            dq_wavefronts, flip_bound, flip_margins, push_state, tol)
 
 
 def make_pair(B, KVH, D, NS, W, C, dtype, func="pow2", eager=True, reduction="mean"):
@@ -511,16 +511,19 @@ def test_backward_on_the_matrix_cores(Z, H, N_CTX, N_KV, masking, layout, dtype)
     check_backward_against_autograd(q, k, v, mask, dtype)
 
 
-@pytest.mark.parametrize("Z,H,N_CTX,N_KV", [(4, 64, 129, 129 + 95), (4, 64, 250, 250), (2, 32, 256, 1025 + 256), (2, 32, 400, 1190 + 400)])
+@pytest.mark.parametrize("Z,H,N_CTX,N_KV", [(4, 64, 129, 129 + 95), (4, 64, 250, 250), (2, 32, 256, 1025 + 256), (4, 32, 400, 1190 + 400),
+                                            (1, 32, 400, 4208 + 400), (1, 24, 1000, 900 + 1000), (5, 12, 720, 720)])
 @pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_backward_dq_by_eight_wavefronts(Z, H, N_CTX, N_KV, D, dtype):
-    """Heads enough for a workgroup of 256 query rows on every compute unit, with and without shares of the keys: the last
-    workgroup short of rows, 64-key stages whose second half lies past the last visible key or on the diagonal.  dq against
-    float64, with the rounded out in delta as the operator defines it: P, dS and the result are rounded at most once each, half a unit (2^-9 or 2^-12) at the most,
-    relative to all rows; for one row relative to it and to the rows' root mean square (a row whose few keys cancel is
-    smaller than what was rounded)."""
+    """Workgroups of 256 query rows, one to four of a head, all running at once, with and without shares of the keys: the last
+    workgroup short of rows, alone or behind full ones, 64-key stages whose second half lies past the last visible key or on the
+    diagonal.  dq against float64, with the rounded out in delta as the operator defines it: P, dS and the result are rounded at
+    most once each, half a unit (2^-9 or 2^-12) at the most, relative to all rows; for one row relative to it and to the rows'
+    root mean square (a row whose few keys cancel is smaller than what was rounded)."""
     from cascading_kv_cache_amd.flash_attention import attention
+
+    assert dq_wavefronts(Z, H, N_CTX, N_KV, D, dtype) == 8
 
     torch.manual_seed(23)
 

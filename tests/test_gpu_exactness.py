@@ -13,6 +13,8 @@ import math
 import pytest
 import torch
 
+from parity_helpers import dq_wavefronts
+
 pytestmark = pytest.mark.gpu
 
 F16, BF16, F32 = torch.float16, torch.bfloat16, torch.float32
@@ -248,6 +250,59 @@ def test_dense_backward_with_less_room_than_it_could_use(Z, H, n_ctx, n_kv, mask
     check_backward(q, k, v, out, lse, mask, do, 0.3, *grads)
     hidden = torch.cat((mask, torch.zeros(n_ctx, dtype=torch.bool, device="cuda")))
     assert (grads[1][:, :, hidden] == 0).all() and (grads[2][:, :, hidden] == 0).all()
+
+
+@pytest.mark.parametrize("dtype", [BF16, F16])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("scale", [0.3, -0.25])
+@pytest.mark.parametrize("room", ["delta", "delta and order", "all"])
+@pytest.mark.parametrize("Z,H,n_ctx,n_kv,masked", [
+    (2, 80, 129, 500 + 129, slice(32, 320)),   # the second workgroup's one row; whole stages and a half of hidden keys
+    (1, 90, 400, 75 + 400, slice(0, 75)),      # no cached key visible; two workgroups a head, the second short of rows
+    (1, 40, 1000, 250 + 1000, None)])          # four, and a diagonal that crosses twelve stages in front of the last's
+def test_dense_backward_with_dq_by_eight_wavefronts(Z, H, n_ctx, n_kv, masked, room, scale, D, dtype):
+    """dq's wide workgroups with the keys sorted and as they lie (masked one by one, a hidden block of 32 left out), with
+    either sign of the scale."""
+    from cascading_kv_cache_amd import _abi
+    from cascading_kv_cache_amd import flash_attention as fa
+
+    assert dq_wavefronts(Z, H, n_ctx, n_kv, D, dtype, shared=room == "all") == 8
+    q, k, v, mask, do = dense_case(Z, H, n_ctx, n_kv, D, dtype)
+    if masked is not None:
+        mask[masked] = True
+    out, _, lse, m = fa._forward(q, k, v, True, scale, mask, 0.9, True)
+    size = _abi.lib().ckv_dense_bwd_workspace_bytes(Z, H, n_ctx)
+    if room == "delta and order":
+        size += _abi.lib().ckv_dense_bwd_key_order_bytes(n_kv)
+    with pytest.MonkeyPatch.context() as patch:
+        if room != "all":
+            patch.setattr(fa, "workspace", lambda device, need, stream: torch.empty(size, dtype=torch.uint8, device=device))
+        grads = fa._backward(q, k, v, out, lse, m, do, scale)
+    check_backward(q, k, v, out, lse, mask, do, scale, *grads)
+
+
+@pytest.mark.parametrize("dtype", [BF16, F16])
+@pytest.mark.parametrize("row", [5, 299])
+def test_infinite_gradient_in_dq_by_eight_wavefronts(row, dtype):
+    """The wavefront that holds the row takes float32 products, in both blocks of every stage: its other rows are what they
+    were to a rounding, everyone else's to the bit."""
+    from cascading_kv_cache_amd import flash_attention as fa
+
+    Z, H, n_ctx, n_kv = 1, 72, 400, 700 + 400
+    assert dq_wavefronts(Z, H, n_ctx, n_kv, 64, dtype) == 8
+    q, k, v, mask, do = dense_case(Z, H, n_ctx, n_kv, 64, dtype)
+    out, _, lse, m = fa._forward(q, k, v, True, 0.5, mask, 0.9, True)
+    clean = fa._backward(q, k, v, out, lse, m, do, 0.5)[0]
+    do[0, 3, row, 7] = float("inf")
+    dq = fa._backward(q, k, v, out, lse, m, do, 0.5)[0]
+    assert not dq[0, 3, row].isfinite().any()
+    mates = [r for r in range(row // 32 * 32, row // 32 * 32 + 32) if r != row]
+    same = torch.ones_like(dq, dtype=torch.bool)
+    same[0, 3, row // 32 * 32:row // 32 * 32 + 32] = False
+    assert torch.equal(dq[same], clean[same])
+    p, ds, size = exact_weights(q, k, v, out, lse, mask, torch.where(do.isinf(), 0.0, do), 0.5)   # the mates' rows are finite
+    exact, spread2 = torch.matmul(ds[0, 3], k[0, 3].double()), torch.matmul(size[0, 3].square(), k[0, 3].double().square())
+    assert_rounded_once(dq[0, 3, mates], exact[mates], spread2[mates].sqrt(), n_kv, "dq")
 
 
 @pytest.mark.parametrize("dtype", [BF16, F16])

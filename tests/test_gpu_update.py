@@ -152,6 +152,21 @@ def test_calls_that_evict_what_they_brought(W, C, func):
     run_stream(gpu, cpu, sum(lengths), lambda: next(left), gen, torch.bfloat16, "ties")
 
 
+@pytest.mark.parametrize("D,dtype,slots", [
+    (8, torch.bfloat16, 131072), (16, torch.float16, 65536), (16, torch.float32, 32768), (64, torch.bfloat16, 16384),
+    (64, torch.bfloat16, 16384 - 16), (128, torch.float32, 4096), (96, torch.float32, 5472), (256, torch.float32, 2048)])
+def test_rows_of_large_caches(D, dtype, slots):
+    """32 MiB of rows and more are moved non-temporally, by 1, 2, 4, 8, 32, 32 (24 of them busy) and 64 lanes a row; sixteen
+    slots fewer in each of 8 units with 64 dims is the last size that is not.  Full cascades, rows that travel through several
+    of them, bit-exact against the oracle after every call."""
+    C = 16
+    gpu, cpu = make_pair(2, 4, D, 4, slots // C, C, dtype, eager=False)
+    gen = torch.Generator().manual_seed(D)
+    W = slots // C
+    lengths = iter([5 * W + 3, W // 2 + 1, 1, 2 * W])
+    run_stream(gpu, cpu, 5 * W + 3 + W // 2 + 1 + 1 + 2 * W, lambda: next(lengths), gen, dtype, "ties")
+
+
 def test_call_larger_than_one_launch():
     """More tokens than one planning launch holds in LDS: the call is split internally."""
     gpu, cpu = make_pair(1, 2, 16, 4, 64, 4, torch.float32, eager=False)
