@@ -28,7 +28,7 @@
 // copies: 100 to 170 cycles each at the issue, whatever else the wavefront does (let out one by one between matrix
 // instructions: dq 514 us, dk/dv level); dq has them 64 keys ahead.  Waiting for them where the work does not need them yet: the
 // compiler put a wait for everything in flight before the first use of registers loaded in front of the loop (arrived; without
-// it dq 436 us, with it 401, by eight wavefronts 386).  Reads from LDS are not it: operands of dK / dV 4 instead of 2 matrix
+// it dq 436 us, with it 401, by eight wavefronts 389, with everything a workgroup starts from requested at once 386).  Reads from LDS are not it: operands of dK / dV 4 instead of 2 matrix
 // instructions ahead, and of dP 2 instead of 1, dk/dv level; dk/dv by eight wavefronts and 64 rows a barrier 628 us instead of 590.
 //
 // The A operands K^T, Q^T and dO^T are read from the row-major tiles in LDS with the transposing read
@@ -615,7 +615,7 @@ __global__ void __launch_bounds__(Team<kWaves>::kThreads, Team<kWaves>::kPerCu) 
         } else {
             wait_copies<0>();
         }
-        // the halves of a stage were last read two barriers ago
+        // the halves of that stage were last read in the step before (two stages) or in the one before it: at least one barrier ago
         if (blk + 1 < nblk) Half::template split<1, kTile>(smem, (st + 1) % kDqStages * kStage, kHalves + (st + 1) % kDqStages * 2 * kTile, wave, lane);
         __syncthreads();
     };
@@ -1055,10 +1055,11 @@ bool bwd_mfma_supported(const ckv_dense_bwd_args& a) {
            aligned16(a.dk) && aligned16(a.dv);
 }
 
-// Shares of the keys for dq (1: no sharing).  A launch has one workgroup per 128 rows of a head, two of which fit a compute
-// unit: with fewer than one per compute unit the keys are dealt out over up to 8 of them, at least 8 blocks of 32 keys each,
-// about two workgroups per compute unit in all, and the shares (float32) are added up by a kernel behind.  8 heads x 1000
-// rows are 64 workgroups, a quarter of the chip.
+// Shares of the keys for dq (1: no sharing), counted in workgroups of four wavefronts, one per 128 rows of a head, two of which
+// fit a compute unit: with fewer than one per compute unit the keys are dealt out over up to 8 of them, at least 8 blocks of 32
+// keys each, about two workgroups per compute unit in all (as many rows and keys as one wide workgroup, which wide_dq may then
+// take in their place), and the shares (float32) are added up by a kernel behind.  8 heads x 1000 rows are 64 workgroups, a
+// quarter of the chip.
 int bwd_mfma_dq_splits(int64_t B, int64_t H, int64_t n_ctx, int64_t n_kv, int cus) {
     constexpr int kDqRows = Team<4>::kOwn;
     const int64_t wgs = (n_ctx + kDqRows - 1) / kDqRows * B * H, blocks = (n_kv + kBlk - 1) / kBlk;

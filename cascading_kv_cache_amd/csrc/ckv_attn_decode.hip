@@ -1835,10 +1835,12 @@ __global__ void __launch_bounds__(256) decode_scores_probs_kernel(DecodeParams p
 }
 
 // Tail and scores in one launch: the first B * H workgroups combine a row each, the others work out the scores of 4096
-// keys of one (b, kvh), for which they first merge the (maximum, sum) pairs of its G heads themselves.  That costs a
-// score workgroup two trips to memory before its own work (with more workgroups than the chip holds at once, 16 streams
-// x 257 tiles, 40 us against 30 us for two launches); when all of them run side by side it is hidden behind the rows:
-// with one stream the step is a chain of short launches, and this takes one out (host and device: about 4 us each).
+// keys of one (b, kvh), for which they merge the (maximum, sum) pairs of its G heads themselves, on top of what a score thread
+// reads, which is requested before.  Where all workgroups run side by side that is hidden behind the rows, and a launch is saved
+// (host and device: about 4 us): one launch against two, us, 1 stream x 64 K slots 6.9 and 6.6 + 4.8, 4 x 32 K 8.9 and 5.8 + 6.1,
+// 2 x 64 K 10.2 and 6.9 + 6.3.  Where they come in rounds every score workgroup pays for its merge: 16 streams x 32 K slots, 1664
+// workgroups, 25.4 and 10.1 + 12.1; 8 x 32 K, 832, 15.2 and 7.2 + 8.0.  The line at two workgroups a compute unit is on the safe
+// side (5 x 32 K, 520 workgroups, 12.4 and 6.2 + 6.5; 16 x 2 K, 640, 8.0 and 4.8 + 4.1).
 template <typename T, int G>
 __global__ void __launch_bounds__(512) decode_finish_kernel(DecodeParams p, float w_one, float beta_pow, int per_unit) {
     __shared__ TailLds sh;

@@ -539,8 +539,8 @@ __device__ inline int k_lds_off(int r, int c) { return r * (2 * kD) + ((c ^ row_
 // stay in flight across it), and the first operands of an iteration can be fetched before its barrier.
 constexpr int kKStages = 3, kVStages = 4;
 __host__ __device__ constexpr int pipe_stages_lds(int head_dim) { return (kKStages + kVStages) * head_dim * 2 * kBN; }   // K0 K1 K2 V0 V1 V2 V3
-// stages, one visibility word and one work-list entry per key tile, the list length
-inline int64_t pipe_lds_bytes(int64_t n_pad, int head_dim) { return pipe_stages_lds(head_dim) + (n_pad / kBN) * 12 + 16; }
+// stages, one visibility word and one work-list entry per key tile
+inline int64_t pipe_lds_bytes(int64_t n_pad, int head_dim) { return pipe_stages_lds(head_dim) + (n_pad / kBN) * 12; }
 constexpr int64_t kLdsLimit = 160 * 1024;
 
 template <typename T, int kD>
@@ -587,7 +587,10 @@ __global__ void __launch_bounds__(512) fwd_pipe_kernel(FwdParams p) {
     int* list_lds = reinterpret_cast<int*>(smem + kPipeLds + 8 * tiles_cap);
     const uint32_t smem_addr = lds_address(smem);
 
-    // ---- the query row this lane owns as MFMA column `col`, requested first: its trip to memory is that of the words below
+    // ---- the query row this lane owns as MFMA column `col`, requested first: its trip to memory is that of the words below.
+    // With the work list by all wavefronts, a first wait for the first K tile alone and (128 dims) shares that leave through
+    // LDS a launch takes 1 to 2 % less (32 heads, us: 509 rows x 16 K slots 143.8 -> 141.1, 300 x 16 K 113.4 -> 111.9, 2048 x 8 K
+    // 265.7 -> 264.4, 4096 x 64 K 3533 -> 3524); one by one only the shares show, at their place below.
     int row_m;
     uint4 qreg[kKK];
     {
@@ -597,8 +600,7 @@ __global__ void __launch_bounds__(512) fwd_pipe_kernel(FwdParams p) {
         const int64_t row_h = kvh * p.G + g;
         const bool row_ok = row_m < p.Q;
         const T* qrow = (const T*)p.qr + ((b * p.H + row_h) * p.Q + row_m) * kD;
-        // one branch around all of them: a choice per piece made eight branches, each with a wait for its own piece at the end
-        // (509 rows x 32 heads x 16 K slots: 147.0 -> 144.2 us)
+        // one branch around all of them: a choice per piece makes eight branches, each with a wait for its own piece at the end
 #pragma unroll
         for (int kk = 0; kk < kKK; kk++) qreg[kk] = make_uint4(0, 0, 0, 0);
         if (row_ok) {
@@ -1047,8 +1049,8 @@ __global__ void __launch_bounds__(512) fwd_pipe_kernel(FwdParams p) {
             }
         } else {
             // Through LDS, half of the dims at a time, so that a store is whole stretches of 256 bytes of four rows: a lane's own
-            // 16 bytes have one neighbour in each of 32 rows (with the start above, 32 heads x 509 rows x 16897 keys in 8 shares:
-            // 145.5 -> 142.8 us).
+            // 16 bytes have one neighbour in each of 32 rows (32 heads x 1024 rows x 16 K slots 249.4 -> 245.8 us, 300 rows 113.0
+            // -> 111.9).
             constexpr int kStep = kD / 2, kLanes = kStep / 4, kPassRows = CKV_WAVE / kLanes;
             constexpr int kPitch = 4 * kStep + 16;   // bytes; the pad spreads the banks
             static_assert(kWaves * 32 * kPitch <= kPipeLds, "fits in the stages");

@@ -733,9 +733,13 @@ __device__ inline void commit_trackers(const UpdateParams& p, const Unit& u) {
 }
 
 // One 16-byte piece of a row per lane.  kOnce: rows are read and written past the L2 (non-temporal).  Nothing here looks at them
-// twice, and the words that do go round in it (chains, position ids, scores) stay: 4096 tokens x 8 units into 64 K slots, the moves
-// 25.0 -> 22.8 us (loads alone 23.5, stores alone 24.3); 2048 x 16 into 16 K 23.1 -> 22.7.  Not for a cache that would stay in the
-// L2 until the next call (kOnceBytes): 256 tokens x 8 units into 512 float32 slots, the next chunk's staging 10.5 -> 11.4.
+// twice, and the words that do go round in it (chains, position ids, scores) stay.  What it gives hangs on what ran before.  Caches
+// of four layers in turn, 8 units, plain -> non-temporal, us: the update alone behind a copy of 256 MiB, 4096 tokens into 64 K
+// slots 24.0 -> 22.1, into 16 K 20.3 -> 18.9, 2048 into 8 K 12.4 -> 11.7; behind its chunk's attention 22.9 -> 22.8, 18.3 -> 17.6
+// and 10.5 -> 10.5, where the next layer's staging takes 111.7 -> 110.8, 50.0 -> 49.2 and 33.4 -> 32.4.  One cache that
+// the last-level cache holds, called again and again behind its attention with no other layer between, loses: 64 MiB 12.0 -> 12.7,
+// 2 x 64 MiB 18.0 -> 20.5 and the staging 64.9 -> 66.2.  Not for a cache that would stay in the L2 until the next call
+// (kOnceBytes): 2048 tokens into 4 K slots, four layers, moves 8.7 -> 7.9 but the staging behind them 25.4 -> 27.0.
 struct RowPiece {
     uint4 k, v;
 };

@@ -413,6 +413,25 @@ def test_dense_operator_forward(Z, H, N_CTX, N_KV, HEAD_DIM, dtype):
     assert_scores_close(scores, want, dtype, "dense scores")
 
 
+@pytest.mark.parametrize("n_kv", [261888, 262144, 262145])
+def test_dense_forward_at_the_limit_of_the_key_tiles(n_kv):
+    """The matrix-core forward kernel of head size 128 keeps 12 bytes per 64 keys beside its 112 KiB of stages: 262144 keys fill
+    a compute unit's 160 KiB to the last byte, one more goes to the kernels for any size.  P and the result are rounded at most
+    once each (half a bfloat16 unit, 2^-9); a tile left out or taken twice would be 1.5 % of these rows."""
+    from cascading_kv_cache_amd.flash_attention import attention
+
+    torch.manual_seed(24)
+    n_ctx = 40
+    q, k, v = (torch.empty((1, 2, n, 128), dtype=torch.bfloat16, device="cuda").normal_(mean=0.0, std=0.5) for n in (n_ctx, n_kv, n_kv))
+    mask = torch.arange(n_kv - n_ctx, device="cuda") % 7 == 3
+    out, _ = attention(q, k, v, True, 0.125, mask, 0.9)
+    hidden = torch.cat((mask[None, :].expand(n_ctx, -1), torch.ones(n_ctx, n_ctx, dtype=torch.bool, device="cuda").triu(1)), dim=-1)
+    for h in range(2):
+        p = torch.softmax((q[0, h].double() @ k[0, h].double().T.contiguous() * 0.125).masked_fill(hidden, float("-inf")), dim=-1)
+        want = p @ v[0, h].double()
+        assert ((out[0, h].double() - want).norm() / want.norm()).item() <= 3 * 2.0 ** -9
+
+
 def test_attention_rejects_cpu_tensors():
     from cascading_kv_cache_amd import _abi
     from cascading_kv_cache_amd.flash_attention import attention
