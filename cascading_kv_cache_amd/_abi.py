@@ -230,6 +230,8 @@ def lib():
         L.ckv_update_workspace_bytes.restype = I64
         L.ckv_attn.argtypes = [C.POINTER(AttnArgs), VP]
         L.ckv_attn.restype = C.c_int
+        L.ckv_attn_update.argtypes = [C.POINTER(AttnArgs), C.POINTER(UpdateArgs), VP]
+        L.ckv_attn_update.restype = C.c_int
         L.ckv_attn_workspace_bytes.argtypes = [I64, I64, I64, I64, I64, I64, I64, C.c_int32]
         L.ckv_attn_workspace_bytes.restype = I64
         L.ckv_attn_dense.argtypes = [C.POINTER(DenseArgs), VP]

@@ -212,10 +212,21 @@ def cascade_attention(query_states, key_states, value_states, cache: CascadingKV
         a.new_scores = new_scores.data_ptr()
         ws = workspace(dev, a._need, stream)
         a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
+        u = a._update
+        if update_cache and u is not None:
+            u.k, u.v, u.s = a.k_new, a.v_new, a.new_scores
+            if u._need > a.workspace_bytes:
+                ws = workspace(dev, u._need, stream)
+                a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
+            u.workspace, u.workspace_bytes = a.workspace, a.workspace_bytes   # used by one after the other
+            on_host = cache._begin_update(u, L, Q, dev, replayable)
+            _abi.check(lib.ckv_attn_update(C.byref(a), C.byref(u), C.c_void_p(stream)), "ckv_attn_update")
+            cache._end_update(L, Q, on_host)
+            return out, new_scores
         _abi.check(lib.ckv_attn(C.byref(a), C.c_void_p(stream)), "ckv_attn")
         if update_cache:
-            if a._update is None:  # of the layouts and placements that the key above holds
-                a._update = cache._update_args(key_states, value_states, new_scores, L)
+            # the first call of the layouts and placements that the key above holds: the update is described while the attention runs
+            a._update = cache._update_args(key_states, value_states, new_scores, L)
             cache.update_state(key_states, value_states, L, score_states=new_scores, _stream=stream,
                                _device_counter=replayable, _args=a._update)
     return out, new_scores

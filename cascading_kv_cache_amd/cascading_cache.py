@@ -403,22 +403,13 @@ class CascadingKVCache:
         if score_states is None:
             score_states = torch.zeros(self.max_batch_size, self.heads, key_states.size(2),
                                        device=key_states.device, dtype=key_states.dtype)
-        if layer_idx == 0:
-            self._seen_tokens += key_states.shape[-2]
-
         a = _args
         if a is None:
             a = self._update_args(key_states, value_states, score_states, layer_idx)
         else:
             a.k, a.v, a.s = key_states.data_ptr(), value_states.data_ptr(), score_states.data_ptr()
         n_new = key_states.shape[-2]
-        table = None if _device_counter else _counter_table(key_states.device)
-        if table is not None and self._seen_host[layer_idx] < table.numel():
-            a.real_token_idx = table.data_ptr() + 8 * self._seen_host[layer_idx]
-        else:
-            table = None
-            self._flush_counter()
-            a.real_token_idx = a._counter
+        on_host = self._begin_update(a, layer_idx, n_new, key_states.device, _device_counter)
         if _stream is None:
             with on_device(key_states.device):
                 stream = raw_stream(key_states.device)
@@ -429,9 +420,24 @@ class CascadingKVCache:
             ws = workspace(key_states.device, a._need, _stream)
             a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
             _abi.check(_abi.lib().ckv_update(C.byref(a), C.c_void_p(_stream)), "ckv_update")
-        # after the kernel, as in the reference (cascading_cache.py:1343-1346)
-        if table is None:
-            self._seen_dev[layer_idx] += n_new
-        else:
+        self._end_update(layer_idx, n_new, on_host)
+
+    def _begin_update(self, a, layer_idx: int, n_new: int, device, device_counter: bool) -> bool:
+        """Points the argument block at the number of tokens seen so far; True: the host knows it."""
+        if layer_idx == 0:
+            self._seen_tokens += n_new
+        table = None if device_counter else _counter_table(device)
+        if table is not None and self._seen_host[layer_idx] < table.numel():
+            a.real_token_idx = table.data_ptr() + 8 * self._seen_host[layer_idx]
+            return True
+        self._flush_counter()
+        a.real_token_idx = a._counter
+        return False
+
+    def _end_update(self, layer_idx: int, n_new: int, on_host: bool):
+        """After the kernels, as in the reference (cascading_cache.py:1343-1346)."""
+        if on_host:
             self._seen_pending[layer_idx] += n_new
+        else:
+            self._seen_dev[layer_idx] += n_new
         self._seen_host[layer_idx] += n_new

@@ -1,5 +1,5 @@
 // Entry points of libckv that are not tied to one kernel family.
-#include "ckv_common.h"
+#include "ckv_attn_internal.h"
 
 #include <cstdint>
 #include <mutex>
@@ -68,6 +68,8 @@ static bool dispatch_timed(int stage) {
 static bool prof_wanted(int stage) { return g_prof_level == 1 || dispatch_timed(stage); }
 
 bool prof_kernel_events_wanted(int stage) { return dispatch_timed(stage); }
+
+bool prof_update_apart() { return g_prof_level == 1 || g_prof_level == 3; }
 
 void prof_kernel_events(int stage, hipEvent_t* start, hipEvent_t* stop) {
     *start = *stop = nullptr;

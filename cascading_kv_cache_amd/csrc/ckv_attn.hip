@@ -101,11 +101,12 @@ extern "C" int64_t ckv_attn_workspace_bytes(int64_t B, int64_t H, int64_t KVH, i
     return bytes;
 }
 
-extern "C" int ckv_attn(const ckv_attn_args* args, void* stream_) {
-    using namespace ckv;
+namespace ckv {
+// `u`: the cache update that the caller runs next, or null; *updated: it has been launched here
+static int run_attn(const ckv_attn_args* args, hipStream_t stream, const ckv_update_args* u, bool* updated) {
+    *updated = false;
     if (!args) return CKV_ERR_NULL;
     const ckv_attn_args& a = *args;
-    hipStream_t stream = reinterpret_cast<hipStream_t>(stream_);
     if (a.dtype != CKV_F32 && a.dtype != CKV_F16 && a.dtype != CKV_BF16) return CKV_ERR_DTYPE;
     if (a.B <= 0 || a.H <= 0 || a.KVH <= 0 || a.Q <= 0 || a.D <= 0 || a.num_sink < 0 || a.S < 0) return CKV_ERR_SHAPE;
     if (a.H % a.KVH != 0 || a.D % 2 != 0) return CKV_ERR_SHAPE;
@@ -118,7 +119,7 @@ extern "C" int ckv_attn(const ckv_attn_args* args, void* stream_) {
     if (!(a.scale > 0.f)) return CKV_ERR_SHAPE;  // queries and keys are each multiplied by its square root
     if (!a.workspace || a.workspace_bytes < ckv_attn_workspace_bytes(a.B, a.H, a.KVH, a.Q, a.D, a.num_sink, a.S, a.dtype))
         return CKV_ERR_WORKSPACE;
-    if (decode_supported(a)) return launch_decode(a, stream);
+    if (decode_supported(a)) return launch_decode(a, stream, u && update_beside_scores(a, *u) ? u : nullptr, updated);
     AttnWorkspace w = carve_attn(a.workspace, a.B, a.H, a.KVH, a.Q, a.D, a.num_sink, a.S, a.dtype);
 
     const int64_t N = a.num_sink + a.S + a.Q;
@@ -209,6 +210,21 @@ extern "C" int ckv_attn(const ckv_attn_args* args, void* stream_) {
         if (rc) return rc;
     }
     return CKV_OK;
+}
+}  // namespace ckv
+
+extern "C" int ckv_attn(const ckv_attn_args* args, void* stream) {
+    bool updated;
+    return ckv::run_attn(args, reinterpret_cast<hipStream_t>(stream), nullptr, &updated);
+}
+
+extern "C" int ckv_attn_update(const ckv_attn_args* args, const ckv_update_args* update, void* stream) {
+    using namespace ckv;
+    // An update that would be refused is refused by ckv_update, behind the attention, as in two calls.
+    bool empty, updated;
+    const bool beside = check_update(update, &empty) == CKV_OK && !empty && !prof_update_apart();
+    if (int rc = run_attn(args, reinterpret_cast<hipStream_t>(stream), beside ? update : nullptr, &updated)) return rc;
+    return updated ? CKV_OK : ckv_update(update, stream);
 }
 
 namespace ckv {

@@ -16,6 +16,7 @@
 //   decode_scores P = exp2(logit - lse) exactly, head reduction, score EMA of every slot and the
 //                 new token's own score (cascade_attention.py:315-330 with q_len == 1).
 #include "ckv_attn_internal.h"
+#include "ckv_update_token.h"
 
 #include <algorithm>
 #include <type_traits>
@@ -115,6 +116,37 @@ struct DecodeParams {
     // of the new token (`tiles - 1`) when it is not one of them.  A cache that is still filling is mostly hidden.
     int tiles_pre;
     int n_vis;         // tiles_pre, or tiles_pre + 1
+    // The cache update in the launch behind the streaming kernel, see TokenPlan; plans null: it is not done there.
+    ckv_update_args u;
+    int32_t* plans;    // [B * KVH][kPlanWords]
+};
+
+// The update of a decoding step beside its scores.  Where the token and the rows it displaces may land, and the trackers after
+// the call, hang on the trackers alone (TokenPath), so a wavefront of the streaming kernel works them out, a (batch, kv head)
+// each, while its first rows are on their way, and leaves them in scratch.  The launch behind it then has everything in one
+// go: the workgroups of the scores leave out the few slots on the token's path, others write the position ids; one
+// workgroup per (batch, kv head) works out the scores of those itself, decides, moves the rows and commits the trackers.
+// Nobody reads what another workgroup of the launch writes, so no order between them is needed.  Plan and moves as launches of
+// their own cost a step of one stream 6.2 us on 2 K slots (one launch) and 9.7 on 64 K (two), most of it trips to memory that
+// the scores make too; the launch they ride in now takes 7.2 where it took 6.0 and 9.5 where it took 7.0.
+constexpr int kPlanCascades = 31;       // lane i: cascade i; a workgroup moves 32 rows at once
+constexpr int kPlanWords = 4 * CKV_WAVE;
+struct TokenPlan {
+    int32_t slot, st, sx;               // lane: TokenPath::slot and the trackers after the call
+    int32_t head;                       // lane 0: stop | ends | takes | sink; lane 1: sinks stored before the call
+    static constexpr int kEnds = 256, kTakes = 512, kSink = 1024;
+    __device__ inline void of(const TokenPath& w, const TokenTrackers& t, int lane) {
+        slot = w.slot;
+        st = w.st_new;
+        sx = w.sx_new;
+        head = lane == 0 ? w.stop | (w.ends ? kEnds : 0) | (w.takes ? kTakes : 0) | (w.sink ? kSink : 0) : (int32_t)t.sinks;
+    }
+    __device__ inline void store(int32_t* words, int lane) const {
+        words[lane] = slot;
+        words[CKV_WAVE + lane] = st;
+        words[2 * CKV_WAVE + lane] = sx;
+        if (lane < 2) words[3 * CKV_WAVE + lane] = head;
+    }
 };
 
 // the j-th tile with items; the rank of a tile among those (-1: the tile has no items, its keys are all hidden)
@@ -765,6 +797,31 @@ struct SharedQueries {
     }
 };
 
+// The wavefront of the streaming kernels that plans the update of a (batch, kv head), where the step has one: the last
+// wavefront of as many workgroups, counted from the end (those from the front may have an item more).  Its words stay in registers until
+// the run is over: a store behind the first copies would be one more thing for the first wait to wait for.
+struct StreamPlanner {
+    int unit;   // -1: none
+    TokenTrackers t;
+    TokenPlan plan;
+    __device__ inline StreamPlanner(const DecodeParams& p, int wave) : t{}, plan{} {
+        const int u = p.stream_wgs - 1 - (int)blockIdx.x;
+        unit = p.plans && wave == kStreamWaves - 1 && u < p.nbh ? u : -1;
+    }
+    __device__ inline void request(const DecodeParams& p, int lane) {
+        if (unit < 0) return;
+        const uint32_t n = (uint32_t)unit / (uint32_t)p.a.KVH;
+        t.request(p.u, n, (int64_t)((uint32_t)unit - n * (uint32_t)p.a.KVH), 0, lane);
+    }
+    __device__ inline void arrived() { asm volatile("" : "+v"(t.st), "+v"(t.sx), "+v"(t.per), "+v"(t.sinks), "+v"(t.index)); }
+    __device__ inline void work_out(const DecodeParams& p, int lane) {
+        if (unit >= 0) plan.of(token_path(p.u, t, lane), t, lane);
+    }
+    __device__ inline void store(const DecodeParams& p, int lane) const {
+        if (unit >= 0) plan.store(p.plans + unit * kPlanWords, lane);
+    }
+};
+
 // the byte offsets of the rows inside a (b, kvh) slab must fit the 32-bit lane offsets of the copies
 inline bool stream_offsets_fit(const ckv_attn_args& a) {
     const int64_t lim = (int64_t)1 << 31, es = 2;
@@ -1008,14 +1065,18 @@ __global__ void __launch_bounds__(kStreamThreads, kStreamWgPerCu) decode_stream_
         kvh = bh - b * KVH;
     }
     SharedQueries<T, G> shared;
+    StreamPlanner planner(p, wave);
     shared.request(p, tid, wave);
+    planner.request(p, lane);
     rows.request(jt);
     rows.copy_from(jt);
     rows.arrived();
     shared.arrived();
+    planner.arrived();
     copy_kq(b, kvh, 0);
     copy_v(b, kvh, 0);
     shared.finish(p, freqs, smem + kStreamOwnQ, tid, wave);
+    planner.work_out(p, lane);
     rows.take(freqs);
     bool request = (jt + 1) * nbh < item1;
     // Loads and stores retire in issue order, so "at most n operations outstanding" with n younger ones issued after the
@@ -1171,6 +1232,7 @@ __global__ void __launch_bounds__(kStreamThreads, kStreamWgPerCu) decode_stream_
         }
     }
     flush();
+    planner.store(p, lane);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1288,14 +1350,18 @@ __global__ void __launch_bounds__(kStreamThreads, kStreamWgPerCu) decode_stream_
         kvh = bh - b * KVH;
     }
     SharedQueries<T, G> shared;
+    StreamPlanner planner(p, wave);
     shared.request(p, tid, wave);
+    planner.request(p, lane);
     rows.request(jt);
     rows.copy_from(jt);
     rows.arrived();
     shared.arrived();
+    planner.arrived();
     copy_kq(b, kvh, 0);
     copy_v(b, kvh, 0);
     shared.finish(p, freqs, smem + kWideOwnQ, tid, wave);
+    planner.work_out(p, lane);
     rows.take(freqs);
     bool request = (jt + 1) * nbh < item1;
     // Per item a wavefront issues, in this order: [the query copy of the next item,] four K copies of the
@@ -1441,6 +1507,7 @@ __global__ void __launch_bounds__(kStreamThreads, kStreamWgPerCu) decode_stream_
         }
     }
     flush();
+    planner.store(p, lane);
 }
 
 // one workgroup per (b, h): 16 groups of 32 threads walk every 16th tile, eight tiles in flight, then merge
@@ -1603,6 +1670,39 @@ __device__ inline void tail_stream_row(const DecodeParams& p, int row, TailLds& 
     }
 }
 
+// The position ids of kPosSlots slots of a (b, kvh) from its TokenPlan, by a workgroup of 512 threads; `id`: unit * blocks + block.
+constexpr int kPosSlots = 4096;
+__host__ __device__ inline int pos_blocks(int64_t S) { return (int)((S + kPosSlots - 1) / kPosSlots); }
+__device__ inline void token_positions(const DecodeParams& p, int id, PosRange* ranges) {
+    const ckv_update_args& A = p.u;
+    const uint32_t W = (uint32_t)A.window_size, S = (uint32_t)A.max_seq_len, tid = threadIdx.x, KVH = (uint32_t)p.a.KVH;
+    const uint32_t blocks = (uint32_t)pos_blocks(S), unit = (uint32_t)id / blocks, first = ((uint32_t)id - unit * blocks) * kPosSlots;
+    const uint32_t b = unit / KVH, kvh = unit - b * KVH;
+    if (tid < CKV_WAVE) {
+        const int32_t* words = p.plans + unit * kPlanWords;
+        PosRange range = pos_range((int)tid, A.cascades, (int32_t)W, words[CKV_WAVE + tid], words[2 * CKV_WAVE + tid]);
+        if (words[3 * CKV_WAVE] & TokenPlan::kSink) range.write = false;
+        if ((int)tid < A.cascades) ranges[tid] = range;
+    }
+    __syncthreads();
+    int64_t* pos = A.pos + (int64_t)b * A.pos_stride[0] + (int64_t)kvh * A.pos_stride[1];
+    if (A.pos_stride[2] == 1 && (reinterpret_cast<uintptr_t>(pos) & 15u) == 0 && (W & 1) == 0) {
+#pragma unroll
+        for (int it = 0; it < kPosSlots / 1024; it++) {
+            const uint32_t j = first + it * 1024 + 2 * tid;
+            if (j >= S) break;
+            const uint32_t i = j / W, r = j - i * W;
+            const PosRange range = ranges[i];
+            if (range.write) *reinterpret_cast<longlong2*>(pos + j) = make_longlong2(range.id_of(r), range.id_of(r + 1));
+        }
+    } else {
+        for (uint32_t j = first + tid; j < first + kPosSlots && j < S; j += 512) {
+            const uint32_t i = j / W;
+            if (ranges[i].write) pos[(int64_t)j * A.pos_stride[2]] = ranges[i].id_of(j - i * W);
+        }
+    }
+}
+
 template <typename T>
 __global__ void __launch_bounds__(512) decode_tail_stream_kernel(DecodeParams p) {
     __shared__ TailLds sh;
@@ -1706,6 +1806,38 @@ __global__ void __launch_bounds__(256) decode_scores_kernel(DecodeParams p, floa
     }
 }
 
+// One key's score after a streaming kernel, of the G heads of its kv head (cascade_attention.py:319-323 with a single query
+// row): e[g] = 2^(logit - tile maximum), c[g] = 2^(tile maximum - normaliser).
+template <typename T, int G, int kMode>
+__device__ inline float key_score(const float (&e)[G], const float (&c)[G], float w) {
+    float vals[G];
+    // cached slots: fp32 product, cast; the new token: product in the tensor dtype
+#pragma unroll
+    for (int g = 0; g < G; g++) vals[g] = round_t<T>(__fmul_rn(e[g] == 0.f ? 0.f : round_t<T>(e[g] * c[g]), w));
+    float r = vals[0];
+    if constexpr (kMode == CKV_REDUCE_MAX) {
+#pragma unroll
+        for (int g = 1; g < G; g++) r = fmaxf(r, vals[g]);
+    } else if constexpr (kMode == CKV_REDUCE_MEAN) {
+        r = 0.f;
+#pragma unroll
+        for (int g = 0; g < G; g++) r = __fadd_rn(r, vals[g]);
+        r = round_t<T>(r / (float)G);
+    } else {  // lower median: rank by counting
+#pragma unroll
+        for (int g = 0; g < G; g++) {
+            int below = 0, equal = 0;
+#pragma unroll
+            for (int h = 0; h < G; h++) {
+                below += vals[h] < vals[g];
+                equal += vals[h] == vals[g];
+            }
+            if (below <= (G - 1) / 2 && (G - 1) / 2 < below + equal) r = vals[g];
+        }
+    }
+    return r;
+}
+
 // The same after the streaming kernel, per kv head: one thread per (b, kvh, 8 consecutive keys), which are one
 // 16-byte piece of each head's fp16 probabilities and share the tile maximum.  Such a thread is little else than trips to memory:
 // what it reads is requested in one go (request) and none of it waits for the normalisers, which finish() takes.  As loads behind
@@ -1742,8 +1874,9 @@ struct ScoresOfGroup {
         old = *reinterpret_cast<const uint4*>(some && whole ? reinterpret_cast<const unsigned char*>(cs + i0) : chunk);
     }
 
-    // lse[g]: the log2-domain normaliser of head g of the kv head
-    __device__ inline void finish(const DecodeParams& p, int64_t b, int64_t kvh, float w_one, float beta_pow, const float (&lse)[G]) {
+    // lse[g]: the log2-domain normaliser of head g of the kv head.  skip: bit k is set where key k keeps its score.
+    __device__ inline void finish(const DecodeParams& p, int64_t b, int64_t kvh, float w_one, float beta_pow, const float (&lse)[G],
+                                  uint32_t skip = 0) {
         if (!some) return;
         const ckv_attn_args& a = p.a;
         float c[G], red[8];
@@ -1754,46 +1887,21 @@ struct ScoresOfGroup {
         }
         const float w_new = round_t<T>(w_one);
         auto reduce = [&](auto mode_tag) {   // a mode per copy of the loop: one branch in front instead of two per key
-            constexpr int mode = decltype(mode_tag)::value;
 #pragma unroll
             for (int k = 0; k < 8; k++) {
-                const float w = n0 + k == p.N - 1 ? w_new : w_one;
-                float vals[G];
-                // cached slots: fp32 product, cast; the new token: product in the tensor dtype
+                float e[G];
 #pragma unroll
                 for (int g = 0; g < G; g++) {
                     const uint32_t word = k < 4 ? (k < 2 ? raw[g].x : raw[g].y) : (k < 6 ? raw[g].z : raw[g].w);
-                    const float e = (float)__builtin_bit_cast(f16x2_t, word)[k & 1];
-                    vals[g] = round_t<T>(__fmul_rn(e == 0.f ? 0.f : round_t<T>(e * c[g]), w));
+                    e[g] = (float)__builtin_bit_cast(f16x2_t, word)[k & 1];
                 }
-                float r = vals[0];
-                if constexpr (mode == CKV_REDUCE_MAX) {
-#pragma unroll
-                    for (int g = 1; g < G; g++) r = fmaxf(r, vals[g]);
-                } else if constexpr (mode == CKV_REDUCE_MEAN) {
-                    r = 0.f;
-#pragma unroll
-                    for (int g = 0; g < G; g++) r = __fadd_rn(r, vals[g]);
-                    r = round_t<T>(r / (float)G);
-                } else {  // lower median: rank by counting
-#pragma unroll
-                    for (int g = 0; g < G; g++) {
-                        int below = 0, equal = 0;
-#pragma unroll
-                        for (int h = 0; h < G; h++) {
-                            below += vals[h] < vals[g];
-                            equal += vals[h] == vals[g];
-                        }
-                        if (below <= (G - 1) / 2 && (G - 1) / 2 < below + equal) r = vals[g];
-                    }
-                }
-                red[k] = r;
+                red[k] = key_score<T, G, decltype(mode_tag)::value>(e, c, n0 + k == p.N - 1 ? w_new : w_one);
             }
         };
         if (a.head_reduction == CKV_REDUCE_MAX) reduce(std::integral_constant<int, CKV_REDUCE_MAX>{});
         else if (a.head_reduction == CKV_REDUCE_MEAN) reduce(std::integral_constant<int, CKV_REDUCE_MEAN>{});
         else reduce(std::integral_constant<int, CKV_REDUCE_MEDIAN>{});
-        if (whole) {
+        if (whole && skip == 0) {
             T* o = reinterpret_cast<T*>(&old);
 #pragma unroll
             for (int k = 0; k < 8; k++) {
@@ -1810,7 +1918,7 @@ struct ScoresOfGroup {
             if (i == a.S) {
                 if (a.new_scores)
                     *((T*)a.new_scores + b * a.new_scores_stride[0] + kvh * a.new_scores_stride[1]) = Elem<T>::from_float(red[k]);
-            } else if (cs) {
+            } else if (cs && (skip >> k & 1u) == 0) {
                 T* c1 = cs + i * a.cache_s_stride[2];
                 const float decayed = round_t<T>(__fmul_rn(beta_pow, Elem<T>::to_float(*c1)));
                 *c1 = Elem<T>::from_float(__fadd_rn(decayed, red[k]));
@@ -1834,63 +1942,235 @@ __global__ void __launch_bounds__(256) decode_scores_probs_kernel(DecodeParams p
     scores.finish(p, b, kvh, w_one, beta_pow, lse);
 }
 
-// Tail and scores in one launch: the first B * H workgroups combine a row each, the others work out the scores of 4096
-// keys of one (b, kvh), for which they merge the (maximum, sum) pairs of its G heads themselves, on top of what a score thread
-// reads, which is requested before.  Where all workgroups run side by side that is hidden behind the rows, and a launch is saved
-// (host and device: about 4 us): one launch against two, us, 1 stream x 64 K slots 6.9 and 6.6 + 4.8, 4 x 32 K 8.9 and 5.8 + 6.1,
-// 2 x 64 K 10.2 and 6.9 + 6.3.  Where they come in rounds every score workgroup pays for its merge: 16 streams x 32 K slots, 1664
-// workgroups, 25.4 and 10.1 + 12.1; 8 x 32 K, 832, 15.2 and 7.2 + 8.0.  The line at two workgroups a compute unit is on the safe
-// side (5 x 32 K, 520 workgroups, 12.4 and 6.2 + 6.5; 16 x 2 K, 640, 8.0 and 4.8 + 4.1).
+// The log2-domain normalisers of the G heads of a (b, kvh) into LDS, a wavefront per head (the first G of a workgroup), from the
+// (maximum, sum) pairs of its tiles.
+template <int G>
+__device__ inline void unit_normalisers(const DecodeParams& p, int unit, float* sh_lse) {
+    static_assert(G <= 8, "a wavefront per head merges the pairs");
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (wave >= G) return;
+    float M = -INFINITY, L = 0.f;
+    constexpr int kBatch = 9;   // tiles of a lane on their way at once: 64 K slots in one trip
+    for (int t0 = lane; t0 < p.n_vis; t0 += 64 * kBatch) {
+        float2 w[kBatch];
+#pragma unroll
+        for (int u = 0; u < kBatch; u++) {
+            const int t = t0 + 64 * u;
+            w[u] = make_float2(-INFINITY, 0.f);
+            if (t < p.n_vis) {
+                const int64_t ck = stream_chunk_of(p, t * p.nbh + unit);
+                w[u] = *reinterpret_cast<const float2*>(p.part_ml + (ck * G + wave) * 2);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < kBatch; u++) {
+            const float m = fmaxf(M, w[u].x);
+            if (m == -INFINITY) continue;
+            L = L * __builtin_amdgcn_exp2f(M - m) + w[u].y * __builtin_amdgcn_exp2f(w[u].x - m);
+            M = m;
+        }
+    }
+    float Mx = M;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) Mx = fmaxf(Mx, __shfl_xor(Mx, off));
+    L = M == -INFINITY ? 0.f : L * __builtin_amdgcn_exp2f(M - Mx);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) L += __shfl_xor(L, off);
+    if (lane == 0) sh_lse[wave] = Mx + __builtin_amdgcn_logf(L);
+}
+
+// The update of a (b, kvh) by a workgroup of 512 threads, see TokenPlan.  Group j of 16 lanes has the row that may come to slot j of the path
+// (the token, or what lies in slot j - 1), requested before anything is known; lane j of wavefront 0 has the score of what
+// lies in slot j, lane 63 the token's, as the workgroups of the scores work them out.
 template <typename T, int G>
+struct TokenUpdate {
+    uint4 rk, rv;      // this lane's pieces of the row
+    int64_t og;        // lane 0 of a group: the row's original index
+    float e[G], tile_m[G];   // wavefront 0: this lane's key, as in ScoresOfGroup
+    uint16_t old;      // its score
+    int slot, head, sinks;
+    int to, st, sx;    // the slot that the row may come to; lanes of group kTrackerGroup: trackers after the call
+    bool wanted, seen;
+    static constexpr int kTrackerGroup = 31;   // a group of 16 lanes that no path reaches: two cascades a lane
+
+    __device__ inline void request(const DecodeParams& p, int unit, int b, int kvh) {
+        const ckv_update_args& A = p.u;
+        const int tid = threadIdx.x, lane = tid & 63, j = tid >> 4, piece = tid & 15;
+        const int32_t* words = p.plans + unit * kPlanWords;
+        head = words[3 * CKV_WAVE];
+        sinks = words[3 * CKV_WAVE + 1];
+        const int stop = head & 255, last = stop - ((head & TokenPlan::kEnds) ? 0 : 1);   // the path's last slot (a sink: none)
+        to = words[j];
+        if (j == kTrackerGroup) {
+            st = words[CKV_WAVE + stop % CKV_WAVE];   // of the one cascade whose count may have changed
+            sx = words[2 * CKV_WAVE + piece];
+            to = words[2 * CKV_WAVE + 16 + piece];
+        }
+        const int from = j > 0 && j <= last ? words[j - 1] : 0;   // a group without a slot of the path reads a row that nobody takes
+        if (j == 0) {
+            const int64_t at = (b * A.kv_stride[0] + kvh * A.kv_stride[1]) * 2;
+            rk = reinterpret_cast<const uint4*>((const char*)A.k + at)[piece];
+            rv = reinterpret_cast<const uint4*>((const char*)A.v + at)[piece];
+            og = *A.real_token_idx + 1;   // cascading_cache.py:388
+        } else {
+            const int64_t at = (b * A.cache_stride[0] + kvh * A.cache_stride[1] + (int64_t)from * A.cache_stride[2]) * 2;
+            rk = reinterpret_cast<const uint4*>((const char*)A.cache_k + at)[piece];
+            rv = reinterpret_cast<const uint4*>((const char*)A.cache_v + at)[piece];
+            og = A.og_pos[b * A.og_pos_stride[0] + kvh * A.og_pos_stride[1] + (int64_t)from * A.og_pos_stride[2]];
+        }
+        if (tid >= CKV_WAVE) return;
+        wanted = lane <= last || lane == CKV_WAVE - 1;
+        slot = words[lane];
+        const int n = lane == CKV_WAVE - 1 ? (int)(p.N - 1) : (int)p.a.num_sink + (lane <= last ? slot : 0);
+        const int jt = wanted ? stream_rank_of(p, n / kSK) : -1;
+        seen = jt >= 0;
+        const int64_t ck = seen ? stream_chunk_of(p, jt * p.nbh + unit) : 0;
+        const _Float16* chunk = reinterpret_cast<const _Float16*>(p.chunks + ck * (G * (kSK + kD) * 2)) + n % kSK;
+#pragma unroll
+        for (int g = 0; g < G; g++) {
+            e[g] = (float)chunk[g * kSK];
+            tile_m[g] = p.part_ml[(ck * G + g) * 2];
+        }
+        old = lane <= last ? ((const uint16_t*)A.cache_s)[b * A.cache_s_stride[0] + kvh * A.cache_s_stride[1] + (int64_t)slot * A.cache_s_stride[2]]
+                           : (uint16_t)0;
+    }
+
+    // sh_score: what the slots of the path are to hold, sh_head: their number and whether the last one keeps its row
+    __device__ inline void decide(const DecodeParams& p, float w_one, float beta_pow, const float* sh_lse, uint16_t* sh_score, int* sh_count) {
+        const int lane = threadIdx.x & 63, stop = head & 255;
+        float c[G], ev[G];
+#pragma unroll
+        for (int g = 0; g < G; g++) {
+            c[g] = __builtin_amdgcn_exp2f(tile_m[g] - sh_lse[g]);
+            ev[g] = seen ? e[g] : 0.f;
+        }
+        const bool token = lane == CKV_WAVE - 1;
+        const float w = token ? round_t<T>(w_one) : w_one;
+        const float red = p.a.head_reduction == CKV_REDUCE_MAX    ? key_score<T, G, CKV_REDUCE_MAX>(ev, c, w)
+                          : p.a.head_reduction == CKV_REDUCE_MEAN ? key_score<T, G, CKV_REDUCE_MEAN>(ev, c, w)
+                                                                  : key_score<T, G, CKV_REDUCE_MEDIAN>(ev, c, w);
+        const float decayed = round_t<T>(__fmul_rn(beta_pow, Elem<T>::to_float(__builtin_bit_cast(T, old))));
+        const T kept = Elem<T>::from_float(token ? red : __fadd_rn(decayed, red));
+        const float mine = Elem<T>::to_float(kept);
+        // the score that comes to slot j: the token's, or that of what lay in slot j - 1
+        float carried = __shfl(mine, lane > 0 ? lane - 1 : CKV_WAVE - 1);
+        const bool lands = (head & TokenPlan::kTakes) != 0 || carried >= mine;
+        const bool moves = lane < stop || ((head & TokenPlan::kEnds) != 0 && lane == stop && lands);
+        const int comes = __shfl((int)__builtin_bit_cast(uint16_t, kept), lane > 0 ? lane - 1 : CKV_WAVE - 1);
+        if (lane < 32) sh_score[lane] = moves ? (uint16_t)comes : __builtin_bit_cast(uint16_t, kept);
+        const unsigned long long moved = __builtin_amdgcn_ballot_w64(moves);
+        if (lane == 0) *sh_count = (head & TokenPlan::kSink) ? 1 : __builtin_popcountll(moved);
+    }
+
+    __device__ inline void commit(const DecodeParams& p, int b, int kvh, const uint16_t* sh_score, int count) {
+        const ckv_update_args& A = p.u;
+        const int tid = threadIdx.x, j = tid >> 4, piece = tid & 15, stop = head & 255;
+        const bool sink = (head & TokenPlan::kSink) != 0;
+        const int64_t at = b * A.tracker_stride[0] + kvh * A.tracker_stride[1];
+        if (j == kTrackerGroup) {
+            if (sink) {
+                if (piece == 0) A.stored_sinks[b * A.stored_sinks_stride[0] + kvh * A.stored_sinks_stride[1]] = sinks + 1;
+                return;
+            }
+            if (piece < stop) A.start_indices[at + piece * A.tracker_stride[2]] = sx;
+            if (piece + 16 < stop) A.start_indices[at + (piece + 16) * A.tracker_stride[2]] = to;
+            if (piece == 0 && (head & TokenPlan::kTakes)) A.stored_tokens[at + stop * A.tracker_stride[2]] = st;
+            return;
+        }
+        const bool holds = !sink && (head & TokenPlan::kEnds) && j == stop;   // challenged in vain: its row stays, its score is due
+        if (j >= count && !holds) return;
+        if (sink) {  // cascading_cache.py:61-109; only the token itself gets here
+            const int64_t i = sinks, so = (b * A.sink_stride[0] + kvh * A.sink_stride[1] + i * A.sink_stride[2]) * 2;
+            reinterpret_cast<uint4*>((char*)A.sink_k + so)[piece] = rk;
+            reinterpret_cast<uint4*>((char*)A.sink_v + so)[piece] = rv;
+            if (piece == 0) {
+                A.sink_pos[b * A.sink_pos_stride[0] + kvh * A.sink_pos_stride[1] + i * A.sink_pos_stride[2]] = i;
+                A.sink_mask[b * A.sink_mask_stride[0] + kvh * A.sink_mask_stride[1] + i * A.sink_mask_stride[2]] = 0;
+            }
+            asm volatile("");   // else the stores of both ways become one, with its strides picked from a copy in scratch memory
+            return;
+        }
+        if (piece == 0) ((uint16_t*)A.cache_s)[b * A.cache_s_stride[0] + kvh * A.cache_s_stride[1] + (int64_t)to * A.cache_s_stride[2]] = sh_score[j];
+        if (j >= count) return;
+        const int64_t so = (b * A.cache_stride[0] + kvh * A.cache_stride[1] + (int64_t)to * A.cache_stride[2]) * 2;
+        reinterpret_cast<uint4*>((char*)A.cache_k + so)[piece] = rk;
+        reinterpret_cast<uint4*>((char*)A.cache_v + so)[piece] = rv;
+        if (piece == 0) {
+            A.og_pos[b * A.og_pos_stride[0] + kvh * A.og_pos_stride[1] + (int64_t)to * A.og_pos_stride[2]] = og;
+            A.mask[b * A.mask_stride[0] + kvh * A.mask_stride[1] + (int64_t)to * A.mask_stride[2]] = 0;
+        }
+    }
+};
+
+// Tail and scores in one launch, and with kUpdate the cache update (TokenPlan): a workgroup per (b, kvh) with the rows that move, in
+// front, as theirs is the longest way; B * H workgroups that combine a row each; those that work out the scores of 4096
+// keys of one (b, kvh), for which they merge the (maximum, sum) pairs of its G heads themselves, on top of what a score thread
+// reads, which is requested before; those that write 4096 position ids.  Three or four launches less than one by one, each of which
+// takes 4 us to come to anything.  A step, us, with separate launches for rows, scores and update and with this one: 1 stream x
+// 2 K slots 24.8 19.4, x 16 K 35.0 29.6, x 64 K 73.8 65.6; 2 x 64 K 124.8 116.7; 4 x 32 K 127.9 116.6; 16 x 2 K 51.8 47.6, x 32 K
+// 440.2 420.8 (up to 4 x 32 K rows and scores were one launch before).  Without an update: 5 x 32 K 146.4 139.5, 16 x 2 K 45.3 42.1,
+// x 32 K 426.4 412.5, 64 x 8 K 439.9 436.8, 16 x 64 K 809.6 818.5: the more workgroups and tiles, the more the merges repeat.
+// These have 4 sinks, where eight keys of a thread are no aligned piece of the scores and the launch of the scores alone takes
+// half as long again; the line is at eight workgroups a compute unit there (1664 in all for 16 x 32 K, 2688 for 16 x 64 K).  With 64
+// sinks 8 x 32 K (832) 218.0 215.1, 12 x 16 K (864) 170.1 168.7, 16 x 32 K 412.7 416.6: it is at four.  (Position ids by the
+// workgroups of the scores: 64 K slots 66.0; a launch for the rows and the ids, then one for scores and update: 16 x 32 K 417;
+// no more than 80 registers, for a workgroup more a compute unit: level.)
+inline int64_t finish_workgroups_per_cu(int64_t num_sink) { return num_sink % 8 == 0 ? 4 : 8; }
+template <typename T, int G, bool kUpdate>
 __global__ void __launch_bounds__(512) decode_finish_kernel(DecodeParams p, float w_one, float beta_pow, int per_unit) {
     __shared__ TailLds sh;
     const ckv_attn_args& a = p.a;
-    const int rows = (int)(a.B * a.H), tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    if ((int)blockIdx.x < rows) {
-        tail_stream_row<T>(p, (int)blockIdx.x, sh);
+    const int tid = threadIdx.x, KVH = (int)a.KVH;
+    float* sh_lse = &sh.m[0];
+    int id = (int)blockIdx.x;
+    if constexpr (kUpdate) {
+        if (id < p.nbh) {
+            uint16_t* sh_score = reinterpret_cast<uint16_t*>(&sh.o[0][0]);
+            int* sh_count = reinterpret_cast<int*>(&sh.l[0]);
+            const int b = (int)((uint32_t)id / (uint32_t)KVH), kvh = id - b * KVH;
+            TokenUpdate<T, G> update;
+            update.request(p, id, b, kvh);
+            unit_normalisers<G>(p, id, sh_lse);
+            __syncthreads();
+            if (tid < CKV_WAVE) update.decide(p, w_one, beta_pow, sh_lse, sh_score, sh_count);
+            __syncthreads();   // and every row is in registers
+            update.commit(p, b, kvh, sh_score, *sh_count);
+            return;
+        }
+        id -= p.nbh;
+    }
+    const int rows = (int)(a.B * a.H);
+    if (id < rows) {
+        tail_stream_row<T>(p, id, sh);
         return;
     }
-    static_assert(G <= 8, "a wavefront per head merges the pairs");
-    const int id = (int)blockIdx.x - rows, unit = (int)((uint32_t)id / (uint32_t)per_unit), KVH = (int)a.KVH;
-    float* sh_lse = &sh.m[0];
-    const int b = (int)((uint32_t)unit / (uint32_t)KVH);
+    id -= rows;
+    if (kUpdate && id >= p.nbh * per_unit) {
+        token_positions(p, id - p.nbh * per_unit, reinterpret_cast<PosRange*>(&sh));
+        return;
+    }
+    const int unit = (int)((uint32_t)id / (uint32_t)per_unit), part = id - unit * per_unit;
+    const int b = (int)((uint32_t)unit / (uint32_t)KVH), kvh = unit - b * KVH;
     ScoresOfGroup<T, G> scores;
-    scores.request(p, ((int64_t)(id - unit * per_unit) * 512 + tid) * 8, b, unit - b * KVH);
-    if (wave < G) {
-        float M = -INFINITY, L = 0.f;
-        constexpr int kBatch = 4;   // tiles of a lane on their way at once
-        for (int t0 = lane; t0 < p.n_vis; t0 += 64 * kBatch) {
-            float2 w[kBatch];
-#pragma unroll
-            for (int u = 0; u < kBatch; u++) {
-                const int t = t0 + 64 * u;
-                w[u] = make_float2(-INFINITY, 0.f);
-                if (t < p.n_vis) {
-                    const int64_t ck = stream_chunk_of(p, t * p.nbh + unit);
-                    w[u] = *reinterpret_cast<const float2*>(p.part_ml + (ck * G + wave) * 2);
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < kBatch; u++) {
-                const float m = fmaxf(M, w[u].x);
-                if (m == -INFINITY) continue;
-                L = L * __builtin_amdgcn_exp2f(M - m) + w[u].y * __builtin_amdgcn_exp2f(w[u].x - m);
-                M = m;
+    scores.request(p, ((int64_t)part * 512 + tid) * 8, b, kvh);
+    uint32_t skip = 0;
+    if constexpr (kUpdate) {
+        const int32_t* words = p.plans + unit * kPlanWords;
+        const int lane = tid & 63, path = words[lane];
+        const int head = __builtin_amdgcn_readfirstlane(words[3 * CKV_WAVE]);
+        if ((head & TokenPlan::kSink) == 0) {
+            for (int j = 0; j <= (head & 255); j++) {   // the slots of the path; -1 behind them, whose distance no key has
+                const int off = __builtin_amdgcn_readlane(path, j) - (int)scores.i0;
+                if ((uint32_t)off < 8u && scores.i0 + off >= 0) skip |= 1u << off;
             }
         }
-        float Mx = M;
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) Mx = fmaxf(Mx, __shfl_xor(Mx, off));
-        L = M == -INFINITY ? 0.f : L * __builtin_amdgcn_exp2f(M - Mx);
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) L += __shfl_xor(L, off);
-        if (lane == 0) sh_lse[wave] = Mx + __builtin_amdgcn_logf(L);
     }
+    unit_normalisers<G>(p, unit, sh_lse);
     __syncthreads();
     float lse[G];
 #pragma unroll
     for (int g = 0; g < G; g++) lse[g] = sh_lse[g];
-    scores.finish(p, b, unit - b * KVH, w_one, beta_pow, lse);
+    scores.finish(p, b, kvh, w_one, beta_pow, lse, skip);
 }
 
 // All heads reduced together (cascade_attention.py:240-242) after a streaming kernel: one thread per (batch, key),
@@ -1972,10 +2252,12 @@ __global__ void __launch_bounds__(kSK) decode_scores_homo_kernel(DecodeParams p,
     }
 }
 
+// *updated: the update that p.plans asks for has been launched too
 template <typename T, int G>
-int run_decode(const DecodeParams& p_in, hipStream_t stream) {
+int run_decode(const DecodeParams& p_in, hipStream_t stream, bool* updated) {
     DecodeParams p = p_in;
     const ckv_attn_args& a = p.a;
+    *updated = false;
     const bool use_stream =
         !std::is_same<T, float>::value && G <= 8 && p.shared_pos && stream_offsets_fit(a) &&
         (p.N + kSK) * a.B * a.KVH < (int64_t)1 << 34;   // items and eighths of their keys are numbered in 32 bits
@@ -1989,6 +2271,14 @@ int run_decode(const DecodeParams& p_in, hipStream_t stream) {
     }
     p.Np = (int64_t)p.tiles * kSK;
     p.own_q = use_stream && a.B * a.H <= kOwnQRows;
+    if (!use_stream) p.plans = nullptr;
+    int64_t finish_blocks = 0;   // of decode_finish_kernel, where the step ends in it
+    if (use_stream && !a.homogeneous_heads && (a.cache_s || a.new_scores)) {
+        DeviceInfo di;
+        if (int rc = current_device_info(&di)) return rc;
+        finish_blocks = a.B * a.H + a.B * a.KVH * ((p.Np / 8 + 511) / 512);
+        if (finish_blocks > finish_workgroups_per_cu(a.num_sink) * (int64_t)di.cus) finish_blocks = 0;
+    }
     p.inv_h = (uint32_t)((65536 + a.H - 1) / a.H);
     {
         // timed stages: a call has this one either way, empty where the streaming kernel rotates the queries itself
@@ -2024,6 +2314,7 @@ int run_decode(const DecodeParams& p_in, hipStream_t stream) {
                 p.stream_wgs = (int)wgs;
                 p.run_q = (int)(p.n_vis * nbh / wgs);
                 p.run_r = (int)(p.n_vis * nbh % wgs);
+                if (finish_blocks == 0 || nbh > wgs) p.plans = nullptr;
                 hipEvent_t ev0, ev1;
                 prof_kernel_events(CKV_STAGE_DECODE, &ev0, &ev1);
                 if constexpr (G <= 4) {
@@ -2052,13 +2343,14 @@ int run_decode(const DecodeParams& p_in, hipStream_t stream) {
         StageScope sc(CKV_STAGE_DECODE_TAIL, stream);
         bool launched = false;
         if constexpr (G <= 8 && !std::is_same<T, float>::value) {
-            DeviceInfo di;
-            if (int rc = current_device_info(&di)) return rc;
-            const int64_t per_unit = (p.Np / 8 + 511) / 512, blocks = a.B * a.H + a.B * a.KVH * per_unit;
-            if (use_stream && !a.homogeneous_heads && (a.cache_s || a.new_scores) && blocks <= 2 * (int64_t)di.cus) {
-                hipLaunchKernelGGL((decode_finish_kernel<T, G>), dim3((unsigned)blocks), dim3(512), 0, stream, p,
-                                   (float)(1.0 - a.beta), (float)a.beta, (int)per_unit);
+            if (finish_blocks > 0) {
+                const int64_t per_unit = (p.Np / 8 + 511) / 512, extra = p.plans ? a.B * a.KVH * (1 + pos_blocks(a.S)) : 0;
+                const dim3 grid((unsigned)(finish_blocks + extra));
+                const float w_one = (float)(1.0 - a.beta), beta = (float)a.beta;
+                if (p.plans) hipLaunchKernelGGL((decode_finish_kernel<T, G, true>), grid, dim3(512), 0, stream, p, w_one, beta, (int)per_unit);
+                else hipLaunchKernelGGL((decode_finish_kernel<T, G, false>), grid, dim3(512), 0, stream, p, w_one, beta, (int)per_unit);
                 CKV_HIP_TRY(hipGetLastError());
+                *updated = p.plans != nullptr;
                 return CKV_OK;
             }
             if (use_stream) {
@@ -2098,13 +2390,13 @@ int run_decode(const DecodeParams& p_in, hipStream_t stream) {
 }
 
 template <typename T>
-int run_decode_g(const DecodeParams& p, int G, hipStream_t stream) {
+int run_decode_g(const DecodeParams& p, int G, hipStream_t stream, bool* updated) {
     switch (G) {
-        case 1: return run_decode<T, 1>(p, stream);
-        case 2: return run_decode<T, 2>(p, stream);
-        case 4: return run_decode<T, 4>(p, stream);
-        case 7: return run_decode<T, 7>(p, stream);
-        case 8: return run_decode<T, 8>(p, stream);
+        case 1: return run_decode<T, 1>(p, stream, updated);
+        case 2: return run_decode<T, 2>(p, stream, updated);
+        case 4: return run_decode<T, 4>(p, stream, updated);
+        case 7: return run_decode<T, 7>(p, stream, updated);
+        case 8: return run_decode<T, 8>(p, stream, updated);
         default: return CKV_ERR_UNSUPPORTED;
     }
 }
@@ -2149,12 +2441,27 @@ inline int64_t ml_area_bytes(int64_t B, int64_t H, int64_t KVH, int64_t tiles) {
 int64_t decode_workspace_bytes(int64_t B, int64_t H, int64_t KVH, int64_t num_sink, int64_t S) {
     const int64_t N = num_sink + S + 1, tiles = (N + kMinTile - 1) / kMinTile;
     return 2 * align_up(B * H * kD * 4, 256) + logits_area_bytes(B, H, KVH, N) + ml_area_bytes(B, H, KVH, tiles) +
-           align_up(B * H * tiles * kD * 4, 256) + align_up(B * H * 4, 256);
+           align_up(B * H * tiles * kD * 4, 256) + align_up(B * H * 4, 256) + B * KVH * kPlanWords * 4;
 }
 
-int launch_decode(const ckv_attn_args& a, hipStream_t stream) {
+// Is `u` the update that belongs to the step `a`, in a form that the launch behind the streaming kernel takes?  One token, the
+// same tensors on both sides (the scores as the step leaves them, rows in 16-byte pieces, which decode_supported has looked
+// at), a score row per kv head, so that nobody else writes the slots on a token's path.
+bool update_beside_scores(const ckv_attn_args& a, const ckv_update_args& u) {
+    auto same = [](const int64_t* x, const int64_t* y, int n) { return std::equal(x, x + n, y); };
+    return u.K == 1 && u.N == a.B && u.H == a.KVH && u.HID == a.D && u.dtype == a.dtype && a.dtype != CKV_F32 && u.cascades <= kPlanCascades &&
+           u.num_sink == a.num_sink && u.max_seq_len == a.S && u.k == a.k_new && u.v == a.v_new && same(u.kv_stride, a.kv_new_stride, 4) &&
+           u.cache_k == a.cache_k && u.cache_v == a.cache_v && same(u.cache_stride, a.cache_stride, 4) &&
+           (a.num_sink == 0 || (u.sink_k == a.sink_k && u.sink_v == a.sink_v && same(u.sink_stride, a.sink_stride, 4))) &&
+           u.cache_s && u.cache_s == a.cache_s && same(u.cache_s_stride, a.cache_s_stride, 3) && u.s == a.new_scores &&
+           same(u.s_stride, a.new_scores_stride, 2) && a.cache_s_stride[2] == 1 && (a.KVH == 1 || a.cache_s_stride[1] >= a.S) &&
+           (a.B == 1 || a.cache_s_stride[0] >= a.S);
+}
+
+int launch_decode(const ckv_attn_args& a, hipStream_t stream, const ckv_update_args* u, bool* updated) {
     DecodeParams p;
     p.a = a;
+    p.u = u ? *u : ckv_update_args{};
     p.N = a.num_sink + a.S + 1;
     p.tiles = (int)((p.N + kTK - 1) / kTK);
     const int64_t G = a.H / a.KVH;
@@ -2172,14 +2479,15 @@ int launch_decode(const ckv_attn_args& a, hipStream_t stream) {
     const int64_t tiles_max = (p.N + kMinTile - 1) / kMinTile;
     p.part_ml = reinterpret_cast<float*>(w); w += ml_area_bytes(a.B, a.H, a.KVH, tiles_max);
     p.part_o = reinterpret_cast<float*>(w); w += align_up(a.B * a.H * tiles_max * kD * 4, 256);
-    p.lse2 = reinterpret_cast<float*>(w);
+    p.lse2 = reinterpret_cast<float*>(w); w += align_up(a.B * a.H * 4, 256);
+    p.plans = u ? reinterpret_cast<int32_t*>(w) : nullptr;
     p.shared_pos = a.sink_pos_stride[0] == 0 && a.sink_pos_stride[1] == 0 && a.pos_stride[0] == 0 && a.pos_stride[1] == 0;
     p.key_scale = sqrtf(a.scale);
     p.scale_log2 = 1.4426950408889634f;  // queries and keys each carry sqrt(scale)
     switch (a.dtype) {
-        case CKV_F32: return run_decode_g<float>(p, (int)G, stream);
-        case CKV_F16: return run_decode_g<__half>(p, (int)G, stream);
-        case CKV_BF16: return run_decode_g<__hip_bfloat16>(p, (int)G, stream);
+        case CKV_F32: return run_decode_g<float>(p, (int)G, stream, updated);
+        case CKV_F16: return run_decode_g<__half>(p, (int)G, stream, updated);
+        case CKV_BF16: return run_decode_g<__hip_bfloat16>(p, (int)G, stream, updated);
         default: return CKV_ERR_DTYPE;
     }
 }

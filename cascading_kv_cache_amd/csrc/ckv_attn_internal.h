@@ -221,6 +221,13 @@ int launch_bwd_mfma(const ckv_dense_bwd_args& a, const float* delta, const int* 
 // ---- single-token decode family (Q == 1, head_dim 128) ----
 bool decode_supported(const ckv_attn_args& a);
 int64_t decode_workspace_bytes(int64_t B, int64_t H, int64_t KVH, int64_t num_sink, int64_t S);
-int launch_decode(const ckv_attn_args& a, hipStream_t stream);
+bool update_beside_scores(const ckv_attn_args& a, const ckv_update_args& u);
+// u: the cache update that follows, checked, or null; *updated: it has been launched with the step's own kernels
+int launch_decode(const ckv_attn_args& a, hipStream_t stream, const ckv_update_args* u, bool* updated);
+
+// everything ckv_update checks before a launch (its scratch too); *empty: nothing to do
+int check_update(const ckv_update_args* args, bool* empty);
+// stages are timed one by one, or the kernels of the update: launches of several stages would blur them
+bool prof_update_apart();
 
 }  // namespace ckv

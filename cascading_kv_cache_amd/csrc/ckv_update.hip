@@ -23,7 +23,8 @@
 // Why this equals the serial loop: within one cascade the n-th insert of a call always lands in
 // ring position (start + stored + n) mod W whatever the scores are; only WHICH arrival owns a
 // slot depends on scores, and that is decided inside the group of arrivals between two inserts.
-#include "ckv_common.h"
+#include "ckv_attn_internal.h"
+#include "ckv_update_token.h"
 
 #include <type_traits>
 
@@ -543,9 +544,9 @@ __global__ void ckv_update_plan_kernel(UpdateParams p) {
 
 // The walk of a single incoming token (the decode step), by one wavefront: lane i fetches what cascade i may need (trackers,
 // period, the scores of its oldest and its newest slot) and works out where a row that comes to cascade i would land, so that
-// all cascades' loads travel together and every division is done once.  The token passes through the full cascades that
-// accept it, pushing their oldest entries on, up to the first cascade that is not full or does not accept: a count of
-// trailing ones.  Same semantics as the general kernel (cascading_cache.py:381-726 for one token).
+// all cascades' loads travel together and every division is done once (token_path).  What is left for the scores to decide is
+// whether the row that comes to the last cascade of the path displaces its newest entry.  Same semantics as the general kernel
+// (cascading_cache.py:381-726 for one token).
 struct TokenWalk {
     int count;            // slots of the chain; the token lands in the first, the old content of each in the next, the last's is dropped
     int slot;             // lane i < count: slot i of the chain
@@ -556,64 +557,32 @@ struct TokenWalk {
 };
 
 __device__ inline TokenWalk walk_token(const ckv_update_args& A, int64_t n, int64_t h, int64_t token, int lane) {
-    const int C = A.cascades;
     const int32_t W = (int32_t)A.window_size;
     const int64_t cs_base = n * A.cache_s_stride[0] + h * A.cache_s_stride[1];
-    const int64_t gidx = *A.real_token_idx + token;  // 0-based global index of the token
-    const int64_t sinks0 = A.stored_sinks[n * A.stored_sinks_stride[0] + h * A.stored_sinks_stride[1]];
+    TokenTrackers t;
+    t.request(A, n, h, token, lane);
     const float tok_score = load_as_float(A.s, n * A.s_stride[0] + h * A.s_stride[1] + token * A.s_stride[2], A.dtype);
-    TokenWalk w;
-    w.st = w.sx = w.count = 0;
-    w.slot = -1;
-    int64_t per = 1;
     float oldest = 0.f, newest = 0.f;
-    int lead = 0;
-    if (lane < C) {
-        w.st = (int32_t)A.stored_tokens[n * A.tracker_stride[0] + h * A.tracker_stride[1] + lane * A.tracker_stride[2]];
-        w.sx = (int32_t)A.start_indices[n * A.tracker_stride[0] + h * A.tracker_stride[1] + lane * A.tracker_stride[2]];
-        per = A.do_cache_every_n[lane];
-        if (w.st > 0) {
-            lead = lane * W + (w.sx > 0 && w.sx <= w.st ? w.sx - 1 : (w.sx - 1 + w.st) % w.st);
-            oldest = load_as_float(A.cache_s, cs_base + ((int64_t)lane * W + w.sx) * A.cache_s_stride[2], A.dtype);
-            newest = load_as_float(A.cache_s, cs_base + (int64_t)lead * A.cache_s_stride[2], A.dtype);
-        }
+    if (t.st > 0) {
+        oldest = load_as_float(A.cache_s, cs_base + ((int64_t)lane * W + t.sx) * A.cache_s_stride[2], A.dtype);
+        newest = load_as_float(A.cache_s, cs_base + (int64_t)token_lead(lane, W, t.st, t.sx) * A.cache_s_stride[2], A.dtype);
     }
-    w.st_new = w.st;
-    w.sx_new = w.sx;
-    w.sink = sinks0 < A.num_sink;
-    w.sinks = (int32_t)sinks0;
-    if (w.sink) {  // cascading_cache.py:399-431
-        w.count = 1;
-        w.slot = (int)(A.max_seq_len + sinks0);
-        return w;
-    }
-    const int64_t rel = gidx - A.num_sink;
-    bool on_period;
-    if (rel >= 0 && rel < (1ll << 32) && __builtin_amdgcn_ballot_w64(per <= 0 || per >= (1ll << 32)) == 0) {
-        on_period = (uint32_t)rel % (uint32_t)per == 0;
-    } else {
-        on_period = lane < C && rel % per == 0;
-    }
-    const bool takes = lane < C && ((A.eager_fill && gidx <= A.max_seq_len + A.num_sink) || on_period || w.st == 0);
-    const uint32_t ahead = (uint32_t)w.sx + (uint32_t)w.st;  // W: the ring's slots; both at most W
-    const int phys = lane * W + (int)(ahead < (uint32_t)W ? ahead : ahead < 2u * (uint32_t)W ? ahead - (uint32_t)W : ahead % (uint32_t)W);
-    const unsigned long long stays = ~__builtin_amdgcn_ballot_w64(takes && w.st >= W);
-    const int stop = stays ? __builtin_ctzll(stays) : CKV_WAVE;  // at most C: the lanes past it take nothing
-    w.count = stop;
-    if (lane < stop) {
-        w.slot = phys;
-        w.sx_new = w.sx + 1 < W ? w.sx + 1 : (w.sx + 1) % W;
-    }
-    if (stop < C) {
-        const float carried = stop == 0 ? tok_score : __shfl(oldest, stop > 0 ? stop - 1 : 0);
+    const TokenPath path = token_path(A, t, lane);
+    TokenWalk w;
+    w.st = t.st;
+    w.sx = t.sx;
+    w.st_new = path.st_new;
+    w.sx_new = path.sx_new;
+    w.sink = path.sink;
+    w.sinks = (int32_t)t.sinks;
+    w.slot = path.slot;
+    w.count = path.sink ? 1 : path.stop;
+    if (path.ends) {
+        const float carried = path.stop == 0 ? tok_score : __shfl(oldest, path.stop > 0 ? path.stop - 1 : 0);
         // an append (or the first entry of an empty cascade); else the newest slot keeps its token unless the arrival's
         // score is at least as large
-        const bool lands = takes || carried >= newest;
-        if (lane == stop && lands) {
-            w.slot = takes ? phys : lead;
-            if (takes) w.st_new = w.st + 1;
-        }
-        w.count += (int)(__builtin_amdgcn_ballot_w64(lands) >> stop & 1);
+        const bool lands = path.takes || carried >= newest;
+        w.count += (int)(__builtin_amdgcn_ballot_w64(lands) >> path.stop & 1);
     }
     return w;
 }
@@ -644,41 +613,6 @@ __global__ void __launch_bounds__(CKV_WAVE) ckv_update_plan1_kernel(UpdateParams
         p.sinks_new[u.bh] = w.sink ? (int32_t)(w.slot - A.max_seq_len) + 1 : w.sinks;
     }
     if (lane < A.cascades) p.trackers[u.bh * A.cascades + lane] = tracker_word(w.st_new, w.sx_new, (int32_t)A.window_size);
-}
-
-// What a cascade's position ids are made of, from the trackers after the call (cascading_cache.py:728-774, 129-142): slot j
-// gets ((j + seg - start) mod seg) + ub - seg, where seg is the number of stored tokens and ub the ids still to hand out (all
-// stored tokens, less a window per earlier cascade).  Lane i of a wavefront holds cascade i.
-struct PosRange {
-    bool write;     // every earlier cascade holds tokens and ids are left
-    uint32_t seg, add;
-    int32_t base;
-    __device__ int64_t id_of(uint32_t j) const {
-        uint32_t x = j + add;
-        if (x >= seg) x -= seg;
-        if (x >= seg) x %= seg;  // slots past the stored tokens of a cascade that is not full
-        return (int64_t)((int32_t)x + base);
-    }
-};
-
-__device__ inline PosRange pos_range(int lane, int C, int32_t W, int32_t st, int32_t sx) {   // by every lane: it sums over them
-    int32_t tot = C * W;   // ids are indices below max_seq_len: they fit 32 bits
-    const unsigned long long below = __builtin_amdgcn_ballot_w64(lane < C && st < W);
-    int first_empty = C;
-    if (below) {
-        tot = lane < C ? st : 0;
-#pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) tot += __shfl_xor(tot, off);
-        const unsigned long long empty = __builtin_amdgcn_ballot_w64(lane < C && st <= 0);
-        if (empty) first_empty = __builtin_ctzll(empty);
-    }
-    const int32_t ub = tot - lane * W;
-    PosRange r;
-    r.seg = (uint32_t)(st < W ? st : W);
-    r.write = lane <= first_empty && (lane == 0 || ub > 0) && r.seg != 0;
-    r.add = r.seg - (uint32_t)sx;  // start < seg or start == 0
-    r.base = ub - (int32_t)r.seg;
-    return r;
 }
 
 // Position pass after the plan kernel has updated the trackers.
@@ -1311,15 +1245,22 @@ int check_update_args(const ckv_update_args* args, bool* empty) {
 }  // namespace
 }  // namespace ckv
 
+namespace ckv {
+int check_update(const ckv_update_args* args, bool* empty) {
+    if (int rc = check_update_args(args, empty)) return rc;
+    if (*empty) return CKV_OK;
+    const ckv_update_args& A = *args;
+    const int64_t need = ckv_update_workspace_bytes(A.N, A.H, A.K, A.max_seq_len, A.cascades);
+    return !A.workspace || A.workspace_bytes < need ? CKV_ERR_WORKSPACE : CKV_OK;
+}
+}  // namespace ckv
+
 extern "C" int ckv_update(const ckv_update_args* args, void* stream_) {
     using namespace ckv;
     bool empty;
-    if (int rc = check_update_args(args, &empty)) return rc;
+    if (int rc = check_update(args, &empty)) return rc;
     if (empty) return CKV_OK;
-    const ckv_update_args& A = *args;
-    const int64_t need = ckv_update_workspace_bytes(A.N, A.H, A.K, A.max_seq_len, A.cascades);
-    if (!A.workspace || A.workspace_bytes < need) return CKV_ERR_WORKSPACE;
-    return run_update(A, A.workspace, reinterpret_cast<hipStream_t>(stream_));
+    return run_update(*args, args->workspace, reinterpret_cast<hipStream_t>(stream_));
 }
 
 extern "C" int64_t ckv_update_static_scratch_bytes(void) { return kStaticScratchBytes; }

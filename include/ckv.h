@@ -212,6 +212,12 @@ int64_t ckv_attn_workspace_bytes(int64_t B, int64_t H, int64_t KVH, int64_t Q, i
 
 int ckv_attn(const ckv_attn_args* args, void* stream);
 
+/* ckv_attn and then ckv_update: the same results, status and requirements as the two calls one behind the other
+ * (a failure of the first leaves out the second).  A single-token step whose update takes the step's own tensors
+ * (k, v, the cache and sink rows, cache_s, new_scores as s) needs launches fewer: the update then runs
+ * beside the scores. */
+int ckv_attn_update(const ckv_attn_args* args, const ckv_update_args* update, void* stream);
+
 /* ------------------------------------------------------------------------------------------
  * Dense-input attention with the signature of the reference operator
  * attention(q, k, v, causal, sm_scale, mask, beta) -> (o, scores) (flash_attention.py:543-652):

@@ -1,0 +1,68 @@
+"""A single-token step whose cache update runs beside its scores (ckv_attn_update) against the same step in two calls
+(ckv_attn, then ckv_update): outputs, new scores and every state tensor bit-identical after every token, from an empty
+cache through sinks, filling and eviction."""
+import pytest
+import torch
+
+from parity_helpers import STATE, bits
+
+pytestmark = pytest.mark.gpu
+
+
+def pair(B, KVH, NS, W, C, dtype, func, eager, reduction):
+    from cascading_kv_cache_amd.cascading_cache import CascadingKVCache
+
+    caches = [CascadingKVCache(window_length=W, num_sink_tokens=NS, max_batch_size=B, heads=KVH, dim=128, max_seq_len=W * C,
+                               device="cuda:0", dtype=dtype, cascade_func=func, eager_fill=eager, head_reduction=reduction,
+                               layers=1, verbose=False) for _ in range(2)]
+    for c in caches:
+        c.beta = 0.9   # scores that differ from slot to slot and change at every step
+    return caches
+
+
+def run_steps(one, two, B, H, KVH, dtype, tokens, gen, prompt=0):
+    from cascading_kv_cache_amd.cascade_attention import cascade_attention, default_inv_freq
+
+    inv_freq = default_inv_freq(128, 5e5, "cuda:0")
+    draw = lambda h, n: (torch.randn(B, n, h, 128, generator=gen) * 0.7).to(dtype).cuda().transpose(1, 2)   # noqa: E731
+    if prompt:
+        q, k, v = draw(H, prompt), draw(KVH, prompt), draw(KVH, prompt)
+        for c in (one, two):
+            cascade_attention(q, k, v, c, 0, inv_freq)
+    for t in range(tokens):
+        q, k, v = draw(H, 1), draw(KVH, 1), draw(KVH, 1)
+        if t % 5 == 3:
+            q = torch.zeros_like(q)   # every visible key weighs the same: ties
+        out1, new1 = cascade_attention(q, k, v, one, 0, inv_freq)
+        out2, new2 = cascade_attention(q, k, v, two, 0, inv_freq, update_cache=False)
+        two.update_state(k, v, 0, new2)
+        torch.cuda.synchronize()
+        assert torch.equal(bits(out1), bits(out2)) and torch.equal(bits(new1), bits(new2)), t
+        for name in STATE:
+            assert torch.equal(bits(getattr(one, name)[0]), bits(getattr(two, name)[0])), (t, name)
+        assert torch.equal(one.seen_tokens_by_layer, two.seen_tokens_by_layer) and one._seen_host == two._seen_host
+
+
+# windows of one slot, odd ones (position ids one by one), one cascade, as many as a workgroup takes and one more (two calls
+# inside), schedules whose periods do not divide each other, more (batch, kv head) pairs than the planning workgroups take
+@pytest.mark.parametrize("B,H,KVH,NS,W,C,dtype,func,eager,reduction,tokens", [
+    (1, 8, 2, 4, 3, 5, torch.bfloat16, "pow2", True, "mean", 60),
+    (2, 4, 4, 1, 4, 4, torch.float16, "pow2", False, "max", 60),
+    (1, 14, 2, 0, 2, 6, torch.bfloat16, "iplus1", True, "median", 60),
+    (3, 8, 1, 2, 1, 7, torch.float16, "1-then-2", True, "mean", 40),
+    (1, 2, 1, 4, 16, 1, torch.bfloat16, "pow2", True, "max", 40),
+    (1, 4, 2, 4, 2, 31, torch.bfloat16, "pow2-1", True, "median", 110),
+    (1, 4, 2, 4, 2, 32, torch.bfloat16, "pow2-1", False, "mean", 40),
+    (33, 8, 8, 3, 4, 3, torch.bfloat16, "pow2-2-4", True, "mean", 24),
+])
+def test_update_beside_the_scores_equals_two_calls(B, H, KVH, NS, W, C, dtype, func, eager, reduction, tokens):
+    one, two = pair(B, KVH, NS, W, C, dtype, func, eager, reduction)
+    run_steps(one, two, B, H, KVH, dtype, tokens, torch.Generator().manual_seed(tokens + C), 0)
+
+
+# several workgroups of scores and position ids per (batch, kv head), and the step in separate launches (its workgroups past
+# eight a compute unit)
+@pytest.mark.parametrize("B,H,KVH,NS,W,C,prompt", [(2, 8, 2, 4, 1500, 3, 4800), (1, 28, 4, 64, 4096, 2, 8600), (40, 8, 8, 4, 8192, 2, 300)])
+def test_update_beside_the_scores_of_many_slots(B, H, KVH, NS, W, C, prompt):
+    one, two = pair(B, KVH, NS, W, C, torch.bfloat16, "pow2", True, "mean")
+    run_steps(one, two, B, H, KVH, torch.bfloat16, 6, torch.Generator().manual_seed(5), prompt)
