@@ -328,7 +328,9 @@ class CascadingKVCache:
         return self.num_sink_tokens if self._seen_host[layer_idx] > self.num_sink_tokens else 0
 
     def get_vals(self, layer_idx: int):
-        pos_shift = self.pos_shift(layer_idx)
+        return self._vals(layer_idx, self.pos[layer_idx][:1, 0] + self.pos_shift(layer_idx))
+
+    def _vals(self, layer_idx: int, pos_row: Tensor):
         return (
             self.sink_keys[layer_idx],
             self.sink_values[layer_idx],
@@ -336,7 +338,7 @@ class CascadingKVCache:
             self.sink_mask[layer_idx],
             self.key_cache[layer_idx],
             self.value_cache[layer_idx],
-            self.pos[layer_idx][:1, 0] + pos_shift,
+            pos_row,
             self.mask[layer_idx],
             self.og_pos[layer_idx],
         )
@@ -354,8 +356,14 @@ class CascadingKVCache:
 
     def update(self, key_states: Tensor, value_states: Tensor, layer_idx: int, score_states: Tensor = None):
         """cascading_cache.py:1297-1348."""
-        self.update_state(key_states, value_states, layer_idx, score_states)
-        return self.get_vals(layer_idx)
+        if key_states.shape[-2] == 0:
+            self.update_state(key_states, value_states, layer_idx, score_states)
+            return self.get_vals(layer_idx)
+        _require_device(key_states, "k")
+        # the shifted position row of get_vals comes from the launch that writes the ids
+        row = torch.empty((1, self.max_seq_len[layer_idx]), dtype=torch.long, device=key_states.device)
+        self.update_state(key_states, value_states, layer_idx, score_states, _row=row)
+        return self._vals(layer_idx, row)
 
     def _update_args(self, key_states: Tensor, value_states: Tensor, score_states: Tensor, L: int):
         """The ``ckv_update`` argument block for these inputs: described once per layer, input layout and
@@ -384,14 +392,14 @@ class CascadingKVCache:
         return a
 
     def update_state(self, key_states: Tensor, value_states: Tensor, layer_idx: int, score_states: Tensor = None,
-                     _stream: Optional[int] = None, _device_counter: bool = False, _args=None):
+                     _stream: Optional[int] = None, _device_counter: bool = False, _args=None, _row: Optional[Tensor] = None):
         """``update`` without building the tuple of views it returns (the shifted position row of
         ``get_vals`` is a device operation of its own); for callers that read the state in place.
 
         The argument block of ``ckv_update`` is described once per layer and input layout and reused:
         between two calls of the same shape only the three input pointers change (single-token steps
         at batch 1 are bound by this host code, not by the device).  ``_stream``: raw stream handle when
-        the caller already holds the device context.  ``_args``: the argument block that ``_update_args`` gave for
+        the caller already holds the device context.  ``_row``: takes the position row of ``get_vals``.  ``_args``: the argument block that ``_update_args`` gave for
         these layouts, when the caller has looked up by layouts and placements that determine it.
 
         The update reads the number of tokens seen so far from device memory (``real_token_idx``).  The host knows
@@ -415,7 +423,11 @@ class CascadingKVCache:
                 stream = raw_stream(key_states.device)
                 ws = workspace(key_states.device, a._need, stream)
                 a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
-                _abi.check(_abi.lib().ckv_update(C.byref(a), C.c_void_p(stream)), "ckv_update")
+                if _row is None:
+                    _abi.check(_abi.lib().ckv_update(C.byref(a), C.c_void_p(stream)), "ckv_update")
+                else:
+                    shift = self.num_sink_tokens if self._seen_host[layer_idx] + n_new > self.num_sink_tokens else 0
+                    _abi.check(_abi.lib().ckv_update_row(C.byref(a), _row.data_ptr(), shift, C.c_void_p(stream)), "ckv_update")
         else:
             ws = workspace(key_states.device, a._need, _stream)
             a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()

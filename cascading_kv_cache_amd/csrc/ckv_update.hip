@@ -51,6 +51,8 @@ struct UpdateParams {
     int32_t* sinks_new;    // [N*H]: sinks stored after the call
     int32_t* trackers;     // [N*H][cascades]: tracker_word of every cascade
     int32_t apply_blocks;  // blocks along x that move rows; the blocks behind them write position ids
+    int64_t* row;          // [S]: the position ids of unit 0 after the call, each with row_shift added, or null
+    int64_t row_shift;
 };
 
 // The (batch, kv head) of a workgroup: grid coordinates y and z, so that no workgroup begins with 64-bit divisions (these
@@ -619,6 +621,13 @@ __global__ void __launch_bounds__(CKV_WAVE) ckv_update_plan1_kernel(UpdateParams
 // One 256-thread block per kPosChunk slots of a cascade and (batch, kv head), so the whole chip writes; the
 // blocks ride at the end of the apply kernels' grid (they need the plan's trackers, not the moved rows).
 constexpr int kPosChunk = 2048;
+
+// Slots j0, j0 + step, .. < end of a cascade in the shifted row that the caller asked for: the ids that the call writes, or those
+// that stay.  In the launch that writes the ids (an add kernel over the finished row took 4 us).
+__device__ inline void position_row(const UpdateParams& p, const PosRange& range, const int64_t* pos, int64_t* row, int j0, int end, int step) {
+    for (int j = j0; j < end; j += step) row[j] = (range.write ? range.id_of((uint32_t)j) : pos[(int64_t)j * p.a.pos_stride[2]]) + p.row_shift;
+}
+
 __device__ inline void update_positions_block(const UpdateParams& p, const Unit& u, int blk) {
     const ckv_update_args& A = p.a;
     const int64_t n = u.n, h = u.h;
@@ -635,15 +644,16 @@ __device__ inline void update_positions_block(const UpdateParams& p, const Unit&
         st = word >= 0 ? W : -1 - word;
         sx = word >= 0 ? word : (int32_t)start;
     }
-    if (!wanted) return;
+    int64_t* pos = A.pos + n * A.pos_stride[0] + h * A.pos_stride[1] + (int64_t)i * W * A.pos_stride[2];
+    int64_t* row = p.row && u.bh == 0 ? p.row + (int64_t)i * W : nullptr;
     PosRange range = pos_range(lane, C, W, st, sx);
     auto of = [&](int v) -> int { return __builtin_amdgcn_readlane(v, i); };
-    range.write = of((int)range.write) != 0;
+    range.write = wanted && of((int)range.write) != 0;
     range.seg = (uint32_t)of((int)range.seg);
     range.add = (uint32_t)of((int)range.add);
     range.base = of(range.base);
+    if (row) position_row(p, range, pos, row, j0 + tid, j0 + kPosChunk < W ? j0 + kPosChunk : W, 256);
     if (!range.write) return;
-    int64_t* pos = A.pos + n * A.pos_stride[0] + h * A.pos_stride[1] + (int64_t)i * W * A.pos_stride[2];
     if (A.pos_stride[2] == 1 && (reinterpret_cast<uintptr_t>(pos) & 15u) == 0 && (W & 1) == 0) {
 #pragma unroll
         for (int it = 0; it < kPosChunk / 512; it++) {
@@ -911,6 +921,14 @@ __global__ void __launch_bounds__(kOneThreads) ckv_update_one_kernel(UpdateParam
         }
     }
     // ---- position ids: they need the plan alone, so their stores go out while the displaced rows are on their way
+    if (p.row && u.bh == 0) {
+        for (int i = 0; i < C; i++) {
+            PosRange range = sh_range[i];
+            range.write = range.write && do_pos;
+            const int64_t* pos = A.pos + n * A.pos_stride[0] + h * A.pos_stride[1] + (int64_t)i * W * A.pos_stride[2];
+            position_row(p, range, pos, p.row + (int64_t)i * W, tid, (int)W, kOneThreads);
+        }
+    }
     if (do_pos) {
         int64_t* pos = A.pos + n * A.pos_stride[0] + h * A.pos_stride[1];
         if (A.pos_stride[2] == 1 && (reinterpret_cast<uintptr_t>(pos) & 15u) == 0 && (W & 1) == 0) {
@@ -1118,7 +1136,7 @@ void launch_timed(int stage, Kernel kernel, dim3 grid, dim3 block, size_t lds, h
     else hipLaunchKernelGGL(kernel, grid, block, lds, stream, p);
 }
 
-int run_update(const ckv_update_args& A, void* workspace, hipStream_t stream) {
+int run_update(const ckv_update_args& A, void* workspace, int64_t* row, int64_t row_shift, hipStream_t stream) {
     const int es = (int)elem_bytes(A.dtype);
     const bool vec = A.kv_stride[3] == 1 && A.cache_stride[3] == 1 && (A.num_sink == 0 || A.sink_stride[3] == 1) &&
                      (A.HID * es) % 16 == 0 && A.HID * es <= 16 * 64 && aligned16(A.k) && aligned16(A.v) &&
@@ -1151,6 +1169,8 @@ int run_update(const ckv_update_args& A, void* workspace, hipStream_t stream) {
     p.k_sub = 0;
     p.do_pos = 0;
     p.apply_blocks = 0;
+    p.row = row;
+    p.row_shift = row_shift;
     const unsigned H = (unsigned)A.H, N = (unsigned)A.N;
     if (A.K == 1 && vec && A.cascades <= kOneWaves && A.HID * es / 16 <= CKV_WAVE &&
         (A.N * A.H >= kOneMinUnits || (A.N * A.H >= kOneFewUnits && A.max_seq_len <= kOneMaxSlots))) {
@@ -1260,7 +1280,16 @@ extern "C" int ckv_update(const ckv_update_args* args, void* stream_) {
     bool empty;
     if (int rc = check_update(args, &empty)) return rc;
     if (empty) return CKV_OK;
-    return run_update(*args, args->workspace, reinterpret_cast<hipStream_t>(stream_));
+    return run_update(*args, args->workspace, nullptr, 0, reinterpret_cast<hipStream_t>(stream_));
+}
+
+extern "C" int ckv_update_row(const ckv_update_args* args, int64_t* row, int64_t shift, void* stream_) {
+    using namespace ckv;
+    bool empty;
+    if (int rc = check_update(args, &empty)) return rc;
+    if (!row) return CKV_ERR_NULL;
+    if (empty) return CKV_ERR_SHAPE;   // no launch that could write the row
+    return run_update(*args, args->workspace, row, shift, reinterpret_cast<hipStream_t>(stream_));
 }
 
 extern "C" int64_t ckv_update_static_scratch_bytes(void) { return kStaticScratchBytes; }
@@ -1276,5 +1305,5 @@ extern "C" int ckv_update_static(const ckv_update_args* args, void* stream_) {
     if (int rc = static_scratch(&ws)) return rc;
     // Nothing in the scratch has to start at zero: the plan kernel writes every chain entry and flag the
     // apply kernel reads, whatever the last call left there.
-    return run_update(A, ws, reinterpret_cast<hipStream_t>(stream_));
+    return run_update(A, ws, nullptr, 0, reinterpret_cast<hipStream_t>(stream_));
 }

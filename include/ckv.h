@@ -124,6 +124,11 @@ int64_t ckv_update_workspace_bytes(int64_t N, int64_t H, int64_t K, int64_t max_
  * adds K to its token counter afterwards (cascading_cache.py:1346). */
 int ckv_update(const ckv_update_args* args, void* stream);
 
+/* ckv_update of at least one token that also leaves the position ids of (batch 0, kv head 0) after the call, each with
+ * `shift` added, in `row` (max_seq_len contiguous int64, apart from every tensor of the call): what get_vals hands out
+ * (cascading_cache.py:1278-1295). */
+int ckv_update_row(const ckv_update_args* args, int64_t* row, int64_t shift, void* stream);
+
 /* ckv_update for callers that cannot allocate: code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc.  No counterpart in the reference.  Same arguments, same kernels and
  * same results as ckv_update, except that `workspace` / `workspace_bytes` are ignored: the scratch is a

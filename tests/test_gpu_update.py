@@ -247,3 +247,20 @@ def test_token_counter_by_table_and_by_device_counter():
     feed(2)
     assert gpu._seen_pending == [2]
     assert_same_state(gpu, cpu, "back on the table")
+
+
+@pytest.mark.parametrize("B,H,D,NS,W,C,dtype,func,eager", [
+    (1, 2, 16, 4, 3, 5, torch.bfloat16, "pow2", True),      # odd windows; a call of two tokens: the cascades' own blocks
+    (2, 16, 128, 5, 4, 4, torch.float16, "iplus1", False),  # single tokens by one launch; ids that only some cascades get
+    (1, 3, 9, 0, 2, 3, torch.float32, "pow2", True),        # rows moved element by element, no sinks
+    (1, 8, 64, 64, 4096, 2, torch.bfloat16, "pow2", True),  # several blocks of ids a cascade; the first call ends in the sinks
+])
+def test_update_returns_the_shifted_position_row(B, H, D, NS, W, C, dtype, func, eager):
+    gpu, _ = make_pair(B, H, D, NS, W, C, dtype, func, eager)
+    gen = torch.Generator().manual_seed(W)
+    for n in [1, 2, 1, 0, 3, 1, 7, 1, 1, min(W * C, 4000), 1, 2]:
+        k, v = ((torch.randn(B, H, n, D, generator=gen)).to(dtype).cuda() for _ in range(2))
+        row = gpu.update(k, v, 0, torch.rand(B, H, n, generator=gen).to(dtype).cuda())[6]
+        want = gpu.get_vals(0)[6]
+        assert row.shape == want.shape and row.dtype == want.dtype and torch.equal(row, want), n
+        assert row.data_ptr() != gpu.pos[0].data_ptr()
