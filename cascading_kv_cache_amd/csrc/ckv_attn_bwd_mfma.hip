@@ -126,7 +126,9 @@ struct BwdMfmaParams {
     const int* n_visible;
     float* part_dq;      // dq in shares of the keys, see dq_splits; null with one share
     int n_split;
-    int per_head;        // workgroups of a (batch, head); > 0: 1-D grid, see unit_of
+    int dq_per_head, dkdv_per_head;        // workgroups of a (batch, head)
+    int dq_by_xcd, dkdv_by_xcd;            // see unit_of
+    int dkdv_blocks;     // of a launch of both: the workgroups behind them do dq
 };
 
 // Workgroup ids go round the 8 XCDs, each with an L2 of its own.  With 8 | B * H all workgroups of a head can run on one
@@ -138,10 +140,9 @@ struct Unit {
     int x;          // workgroup of the head
     int64_t bh;
 };
-__device__ inline Unit unit_of(const BwdMfmaParams& p) {
-    if (p.per_head == 0) return Unit{(int)blockIdx.x, (int64_t)blockIdx.y};
-    const int j = (int)blockIdx.x >> 3;
-    return Unit{j % p.per_head, (int64_t)((int)blockIdx.x & 7) + 8 * (j / p.per_head)};
+__device__ inline Unit unit_of(int id, int per_head, bool by_xcd) {   // id: workgroup of the tensor
+    const int j = by_xcd ? id >> 3 : id;
+    return Unit{j % per_head, by_xcd ? (int64_t)(id & 7) + 8 * (j / per_head) : (int64_t)(j / per_head)};
 }
 
 // 128 dims: a row is all 64 banks, so 16 consecutive rows need 16 different slots for one piece, and the four rows of a
@@ -401,21 +402,18 @@ __device__ inline float keep_if_bit(float v, uint32_t word, int bit) {
 // dq
 // ---------------------------------------------------------------------------------------------
 template <typename T, int kHD, bool kWide, int kWaves>
-__global__ void __launch_bounds__(Team<kWaves>::kThreads, Team<kWaves>::kPerCu) bwd_mfma_dq_kernel(BwdMfmaParams p) {
+__device__ __forceinline__ void dq_workgroup(const BwdMfmaParams& p, const Unit& unit, unsigned char* const smem) {   // dq_lds of it
     constexpr int kOwn = Team<kWaves>::kOwn, kSub = Team<kWaves>::kSub, kRows = Team<kWaves>::kRows, kDqStages = Team<kWaves>::kStages;
     constexpr int kBlkBytes = Geo<kHD>::kTile, kTile = kSub * kBlkBytes, kStage = 2 * kTile;   // K, V
     constexpr int kCopies = 2 * (kHD / 64);                      // of a wavefront and stage
     constexpr int kMine = kRows / kWaves;                        // rows of a stage that a wavefront copies
     typedef Halves<T, kHD> Half;                                 // of K: two tiles per stage
     constexpr uint32_t kHalves = kDqStages * kStage, kRowNumbers = kHalves + (Half::kSplit ? kDqStages * 2 * kTile : 0);
-    extern __shared__ __attribute__((aligned(16))) unsigned char dyn_smem[];   // dq_lds of them
-    unsigned char* const smem = dyn_smem;
     const ckv_dense_bwd_args& a = p.a;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / CKV_WAVE), lane = tid % CKV_WAVE, h = lane >> 5;
     const Keys keys(p);
     const int64_t n_ctx = a.n_ctx;
     const int n_cached = (int)keys.n_cached, n_seen = (int)keys.n_seen;   // below 2^31, see bwd_mfma_supported
-    const Unit unit = unit_of(p);
     const int64_t bh = unit.bh, b = bh / a.H, hd = bh % a.H;
     const int share = unit.x % p.n_split;
     const int m_wg = unit.x / p.n_split * kOwn;
@@ -653,6 +651,12 @@ __global__ void __launch_bounds__(Team<kWaves>::kThreads, Team<kWaves>::kPerCu) 
     }
 }
 
+template <typename T, int kHD, bool kWide, int kWaves>
+__global__ void __launch_bounds__(Team<kWaves>::kThreads, Team<kWaves>::kPerCu) bwd_mfma_dq_kernel(BwdMfmaParams p) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char dyn_smem[];
+    dq_workgroup<T, kHD, kWide, kWaves>(p, unit_of((int)blockIdx.x, p.dq_per_head, p.dq_by_xcd), dyn_smem);
+}
+
 // the shares of dq added up in order and rounded once; a thread takes four dims of a row
 template <typename T, int kHD>
 __global__ void __launch_bounds__(kThreads) bwd_dq_sum_kernel(BwdMfmaParams p) {
@@ -675,11 +679,10 @@ __global__ void __launch_bounds__(kThreads) bwd_dq_sum_kernel(BwdMfmaParams p) {
 // dk, dv
 // ---------------------------------------------------------------------------------------------
 template <typename T, int kHD>
-__global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dkdv_kernel(BwdMfmaParams p) {
+__device__ __forceinline__ void dkdv_workgroup(const BwdMfmaParams& p, const Unit& unit, unsigned char* const dyn_smem) {   // kDkdvLds of it
     typedef Halves<T, kHD> Half;   // of Q and dO
     typedef Geo<kHD, Half::kSplit> G;
     constexpr int kTile = G::kTile;
-    extern __shared__ __attribute__((aligned(16))) unsigned char dyn_smem[];
     typedef float (*RowPtr)[2][kBlk];
     RowPtr rowv = reinterpret_cast<RowPtr>(dyn_smem + G::kDkdvRowv);                        // [stage][-lse log2 e, -delta]
     int* odd_rows = reinterpret_cast<int*>(dyn_smem + G::kDkdvOdd);               // [stage] some row's delta is not finite
@@ -689,7 +692,6 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dkdv_kernel(BwdMfmaParam
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / CKV_WAVE), lane = tid % CKV_WAVE, h = lane >> 5;
     const Keys keys(p);
     const int n_ctx = (int)a.n_ctx, n_cached = (int)keys.n_cached;   // below 2^31, see bwd_mfma_supported
-    const Unit unit = unit_of(p);
     const int64_t bh = unit.bh, b = bh / a.H, hd = bh % a.H;
     const int n_wg = unit.x * kOwn;
     const int n_lane = n_wg + wave * 32 + (lane & 31);  // this lane's key
@@ -969,6 +971,21 @@ __global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dkdv_kernel(BwdMfmaParam
     store(dv, a.dv);
 }
 
+template <typename T, int kHD>
+__global__ void __launch_bounds__(kThreads, 2) bwd_mfma_dkdv_kernel(BwdMfmaParams p) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char dyn_smem[];
+    dkdv_workgroup<T, kHD>(p, unit_of((int)blockIdx.x, p.dkdv_per_head, p.dkdv_by_xcd), dyn_smem);
+}
+
+// dk / dv and dq in one launch, the longer workgroups first.
+template <typename T, int kHD>
+__global__ void __launch_bounds__(kThreads, 2) bwd_mfma_both_kernel(BwdMfmaParams p) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char dyn_smem[];
+    const int id = (int)blockIdx.x - p.dkdv_blocks;
+    if (id < 0) dkdv_workgroup<T, kHD>(p, unit_of((int)blockIdx.x, p.dkdv_per_head, p.dkdv_by_xcd), dyn_smem);
+    else dq_workgroup<T, kHD, false, kWaves>(p, unit_of(id, p.dq_per_head, p.dq_by_xcd), dyn_smem);
+}
+
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 // unit stride along the head dim, 16-byte addressable rows, and 32 rows apart still within a 32-bit byte offset
 inline bool rows_ok(const int64_t* st) {
@@ -999,45 +1016,74 @@ inline bool wide_dq(int64_t n_ctx, int64_t units, int64_t cus) {
     return 2 * wide == narrow && wide * units <= cus && narrow * units > cus;
 }
 
+// dk / dv and dq in one launch (dq by workgroups of four wavefronts) while the workgroups of dk / dv are few: one launch after the other
+// leaves units idle at the end of each, and with fewer workgroups than places half of every unit throughout.  Time of one launch over
+// that of two (and of wide dq where wide_dq takes it), by the number of dk / dv's workgroups, heads x rows x cached keys, 128 dims bf16 / 64
+// dims f16:
+//   4 (2 x 64 x 128)  0.55 / 0.59        272 (2 x 1024 x 16384)  0.69 / 0.67       320 (8 x 1000 x 4095, a quarter masked)  0.81 / 0.76
+//   576 (8 x 1024 x 8192)  0.92 / 0.93   640 (16 x 1024 x 4096)  0.88 / 0.92       768 (32 x 1024 x 2048)  0.91 / 0.92
+//   1216 (64 x 300 x 2048)  0.93 / 0.93  1280 (32 x 1024 x 4096, half masked)  0.99 / 0.97
+//   1536 (64 x 1024 x 2048)  1.02 / 0.99   4352 (32 x 1024 x 16384)  1.10 / 1.08   8256 (64 x 100 x 16384)  1.06 / 1.04
+// (8 heads x 1000 rows x 5095 keys of 64 dims in float16: 123.8 -> 94.1 us.)  Many rounds of dk / dv run better by themselves.
+inline bool both_at_once(int64_t dkdv_blocks, int64_t cus) { return dkdv_blocks <= 5 * cus; }
+
 template <typename T, int kHD>
 int run(const BwdMfmaParams& p_in, hipStream_t stream) {
     BwdMfmaParams p = p_in;
     const ckv_dense_bwd_args& a = p.a;
-    auto grid_of = [&](int64_t per_head, int64_t most) {
-        const int64_t heads = a.B * a.H;
-        const bool by_xcd = heads % 8 == 0 && heads * per_head <= most;
-        p.per_head = by_xcd ? (int)per_head : 0;
-        return by_xcd ? dim3((unsigned)(heads * per_head)) : dim3((unsigned)per_head, (unsigned)heads);
+    const int64_t heads = a.B * a.H, cus = mfma_device_cus();
+    auto by_xcd = [&](int64_t blocks, int64_t most) { return heads % 8 == 0 && blocks <= most ? 1 : 0; };
+    const int64_t dkdv_blocks = (a.n_kv + kOwn - 1) / kOwn * heads;
+    p.dkdv_per_head = (int)((a.n_kv + kOwn - 1) / kOwn);
+    p.dkdv_by_xcd = by_xcd(dkdv_blocks, 2 * cus);
+    p.dkdv_blocks = (int)dkdv_blocks;
+    constexpr int kDkdvLds = Geo<kHD, Halves<T, kHD>::kSplit>::kDkdvLds;
+    auto dq_blocks = [&](int own) -> int64_t {
+        p.dq_per_head = (int)((a.n_ctx + own - 1) / own * p.n_split);
+        p.dq_by_xcd = heads % 8 == 0;
+        return heads * p.dq_per_head;
     };
+    if (dkdv_blocks > 0x3fffffff || (a.n_ctx + kOwn - 1) / kOwn * p.n_split * heads > 0x3fffffff) return CKV_ERR_UNSUPPORTED;
     auto launch_dq = [&](auto waves_tag, auto wide_rows_tag) -> int {
-        constexpr int kWaves = decltype(waves_tag)::value, kOwn = Team<kWaves>::kOwn;
+        constexpr int kWaves = decltype(waves_tag)::value;
         constexpr int kLds = dq_lds<T, kHD, kWaves>();
         auto* kernel = bwd_mfma_dq_kernel<T, kHD, decltype(wide_rows_tag)::value, kWaves>;
         if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(kernel), kLds)) return rc;
-        const dim3 grid = grid_of((a.n_ctx + kOwn - 1) / kOwn * p.n_split, 0x7fffffff);
-        hipLaunchKernelGGL(kernel, grid, dim3(Team<kWaves>::kThreads), kLds, stream, p);
+        const int64_t blocks = dq_blocks(Team<kWaves>::kOwn);
+        hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(Team<kWaves>::kThreads), kLds, stream, p);
         CKV_HIP_TRY(hipGetLastError());
+        return CKV_OK;
+    };
+    auto sum_shares = [&]() -> int {
+        if (p.n_split > 1) {
+            const int64_t threads = heads * a.n_ctx * (kHD / 4);
+            hipLaunchKernelGGL((bwd_dq_sum_kernel<T, kHD>), dim3((unsigned)((threads + kThreads - 1) / kThreads)), dim3(kThreads), 0,
+                               stream, p);
+            CKV_HIP_TRY(hipGetLastError());
+        }
         return CKV_OK;
     };
     constexpr std::integral_constant<int, 4> narrow{};
     constexpr std::integral_constant<int, 8> wide{};
-    if (a.n_kv * a.kv_stride[2] * 2 >= (int64_t)1 << 32) {
+    const bool far_rows = a.n_kv * a.kv_stride[2] * 2 >= (int64_t)1 << 32;
+    if (!far_rows && both_at_once(dkdv_blocks, cus)) {
+        constexpr int kLds = kDkdvLds > dq_lds<T, kHD, kWaves>() ? kDkdvLds : dq_lds<T, kHD, kWaves>();
+        if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(bwd_mfma_both_kernel<T, kHD>), kLds)) return rc;
+        const int64_t blocks = dkdv_blocks + dq_blocks(kOwn);
+        hipLaunchKernelGGL((bwd_mfma_both_kernel<T, kHD>), dim3((unsigned)blocks), dim3(kThreads), kLds, stream, p);
+        CKV_HIP_TRY(hipGetLastError());
+        return sum_shares();
+    }
+    if (far_rows) {
         if (int rc = launch_dq(narrow, std::true_type{})) return rc;
-    } else if (wide_dq(a.n_ctx, a.B * a.H * p.n_split, mfma_device_cus())) {
+    } else if (wide_dq(a.n_ctx, heads * p.n_split, cus)) {
         if (int rc = launch_dq(wide, std::false_type{})) return rc;
     } else if (int rc = launch_dq(narrow, std::false_type{})) {
         return rc;
     }
-    if (p.n_split > 1) {
-        const int64_t threads = a.B * a.H * a.n_ctx * (kHD / 4);
-        hipLaunchKernelGGL((bwd_dq_sum_kernel<T, kHD>), dim3((unsigned)((threads + kThreads - 1) / kThreads)), dim3(kThreads), 0,
-                           stream, p);
-        CKV_HIP_TRY(hipGetLastError());
-    }
-    constexpr int kDkdvLds = Geo<kHD, Halves<T, kHD>::kSplit>::kDkdvLds;
+    if (int rc = sum_shares()) return rc;
     if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(bwd_mfma_dkdv_kernel<T, kHD>), kDkdvLds)) return rc;
-    const dim3 grid_dkdv = grid_of((a.n_kv + kOwn - 1) / kOwn, 2 * (int64_t)mfma_device_cus());
-    hipLaunchKernelGGL((bwd_mfma_dkdv_kernel<T, kHD>), grid_dkdv, dim3(kThreads), kDkdvLds, stream, p);
+    hipLaunchKernelGGL((bwd_mfma_dkdv_kernel<T, kHD>), dim3((unsigned)dkdv_blocks), dim3(kThreads), kDkdvLds, stream, p);
     CKV_HIP_TRY(hipGetLastError());
     return CKV_OK;
 }
@@ -1073,7 +1119,8 @@ int bwd_mfma_dq_splits(int64_t B, int64_t H, int64_t n_ctx, int64_t n_kv, int cu
 int launch_bwd_mfma(const ckv_dense_bwd_args& a, const float* delta, const int* key_order, const int* n_visible, float* part_dq,
                     int n_split, hipStream_t stream) {
     BwdMfmaParams p;
-    p.per_head = 0;
+    p.dq_per_head = p.dkdv_per_head = p.dkdv_blocks = 1;
+    p.dq_by_xcd = p.dkdv_by_xcd = 0;
     p.part_dq = part_dq;
     p.n_split = part_dq ? n_split : 1;
     p.a = a;
@@ -1086,7 +1133,11 @@ int launch_bwd_mfma(const ckv_dense_bwd_args& a, const float* delta, const int* 
 
 }  // namespace ckv
 
-// wavefronts of dq's workgroups for rows addressed in 32 bits (cus 0: the current device's), for tests that aim at one kernel
+// For tests that aim at one kernel (cus 0: the current device's): are dk / dv and dq one launch; where not, and for rows
+// addressed in 32 bits, the wavefronts of dq's workgroups
+extern "C" int ckv_dense_bwd_one_launch(int64_t n_kv, int64_t heads, int64_t cus) {
+    return ckv::both_at_once((n_kv + ckv::kOwn - 1) / ckv::kOwn * heads, cus > 0 ? cus : ckv::mfma_device_cus());
+}
 extern "C" int ckv_dense_bwd_dq_wavefronts(int64_t n_ctx, int64_t units, int64_t cus) {
     return ckv::wide_dq(n_ctx, units, cus > 0 ? cus : ckv::mfma_device_cus()) ? 8 : 4;
 }

@@ -143,3 +143,10 @@ def dq_wavefronts(Z, H, n_ctx, n_kv, D, dtype, shared=True):
     shares = max(1, size // (Z * H * n_ctx * D * 4))
     rule = ctypes.CDLL(_abi.LIB_PATH).ckv_dense_bwd_dq_wavefronts
     return rule(ctypes.c_int64(n_ctx), ctypes.c_int64(Z * H * shares), ctypes.c_int64(0))
+
+
+def backward_in_one_launch(Z, H, n_kv):
+    """whether dk, dv and dq of the dense operator share a launch on this device (dq in workgroups of four wavefronts)"""
+    from cascading_kv_cache_amd import _abi
+
+    return bool(ctypes.CDLL(_abi.LIB_PATH).ckv_dense_bwd_one_launch(ctypes.c_int64(n_kv), ctypes.c_int64(Z * H), ctypes.c_int64(0)))

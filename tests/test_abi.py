@@ -312,3 +312,9 @@ def test_dq_by_eight_wavefronts_where_all_run_at_once(lib, n_ctx, units, wavefro
     """The dense operator's dq on 256 compute units: workgroups of eight wavefronts where each has a unit of its own and those
     of four would share them.  With a round and a bit of them (65 heads of 1000 rows) the kernel took a third longer."""
     assert C.CDLL(_abi.LIB_PATH).ckv_dense_bwd_dq_wavefronts(C.c_int64(n_ctx), C.c_int64(units), C.c_int64(256)) == wavefronts
+
+
+@pytest.mark.parametrize("n_kv,heads,one", [(1, 1, 1), (128 * 20, 64, 1), (128 * 20 + 1, 64, 0), (128 * 1280, 1, 1), (128 * 1280 + 1, 1, 0)])
+def test_backward_in_one_launch_up_to_five_workgroups_a_unit(lib, n_kv, heads, one):
+    """The dense operator's dk, dv and dq on 256 compute units: one launch up to 1280 workgroups of 128 keys."""
+    assert C.CDLL(_abi.LIB_PATH).ckv_dense_bwd_one_launch(C.c_int64(n_kv), C.c_int64(heads), C.c_int64(256)) == one

@@ -16,7 +16,7 @@ from oracle.update import OracleCache
 pytestmark = pytest.mark.gpu
 
 from parity_helpers import (META, STATE, FlipLedger, assert_scores_close, check_update_against_replay, clone_oracle,
-                            dq_wavefronts, flip_bound, flip_margins, push_state, tol)
+                            backward_in_one_launch, dq_wavefronts, flip_bound, flip_margins, push_state, tol)
 
 
 def make_pair(B, KVH, D, NS, W, C, dtype, func="pow2", eager=True, reduction="mean"):
@@ -530,8 +530,10 @@ def test_backward_on_the_matrix_cores(Z, H, N_CTX, N_KV, masking, layout, dtype)
     check_backward_against_autograd(q, k, v, mask, dtype)
 
 
+# 1590, 761 and 2700 keys: dk and dv in a launch of their own, where the wide workgroups run (the others share it in narrow ones)
 @pytest.mark.parametrize("Z,H,N_CTX,N_KV", [(4, 64, 129, 129 + 95), (4, 64, 250, 250), (2, 32, 256, 1025 + 256), (4, 32, 400, 1190 + 400),
-                                            (1, 32, 400, 4208 + 400), (1, 24, 1000, 900 + 1000), (5, 12, 720, 720)])
+                                            (1, 32, 400, 4208 + 400), (1, 24, 1000, 900 + 1000), (5, 12, 720, 720),
+                                            (4, 64, 250, 511 + 250), (2, 32, 1000, 1700 + 1000)])
 @pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_backward_dq_by_eight_wavefronts(Z, H, N_CTX, N_KV, D, dtype):
@@ -543,6 +545,7 @@ def test_backward_dq_by_eight_wavefronts(Z, H, N_CTX, N_KV, D, dtype):
     from cascading_kv_cache_amd.flash_attention import attention
 
     assert dq_wavefronts(Z, H, N_CTX, N_KV, D, dtype) == 8
+    assert backward_in_one_launch(Z, H, N_KV) == (N_KV not in (1190 + 400, 511 + 250, 1700 + 1000))
 
     torch.manual_seed(23)
 

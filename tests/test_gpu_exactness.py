@@ -13,7 +13,7 @@ import math
 import pytest
 import torch
 
-from parity_helpers import dq_wavefronts
+from parity_helpers import backward_in_one_launch, dq_wavefronts
 
 pytestmark = pytest.mark.gpu
 
@@ -259,7 +259,9 @@ def test_dense_backward_with_less_room_than_it_could_use(Z, H, n_ctx, n_kv, mask
 @pytest.mark.parametrize("Z,H,n_ctx,n_kv,masked", [
     (2, 80, 129, 500 + 129, slice(32, 320)),   # the second workgroup's one row; whole stages and a half of hidden keys
     (1, 90, 400, 75 + 400, slice(0, 75)),      # no cached key visible; two workgroups a head, the second short of rows
-    (1, 40, 1000, 250 + 1000, None)])          # four, and a diagonal that crosses twelve stages in front of the last's
+    (1, 40, 1000, 250 + 1000, None),           # four, and a diagonal that crosses twelve stages in front of the last's
+    (2, 80, 129, 1000 + 129, slice(32, 320)),  # as the first and the second, with keys enough that dk and dv are a launch of their own
+    (1, 90, 400, 1500 + 400, slice(0, 1500))])
 def test_dense_backward_with_dq_by_eight_wavefronts(Z, H, n_ctx, n_kv, masked, room, scale, D, dtype):
     """dq's wide workgroups with the keys sorted and as they lie (masked one by one, a hidden block of 32 left out), with
     either sign of the scale."""
@@ -267,6 +269,7 @@ def test_dense_backward_with_dq_by_eight_wavefronts(Z, H, n_ctx, n_kv, masked, r
     from cascading_kv_cache_amd import flash_attention as fa
 
     assert dq_wavefronts(Z, H, n_ctx, n_kv, D, dtype, shared=room == "all") == 8
+    assert (n_kv in (1000 + 129, 1500 + 400)) == (not backward_in_one_launch(Z, H, n_kv))
     q, k, v, mask, do = dense_case(Z, H, n_ctx, n_kv, D, dtype)
     if masked is not None:
         mask[masked] = True
@@ -282,14 +285,14 @@ def test_dense_backward_with_dq_by_eight_wavefronts(Z, H, n_ctx, n_kv, masked, r
 
 
 @pytest.mark.parametrize("dtype", [BF16, F16])
-@pytest.mark.parametrize("row", [5, 299])
-def test_infinite_gradient_in_dq_by_eight_wavefronts(row, dtype):
+@pytest.mark.parametrize("row,cached", [(5, 700), (299, 700), (5, 2000), (299, 2000)])   # dk and dv beside dq, and in a launch of their own
+def test_infinite_gradient_in_dq_by_eight_wavefronts(row, cached, dtype):
     """The wavefront that holds the row takes float32 products, in both blocks of every stage: its other rows are what they
     were to a rounding, everyone else's to the bit."""
     from cascading_kv_cache_amd import flash_attention as fa
 
-    Z, H, n_ctx, n_kv = 1, 72, 400, 700 + 400
-    assert dq_wavefronts(Z, H, n_ctx, n_kv, 64, dtype) == 8
+    Z, H, n_ctx, n_kv = 1, 72, 400, cached + 400
+    assert dq_wavefronts(Z, H, n_ctx, n_kv, 64, dtype) == 8 and backward_in_one_launch(Z, H, n_kv) == (cached == 700)
     q, k, v, mask, do = dense_case(Z, H, n_ctx, n_kv, 64, dtype)
     out, _, lse, m = fa._forward(q, k, v, True, 0.5, mask, 0.9, True)
     clean = fa._backward(q, k, v, out, lse, m, do, 0.5)[0]
