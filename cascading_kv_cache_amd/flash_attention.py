@@ -17,10 +17,28 @@ import ctypes as C
 import torch
 
 from . import _abi
-from .cascading_cache import _require_device, workspace
+from .cascading_cache import _require_device, on_device, raw_stream, workspace
 
 
 MAX_BACKWARD_HEAD_DIM = 192   # ckv_attn_dense_bwd stages fp32 tiles of head_dim + 1 columns in LDS
+
+
+# Argument blocks without their pointers, and the scratch they need, by what they are made of: sizes, strides, types, the device.
+# A call takes a copy of the bytes (the backward runs on a thread of autograd's own): of the host time of a call, 100 to 190 us by
+# the speed of the core, 25 to 45 less with the missing fill of backward() below.
+_BLOCKS = {}
+
+
+def _block(struct, key, describe):
+    key = (struct,) + key
+    block = _BLOCKS.get(key)
+    if block is None:
+        a = struct()
+        need = describe(a)
+        if len(_BLOCKS) > 64:
+            _BLOCKS.clear()
+        block = _BLOCKS[key] = (bytes(a), need)
+    return struct.from_buffer_copy(block[0]), block[1]
 
 
 def _forward(q, k, v, causal, sm_scale, mask, beta, want_lse):
@@ -37,28 +55,33 @@ def _forward(q, k, v, causal, sm_scale, mask, beta, want_lse):
         if mask.dtype != torch.bool:
             mask = mask != 0
     lib = _abi.lib()
-    o = torch.empty((B, H, n_ctx, D), dtype=q.dtype, device=q.device)
-    scores = torch.empty((B, H, n_kv), dtype=q.dtype, device=q.device)
-    lse = torch.empty((B, H, n_ctx), dtype=torch.float32, device=q.device) if want_lse else None
-    a = _abi.DenseArgs()
-    a.q, a.k, a.v = q.data_ptr(), k.data_ptr(), v.data_ptr()
-    _abi.set_strides(a.q_stride, q)
-    _abi.set_strides(a.kv_stride, k)
-    a.mask = mask.data_ptr() if mask is not None and mask.numel() > 0 else None
-    a.out = o.data_ptr()
-    _abi.set_strides(a.out_stride, o)
-    a.scores = scores.data_ptr()
-    _abi.set_strides(a.scores_stride, scores)
-    a.B, a.H, a.n_ctx, a.n_kv, a.D = B, H, n_ctx, n_kv, D
-    a.scale = float(sm_scale)
-    a.beta = float(beta)
-    a.causal = int(bool(causal))
-    a.dtype = _abi.dtype_code(q.dtype)
-    a.lse = lse.data_ptr() if want_lse else None
-    with torch.cuda.device(q.device):
-        need = lib.ckv_dense_workspace_bytes(B, H, n_ctx, n_kv, D, a.dtype)
-        stream = torch.cuda.current_stream(q.device).cuda_stream
-        ws = workspace(q.device, need, stream)
+    dev = q.device
+    o = torch.empty((B, H, n_ctx, D), dtype=q.dtype, device=dev)
+    scores = torch.empty((B, H, n_kv), dtype=q.dtype, device=dev)
+    lse = torch.empty((B, H, n_ctx), dtype=torch.float32, device=dev) if want_lse else None
+
+    def describe(a):
+        _abi.set_strides(a.q_stride, q)
+        _abi.set_strides(a.kv_stride, k)
+        _abi.set_strides(a.out_stride, o)
+        _abi.set_strides(a.scores_stride, scores)
+        a.B, a.H, a.n_ctx, a.n_kv, a.D = B, H, n_ctx, n_kv, D
+        a.scale = float(sm_scale)
+        a.beta = float(beta)
+        a.causal = int(bool(causal))
+        a.dtype = _abi.dtype_code(q.dtype)
+        return lib.ckv_dense_workspace_bytes(B, H, n_ctx, n_kv, D, a.dtype)
+
+    with on_device(dev):
+        a, need = _block(_abi.DenseArgs, (q.shape, q.stride(), k.shape, k.stride(), q.dtype, dev, float(sm_scale), float(beta), bool(causal)),
+                         describe)
+        a.q, a.k, a.v = q.data_ptr(), k.data_ptr(), v.data_ptr()
+        a.mask = mask.data_ptr() if mask is not None and mask.numel() > 0 else None
+        a.out = o.data_ptr()
+        a.scores = scores.data_ptr()
+        a.lse = lse.data_ptr() if want_lse else None
+        stream = raw_stream(dev)
+        ws = workspace(dev, need, stream)
         a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
         _abi.check(lib.ckv_attn_dense(C.byref(a), C.c_void_p(stream)), "ckv_attn_dense")
     return o, scores, lse, mask
@@ -68,28 +91,32 @@ def _backward(q, k, v, o, lse, mask, do, sm_scale):
     lib = _abi.lib()
     B, H, n_ctx, D = q.shape
     n_kv = k.size(2)
-    dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(k)
-    if not _abi.same_layout(dk, dv):  # empty_like keeps the strides of its source: k and v share theirs
-        dv = torch.empty_strided(dk.shape, dk.stride(), dtype=dk.dtype, device=dk.device)
-    a = _abi.DenseBwdArgs()
-    a.q, a.k, a.v, a.out, a.lse, a.dout = (q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr(),
-                                           do.data_ptr())
-    _abi.set_strides(a.q_stride, q)
-    _abi.set_strides(a.kv_stride, k)
-    _abi.set_strides(a.out_stride, o)
-    _abi.set_strides(a.dout_stride, do)
-    a.mask = mask.data_ptr() if mask is not None and mask.numel() > 0 else None
-    a.dq, a.dk, a.dv = dq.data_ptr(), dk.data_ptr(), dv.data_ptr()
-    _abi.set_strides(a.dq_stride, dq)
-    _abi.set_strides(a.dkv_stride, dk)
-    a.B, a.H, a.n_ctx, a.n_kv, a.D = B, H, n_ctx, n_kv, D
-    a.scale = float(sm_scale)
-    a.dtype = _abi.dtype_code(q.dtype)
-    with torch.cuda.device(q.device):
+    dev = q.device
+    dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(k)   # of one layout: k and v share theirs
+
+    def describe(a):
+        _abi.set_strides(a.q_stride, q)
+        _abi.set_strides(a.kv_stride, k)
+        _abi.set_strides(a.out_stride, o)
+        _abi.set_strides(a.dout_stride, do)
+        _abi.set_strides(a.dq_stride, dq)
+        _abi.set_strides(a.dkv_stride, dk)
+        a.B, a.H, a.n_ctx, a.n_kv, a.D = B, H, n_ctx, n_kv, D
+        a.scale = float(sm_scale)
+        a.dtype = _abi.dtype_code(q.dtype)
         need = lib.ckv_dense_bwd_workspace_bytes(B, H, n_ctx) + lib.ckv_dense_bwd_key_order_bytes(n_kv)
-        need += lib.ckv_dense_bwd_split_bytes(B, H, n_ctx, n_kv, D, a.dtype)   # depends on the device's compute units
-        stream = torch.cuda.current_stream(q.device).cuda_stream
-        ws = workspace(q.device, need, stream)
+        return need + lib.ckv_dense_bwd_split_bytes(B, H, n_ctx, n_kv, D, a.dtype)   # depends on the device's compute units
+
+    with on_device(dev):
+        # the gradients' strides follow from those of q and k
+        a, need = _block(_abi.DenseBwdArgs, (q.shape, q.stride(), k.shape, k.stride(), o.stride(), do.stride(), q.dtype, dev, float(sm_scale),
+                                             dq.stride(), dk.stride()), describe)
+        a.q, a.k, a.v, a.out, a.lse, a.dout = (q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr(),
+                                               do.data_ptr())
+        a.mask = mask.data_ptr() if mask is not None and mask.numel() > 0 else None
+        a.dq, a.dk, a.dv = dq.data_ptr(), dk.data_ptr(), dv.data_ptr()
+        stream = raw_stream(dev)
+        ws = workspace(dev, need, stream)
         a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
         _abi.check(lib.ckv_attn_dense_bwd(C.byref(a), C.c_void_p(stream)), "ckv_attn_dense_bwd")
     return dq, dk, dv
@@ -113,11 +140,14 @@ class _attention(torch.autograd.Function):
                                                                                               device=q.device))
             ctx.sm_scale = sm_scale
         ctx.mark_non_differentiable(scores)
+        ctx.set_materialize_grads(False)   # else the scores' missing gradient is filled with zeros, a launch per call
         return o, scores
 
     @staticmethod
     def backward(ctx, do, d_scores):
         q, k, v, o, lse, mask = ctx.saved_tensors
+        if do is None:   # nobody asks for a gradient of o
+            return None, None, None, None, None, None, None
         if do.dtype != q.dtype:
             do = do.to(q.dtype)
         dq, dk, dv = _backward(q, k, v, o, lse, mask, do, ctx.sm_scale)

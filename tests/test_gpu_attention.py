@@ -869,3 +869,30 @@ def test_backward_of_rows_that_span_four_gibibytes(D, dtype):
         results.append((out, lse) + fa._backward(q, kk, vv, out, lse, m, do, 0.5))
     for name, a, b in zip(("out", "lse", "dq", "dk", "dv"), *results):
         assert torch.equal(a, b), name
+
+
+def test_dense_operator_does_not_mix_up_layouts():
+    """Calls that differ in one thing only (sizes, strides of an input or of the gradient, scale, beta, mask, gradients wanted or
+    not) one behind the other, against the same calls with nothing kept from a call before."""
+    from cascading_kv_cache_amd import flash_attention as fa
+
+    gen = torch.Generator().manual_seed(3)
+
+    def rows(n, apart):   # (1, 3, n, 64), heads or tokens outermost
+        t = torch.randn(1, *((n, 3, 64) if apart else (3, n, 64)), generator=gen).half().cuda()
+        return (t.transpose(1, 2) if apart else t).requires_grad_()
+
+    def call(q, k, v, scale, beta, mask, do):
+        o, s = fa.attention(q, k, v, True, scale, mask, beta)
+        return (o, s) if do is None else (o, s) + torch.autograd.grad(o, (q, k, v), do)
+
+    hidden = torch.arange(70, device="cuda") % 3 == 0
+    base = dict(q=rows(40, True), k=rows(110, True), v=rows(110, True), scale=0.5, beta=0.99, mask=hidden, do=rows(40, True).detach())
+    calls = [base, dict(base, scale=0.25), dict(base, beta=0.5), dict(base, q=rows(40, False)), dict(base, k=rows(110, False), v=rows(110, False)),
+             dict(base, do=rows(40, False).detach()), dict(base, mask=torch.zeros_like(hidden)), dict(base, do=None),
+             dict(base, q=rows(50, True), do=rows(50, True).detach(), mask=hidden[:60])]
+    kept = [call(**c) for c in calls + calls][len(calls):]
+    for c, got in zip(calls, kept):
+        fa._BLOCKS.clear()
+        for a, b in zip(got, call(**c)):
+            assert a.shape == b.shape and a.stride() == b.stride() and torch.equal(a, b)
