@@ -950,7 +950,7 @@ struct StreamRows {
     }
 };
 
-template <typename T, int G>
+template <typename T, int G, bool kPlan>
 __global__ void __launch_bounds__(kStreamThreads, kStreamWgPerCu) decode_stream_kernel(DecodeParams p) {
     extern __shared__ __align__(16) unsigned char smem[];
     const uint32_t lds_base = lds_address(smem);
@@ -1065,18 +1065,18 @@ __global__ void __launch_bounds__(kStreamThreads, kStreamWgPerCu) decode_stream_
         kvh = bh - b * KVH;
     }
     SharedQueries<T, G> shared;
-    StreamPlanner planner(p, wave);
+    StreamPlanner planner(p, kPlan ? wave : -1);
     shared.request(p, tid, wave);
-    planner.request(p, lane);
+    if constexpr (kPlan) planner.request(p, lane);
     rows.request(jt);
     rows.copy_from(jt);
     rows.arrived();
     shared.arrived();
-    planner.arrived();
+    if constexpr (kPlan) planner.arrived();
     copy_kq(b, kvh, 0);
     copy_v(b, kvh, 0);
     shared.finish(p, freqs, smem + kStreamOwnQ, tid, wave);
-    planner.work_out(p, lane);
+    if constexpr (kPlan) planner.work_out(p, lane);
     rows.take(freqs);
     bool request = (jt + 1) * nbh < item1;
     // Loads and stores retire in issue order, so "at most n operations outstanding" with n younger ones issued after the
@@ -1232,7 +1232,7 @@ __global__ void __launch_bounds__(kStreamThreads, kStreamWgPerCu) decode_stream_
         }
     }
     flush();
-    planner.store(p, lane);
+    if constexpr (kPlan) planner.store(p, lane);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1271,7 +1271,7 @@ __device__ inline void wait_vm(int n, bool lds_too) {  // s_waitcnt vmcnt(n) [lg
     }
 }
 
-template <typename T, int G>
+template <typename T, int G, bool kPlan>
 __global__ void __launch_bounds__(kStreamThreads, kStreamWgPerCu) decode_stream_wide_kernel(DecodeParams p) {
     static_assert(G > 4 && G <= 8, "the query block and the logit planes hold 8 heads");
     extern __shared__ __align__(16) unsigned char smem[];
@@ -1350,18 +1350,18 @@ __global__ void __launch_bounds__(kStreamThreads, kStreamWgPerCu) decode_stream_
         kvh = bh - b * KVH;
     }
     SharedQueries<T, G> shared;
-    StreamPlanner planner(p, wave);
+    StreamPlanner planner(p, kPlan ? wave : -1);
     shared.request(p, tid, wave);
-    planner.request(p, lane);
+    if constexpr (kPlan) planner.request(p, lane);
     rows.request(jt);
     rows.copy_from(jt);
     rows.arrived();
     shared.arrived();
-    planner.arrived();
+    if constexpr (kPlan) planner.arrived();
     copy_kq(b, kvh, 0);
     copy_v(b, kvh, 0);
     shared.finish(p, freqs, smem + kWideOwnQ, tid, wave);
-    planner.work_out(p, lane);
+    if constexpr (kPlan) planner.work_out(p, lane);
     rows.take(freqs);
     bool request = (jt + 1) * nbh < item1;
     // Per item a wavefront issues, in this order: [the query copy of the next item,] four K copies of the
@@ -1507,7 +1507,7 @@ __global__ void __launch_bounds__(kStreamThreads, kStreamWgPerCu) decode_stream_
         }
     }
     flush();
-    planner.store(p, lane);
+    if constexpr (kPlan) planner.store(p, lane);
 }
 
 // one workgroup per (b, h): 16 groups of 32 threads walk every 16th tile, eight tiles in flight, then merge
@@ -2302,10 +2302,6 @@ int run_decode(const DecodeParams& p_in, hipStream_t stream, bool* updated) {
             // streaming kernel: as many workgroups as run at once, items dealt out evenly
             if constexpr (G <= 8) {
                 constexpr int lds_s = G <= 4 ? kStreamLds : kWideLds;
-                const void* kernel;
-                if constexpr (G <= 4) kernel = reinterpret_cast<const void*>(decode_stream_kernel<T, G>);
-                else kernel = reinterpret_cast<const void*>(decode_stream_wide_kernel<T, G>);
-                if (int rc = ensure_dynamic_lds(kernel, lds_s)) return rc;
                 DeviceInfo di;
                 if (int rc = current_device_info(&di)) return rc;
                 int64_t wgs = (di.cus > 0 ? di.cus : 256) * kStreamWgPerCu;
@@ -2317,20 +2313,16 @@ int run_decode(const DecodeParams& p_in, hipStream_t stream, bool* updated) {
                 if (finish_blocks == 0 || nbh > wgs) p.plans = nullptr;
                 hipEvent_t ev0, ev1;
                 prof_kernel_events(CKV_STAGE_DECODE, &ev0, &ev1);
-                if constexpr (G <= 4) {
-                    if (ev0)
-                        hipExtLaunchKernelGGL((decode_stream_kernel<T, G>), dim3((unsigned)wgs), dim3(kStreamThreads),
-                                              (uint32_t)lds_s, stream, ev0, ev1, 0u, p);
-                    else
-                        hipLaunchKernelGGL((decode_stream_kernel<T, G>), dim3((unsigned)wgs), dim3(kStreamThreads), lds_s, stream, p);
-                } else {
-                    if (ev0)
-                        hipExtLaunchKernelGGL((decode_stream_wide_kernel<T, G>), dim3((unsigned)wgs), dim3(kStreamThreads),
-                                              (uint32_t)lds_s, stream, ev0, ev1, 0u, p);
-                    else
-                        hipLaunchKernelGGL((decode_stream_wide_kernel<T, G>), dim3((unsigned)wgs), dim3(kStreamThreads), lds_s,
-                                           stream, p);
-                }
+                // The planning wavefront is compiled in only where the step has a plan: skipped by a branch, it still cost the large
+                // launches, which have none, 1.3 % (16 streams x 32 K slots 386.4 -> 391.5 us, the step 412.7 -> 418.2).
+                void (*kernel)(DecodeParams);
+                if constexpr (G <= 4) kernel = p.plans ? decode_stream_kernel<T, G, true> : decode_stream_kernel<T, G, false>;
+                else kernel = p.plans ? decode_stream_wide_kernel<T, G, true> : decode_stream_wide_kernel<T, G, false>;
+                if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(kernel), lds_s)) return rc;
+                if (ev0)
+                    hipExtLaunchKernelGGL(kernel, dim3((unsigned)wgs), dim3(kStreamThreads), (uint32_t)lds_s, stream, ev0, ev1, 0u, p);
+                else
+                    hipLaunchKernelGGL(kernel, dim3((unsigned)wgs), dim3(kStreamThreads), lds_s, stream, p);
             }
         } else {
             if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(decode_main_mfma_kernel<T, G>), lds)) return rc;
