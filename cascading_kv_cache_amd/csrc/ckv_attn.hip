@@ -19,7 +19,7 @@ struct Carver {
 
 struct AttnWorkspace {
     void *qr, *kr, *vc;
-    unsigned long long* tile_vis;
+    unsigned long long* tile_vis;   // float32: a word per 32 keys
     uint8_t* kmasked;
     float *lse, *lse2, *colsum, *w_ema, *w_new, *part_o, *part_l2;
     int64_t bytes;
@@ -30,21 +30,23 @@ AttnWorkspace carve_attn(void* base, int64_t B, int64_t H, int64_t KVH, int64_t 
     const int64_t es = elem_bytes(dtype), N = NS + S + Q, n_pad = mfma_n_pad(N);
     Carver c(base);
     AttnWorkspace w;
-    w.qr = c.take((B * H * Q + kColSlack) * D * es);  // rows of slack for the MFMA column pass
-    w.kr = c.take(B * KVH * n_pad * D * es);   // padded to whole key tiles for the MFMA family
-    w.vc = c.take(B * KVH * n_pad * D * es);
+    const bool split = f32_split_supported(dtype, B, H, KVH, Q, N, D);
+    const int64_t rows = split ? f32_split_plane_bytes(B * KVH, N, D) : B * KVH * n_pad * D * es;   // padded to whole key tiles for the MFMA family
+    w.qr = c.take(split ? f32_split_plane_bytes(B * H, Q, D) : (B * H * Q + kColSlack) * D * es);    // rows of slack for the MFMA column pass
+    w.kr = c.take(rows);
+    w.vc = c.take(rows);
     w.tile_vis = (unsigned long long*)c.take(n_pad / 64 * 8);
     w.kmasked = (uint8_t*)c.take(NS + S);
     w.lse = (float*)c.take(B * H * Q * 4);
-    w.lse2 = (float*)c.take((B * H * Q + kColSlack) * 4);
+    w.lse2 = (float*)c.take(split ? B * H * Q * 8 : (B * H * Q + kColSlack) * 4);   // float32: pairs
     w.colsum = (float*)c.take(B * H * N * 4);
     w.w_ema = (float*)c.take((Q + kColSlack) * 4);
     w.w_new = (float*)c.take(Q * 4);
     // shares of the forward kernel when few query rows would leave the chip idle
     int splits = mfma_supported(dtype, D, H, KVH, Q) && Q > 1 ? mfma_fwd_splits_for_workspace(B, H, KVH, Q, N, false) : 1;
-    if (dtype == CKV_F32 && (D == 64 || D == 128)) splits = f32_mfma_splits(B, H, KVH, Q, N, mfma_device_cus());
+    if (split) splits = f32_split_shares(B, H, KVH, Q, N, mfma_device_cus());
     w.part_o = splits > 1 ? (float*)c.take(splits * B * H * Q * D * 4) : nullptr;
-    w.part_l2 = splits > 1 ? (float*)c.take(splits * B * H * Q * 4) : nullptr;
+    w.part_l2 = splits > 1 ? (float*)c.take(splits * B * H * Q * (split ? 8 : 4)) : nullptr;
     w.bytes = c.off;
     return w;
 }
@@ -164,10 +166,12 @@ static int run_attn(const ckv_attn_args* args, hipStream_t stream, const ckv_upd
         rc = launch_mfma(mp, stream);
         if (rc) return rc;
     } else {
-        PrepProblem pp{&a, w.qr, w.kr, w.vc, w.kmasked, want_scores ? w.w_ema : nullptr, w.w_new};
-        rc = launch_prep_generic(pp, stream);
-        if (rc) return rc;
-
+        const bool split = f32_split_supported(a.dtype, a.B, a.H, a.KVH, a.Q, N, a.D);
+        if (!split) {
+            PrepProblem pp{&a, w.qr, w.kr, w.vc, w.kmasked, want_scores ? w.w_ema : nullptr, w.w_new};
+            rc = launch_prep_generic(pp, stream);
+            if (rc) return rc;
+        }
         CoreProblem cp;
         cp.q = w.qr;
         contiguous_strides(cp.q_stride, a.H, a.Q, a.D);
@@ -185,7 +189,15 @@ static int run_attn(const ckv_attn_args* args, hipStream_t stream, const ckv_upd
         cp.B = a.B; cp.H = a.H; cp.KVH = a.KVH; cp.Q = a.Q; cp.N = N; cp.D = a.D;
         cp.scale = 1.f;  // the staged queries and keys each carry sqrt(scale), rounded in as the eager path does
         cp.dtype = a.dtype;
-        rc = f32_mfma_supported(cp) ? launch_f32_mfma(cp, w.part_o, w.part_l2, stream) : launch_core_generic(cp, stream);
+        if (split) {
+            const F32Planes f{w.qr, w.kr, w.vc, (uint32_t*)w.tile_vis, (int)((a.Q + 31) / 32),
+                              (uint32_t)(reinterpret_cast<char*>(w.w_new) - reinterpret_cast<char*>(w.w_ema))};
+            if (!a.lse) cp.lse = nullptr;
+            rc = launch_f32_split(a, cp, f, want_scores ? w.w_ema : nullptr, w.w_new, (float2*)w.lse2, w.part_o,
+                                  (float2*)w.part_l2, stream);
+        } else {
+            rc = launch_core_generic(cp, stream);
+        }
         if (rc) return rc;
     }
     if (a.lse) {
@@ -324,7 +336,7 @@ extern "C" int ckv_attn_dense(const ckv_dense_args* args, void* stream_) {
     cp.B = a.B; cp.H = a.H; cp.KVH = a.H; cp.Q = a.n_ctx; cp.N = a.n_kv; cp.D = a.D;
     cp.scale = a.scale;
     cp.dtype = a.dtype;
-    rc = f32_mfma_supported(cp) ? launch_f32_mfma(cp, nullptr, nullptr, stream) : launch_core_generic(cp, stream);
+    rc = f32_mfma_supported(cp) ? launch_f32_mfma(cp, stream) : launch_core_generic(cp, stream);
     if (rc) return rc;
     if (a.scores) {
         rc = launch_cast_scores(colsum, a.scores, a.scores_stride, a.B, a.H, a.n_kv, a.dtype, stream);

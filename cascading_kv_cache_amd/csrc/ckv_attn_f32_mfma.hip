@@ -1,4 +1,5 @@
-// float32 attention and score sums on the matrix cores (v_mfma_f32_32x32x2_f32), head_dim 64 and 128.
+// The dense operator's float32 attention and score sums on the matrix cores (v_mfma_f32_32x32x2_f32), head_dim 64 and 128, from its
+// operands where they lie.  Cached chunks, which are staged anyway, take the bfloat16 instruction (ckv_attn_f32_split.hip).
 //
 // The float32 matrix instructions multiply and accumulate in float32 (every product enters the accumulator through a
 // fused multiply-add), at twice the rate of the vector ALU and with one operand register per lane instead of LDS reads
@@ -80,29 +81,20 @@ __device__ inline f32x16 zero16() {
 // matrix row of accumulator register v in lane half `half`
 __device__ inline int acc_row(int v, int half) { return 8 * (v >> 2) + 4 * half + (v & 3); }
 
-struct F32Fwd {
-    CoreProblem c;
-    int n_split;     // shares of the key blocks per row tile: few rows would leave most of the chip idle
-    float* part_o;   // (n_split, B*H*Q, D) and
-    float* part_l;   // (n_split, B*H*Q): every share normalised by its own sum, and the logarithm of that
-};
-
 template <int D>
-__global__ void __launch_bounds__(kFwdWaves* CKV_WAVE) fwd_f32_mfma_kernel(F32Fwd f) {
+__global__ void __launch_bounds__(kFwdWaves* CKV_WAVE) fwd_f32_mfma_kernel(CoreProblem p) {
     using G_ = Geo<D>;
     constexpr int NP = G_::kPieces, DB = G_::kDB;
     extern __shared__ __attribute__((aligned(16))) float lds[];
     float4* q_lds = reinterpret_cast<float4*>(lds);                  // [piece][lane]
     float* o_lds = lds + G_::kQ / 4;                                  // [wave][row][kPitch]
     float* ml_lds = o_lds + kFwdWaves * kRows * G_::kPitch;           // [max, sum][wave][row]
-    const CoreProblem& p = f.c;
     const int tid = threadIdx.x, lane = tid & 63, col = lane & 31, half = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // kv heads go round the XCDs (when they divide evenly), so a head's keys stay in one L2; heavy row tiles first
     const int nbkv = (int)(p.B * p.KVH), KVH = (int)p.KVH, G = (int)p.H / KVH;
     const int n_rt = (int)(((int)p.Q * G + kRows - 1) / kRows);
-    const int bkv = blockIdx.x % nbkv, rest = blockIdx.x / nbkv;
-    const int split = rest % f.n_split, rt = n_rt - 1 - rest / f.n_split;
+    const int bkv = blockIdx.x % nbkv, rt = n_rt - 1 - (int)(blockIdx.x / nbkv);
     const int64_t b = bkv / KVH, kvh = bkv % KVH;
     const int N = (int)p.N, Q = (int)p.Q, Nc = N - Q;
     const float* kb = (const float*)p.k + b * p.kv_stride[0] + kvh * p.kv_stride[1];
@@ -186,9 +178,9 @@ __global__ void __launch_bounds__(kFwdWaves* CKV_WAVE) fwd_f32_mfma_kernel(F32Fw
     // its keys behind the logits, its values behind the second product.  So a wavefront waits for memory once, at its first
     // block, which is requested with the queries and before its mask is known (nearly always wanted, and in bounds).
     // Loads and copies retire in issue order; "at most n outstanding" below counts what was issued behind the wanted ones.
-    const int step = kFwdWaves * f.n_split;
+    constexpr int step = kFwdWaves;
     auto mask_byte = [&](int n) -> int { return n < Nc ? (p.kmasked ? p.kmasked[n] : 0) : n < N ? 0 : 1; };
-    int blk = split * kFwdWaves + wave;
+    int blk = wave;
     int hidden = blk < nblk ? mask_byte(blk * kKeys + col) : 1;
     Vec<DB> vf[16];
     constexpr int kValueLoads = 16;
@@ -314,7 +306,7 @@ __global__ void __launch_bounds__(kFwdWaves* CKV_WAVE) fwd_f32_mfma_kernel(F32Fw
     if (__ballot(zero != 0.f) != 0ull) {
 #pragma unroll
         for (int db = 0; db < DB; db++) o[db] = zero16();
-        for (int blk = split * kFwdWaves + wave; blk < nblk; blk += kFwdWaves * f.n_split) {
+        for (int blk = wave; blk < nblk; blk += step) {
             const int n0 = blk * kKeys;
             const uint32_t vis = visible_keys(n0 + col);
             if (vis == 0u) continue;
@@ -396,53 +388,13 @@ __global__ void __launch_bounds__(kFwdWaves* CKV_WAVE) fwd_f32_mfma_kernel(F32Fw
     for (int w = 0; w < kFwdWaves; w++)
 #pragma unroll
         for (int i = 0; i < kPer; i++) acc[i] += o_lds[(w * kRows + r) * G_::kPitch + d0 + i];
-    // A row without a probability above zero (all its logits overflowed) or with a NaN among them is NaN, however many
-    // shares its keys are in; a share without one says so by -inf, a NaN has to reach the merge.
+    // A row without a probability above zero (all its logits overflowed) or with a NaN among them is NaN.
     const float inv = 1.f / L;
-    const int64_t row = (b * p.H + kvh * G + g) * p.Q + m, rows = p.B * p.H * p.Q;
-    if (f.n_split > 1) {
-        float* po = f.part_o + (split * rows + row) * D + d0;
-#pragma unroll
-        for (int i = 0; i < kPer; i++) po[i] = L == 0.f ? 0.f : acc[i] * inv;
-        if (d0 == 0) f.part_l[split * rows + row] = L == 0.f ? -INFINITY : M + logf(L);
-        return;
-    }
+    const int64_t row = (b * p.H + kvh * G + g) * p.Q + m;
     float* orow = (float*)p.out + b * p.out_stride[0] + (kvh * G + g) * p.out_stride[1] + m * p.out_stride[2];
 #pragma unroll
     for (int i = 0; i < kPer; i++) orow[(d0 + i) * p.out_stride[3]] = acc[i] * inv;
     if (d0 == 0 && p.lse) p.lse[row] = M + logf(L);
-}
-
-// the shares of a row: one row per D / 4 lanes
-template <int D>
-__global__ void __launch_bounds__(256) fwd_f32_combine_kernel(F32Fwd f) {
-    const CoreProblem& p = f.c;
-    constexpr int kLanes = D / 4;
-    const int64_t rows = p.B * p.H * p.Q;
-    const int64_t row = (int64_t)blockIdx.x * (256 / kLanes) + threadIdx.x / kLanes;
-    if (row >= rows) return;
-    const int d4 = threadIdx.x % kLanes;
-    float M = -INFINITY, L = 0.f;
-    for (int s = 0; s < f.n_split; s++) M = fmaxf(M, f.part_l[s * rows + row]);
-    float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int s = 0; s < f.n_split; s++) {
-        const float l = f.part_l[s * rows + row];
-        if (l == -INFINITY) continue;
-        const float w = expf(l - M);
-        if (w == 0.f) continue;
-        const float4 v = *reinterpret_cast<const float4*>(f.part_o + (s * rows + row) * D + 4 * d4);
-        L += w;
-        o.x = fmaf(v.x, w, o.x); o.y = fmaf(v.y, w, o.y); o.z = fmaf(v.z, w, o.z); o.w = fmaf(v.w, w, o.w);
-    }
-    const float inv = 1.f / L;
-    int64_t m, h;
-    const int64_t b = div_index(div_index(row, p.Q, m), p.H, h);
-    float* dst = (float*)p.out + b * p.out_stride[0] + h * p.out_stride[1] + m * p.out_stride[2];
-    dst[(4 * d4) * p.out_stride[3]] = o.x * inv;
-    dst[(4 * d4 + 1) * p.out_stride[3]] = o.y * inv;
-    dst[(4 * d4 + 2) * p.out_stride[3]] = o.z * inv;
-    dst[(4 * d4 + 3) * p.out_stride[3]] = o.w * inv;
-    if (d4 == 0 && p.lse) p.lse[row] = M + logf(L);
 }
 
 template <int D, int kGroups>
@@ -572,25 +524,14 @@ __global__ void __launch_bounds__(Col<kGroups>::kWaves* CKV_WAVE, 2) colsum_f32_
 }
 
 template <int D>
-int run(const CoreProblem& p, float* part_o, float* part_l, hipStream_t stream) {
+int run(const CoreProblem& p, hipStream_t stream) {
     const int64_t G = p.H / p.KVH, tiles = (p.Q * G + kRows - 1) / kRows;
     {
         StageScope sc(CKV_STAGE_FWD, stream);
-        F32Fwd f;
-        f.c = p;
-        f.n_split = part_o && part_l ? f32_mfma_splits(p.B, p.H, p.KVH, p.Q, p.N, mfma_device_cus()) : 1;
-        f.part_o = part_o;
-        f.part_l = part_l;
         const int lds = Geo<D>::kFwdLds;
         if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(fwd_f32_mfma_kernel<D>), lds)) return rc;
-        hipLaunchKernelGGL(fwd_f32_mfma_kernel<D>, dim3((unsigned)(tiles * f.n_split * p.B * p.KVH)), dim3(kFwdWaves * CKV_WAVE),
-                           lds, stream, f);
+        hipLaunchKernelGGL(fwd_f32_mfma_kernel<D>, dim3((unsigned)(tiles * p.B * p.KVH)), dim3(kFwdWaves * CKV_WAVE), lds, stream, p);
         CKV_HIP_TRY(hipGetLastError());
-        if (f.n_split > 1) {
-            constexpr int per = 256 / (D / 4);
-            hipLaunchKernelGGL(fwd_f32_combine_kernel<D>, dim3((unsigned)((p.B * p.H * p.Q + per - 1) / per)), dim3(256), 0, stream, f);
-            CKV_HIP_TRY(hipGetLastError());
-        }
     }
     if (p.colsum) {
         StageScope sc(CKV_STAGE_SCORES, stream);
@@ -620,16 +561,6 @@ bool rows16(const int64_t* st, const void* base) {
 
 }  // namespace
 
-// One workgroup fills a compute unit (eight wavefronts of some 220 registers), so a launch with fewer row tiles than
-// that shares the key blocks of a tile out, at least two per wavefront, as long as the shares still fit one round.
-int f32_mfma_splits(int64_t B, int64_t H, int64_t KVH, int64_t Q, int64_t n, int cus) {
-    const int64_t wgs = ((Q * (H / KVH) + kRows - 1) / kRows) * B * KVH, blocks = (n + kKeys - 1) / kKeys;
-    int64_t s = cus / wgs;
-    if (s > blocks / (2 * kFwdWaves)) s = blocks / (2 * kFwdWaves);
-    if (s > 16) s = 16;
-    return s < 1 ? 1 : (int)s;
-}
-
 bool f32_mfma_supported(const CoreProblem& p) {
     return p.dtype == CKV_F32 && (p.D == 64 || p.D == 128) && p.N < ((int64_t)1 << 31) - 64 &&
            p.B * p.H * ((p.N + kKeys - 1) / kKeys) < ((int64_t)1 << 31) &&
@@ -637,8 +568,6 @@ bool f32_mfma_supported(const CoreProblem& p) {
            rows16(p.kv_stride, p.k) && rows16(p.kv_stride, p.v);
 }
 
-int launch_f32_mfma(const CoreProblem& p, float* part_o, float* part_l, hipStream_t stream) {
-    return p.D == 64 ? run<64>(p, part_o, part_l, stream) : run<128>(p, part_o, part_l, stream);
-}
+int launch_f32_mfma(const CoreProblem& p, hipStream_t stream) { return p.D == 64 ? run<64>(p, stream) : run<128>(p, stream); }
 
 }  // namespace ckv

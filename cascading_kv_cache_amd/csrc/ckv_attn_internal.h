@@ -40,11 +40,27 @@ struct CoreProblem {
 // matrix cores (16-bit and float32) do not cover.
 int launch_core_generic(const CoreProblem& p, hipStream_t stream);
 
-// The same in float32 on the matrix cores: head_dim 64 and 128, rows of 16-byte pieces, lse wanted.  part_o / part_l:
-// f32_mfma_splits shares of (B*H*Q, D) / (B*H*Q) floats, or null (then the keys of a row tile are not shared out).
+// The same in float32 on the matrix cores: head_dim 64 and 128, rows of 16-byte pieces, lse wanted.
 bool f32_mfma_supported(const CoreProblem& p);
-int f32_mfma_splits(int64_t B, int64_t H, int64_t KVH, int64_t Q, int64_t n, int cus);
-int launch_f32_mfma(const CoreProblem& p, float* part_o, float* part_l, hipStream_t stream);
+int launch_f32_mfma(const CoreProblem& p, hipStream_t stream);
+
+// ckv_attn in float32, head_dim 64 and 128, on the bfloat16 matrix cores: staging, attention and score sums.  The staged operands, in
+// tiles of 32 rows, three planes each (f32_split_plane_bytes): queries (B, H), keys and values (B, KVH); a word per 32 keys,
+// a bit for each that is there and not masked (f32_split_vis_bytes).
+struct F32Planes {
+    void *q, *k, *v;
+    uint32_t* vis;
+    int q_tiles;         // of a head
+    uint32_t w_new_at;   // bytes from the weights w_ema to w_new, which lie behind them
+};
+bool f32_split_supported(int dtype, int64_t B, int64_t H, int64_t KVH, int64_t Q, int64_t n, int64_t D);
+int f32_split_shares(int64_t B, int64_t H, int64_t KVH, int64_t Q, int64_t n, int cus);
+int64_t f32_split_plane_bytes(int64_t units, int64_t rows, int64_t D);
+int64_t f32_split_vis_bytes(int64_t n);
+// `p`: sizes, out, lse (null: not wanted), colsum and the weights; its operands are not read.  norm: scratch, B*H*Q pairs.  part_o / part_l: f32_split_shares shares of
+// (B*H*Q, D) floats / (B*H*Q) pairs, or null (then the keys of a row tile are not shared out).
+int launch_f32_split(const ckv_attn_args& a, const CoreProblem& p, const F32Planes& f, float* w_ema, float* w_new, float2* norm,
+                     float* part_o, float2* part_l, hipStream_t stream);
 
 // weights of the score sums (cascade_attention.py:270-282, 315-317), rounded like the eager path
 // w_ema gets 64 trailing zeros (slack read by the MFMA column pass)

@@ -487,3 +487,64 @@ def test_the_filled_slots_hint_changes_no_bit_of_a_chunk(D, dtype, H, KVH, W, C,
         results.append([t.clone().view(torch.uint8) for t in (out, new_scores, cache.score_cache[0])])
     for a, b in zip(*results):
         assert torch.equal(a, b)
+
+
+def float32_chunk(Q, D, H, KVH, S, seed):
+    """A chunk of a first call: an empty cache whose hidden slots hold NaN, no rotation (all frequencies zero)."""
+    from cascading_kv_cache_amd.cascading_cache import CascadingKVCache
+
+    cache = CascadingKVCache(window_length=S // 2, num_sink_tokens=3, max_batch_size=1, heads=KVH, dim=D, max_seq_len=S,
+                             device="cuda:0", dtype=F32, layers=1, verbose=False)
+    for t in (cache.key_cache[0], cache.value_cache[0], cache.sink_keys[0], cache.sink_values[0]):
+        t.fill_(float("nan"))
+    gen = torch.Generator().manual_seed(seed)
+    q, k, v = (torch.randn(1, h, Q, D, generator=gen).cuda() for h in (H, KVH, KVH))
+    return cache, q, k, v, torch.zeros(D // 2, device="cuda")
+
+
+@pytest.mark.parametrize("D,Q,H,KVH,S", [(128, 70, 4, 2, 64), (64, 33, 7, 1, 10), (128, 31, 2, 2, 700), (64, 300, 8, 2, 98)])
+def test_float32_chunk_of_values_that_three_planes_do_not_take(D, Q, H, KVH, S):
+    """Infinite, NaN and the largest finite values in queries, keys and values of a float32 chunk, whose operands are the sums of
+    three bfloat16 planes: what is not finite reaches the rows that it reaches in float64, and no other."""
+    from cascading_kv_cache_amd.cascade_attention import cascade_attention
+
+    cache, q, k, v, freq = float32_chunk(Q, D, H, KVH, S, 3)
+    q[0, 0, 7, 3] = float("inf")          # its row is NaN: the rotation multiplies it by zero
+    q[0, 1, 9, 0] = float("nan")
+    q[0, 0, ::2, 5], q[0, 0, 1::2, 5] = 100., -100.
+    k[0, 0, 12, 5] = 3e38                 # logits past the largest number: NaN for every other row, the rest do not see the key
+    v[0, 0, 4, 2] = float("inf")
+    v[0, 0, 6, 2] = float("-inf")         # from row 6 on both: NaN
+    v[0, -1, 20, 1] = 3.4e38              # rounds to no finite bfloat16
+    v[0, -1, 21, 0] = float("nan")
+    out, scores = cascade_attention(q, k, v, cache, 0, freq, update_cache=False)
+    G = H // KVH
+    kk, vv = (t.double().cpu().repeat_interleave(G, 1) for t in (k, v))
+    logits = ((q.double().cpu()[..., None, :] * kk[:, :, None]).sum(-1) / D ** 0.5).float().double()
+    logits[0, 0, 7] = float("nan")
+    p = logits.masked_fill(torch.ones(Q, Q, dtype=torch.bool).triu(1), float("-inf")).softmax(-1)
+    # a key of probability zero counts for nothing, whatever its value
+    terms = torch.where(p[..., None] == 0, 0., p[..., None] * vv[:, :, None])
+    want, got = terms.sum(-2), out.double().cpu()
+    for test in (torch.isnan, torch.isposinf, torch.isneginf):
+        assert torch.equal(test(got), test(want))
+    assert torch.isnan(want).any() and torch.isposinf(want).any() and torch.isfinite(want).sum() > want.numel() // 2
+    fine = torch.isfinite(want)
+    # a float32 sum of up to Q terms; logits of up to 100 * 4 / 8 = 2^6 are off by a unit or two
+    size = terms.abs().sum(-2)[fine]
+    assert ((got - want)[fine].abs() <= 2.0 ** -23 * (Q ** 0.5 + 2 * 2 ** 6) * size).all()
+    assert torch.isnan(scores[0, 0, :8]).all() and (KVH == 1 or torch.isfinite(scores[0, -1, 10:]).all())   # rows 7 and 9
+
+
+@pytest.mark.parametrize("D,Q,H,KVH,S", [(128, 65, 4, 2, 64), (64, 40, 7, 1, 30)])
+def test_float32_chunk_of_rows_that_are_not_aligned(D, Q, H, KVH, S):
+    """Rows that start at any element are staged element by element: the same result to the bit."""
+    from cascading_kv_cache_amd.cascade_attention import cascade_attention
+
+    results = []
+    for layout in (lambda t: t, lambda t: torch.cat((t[..., :1], t), -1)[..., 1:]):
+        cache, q, k, v, freq = float32_chunk(Q, D, H, KVH, S, 5)
+        q, k, v = (layout(t) for t in (q, k, v))
+        results.append(cascade_attention(q, k, v, cache, 0, freq + 0.01, update_cache=False))
+    assert torch.equal(q, float32_chunk(Q, D, H, KVH, S, 5)[1]) and q.data_ptr() % 16 != 0
+    assert all(torch.equal(a, b) for a, b in zip(*results))
