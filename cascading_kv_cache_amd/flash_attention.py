@@ -92,7 +92,7 @@ def _backward(q, k, v, o, lse, mask, do, sm_scale):
     B, H, n_ctx, D = q.shape
     n_kv = k.size(2)
     dev = q.device
-    dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(k)   # of one layout: k and v share theirs
+    dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(k)   # one description serves dk and dv
 
     def describe(a):
         _abi.set_strides(a.q_stride, q)
@@ -146,8 +146,8 @@ class _attention(torch.autograd.Function):
     @staticmethod
     def backward(ctx, do, d_scores):
         q, k, v, o, lse, mask = ctx.saved_tensors
-        if do is None:   # nobody asks for a gradient of o
-            return None, None, None, None, None, None, None
+        if do is None:   # nothing comes back through o
+            return torch.zeros_like(q), torch.zeros_like(k), torch.zeros_like(v), None, None, None, None
         if do.dtype != q.dtype:
             do = do.to(q.dtype)
         dq, dk, dv = _backward(q, k, v, o, lse, mask, do, ctx.sm_scale)
