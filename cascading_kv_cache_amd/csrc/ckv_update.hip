@@ -288,22 +288,20 @@ __device__ inline void plan_closed(const UpdateParams& p, const Unit& u, const C
 __device__ inline int32_t tracker_word(int32_t stored, int32_t start, int32_t W) { return stored >= W ? start : -1 - stored; }
 
 // Workgroups of a unit: one per cascade and extra ones for those with more inserts than threads, as far as they go (with
-// periods that double, cascades of a call of K tokens insert at most 2 K between them).
-__global__ void __launch_bounds__(kClosedThreads) ckv_update_plan_steady_kernel(UpdateParams p) {
-    extern __shared__ __align__(16) unsigned char smem[];
+// periods that double, cascades of a call of K tokens insert at most 2 K between them).  False: the unit is not planned here.
+__device__ inline bool plan_steady(const UpdateParams& p, const Unit& u, int block, int extra, unsigned char* smem) {
     const ckv_update_args& A = p.a;
-    const Unit u(A);
     const int tid = threadIdx.x, lane = tid % CKV_WAVE, T = kClosedThreads;
-    const int C = A.cascades, block = (int)blockIdx.x, extra = (int)gridDim.x - C;
+    const int C = A.cascades;
     const int64_t seen = *A.real_token_idx + p.token_offset;  // tokens before token 0 of this launch
     ClosedCascade forms;
     unsigned long long touched;
-    const bool closed = closed_forms(A, u, seen, p.k_sub, lane, forms, touched);
+    if (!closed_forms(A, u, seen, p.k_sub, lane, forms, touched)) return false;
+    if (block < 0) return true;
     if (block == 0 && tid == 0) {
-        p.flags[u.bh] = closed ? kPlanned | kPosChange : 0;
-        if (closed) p.sinks_new[u.bh] = (int32_t)A.stored_sinks[u.n * A.stored_sinks_stride[0] + u.h * A.stored_sinks_stride[1]];
+        p.flags[u.bh] = kPlanned | kPosChange;
+        p.sinks_new[u.bh] = (int32_t)A.stored_sinks[u.n * A.stored_sinks_stride[0] + u.h * A.stored_sinks_stride[1]];
     }
-    if (!closed) return;
     int mine = block, part = 0;
     const int want = lane < C && forms.E > T ? (forms.E - 1) / T : 0;
     int before = want;  // extra workgroups the cascades before this lane's want
@@ -315,7 +313,7 @@ __global__ void __launch_bounds__(kClosedThreads) ckv_update_plan_steady_kernel(
     before -= want;
     if (block >= C) {
         const unsigned long long here = __builtin_amdgcn_ballot_w64(before <= block - C && block - C < before + want);
-        if (here == 0) return;
+        if (here == 0) return true;
         mine = __builtin_ctzll(here);
         part = block - C - __shfl(before, mine) + 1;
     }
@@ -325,15 +323,20 @@ __global__ void __launch_bounds__(kClosedThreads) ckv_update_plan_steady_kernel(
         p.trackers[u.bh * C + mine] = (int32_t)(((uint32_t)forms.sx + (uint32_t)forms.E) % (uint32_t)A.window_size);
     }
     plan_closed(p, u, forms, touched, mine, part, parts, smem);
+    return true;
 }
 
-__global__ void ckv_update_plan_kernel(UpdateParams p) {
+__global__ void __launch_bounds__(kClosedThreads) ckv_update_plan_steady_kernel(UpdateParams p) {
     extern __shared__ __align__(16) unsigned char smem[];
+    const Unit u(p.a);
+    if (!plan_steady(p, u, (int)blockIdx.x, (int)gridDim.x - p.a.cascades, smem) && blockIdx.x == 0 && threadIdx.x == 0) p.flags[u.bh] = 0;
+}
+
+// The walk over all arrivals, a workgroup per unit.
+__device__ inline void plan_walk(const UpdateParams& p, const Unit& u, unsigned char* smem) {
     const ckv_update_args& A = p.a;
     const int tid = threadIdx.x, T = blockDim.x;
-    const Unit u(A);
     const int64_t n = u.n, h = u.h, bh = u.bh;
-    if (p.flags[bh] & kPlanned) return;  // the steady-state kernel has planned this unit
     const int cap = p.k_sub;
     const int C = A.cascades;
     const int64_t W = A.window_size, S = A.max_seq_len, NS = A.num_sink;
@@ -542,6 +545,23 @@ __global__ void ckv_update_plan_kernel(UpdateParams p) {
 
     // the position ids change only when the last token of the call went to the cascades
     if (tid == 0) p.flags[bh] = cap > n_sink_new ? kPosChange : 0;
+}
+
+__global__ void ckv_update_plan_kernel(UpdateParams p) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    const Unit u(p.a);
+    if (p.flags[u.bh] & kPlanned) return;  // the steady-state kernel has planned this unit
+    plan_walk(p, u, smem);
+}
+
+// Both in one launch: the first workgroup of a unit walks its arrivals if the others, which look at the same trackers (apply commits
+// them), find that the closed forms do not hold.  A launch that mostly returns took a call 4 to 5 us, its instructions being cold: 256
+// tokens into 512 float32 slots 74.6 -> 70.2 us behind their attention, 509 into 16 K 290 -> 288.
+__global__ void __launch_bounds__(kClosedThreads) ckv_update_plan_both_kernel(UpdateParams p) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    const Unit u(p.a);
+    const int block = (int)blockIdx.x - 1;
+    if (!plan_steady(p, u, block, (int)gridDim.x - 1 - p.a.cascades, smem) && block < 0) plan_walk(p, u, smem);
 }
 
 // The walk of a single incoming token (the decode step), by one wavefront: lane i fetches what cascade i may need (trackers,
@@ -1080,6 +1100,10 @@ __global__ void ckv_update_apply_elem_kernel(UpdateParams p) {
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
+// One launch for both planners where the walk's LDS lets as many workgroups on a compute unit as their threads do, four (1092 tokens).
+// Past that their LDS would make rounds of the workgroups of the closed forms, which a long call has most of.
+constexpr size_t kBothLds = 40 * 1024;
+
 inline size_t plan_lds_bytes(int cap) {
     return (size_t)cap * 24 + (size_t)(cap + 1) * 8 + (size_t)(cap + 2) * 4 + kMaxCascades * 20 + 64 * sizeof(int) + 64;
 }
@@ -1187,16 +1211,19 @@ int run_update(const ckv_update_args& A, void* workspace, int64_t* row, int64_t 
         if (A.K == 1) {  // the decode step: one wavefront per unit
             launch_timed(CKV_STAGE_PLAN, ckv_update_plan1_kernel, dim3(1, H, N), dim3(CKV_WAVE), 0, stream, p);
         } else {
-            // every unit first gets the chance of the closed forms; the general kernel takes the others
-            const size_t lds_closed = (size_t)ksub * 16;
-            if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(ckv_update_plan_steady_kernel), (int)lds_closed)) return rc;
-            launch_timed(CKV_STAGE_PLAN, ckv_update_plan_steady_kernel, dim3((unsigned)(A.cascades + 2 * ksub / kClosedThreads), H, N),
-                         dim3(kClosedThreads), lds_closed, stream, p);
-            CKV_HIP_TRY(hipGetLastError());
-            const int T = ksub <= 256 ? 256 : 1024;  // few tokens: a small block plans them
-            const size_t lds = plan_lds_bytes(ksub);
-            if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(ckv_update_plan_kernel), (int)lds)) return rc;
-            launch_timed(CKV_STAGE_PLAN, ckv_update_plan_kernel, dim3(1, H, N), dim3(T), lds, stream, p);
+            // every unit first gets the chance of the closed forms; the walk takes the others
+            const unsigned closed = (unsigned)(A.cascades + 2 * ksub / kClosedThreads);
+            const size_t lds_closed = (size_t)ksub * 16, lds = plan_lds_bytes(ksub);
+            if (lds <= kBothLds) {
+                launch_timed(CKV_STAGE_PLAN, ckv_update_plan_both_kernel, dim3(closed + 1, H, N), dim3(kClosedThreads), lds, stream, p);
+                StageScope sc(CKV_STAGE_PLAN, stream);   // timed stages: a chunk has two of these either way
+            } else {
+                if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(ckv_update_plan_steady_kernel), (int)lds_closed)) return rc;
+                launch_timed(CKV_STAGE_PLAN, ckv_update_plan_steady_kernel, dim3(closed, H, N), dim3(kClosedThreads), lds_closed, stream, p);
+                CKV_HIP_TRY(hipGetLastError());
+                if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(ckv_update_plan_kernel), (int)lds)) return rc;
+                launch_timed(CKV_STAGE_PLAN, ckv_update_plan_kernel, dim3(1, H, N), dim3(1024), lds, stream, p);
+            }
         }
         CKV_HIP_TRY(hipGetLastError());
         // the position ids of the last launch of a call are written by extra blocks of the apply grid
