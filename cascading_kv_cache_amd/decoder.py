@@ -4,8 +4,8 @@ strides, then greedy decoding one token at a time (cascade/models/cascade_attent
 
 The reference patches Hugging Face Llama / Qwen2 models; this module carries just enough of such a
 decoder (embedding, RMSNorm, gated MLP, untied head; projections with optional bias) to run the
-benchmark shapes end to end with random weights.  Everything outside attention is plain PyTorch;
-attention, scores and the cache are the library's (:class:`ProjectedCascadeAttention`).
+benchmark shapes end to end with random weights.  Everything outside attention is plain PyTorch but the
+gate of a fused MLP; attention, scores and the cache are the library's (:class:`ProjectedCascadeAttention`).
 
     python -m cascading_kv_cache_amd.decoder --preset llama3.1-8b --layers 4 --prompt 16384 --stride 4096 --new 32
 """
@@ -17,7 +17,8 @@ from dataclasses import dataclass, replace
 import torch
 from torch import nn
 
-from .cascading_cache import CascadingKVCache
+from . import _abi
+from .cascading_cache import CascadingKVCache, on_device, raw_stream
 from .latency import ProjectedCascadeAttention
 
 
@@ -60,6 +61,26 @@ class RMSNorm(nn.Module):
         return self.weight * xf.to(x.dtype)
 
 
+_functorch_levels = getattr(getattr(torch._C, "_functorch", None), "peek_interpreter_stack", lambda: None)   # not public
+_GATED_TYPES = (torch.bfloat16, torch.float16, torch.float32)
+
+
+def gated_silu(gate_up):
+    """``silu(gate) * up`` of rows of ``gate | up``: one launch of the library, the same bits, where nobody follows what is done
+    (gradients of either mode, vmap, tracing)."""
+    if (gate_up.device.type != "cuda" or torch.is_grad_enabled() or gate_up.requires_grad or not gate_up.is_contiguous()
+            or gate_up.dtype not in _GATED_TYPES or torch.autograd.forward_ad._current_level >= 0 or _functorch_levels() is not None
+            or torch.jit.is_tracing() or torch.compiler.is_compiling()):
+        gate, up = gate_up.chunk(2, dim=-1)
+        return nn.functional.silu(gate) * up
+    inter = gate_up.size(-1) // 2
+    out = torch.empty(gate_up.shape[:-1] + (inter,), dtype=gate_up.dtype, device=gate_up.device)
+    with on_device(gate_up.device):
+        _abi.check(_abi.lib().ckv_gated_silu(gate_up.data_ptr(), out.data_ptr(), gate_up.numel() // (2 * inter), inter, 2 * inter,
+                                             _abi.dtype_code(gate_up.dtype), raw_stream(gate_up.device)), "ckv_gated_silu")
+    return out
+
+
 class GatedMLP(nn.Module):
     def __init__(self, cfg, dtype, device):
         super().__init__()
@@ -81,8 +102,7 @@ class GatedMLP(nn.Module):
     def forward(self, x):
         if self._w_gate_up is None:
             return self.down_proj(nn.functional.silu(self.gate_proj(x)) * self.up_proj(x))
-        gate, up = nn.functional.linear(x, self._w_gate_up).chunk(2, dim=-1)
-        return self.down_proj(nn.functional.silu(gate) * up)
+        return self.down_proj(gated_silu(nn.functional.linear(x, self._w_gate_up)))
 
 
 class DecoderLayer(nn.Module):

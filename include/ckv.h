@@ -315,6 +315,10 @@ int ckv_attn_dense_bwd(const ckv_dense_bwd_args* args, void* stream);
 int ckv_chunk_positions(const int64_t* key_pos, int64_t n_key, int64_t key_shift, const int64_t* sink_pos,
                         int64_t n_sink, int64_t q_len, int64_t* q_pos, void* stream);
 
+/* out (rows, inter) = silu(gate) * up of rows of gate | up, row_stride >= 2 * inter elements apart: the middle of a gated MLP whose
+ * two projections are one matrix product, each of the two operations rounded to the tensor dtype. */
+int ckv_gated_silu(const void* gate_up, void* out, int64_t rows, int64_t inter, int64_t row_stride, int32_t dtype, void* stream);
+
 /* ------------------------------------------------------------------------------------------
  * Stage timing (the reference's BENCHMARK=True switch, cascading_cache.py:986-1026, extended to
  * every kernel stage).  While enabled, each stage of ckv_attn / ckv_update is bracketed by HIP

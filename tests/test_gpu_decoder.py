@@ -201,3 +201,30 @@ def test_chunked_prefill_equals_one_dense_shot_while_the_stream_fits(dtype):
     assert torch.equal(chunked.argmax(-1)[clear], dense.argmax(-1)[clear])
     assert cache.seen_tokens_by_layer.cpu().tolist() == [n] * cfg.num_layers
     assert int(cache.start_indices[0].sum()) == 0, "nothing may have been evicted"
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("shape,offset", [((1, 1, 14336), 0), ((1, 1, 18944), 0), ((2, 37, 1000), 0), ((1, 3, 13), 0), ((1, 5, 64), 1)])
+def test_gate_in_one_launch_has_the_bits_of_the_two_operations(shape, offset, dtype):
+    """Rows of 16-byte pieces, of other lengths and from other addresses, with every 16-bit gate there is in the larger ones."""
+    from cascading_kv_cache_amd.decoder import gated_silu
+
+    gen = torch.Generator().manual_seed(11)
+    full = shape[:-1] + (2 * shape[-1],)
+    x = torch.empty(torch.Size(full).numel() + offset, dtype=dtype, device="cuda")[offset:].view(full)
+    for low in range(-32768, 32768, shape[-1]) if dtype != torch.float32 and shape[-1] >= 1000 else [None]:
+        x.copy_(torch.randn(full, generator=gen) * 4)
+        if low is not None:
+            bits = torch.arange(low, low + shape[-1], device="cuda").clamp(max=32767).to(torch.int16)
+            x[..., :shape[-1]] = bits.view(dtype).expand(shape)
+        gate, up = x.chunk(2, dim=-1)
+        want = torch.nn.functional.silu(gate) * up
+        with torch.no_grad():
+            got = gated_silu(x)
+        assert got.shape == want.shape and got.is_contiguous()
+        kind = torch.int32 if dtype == torch.float32 else torch.int16
+        finite = ~torch.isnan(want)
+        assert torch.equal(torch.isnan(got), ~finite) and torch.equal(got[finite].view(kind), want[finite].view(kind))
+    x.requires_grad_()
+    gated_silu(x).sum().backward()   # gradients come from the two operations
+    assert x.grad.shape == x.shape
