@@ -15,7 +15,7 @@ import torch
 from torch import nn
 
 from . import _abi
-from .cascading_cache import CascadingKVCache, _require_device, on_device, raw_stream, workspace
+from .cascading_cache import CascadingKVCache, _counter_table, _require_device, on_device, raw_stream, workspace
 
 
 _DEBUG_COUNTERS = os.environ.get("CKV_DEBUG_COUNTERS", "0") not in ("", "0")
@@ -48,12 +48,18 @@ def chunk_positions(cache: CascadingKVCache, layer_idx: int, q_len: int, do_og_p
     if not do_og_pos and cache.eager_fill and S > 0 and not _replayable:
         start = min(int(cache._seen_host[layer_idx]), S + NS)
         memo = cache.__dict__.setdefault("_steady_q_pos", {})
-        key = (start, q_len, dev)
+        own = _stream is None   # a caller's own ids, which it may write to; the library's are a part of a table of integers
+        key = (start, q_len, dev, own)
         ids = memo.get(key)
         if ids is None:
             if len(memo) > 16:
                 memo.clear()
-            ids = memo[key] = torch.arange(start, start + q_len, device=dev, dtype=torch.long)
+            table = None if own else _counter_table(dev)
+            if table is not None and start + q_len <= table.numel():
+                ids = table[start:start + q_len]
+            else:
+                ids = torch.arange(start, start + q_len, device=dev, dtype=torch.long)
+            memo[key] = ids
         return ids
     out = torch.empty(q_len, device=dev, dtype=torch.long)
     key_ptr, n_key, shift, sink_ptr, n_sink = None, 0, 0, None, 0

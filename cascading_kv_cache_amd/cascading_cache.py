@@ -236,11 +236,17 @@ class CascadingKVCache:
         self._seen_host = [0 for _ in range(self.layers)]
         self._seen_pending = [0 for _ in range(self.layers)]
         self._seen_dev.zero_()
+        small = {}   # by type: cleared together, a launch for many
         for group in (self.stored_tokens, self.stored_sinks, self.start_indices, self.pos, self.sink_pos,
                       self.key_cache, self.value_cache, self.score_cache, self.sink_keys, self.sink_values,
                       self.og_pos):
             for t in group:
-                t.zero_()
+                if t.numel() < 1 << 20:
+                    small.setdefault(t.dtype, []).append(t)
+                else:
+                    t.zero_()
+        for tensors in small.values():
+            torch._foreach_zero_(tensors)
         for group in (self.do_cache, self.mask, self.sink_mask):
             for t in group:
                 t.fill_(True)
