@@ -117,7 +117,7 @@ def fill_to_steady_state(cache, cfg, pool, inv_freq):
 def update_traffic(workload, single_token=False):
     """Measured HBM bytes of one cache update: the sum over its launches (None when any figure is stale)."""
     names = (["ckv_update_one_kernel"] if single_token else
-             ["ckv_update_plan_steady_kernel", "ckv_update_plan_kernel", "ckv_update_apply_vec_kernel"])
+             ["ckv_update_plan_both_kernel", "ckv_update_apply_vec_kernel"])
     parts = [measured_traffic(k, workload) for k in names]
     return None if any(x is None for x in parts) else sum(parts)
 
@@ -313,7 +313,7 @@ def run_layer(steps, warmup, dtype, device):
                                   peak=PEAK_HBM_GBPS, unit="GB/s",
                                   frac=ubytes / (upd_ms * 1e-3) / 1e9 / PEAK_HBM_GBPS if upd_ms else 0.0,
                                   traffic=update_traffic("layer64k"),
-                                  kernel="ckv_update_plan_steady_kernel + ckv_update_plan_kernel + ckv_update_apply_vec_kernel",
+                                  kernel="ckv_update_plan_both_kernel + ckv_update_apply_vec_kernel",
                                   kernel_ms=upd_ms,
                                   algorithmic_gb_per_launch=ubytes / 1e9), **ucount),
     )

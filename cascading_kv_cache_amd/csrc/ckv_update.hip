@@ -291,7 +291,7 @@ __device__ inline int32_t tracker_word(int32_t stored, int32_t start, int32_t W)
 // periods that double, cascades of a call of K tokens insert at most 2 K between them).  False: the unit is not planned here.
 __device__ inline bool plan_steady(const UpdateParams& p, const Unit& u, int block, int extra, unsigned char* smem) {
     const ckv_update_args& A = p.a;
-    const int tid = threadIdx.x, lane = tid % CKV_WAVE, T = kClosedThreads;
+    const int tid = threadIdx.x, lane = tid % CKV_WAVE, T = blockDim.x;
     const int C = A.cascades;
     const int64_t seen = *A.real_token_idx + p.token_offset;  // tokens before token 0 of this launch
     ClosedCascade forms;
@@ -557,7 +557,8 @@ __global__ void ckv_update_plan_kernel(UpdateParams p) {
 // Both in one launch: the first workgroup of a unit walks its arrivals if the others, which look at the same trackers (apply commits
 // them), find that the closed forms do not hold.  A launch that mostly returns took a call 4 to 5 us, its instructions being cold: 256
 // tokens into 512 float32 slots 74.6 -> 70.2 us behind their attention, 509 into 16 K 290 -> 288.
-__global__ void __launch_bounds__(kClosedThreads) ckv_update_plan_both_kernel(UpdateParams p) {
+template <int kThreads>
+__global__ void __launch_bounds__(kThreads) ckv_update_plan_both_kernel(UpdateParams p) {
     extern __shared__ __align__(16) unsigned char smem[];
     const Unit u(p.a);
     const int block = (int)blockIdx.x - 1;
@@ -1100,8 +1101,11 @@ __global__ void ckv_update_apply_elem_kernel(UpdateParams p) {
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
-// One launch for both planners where the walk's LDS lets as many workgroups on a compute unit as their threads do, four (1092 tokens).
-// Past that their LDS would make rounds of the workgroups of the closed forms, which a long call has most of.
+// One launch for both planners where the walk's LDS lets as many workgroups on a compute unit as their threads do, four (1092 tokens),
+// or where all of them run at once, one on a unit.  Past that their LDS would make rounds of the workgroups of the closed forms.  One on
+// a unit they have 1024 threads: the walk of 4096 tokens into 64 K slots takes 8 to 18 % longer with 512, more than the launch
+// saved (calls of a cache that fills, us, two launches, one with 512 and with 1024 threads: the third 46.6 47.5 40.4, the tenth 91.5 105.0
+// 86.2, the sixteenth 138.3 163.8 133.3; full 31.4 28.4 30.1).
 constexpr size_t kBothLds = 40 * 1024;
 
 inline size_t plan_lds_bytes(int cap) {
@@ -1214,9 +1218,18 @@ int run_update(const ckv_update_args& A, void* workspace, int64_t* row, int64_t 
             // every unit first gets the chance of the closed forms; the walk takes the others
             const unsigned closed = (unsigned)(A.cascades + 2 * ksub / kClosedThreads);
             const size_t lds_closed = (size_t)ksub * 16, lds = plan_lds_bytes(ksub);
-            if (lds <= kBothLds) {
-                launch_timed(CKV_STAGE_PLAN, ckv_update_plan_both_kernel, dim3(closed + 1, H, N), dim3(kClosedThreads), lds, stream, p);
+            auto launch_both = [&](auto threads) -> int {
+                auto kernel = ckv_update_plan_both_kernel<threads.value>;
+                if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(kernel), (int)lds)) return rc;
+                launch_timed(CKV_STAGE_PLAN, kernel, dim3((unsigned)(A.cascades + 2 * ksub / threads.value) + 1, H, N), dim3(threads.value), lds,
+                             stream, p);
                 StageScope sc(CKV_STAGE_PLAN, stream);   // timed stages: a chunk has two of these either way
+                return CKV_OK;
+            };
+            if (lds <= kBothLds) {
+                if (int rc = launch_both(std::integral_constant<int, kClosedThreads>{})) return rc;
+            } else if ((int64_t)(A.cascades + 2 * ksub / 1024 + 1) * A.N * A.H <= di.cus) {
+                if (int rc = launch_both(std::integral_constant<int, 1024>{})) return rc;
             } else {
                 if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(ckv_update_plan_steady_kernel), (int)lds_closed)) return rc;
                 launch_timed(CKV_STAGE_PLAN, ckv_update_plan_steady_kernel, dim3(closed, H, N), dim3(kClosedThreads), lds_closed, stream, p);

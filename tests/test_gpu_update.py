@@ -152,12 +152,13 @@ def test_calls_that_evict_what_they_brought(W, C, func):
     run_stream(gpu, cpu, sum(lengths), lambda: next(left), gen, torch.bfloat16, "ties")
 
 
+@pytest.mark.parametrize("B,H", [(2, 2), (8, 8)])   # past 1092 tokens: one launch while its workgroups are at most the compute units
 @pytest.mark.parametrize("W,C,func", [(600, 3, "pow2"), (2048, 2, "pow2"), (300, 4, "iplus1")])
-def test_calls_around_the_line_of_one_launch_for_both_plans(W, C, func):
+def test_calls_around_the_line_of_one_launch_for_both_plans(B, H, W, C, func):
     """Up to 1092 tokens both planners share a launch, which the walk's first workgroup uses while the cache fills and the others
     once it is full; two cascades of 2048 stay in the walk for three calls and are in the closed forms after that."""
     gen = torch.Generator().manual_seed(37)
-    gpu, cpu = make_pair(2, 2, 8, 5, W, C, torch.float32, func=func)
+    gpu, cpu = make_pair(B, H, 4, 5, W, C, torch.float32, func=func)
     lengths = iter([1092, 1093, 1092, 1091, 1093, 2, 1092, 1093])
     run_stream(gpu, cpu, 4 * 1092 + 3 * 1093 + 1, lambda: next(lengths), gen, torch.float32, "ties")
 
