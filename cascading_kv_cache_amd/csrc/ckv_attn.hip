@@ -56,7 +56,7 @@ AttnWorkspace carve_attn(void* base, int64_t B, int64_t H, int64_t KVH, int64_t 
 struct DenseWorkspace {
     void *qr, *kr, *vc;
     unsigned long long* tile_vis;
-    float *lse, *lse2, *w_ema, *w_new, *part_o, *part_l2;
+    float *lse, *lse2, *w_ema, *w_new, *part_o, *part_l2, *part_scores;
     int *key_order, *n_visible;
     int64_t bytes;
 };
@@ -78,6 +78,8 @@ DenseWorkspace carve_dense(void* base, int64_t B, int64_t H, int64_t n_ctx, int6
     const int splits = mfma_fwd_splits_for_workspace(B, H, H, n_ctx, n_kv, true);
     w.part_o = splits > 1 ? (float*)c.take(splits * rows * D * 4) : nullptr;
     w.part_l2 = splits > 1 ? (float*)c.take(splits * rows * 4) : nullptr;
+    const int shares = dense_row_shares(B, H, n_ctx, n_kv, mfma_device_cus());
+    w.part_scores = shares > 1 ? (float*)c.take(shares * B * H * n_kv * 4) : nullptr;
     w.bytes = c.off;
     return w;
 }
@@ -295,6 +297,7 @@ extern "C" int ckv_attn_dense(const ckv_dense_args* args, void* stream_) {
         mp.lse2 = w.lse2;
         mp.colsum = nullptr;
         mp.scores = a.scores;
+        mp.part_scores = w.part_scores;
         for (int i = 0; i < 3; i++) mp.scores_stride[i] = a.scores_stride[i];
         mp.part_o = w.part_o; mp.part_l2 = w.part_l2;
         mp.w_ema = w.w_ema; mp.w_new = w.w_new;

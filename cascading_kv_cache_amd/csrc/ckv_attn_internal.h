@@ -198,6 +198,7 @@ struct MfmaProblem {
     float* colsum;         // (B, H, n) or null
     void* scores = nullptr;  // takes colsum's place: (B, H, n) in the tensor dtype, at the row each key came from
     int64_t scores_stride[3] = {0, 0, 0};
+    float* part_scores = nullptr;  // (dense_row_shares, B*H, n): where the sums of a key are shared out, or null
     // keys in another order than they lie in memory (launch_dense_prologue): seg[0] then holds all keys
     const int* key_order = nullptr;
     const int* n_visible = nullptr;
@@ -222,6 +223,7 @@ int64_t mfma_n_pad(int64_t n);
 // shares of the key tiles per query tile on a chip of `cus` compute units; what a workspace must hold
 int mfma_fwd_splits(int64_t B, int64_t H, int64_t KVH, int64_t Q, int64_t n, int cus, bool dense);
 int mfma_fwd_splits_for_workspace(int64_t B, int64_t H, int64_t KVH, int64_t Q, int64_t n, bool dense);
+int dense_row_shares(int64_t B, int64_t H, int64_t n_ctx, int64_t n_kv, int cus);
 int mfma_device_cus();  // compute units of the current device (256 where none can be asked)
 bool mfma_fits(int64_t n, int64_t D);  // the per-tile bookkeeping of n keys fits in LDS
 int launch_mfma(const MfmaProblem& p, hipStream_t stream);

@@ -1215,6 +1215,8 @@ struct ColsumParams {
     const int* key_order; // row each key came from
     void* scores;         // (B, H, N) in the tensor dtype, at the row each key came from: takes the place of colsum
     int64_t scores_stride[3];
+    int row_shares;       // the query tiles of a key block are shared out over this many workgroups (1: the block's own), each of which
+    float* part;          // leaves its sums in (row_shares, B*H, N), see colsum_merge_kernel
     int wnew_uniform;     // every entry of w_new has the value wnew_value (beta rounds to one in the tensor dtype)
     float wnew_value;
 };
@@ -1227,7 +1229,7 @@ __host__ __device__ constexpr int cs_stage(int head_dim) { return kQT2 * 2 * hea
 // S = Q K^T).  The (head, query-tile) sequence streams through a double-buffered LDS stage filled
 // by asynchronous copies; lane (col, half) owns key column `col` of each 32-key subtile, so the
 // weighted column sums never leave the lane.
-template <typename T, int kD>
+template <typename T, int kD, bool kShares>
 __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
     extern __shared__ __align__(16) unsigned char smem[];
     constexpr int kKK = kD / 16, kRowBytes = 2 * kD, kCsStage = cs_stage(kD);
@@ -1244,11 +1246,16 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
     // block of one kv head runs on one XCD so that head's query stream stays in that XCD's L2.
     // A key block is shared out over gsplit workgroups, each taking G / gsplit heads: units small
     // enough that the last round of workgroups costs little.
-    int bkv_i, kb_i, g_first;
+    int bkv_i, kb_i, g_first, share = 0;
     const int g_cnt = p.G / p.gsplit;
     {
         const int nkb = p.nkb * p.gsplit, cb0 = (Nc / 256) * p.gsplit, heavy = nkb - cb0;
         int id = blockIdx.x, nb = p.nbkv, first = 0, stride = 1;
+        if (kShares) {   // shares outermost: a multiple of the XCDs apart where the order looks at them
+            const int blocks = nb * nkb;
+            share = id / blocks;
+            id -= share * blocks;
+        }
         if (p.xcd_aware) {
             first = id & 7;
             stride = 8;
@@ -1306,7 +1313,14 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
         for (int i = tid; i < Q; i += 256) wnew_lds[i] = p.w_new[i];
     }
     auto wnew_at = [&](int i) -> float { return p.wnew_uniform ? p.wnew_value : wnew_lds[i]; };
-    const int nmt = (Q - m_first + kQT2 - 1) / kQT2;  // query tiles per head
+    int nmt = (Q - m_first + kQT2 - 1) / kQT2;  // query tiles per head
+    int m_end = Q;                              // where the workgroup's share of them ends
+    if (kShares && nmt > 0) {
+        const int t0 = share * nmt / p.row_shares, t1 = (share + 1) * nmt / p.row_shares;
+        m_end = m_first + t1 * kQT2 < Q ? m_first + t1 * kQT2 : Q;
+        m_first += t0 * kQT2;
+        nmt = t1 - t0;
+    }
     // A block without a single visible key (the empty part of a cache that is still filling) has nothing but zeros to
     // write: with 1000 of 16384 slots filled and a 488-token chunk that is 63 of 67 blocks.
     const unsigned long long* vis = p.tile_vis + key_blk / kBN;
@@ -1353,7 +1367,9 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
     };
 
     auto store = [&](int64_t h, int64_t n, float v) {
-        if (p.scores) {
+        if (kShares) {
+            p.part[((share * p.B + b) * p.H + h) * p.N + n] = v;
+        } else if (p.scores) {
             T* dst = (T*)p.scores + b * p.scores_stride[0] + h * p.scores_stride[1];
             dst[(p.key_order ? p.key_order[n] : n) * p.scores_stride[2]] = Elem<T>::from_float(v);
         } else {
@@ -1556,7 +1572,7 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
                 }
             }
         }
-        if (mt + kQT2 >= Q) {  // head finished: combine the two lane halves and store
+        if (mt + kQT2 >= m_end) {  // head finished: combine the two lane halves and store
             const int64_t h = kvh * p.G + g;
 #pragma unroll
             for (int ks = 0; ks < 2; ks++) {
@@ -1582,7 +1598,7 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
     int g_cur = g_first, mt_cur = m_first;    // step being consumed
     auto advance = [&](int& g, int& mt) {
         mt += kQT2;
-        if (mt >= Q) {
+        if (mt >= m_end) {
             mt = m_first;
             g++;
         }
@@ -1616,6 +1632,19 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
                 if (half == 0 && n < p.N) store(kvh * p.G + g, n, 0.f);
             }
     }
+}
+
+// The shares of a key's sums added up in order, at the row the key came from.
+template <typename T>
+__global__ void __launch_bounds__(256) colsum_merge_kernel(ColsumParams p) {
+    const int64_t n = (int64_t)blockIdx.x * 256 + threadIdx.x, bh = blockIdx.y, heads = p.B * p.H;
+    if (n >= p.N) return;
+    float sum = 0.f;
+    for (int r = 0; r < p.row_shares; r++) sum += p.part[(r * heads + bh) * p.N + n];
+    int64_t h;
+    const int64_t b = div_index(bh, p.H, h);
+    T* dst = (T*)p.scores + b * p.scores_stride[0] + h * p.scores_stride[1];
+    dst[(p.key_order ? p.key_order[n] : n) * p.scores_stride[2]] = Elem<T>::from_float(sum);
 }
 
 template <typename T, int kD>
@@ -1776,10 +1805,17 @@ int run_mfma(const MfmaProblem& mp, hipStream_t stream) {
         //   8.5 (1 x 4096 x 64 K) 1815 1814    16 (2 x 33 x 64 K) 190  145       16 (2 x 1500 x 64 K) 1394 1363
         const int64_t of_two = (int64_t)cp.nkb * cp.nbkv * (G / 2);
         cp.gsplit = (G % 2 == 0 && G >= 4 && of_two >= 4 * 2 * (int64_t)cus) ? G / 2 : G;
-        const dim3 grid((unsigned)(cp.nkb * cp.nbkv * cp.gsplit));
+        cp.row_shares = mp.scores && mp.part_scores ? dense_row_shares(mp.B, mp.H, mp.Q, n, cus) : 1;
+        cp.part = mp.part_scores;
+        const dim3 grid((unsigned)(cp.nkb * cp.nbkv * cp.gsplit * cp.row_shares));
         const int lds = 2 * cs_stage(kD) + (cp.wnew_uniform ? 0 : (int)mp.Q * 4);
-        if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(colsum_mfma_kernel<T, kD>), lds)) return rc;
-        hipLaunchKernelGGL((colsum_mfma_kernel<T, kD>), grid, dim3(256), lds, stream, cp);
+        auto kernel = cp.row_shares > 1 ? colsum_mfma_kernel<T, kD, true> : colsum_mfma_kernel<T, kD, false>;
+        if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(kernel), lds)) return rc;
+        hipLaunchKernelGGL(kernel, grid, dim3(256), lds, stream, cp);
+        if (cp.row_shares > 1) {
+            CKV_HIP_TRY(hipGetLastError());
+            hipLaunchKernelGGL(colsum_merge_kernel<T>, dim3((unsigned)((n + 255) / 256), (unsigned)(mp.B * mp.H)), dim3(256), 0, stream, cp);
+        }
         CKV_HIP_TRY(hipGetLastError());
     }
     return CKV_OK;
@@ -1793,6 +1829,18 @@ bool mfma_supported(int dtype, int64_t D, int64_t H, int64_t KVH, int64_t Q) {
     if (Q > 16384) return false;  // the column pass keeps a Q-long weight table in LDS beside its two stages
     const int64_t G = H / KVH;
     return G >= 1 && G <= kRows / 32;  // at least 32 positions per workgroup
+}
+
+// Workgroups that share the query tiles of a key block in the dense operator's score sums.  Two workgroups of four wavefronts run on
+// a unit, and one takes some 4 us a tile: with few heads and keys most of the chip is idle meanwhile.  The merge is a launch of 3 to
+// 4 us, so a share has to save at least two tiles.  The whole operator, forward, us, without and with shares, 64 dims f16 / 128 dims
+// bf16, heads x rows x cached keys:  2 x 384 x 1000 (2 shares) 57.7 49.3 / 55.2 48.4   2 x 1024 x 1000 (8) 64.8 48.8 / 68.9 49.6
+//   3 x 300 x 8000 (3) 59.7 54.1 / 63.5 58.2   8 x 1000 x 4095 (3) 80.1 71.0 / 82.6 76.9   32 x 900 x 500 (2) 85.1 80.8 / 84.4 81.0
+int dense_row_shares(int64_t B, int64_t H, int64_t n_ctx, int64_t n_kv, int cus) {
+    const int64_t wgs = (n_kv + 255) / 256 * B * H, tiles = (n_ctx + kQT2 - 1) / kQT2;
+    if (B * H > 65535) return 1;
+    const int64_t shares = std::min<int64_t>(2 * (int64_t)cus / wgs, tiles);
+    return shares > 1 && tiles - (tiles + shares - 1) / shares >= 2 ? (int)shares : 1;
 }
 
 int64_t mfma_n_pad(int64_t n) { return align_up(n, 256); }

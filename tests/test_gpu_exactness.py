@@ -548,3 +548,26 @@ def test_float32_chunk_of_rows_that_are_not_aligned(D, Q, H, KVH, S):
         results.append(cascade_attention(q, k, v, cache, 0, freq + 0.01, update_cache=False))
     assert torch.equal(q, float32_chunk(Q, D, H, KVH, S, 5)[1]) and q.data_ptr() % 16 != 0
     assert all(torch.equal(a, b) for a, b in zip(*results))
+
+
+@pytest.mark.parametrize("dtype", [BF16, F16])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("Z,H,n_ctx,n_kv", [
+    (1, 1, 385, 385), (1, 2, 384, 100 + 384), (1, 3, 1000, 900 + 1000),   # a share of 128 to 256 rows; blocks of chunk keys have fewer
+    (1, 8, 257, 257), (3, 5, 513, 31 + 513), (1, 16, 900, 7000 + 900)])   # one share of two tiles, and where blocks fill the chip
+def test_dense_score_sums_in_shares_of_the_rows(Z, H, n_ctx, n_kv, D, dtype):
+    """Few blocks of keys share their query tiles out over workgroups, whose sums are added in order."""
+    from cascading_kv_cache_amd import flash_attention as fa
+
+    q, k, v, mask, _ = dense_case(Z, H, n_ctx, n_kv, D, dtype)
+    scale = 0.5 if D == 64 else 0.1
+    _, scores, _, _ = fa._forward(q, k, v, True, scale, mask, 0.9, False)
+    _, p, _, _ = exact_attention(q, k, v, visible(n_ctx, n_kv, mask), scale)
+    w = (0.1 * 0.9 ** torch.arange(n_ctx - 1, -1, -1, device="cuda", dtype=torch.float64))[None, None, :, None]
+    want = (w * p).sum(2)
+    if D == 64:
+        assert_rounded_once(scores, want, (w * p).square().sum(2).sqrt(), n_ctx, "scores")
+    else:   # the staged queries are rounded, logits of some 8 are off by 2^-8 (2^-11) of that, and a score by as much
+        assert (scores.double() - want).norm() <= 8 * HALF_ULP[dtype] * want.norm()
+    hidden = torch.cat((mask, torch.zeros(n_ctx, dtype=torch.bool, device="cuda")))
+    assert (scores[:, :, hidden] == 0).all()
