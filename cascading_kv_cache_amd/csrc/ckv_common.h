@@ -66,6 +66,7 @@ struct Elem<__half> {
 // stage timing hooks (ckv_profile_enable / ckv_profile_read); no-ops while disabled
 void prof_begin(int stage, hipStream_t stream);
 void prof_end(int stage, hipStream_t stream);
+void prof_empty(int stage);   // counted, of no length
 // Timing of a single kernel by events attached to its own dispatch (hipExtLaunchKernelGGL): unlike an
 // event record in the stream, this puts nothing between the kernel and its neighbours.  Used when only
 // the attention main kernels are timed.
