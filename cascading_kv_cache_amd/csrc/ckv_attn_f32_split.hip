@@ -941,7 +941,6 @@ bool f32_split_supported(int dtype, int64_t B, int64_t H, int64_t KVH, int64_t Q
 }
 
 int64_t f32_split_plane_bytes(int64_t units, int64_t rows, int64_t D) { return units * ((rows + 31) / 32) * 32 * D * 2 * kPlanes; }
-int64_t f32_split_vis_bytes(int64_t n) { return (n + kKeys - 1) / kKeys * 4; }
 
 int launch_f32_split(const ckv_attn_args& a, const CoreProblem& p, const F32Planes& f, float* w_ema, float* w_new, float2* norm,
                      float* part_o, float2* part_l, hipStream_t stream) {

@@ -46,7 +46,7 @@ int launch_f32_mfma(const CoreProblem& p, hipStream_t stream);
 
 // ckv_attn in float32, head_dim 64 and 128, on the bfloat16 matrix cores: staging, attention and score sums.  The staged operands, in
 // tiles of 32 rows, three planes each (f32_split_plane_bytes): queries (B, H), keys and values (B, KVH); a word per 32 keys,
-// a bit for each that is there and not masked (f32_split_vis_bytes).
+// a bit for each that is there and not masked.
 struct F32Planes {
     void *q, *k, *v;
     uint32_t* vis;
@@ -56,7 +56,6 @@ struct F32Planes {
 bool f32_split_supported(int dtype, int64_t B, int64_t H, int64_t KVH, int64_t Q, int64_t n, int64_t D);
 int f32_split_shares(int64_t B, int64_t H, int64_t KVH, int64_t Q, int64_t n, int cus);
 int64_t f32_split_plane_bytes(int64_t units, int64_t rows, int64_t D);
-int64_t f32_split_vis_bytes(int64_t n);
 // `p`: sizes, out, lse (null: not wanted), colsum and the weights; its operands are not read.  norm: scratch, B*H*Q pairs.  part_o / part_l: f32_split_shares shares of
 // (B*H*Q, D) floats / (B*H*Q) pairs, or null (then the keys of a row tile are not shared out).
 int launch_f32_split(const ckv_attn_args& a, const CoreProblem& p, const F32Planes& f, float* w_ema, float* w_new, float2* norm,
