@@ -116,10 +116,15 @@ struct DecodeParams {
     // of the new token (`tiles - 1`) when it is not one of them.  A cache that is still filling is mostly hidden.
     int tiles_pre;
     int n_vis;         // tiles_pre, or tiles_pre + 1
-    // The cache update in the launch behind the streaming kernel, see TokenPlan; plans null: it is not done there.
-    ckv_update_args u;
-    int32_t* plans;    // [B * KVH][kPlanWords]
+    int32_t* plans;    // [B * KVH][kPlanWords], see TokenPlan; null: the cache update is not done in the launch behind the streaming kernel
 };
+// What the kernels of a step with an update get.  The others do without: a kernel with 600 bytes more of arguments takes half a
+// microsecond longer to start.
+struct DecodePlanParams : DecodeParams {
+    ckv_update_args u;
+};
+template <bool kPlan>
+using StepParams = std::conditional_t<kPlan, DecodePlanParams, DecodeParams>;
 
 // The update of a decoding step beside its scores.  Where the token and the rows it displaces may land, and the trackers after
 // the call, hang on the trackers alone (TokenPath), so a wavefront of the streaming kernel works them out, a (batch, kv head)
@@ -808,13 +813,13 @@ struct StreamPlanner {
         const int u = p.stream_wgs - 1 - (int)blockIdx.x;
         unit = p.plans && wave == kStreamWaves - 1 && u < p.nbh ? u : -1;
     }
-    __device__ inline void request(const DecodeParams& p, int lane) {
+    __device__ inline void request(const DecodePlanParams& p, int lane) {
         if (unit < 0) return;
         const uint32_t n = (uint32_t)unit / (uint32_t)p.a.KVH;
         t.request(p.u, n, (int64_t)((uint32_t)unit - n * (uint32_t)p.a.KVH), 0, lane);
     }
     __device__ inline void arrived() { asm volatile("" : "+v"(t.st), "+v"(t.sx), "+v"(t.per), "+v"(t.sinks), "+v"(t.index)); }
-    __device__ inline void work_out(const DecodeParams& p, int lane) {
+    __device__ inline void work_out(const DecodePlanParams& p, int lane) {
         if (unit >= 0) plan.of(token_path(p.u, t, lane), t, lane);
     }
     __device__ inline void store(const DecodeParams& p, int lane) const {
@@ -951,7 +956,7 @@ struct StreamRows {
 };
 
 template <typename T, int G, bool kPlan>
-__global__ void __launch_bounds__(kStreamThreads, kStreamWgPerCu) decode_stream_kernel(DecodeParams p) {
+__global__ void __launch_bounds__(kStreamThreads, kStreamWgPerCu) decode_stream_kernel(StepParams<kPlan> p) {
     extern __shared__ __align__(16) unsigned char smem[];
     const uint32_t lds_base = lds_address(smem);
     const ckv_attn_args& a = p.a;
@@ -1272,7 +1277,7 @@ __device__ inline void wait_vm(int n, bool lds_too) {  // s_waitcnt vmcnt(n) [lg
 }
 
 template <typename T, int G, bool kPlan>
-__global__ void __launch_bounds__(kStreamThreads, kStreamWgPerCu) decode_stream_wide_kernel(DecodeParams p) {
+__global__ void __launch_bounds__(kStreamThreads, kStreamWgPerCu) decode_stream_wide_kernel(StepParams<kPlan> p) {
     static_assert(G > 4 && G <= 8, "the query block and the logit planes hold 8 heads");
     extern __shared__ __align__(16) unsigned char smem[];
     const uint32_t lds_base = lds_address(smem);
@@ -1673,7 +1678,7 @@ __device__ inline void tail_stream_row(const DecodeParams& p, int row, TailLds& 
 // The position ids of kPosSlots slots of a (b, kvh) from its TokenPlan, by a workgroup of 512 threads; `id`: unit * blocks + block.
 constexpr int kPosSlots = 4096;
 __host__ __device__ inline int pos_blocks(int64_t S) { return (int)((S + kPosSlots - 1) / kPosSlots); }
-__device__ inline void token_positions(const DecodeParams& p, int id, PosRange* ranges) {
+__device__ inline void token_positions(const DecodePlanParams& p, int id, PosRange* ranges) {
     const ckv_update_args& A = p.u;
     const uint32_t W = (uint32_t)A.window_size, S = (uint32_t)A.max_seq_len, tid = threadIdx.x, KVH = (uint32_t)p.a.KVH;
     const uint32_t blocks = (uint32_t)pos_blocks(S), unit = (uint32_t)id / blocks, first = ((uint32_t)id - unit * blocks) * kPosSlots;
@@ -1993,7 +1998,7 @@ struct TokenUpdate {
     bool wanted, seen;
     static constexpr int kTrackerGroup = 31;   // a group of 16 lanes that no path reaches: two cascades a lane
 
-    __device__ inline void request(const DecodeParams& p, int unit, int b, int kvh) {
+    __device__ inline void request(const DecodePlanParams& p, int unit, int b, int kvh) {
         const ckv_update_args& A = p.u;
         const int tid = threadIdx.x, lane = tid & 63, j = tid >> 4, piece = tid & 15;
         const int32_t* words = p.plans + unit * kPlanWords;
@@ -2036,7 +2041,7 @@ struct TokenUpdate {
     }
 
     // sh_score: what the slots of the path are to hold, sh_head: their number and whether the last one keeps its row
-    __device__ inline void decide(const DecodeParams& p, float w_one, float beta_pow, const float* sh_lse, uint16_t* sh_score, int* sh_count) {
+    __device__ inline void decide(const DecodePlanParams& p, float w_one, float beta_pow, const float* sh_lse, uint16_t* sh_score, int* sh_count) {
         const int lane = threadIdx.x & 63, stop = head & 255;
         float c[G], ev[G];
 #pragma unroll
@@ -2062,7 +2067,7 @@ struct TokenUpdate {
         if (lane == 0) *sh_count = (head & TokenPlan::kSink) ? 1 : __builtin_popcountll(moved);
     }
 
-    __device__ inline void commit(const DecodeParams& p, int b, int kvh, const uint16_t* sh_score, int count) {
+    __device__ inline void commit(const DecodePlanParams& p, int b, int kvh, const uint16_t* sh_score, int count) {
         const ckv_update_args& A = p.u;
         const int tid = threadIdx.x, j = tid >> 4, piece = tid & 15, stop = head & 255;
         const bool sink = (head & TokenPlan::kSink) != 0;
@@ -2115,9 +2120,12 @@ struct TokenUpdate {
 // sinks 8 x 32 K (832) 218.0 215.1, 12 x 16 K (864) 170.1 168.7, 16 x 32 K 412.7 416.6: it is at four.  (Position ids by the
 // workgroups of the scores: 64 K slots 66.0; a launch for the rows and the ids, then one for scores and update: 16 x 32 K 417;
 // no more than 80 registers, for a workgroup more a compute unit: level.)
-inline int64_t finish_workgroups_per_cu(int64_t num_sink) { return num_sink % 8 == 0 ? 4 : 8; }
+// More than four heads per kv head: two workgroups a compute unit are all that run at once and the scores of a key are longer, so the line
+// is at one round, and the update comes along only where its workgroups are part of it (10 streams x 16 K slots, 28 heads on 4, median:
+// rows, scores and update 21.4 us in one launch of 720 workgroups, 13.2 + 6.8 apart; mean 16.0 and 9.0 + 7.4).
+inline int64_t finish_workgroups_per_cu(int64_t num_sink, int G) { return G > 4 ? 2 : num_sink % 8 == 0 ? 4 : 8; }
 template <typename T, int G, bool kUpdate>
-__global__ void __launch_bounds__(512) decode_finish_kernel(DecodeParams p, float w_one, float beta_pow, int per_unit) {
+__global__ void __launch_bounds__(512) decode_finish_kernel(StepParams<kUpdate> p, float w_one, float beta_pow, int per_unit) {
     __shared__ TailLds sh;
     const ckv_attn_args& a = p.a;
     const int tid = threadIdx.x, KVH = (int)a.KVH;
@@ -2145,9 +2153,11 @@ __global__ void __launch_bounds__(512) decode_finish_kernel(DecodeParams p, floa
         return;
     }
     id -= rows;
-    if (kUpdate && id >= p.nbh * per_unit) {
-        token_positions(p, id - p.nbh * per_unit, reinterpret_cast<PosRange*>(&sh));
-        return;
+    if constexpr (kUpdate) {
+        if (id >= p.nbh * per_unit) {
+            token_positions(p, id - p.nbh * per_unit, reinterpret_cast<PosRange*>(&sh));
+            return;
+        }
     }
     const int unit = (int)((uint32_t)id / (uint32_t)per_unit), part = id - unit * per_unit;
     const int b = (int)((uint32_t)unit / (uint32_t)KVH), kvh = unit - b * KVH;
@@ -2254,8 +2264,9 @@ __global__ void __launch_bounds__(kSK) decode_scores_homo_kernel(DecodeParams p,
 
 // *updated: the update that p.plans asks for has been launched too
 template <typename T, int G>
-int run_decode(const DecodeParams& p_in, hipStream_t stream, bool* updated) {
-    DecodeParams p = p_in;
+int run_decode(const DecodePlanParams& p_in, hipStream_t stream, bool* updated) {
+    DecodePlanParams with_update = p_in;
+    DecodeParams& p = with_update;
     const ckv_attn_args& a = p.a;
     *updated = false;
     const bool use_stream =
@@ -2277,7 +2288,9 @@ int run_decode(const DecodeParams& p_in, hipStream_t stream, bool* updated) {
         DeviceInfo di;
         if (int rc = current_device_info(&di)) return rc;
         finish_blocks = a.B * a.H + a.B * a.KVH * ((p.Np / 8 + 511) / 512);
-        if (finish_blocks > finish_workgroups_per_cu(a.num_sink) * (int64_t)di.cus) finish_blocks = 0;
+        const int64_t line = finish_workgroups_per_cu(a.num_sink, G) * (int64_t)di.cus;
+        if (finish_blocks > line) finish_blocks = 0;
+        if (G > 4 && finish_blocks + a.B * a.KVH * (1 + pos_blocks(a.S)) > line) p.plans = nullptr;
     }
     p.inv_h = (uint32_t)((65536 + a.H - 1) / a.H);
     {
@@ -2315,14 +2328,18 @@ int run_decode(const DecodeParams& p_in, hipStream_t stream, bool* updated) {
                 prof_kernel_events(CKV_STAGE_DECODE, &ev0, &ev1);
                 // The planning wavefront is compiled in only where the step has a plan: skipped by a branch, it still cost the large
                 // launches, which have none, 1.3 % (16 streams x 32 K slots 386.4 -> 391.5 us, the step 412.7 -> 418.2).
-                void (*kernel)(DecodeParams);
-                if constexpr (G <= 4) kernel = p.plans ? decode_stream_kernel<T, G, true> : decode_stream_kernel<T, G, false>;
-                else kernel = p.plans ? decode_stream_wide_kernel<T, G, true> : decode_stream_wide_kernel<T, G, false>;
-                if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(kernel), lds_s)) return rc;
-                if (ev0)
-                    hipExtLaunchKernelGGL(kernel, dim3((unsigned)wgs), dim3(kStreamThreads), (uint32_t)lds_s, stream, ev0, ev1, 0u, p);
-                else
-                    hipLaunchKernelGGL(kernel, dim3((unsigned)wgs), dim3(kStreamThreads), lds_s, stream, p);
+                auto launch = [&](auto* kernel, const auto& params) -> int {
+                    if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(kernel), lds_s)) return rc;
+                    if (ev0)
+                        hipExtLaunchKernelGGL(kernel, dim3((unsigned)wgs), dim3(kStreamThreads), (uint32_t)lds_s, stream, ev0, ev1, 0u, params);
+                    else
+                        hipLaunchKernelGGL(kernel, dim3((unsigned)wgs), dim3(kStreamThreads), lds_s, stream, params);
+                    return CKV_OK;
+                };
+                int rc;
+                if constexpr (G <= 4) rc = p.plans ? launch(decode_stream_kernel<T, G, true>, with_update) : launch(decode_stream_kernel<T, G, false>, p);
+                else rc = p.plans ? launch(decode_stream_wide_kernel<T, G, true>, with_update) : launch(decode_stream_wide_kernel<T, G, false>, p);
+                if (rc) return rc;
             }
         } else {
             if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(decode_main_mfma_kernel<T, G>), lds)) return rc;
@@ -2339,7 +2356,7 @@ int run_decode(const DecodeParams& p_in, hipStream_t stream, bool* updated) {
                 const int64_t per_unit = (p.Np / 8 + 511) / 512, extra = p.plans ? a.B * a.KVH * (1 + pos_blocks(a.S)) : 0;
                 const dim3 grid((unsigned)(finish_blocks + extra));
                 const float w_one = (float)(1.0 - a.beta), beta = (float)a.beta;
-                if (p.plans) hipLaunchKernelGGL((decode_finish_kernel<T, G, true>), grid, dim3(512), 0, stream, p, w_one, beta, (int)per_unit);
+                if (p.plans) hipLaunchKernelGGL((decode_finish_kernel<T, G, true>), grid, dim3(512), 0, stream, with_update, w_one, beta, (int)per_unit);
                 else hipLaunchKernelGGL((decode_finish_kernel<T, G, false>), grid, dim3(512), 0, stream, p, w_one, beta, (int)per_unit);
                 CKV_HIP_TRY(hipGetLastError());
                 *updated = p.plans != nullptr;
@@ -2382,7 +2399,7 @@ int run_decode(const DecodeParams& p_in, hipStream_t stream, bool* updated) {
 }
 
 template <typename T>
-int run_decode_g(const DecodeParams& p, int G, hipStream_t stream, bool* updated) {
+int run_decode_g(const DecodePlanParams& p, int G, hipStream_t stream, bool* updated) {
     switch (G) {
         case 1: return run_decode<T, 1>(p, stream, updated);
         case 2: return run_decode<T, 2>(p, stream, updated);
@@ -2451,7 +2468,7 @@ bool update_beside_scores(const ckv_attn_args& a, const ckv_update_args& u) {
 }
 
 int launch_decode(const ckv_attn_args& a, hipStream_t stream, const ckv_update_args* u, bool* updated) {
-    DecodeParams p;
+    DecodePlanParams p;
     p.a = a;
     p.u = u ? *u : ckv_update_args{};
     p.N = a.num_sink + a.S + 1;
