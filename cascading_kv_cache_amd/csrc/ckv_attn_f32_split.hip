@@ -672,7 +672,7 @@ __global__ void __launch_bounds__(256) fwd_f32_combine_kernel(F32Fwd f) {
     float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
     for (int s = 0; s < f.n_split; s++) {
         const float2 l = f.part_l[s * rows + row];
-        if (l.x == -INFINITY) continue;
+        if (l.x == -INFINITY && l.y == 0.f) continue;   // without a largest logit, but with a sum: a NaN
         const float w = exp2_fast(l.x - M) * l.y;
         if (w == 0.f) continue;
         const float4 v = *reinterpret_cast<const float4*>(f.part_o + (s * rows + row) * D + 4 * d4);

@@ -470,6 +470,21 @@ def test_a_key_that_is_nan_makes_every_row_that_sees_it_nan_however_its_keys_are
     assert torch.isnan(out[:, 4:]).all() and torch.isfinite(out[:, :4].float()).all()
 
 
+@pytest.mark.parametrize("D,dtype", [(64, F32), (128, F32), (64, BF16), (64, F16), (128, BF16), (128, F16)])
+@pytest.mark.parametrize("H,KVH,W,C,filled,Q", [(32, 8, 320, 4, 200, 64), (8, 2, 512, 4, 100, 40)])
+def test_a_share_of_the_keys_with_nothing_but_nan_reaches_its_rows(H, KVH, W, C, filled, Q, D, dtype):
+    """Every cached key is NaN and every key of the chunk finite: they lie in different shares."""
+    from cascading_kv_cache_amd.cascade_attention import cascade_attention
+
+    cache, q, k, v, inv_freq = cascade_case(1, H, KVH, D, 4, W, C, filled, Q, dtype)
+    cache.key_cache[0][:, 1] = NAN
+    cache.sink_keys[0][:, 1] = NAN
+    out, scores = cascade_attention(q, k, v, cache, 0, inv_freq, update_cache=False)
+    G = H // KVH
+    assert torch.isnan(out[:, G:2 * G]).all() and torch.isnan(scores[:, 1]).all()
+    assert torch.isfinite(out[:, :G].float()).all() and torch.isfinite(scores[:, 0].float()).all()
+
+
 @pytest.mark.parametrize("D,dtype", [(128, BF16), (128, F16), (64, F16), (128, F32)])
 @pytest.mark.parametrize("H,KVH,W,C,filled,Q", [(8, 2, 1024, 4, 1000, 128), (32, 8, 1024, 4, 4095, 300), (8, 2, 2048, 8, 3000, 33),
                                                 (7, 1, 64, 2, 90, 40)])
