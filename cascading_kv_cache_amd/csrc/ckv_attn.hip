@@ -20,6 +20,8 @@ struct Carver {
 struct AttnWorkspace {
     void *qr, *kr, *vc;
     unsigned long long* tile_vis;   // float32: a word per 32 keys
+    uint2* odd_kv;                  // see F32Planes
+    uint32_t* odd_q;
     uint8_t* kmasked;
     float *lse, *lse2, *colsum, *w_ema, *w_new, *part_o, *part_l2;
     int64_t bytes;
@@ -36,6 +38,8 @@ AttnWorkspace carve_attn(void* base, int64_t B, int64_t H, int64_t KVH, int64_t 
     w.kr = c.take(rows);
     w.vc = c.take(rows);
     w.tile_vis = (unsigned long long*)c.take(n_pad / 64 * 8);
+    w.odd_kv = split ? (uint2*)c.take(B * KVH * ((N + 31) / 32) * 8) : nullptr;
+    w.odd_q = split ? (uint32_t*)c.take(B * H * ((Q + 31) / 32) * 4) : nullptr;
     w.kmasked = (uint8_t*)c.take(NS + S);
     w.lse = (float*)c.take(B * H * Q * 4);
     w.lse2 = (float*)c.take(split ? B * H * Q * 8 : (B * H * Q + kColSlack) * 4);   // float32: pairs
@@ -192,7 +196,7 @@ static int run_attn(const ckv_attn_args* args, hipStream_t stream, const ckv_upd
         cp.scale = 1.f;  // the staged queries and keys each carry sqrt(scale), rounded in as the eager path does
         cp.dtype = a.dtype;
         if (split) {
-            const F32Planes f{w.qr, w.kr, w.vc, (uint32_t*)w.tile_vis, (int)((a.Q + 31) / 32),
+            const F32Planes f{w.qr, w.kr, w.vc, (uint32_t*)w.tile_vis, w.odd_q, w.odd_kv, (int)((a.Q + 31) / 32),
                               (uint32_t)(reinterpret_cast<char*>(w.w_new) - reinterpret_cast<char*>(w.w_ema))};
             if (!a.lse) cp.lse = nullptr;
             rc = launch_f32_split(a, cp, f, want_scores ? w.w_ema : nullptr, w.w_new, (float2*)w.lse2, w.part_o,

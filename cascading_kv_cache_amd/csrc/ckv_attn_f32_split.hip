@@ -1,6 +1,13 @@
-// float32 attention of cached chunks on the bfloat16 matrix cores, head_dim 64 and 128: every float32 operand is the exact sum of
-// three bfloat16 planes (high, middle, low), and a product is the six of its nine plane products that float32 can tell from zero
-// (the three left out are below 2^-25 of it); all of them are exact and summed in float32.
+// float32 attention of cached chunks on the bfloat16 matrix cores, head_dim 64 and 128: a float32 operand of ordinary size is the
+// exact sum of three bfloat16 planes (high, middle, low), and a product is the six of its nine plane products that float32 can tell from
+// zero (the three left out are below 2^-25 of it); all of them are exact and summed in float32.
+//
+// The low planes of values below 2^-109 would be smaller than any bfloat16 (at 2^-122 a value would keep 12 bits), and those of the largest
+// and of infinite values are no numbers.  A part of a tile with a value that is not zero and below 2^-100, or past 3.38e38, is
+// staged raw: its bits, eleven to a plane, as finite bfloat16 numbers.  Blocks of keys that meet a raw part, and those in which a row has
+// a probability below 2^-100 of its largest (2^-126 for the score sums, which have no planes of it), are worked out by the
+// float32 instruction from the operands put together, with exponentials down to the smallest subnormal number.  What that costs the others (32 heads x 256 rows x 516 + 256 keys x 128): 0.2 us
+// of the forward kernel's 26 and 0.6 of the score kernel's 16.
 //
 // 32 heads x 256 rows x 516 + 256 keys x 128, us: forward 45.8 -> 27.5 (1.2 MB of operands a workgroup from the L2, 16 TB/s in all,
 // and the first pass through the loop's instructions), scores 30.8 -> 18.4 (products and vector work one behind the other: exponentials
@@ -23,8 +30,8 @@
 //            streams then, each with its queries straight from memory.
 //
 // Zero times infinity is NaN, here also where a plane of a finite operand is zero: a block whose logits are not all finite
-// is worked out again by float32 products of the operands put together, and a wavefront whose accumulators are not finite goes
-// over its keys once more, finite values through the matrix pipe and the others where their probability is above zero.
+// is worked out by the float32 instruction too, and a wavefront whose accumulators are not finite goes over its keys once
+// more, finite values through the matrix pipe and the others where their probability is above zero.
 #include "ckv_attn_internal.h"
 
 #include <type_traits>
@@ -58,6 +65,11 @@ struct Geo {
     static constexpr int kTileVec = kPieces * CKV_WAVE, kTile = kTileVec * 16;
     static constexpr int kFwdLds = kTile + kFwdWaves * kRows * kPitch * 4 + 2 * kFwdWaves * kRows * 4;
     static_assert(kFwdLds <= 160 * 1024, "a compute unit's LDS");
+    // A tile's word of F32Planes::odd_*: a field for each wavefront that stages a part of the tile, not zero where its part is raw.
+    static constexpr int kParts = kSteps / 2, kField = 32 / kParts;   // queries and keys: steps c and c + kParts
+    typedef std::conditional_t<kField == 8, uint8_t, uint16_t> Field;
+    __device__ static bool raw_step(uint32_t word, int c) { return (word >> (c % kParts * kField) & 1u) != 0u; }
+    __device__ static bool raw_values(uint32_t word, int ks) { return (word >> (16 * ks) & 1u) != 0u; }
 };
 
 template <int N>
@@ -94,46 +106,51 @@ __device__ inline void split2(float a, float b, uint32_t& h, uint32_t& m, uint32
     m = pack2(ra, rb);
     l = pack2(ra - low_of(m), rb - high_of(m));
 }
-// The same of values that may be infinite, NaN, or finite and rounded to infinity: the high plane is finite where the value is, and where
-// it is not the others are zero.
-__device__ inline float bounded_rest(float x, float& h) {
-    const float r = x - h;
-    if (isfinite(r)) return r;
-    if (!isfinite(x)) return 0.f;
-    h = __uint_as_float(__float_as_uint(x) & 0xffff0000u);
-    return x - h;
-}
-__device__ inline void split2_any(float a, float b, uint32_t& h, uint32_t& m, uint32_t& l) {
-    h = pack2(a, b);
-    float ha = low_of(h), hb = high_of(h);
-    const float ra = bounded_rest(a, ha), rb = bounded_rest(b, hb);
-    h = __float_as_uint(ha) >> 16 | __float_as_uint(hb);
-    m = pack2(ra, rb);
-    l = pack2(ra - low_of(m), rb - high_of(m));
-}
-// eight values' pieces of the three planes; values that round to no finite bfloat16 are left to a branch that no wavefront fetches
-// without one (a wavefront of the staging runs its instructions once: it is bound by fetching them)
-__device__ inline void split8(const float (&x)[8], uint4 (&out)[kPlanes]) {
-    bool odd = false;
-#pragma unroll
-    for (int e = 0; e < 8; e++) odd = odd || !(fabsf(x[e]) < 3.38e38f);
+// Does everything that it was shown fit the planes to the last bit, with room below for the lowest one?  The matrix instruction takes
+// subnormal operands as they are, but the low plane of a value below 2^-109 would need smaller ones still, and the largest
+// finite values round to infinity.  A NaN is NaN in the high plane.
+struct Range {
+    float top = 0.f;
+    uint32_t low = ~0u;   // twice the bits (no sign), less one: zero comes last
+    __device__ inline void show(float x) {
+        top = fmaxf(top, fabsf(x));
+        const uint32_t twice = (__float_as_uint(x) << 1) - 1u;
+        low = twice < low ? twice : low;
+    }
+    __device__ inline bool fits() const { return top < 3.38e38f && low >= 2u * 0x0d800000u - 1u; }   // bits of 2^-100
+};
+// Eleven bits of a value that the planes do not take, as a finite bfloat16: sign, lower exponent and mantissa, the upper exponent being
+// 01111.  Three of them are the 32.
+__device__ inline uint32_t raw_word(uint32_t f) { return (f & 0x400u) << 5 | 0x3c00u | (f & 0x3ffu); }
+__device__ inline uint32_t raw_bits(uint32_t w) { return (w >> 5 & 0x400u) | (w & 0x3ffu); }
+// eight values' pieces of the three planes; `raw` (one for the wavefront): of their bits
+__device__ inline void split8(const float (&x)[8], bool raw, uint4 (&out)[kPlanes]) {
     uint32_t w[kPlanes][4];
-    if (__ballot(odd) == 0ull) {
+    if (__builtin_expect(!raw, 1)) {
 #pragma unroll
         for (int i = 0; i < 4; i++) split2(x[2 * i], x[2 * i + 1], w[0][i], w[1][i], w[2][i]);
     } else {
 #pragma unroll
-        for (int i = 0; i < 4; i++) split2_any(x[2 * i], x[2 * i + 1], w[0][i], w[1][i], w[2][i]);
+        for (int i = 0; i < 4; i++) {
+            const uint32_t a = __float_as_uint(x[2 * i]), b = __float_as_uint(x[2 * i + 1]);
+            w[0][i] = raw_word(a >> 21) | raw_word(b >> 21) << 16;
+            w[1][i] = raw_word(a >> 10) | raw_word(b >> 10) << 16;
+            w[2][i] = raw_word(a & 0x3ffu) | raw_word(b & 0x3ffu) << 16;
+        }
     }
 #pragma unroll
     for (int pl = 0; pl < kPlanes; pl++) out[pl] = make_uint4(w[pl][0], w[pl][1], w[pl][2], w[pl][3]);
 }
 
 __device__ inline uint32_t word_of(const uint4& x, int i) { return i == 0 ? x.x : i == 1 ? x.y : i == 2 ? x.z : x.w; }
-// element e of three planes' pieces, put together
-__device__ inline float whole_of(const uint4 (&x)[kPlanes], int e) {
+// element e of three planes' pieces (raw: of its bits), put together
+__device__ inline float whole_of(const uint4 (&x)[kPlanes], int e, bool raw) {
     const uint32_t h = word_of(x[0], e >> 1), m = word_of(x[1], e >> 1), l = word_of(x[2], e >> 1);
-    return e & 1 ? high_of(h) + (high_of(m) + high_of(l)) : low_of(h) + (low_of(m) + low_of(l));
+    const int at = 16 * (e & 1);
+    const uint32_t bits = raw_bits(h >> at) << 21 | raw_bits(m >> at) << 10 | raw_bits(l >> at);
+    const float sum = e & 1 ? high_of(h) + (high_of(m) + high_of(l)) : low_of(h) + (low_of(m) + low_of(l));
+    const uint32_t pick = raw ? ~0u : 0u;   // no branch: there are sixteen of these behind each other
+    return __uint_as_float((bits & pick) | (__float_as_uint(sum) & ~pick));
 }
 
 // the plane products of one step, the small ones in an accumulator of their own
@@ -148,6 +165,7 @@ __device__ inline void mma_planes(const uint4 (&a)[kPlanes], const uint4 (&b)[kP
 
 // Logits, their maxima and the normalisers between the kernels are to the base 2: the staged queries carry log2 e.
 __device__ inline float exp2_fast(float x) { return __builtin_amdgcn_exp2f(x); }   // results below the smallest normal number are zero
+constexpr float kFaint = -100.f;   // a probability's logit below the largest, from which on its planes would lose bits
 
 // a word that no kernel of this launch writes, at a uniform index
 __device__ inline uint32_t uniform_word(const uint32_t* words, int i) {
@@ -195,7 +213,8 @@ struct KeySource {
 struct F32Stage {
     ckv_attn_args a;
     uint4 *q, *k, *v;       // see F32Planes
-    uint32_t* vis;
+    uint32_t *vis, *odd_q;
+    uint2* odd_kv;
     float *w_ema, *w_new;   // the weights of the score sums, or null
     float post_q, post_k;   // what rotated queries and keys are multiplied by
     int nblk, q_tiles;
@@ -281,9 +300,18 @@ __global__ void __launch_bounds__(256) stage_f32_kernel(F32Stage p) {
             x2[e] = there ? __fmul_rn(r2, post) : 0.f;
         }
         uint4* dst = (key ? p.k : p.q) + (int64_t)tile * G_::kTileVec + lane;
+        Range range;
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            range.show(x1[e]);
+            range.show(x2[e]);
+        }
+        const bool raw = __ballot(!range.fits()) != 0ull;
         uint4 w1[kPlanes], w2[kPlanes];
-        split8(x1, w1);
-        split8(x2, w2);
+        split8(x1, raw, w1);
+        split8(x2, raw, w2);
+        typedef typename G_::Field Field;
+        if (lane == 0) reinterpret_cast<Field*>(key ? &p.odd_kv[tile].x : &p.odd_q[tile])[c] = raw ? 1 : 0;
 #pragma unroll
         for (int pl = 0; pl < kPlanes; pl++) {
             dst[(c * kPlanes + pl) * CKV_WAVE] = w1[pl];
@@ -316,12 +344,20 @@ __global__ void __launch_bounds__(256) stage_f32_kernel(F32Stage p) {
             for (int db = 0; db < DB; db++) x[db][e] = t[db];
         }
         uint4* dst = p.v + (int64_t)tile * G_::kTileVec + lane;
+        Range range;
+#pragma unroll
+        for (int db = 0; db < DB; db++)
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                x[db][e] = seen[e] ? x[db][e] : 0.f;   // a key that nobody sees may hold anything
+                range.show(x[db][e]);
+            }
+        const bool raw = __ballot(!range.fits()) != 0ull;
+        if (lane == 0) reinterpret_cast<uint16_t*>(&p.odd_kv[tile].y)[ks] = raw ? 1 : 0;
 #pragma unroll
         for (int db = 0; db < DB; db++) {
-#pragma unroll
-            for (int e = 0; e < 8; e++) x[db][e] = seen[e] ? x[db][e] : 0.f;   // a key that nobody sees may hold anything
             uint4 w[kPlanes];
-            split8(x[db], w);
+            split8(x[db], raw, w);
 #pragma unroll
             for (int pl = 0; pl < kPlanes; pl++) dst[((db * 2 + ks) * kPlanes + pl) * CKV_WAVE] = w[pl];
         }
@@ -386,13 +422,21 @@ __global__ void __launch_bounds__(kFwdWaves* CKV_WAVE) fwd_f32_split_kernel(F32F
         return vis & (last >= 31 ? ~0u : (last < 0 ? 0u : (2u << last) - 1u));   // cached keys lie in front of the chunk keys: row_m >= 0 lets them all through
     };
     // the wavefront's first block from `blk` on with a visible key
-    uint32_t vis = 0u;
+    const uint32_t* odd_kv = reinterpret_cast<const uint32_t*>(f.f.odd_kv + (int64_t)bkv * all_blocks);
+    uint32_t vis = 0u, odd_k = 0u, odd_v = 0u;
     auto visible_from = [&](int blk) {
         for (vis = 0u; blk < nblk; blk += step) {
             vis = uniform_word(f.f.vis, blk);
+            odd_k = uniform_word(odd_kv, 2 * blk);
+            odd_v = uniform_word(odd_kv, 2 * blk + 1);
             if (vis != 0u) break;
         }
         return blk;
+    };
+    // the word of the tile of this lane's query
+    auto odd_query = [&]() {
+        const int g = rt * kRows + col - row_m * G;
+        return row_m < Q ? f.f.odd_q[(b * p.H + kvh * G + g) * f.f.q_tiles + row_m / 32] : 0u;
     };
     uint4 kf[NS][kPlanes];   // the block's keys
     auto load_keys = [&](int blk, int c0, int c1) {
@@ -418,15 +462,17 @@ __global__ void __launch_bounds__(kFwdWaves* CKV_WAVE) fwd_f32_split_kernel(F32F
             else q_lds[t * CKV_WAVE + lane] = make_uint4(0u, 0u, 0u, 0u);
         }
     }
+    const bool odd_queries = __ballot(odd_query() != 0u) != 0ull;
     int blk = visible_from(blk_first);
     if (vis != 0u && blk != blk_first) load_keys(blk, 0, NS);
     wait_copies<0>();
     __syncthreads();
 
     // the logits of a block's keys (lane = its query) by float32 products, whatever the operands hold
-    auto plain_logits = [&](int blk) {
+    auto plain_logits = [&](int blk, uint32_t odd_k) {
         f32x16 s = zero16();
         const uint4* from = kb + (int64_t)blk * G_::kTileVec;
+        const uint32_t odd_q = odd_query();
 #pragma unroll 1
         for (int c = 0; c < NS; c++) {
             uint4 k[kPlanes], q[kPlanes];
@@ -436,7 +482,7 @@ __global__ void __launch_bounds__(kFwdWaves* CKV_WAVE) fwd_f32_split_kernel(F32F
                 q[pl] = q_lds[(c * kPlanes + pl) * CKV_WAVE + lane];
             }
 #pragma unroll
-            for (int e = 0; e < 8; e++) s = mma32(whole_of(k, e), whole_of(q, e), s);
+            for (int e = 0; e < 8; e++) s = mma32(whole_of(k, e, G_::raw_step(odd_k, c)), whole_of(q, e, G_::raw_step(odd_q, c)), s);
         }
         return s;
     };
@@ -491,16 +537,25 @@ __global__ void __launch_bounds__(kFwdWaves* CKV_WAVE) fwd_f32_split_kernel(F32F
                 for (int pl = 0; pl < kPlanes; pl++) vf[db][ks][pl] = from[((db * 2 + ks) * kPlanes + pl) * CKV_WAVE];
         __builtin_amdgcn_sched_barrier(0);
         const int here = blk;
+        const uint32_t odd_here = odd_k, odd_values = odd_v;
         blk = visible_from(blk + step);
         const uint32_t allow = seen_keys(vis_now, n0);   // bit r: key r of the block is visible to this lane's query
         const bool whole = __ballot(allow != ~0u) == 0ull;
 #pragma unroll
         for (int v = 0; v < 16; v++) s[v] += small[v];
-        float m_new, ref, sum;
-        auto probabilities = [&]() {
+        float m_new, ref, sum, low;
+        auto largest = [&]() {
+            low = INFINITY;   // the smallest logit of a key that the row sees
             if (!whole) {
 #pragma unroll
-                for (int v = 0; v < 16; v++) s[v] = (allow >> acc_row(v, half)) & 1u ? s[v] : -INFINITY;
+                for (int v = 0; v < 16; v++) {
+                    const bool sees = (allow >> acc_row(v, half)) & 1u;
+                    low = fminf(low, sees ? s[v] : INFINITY);
+                    s[v] = sees ? s[v] : -INFINITY;
+                }
+            } else {
+#pragma unroll
+                for (int v = 0; v < 16; v++) low = fminf(low, s[v]);
             }
             float mx = -INFINITY;
 #pragma unroll
@@ -509,18 +564,24 @@ __global__ void __launch_bounds__(kFwdWaves* CKV_WAVE) fwd_f32_split_kernel(F32F
             m_new = fmaxf(m_run, mx);
             ref = m_new == -INFINITY ? 0.f : m_new;   // nothing visible yet: every exponential is 0
             sum = 0.f;
+        };
+        largest();
+#pragma unroll
+        for (int v = 0; v < 16; v++) {
+            s[v] = exp2_fast(s[v] - ref);
+            sum += s[v];
+        }
+        const bool plain = (odd_here | odd_values) != 0u || odd_queries || __ballot(isnan(sum) || low - ref < kFaint) != 0ull;
+        if (__builtin_expect(plain, 0)) {
+            s = plain_logits(here, odd_here);
+            largest();
 #pragma unroll
             for (int v = 0; v < 16; v++) {
-                s[v] = exp2_fast(s[v] - ref);
+                s[v] = exp2f(s[v] - ref);
                 sum += s[v];
             }
-        };
-        probabilities();
-        if (__ballot(isnan(sum)) != 0ull) {
-            s = plain_logits(here);
-            probabilities();
         }
-        const float alpha = m_run == -INFINITY ? 0.f : exp2_fast(m_run - ref);
+        const float alpha = m_run == -INFINITY ? 0.f : exp2f(m_run - ref);
         l_run = l_run * alpha + sum;
         if (__ballot(m_new != m_run) != 0ull) {
 #pragma unroll
@@ -529,6 +590,20 @@ __global__ void __launch_bounds__(kFwdWaves* CKV_WAVE) fwd_f32_split_kernel(F32F
                 for (int v = 0; v < 16; v++) o[db][v] *= alpha;
         }
         m_run = m_new;
+        if (__builtin_expect(plain, 0)) {
+#pragma unroll
+            for (int db = 0; db < DB; db++)
+#pragma unroll
+                for (int ks = 0; ks < 2; ks++) {
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int e = 0; e < 8; e++) o[db] = mma32(whole_of(vf[db][ks], e, G_::raw_values(odd_values, ks)), s[8 * ks + e], o[db]);
+                }
+            __builtin_amdgcn_sched_barrier(0);
+            // The products below add nothing: their operands are finite.  A way around them had the compiler spill 120 registers and more.
+#pragma unroll
+            for (int v = 0; v < 16; v++) s[v] = 0.f;
+        }
         uint4 pb[2][kPlanes];
         split_probabilities(s, pb);
 #pragma unroll
@@ -553,19 +628,10 @@ __global__ void __launch_bounds__(kFwdWaves* CKV_WAVE) fwd_f32_split_kernel(F32F
 #pragma unroll
         for (int db = 0; db < DB; db++) o[db] = zero16();
         for (blk = visible_from(split * kFwdWaves + wave); blk < nblk; blk = visible_from(blk + step)) {
-            f32x16 s = plain_logits(blk);
+            f32x16 s = plain_logits(blk, odd_k);
             const uint32_t allow = seen_keys(vis, blk * kKeys);
 #pragma unroll
             for (int v = 0; v < 16; v++) s[v] = (allow >> acc_row(v, half)) & 1u ? exp2f(s[v] - m_run) : 0.f;
-            uint4 pb[2][kPlanes], counts[2];   // counts: one where the probability is above zero
-            split_probabilities(s, pb);
-#pragma unroll
-            for (int ks = 0; ks < 2; ks++) {
-                uint32_t w[4];
-#pragma unroll
-                for (int i = 0; i < 4; i++) w[i] = pack2(s[8 * ks + 2 * i] > 0.f ? 1.f : 0.f, s[8 * ks + 2 * i + 1] > 0.f ? 1.f : 0.f);
-                counts[ks] = make_uint4(w[0], w[1], w[2], w[3]);
-            }
             const uint4* from = vb + (int64_t)blk * G_::kTileVec;
 #pragma unroll
             for (int db = 0; db < DB; db++) {
@@ -573,23 +639,17 @@ __global__ void __launch_bounds__(kFwdWaves* CKV_WAVE) fwd_f32_split_kernel(F32F
                 bool odd = false;
 #pragma unroll
                 for (int ks = 0; ks < 2; ks++) {
-                    uint4 vf[kPlanes];
+                    uint4 v3[kPlanes];
 #pragma unroll
-                    for (int pl = 0; pl < kPlanes; pl++) vf[pl] = from[((db * 2 + ks) * kPlanes + pl) * CKV_WAVE];
-                    uint32_t clean[4], rising[4], falling[4];
+                    for (int pl = 0; pl < kPlanes; pl++) v3[pl] = from[((db * 2 + ks) * kPlanes + pl) * CKV_WAVE];
 #pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        const uint32_t w = word_of(vf[0], i);
-                        const float x[2] = {low_of(w), high_of(w)};
-                        odd = odd || !isfinite(x[0]) || !isfinite(x[1]);
-                        clean[i] = (isfinite(x[0]) ? w & 0xffffu : 0u) | (isfinite(x[1]) ? w & 0xffff0000u : 0u);
-                        rising[i] = pack2(x[0] == INFINITY || isnan(x[0]) ? 1.f : 0.f, x[1] == INFINITY || isnan(x[1]) ? 1.f : 0.f);
-                        falling[i] = pack2(x[0] == -INFINITY || isnan(x[0]) ? 1.f : 0.f, x[1] == -INFINITY || isnan(x[1]) ? 1.f : 0.f);
+                    for (int e = 0; e < 8; e++) {
+                        const float x = whole_of(v3, e, G_::raw_values(odd_v, ks)), counts = s[8 * ks + e] > 0.f ? 1.f : 0.f;
+                        odd = odd || !isfinite(x);
+                        o[db] = mma32(isfinite(x) ? x : 0.f, s[8 * ks + e], o[db]);
+                        up = mma32(x == INFINITY || isnan(x) ? 1.f : 0.f, counts, up);
+                        down = mma32(x == -INFINITY || isnan(x) ? 1.f : 0.f, counts, down);
                     }
-                    vf[0] = make_uint4(clean[0], clean[1], clean[2], clean[3]);
-                    o[db] = mma_values(vf, pb[ks], o[db]);
-                    up = mma(make_uint4(rising[0], rising[1], rising[2], rising[3]), counts[ks], up);
-                    down = mma(make_uint4(falling[0], falling[1], falling[2], falling[3]), counts[ks], down);
                 }
                 if (__ballot(odd) == 0ull) continue;
 #pragma unroll
@@ -609,7 +669,7 @@ __global__ void __launch_bounds__(kFwdWaves* CKV_WAVE) fwd_f32_split_kernel(F32F
         float M = -INFINITY;
 #pragma unroll
         for (int w = 0; w < kFwdWaves; w++) M = fmaxf(M, ml_lds[w * kRows + col]);
-        const float sc = m_run == -INFINITY ? 0.f : exp2_fast(m_run - M);
+        const float sc = m_run == -INFINITY ? 0.f : exp2f(m_run - M);
         float* ow = o_lds + (wave * kRows + col) * G_::kPitch;
 #pragma unroll
         for (int v = 0; v < 16; v++) {
@@ -631,7 +691,7 @@ __global__ void __launch_bounds__(kFwdWaves* CKV_WAVE) fwd_f32_split_kernel(F32F
 #pragma unroll
     for (int w = 0; w < kFwdWaves; w++) {
         const float mw = ml_lds[w * kRows + r], lw = ml_lds[(kFwdWaves + w) * kRows + r];
-        const float sc = mw == -INFINITY ? 1.f : exp2_fast(mw - M);   // no largest logit but a sum: a NaN
+        const float sc = mw == -INFINITY ? 1.f : exp2f(mw - M);   // no largest logit but a sum: a NaN
         L = lw != 0.f ? fmaf(lw, sc, L) : L;
     }
     float acc[kPer];
@@ -673,7 +733,7 @@ __global__ void __launch_bounds__(256) fwd_f32_combine_kernel(F32Fwd f) {
     for (int s = 0; s < f.n_split; s++) {
         const float2 l = f.part_l[s * rows + row];
         if (l.x == -INFINITY && l.y == 0.f) continue;   // without a largest logit, but with a sum: a NaN
-        const float w = exp2_fast(l.x - M) * l.y;
+        const float w = exp2f(l.x - M) * l.y;
         if (w == 0.f) continue;
         const float4 v = *reinterpret_cast<const float4*>(f.part_o + (s * rows + row) * D + 4 * d4);
         L += w;
@@ -725,6 +785,11 @@ __global__ void __launch_bounds__(Col<kGroups>::kWaves* CKV_WAVE, 2) colsum_f32_
         }
     };
     if (t_first < n_tiles) copy_stage(t_first, 0);
+    // not zero in some lane: a part of the block's keys or of some tile's queries is raw
+    const uint32_t* odd_key = reinterpret_cast<const uint32_t*>(f.odd_kv + (int64_t)bkv * all_blocks + block);
+    const uint32_t* odd_queries = f.odd_q + (b * p.H + h) * f.q_tiles;
+    uint32_t odd = *odd_key;
+    for (int i = lane; i < n_tiles; i += CKV_WAVE) odd |= odd_queries[i];
     const uint32_t vis = n0 / kKeys < all_blocks ? uniform_word(f.vis, block) : 0u;
     uint4 kf[NS][kPlanes];
     const uint4* kfrom = (const uint4*)f.k + ((int64_t)bkv * all_blocks + block) * G_::kTileVec + lane;
@@ -740,8 +805,9 @@ __global__ void __launch_bounds__(Col<kGroups>::kWaves* CKV_WAVE, 2) colsum_f32_
     float top[16], inv[16], w[16];
     const int weight_back = by_distance ? nrel : 0;
     const uint32_t weight_at = by_distance ? f.w_new_at : 0u;
+    auto all_see = [&](int t) { return t * kRows + kRows <= Q && t * kRows >= n0 + kKeys - 1 - Nc; };   // all rows of a tile, every key
     auto request_rows = [&](int t) {
-        if (t * kRows + kRows <= Q && t * kRows >= n0 + kKeys - 1 - Nc) {
+        if (all_see(t)) {
 #pragma unroll
             for (int i4 = 0; i4 < 4; i4++) {
                 const int m0 = t * kRows + 8 * i4 + 4 * half;
@@ -772,6 +838,7 @@ __global__ void __launch_bounds__(Col<kGroups>::kWaves* CKV_WAVE, 2) colsum_f32_
     };
     auto plain_logits = [&](int t, int stage) {   // by float32 products, whatever the operands hold
         f32x16 s = zero16();
+        const uint32_t odd_q = odd_queries[t], odd_k = *odd_key;
 #pragma unroll 1
         for (int c = 0; c < NS; c++) {
             uint4 q3[kPlanes], k3[kPlanes];
@@ -781,7 +848,7 @@ __global__ void __launch_bounds__(Col<kGroups>::kWaves* CKV_WAVE, 2) colsum_f32_
                 k3[pl] = kfrom[(c * kPlanes + pl) * CKV_WAVE];
             }
 #pragma unroll
-            for (int e = 0; e < 8; e++) s = mma32(whole_of(q3, e), whole_of(k3, e), s);
+            for (int e = 0; e < 8; e++) s = mma32(whole_of(q3, e, G_::raw_step(odd_q, c)), whole_of(k3, e, G_::raw_step(odd_k, c)), s);
         }
 #pragma unroll
         for (int v = 0; v < 16; v++) {   // a row that does not see the key may hold anything
@@ -814,16 +881,22 @@ __global__ void __launch_bounds__(Col<kGroups>::kWaves* CKV_WAVE, 2) colsum_f32_
         for (int v = 0; v < 16; v++) s[v] += small[v];
         const bool second = kAcc == 2 && ((t - t_own) & 2);
         const float before = second ? acc[kAcc - 1] : acc[0];
-        auto add_tile = [&]() {
-            float a = before;
+        float a = before, low = 0.f;   // the smallest logit of a row that sees the key, less the row's largest
+        if (all_see(t)) {
 #pragma unroll
-            for (int v = 0; v < 16; v++) a = fmaf(w[v] * inv[v], exp2_fast(s[v] - top[v]), a);
-            return a;
-        };
-        float a = add_tile();
-        if (__ballot(live && !isfinite(a)) != 0ull) {   // a key that nobody sees may come out as anything
+            for (int v = 0; v < 16; v++) low = fminf(low, s[v] - top[v]);
+        } else {
+#pragma unroll
+            for (int v = 0; v < 16; v++) low = fminf(low, top[v] == INFINITY ? 0.f : s[v] - top[v]);
+        }
+#pragma unroll
+        for (int v = 0; v < 16; v++) a = fmaf(w[v] * inv[v], exp2_fast(s[v] - top[v]), a);
+        // a key that nobody sees may come out as anything
+        if (__builtin_expect(__ballot(odd != 0u || (live && (!isfinite(a) || low < -126.f))) != 0ull, 0)) {
             s = plain_logits(t, stage);
-            a = add_tile();
+            a = before;
+#pragma unroll
+            for (int v = 0; v < 16; v++) a = fmaf(w[v] * inv[v], exp2f(s[v] - top[v]), a);
         }
         if (second) acc[kAcc - 1] = a;
         else acc[0] = a;
@@ -860,6 +933,8 @@ int run(const ckv_attn_args& a, const CoreProblem& p, const F32Planes& f, float*
         st.k = (uint4*)f.k;
         st.v = (uint4*)f.v;
         st.vis = f.vis;
+        st.odd_kv = f.odd_kv;
+        st.odd_q = f.odd_q;
         st.w_ema = w_ema;
         st.w_new = w_new;
         // on queries and keys: nothing is multiplied behind the products

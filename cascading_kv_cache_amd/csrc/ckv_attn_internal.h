@@ -46,10 +46,12 @@ int launch_f32_mfma(const CoreProblem& p, hipStream_t stream);
 
 // ckv_attn in float32, head_dim 64 and 128, on the bfloat16 matrix cores: staging, attention and score sums.  The staged operands, in
 // tiles of 32 rows, three planes each (f32_split_plane_bytes): queries (B, H), keys and values (B, KVH); a word per 32 keys,
-// a bit for each that is there and not masked.
+// a bit for each that is there and not masked; of every tile, which parts hold values that three planes do not take (odd_kv: keys and
+// values; odd_q).
 struct F32Planes {
     void *q, *k, *v;
-    uint32_t* vis;
+    uint32_t *vis, *odd_q;
+    uint2* odd_kv;
     int q_tiles;         // of a head
     uint32_t w_new_at;   // bytes from the weights w_ema to w_new, which lie behind them
 };

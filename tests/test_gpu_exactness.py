@@ -551,6 +551,82 @@ def test_float32_chunk_of_values_that_three_planes_do_not_take(D, Q, H, KVH, S):
     assert torch.isnan(scores[0, 0, :8]).all() and (KVH == 1 or torch.isfinite(scores[0, -1, 10:]).all())   # rows 7 and 9
 
 
+def ema_scores(p, beta, G):
+    """What a chunk adds to the scores of the keys in front of it, in float64: the weighted sums over its rows, averaged over a kv head's."""
+    Q = p.size(2)
+    w = (1 - beta) * beta ** torch.arange(Q - 1, -1, -1, device=p.device, dtype=torch.float64)
+    sums = (p * w[:, None]).sum(2)
+    return sums.reshape(p.size(0), -1, G, sums.size(-1)).mean(2)
+
+
+@pytest.mark.parametrize("octaves", [-112, -122])
+@pytest.mark.parametrize("B,H,KVH,D,NS,W,C,filled,Q", [(1, 32, 8, 128, 4, 128, 4, 400, 96), (1, 8, 2, 128, 4, 512, 4, 2000, 40),
+                                                       (2, 7, 1, 64, 3, 90, 2, 100, 33), (1, 8, 2, 64, 4, 512, 4, 1500, 70)])
+def test_float32_chunk_of_operands_far_below_one(B, H, KVH, D, NS, W, C, filled, Q, octaves):
+    """Values, and keys against queries as far above one, of which the lowest of three bfloat16 planes would be no number
+    or half of one: no bits are lost."""
+    from cascading_kv_cache_amd.cascade_attention import cascade_attention
+
+    cache, q, k, v, inv_freq = cascade_case(B, H, KVH, D, NS, W, C, filled, Q, F32)
+    cache.beta = 0.9
+    small = 2.0 ** octaves
+    qs, ks, vs, mask = staged(cache, q, k, v)
+    see = visible(Q, ks.size(2), mask)
+    before = cache.score_cache[0].clone()
+    # values
+    cache.value_cache[0].mul_(small)
+    cache.sink_values[0].mul_(small)
+    ref, p, _, spread = exact_attention(qs, ks, vs, see, 1.0)
+    out, scores = cascade_attention(q, k, v * small, cache, 0, inv_freq, update_cache=False)
+    assert_rounded_once(out * 2.0 ** -octaves, ref, spread, ks.size(2), "small values")
+    want = cache.beta ** Q * before.double() + ema_scores(p, cache.beta, H // KVH)[..., NS:-Q]
+    seen = ~mask[NS:]
+    assert ((cache.score_cache[0].double() - want).abs()[..., seen] <= 2.0 ** -17 * want[..., seen]).all()
+    # keys, and queries the other way
+    cache.value_cache[0].mul_(1 / small)
+    cache.sink_values[0].mul_(1 / small)
+    cache.score_cache[0].copy_(before)
+    for t in (cache.key_cache[0], cache.sink_keys[0]):
+        t.mul_(small)
+    out2, scores2 = cascade_attention(q / small, k * small, v, cache, 0, inv_freq, update_cache=False)
+    assert_rounded_once(out2, ref, spread, ks.size(2), "small keys")
+    assert ((cache.score_cache[0].double() - want).abs()[..., seen] <= 2.0 ** -17 * want[..., seen]).all()
+    assert ((scores2 - scores).abs() <= 2.0 ** -17 * scores).all()
+
+
+@pytest.mark.parametrize("octaves", [-104, -130])
+@pytest.mark.parametrize("H,KVH,D,NS,W,C,filled,Q", [(32, 8, 128, 4, 128, 4, 400, 96), (8, 2, 128, 4, 512, 4, 2000, 40), (7, 1, 64, 3, 90, 2, 100, 33)])
+def test_float32_chunk_of_faint_probabilities(H, KVH, D, NS, W, C, filled, Q, octaves):
+    """A sink that takes all but 2^-104 (2^-130: less than the smallest normal number) of every row, and whose value is zero: what is left
+    of the row is sums of the others."""
+    from cascading_kv_cache_amd.cascade_attention import cascade_attention
+
+    cache, q, k, v, inv_freq = cascade_case(1, H, KVH, D, NS, W, C, filled, Q, F32)
+    cache.beta = 0.5
+    rs = math.sqrt(1 / math.sqrt(D))
+    q[..., 0] = 1.0 / rs
+    for t in (k, cache.key_cache[0], cache.sink_keys[0]):
+        t[..., 0] = 0.0
+    cache.sink_keys[0][:, :, 0] = 0.0
+    cache.sink_keys[0][:, :, 0, 0] = -octaves * math.log(2.0) / rs
+    cache.sink_values[0][:, :, 0] = 0.0
+    cache.score_cache[0].zero_()
+    qs, ks, vs, mask = staged(cache, q, k, v)
+    see = visible(Q, ks.size(2), mask)
+    logits = torch.matmul(qs.double(), ks.double().transpose(2, 3).contiguous()).masked_fill(~see, float("-inf"))
+    p = (logits - logits.amax(-1, keepdim=True)).exp()   # torch's softmax on the device has zeros below 2^-126
+    p /= p.sum(-1, keepdim=True)
+    ref, spread = torch.matmul(p, vs.double()), torch.matmul(p * p, vs.double() ** 2).sqrt()
+    assert (ref != 0).all()
+    out, _ = cascade_attention(q, k, v, cache, 0, inv_freq, update_cache=False)
+    # a logit of 90 is off by 2^-18 or so, and a subnormal of 2^-130 holds 19 bits
+    bound = 2.0 ** -15 * (ref.abs() + spread) + 2.0 ** -147
+    assert ((out.double() - ref).abs() <= bound).all()
+    want = ema_scores(p, cache.beta, H // KVH)[..., NS:-Q]
+    seen = ~mask[NS:]
+    assert ((cache.score_cache[0].double() - want).abs()[..., seen] <= 2.0 ** -15 * want[..., seen] + Q * 2.0 ** -149).all()
+
+
 @pytest.mark.parametrize("D,Q,H,KVH,S", [(128, 65, 4, 2, 64), (64, 40, 7, 1, 30)])
 def test_float32_chunk_of_rows_that_are_not_aligned(D, Q, H, KVH, S):
     """Rows that start at any element are staged element by element: the same result to the bit."""
