@@ -8,6 +8,7 @@ There is no CPU path: tensors must live on a HIP device and the library must be 
 """
 import contextlib
 import ctypes as C
+import threading
 from typing import List, Optional, Union
 
 import torch
@@ -19,17 +20,24 @@ _WORKSPACES = {}
 
 
 _COUNTER_TABLES = {}
+_COUNTER_LOCK = threading.Lock()
 COUNTER_TABLE_ENTRIES = 1 << 21
 
 
-def _counter_table(device) -> Tensor:
-    """``0, 1, 2, ...`` as int64 on ``device`` (16 MiB, built once): element n is a device-resident n."""
+def _counter_table(device) -> Optional[Tensor]:
+    """``0, 1, 2, ...`` as int64 on ``device`` (16 MiB, built once): element n is a device-resident n.  Every stream and
+    thread reads it without looking at who built it, so the stream that does is waited for.  None while the current stream is
+    being captured and there is no table: it would be filled by the replays."""
     device = torch.device(device)
     key = (device.type, device.index if device.index is not None else torch.cuda.current_device())
     t = _COUNTER_TABLES.get(key)
-    if t is None:
-        t = torch.arange(COUNTER_TABLE_ENTRIES, dtype=torch.long, device=device)
-        _COUNTER_TABLES[key] = t
+    if t is None and not torch.cuda.is_current_stream_capturing():
+        with _COUNTER_LOCK:
+            t = _COUNTER_TABLES.get(key)
+            if t is None:
+                t = torch.arange(COUNTER_TABLE_ENTRIES, dtype=torch.long, device=device)
+                torch.cuda.current_stream(device).synchronize()
+                _COUNTER_TABLES[key] = t
     return t
 
 

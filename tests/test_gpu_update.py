@@ -260,6 +260,23 @@ def test_token_counter_by_table_and_by_device_counter():
     assert_same_state(gpu, cpu, "back on the table")
 
 
+def test_token_counter_table_is_whole_on_every_stream(monkeypatch):
+    """The table is built on a stream with work in front of it; a stream that knows nothing of that one reads it at once."""
+    from cascading_kv_cache_amd import cascading_cache as cc
+
+    torch.full((cc.COUNTER_TABLE_ENTRIES,), -1, dtype=torch.long, device="cuda:0")   # what the memory holds before
+    first, second = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    monkeypatch.setattr(cc, "_COUNTER_TABLES", {})
+    with torch.cuda.stream(first):
+        torch.cuda._sleep(100_000_000)
+        table = cc._counter_table("cuda:0")
+    with torch.cuda.stream(second):
+        seen = table.clone()
+    torch.cuda.synchronize()
+    assert torch.equal(seen, torch.arange(cc.COUNTER_TABLE_ENTRIES, device="cuda:0"))
+
+
 @pytest.mark.parametrize("B,H,D,NS,W,C,dtype,func,eager", [
     (1, 2, 16, 4, 3, 5, torch.bfloat16, "pow2", True),      # odd windows; a call of two tokens: the cascades' own blocks
     (2, 16, 128, 5, 4, 4, torch.float16, "iplus1", False),  # single tokens by one launch; ids that only some cascades get

@@ -228,3 +228,28 @@ def test_the_stream_handle_comes_from_the_public_call_where_torch_has_no_other(m
     assert cc.raw_stream(device) == 103
     monkeypatch.setattr(cc, "_current_raw_stream", lambda index: 200 + index)
     assert cc.raw_stream(device) == 203
+
+
+def test_the_counter_table_is_published_when_it_is_filled(monkeypatch):
+    """Other streams and threads read the table without an event: the stream that fills it is waited for first, a second caller gets the
+    first one's, and a stream that is being captured builds none."""
+    from cascading_kv_cache_amd import cascading_cache as cc
+
+    waits = []
+
+    class Stream:
+        def synchronize(self):
+            waits.append(dict(cc._COUNTER_TABLES))
+
+    capturing = [True]
+    monkeypatch.setattr(cc, "_COUNTER_TABLES", {})
+    monkeypatch.setattr(cc, "COUNTER_TABLE_ENTRIES", 16)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: Stream())
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing[0])
+    device = torch.device("cpu", 0)
+    assert cc._counter_table(device) is None and not cc._COUNTER_TABLES
+    capturing[0] = False
+    table = cc._counter_table(device)
+    assert waits == [{}] and torch.equal(table, torch.arange(16))
+    capturing[0] = True
+    assert cc._counter_table(device) is table and len(waits) == 1
