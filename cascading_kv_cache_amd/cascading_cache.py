@@ -469,3 +469,11 @@ class CascadingKVCache:
         else:
             self._seen_dev[layer_idx] += n_new
         self._seen_host[layer_idx] += n_new
+
+
+_UPDATE_STATE = CascadingKVCache.update_state
+
+
+def own_update_state(cache) -> bool:
+    """Is ``cache.update_state`` the one above?  A subclass, a wrapper or a caller that put another in its place is to be called."""
+    return getattr(cache.update_state, "__func__", None) is _UPDATE_STATE

@@ -66,3 +66,31 @@ def test_update_beside_the_scores_equals_two_calls(B, H, KVH, NS, W, C, dtype, f
 def test_update_beside_the_scores_of_many_slots(B, H, KVH, NS, W, C, prompt):
     one, two = pair(B, KVH, NS, W, C, torch.bfloat16, "pow2", True, "mean")
     run_steps(one, two, B, H, KVH, torch.bfloat16, 6, torch.Generator().manual_seed(5), prompt)
+
+
+def test_a_cache_with_an_update_of_its_own_is_asked_every_time():
+    from cascading_kv_cache_amd.cascade_attention import cascade_attention, default_inv_freq
+    from cascading_kv_cache_amd.cascading_cache import CascadingKVCache
+
+    class Counting(CascadingKVCache):
+        calls = 0
+
+        def update_state(self, *args, **kw):
+            self.calls += 1
+            return super().update_state(*args, **kw)
+
+    args = dict(window_length=8, num_sink_tokens=4, max_batch_size=1, heads=2, dim=128, max_seq_len=32, device="cuda:0",
+                dtype=torch.bfloat16, layers=1, verbose=False)
+    plain, counting, patched = CascadingKVCache(**args), Counting(**args), CascadingKVCache(**args)
+    given = []
+    inner = patched.update_state
+    patched.update_state = lambda *a, **kw: (given.append(1), inner(*a, **kw))[1]
+    inv_freq, gen = default_inv_freq(128, 5e5, "cuda:0"), torch.Generator().manual_seed(3)
+    for n in (20, 1, 1, 1, 3, 1):
+        q, k, v = ((torch.randn(1, h, n, 128, generator=gen)).bfloat16().cuda() for h in (8, 2, 2))
+        outs = [cascade_attention(q, k, v, c, 0, inv_freq)[0] for c in (plain, counting, patched)]
+        assert torch.equal(bits(outs[0]), bits(outs[1])) and torch.equal(bits(outs[0]), bits(outs[2]))
+    assert counting.calls == 6 and len(given) == 6
+    for c in (counting, patched):
+        for name in STATE:
+            assert torch.equal(bits(getattr(plain, name)[0]), bits(getattr(c, name)[0])), name
