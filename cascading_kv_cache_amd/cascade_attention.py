@@ -15,7 +15,7 @@ import torch
 from torch import nn
 
 from . import _abi
-from .cascading_cache import CascadingKVCache, _counter_table, _require_device, on_device, own_update_state, raw_stream, workspace
+from .cascading_cache import CascadingKVCache, _counter_table, _require_device, on_device, own, raw_stream, workspace
 
 
 _DEBUG_COUNTERS = os.environ.get("CKV_DEBUG_COUNTERS", "0") not in ("", "0")
@@ -219,7 +219,7 @@ def cascade_attention(query_states, key_states, value_states, cache: CascadingKV
         ws = workspace(dev, a._need, stream)
         a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
         u = a._update
-        if update_cache and u is not None and own_update_state(cache):
+        if update_cache and u is not None and own(cache, "update_state"):
             u.k, u.v, u.s = a.k_new, a.v_new, a.new_scores
             if u._need > a.workspace_bytes:
                 ws = workspace(dev, u._need, stream)

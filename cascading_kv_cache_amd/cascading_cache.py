@@ -372,7 +372,7 @@ class CascadingKVCache:
 
     def update(self, key_states: Tensor, value_states: Tensor, layer_idx: int, score_states: Tensor = None):
         """cascading_cache.py:1297-1348."""
-        if key_states.shape[-2] == 0:
+        if key_states.shape[-2] == 0 or not own(self, "update_state", "get_vals", "pos_shift"):
             self.update_state(key_states, value_states, layer_idx, score_states)
             return self.get_vals(layer_idx)
         _require_device(key_states, "k")
@@ -471,9 +471,9 @@ class CascadingKVCache:
         self._seen_host[layer_idx] += n_new
 
 
-_UPDATE_STATE = CascadingKVCache.update_state
+_OWN = {name: getattr(CascadingKVCache, name) for name in ("update_state", "get_vals", "pos_shift")}
 
 
-def own_update_state(cache) -> bool:
-    """Is ``cache.update_state`` the one above?  A subclass, a wrapper or a caller that put another in its place is to be called."""
-    return getattr(cache.update_state, "__func__", None) is _UPDATE_STATE
+def own(cache, *names) -> bool:
+    """Are these methods of ``cache`` the ones above?  What a subclass, a wrapper or a caller put in their place is to be called."""
+    return all(getattr(getattr(cache, name), "__func__", None) is _OWN[name] for name in names)

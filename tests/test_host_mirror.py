@@ -253,3 +253,39 @@ def test_the_counter_table_is_published_when_it_is_filled(monkeypatch):
     assert waits == [{}] and torch.equal(table, torch.arange(16))
     capturing[0] = True
     assert cc._counter_table(device) is table and len(waits) == 1
+
+
+def test_update_asks_the_methods_that_a_subclass_overrides(monkeypatch):
+    """``update`` is ``update_state`` with its three or four arguments and then ``get_vals``, whoever provides them."""
+    asked = []
+
+    class Own(CascadingKVCache):
+        def update_state(self, key_states, value_states, layer_idx, score_states=None):
+            asked.append("update_state")
+
+        def get_vals(self, layer_idx):
+            asked.append("get_vals")
+            return super().get_vals(layer_idx)
+
+        def pos_shift(self, layer_idx):
+            asked.append("pos_shift")
+            return 7
+
+    args = dict(window_length=4, num_sink_tokens=2, max_batch_size=1, heads=1, dim=8, max_seq_len=8, device="cpu",
+                dtype=torch.float32, layers=1, verbose=False)
+    cache = Own(**args)
+    k = torch.zeros(1, 1, 3, 8)
+    assert torch.equal(cache.update(k, k, 0)[6], cache.pos[0][:1, 0] + 7)
+    assert asked == ["update_state", "get_vals", "pos_shift"]
+    from cascading_kv_cache_amd import cascading_cache as cc
+
+    stub = lambda self, *a: asked.append(a)   # noqa: E731  (takes no row)
+    monkeypatch.setattr(CascadingKVCache, "update_state", stub)
+    monkeypatch.setitem(cc._OWN, "update_state", stub)
+    for name in ("update_state", "get_vals", "pos_shift"):   # one of them, on the object
+        cache = CascadingKVCache(**args)
+        asked.clear()
+        inner = getattr(cache, name)
+        setattr(cache, name, lambda *a, _inner=inner, _name=name: (asked.append(_name), _inner(*a))[1])
+        cache.update(k, k, 0)
+        assert name in asked
