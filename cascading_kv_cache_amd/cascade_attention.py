@@ -225,7 +225,7 @@ def cascade_attention(query_states, key_states, value_states, cache: CascadingKV
                 ws = workspace(dev, u._need, stream)
                 a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
             u.workspace, u.workspace_bytes = a.workspace, a.workspace_bytes   # used by one after the other
-            on_host = cache._begin_update(u, L, Q, dev, replayable)
+            on_host = cache._begin_update(u, L, dev, replayable)
             _abi.check(lib.ckv_attn_update(C.byref(a), C.byref(u), C.c_void_p(stream)), "ckv_attn_update")
             cache._end_update(L, Q, on_host)
             return out, new_scores

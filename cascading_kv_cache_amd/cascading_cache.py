@@ -433,7 +433,7 @@ class CascadingKVCache:
         else:
             a.k, a.v, a.s = key_states.data_ptr(), value_states.data_ptr(), score_states.data_ptr()
         n_new = key_states.shape[-2]
-        on_host = self._begin_update(a, layer_idx, n_new, key_states.device, _device_counter)
+        on_host = self._begin_update(a, layer_idx, key_states.device, _device_counter)
         if _stream is None:
             with on_device(key_states.device):
                 stream = raw_stream(key_states.device)
@@ -450,10 +450,8 @@ class CascadingKVCache:
             _abi.check(_abi.lib().ckv_update(C.byref(a), C.c_void_p(_stream)), "ckv_update")
         self._end_update(layer_idx, n_new, on_host)
 
-    def _begin_update(self, a, layer_idx: int, n_new: int, device, device_counter: bool) -> bool:
+    def _begin_update(self, a, layer_idx: int, device, device_counter: bool) -> bool:
         """Points the argument block at the number of tokens seen so far; True: the host knows it."""
-        if layer_idx == 0:
-            self._seen_tokens += n_new
         table = None if device_counter else _counter_table(device)
         if table is not None and self._seen_host[layer_idx] < table.numel():
             a.real_token_idx = table.data_ptr() + 8 * self._seen_host[layer_idx]
@@ -463,7 +461,10 @@ class CascadingKVCache:
         return False
 
     def _end_update(self, layer_idx: int, n_new: int, on_host: bool):
-        """After the kernels, as in the reference (cascading_cache.py:1343-1346)."""
+        """All counters, after the kernels (cascading_cache.py:1343-1346; the reference counts ``_seen_tokens`` in front of them,
+        1314-1315): a call that is refused has counted nothing."""
+        if layer_idx == 0:
+            self._seen_tokens += n_new
         if on_host:
             self._seen_pending[layer_idx] += n_new
         else:

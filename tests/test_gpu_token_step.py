@@ -94,3 +94,23 @@ def test_a_cache_with_an_update_of_its_own_is_asked_every_time():
     for c in (counting, patched):
         for name in STATE:
             assert torch.equal(bits(getattr(plain, name)[0]), bits(getattr(c, name)[0])), name
+
+
+def test_a_refused_step_counts_nothing(monkeypatch):
+    from cascading_kv_cache_amd import _abi
+    from cascading_kv_cache_amd.cascade_attention import cascade_attention, default_inv_freq
+
+    cache, _ = pair(1, 2, 4, 8, 2, torch.bfloat16, "pow2", True, "mean")
+    inv_freq = default_inv_freq(128, 5e5, "cuda:0")
+    q, k = (torch.zeros(1, h, 1, 128, dtype=torch.bfloat16, device="cuda:0") for h in (8, 2))
+    for _ in range(2):
+        cascade_attention(q, k, k, cache, 0, inv_freq)
+    before = cache._seen_tokens, list(cache._seen_host), list(cache._seen_pending)
+    assert before == (2, [2], [2])
+    for name in ("ckv_attn_update", "ckv_update"):   # what the library says to a call that it refuses
+        monkeypatch.setattr(_abi.lib(), name, lambda *args: 3)
+    with pytest.raises(_abi.CkvError):
+        cascade_attention(q, k, k, cache, 0, inv_freq)
+    with pytest.raises(_abi.CkvError):
+        cache.update_state(k, k, 0, k[..., 0])
+    assert (cache._seen_tokens, cache._seen_host, cache._seen_pending) == before
