@@ -47,15 +47,18 @@ def chunk_positions(cache: CascadingKVCache, layer_idx: int, q_len: int, do_og_p
     S, NS = cache.max_seq_len[layer_idx], cache.num_sink_tokens
     if not do_og_pos and cache.eager_fill and S > 0 and not _replayable:
         start = min(int(cache._seen_host[layer_idx]), S + NS)
-        memo = cache.__dict__.setdefault("_steady_q_pos", {})
-        own = _stream is None   # a caller's own ids, which it may write to; the library's are a part of a table of integers
-        key = (start, q_len, dev, own)
+        if _stream is None:
+            return torch.arange(start, start + q_len, device=dev, dtype=torch.long)   # not kept: a caller may write to it
+        memo = cache.__dict__.setdefault("_steady_q_pos", {})   # read only: a part of the table of integers, where it reaches
+        key = (start, q_len, dev)
         ids = memo.get(key)
         if ids is None:
             if len(memo) > 16:
                 memo.clear()
-            table = None if own else _counter_table(dev)
-            if table is not None and start + q_len <= table.numel():
+            table = _counter_table(dev)
+            if table is None:   # being captured: filled by the replays
+                return torch.arange(start, start + q_len, device=dev, dtype=torch.long)
+            if start + q_len <= table.numel():
                 ids = table[start:start + q_len]
             else:
                 ids = torch.arange(start, start + q_len, device=dev, dtype=torch.long)

@@ -376,6 +376,22 @@ def test_chunk_positions_kernel(do_og_pos, eager):
         assert torch.equal(chunk_positions(gpu, 0, 5, do_og_pos).cpu(), want)
 
 
+def test_chunk_positions_belong_to_the_caller():
+    """Ids that a caller wrote to are nobody else's: not the next caller's, and not those of the library's own calls."""
+    from cascading_kv_cache_amd.cascade_attention import cascade_attention, chunk_positions, default_inv_freq
+
+    gpu, cpu = make_pair(1, 2, 32, 4, 16, 4, torch.float32, eager=True)
+    inv_freq = default_inv_freq(32, 1e4, "cuda:0")
+    q, k = (torch.randn(1, h, 90, 32, generator=torch.Generator().manual_seed(h)).cuda() for h in (4, 2))
+    cascade_attention(q, k, k, gpu, 0, inv_freq)      # full: the ids of a chunk of a length are the same from now on
+    first = cascade_attention(q[:, :, :5], k[:, :, :5], k[:, :, :5], gpu, 0, inv_freq, update_cache=False)[0]
+    mine = chunk_positions(gpu, 0, 5)
+    want = mine.clone()
+    mine += 1000
+    assert torch.equal(chunk_positions(gpu, 0, 5), want)
+    assert torch.equal(cascade_attention(q[:, :, :5], k[:, :, :5], k[:, :, :5], gpu, 0, inv_freq, update_cache=False)[0], first)
+
+
 def dense_reference(q, k, v, mask, sm_scale):
     n_ctx, n_kv = q.size(2), k.size(2)
     logits = torch.matmul(q.float(), k.float().transpose(2, 3)) * sm_scale
