@@ -61,16 +61,23 @@ class RMSNorm(nn.Module):
         return self.weight * xf.to(x.dtype)
 
 
-_functorch_levels = getattr(getattr(torch._C, "_functorch", None), "peek_interpreter_stack", lambda: None)   # not public
 _GATED_TYPES = (torch.bfloat16, torch.float16, torch.float32)
+# not public: where torch lacks one of them, somebody may be following
+_function_modes = getattr(torch._C, "_len_torch_function_stack", lambda: 1)
+_dispatch_modes = getattr(torch._C, "_len_torch_dispatch_stack", lambda: 1)
+_functorch_levels = getattr(getattr(torch._C, "_functorch", None), "peek_interpreter_stack", lambda: 1)
+
+
+def _followed(x) -> bool:
+    """May anybody follow torch's operations on ``x``: gradients of either mode, vmap, tracing, a tensor subclass, a mode?"""
+    return (type(x) is not torch.Tensor or torch.is_grad_enabled() or x.requires_grad or _function_modes() != 0 or _dispatch_modes() != 0
+            or getattr(torch.autograd.forward_ad, "_current_level", 0) >= 0 or _functorch_levels() is not None
+            or torch.jit.is_tracing() or torch.compiler.is_compiling())
 
 
 def gated_silu(gate_up):
-    """``silu(gate) * up`` of rows of ``gate | up``: one launch of the library, the same bits, where nobody follows what is done
-    (gradients of either mode, vmap, tracing)."""
-    if (gate_up.device.type != "cuda" or torch.is_grad_enabled() or gate_up.requires_grad or not gate_up.is_contiguous()
-            or gate_up.dtype not in _GATED_TYPES or torch.autograd.forward_ad._current_level >= 0 or _functorch_levels() is not None
-            or torch.jit.is_tracing() or torch.compiler.is_compiling()):
+    """``silu(gate) * up`` of rows of ``gate | up``: one launch of the library, the same bits, where nobody follows what is done."""
+    if gate_up.device.type != "cuda" or not gate_up.is_contiguous() or gate_up.dtype not in _GATED_TYPES or _followed(gate_up):
         gate, up = gate_up.chunk(2, dim=-1)
         return nn.functional.silu(gate) * up
     inter = gate_up.size(-1) // 2

@@ -289,3 +289,40 @@ def test_update_asks_the_methods_that_a_subclass_overrides(monkeypatch):
         setattr(cache, name, lambda *a, _inner=inner, _name=name: (asked.append(_name), _inner(*a))[1])
         cache.update(k, k, 0)
         assert name in asked
+
+
+def test_the_gate_stays_with_torch_where_somebody_follows_it(monkeypatch):
+    """Gradients of either mode, vmap, dispatch and function modes, subclasses; a torch without the private names that tell is one where
+    somebody may."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    from cascading_kv_cache_amd import decoder
+
+    class Function(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    class Dispatch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    x = torch.randn(2, 8)
+    assert decoder._followed(x)   # gradients are on
+    with torch.no_grad():
+        assert not decoder._followed(x)
+        for mode in (Function, Dispatch):
+            with mode():
+                assert decoder._followed(x)
+        with FakeTensorMode() as mode:
+            assert decoder._followed(mode.from_tensor(x))
+        with torch.autograd.forward_ad.dual_level():
+            assert decoder._followed(x)
+        seen = []
+        torch.vmap(lambda row: (seen.append(decoder._followed(row)), row)[1])(x)
+        assert seen == [True]
+        assert decoder._followed(torch.nn.Parameter(x, requires_grad=False))
+        monkeypatch.delattr(torch.autograd.forward_ad, "_current_level")
+        assert decoder._followed(x)
+        assert torch.equal(decoder.gated_silu(x), torch.nn.functional.silu(x[:, :4]) * x[:, 4:])
