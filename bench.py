@@ -169,7 +169,8 @@ def update_bytes(cache, cfg, k, v, new_scores, es=2):
 
 def update_kernel_ms(cache, k, v, new_scores, reps=20):
     """Kernel time of one cache update: the durations of all its kernels (plan and apply launches), each timed by
-    events attached to its own dispatch, summed per call.  The calls advance the (steady-state) cache."""
+    events attached to its own dispatch, summed per call.  The calls advance the (steady-state) cache.  (The timers count
+    the plan as two also where both planners share a launch.)"""
     from cascading_kv_cache_amd import _abi
 
     for _ in range(3):
@@ -183,7 +184,7 @@ def update_kernel_ms(cache, k, v, new_scores, reps=20):
     st = _abi.profile_read()
     _abi.profile_enable(0)
     return (st["plan"][0] + st["apply"][0]) / reps, {"plan_ms": st["plan"][0] / reps, "apply_ms": st["apply"][0] / reps,
-                                                       "launches_per_call": (st["plan"][1] + st["apply"][1]) / reps}
+                                                       "planners_and_apply_per_call": (st["plan"][1] + st["apply"][1]) / reps}
 
 
 def stage_table(stages, calls=None):
@@ -301,7 +302,7 @@ def run_layer(steps, warmup, dtype, device):
                      if attn_ms else None),
         decode=dict(workload="single-token steps on the headline cache (B=1, 64 sinks + 8 x 8192 slots, full)",
                     tokens_per_s=B / token_s, ms_per_step=token_s * 1e3, ms_per_step_graph_replay=token_graph_s * 1e3,
-                    stage_ms=dec_stages,
+                    stage_ms=dec_stages, stage_ms_note="stages one by one, the update in launches of its own; a step runs it beside the scores",
                     roofline=dict(bound="hbm", achieved=dec_achieved, peak=PEAK_HBM_GBPS, unit="GB/s",
                                   frac=dec_achieved / PEAK_HBM_GBPS,
                                   traffic=measured_traffic("decode_stream_kernel", "layer64k"),

@@ -324,7 +324,11 @@ int ckv_gated_silu(const void* gate_up, void* out, int64_t rows, int64_t inter, 
  * every kernel stage).  While enabled, each stage of ckv_attn / ckv_update is bracketed by HIP
  * events on the caller's stream; ckv_profile_read waits for them, ADDS the elapsed milliseconds
  * and launch counts per stage into the caller's arrays (length CKV_STAGE_COUNT) and forgets
- * them.  Process-wide and not thread-safe: a measurement aid, off by default.
+ * them.  The plan of a call of several tokens is counted as two (closed forms, walk) also where
+ * both are one launch: its time is with the first, the second has none.  Levels 1 and 3 run a
+ * single token's cache update in launches of its own, which ckv_attn_update does otherwise only
+ * where it cannot run beside the scores: they show what the stages take one by one, not what
+ * such a step takes.  Process-wide and not thread-safe: a measurement aid, off by default.
  * ---------------------------------------------------------------------------------------- */
 typedef enum ckv_stage {
     CKV_STAGE_PREP = 0,        /* rotate + gather prologue                      */
