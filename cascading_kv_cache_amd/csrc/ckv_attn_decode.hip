@@ -2262,6 +2262,21 @@ __global__ void __launch_bounds__(kSK) decode_scores_homo_kernel(DecodeParams p,
     }
 }
 
+// How a step after a streaming kernel ends, see decode_finish_kernel: workgroups of rows and scores in one launch (0: in launches of
+// their own), and whether a cache update comes along.  stream_wgs: workgroups of the streaming kernel.
+struct StepEnd {
+    int64_t finish_blocks;
+    bool update;
+};
+inline StepEnd step_end(int64_t B, int64_t H, int64_t KVH, int64_t num_sink, int64_t S, int64_t stream_wgs, int64_t cus) {
+    const int64_t tiles = (num_sink + S + 1 + kSK - 1) / kSK, units = B * KVH, G = H / KVH;
+    const int64_t blocks = B * H + units * ((tiles * kSK / 8 + 511) / 512), line = finish_workgroups_per_cu(num_sink, (int)G) * cus;
+    if (blocks > line) return {0, false};
+    return {blocks, units <= stream_wgs && (G <= 4 || blocks + units * (1 + pos_blocks(S)) <= line)};
+}
+// as many as run at once, at most one a (tile, unit)
+inline int64_t stream_workgroups(int64_t items, int64_t cus) { return std::min({(cus > 0 ? cus : 256) * kStreamWgPerCu, (int64_t)kStreamMaxWgs, items}); }
+
 // *updated: the update that p.plans asks for has been launched too
 template <typename T, int G>
 int run_decode(const DecodePlanParams& p_in, hipStream_t stream, bool* updated) {
@@ -2282,16 +2297,16 @@ int run_decode(const DecodePlanParams& p_in, hipStream_t stream, bool* updated) 
     }
     p.Np = (int64_t)p.tiles * kSK;
     p.own_q = use_stream && a.B * a.H <= kOwnQRows;
-    if (!use_stream) p.plans = nullptr;
-    int64_t finish_blocks = 0;   // of decode_finish_kernel, where the step ends in it
-    if (use_stream && !a.homogeneous_heads && (a.cache_s || a.new_scores)) {
+    StepEnd end{0, false};
+    if (use_stream) {
         DeviceInfo di;
         if (int rc = current_device_info(&di)) return rc;
-        finish_blocks = a.B * a.H + a.B * a.KVH * ((p.Np / 8 + 511) / 512);
-        const int64_t line = finish_workgroups_per_cu(a.num_sink, G) * (int64_t)di.cus;
-        if (finish_blocks > line) finish_blocks = 0;
-        if (G > 4 && finish_blocks + a.B * a.KVH * (1 + pos_blocks(a.S)) > line) p.plans = nullptr;
+        p.stream_wgs = (int)stream_workgroups((int64_t)p.n_vis * p.nbh, di.cus);
+        if (!a.homogeneous_heads && (a.cache_s || a.new_scores))
+            end = step_end(a.B, a.H, a.KVH, a.num_sink, a.S, p.stream_wgs, di.cus);
     }
+    const int64_t finish_blocks = end.finish_blocks;   // of decode_finish_kernel, where the step ends in it
+    if (!end.update) p.plans = nullptr;
     p.inv_h = (uint32_t)((65536 + a.H - 1) / a.H);
     {
         // timed stages: a call has this one either way, empty where the streaming kernel rotates the queries itself
@@ -2315,15 +2330,9 @@ int run_decode(const DecodePlanParams& p_in, hipStream_t stream, bool* updated) 
             // streaming kernel: as many workgroups as run at once, items dealt out evenly
             if constexpr (G <= 8) {
                 constexpr int lds_s = G <= 4 ? kStreamLds : kWideLds;
-                DeviceInfo di;
-                if (int rc = current_device_info(&di)) return rc;
-                int64_t wgs = (di.cus > 0 ? di.cus : 256) * kStreamWgPerCu;
-                if (wgs > kStreamMaxWgs) wgs = kStreamMaxWgs;
-                if (wgs > p.n_vis * nbh) wgs = p.n_vis * nbh;
-                p.stream_wgs = (int)wgs;
+                const int64_t wgs = p.stream_wgs;
                 p.run_q = (int)(p.n_vis * nbh / wgs);
                 p.run_r = (int)(p.n_vis * nbh % wgs);
-                if (finish_blocks == 0 || nbh > wgs) p.plans = nullptr;
                 hipEvent_t ev0, ev1;
                 prof_kernel_events(CKV_STAGE_DECODE, &ev0, &ev1);
                 // The planning wavefront is compiled in only where the step has a plan: skipped by a branch, it still cost the large
@@ -2502,3 +2511,18 @@ int launch_decode(const ckv_attn_args& a, hipStream_t stream, const ckv_update_a
 }
 
 }  // namespace ckv
+
+// For tests that aim at one way (a full cache on `cus` compute units, 0: the current device's): does a step of 16-bit tensors end in one
+// launch for rows and scores (1), one with the update too (2), or in launches apart (0)?
+extern "C" int ckv_decode_step_end(int64_t B, int64_t H, int64_t KVH, int64_t num_sink, int64_t S, int64_t cus) {
+    using namespace ckv;
+    if (cus <= 0) cus = mfma_device_cus();
+    const int64_t tiles = (num_sink + S + 1 + kSK - 1) / kSK;
+    const StepEnd end = step_end(B, H, KVH, num_sink, S, stream_workgroups(tiles * B * KVH, cus), cus);
+    return end.update ? 2 : end.finish_blocks > 0 ? 1 : 0;
+}
+
+// ... and is `update` one that belongs to the step `args`?
+extern "C" int ckv_decode_update_belongs(const ckv_attn_args* args, const ckv_update_args* update) {
+    return ckv::decode_supported(*args) && ckv::update_beside_scores(*args, *update);
+}

@@ -318,3 +318,15 @@ def test_dq_by_eight_wavefronts_where_all_run_at_once(lib, n_ctx, units, wavefro
 def test_backward_in_one_launch_up_to_five_workgroups_a_unit(lib, n_kv, heads, one):
     """The dense operator's dk, dv and dq on 256 compute units: one launch up to 1280 workgroups of 128 keys."""
     assert C.CDLL(_abi.LIB_PATH).ckv_dense_bwd_one_launch(C.c_int64(n_kv), C.c_int64(heads), C.c_int64(256)) == one
+
+
+@pytest.mark.parametrize("B,H,KVH,NS,S,end", [
+    (1, 32, 8, 4, 2048, 2), (1, 32, 8, 64, 65536, 2), (16, 32, 8, 64, 32768, 0),
+    (12, 32, 8, 64, 16384, 2), (15, 32, 8, 64, 16384, 0), (15, 32, 8, 4, 16384, 2), (28, 32, 8, 4, 16384, 2), (29, 32, 8, 4, 16384, 0),
+    (32, 8, 8, 4, 16384, 2), (33, 8, 8, 4, 16384, 1),                             # 256 and 264 (batch, kv head) pairs
+    (7, 28, 4, 64, 16384, 2), (8, 28, 4, 64, 16384, 1), (10, 28, 4, 64, 16384, 1), (11, 28, 4, 64, 16384, 0),
+])
+def test_how_a_single_token_step_ends(lib, B, H, KVH, NS, S, end):
+    """On 256 compute units: rows and scores in one launch (1) up to four workgroups a unit, eight where the scores are no whole
+    pieces, two with more than four heads per kv head, where the update (2) counts among them; up to 256 pairs."""
+    assert C.CDLL(_abi.LIB_PATH).ckv_decode_step_end(*(C.c_int64(n) for n in (B, H, KVH, NS, S, 256))) == end

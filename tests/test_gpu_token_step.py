@@ -1,6 +1,8 @@
 """A single-token step whose cache update runs beside its scores (ckv_attn_update) against the same step in two calls
 (ckv_attn, then ckv_update): outputs, new scores and every state tensor bit-identical after every token, from an empty
 cache through sinks, filling and eviction."""
+import ctypes
+
 import pytest
 import torch
 
@@ -43,6 +45,21 @@ def run_steps(one, two, B, H, KVH, dtype, tokens, gen, prompt=0):
         assert torch.equal(one.seen_tokens_by_layer, two.seen_tokens_by_layer) and one._seen_host == two._seen_host
 
 
+def step_end(cache, H):
+    """How the single-token steps that ``cache`` has seen end on this device: launches apart (0), rows and scores in one (1), the update too
+    (2); and whether their argument blocks are such that the update may come along."""
+    from cascading_kv_cache_amd import _abi
+
+    lib = ctypes.CDLL(_abi.LIB_PATH)
+    B, KVH, S = cache.key_cache[0].shape[:3]
+    blocks = [a for a in cache._attn_memo.values() if a.Q == 1 and a._update is not None]
+    assert blocks
+    belongs = {lib.ckv_decode_update_belongs(ctypes.byref(a), ctypes.byref(a._update)) for a in blocks}
+    assert len(belongs) == 1
+    sizes = [ctypes.c_int64(n) for n in (B, H, KVH, cache.num_sink_tokens, S, 0)]
+    return lib.ckv_decode_step_end(*sizes), bool(belongs.pop())
+
+
 # windows of one slot, odd ones (position ids one by one), one cascade, as many as a workgroup takes and one more (two calls
 # inside), schedules whose periods do not divide each other, more (batch, kv head) pairs than the planning workgroups take
 @pytest.mark.parametrize("B,H,KVH,NS,W,C,dtype,func,eager,reduction,tokens", [
@@ -58,14 +75,19 @@ def run_steps(one, two, B, H, KVH, dtype, tokens, gen, prompt=0):
 def test_update_beside_the_scores_equals_two_calls(B, H, KVH, NS, W, C, dtype, func, eager, reduction, tokens):
     one, two = pair(B, KVH, NS, W, C, dtype, func, eager, reduction)
     run_steps(one, two, B, H, KVH, dtype, tokens, torch.Generator().manual_seed(tokens + C), 0)
+    assert step_end(one, H) == (2 if B < 33 else 1, C < 32)
 
 
-# several workgroups of scores and position ids per (batch, kv head), and the step in separate launches (its workgroups past
-# eight a compute unit)
-@pytest.mark.parametrize("B,H,KVH,NS,W,C,prompt", [(2, 8, 2, 4, 1500, 3, 4800), (1, 28, 4, 64, 4096, 2, 8600), (40, 8, 8, 4, 8192, 2, 300)])
-def test_update_beside_the_scores_of_many_slots(B, H, KVH, NS, W, C, prompt):
+# several workgroups of scores and position ids per (batch, kv head); more (batch, kv head) pairs than the planning workgroups take; the
+# step in separate launches (its workgroups past four a compute unit); more than four heads per kv head and the update's workgroups past
+# the one round
+@pytest.mark.parametrize("B,H,KVH,NS,W,C,prompt,end", [(2, 8, 2, 4, 1500, 3, 4800, 2), (1, 28, 4, 64, 4096, 2, 8600, 2),
+                                                       (40, 8, 8, 4, 8192, 2, 300, 1), (32, 8, 8, 64, 6144, 2, 300, 0),
+                                                       (10, 28, 4, 64, 4096, 4, 700, 1)])
+def test_update_beside_the_scores_of_many_slots(B, H, KVH, NS, W, C, prompt, end):
     one, two = pair(B, KVH, NS, W, C, torch.bfloat16, "pow2", True, "mean")
     run_steps(one, two, B, H, KVH, torch.bfloat16, 6, torch.Generator().manual_seed(5), prompt)
+    assert step_end(one, H) == (end, True)
 
 
 def test_a_cache_with_an_update_of_its_own_is_asked_every_time():
