@@ -556,7 +556,8 @@ __global__ void ckv_update_plan_kernel(UpdateParams p) {
 
 // Both in one launch: the first workgroup of a unit walks its arrivals if the others, which look at the same trackers (apply commits
 // them), find that the closed forms do not hold.  A launch that mostly returns took a call 4 to 5 us, its instructions being cold: 256
-// tokens into 512 float32 slots 74.6 -> 70.2 us behind their attention, 509 into 16 K 290 -> 288.
+// tokens into 512 float32 slots 74.6 -> 70.2 us behind their attention, 509 into 16 K 282.2 -> 280.3, hardly more than two runs
+// of one side differ.
 template <int kThreads>
 __global__ void __launch_bounds__(kThreads) ckv_update_plan_both_kernel(UpdateParams p) {
     extern __shared__ __align__(16) unsigned char smem[];
@@ -1223,7 +1224,7 @@ int run_update(const ckv_update_args& A, void* workspace, int64_t* row, int64_t 
                 if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(kernel), (int)lds)) return rc;
                 launch_timed(CKV_STAGE_PLAN, kernel, dim3((unsigned)(A.cascades + 2 * ksub / threads.value) + 1, H, N), dim3(threads.value), lds,
                              stream, p);
-                prof_empty(CKV_STAGE_PLAN);   // a chunk has two of these either way
+                prof_empty(CKV_STAGE_PLAN);   // counted as two either way
                 return CKV_OK;
             };
             if (lds <= kBothLds) {
