@@ -9,7 +9,7 @@
 // 5700 cycles next to the other wavefront's 64 products, which take 4400 alone, and 1700 by themselves), so what is not
 // arithmetic of the attention -- masks of whole blocks, addresses of rows -- is kept off the vector pipe.
 //
-//   forward  one workgroup = one kv head x 32 (position, head) rows; its eight wavefronts take the 32-key blocks in
+//   forward  one workgroup = one head x 32 rows; its eight wavefronts take the 32-key blocks in
 //            turn, each with an online softmax of its own, and merge at the end through LDS.  S^T = K Q^T keeps a query
 //            in one lane pair, and register v of S^T is, as it stands, the B operand of step v of O^T += V^T P^T: nothing
 //            is moved between the two products.  Values go from memory straight to the operand registers (no two
@@ -20,7 +20,7 @@
 //            workgroups); two streams of its wavefronts take the 32-row query tiles, which come through LDS, in turn.
 //            S = Q K^T keeps a key in one lane pair, so a weighted sum stays in its lane until the end.  With a block of
 //            keys a workgroup and queries straight to registers the scores took 34 us (28 heads x 2568 keys, 512 rows: 156,
-//            now 130), with a barrier a tile 31.3.
+//            now 123), with a barrier a tile 31.3.
 //
 // A matrix instruction multiplies every row of a tile by every value, and zero times infinity or NaN is NaN, while a value
 // whose key has probability zero counts for nothing, whatever it holds (the vector kernels do not touch it).  So a wavefront
@@ -91,17 +91,16 @@ __global__ void __launch_bounds__(kFwdWaves* CKV_WAVE) fwd_f32_mfma_kernel(CoreP
     float* ml_lds = o_lds + kFwdWaves * kRows * G_::kPitch;           // [max, sum][wave][row]
     const int tid = threadIdx.x, lane = tid & 63, col = lane & 31, half = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    // kv heads go round the XCDs (when they divide evenly), so a head's keys stay in one L2; heavy row tiles first
-    const int nbkv = (int)(p.B * p.KVH), KVH = (int)p.KVH, G = (int)p.H / KVH;
-    const int n_rt = (int)(((int)p.Q * G + kRows - 1) / kRows);
-    const int bkv = blockIdx.x % nbkv, rt = n_rt - 1 - (int)(blockIdx.x / nbkv);
-    const int64_t b = bkv / KVH, kvh = bkv % KVH;
+    // heads go round the XCDs (when they divide evenly), so a head's keys stay in one L2; heavy row tiles first
+    const int heads = (int)(p.B * p.H), H = (int)p.H, n_rt = ((int)p.Q + kRows - 1) / kRows;
+    const int bh = blockIdx.x % heads, rt = n_rt - 1 - (int)(blockIdx.x / heads);
+    const int64_t b = bh / H, h = bh % H;
     const int N = (int)p.N, Q = (int)p.Q, Nc = N - Q;
-    const float* kb = (const float*)p.k + b * p.kv_stride[0] + kvh * p.kv_stride[1];
-    const float* vb = (const float*)p.v + b * p.kv_stride[0] + kvh * p.kv_stride[1];
+    const float* kb = (const float*)p.k + b * p.kv_stride[0] + h * p.kv_stride[1];
+    const float* vb = (const float*)p.v + b * p.kv_stride[0] + h * p.kv_stride[1];
 
-    const int row_m = (rt * kRows + col) / G;            // this lane's query
-    int m_hi = (rt * kRows + kRows - 1) / G;
+    const int row_m = rt * kRows + col;                  // this lane's query
+    int m_hi = rt * kRows + kRows - 1;
     if (m_hi > Q - 1) m_hi = Q - 1;
     const int nblk = (Nc + m_hi) / kKeys + 1;            // blocks some row of the tile may see
     // bit r: key r of the block is there and not masked
@@ -187,9 +186,9 @@ __global__ void __launch_bounds__(kFwdWaves* CKV_WAVE) fwd_f32_mfma_kernel(CoreP
     {
 #pragma unroll
         for (int t = 0; t < NP / kFwdWaves; t++) {
-            const int c = t * kFwdWaves + wave, rf = rt * kRows + col, m = rf / G, g = rf % G;
-            if (m < Q)
-                async_copy16_from((const float*)p.q + b * p.q_stride[0] + (kvh * G + g) * p.q_stride[1] + m * p.q_stride[2] + 8 * c + 4 * half,
+            const int c = t * kFwdWaves + wave;
+            if (row_m < Q)
+                async_copy16_from((const float*)p.q + b * p.q_stride[0] + h * p.q_stride[1] + row_m * p.q_stride[2] + 8 * c + 4 * half,
                                   lds_address(q_lds) + c * (CKV_WAVE * 16));
             else
                 q_lds[c * CKV_WAVE + lane] = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -371,7 +370,7 @@ __global__ void __launch_bounds__(kFwdWaves* CKV_WAVE) fwd_f32_mfma_kernel(CoreP
     // sixteen threads per row
     constexpr int kPer = D / 16;
     const int r = tid >> 4, d0 = (tid & 15) * kPer;
-    const int rf = rt * kRows + r, m = rf / G, g = rf % G;
+    const int m = rt * kRows + r;
     if (m >= Q) return;
     float M = -INFINITY, L = 0.f;
 #pragma unroll
@@ -390,8 +389,8 @@ __global__ void __launch_bounds__(kFwdWaves* CKV_WAVE) fwd_f32_mfma_kernel(CoreP
         for (int i = 0; i < kPer; i++) acc[i] += o_lds[(w * kRows + r) * G_::kPitch + d0 + i];
     // A row without a probability above zero (all its logits overflowed) or with a NaN among them is NaN.
     const float inv = 1.f / L;
-    const int64_t row = (b * p.H + kvh * G + g) * p.Q + m;
-    float* orow = (float*)p.out + b * p.out_stride[0] + (kvh * G + g) * p.out_stride[1] + m * p.out_stride[2];
+    const int64_t row = (b * p.H + h) * p.Q + m;
+    float* orow = (float*)p.out + b * p.out_stride[0] + h * p.out_stride[1] + m * p.out_stride[2];
 #pragma unroll
     for (int i = 0; i < kPer; i++) orow[(d0 + i) * p.out_stride[3]] = acc[i] * inv;
     if (d0 == 0 && p.lse) p.lse[row] = M + logf(L);
@@ -407,13 +406,12 @@ __global__ void __launch_bounds__(Col<kGroups>::kWaves* CKV_WAVE, 2) colsum_f32_
     const int tid = threadIdx.x, lane = tid & 63, col = lane & 31, half = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int group = wave % kColGroups, stream = wave / kColGroups;
-    const int nbkv = (int)(p.B * p.KVH), KVH = (int)p.KVH, G = (int)p.H / KVH;
+    const int heads = (int)(p.B * p.H), H = (int)p.H;
     const int N = (int)p.N, Q = (int)p.Q, Nc = N - Q, nblk = (N + kColKeys - 1) / kColKeys;
-    // kv heads round the XCDs; blocks of chunk keys see fewer rows and come last
-    const int bkv = blockIdx.x % nbkv, rest = blockIdx.x / nbkv;
-    const int g = rest % G, blk = rest / G;
+    // heads round the XCDs; blocks of chunk keys see fewer rows and come last
+    const int bh = blockIdx.x % heads, blk = blockIdx.x / heads;
     if (blk >= nblk) return;
-    const int64_t b = bkv / KVH, kvh = bkv % KVH, h = kvh * G + g;
+    const int64_t b = bh / H, h = bh % H;
     const int n0 = blk * kColKeys + group * kKeys, n = n0 + col, nrel = n - Nc;   // nrel >= 0: a chunk key
     const int masked = n < Nc && p.kmasked ? p.kmasked[n] : 0;
     const float* qb = (const float*)p.q + b * p.q_stride[0] + h * p.q_stride[1];
@@ -435,14 +433,14 @@ __global__ void __launch_bounds__(Col<kGroups>::kWaves* CKV_WAVE, 2) colsum_f32_
     if (t_first + wave < n_tiles) copy_queries(t_first + wave);
     float4 kf[NP];
     {
-        const float* kr = (const float*)p.k + b * p.kv_stride[0] + kvh * p.kv_stride[1] +
+        const float* kr = (const float*)p.k + b * p.kv_stride[0] + h * p.kv_stride[1] +
                           (int64_t)(n < N ? n : N - 1) * p.kv_stride[2] + 4 * half;
 #pragma unroll
         for (int c = 0; c < NP; c++) kf[c] = *reinterpret_cast<const float4*>(kr + 8 * c);
     }
     const bool live = n < N && masked == 0;
     const bool wanted = __ballot(live) != 0ull;
-    const bool chunk_keys = n0 + kKeys > Nc, by_distance = nrel >= 0 && p.new_mode;
+    const bool chunk_keys = n0 + kKeys > Nc;
     float acc[kAcc] = {};   // of this stream's tiles with the same (t - t_own) mod 4; of a key nobody sees, anything
     const int t_end = __syncthreads_or(wanted) ? n_tiles : t_first;
     for (int t0 = t_first; t0 < t_end; t0 += kColWaves) {
@@ -469,9 +467,9 @@ __global__ void __launch_bounds__(Col<kGroups>::kWaves* CKV_WAVE, 2) colsum_f32_
                 } else {
 #pragma unroll
                     for (int e = 0; e < 4; e++) {
-                        const int m = m0 + e < Q ? m0 + e : Q - 1, d = m - nrel;
+                        const int m = m0 + e < Q ? m0 + e : Q - 1;
                         ls[i4].v[e] = lse[m];
-                        w[i4].v[e] = by_distance ? p.w_new[d > 0 ? d : 0] : p.w_ema[m];
+                        w[i4].v[e] = p.w_ema[m];
                     }
                 }
             }
@@ -525,19 +523,19 @@ __global__ void __launch_bounds__(Col<kGroups>::kWaves* CKV_WAVE, 2) colsum_f32_
 
 template <int D>
 int run(const CoreProblem& p, hipStream_t stream) {
-    const int64_t G = p.H / p.KVH, tiles = (p.Q * G + kRows - 1) / kRows;
+    const int64_t tiles = (p.Q + kRows - 1) / kRows;
     {
         StageScope sc(CKV_STAGE_FWD, stream);
         const int lds = Geo<D>::kFwdLds;
         if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(fwd_f32_mfma_kernel<D>), lds)) return rc;
-        hipLaunchKernelGGL(fwd_f32_mfma_kernel<D>, dim3((unsigned)(tiles * p.B * p.KVH)), dim3(kFwdWaves * CKV_WAVE), lds, stream, p);
+        hipLaunchKernelGGL(fwd_f32_mfma_kernel<D>, dim3((unsigned)(tiles * p.B * p.H)), dim3(kFwdWaves * CKV_WAVE), lds, stream, p);
         CKV_HIP_TRY(hipGetLastError());
     }
     if (p.colsum) {
         StageScope sc(CKV_STAGE_SCORES, stream);
         // Four blocks of keys share their workgroup's query tiles, unless that leaves more than a quarter of the chip idle (28 heads
         // x 276 and 32 x 360 keys, 16 and 100 rows, 84 and 96 workgroups: 9.6 and 17.5 us against 7.8 and 12.3 with one block each;
-        // 32 x 776 keys, 256 rows, 224 workgroups: 30.7 against 34, 28 x 2568 keys, 512 rows: 130 against 156).
+        // 32 x 776 keys, 256 rows, 224 workgroups: 30.7 against 34, 28 x 2568 keys, 512 rows: 123 against 156).
         auto launch = [&](auto groups) -> int {
             using C_ = Col<groups.value>;
             auto kernel = colsum_f32_mfma_kernel<D, groups.value>;
@@ -562,10 +560,10 @@ bool rows16(const int64_t* st, const void* base) {
 }  // namespace
 
 bool f32_mfma_supported(const CoreProblem& p) {
-    return p.dtype == CKV_F32 && (p.D == 64 || p.D == 128) && p.N < ((int64_t)1 << 31) - 64 &&
-           p.B * p.H * ((p.N + kKeys - 1) / kKeys) < ((int64_t)1 << 31) &&
-           ((p.Q * (p.H / p.KVH) + kRows - 1) / kRows) * 16 * p.B * p.KVH < ((int64_t)1 << 31) && p.lse && rows16(p.q_stride, p.q) &&
-           rows16(p.kv_stride, p.k) && rows16(p.kv_stride, p.v);
+    // every head its own kv head, every key weighted by the query row alone
+    return p.dtype == CKV_F32 && (p.D == 64 || p.D == 128) && p.KVH == p.H && !p.new_mode && p.N < ((int64_t)1 << 31) - 64 &&
+           p.B * p.H * ((p.N + kKeys - 1) / kKeys) < ((int64_t)1 << 31) &&   // at least as many as tiles of queries
+           p.lse && rows16(p.q_stride, p.q) && rows16(p.kv_stride, p.k) && rows16(p.kv_stride, p.v);
 }
 
 int launch_f32_mfma(const CoreProblem& p, hipStream_t stream) { return p.D == 64 ? run<64>(p, stream) : run<128>(p, stream); }

@@ -40,7 +40,8 @@ struct CoreProblem {
 // matrix cores (16-bit and float32) do not cover.
 int launch_core_generic(const CoreProblem& p, hipStream_t stream);
 
-// The same in float32 on the matrix cores: head_dim 64 and 128, rows of 16-byte pieces, lse wanted.
+// The same in float32 on the matrix cores, for the dense operator: head_dim 64 and 128, rows of 16-byte pieces, lse wanted, KVH == H, weights
+// by row alone (new_mode 0).
 bool f32_mfma_supported(const CoreProblem& p);
 int launch_f32_mfma(const CoreProblem& p, hipStream_t stream);
 
