@@ -1188,8 +1188,8 @@ __global__ void __launch_bounds__(kStreamThreads, kStreamWgPerCu) decode_stream_
                 }
                 if (e == 0) { e_half.x = hk.x; e_half.y = hk.y; } else { e_half.z = hk.x; e_half.w = hk.y; }
             }
-            m_t = m;
             l_t = mod4_sum(lloc);
+            m_t = l_t == 0.f ? m : ms;   // keys that are all NaN: no largest logit, but a sum, which the merges are to meet
         }
         __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
         __builtin_amdgcn_wave_barrier();
@@ -1467,8 +1467,8 @@ __global__ void __launch_bounds__(kStreamThreads, kStreamWgPerCu) decode_stream_
                     e_mine = make_uint2(Mma16<__half>::pack2(e0, e1), Mma16<__half>::pack2(e2, e3));
                 }
             }
-            m_t = m;
             l_t = rows4_sum(lloc);
+            m_t = l_t == 0.f ? m : ms;   // as in the narrow kernel
         }
         // ---- weighted V sum on the matrix pipe: this wavefront's dims over all keys of the tile.  Lane
         //      16 q + g (g < G) ends up with dims 16 (kDb wave + b2) + 4 q .. + 3 of head g.

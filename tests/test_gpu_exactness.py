@@ -485,6 +485,31 @@ def test_a_share_of_the_keys_with_nothing_but_nan_reaches_its_rows(H, KVH, W, C,
     assert torch.isfinite(out[:, :G].float()).all() and torch.isfinite(scores[:, 0].float()).all()
 
 
+def check_nan_keys(H, KVH, D, W, C, filled, Q, dtype, where, **kw):
+    """Keys of kv head 1 that are all NaN, the cached ones or the chunk's: its rows are NaN and so are the chunk's scores; no others are."""
+    from cascading_kv_cache_amd.cascade_attention import cascade_attention
+
+    cache, q, k, v, inv_freq = cascade_case(1, H, KVH, D, 4, W, C, filled, Q, dtype)
+    for t in (cache.key_cache[0], cache.sink_keys[0]) if where == "cached" else (k,):
+        t[:, 1] = NAN
+    G = H // KVH
+    for update in (False, True, True):   # a step of one token: from the second update on it runs beside the scores
+        if where == "cached":            # where the last token's own key has gone in the meantime
+            cache.key_cache[0][:, 1] = NAN
+        out, scores = cascade_attention(q, k, v, cache, 0, inv_freq, update_cache=update, **kw)
+        assert torch.isnan(out[:, G:2 * G]).all() and torch.isnan(scores[:, 1]).all()
+        assert torch.isfinite(out[:, :G].float()).all() and torch.isfinite(scores[:, 0].float()).all()
+
+
+@pytest.mark.parametrize("dtype", [BF16, F16, F32])
+@pytest.mark.parametrize("where", ["cached", "chunk"])
+@pytest.mark.parametrize("do_og_pos", [False, True])
+@pytest.mark.parametrize("H,KVH,W,C,filled", [(8, 2, 64, 1, 40), (8, 2, 512, 4, 100), (14, 2, 512, 4, 1500), (32, 8, 4096, 4, 9000)])
+def test_nan_keys_in_a_single_token_step(H, KVH, W, C, filled, where, do_og_pos, dtype):
+    """Whole tiles of them, also as the only tile with a visible key."""
+    check_nan_keys(H, KVH, 128, W, C, filled, 1, dtype, where, do_og_pos=do_og_pos)
+
+
 @pytest.mark.parametrize("D,dtype", [(128, BF16), (128, F16), (64, F16), (128, F32)])
 @pytest.mark.parametrize("H,KVH,W,C,filled,Q", [(8, 2, 1024, 4, 1000, 128), (32, 8, 1024, 4, 4095, 300), (8, 2, 2048, 8, 3000, 33),
                                                 (7, 1, 64, 2, 90, 40)])
