@@ -222,7 +222,7 @@ __global__ void __launch_bounds__(256) fwd_generic_kernel(CoreProblem p) {
         }
         float cmax = s;
         for (int off = 32; off > 0; off >>= 1) cmax = fmaxf(cmax, __shfl_xor(cmax, off));
-        if (cmax == -INFINITY) continue;  // nothing visible in this chunk
+        if (cmax == -INFINITY && __ballot(isnan(s)) == 0ull) continue;  // nothing visible in this chunk (a maximum passes NaN over)
         const float m_new = fmaxf(m_run, cmax);
         const float pe = valid ? expf(s - m_new) : 0.f;
         float csum = pe;
@@ -357,7 +357,7 @@ __global__ void __launch_bounds__(256) fwd_generic_rows_kernel(CoreProblem p) {
             const float s = valid ? acc[i] * p.scale : -INFINITY;
             float cmax = s;
             for (int off = 32; off > 0; off >>= 1) cmax = fmaxf(cmax, __shfl_xor(cmax, off));
-            if (cmax == -INFINITY) continue;  // nothing visible in this chunk
+            if (cmax == -INFINITY && __ballot(isnan(s)) == 0ull) continue;  // nothing visible in this chunk (a maximum passes NaN over)
             const float m_new = fmaxf(m_run[i], cmax);
             const float pe = valid ? expf(s - m_new) : 0.f;
             float csum = pe;

@@ -510,6 +510,14 @@ def test_nan_keys_in_a_single_token_step(H, KVH, W, C, filled, where, do_og_pos,
     check_nan_keys(H, KVH, 128, W, C, filled, 1, dtype, where, do_og_pos=do_og_pos)
 
 
+@pytest.mark.parametrize("D,Q,dtype", [(64, 1, BF16), (64, 1, F16), (96, 1, F32), (96, 33, F32), (96, 33, BF16), (40, 2, F32), (192, 70, F16),
+                                       (64, 33, BF16), (128, 40, F16), (64, 70, F32), (128, 33, F32)])
+@pytest.mark.parametrize("where", ["cached", "chunk"])
+@pytest.mark.parametrize("W,C,filled", [(64, 1, 40), (64, 1, 60), (512, 4, 100), (512, 4, 1500)])   # 44 and 64 visible keys: part of a
+def test_nan_keys_at_any_head_size(W, C, filled, where, D, Q, dtype):                               # chunk of 64 and all of it
+    check_nan_keys(8, 2, D, W, C, filled, Q, dtype, where)
+
+
 @pytest.mark.parametrize("D,dtype", [(128, BF16), (128, F16), (64, F16), (128, F32)])
 @pytest.mark.parametrize("H,KVH,W,C,filled,Q", [(8, 2, 1024, 4, 1000, 128), (32, 8, 1024, 4, 4095, 300), (8, 2, 2048, 8, 3000, 33),
                                                 (7, 1, 64, 2, 90, 40)])
