@@ -6,13 +6,14 @@
 // and of infinite values are no numbers.  A part of a tile with a value that is not zero and below 2^-100, or past 3.38e38, is
 // staged raw: its bits, eleven to a plane, as finite bfloat16 numbers.  Blocks of keys that meet a raw part, and those in which a row has
 // a probability below 2^-100 of its largest (2^-126 for the score sums, which have no planes of it), are worked out by the
-// float32 instruction from the operands put together, with exponentials down to the smallest subnormal number.  What that costs the others (32 heads x 256 rows x 516 + 256 keys x 128): 0.2 us
-// of the forward kernel's 26 and 0.6 of the score kernel's 16.
+// float32 instruction from the operands put together, with exponentials down to the smallest subnormal number.  What that costs
+// the others (32 heads x 256 rows x 516 + 256 keys x 128): half a microsecond each of the forward kernel's 26 and the score kernel's 16.
 //
-// 32 heads x 256 rows x 516 + 256 keys x 128, us: forward 45.8 -> 27.5 (1.2 MB of operands a workgroup from the L2, 16 TB/s in all,
-// and the first pass through the loop's instructions), scores 30.8 -> 18.4 (products and vector work one behind the other: exponentials
-// beside the next tile's products measured the same), staging 10.3 -> 15 (5.5 of it stores: 1.5 times the bytes); a whole
-// call 97.1 -> 74.9, 512 rows x 2052 + 512 keys 222 + 156 + 16 -> 127 + 88 + 19.  Relative error against float64, 2-norm: output
+// 32 heads x 256 rows x 516 + 256 keys x 128, us, on the float32 instruction and now: forward 44.0 -> 26.5 (1.2 MB of operands a
+// workgroup from the L2, 16 TB/s in all, and the first pass through the loop's instructions), scores 29.8 -> 16.6 (products and vector
+// work one behind the other: exponentials beside the next tile's products measured the same), staging 10.1 -> 15.1 (5.5 of it stores:
+// 1.5 times the bytes); a whole call with its update 97.3 -> 70.9 (4.5 of it by a launch less in the update), 512 rows x
+// 2052 + 512 keys 207 + 147 + 15 -> 128 + 85 + 19.  Relative error against float64, 2-norm: output
 // 4.4e-7 -> 2.3e-7, new scores 1.7e-7 -> 0.5e-7 (a row's largest logit and sum reach the scores apart, not as one logarithm).
 //
 // Why: the float32 instruction (32x32x2) takes 64 cycles for 2 terms of a sum and vector instructions do not run beside
@@ -163,7 +164,8 @@ __device__ inline void mma_planes(const uint4 (&a)[kPlanes], const uint4 (&b)[kP
     large = mma(a[0], b[0], large);
 }
 
-// Logits, their maxima and the normalisers between the kernels are to the base 2: the staged queries carry log2 e.
+// Logits, their maxima and the normalisers between the kernels are to the base 2: the staged queries carry log2 e.  (So logits past 2.35e38
+// overflow, of the 3.4e38 that float32 holds.)
 __device__ inline float exp2_fast(float x) { return __builtin_amdgcn_exp2f(x); }   // results below the smallest normal number are zero
 constexpr float kFaint = -100.f;   // a probability's logit below the largest, from which on its planes would lose bits
 
@@ -882,15 +884,17 @@ __global__ void __launch_bounds__(Col<kGroups>::kWaves* CKV_WAVE, 2) colsum_f32_
         const bool second = kAcc == 2 && ((t - t_own) & 2);
         const float before = second ? acc[kAcc - 1] : acc[0];
         float a = before, low = 0.f;   // the smallest logit of a row that sees the key, less the row's largest
-        if (all_see(t)) {
 #pragma unroll
-            for (int v = 0; v < 16; v++) low = fminf(low, s[v] - top[v]);
-        } else {
+        for (int v = 0; v < 16; v++) {
+            const float x = s[v] - top[v];
+            low = fminf(low, x);
+            a = fmaf(w[v] * inv[v], exp2_fast(x), a);
+        }
+        if (low == -INFINITY) {   // as a row that does not see it has it
+            low = 0.f;
 #pragma unroll
             for (int v = 0; v < 16; v++) low = fminf(low, top[v] == INFINITY ? 0.f : s[v] - top[v]);
         }
-#pragma unroll
-        for (int v = 0; v < 16; v++) a = fmaf(w[v] * inv[v], exp2_fast(s[v] - top[v]), a);
         // a key that nobody sees may come out as anything
         if (__builtin_expect(__ballot(odd != 0u || (live && (!isfinite(a) || low < -126.f))) != 0ull, 0)) {
             s = plain_logits(t, stage);
