@@ -616,8 +616,8 @@ def run_gpu_config1(device):
     dt = min(stream() for _ in range(3))
     assert cache._seen_host[0] == 4096 and not bool(cache.mask[0].any())
     return dict(value=4096 / dt, unit="tokens/s", seconds=dt, dtype="f32",
-                sample="config 1 in full on the device: 4096 tokens in 16 chunks of 256, float32 (float32 "
-                       "matrix instructions); best of 3 streams")
+                sample="config 1 in full on the device: 4096 tokens in 16 chunks of 256, float32 (bfloat16 "
+                       "matrix instructions, three planes an operand); best of 3 streams")
 
 
 def run_short_strides(cache, dtype, device):
