@@ -477,4 +477,7 @@ _OWN = {name: getattr(CascadingKVCache, name) for name in ("update_state", "get_
 
 def own(cache, *names) -> bool:
     """Are these methods of ``cache`` the ones above?  What a subclass, a wrapper or a caller put in their place is to be called."""
-    return all(getattr(getattr(cache, name), "__func__", None) is _OWN[name] for name in names)
+    for name in names:
+        if getattr(getattr(cache, name), "__func__", None) is not _OWN[name]:
+            return False
+    return True
