@@ -224,6 +224,8 @@ def lib():
         L.ckv_update.restype = C.c_int
         L.ckv_gated_silu.argtypes = [VP, VP, I64, I64, I64, C.c_int32, VP]
         L.ckv_gated_silu.restype = C.c_int
+        L.ckv_linear_rows.argtypes = [VP, VP, VP, VP, VP, C.c_float, VP, I64, I64, I64, I64, C.c_int32, C.c_int32, C.c_int32, C.c_int32, VP]
+        L.ckv_linear_rows.restype = C.c_int
         L.ckv_update_row.argtypes = [C.POINTER(UpdateArgs), VP, I64, VP]
         L.ckv_update_row.restype = C.c_int
         L.ckv_update_static.argtypes = [C.POINTER(UpdateArgs), VP]

@@ -353,14 +353,17 @@ class CascadeAttention(nn.Module):
         query_states, key_states, value_states = self.qkv(
             hidden_states, (bsz, q_len, self.num_heads, self.head_dim),
             (bsz, q_len, self.num_key_value_heads, self.head_dim))
-        if not hasattr(self, "_inv_freq") or self._inv_freq.device != hidden_states.device:
-            self._inv_freq = default_inv_freq(self.head_dim, self.rope_theta, hidden_states.device)
+        out = self.o_proj(self.attend(query_states, key_states, value_states, past_key_value, homogeneous_heads, do_og_pos))
+        return out, None, past_key_value
+
+    def attend(self, query_states, key_states, value_states, past_key_value, homogeneous_heads, do_og_pos):
+        """What lies between the projections: ``(batch, heads, tokens, head_dim)`` in, ``(batch, tokens, hidden)`` out."""
+        if not hasattr(self, "_inv_freq") or self._inv_freq.device != query_states.device:
+            self._inv_freq = default_inv_freq(self.head_dim, self.rope_theta, query_states.device)
         out, _ = cascade_attention(query_states, key_states, value_states, past_key_value, self.layer_idx,
                                    self._inv_freq, head_reduction=self.config._head_reduction,
                                    homogeneous_heads=homogeneous_heads, do_og_pos=do_og_pos)
-        out = out.transpose(1, 2).contiguous().view(bsz, q_len, -1)
-        out = self.o_proj(out)
-        return out, None, past_key_value
+        return out.transpose(1, 2).contiguous().view(out.size(0), out.size(2), -1)
 
     # -- the reference mixin's remaining surface -------------------------------------------------------------
     # ``forward_cascade`` above never calls these (the fused operator rotates, concatenates and reduces inside

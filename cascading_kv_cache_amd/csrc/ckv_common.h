@@ -63,6 +63,13 @@ struct Elem<__half> {
     __device__ static __half from_float(float v) { return __float2half(v); }
 };
 
+// silu(gate) * up, rounded as the two operations are that it stands for
+template <typename T>
+__device__ inline T gated(T gate, T up) {
+    const float x = Elem<T>::to_float(gate), s = Elem<T>::to_float(Elem<T>::from_float(x / (1.f + expf(-x))));
+    return Elem<T>::from_float(s * Elem<T>::to_float(up));
+}
+
 // stage timing hooks (ckv_profile_enable / ckv_profile_read); no-ops while disabled
 void prof_begin(int stage, hipStream_t stream);
 void prof_end(int stage, hipStream_t stream);

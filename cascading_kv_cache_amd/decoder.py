@@ -4,8 +4,9 @@ strides, then greedy decoding one token at a time (cascade/models/cascade_attent
 
 The reference patches Hugging Face Llama / Qwen2 models; this module carries just enough of such a
 decoder (embedding, RMSNorm, gated MLP, untied head; projections with optional bias) to run the
-benchmark shapes end to end with random weights.  Everything outside attention is plain PyTorch but the
-gate of a fused MLP; attention, scores and the cache are the library's (:class:`ProjectedCascadeAttention`).
+benchmark shapes end to end with random weights.  Attention, scores and the cache are the library's
+(:class:`ProjectedCascadeAttention`), and so are, once the projections are fused, the gate and the products of a decoding step
+(``row_products.py``); everything else is plain PyTorch.
 
     python -m cascading_kv_cache_amd.decoder --preset llama3.1-8b --layers 4 --prompt 16384 --stride 4096 --new 32
 """
@@ -17,9 +18,9 @@ from dataclasses import dataclass, replace
 import torch
 from torch import nn
 
-from . import _abi
-from .cascading_cache import CascadingKVCache, on_device, raw_stream
+from .cascading_cache import CascadingKVCache
 from .latency import ProjectedCascadeAttention
+from .row_products import FAST_ORDER, MAX_ROWS, ROW_TYPES, followed as _followed, gated_silu, library_orders, plain, row_linear
 
 
 @dataclass
@@ -61,33 +62,6 @@ class RMSNorm(nn.Module):
         return self.weight * xf.to(x.dtype)
 
 
-_GATED_TYPES = (torch.bfloat16, torch.float16, torch.float32)
-# not public: where torch lacks one of them, somebody may be following
-_function_modes = getattr(torch._C, "_len_torch_function_stack", lambda: 1)
-_dispatch_modes = getattr(torch._C, "_len_torch_dispatch_stack", lambda: 1)
-_functorch_levels = getattr(getattr(torch._C, "_functorch", None), "peek_interpreter_stack", lambda: 1)
-
-
-def _followed(x) -> bool:
-    """May anybody follow torch's operations on ``x``: gradients of either mode, vmap, tracing, a tensor subclass, a mode?"""
-    return (type(x) is not torch.Tensor or torch.is_grad_enabled() or x.requires_grad or _function_modes() != 0 or _dispatch_modes() != 0
-            or getattr(torch.autograd.forward_ad, "_current_level", 0) >= 0 or _functorch_levels() is not None
-            or torch.jit.is_tracing() or torch.compiler.is_compiling())
-
-
-def gated_silu(gate_up):
-    """``silu(gate) * up`` of rows of ``gate | up``: one launch of the library, the same bits, where nobody follows what is done."""
-    if gate_up.device.type != "cuda" or not gate_up.is_contiguous() or gate_up.dtype not in _GATED_TYPES or _followed(gate_up):
-        gate, up = gate_up.chunk(2, dim=-1)
-        return nn.functional.silu(gate) * up
-    inter = gate_up.size(-1) // 2
-    out = torch.empty(gate_up.shape[:-1] + (inter,), dtype=gate_up.dtype, device=gate_up.device)
-    with on_device(gate_up.device):
-        _abi.check(_abi.lib().ckv_gated_silu(gate_up.data_ptr(), out.data_ptr(), gate_up.numel() // (2 * inter), inter, 2 * inter,
-                                             _abi.dtype_code(gate_up.dtype), raw_stream(gate_up.device)), "ckv_gated_silu")
-    return out
-
-
 class GatedMLP(nn.Module):
     def __init__(self, cfg, dtype, device):
         super().__init__()
@@ -122,8 +96,27 @@ class DecoderLayer(nn.Module):
         self.mlp = GatedMLP(cfg, dtype, device)
         self.input_layernorm = RMSNorm(cfg.hidden_size, cfg.rms_eps, dtype, device)
         self.post_attention_layernorm = RMSNorm(cfg.hidden_size, cfg.rms_eps, dtype, device)
+        self._orders = None   # of the products of few rows, see CascadeDecoder.fuse_projections
+
+    def _as_rows(self, x, cache) -> bool:
+        """Are these few rows whose operations nobody follows, and is every module its own?"""
+        attn, mlp = self.self_attn, self.mlp
+        return (self._orders is not None and x.dim() == 3 and x.size(0) * x.size(1) in self._orders["any"] and x.is_cuda and not _followed(x)
+                and not torch.is_autocast_enabled() and isinstance(cache, CascadingKVCache)
+                and plain(attn, ProjectedCascadeAttention, "forward_cascade", "qkv", "attend") and plain(mlp, GatedMLP)
+                and attn._w_qkv is not None and mlp._w_gate_up is not None
+                and plain(attn.o_proj, nn.Linear) and plain(mlp.down_proj, nn.Linear)
+                and attn.o_proj.bias is None and mlp.down_proj.bias is None
+                and all(plain(norm, RMSNorm) and norm.fused for norm in (self.input_layernorm, self.post_attention_layernorm)))
 
     def forward(self, x, cache):
+        if self._as_rows(x, cache):   # five launches around attention's instead of eleven
+            attn, mlp, orders = self.self_attn, self.mlp, self._orders
+            qkv = row_linear(x, attn._w_qkv, orders["qkv"], bias=attn._b_qkv, norm=self.input_layernorm)
+            x = row_linear(attn.attend(*attn.split_qkv(qkv), cache, attn.config._homogeneous_heads, attn.config._do_og_pos),
+                           attn.o_proj.weight, orders["o"], residual=x)
+            hidden = row_linear(x, mlp._w_gate_up, orders["gate_up"], norm=self.post_attention_layernorm, gated=True)
+            return row_linear(hidden, mlp.down_proj.weight, orders["down"], residual=x)
         x = x + self.self_attn(self.input_layernorm(x), use_cache=True, past_key_value=cache)[0]
         return x + self.mlp(self.post_attention_layernorm(x))
 
@@ -159,6 +152,11 @@ class CascadeDecoder(nn.Module):
             layer.mlp.fuse_projections()
             layer.input_layernorm.fused = layer.post_attention_layernorm.fused = True
         self.norm.fused = True
+        for layer in self.layers:
+            attn, mlp = layer.self_attn, layer.mlp
+            layer._orders = dict(qkv=library_orders(attn._w_qkv, attn._b_qkv), o=library_orders(attn.o_proj.weight),
+                                 gate_up=library_orders(mlp._w_gate_up), down=library_orders(mlp.down_proj.weight))
+            layer._orders["any"] = set().union(*layer._orders.values())
         return self
 
     def new_cache(self, window, cascades, batch=1, num_sink_tokens=64, **kw):
@@ -181,6 +179,9 @@ class CascadeDecoder(nn.Module):
             x = layer(x, cache)
         if last_only:
             x = x[:, -1:]
+        if (self.norm.fused and x.is_cuda and 0 < x.size(0) * x.size(1) <= MAX_ROWS and not _followed(x) and not torch.is_autocast_enabled()
+                and plain(self.norm, RMSNorm) and plain(self.lm_head, nn.Linear) and x.dtype in ROW_TYPES):
+            return row_linear(x, self.lm_head.weight, {x.size(0) * x.size(1): FAST_ORDER}, bias=self.lm_head.bias, norm=self.norm)
         return self.lm_head(self.norm(x))
 
 

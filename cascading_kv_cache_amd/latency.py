@@ -62,8 +62,14 @@ class ProjectedCascadeAttention(CascadeAttention):
     def qkv(self, x, size, kv_size):
         if self._w_qkv is None:
             return super().qkv(x, size, kv_size)
+        return self.split_qkv(nn.functional.linear(x, self._w_qkv, self._b_qkv), size, kv_size)
+
+    def split_qkv(self, rows, size=None, kv_size=None):
+        """Rows of ``q | k | v`` as ``qkv`` returns them."""
+        size = size or (*rows.shape[:2], self.num_heads, self.head_dim)
+        kv_size = kv_size or (*rows.shape[:2], self.num_key_value_heads, self.head_dim)
         n_q, n_kv = self.q_proj.weight.size(0), self.k_proj.weight.size(0)
-        q, k, v = nn.functional.linear(x, self._w_qkv, self._b_qkv).split((n_q, n_kv, n_kv), dim=-1)
+        q, k, v = rows.split((n_q, n_kv, n_kv), dim=-1)
         return q.view(*size).transpose(1, 2), k.view(*kv_size).transpose(1, 2), v.view(*kv_size).transpose(1, 2)
 
 

@@ -1,0 +1,136 @@
+"""Products of a few rows: the projections of a decoding step, each with what surrounds it in a decoder layer (norm in front; bias,
+gate or residual behind) in one launch of the library, the same bits as the operations it stands for.
+
+A product's bits hang on the order its float32 sums are added up in, and a rounding that flips in one hidden state is a percent of
+the logits of a decoder of random weights further on.  So the library's kernel is used where one of the orders it knows is that of
+torch's product of the same sizes (:func:`library_orders` tries them, once, when a decoder fuses its projections), and torch's product
+stays everywhere else.
+"""
+import torch
+from torch import nn
+
+from . import _abi
+from .cascading_cache import on_device, raw_stream
+
+ROW_TYPES = (torch.bfloat16, torch.float16)
+_GATED_TYPES = (torch.bfloat16, torch.float16, torch.float32)
+#: (parts, unit) of ``ckv_linear_rows``
+ORDERS = ((1, 1), (4, 1), (4, 2), (2, 2))
+#: of a product whose roundings nothing is computed from (the head of a decoder): the fastest, 128256 x 4096 in bf16 158 us, (1, 1) 176
+FAST_ORDER = (4, 1)
+MAX_ROWS = 16
+# not public: where torch lacks one of them, somebody may be following
+_function_modes = getattr(torch._C, "_len_torch_function_stack", lambda: 1)
+_dispatch_modes = getattr(torch._C, "_len_torch_dispatch_stack", lambda: 1)
+_functorch_levels = getattr(getattr(torch._C, "_functorch", None), "peek_interpreter_stack", lambda: 1)
+
+
+def followed(x) -> bool:
+    """May anybody follow torch's operations on ``x``: gradients of either mode, vmap, tracing, a tensor subclass, a mode?"""
+    return (type(x) is not torch.Tensor or torch.is_grad_enabled() or x.requires_grad or _function_modes() != 0 or _dispatch_modes() != 0
+            or getattr(torch.autograd.forward_ad, "_current_level", 0) >= 0 or _functorch_levels() is not None
+            or torch.jit.is_tracing() or torch.compiler.is_compiling())
+
+
+def plain(module, kind, *methods) -> bool:
+    """Is calling ``module`` nothing but ``kind.forward`` (and the named methods ``kind``'s own): no subclass, no hooks, no method put on
+    the object?"""
+    every = nn.modules.module
+    return (type(module) is kind and not module._forward_hooks and not module._forward_pre_hooks
+            and not getattr(every, "_global_forward_hooks", True) and not getattr(every, "_global_forward_pre_hooks", True)
+            and not any(name in module.__dict__ for name in ("forward", *methods)))
+
+
+def gated_silu(gate_up):
+    """``silu(gate) * up`` of rows of ``gate | up``: one launch of the library, the same bits, where nobody follows what is done."""
+    if gate_up.device.type != "cuda" or not gate_up.is_contiguous() or gate_up.dtype not in _GATED_TYPES or followed(gate_up):
+        gate, up = gate_up.chunk(2, dim=-1)
+        return nn.functional.silu(gate) * up
+    inter = gate_up.size(-1) // 2
+    out = torch.empty(gate_up.shape[:-1] + (inter,), dtype=gate_up.dtype, device=gate_up.device)
+    with on_device(gate_up.device):
+        _abi.check(_abi.lib().ckv_gated_silu(gate_up.data_ptr(), out.data_ptr(), gate_up.numel() // (2 * inter), inter, 2 * inter,
+                                             _abi.dtype_code(gate_up.dtype), raw_stream(gate_up.device)), "ckv_gated_silu")
+    return out
+
+
+def _fits(rows, n, k, order, norm) -> bool:
+    """Sizes that ``ckv_linear_rows`` takes: the rows, the norm's weights and a ring of stages share the LDS of a compute unit."""
+    ring = {1: 4 * 4, 2: 2 * 12, 4: 4 * 6}[order[0]] * 2048
+    return 0 < rows <= MAX_ROWS and n % 16 == 0 and k % 64 == 0 and ring + rows * (2 * k + 16) + 2 * k * norm + 256 <= 160 * 1024
+
+
+def _at(t) -> int:
+    return 0 if t is None else t.data_ptr()
+
+
+def linear_rows(x, weight, order, bias=None, residual=None, norm=None, eps=0.0, gated=False):
+    """``ckv_linear_rows`` of ``x (B, q, k)``, whose rows lie a fixed stride apart."""
+    n, k = weight.shape
+    out = torch.empty(x.shape[:-1] + (n // 2 if gated else n,), dtype=x.dtype, device=x.device)
+    stride = x.stride(0) if x.size(1) == 1 else x.stride(1)
+    with on_device(x.device):
+        _abi.check(_abi.lib().ckv_linear_rows(x.data_ptr(), weight.data_ptr(), _at(bias), _at(residual), _at(norm), eps, out.data_ptr(),
+                                              x.size(0) * x.size(1), n, k, max(stride, k), int(gated), order[0], order[1],
+                                              _abi.dtype_code(x.dtype), raw_stream(x.device)), "ckv_linear_rows")
+    return out
+
+
+def _rows_apart(x) -> bool:
+    """Are the rows of ``x (B, q, k)`` contiguous, a fixed stride of whole 16-byte pieces apart, and aligned?"""
+    if x.dim() != 3 or x.stride(2) != 1 or x.data_ptr() % 16:
+        return False
+    b, q, k = x.shape
+    sb, sq, _ = x.stride()
+    return (b == 1 or (sb if q == 1 else sq * q) == sb) and (b * q == 1 or (sb if q == 1 else sq) % 8 == 0) and (q == 1 or sq >= k) and (b == 1 or sb >= k)
+
+
+def _operand(t, x, *shape) -> bool:
+    return (type(t) in (torch.Tensor, nn.Parameter) and t.dtype == x.dtype and t.device == x.device and t.shape == shape and t.is_contiguous()
+            and t.data_ptr() % 16 == 0)
+
+
+def row_linear(x, weight, orders, bias=None, norm=None, residual=None, gated=False):
+    """``residual + linear(norm(x))``, or the gate of it, of ``x (B, q, k)`` (nobody follows, see :func:`followed`): one launch where
+    ``orders`` (rows: order) has one for so many rows.  ``norm``: a fused RMSNorm module."""
+    rows, (n, k) = x.size(0) * x.size(1), weight.shape   # three dimensions: the callers ask
+    order = orders.get(rows)
+    if (order is not None and x.size(2) == k and (order[0] == 1 or not gated) and _fits(rows, n, k, order, norm is not None) and _rows_apart(x)
+            and _operand(weight, x, n, k) and (bias is None or _operand(bias, x, n)) and (norm is None or _operand(norm.weight, x, k))
+            and (residual is None or _operand(residual, x, x.size(0), x.size(1), n))):
+        return linear_rows(x, weight, order, bias, residual, None if norm is None else norm.weight, 0.0 if norm is None else norm.eps, gated)
+    y = nn.functional.linear(x if norm is None else norm(x), weight, bias)
+    if gated:
+        y = gated_silu(y)
+    return y if residual is None else residual + y
+
+
+#: what library_orders has found, by device, type and sizes: facts about torch's products, not about a weight
+_FOUND = {}
+
+
+def library_orders(weight, bias=None, most_rows=4):
+    """``{rows: order}`` whose bits are those of ``torch.nn.functional.linear`` for so many rows of 16 bits, found by trying: at least
+    eight random rows each, more while two orders agree (a wrong order differs in about one output of 4096 a row).  2 ms a size, once."""
+    if weight.device.type != "cuda" or weight.dtype not in ROW_TYPES or not weight.is_contiguous():
+        return {}
+    n, k = weight.shape
+    key = (weight.device, weight.dtype, n, k, bias is not None, most_rows)
+    if key in _FOUND:
+        return _FOUND[key]
+    if torch.cuda.is_current_stream_capturing():
+        return {}
+    orders = {}
+    gen = torch.Generator(device=weight.device).manual_seed(n + k)
+    with torch.no_grad():
+        for rows in range(1, most_rows + 1):
+            left, tried = [o for o in ORDERS if _fits(rows, n, k, o, False)], 0
+            while left and (tried < 8 or (len(left) > 1 and tried < 32)):
+                x = torch.randn(rows, 1, k, generator=gen, device=weight.device).to(weight.dtype)
+                want = nn.functional.linear(x, weight, bias)
+                left = [o for o in left if torch.equal(linear_rows(x, weight, o, bias), want)]
+                tried += rows
+            if left:
+                orders[rows] = left[0]
+    _FOUND[key] = orders
+    return orders

@@ -319,6 +319,16 @@ int ckv_chunk_positions(const int64_t* key_pos, int64_t n_key, int64_t key_shift
  * two projections are one matrix product, each of the two operations rounded to the tensor dtype. */
 int ckv_gated_silu(const void* gate_up, void* out, int64_t rows, int64_t inter, int64_t row_stride, int32_t dtype, void* stream);
 
+/* out = x W^T of a few rows (a decoding step's projections), x (rows <= 16, k), W (n, k) contiguous, 16-bit, n % 16 == 0, k % 64 == 0,
+ * x and W 16-byte aligned.  Optional: `norm` (k): RMSNorm of the rows with `eps` in front, rounded to the tensor dtype; `bias` (n), added
+ * in float32; `residual` (rows, n), added to the rounded product; `gated`: W holds n / 2 gate rows and n / 2 up rows, out
+ * (rows, n / 2) = silu(gate) * up as ckv_gated_silu has it (no bias or residual then; parts 1).  The float32 sum of an output is made of
+ * `parts` chains of matrix instructions, added in order: part p takes stretches p, p + parts, ... of `unit` * 64 elements; (parts, unit)
+ * is (1, 1), (2, 2), (4, 1) or (4, 2). */
+int ckv_linear_rows(const void* x, const void* w, const void* bias, const void* residual, const void* norm, float eps, void* out,
+                    int64_t rows, int64_t n, int64_t k, int64_t x_stride, int32_t gated, int32_t parts, int32_t unit, int32_t dtype,
+                    void* stream);
+
 /* ------------------------------------------------------------------------------------------
  * Stage timing (the reference's BENCHMARK=True switch, cascading_cache.py:986-1026, extended to
  * every kernel stage).  While enabled, each stage of ckv_attn / ckv_update is bracketed by HIP

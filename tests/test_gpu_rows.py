@@ -1,0 +1,94 @@
+"""Products of a few rows (``ckv_linear_rows``) and the decoder's steps that use them."""
+from dataclasses import replace
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+from cascading_kv_cache_amd import row_products as rp
+
+pytestmark = pytest.mark.gpu
+
+HALF_ULP = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}   # of 7 and 10 fraction bits
+
+
+def operands(rows, n, k, dtype, seed=0):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    rand = lambda *s: torch.randn(*s, generator=g, device="cuda").to(dtype)   # noqa: E731
+    return rand(rows, 1, k), rand(n, k) * 0.1, rand(n), rand(rows, 1, n), 1 + 0.1 * rand(k)
+
+
+def bound(x, w, dtype):
+    """One rounding of the result, float32 sums of k products in any order, and float16's smallest step."""
+    size = x.double().abs() @ w.double().abs().T
+    return HALF_ULP[dtype] * (x.double() @ w.double().T).abs() + x.size(-1) * 2.0 ** -24 * size + 2.0 ** -24
+
+
+# one group and part of a workgroup's, fewer stretches than parts or stages, remainders of both; the largest rows that fit
+@pytest.mark.parametrize("order", rp.ORDERS)
+@pytest.mark.parametrize("rows,n,k", [(1, 16, 64), (2, 48, 128), (16, 80, 192), (3, 16, 576), (1, 4096, 832), (5, 96, 1600), (1, 64, 3584),
+                                      (2, 32, 18944)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_rows_against_float64(order, rows, n, k, dtype):
+    x, w, bias, res, norm = operands(rows, n, k, dtype)
+    assert rp._fits(rows, n, k, order, False)
+    exact = x.double() @ w.double().T
+    got = rp.linear_rows(x, w, order)
+    lim = bound(x, w, dtype)
+    assert got.shape == (rows, 1, n) and ((got.double() - exact).abs() <= lim).all()
+    assert ((rp.linear_rows(x, w, order, bias).double() - exact - bias.double()).abs() <= lim + HALF_ULP[dtype] * (exact + bias.double()).abs()).all()
+    assert torch.equal(rp.linear_rows(x, w, order, residual=res), res + got)
+    if rp._fits(rows, n, k, order, True):
+        normed = F.rms_norm(x.double(), (k,), norm.double(), 1e-5)
+        err = (rp.linear_rows(x, w, order, norm=norm, eps=1e-5).double() - normed @ w.double().T).abs()
+        # each element of the normalised row is rounded once on its way
+        assert (err <= bound(normed, w, dtype) + HALF_ULP[dtype] * (normed.abs() @ w.double().abs().T)).all()
+    if order[0] == 1:
+        up = n // 32 * 16
+        if up:
+            both = rp.linear_rows(x, w[:2 * up].contiguous(), order)
+            gate, other = both.chunk(2, -1)
+            assert torch.equal(rp.linear_rows(x, w[:2 * up].contiguous(), order, gated=True), F.silu(gate) * other)
+
+
+def test_rows_a_stride_apart():
+    base = torch.randn(3, 7, 256, device="cuda").bfloat16()
+    w = torch.randn(32, 256, device="cuda").bfloat16()
+    for x in (base[:, -1:], base[:1, 2:5], base[::2, 3:4]):
+        assert rp._rows_apart(x)
+        assert torch.equal(rp.linear_rows(x, w, (1, 1)), rp.linear_rows(x.contiguous(), w, (1, 1)))
+    for x in (base[:, 1:3], base.transpose(1, 2), base[:, :1, 1:], base[:, :, ::2]):
+        assert not rp._rows_apart(x)
+
+
+@pytest.mark.parametrize("preset", ["llama3.1-8b", "qwen2-7b", "tiny"])
+def test_steps_of_a_fused_decoder_have_the_bits_of_torchs_products(preset):
+    """One layer's steps by row products where an order is torch's, and by torch's operations: the same bits in the cache, and logits that
+    differ by the order of the head's sums alone.  Hooks on a module see their calls."""
+    from cascading_kv_cache_amd.decoder import PRESETS, CascadeDecoder
+
+    cfg = replace(PRESETS[preset], num_layers=1, vocab_size=512)
+    model = CascadeDecoder(cfg, init_on_device=True).fuse_projections()
+    plain = CascadeDecoder(cfg, init_on_device=True).fuse_projections()
+    for layer in plain.layers:
+        layer._orders = None
+    if preset != "tiny":
+        assert all(model.layers[0]._orders[name] for name in ("qkv", "o", "gate_up", "down")), model.layers[0]._orders
+    for batch in (1, 2, 5):
+        ids = torch.randint(0, 512, (batch, 40), device="cuda")
+        a, b = (m.new_cache(256, 2, batch=batch, num_sink_tokens=4) for m in (model, plain))
+        with torch.no_grad():
+            for cut in [ids[:, :32]] + [ids[:, i:i + 1] for i in range(32, 40)]:
+                la, lb = model(cut, a), plain(cut, b)
+                assert (la - lb).abs().max() <= 2.0 ** -7 * lb.abs().max()
+        assert torch.equal(a.key_cache[0], b.key_cache[0]) and torch.equal(a.value_cache[0], b.value_cache[0])
+    seen = []
+    cache = model.new_cache(256, 2, num_sink_tokens=4)
+    one = ids[:1, :1]
+    with torch.no_grad():
+        for module in (model.layers[0].self_attn.o_proj, model.layers[0].mlp, model.layers[0].input_layernorm, model.norm, model.lm_head):
+            handle = module.register_forward_hook(lambda m, i, o: seen.append(m))
+            model(one, cache)
+            handle.remove()
+            assert seen and seen[-1] is module
+    model(one, cache).sum().backward() if preset == "tiny" else None   # gradients take torch's operations
