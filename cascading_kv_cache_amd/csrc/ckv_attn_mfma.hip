@@ -1215,6 +1215,7 @@ struct ColsumParams {
     const int* key_order; // row each key came from
     void* scores;         // (B, H, N) in the tensor dtype, at the row each key came from: takes the place of colsum
     int64_t scores_stride[3];
+    int64_t empty_from, empty_to;  // as in StageParams
     int row_shares;       // the query tiles of a key block are shared out over this many workgroups (1: the block's own), each of which
     float* part;          // leaves its sums in (row_shares, B*H, N), see colsum_merge_kernel
     int wnew_uniform;     // every entry of w_new has the value wnew_value (beta rounds to one in the tensor dtype)
@@ -1283,22 +1284,6 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
     const int64_t key_blk = (int64_t)kb_i * 256;          // first key of the workgroup
     const int64_t key_w = key_blk + wave * 64;            // first key of this wavefront
 
-    uint4 kreg[2][kKK];
-    const char* kbase = (const char*)p.kr + bkv * p.n_pad * kD * (int64_t)sizeof(T);
-    bool live[2];
-    int nrel[2];
-#pragma unroll
-    for (int ks = 0; ks < 2; ks++) {
-        const int64_t n = key_w + 32 * ks + col;
-#pragma unroll
-        for (int kk = 0; kk < kKK; kk++) {
-            kreg[ks][kk] = n < p.n_pad ? *reinterpret_cast<const uint4*>(kbase + (n / kBN) * (int64_t)(kBN * kD * sizeof(T)) +
-                                                                         k_image_off((int)(n % kBN), 2 * kk + half))
-                                       : make_uint4(0, 0, 0, 0);
-        }
-        live[ks] = n < N && ((p.tile_vis[n / kBN] >> (n % kBN)) & 1ull);
-        nrel[ks] = (int)(n - Nc);
-    }
     // first query tile that can see any key of the workgroup
     int m_first = (int)(key_blk - Nc);
     if (m_first < 0) m_first = 0;
@@ -1306,13 +1291,11 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
     const bool chunk_keys = key_blk + 255 >= Nc;  // some key of the workgroup belongs to the chunk
     const int last_nrel = (int)(key_blk + 255 - Nc);
     const bool new_chunk = chunk_keys && p.new_mode;
-    const bool pure_chunk = key_blk >= Nc;        // no cached key in the workgroup
     // the weights of chunk keys by distance: a table in LDS, unless every entry is the same value (then the
     // launch reserves no LDS for it, and two workgroups fit a compute unit whatever the chunk length)
     if (new_chunk && !p.wnew_uniform) {
         for (int i = tid; i < Q; i += 256) wnew_lds[i] = p.w_new[i];
     }
-    auto wnew_at = [&](int i) -> float { return p.wnew_uniform ? p.wnew_value : wnew_lds[i]; };
     int nmt = (Q - m_first + kQT2 - 1) / kQT2;  // query tiles per head
     int m_end = Q;                              // where the workgroup's share of them ends
     if (kShares && nmt > 0) {
@@ -1321,12 +1304,6 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
         m_first += t0 * kQT2;
         nmt = t1 - t0;
     }
-    // A block without a single visible key (the empty part of a cache that is still filling) has nothing but zeros to
-    // write: with 1000 of 16384 slots filled and a 488-token chunk that is 63 of 67 blocks.
-    const unsigned long long* vis = p.tile_vis + key_blk / kBN;
-    const bool hidden = p.n_visible ? key_blk >= N : (vis[0] | vis[1] | vis[2] | vis[3]) == 0ull;
-    const int n_steps = hidden ? 0 : nmt * g_cnt;
-
     // async copy assignments: the Q tile is copied in blocks of 1 KiB (a quarter of them per wavefront); wavefront 0
     // also brings the tile's normalisers, wavefront 1 its weights (kQT2 / 4 lanes x 16 bytes each)
     constexpr int kQBlocks = kQT2 * kRowBytes / 4096;   // per wavefront
@@ -1376,6 +1353,43 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
             p.colsum[(b * p.H + h) * p.N + n] = v;
         }
     };
+    auto store_zeros = [&] {
+        for (int g = g_first; g < g_first + g_cnt; g++)
+#pragma unroll
+            for (int ks = 0; ks < 2; ks++) {
+                const int64_t n = key_w + 32 * ks + col;
+                if (half == 0 && n < p.N) store(kvh * p.G + g, n, 0.f);
+            }
+    };
+    // Slots that the host knows to be empty, whose keys were not even staged (512 rows, 1000 of 16384 slots filled: 62 of 67 blocks),
+    // and hidden keys sorted behind the visible ones: nothing is read.
+    if ((key_blk >= p.empty_from && key_blk + 256 <= p.empty_to) || key_blk >= N) {
+        store_zeros();
+        return;
+    }
+    // The first query tile, the keys and their visibility are requested side by side: a workgroup of 509 rows lives some 15 us
+    if (nmt > 0) issue(g_first, m_first, 0);
+    uint4 kreg[2][kKK];
+    const char* kbase = (const char*)p.kr + bkv * p.n_pad * kD * (int64_t)sizeof(T);
+    bool live[2];
+    int nrel[2];
+#pragma unroll
+    for (int ks = 0; ks < 2; ks++) {
+        const int64_t n = key_w + 32 * ks + col;
+#pragma unroll
+        for (int kk = 0; kk < kKK; kk++) {
+            kreg[ks][kk] = n < p.n_pad ? *reinterpret_cast<const uint4*>(kbase + (n / kBN) * (int64_t)(kBN * kD * sizeof(T)) +
+                                                                         k_image_off((int)(n % kBN), 2 * kk + half))
+                                       : make_uint4(0, 0, 0, 0);
+        }
+        live[ks] = n < N && ((p.tile_vis[n / kBN] >> (n % kBN)) & 1ull);
+        nrel[ks] = (int)(n - Nc);
+    }
+    // a block without a single visible key has nothing but zeros to write
+    const unsigned long long* vis = p.tile_vis + key_blk / kBN;
+    const bool hidden = !p.n_visible && (vis[0] | vis[1] | vis[2] | vis[3]) == 0ull;
+    const int n_steps = hidden ? 0 : nmt * g_cnt;
+
     float acc[2] = {0.f, 0.f};
     auto tile_step = [&](auto stage_tag, int g, int mt) {
         constexpr int ST = decltype(stage_tag)::value;
@@ -1488,89 +1502,86 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
                 }
             }
         } else {
-            // special cases, one 32-row subtile at a time
-            bool chunk_lane[2];
-#pragma unroll
-            for (int ks = 0; ks < 2; ks++) chunk_lane[ks] = nrel[ks] >= 0;
-            // a chunk key takes the weight of its distance m - n; a cached key (only in the block that
-            // straddles the chunk start) takes the row's EMA weight
-            auto weight_of = [&](int ks, int r) -> float {
-                return chunk_lane[ks] ? wnew_at(mt + 4 * half - nrel[ks] + r) : w_lds[4 * half + r];
-            };
+            // Tiles with chunk keys on the diagonal or with the weights of chunk keys, one 32-row subtile at a time.  How a wavefront's
+            // keys weigh is a type here and not a test by the element: as one it became a choice of addresses, 128 flat loads a
+            // subtile, each with a wait for everything in flight (512 rows, 1000 of 16384 slots filled: the kernel 52 us, now 24.5;
+            // 2 x 2048 rows x 16 K slots 560 and 540; dense, 8 x 1000 x 5095 x 64 dims 20 and 13.4).  Rows past the chunk end need
+            // no test: their probability is zero (see hide_rows).
+            const int nrel_w = (int)(key_w - Nc);   // this wavefront's first key among the chunk keys (negative: cached)
+            enum Weights { kByRow, kAlike, kMixed };
+            auto special = [&](auto weights_tag, auto uniform_tag) {
+                constexpr int kWeights = decltype(weights_tag)::value;
+                constexpr bool kUniform = decltype(uniform_tag)::value;
 #pragma unroll 1
-            for (int c = 0; c < kCsSub; c++) {
-                const int row0 = mt + 32 * c;
-                const int nrel_w = (int)(key_w - Nc);   // this wavefront's first key among the chunk keys (negative: cached)
-                if (row0 >= Q) break;
-                if (row0 + 31 < nrel_w) continue;       // before every key of the wavefront
-                const bool plain = row0 + 31 < Q && row0 >= nrel_w + 63;   // every row sees every key of the wavefront
-                const bool fast_new = plain && new_chunk;
-                f32x16 sacc[2];
-                sacc[0] = sacc[1] = row_init(c);
-                const auto nl = norms_of(c);
+                for (int c = 0; c < kCsSub; c++) {
+                    const int row0 = mt + 32 * c;
+                    if (row0 >= Q) break;
+                    if (row0 + 31 < nrel_w) continue;   // before every key of the wavefront
+                    f32x16 sacc[2];
+                    sacc[0] = sacc[1] = row_init(c);
+                    const auto nl = norms_of(c);
 #pragma unroll
-                for (int kk = 0; kk < kKK; kk++) {
-                    const uint4 a = *reinterpret_cast<const uint4*>(q_lds + q_off[kk] + c * (32 * kRowBytes));
-                    sacc[0] = Mma<T>::mma(a, kreg[0][kk], sacc[0]);
-                    sacc[1] = Mma<T>::mma(a, kreg[1][kk], sacc[1]);
-                }
-                if (fast_new && p.wnew_uniform && __builtin_amdgcn_ballot_w64(!(chunk_lane[0] && chunk_lane[1])) == 0ull) {
-                    // every key of the wavefront is a chunk key and all of them weigh the same: P and the
-                    // products are rounded to the tensor dtype two at a time by the packed conversions, and
-                    // the rounded products join the sum through a dot product with a pair of ones
-                    const float wu = p.wnew_value;
-#pragma unroll
-                    for (int v = 0; v < 16; v += 2) {
-#pragma unroll
-                        for (int ks = 0; ks < 2; ks++) {
-                            const uint32_t u = Mma<T>::pack2(prob(sacc[ks][v], nl, v), prob(sacc[ks][v + 1], nl, v + 1));
-                            acc[ks] = Mma<T>::sum2(Mma<T>::pack2(Mma<T>::lo_f(u) * wu, Mma<T>::hi_f(u) * wu), acc[ks]);
-                        }
+                    for (int kk = 0; kk < kKK; kk++) {
+                        const uint4 a = *reinterpret_cast<const uint4*>(q_lds + q_off[kk] + c * (32 * kRowBytes));
+                        sacc[0] = Mma<T>::mma(a, kreg[0][kk], sacc[0]);
+                        sacc[1] = Mma<T>::mma(a, kreg[1][kk], sacc[1]);
                     }
-                } else if (fast_new) {
-                    // no masks; the eager path holds P and the products of chunk keys in the tensor dtype
+                    // row 8 (v / 4) + v % 4 of the lane's half sees a key at distance `ahead` or less in front of row 0 of it (cached: all do)
+                    int ahead[2];
 #pragma unroll
-                    for (int v4 = 0; v4 < 4; v4++) {
-                        const int r0 = 32 * c + 8 * v4;
+                    for (int ks = 0; ks < 2; ks++) ahead[ks] = nrel[ks] - row0 - 4 * half;
+                    auto seen = [&](float e, int ks, int v) { return 8 * (v >> 2) + (v & 3) >= ahead[ks] ? e : 0.f; };
+                    if constexpr (kWeights == kAlike) {
+                        // every key of the wavefront is a chunk key and all of them weigh the same: P and the
+                        // products are rounded to the tensor dtype two at a time by the packed conversions, and
+                        // the rounded products join the sum through a dot product with a pair of ones
+                        const float wu = p.wnew_value;
+                        auto add = [&](auto masked) {
 #pragma unroll
-                        for (int e = 0; e < 4; e++) {
+                            for (int v = 0; v < 16; v += 2) {
+#pragma unroll
+                                for (int ks = 0; ks < 2; ks++) {
+                                    float e0 = prob(sacc[ks][v], nl, v), e1 = prob(sacc[ks][v + 1], nl, v + 1);
+                                    if constexpr (decltype(masked)::value) {
+                                        e0 = seen(e0, ks, v);
+                                        e1 = seen(e1, ks, v + 1);
+                                    }
+                                    const uint32_t u = Mma<T>::pack2(e0, e1);
+                                    acc[ks] = Mma<T>::sum2(Mma<T>::pack2(Mma<T>::lo_f(u) * wu, Mma<T>::hi_f(u) * wu), acc[ks]);
+                                }
+                            }
+                        };
+                        if (row0 >= nrel_w + 63) add(std::false_type{});
+                        else add(std::true_type{});
+                    } else {
+                        float we[16];
+                        load_weights(c, we);
+#pragma unroll
+                        for (int v = 0; v < 16; v++) {
 #pragma unroll
                             for (int ks = 0; ks < 2; ks++) {
-                                const float pe = prob(sacc[ks][4 * v4 + e], nl, 4 * v4 + e);
-                                const float w = weight_of(ks, r0 + e);
-                                if (pure_chunk) {
-                                    acc[ks] += Mma<T>::round1(Mma<T>::round1(pe) * w);
+                                const float pe = seen(prob(sacc[ks][v], nl, v), ks, v), as_cached = fmaf(we[v], pe, acc[ks]);
+                                if constexpr (kWeights == kByRow) {
+                                    acc[ks] = as_cached;
                                 } else {
-                                    const float prod = (chunk_lane[ks] ? Mma<T>::round1(pe) : pe) * w;
-                                    acc[ks] += chunk_lane[ks] ? Mma<T>::round1(prod) : prod;
+                                    // a chunk key takes the weight of its distance from the row; a cached key (where the chunk
+                                    // starts inside the wavefront) takes the row's EMA weight.  The eager path holds P and the
+                                    // products of chunk keys in the tensor dtype.  Both are worked out and one is picked.
+                                    const int r = 8 * (v >> 2) + (v & 3) - ahead[ks];
+                                    float w = p.wnew_value;
+                                    if constexpr (!kUniform) w = wnew_lds[nrel[ks] >= 0 && r >= 0 && r < Q ? r : 0];
+                                    const float as_new = acc[ks] + Mma<T>::round1(Mma<T>::round1(pe) * w);
+                                    acc[ks] = nrel[ks] >= 0 ? as_new : as_cached;
                                 }
                             }
                         }
                     }
-                } else {
-#pragma unroll
-                    for (int v = 0; v < 16; v++) {
-                        const int r = 32 * c + 8 * (v >> 2) + 4 * half + (v & 3);
-                        const int m = mt + r;
-                        const bool row_in = m < Q;
-                        const float we = w_lds[r];
-#pragma unroll
-                        for (int ks = 0; ks < 2; ks++) {
-                            float pe = prob(sacc[ks][v], nl, v);
-                            const bool is_chunk = nrel[ks] >= 0;
-                            const bool vis = row_in && (!is_chunk || m >= nrel[ks]);
-                            pe = vis ? pe : 0.f;
-                            if (is_chunk && p.new_mode) {
-                                // the eager path holds P and the products in the tensor dtype
-                                const float w = vis ? wnew_at(m - nrel[ks]) : 0.f;
-                                acc[ks] += Mma<T>::round1(Mma<T>::round1(pe) * w);
-                            } else {
-                                acc[ks] = fmaf(row_in ? we : 0.f, pe, acc[ks]);
-                            }
-                        }
-                    }
                 }
-            }
+            };
+            if (!p.new_mode) special(std::integral_constant<int, kByRow>{}, std::true_type{});
+            else if (!p.wnew_uniform) special(std::integral_constant<int, kMixed>{}, std::false_type{});
+            else if (nrel_w >= 0) special(std::integral_constant<int, kAlike>{}, std::true_type{});
+            else special(std::integral_constant<int, kMixed>{}, std::true_type{});
         }
         if (mt + kQT2 >= m_end) {  // head finished: combine the two lane halves and store
             const int64_t h = kvh * p.G + g;
@@ -1603,7 +1614,6 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
             g++;
         }
     };
-    if (n_steps > 0) issue(g_first, m_first, 0);
     for (int step = 0; step < n_steps; step += 2) {
         int g_n = g_cur, mt_n = mt_cur;
         advance(g_n, mt_n);
@@ -1624,13 +1634,9 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
             mt_cur = mt_n2;
         }
     }
-    if (n_steps <= 0) {  // no query can see these keys (padding blocks, and hidden keys sorted behind the visible ones)
-        for (int g = g_first; g < g_first + g_cnt; g++)
-#pragma unroll
-            for (int ks = 0; ks < 2; ks++) {
-                const int64_t n = key_w + 32 * ks + col;
-                if (half == 0 && n < p.N) store(kvh * p.G + g, n, 0.f);
-            }
+    if (n_steps <= 0) {  // no query can see these keys
+        wait_copies<0>();   // the tile that nobody reads has landed before its place goes to another workgroup
+        store_zeros();
     }
 }
 
@@ -1772,6 +1778,7 @@ int run_mfma(const MfmaProblem& mp, hipStream_t stream) {
         cp.w_ema = mp.w_ema; cp.w_new = mp.w_new; cp.colsum = mp.colsum;
         cp.B = mp.B; cp.H = mp.H; cp.KVH = mp.KVH; cp.Q = mp.Q; cp.N = n; cp.Nc = n - mp.Q; cp.n_pad = n_pad;
         cp.n_visible = mp.n_visible; cp.key_order = mp.key_order;
+        cp.empty_from = mp.empty_from; cp.empty_to = mp.empty_to;
         cp.scores = mp.scores;
         for (int j = 0; j < 3; j++) cp.scores_stride[j] = mp.scores_stride[j];
         cp.G = G;

@@ -1,0 +1,34 @@
+"""Score sums of a chunk's own keys: weights that are all alike (the default beta) and weights by distance, wavefronts whose 64 keys are
+all the chunk's and the one in which the chunk starts, lengths around the 32-row subtiles and the 128-row tiles."""
+import pytest
+import torch
+
+from oracle.attention import OracleCascadeAttention
+from parity_helpers import assert_scores_close, push_state, tol
+from test_gpu_attention import make_pair
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("D,dtype", [(128, torch.bfloat16), (128, torch.float16), (64, torch.bfloat16)])
+@pytest.mark.parametrize("NS", [3, 64])
+@pytest.mark.parametrize("beta", [None, 0.9])
+def test_scores_of_the_chunks_own_keys(beta, NS, D, dtype):
+    from cascading_kv_cache_amd.cascade_attention import cascade_attention, default_inv_freq
+
+    B, H, KVH, W, C = 1, 4, 2, 128, 8
+    gpu, cpu = make_pair(B, KVH, D, NS, W, C, dtype)
+    if beta is not None:
+        gpu.beta = cpu.beta = beta
+    layer = OracleCascadeAttention(H, KVH, D, rope_theta=5e5, head_reduction="mean")
+    inv_freq = default_inv_freq(D, 5e5, "cuda:0")
+    gen = torch.Generator().manual_seed(3)
+    for q_len in (600, 300, 33, 129, 31, 64, 97):   # the last over a cache that evicts
+        q, k, v = ((torch.randn(B, h, q_len, D, generator=gen) * 0.7).to(dtype) for h in (H, KVH, KVH))
+        push_state(gpu, cpu)
+        out, new = cascade_attention(q.cuda(), k.cuda(), v.cuda(), gpu, 0, inv_freq, update_cache=False)
+        scores = gpu.score_cache[0].cpu()
+        want = layer.forward(q, k, v, cpu)
+        assert (out.float().cpu() - want.float()).abs().max() <= tol(dtype)
+        assert_scores_close(new, layer.last_new_scores[:, :KVH], dtype, f"new-token scores, {q_len} rows")
+        assert_scores_close(scores, layer.last_score_cache, dtype, f"score cache, {q_len} rows")
