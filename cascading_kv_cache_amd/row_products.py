@@ -6,6 +6,8 @@ the logits of a decoder of random weights further on.  So the library's kernel i
 torch's product of the same sizes (:func:`library_orders` tries them, once, when a decoder fuses its projections), and torch's product
 stays everywhere else.
 """
+import math
+
 import torch
 from torch import nn
 
@@ -110,11 +112,16 @@ _FOUND = {}
 
 
 def library_orders(weight, bias=None, most_rows=4):
-    """``{rows: order}`` whose bits are those of ``torch.nn.functional.linear`` for so many rows of 16 bits, found by trying: at least
-    eight random rows each, more while two orders agree (a wrong order differs in about one output of 4096 a row).  2 ms a size, once."""
+    """``{rows: order}`` whose bits are those of ``torch.nn.functional.linear`` for so many rows of 16 bits, found by trying random rows,
+    2 ms a size, once.  Two orders differ in few outputs (4096 x 4096: one of 4000 to 6000), in proportion to the root of the products
+    summed up: enough rows are tried to expect eight differences of a wrong one, twice as many while two are left.  Products so small
+    that this would take more than 64 rows stay with torch."""
     if weight.device.type != "cuda" or weight.dtype not in ROW_TYPES or not weight.is_contiguous():
         return {}
     n, k = weight.shape
+    enough = math.ceil(3.5e6 / (n * math.sqrt(k)))
+    if enough > 64:
+        return {}
     key = (weight.device, weight.dtype, n, k, bias is not None, most_rows)
     if key in _FOUND:
         return _FOUND[key]
@@ -125,7 +132,7 @@ def library_orders(weight, bias=None, most_rows=4):
     with torch.no_grad():
         for rows in range(1, most_rows + 1):
             left, tried = [o for o in ORDERS if _fits(rows, n, k, o, False)], 0
-            while left and (tried < 8 or (len(left) > 1 and tried < 32)):
+            while left and (tried < enough or (len(left) > 1 and tried < 2 * enough)):
                 x = torch.randn(rows, 1, k, generator=gen, device=weight.device).to(weight.dtype)
                 want = nn.functional.linear(x, weight, bias)
                 left = [o for o in left if torch.equal(linear_rows(x, weight, o, bias), want)]

@@ -72,7 +72,9 @@ def test_steps_of_a_fused_decoder_have_the_bits_of_torchs_products(preset):
     plain = CascadeDecoder(cfg, init_on_device=True).fuse_projections()
     for layer in plain.layers:
         layer._orders = None
-    if preset != "tiny":
+    if preset == "tiny":   # too few outputs to tell one order from another by
+        assert not any(model.layers[0]._orders.values())
+    else:
         assert all(model.layers[0]._orders[name] for name in ("qkv", "o", "gate_up", "down")), model.layers[0]._orders
     for batch in (1, 2, 5):
         ids = torch.randint(0, 512, (batch, 40), device="cuda")
