@@ -1862,18 +1862,19 @@ int64_t mfma_n_pad(int64_t n) { return align_up(n, 256); }
 // two tiles each: 2300 x 8 K  1: 391  3: 353  8: 416.  (64 dims: 1: 503  3: 398  6: 382; masked keys of the dense operator, which
 // cost nothing, count like the others.)  With no more than a share to 16 tiles of a chunk, and to 8 of the dense operator's, a whole
 // call took, us, 32 heads on 8 kv heads, then and now:  16 rows x 1 K slots 57.8 47.5   33 x 2 K 67.1 55.7   16 x 4 K 76.4 63.7
-//   300 x 2 K 85.1 75.4   300 x 7 K 132.2 113.1   2 x 500 x 4 K 178.5 166.4   1000 x 2 K 147.9 138.8   1000 x 1 K 122.5 122.7; dense,
+//   300 x 2 K 85.1 75.4   300 x 7 K 132.2 113.1   300 x 8 K 139.0 120.6   500 x 12 K 208.0 197.4   2 x 500 x 4 K 178.5 166.4   1000 x 2 K
+//   147.9 138.8   1500 x 8 K 376.8 358.5   1000 x 1 K 122.5 122.7   200 x 10 K 115.6 115.8 (28 heads on 4: 106.0 108.5); dense,
 //   forward, 64 dims: 2 heads x 100 rows x 1000 cached keys 37.9 30.7   3 x 300 x 500 43.5 33.7   8 x 1000 x 500 49.9 47.4.
-// Twice as many shares as fill one round lose (300 x 4 K  4: 91.8  8: 102.8).
+// Twice as many shares as fill one round lose (300 x 4 K, the call  4: 91.8  8: 102.8).
 //
-// Chunks of fewer workgroups than units over caches of 8 K slots and more keep the counts that streams have always had, because a
+// Chunks of fewer workgroups than units over caches of 16 K slots and more keep the counts that streams have always had, because a
 // decoder of random weights turns the changed rounding of one hidden state into a percent of its logits: about two workgroups per
 // unit, at most 8 shares; where 8 shares would be of more than 32 tiles, the cheapest count from 8 to 32 by the estimate.  Forward +
 // merge in us, by shares:     509 rows x 16 K  4: 141  8: 155    488 x 16 K, 1000 slots filled  4: 34  8: 47
 //   128 x 64 K   8: 175  16: 134  32: 160        32 x 64 K  8: 162  16: 95  32: 90      509 x 32 K  4: 237  8: 250
 int mfma_fwd_splits(int64_t B, int64_t H, int64_t KVH, int64_t Q, int64_t n, int cus, bool dense) {
     constexpr double kTileUs = 1.6, kStartUs = 16.0, kMergeUs = 6.0, kMergeWgUs = 0.058;
-    constexpr int64_t kMaxShares = 32, kMaxShareBytes = (int64_t)256 << 20, kFew = 8, kMinTiles = 2, kMinTilesMany = 32, kManyTiles = 128;
+    constexpr int64_t kMaxShares = 32, kMaxShareBytes = (int64_t)256 << 20, kFew = 8, kMinTiles = 2, kMinTilesMany = 32, kManyTiles = 256;
     const int64_t G = H / KVH;
     const int64_t wgs = ((Q * G + kRows - 1) / kRows) * B * KVH, tiles = (n + kBN - 1) / kBN;
     if (wgs >= 4 * (int64_t)cus) return 1;   // at most an eighth of the launch can be an empty round
