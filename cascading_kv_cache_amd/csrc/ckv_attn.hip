@@ -279,10 +279,15 @@ extern "C" int ckv_attn_dense(const ckv_dense_args* args, void* stream_) {
         // touches a masked one: half the keys masked at random is half the work.
         const int64_t n_cache = a.n_kv - a.n_ctx;
         DenseWorkspace w = carve_dense(a.workspace, a.B, a.H, a.n_ctx, a.n_kv, a.D);
-        int rc = launch_dense_prologue(a.mask, n_cache, a.n_ctx, w.key_order, w.n_visible, a.scores ? w.w_ema : nullptr, w.w_new,
-                                       a.beta, a.dtype, stream);
-        if (rc) return rc;
         MfmaProblem mp;
+        mp.own_order = order_by_staging(n_cache);
+        mp.order_mask = a.mask;
+        mp.make_weights = mp.own_order && a.scores;
+        if (!mp.own_order) {
+            const int rc = launch_dense_prologue(a.mask, n_cache, a.n_ctx, w.key_order, w.n_visible, a.scores ? w.w_ema : nullptr, w.w_new,
+                                                 a.beta, a.dtype, stream);
+            if (rc) return rc;
+        }
         const MfmaSegment none{nullptr, nullptr, {0, 0, 0, 0}, nullptr, {0, 0}, 0, nullptr, 0};
         mp.seg[0] = MfmaSegment{a.k, a.v, {a.kv_stride[0], a.kv_stride[1], a.kv_stride[2], a.kv_stride[3]},
                                 nullptr, {0, 0}, 0, nullptr, a.n_kv};

@@ -202,8 +202,10 @@ struct MfmaProblem {
     int64_t scores_stride[3] = {0, 0, 0};
     float* part_scores = nullptr;  // (dense_row_shares, B*H, n): where the sums of a key are shared out, or null
     // keys in another order than they lie in memory (launch_dense_prologue): seg[0] then holds all keys
-    const int* key_order = nullptr;
-    const int* n_visible = nullptr;
+    int* key_order = nullptr;
+    int* n_visible = nullptr;
+    int own_order = 0;     // the staging launch works the order out (order_by_staging), from this mask
+    const uint8_t* order_mask = nullptr;
     float* part_o;         // (mfma_fwd_splits, B*H*Q, D) and
     float* part_l2;        // (mfma_fwd_splits, B*H*Q): the forward kernel's shares, when it splits the keys
     float* w_ema;
@@ -226,6 +228,7 @@ int64_t mfma_n_pad(int64_t n);
 int mfma_fwd_splits(int64_t B, int64_t H, int64_t KVH, int64_t Q, int64_t n, int cus, bool dense);
 int mfma_fwd_splits_for_workspace(int64_t B, int64_t H, int64_t KVH, int64_t Q, int64_t n, bool dense);
 int dense_row_shares(int64_t B, int64_t H, int64_t n_ctx, int64_t n_kv, int cus);
+bool order_by_staging(int64_t n_cached);
 int mfma_device_cus();  // compute units of the current device (256 where none can be asked)
 bool mfma_fits(int64_t n, int64_t D);  // the per-tile bookkeeping of n keys fits in LDS
 int launch_mfma(const MfmaProblem& p, hipStream_t stream);

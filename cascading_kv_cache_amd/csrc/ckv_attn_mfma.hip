@@ -128,6 +128,10 @@ struct StageParams {
     const int* key_order;
     const int* n_visible;
     int64_t n_chunk;
+    // The order is not there yet (this launch writes it, see order_by_staging): a block finds its tile's keys in the mask itself.
+    int own_order;
+    const uint8_t* order_mask;     // (n_cached), 1 = masked
+    int64_t n_cached;
     int64_t empty_from, empty_to;  // keys no query can see because their slots are still empty (none: both 0)
 };
 
@@ -169,7 +173,59 @@ struct StageLds {
         uint2 trig[kD / 16][256];
     };
     float freqs[kD / 2];
+    int picked[kBN], sums[2][4];   // see keys_of_tile
 };
+
+// The cached keys of ranks first .. first + 63 among the visible ones, into `picked`, by a workgroup of 256 threads.  Returns how many are
+// visible, or a number past the last of these ranks.
+__device__ inline int keys_of_tile(const uint8_t* mask, int n_cached, int first, int* picked, int (*sums)[4]) {
+    constexpr int kPer = 16, kStretch = 256 * kPer;
+    const int tid = threadIdx.x, lane = tid % CKV_WAVE, wave = tid / CKV_WAVE;
+    const bool vec = (reinterpret_cast<uintptr_t>(mask) & 15) == 0;
+    // this thread's 16 keys of a stretch as a word of bits, one per visible key
+    auto visible = [&](int base) -> uint32_t {
+        const int k0 = base + tid * kPer;
+        uint32_t bits = 0;
+        if (vec && k0 + kPer <= n_cached) {
+            const uint4 m = *reinterpret_cast<const uint4*>(mask + k0);
+            const uint32_t w[4] = {m.x, m.y, m.z, m.w};
+#pragma unroll
+            for (int i = 0; i < kPer; i++) bits |= (((w[i >> 2] >> (8 * (i & 3))) & 0xffu) == 0u ? 1u : 0u) << i;
+        } else {
+            for (int i = 0; i < kPer; i++)
+                if (k0 + i < n_cached && mask[k0 + i] == 0) bits |= 1u << i;
+        }
+        return bits;
+    };
+    int seen = 0, round = 0;   // visible keys in the stretches before
+    uint32_t next = n_cached > 0 ? visible(0) : 0u;
+    for (int base = 0; base < n_cached && seen < first + kBN; base += kStretch, round ^= 1) {
+        uint32_t bits = next;
+        if (base + kStretch < n_cached) next = visible(base + kStretch);
+        const int mine = __popc(bits);
+        int incl = mine;
+#pragma unroll
+        for (int off = 1; off < CKV_WAVE; off <<= 1) {
+            const int v = __shfl_up(incl, off);
+            if (lane >= off) incl += v;
+        }
+        if (lane == CKV_WAVE - 1) sums[round][wave] = incl;
+        __syncthreads();   // the sums of the next stretch go to the other half
+        int rank = seen + incl - mine;
+#pragma unroll
+        for (int w = 0; w < 4; w++) {
+            const int v = sums[round][w];
+            rank += w < wave ? v : 0;
+            seen += v;
+        }
+        if (rank < first + kBN && rank + mine > first) {
+            for (; bits; bits &= bits - 1, rank++)
+                if (rank >= first && rank < first + kBN) picked[rank - first] = base + tid * kPer + __ffs(bits) - 1;
+        }
+    }
+    __syncthreads();
+    return seen;
+}
 
 // frequencies of the rotation pairs into LDS (visible after a barrier)
 template <int kD>
@@ -213,10 +269,11 @@ __device__ inline void stage_keys_block(const StageParams& p, int tile_i, int sp
     int64_t n_all = p.n;
     if (p.key_order) {
         // visible keys first: what lies behind them is read by nobody.  The order indexes segment 0, which holds all keys.
-        n_all = *p.n_visible + p.n_chunk;
+        const int64_t vis = p.own_order ? keys_of_tile(p.order_mask, (int)p.n_cached, (int)(tile * kBN), lds.picked, lds.sums) : *p.n_visible;
+        n_all = vis + p.n_chunk;
         if (tile * kBN >= n_all) return;
         if (n < n_all) {
-            local = p.key_order[n];
+            local = !p.own_order ? p.key_order[n] : n < vis ? lds.picked[key] : p.n_cached + (n - vis);
             sidx = 0;
         }
     } else if (n < p.n) {
@@ -481,13 +538,17 @@ struct StageGrid {
 struct StageWeights {
     float *w_ema, *w_new;
     double beta;
+    int* key_order;   // written by the first block where the staging blocks find their keys themselves
+    int* n_visible;
 };
 template <typename T, int kD>
 __global__ void __launch_bounds__(256) stage_kernel(StageParams sp, StageQParams sq, StageGrid g, StageWeights sw) {
     __shared__ __align__(16) StageLds<kD> lds;
     const int nk = g.k_bx * g.k_by;
-    int id = blockIdx.x;
-    if (id < nk) {
+    int id = (int)blockIdx.x - (sp.own_order ? 1 : 0);
+    if (id < 0) {
+        key_order_block<256>(sp.order_mask, sp.n_cached, sp.n_chunk, sw.key_order, sw.n_visible);
+    } else if (id < nk) {
         stage_keys_block<T, kD>(sp, id % g.k_bx, id / g.k_bx, g.k_by, lds);
     } else {
         id -= nk;
@@ -1690,6 +1751,7 @@ int run_mfma(const MfmaProblem& mp, hipStream_t stream) {
         sp.empty_from = mp.empty_from; sp.empty_to = mp.empty_to;
         sp.B = mp.B; sp.KVH = mp.KVH; sp.n = n; sp.n_pad = n_pad;
         sp.key_order = mp.key_order; sp.n_visible = mp.n_visible; sp.n_chunk = mp.Q;
+        sp.own_order = mp.own_order; sp.order_mask = mp.order_mask; sp.n_cached = n - mp.Q;
         const int64_t nbh = mp.B * mp.KVH;
         // shared positions: a block walks several (b, kvh) units with one set of cos/sin, the next unit's rows
         // always on their way
@@ -1728,9 +1790,9 @@ int run_mfma(const MfmaProblem& mp, hipStream_t stream) {
             if (by < 1) by = 1;
             StageGrid g;
             g.q_bx = (int)bx; g.q_by = (int)by; g.k_bx = (int)(n_pad / kBN); g.k_by = (int)splits;
-            const StageWeights sw{mp.w_ema, mp.w_new, mp.beta};
+            const StageWeights sw{mp.w_ema, mp.w_new, mp.beta, mp.key_order, mp.n_visible};
             const int64_t w_blocks = mp.make_weights ? (mp.Q + kColSlack + 255) / 256 : 0;
-            const int64_t blocks = bx * by + (n_pad / kBN) * splits + w_blocks;
+            const int64_t blocks = bx * by + (n_pad / kBN) * splits + w_blocks + (mp.own_order ? 1 : 0);
             if (blocks > 0x7fffffff) return CKV_ERR_UNSUPPORTED;
             hipLaunchKernelGGL((stage_kernel<T, kD>), dim3((unsigned)blocks), dim3(256), 0, stream, sp, sq, g, sw);
         }
@@ -1851,6 +1913,13 @@ int dense_row_shares(int64_t B, int64_t H, int64_t n_ctx, int64_t n_kv, int cus)
 }
 
 int64_t mfma_n_pad(int64_t n) { return align_up(n, 256); }
+
+// Do the dense operator's staging blocks look for their keys in the mask, instead of in an order that a launch in front of them has
+// written?  That launch takes 5.5 us, in which one workgroup works; a block's look takes half a microsecond for every 4096 mask bytes.
+// The operator, forward, us, 128 dims, heads x rows x cached keys, with the launch and without: 2 x 33 x 64 27.0 23.2   8 x 200 x 2 K 43.8
+// 41.3   3 x 300 x 8 K 53.4 49.0   2 x 1000 x 16 K 71.1 63.4   64 x 1000 x 16 K 503.5 497.6   2 x 100 x 20 K 50.8 45.5   8 x 300 x 30 K
+// 99.6 103.5   8 x 300 x 60 K 166.4 178.5   32 x 100 x 60 K 411.3 398.4: by 16 K it is never the slower way.
+bool order_by_staging(int64_t n_cached) { return n_cached <= 16384; }
 
 // Shares of a query tile's key tiles (1: no splitting) on a chip of `cus` compute units, each of which holds one workgroup
 // of the forward kernel at a time.  The count is a matter of sizes alone, never of how many slots hold a token: it sets the
