@@ -50,7 +50,8 @@ AttnWorkspace carve_attn(void* base, int64_t B, int64_t H, int64_t KVH, int64_t 
     int splits = mfma_supported(dtype, D, H, KVH, Q) && Q > 1 ? mfma_fwd_splits_for_workspace(B, H, KVH, Q, N, false) : 1;
     if (split) splits = f32_split_shares(B, H, KVH, Q, N, mfma_device_cus());
     w.part_o = splits > 1 ? (float*)c.take(splits * B * H * Q * D * 4) : nullptr;
-    w.part_l2 = splits > 1 ? (float*)c.take(splits * B * H * Q * (split ? 8 : 4)) : nullptr;
+    // whole tiles of rows of a share are read by the score kernel
+    w.part_l2 = splits > 1 ? (float*)c.take((splits * B * H * Q + kColSlack) * (split ? 8 : 4)) : nullptr;
     w.bytes = c.off;
     return w;
 }
@@ -81,7 +82,7 @@ DenseWorkspace carve_dense(void* base, int64_t B, int64_t H, int64_t n_ctx, int6
     w.n_visible = (int*)c.take(4);
     const int splits = mfma_fwd_splits_for_workspace(B, H, H, n_ctx, n_kv, true);
     w.part_o = splits > 1 ? (float*)c.take(splits * rows * D * 4) : nullptr;
-    w.part_l2 = splits > 1 ? (float*)c.take(splits * rows * 4) : nullptr;
+    w.part_l2 = splits > 1 ? (float*)c.take((splits * rows + kColSlack) * 4) : nullptr;
     const int shares = dense_row_shares(B, H, n_ctx, n_kv, mfma_device_cus());
     w.part_scores = shares > 1 ? (float*)c.take(shares * B * H * n_kv * 4) : nullptr;
     w.bytes = c.off;

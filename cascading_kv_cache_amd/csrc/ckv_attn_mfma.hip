@@ -1203,57 +1203,100 @@ __global__ void __launch_bounds__(512) fwd_pipe_kernel(FwdParams p) {
     }
 }
 
-// Merge of the forward kernel's shares: one row per kD / 4 lanes (4 dims each).
+// Merge of the forward kernel's shares by a workgroup of 256 threads: a row per kD / 4 lanes (4 dims each), and with few shares several
+// rows a thread, so that eight loads are always on their way at once.  A batch is kShares shares of 8 / kShares rows.
+template <int kD>
+constexpr int kMergeRows = 256 / (kD / 4);
+inline __host__ __device__ int merge_batch(int n_split) { return n_split <= 2 ? 2 : n_split <= 4 ? 4 : 8; }
+template <int kD>
+inline int64_t merge_blocks(int64_t rows, int n_split) {
+    const int64_t per = kMergeRows<kD> * (8 / merge_batch(n_split));
+    return (rows + per - 1) / per;
+}
+template <typename T, int kD, int kShares>
+__device__ inline void merge_rows_of(const FwdParams& p, int64_t block) {
+    const int64_t rows = p.B * p.H * p.Q;
+    constexpr int kLanes = kD / 4, kRowsEach = 8 / kShares;
+    const int64_t row0 = block * (kMergeRows<kD> * kRowsEach) + threadIdx.x / kLanes;
+    if (row0 >= rows) return;
+    const int d4 = threadIdx.x % kLanes;
+    int64_t row[kRowsEach];   // past the last row: the first one again
+#pragma unroll
+    for (int i = 0; i < kRowsEach; i++) row[i] = row0 + i * kMergeRows<kD> < rows ? row0 + i * kMergeRows<kD> : row0;
+    float M[kRowsEach];
+#pragma unroll
+    for (int i = 0; i < kRowsEach; i++) M[i] = -INFINITY;
+    for (int s0 = 0; s0 < p.n_split; s0 += kShares) {   // all normalisers first, they are the shorter trip
+        float l2[kRowsEach][kShares];
+#pragma unroll
+        for (int i = 0; i < kRowsEach; i++)
+#pragma unroll
+            for (int u = 0; u < kShares; u++) l2[i][u] = s0 + u < p.n_split ? p.part_l2[(s0 + u) * rows + row[i]] : -INFINITY;
+#pragma unroll
+        for (int i = 0; i < kRowsEach; i++)
+#pragma unroll
+            for (int u = 0; u < kShares; u++) M[i] = fmaxf(M[i], l2[i][u]);
+    }
+    float L[kRowsEach];
+    float4 o[kRowsEach];
+#pragma unroll
+    for (int i = 0; i < kRowsEach; i++) {
+        L[i] = 0.f;
+        o[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+    for (int s0 = 0; s0 < p.n_split; s0 += kShares) {
+        float l2[kRowsEach][kShares];
+        float4 v[kRowsEach][kShares];
+#pragma unroll
+        for (int i = 0; i < kRowsEach; i++)
+#pragma unroll
+            for (int u = 0; u < kShares; u++) {
+                const int s_ = s0 + u < p.n_split ? s0 + u : s0;
+                l2[i][u] = s0 + u < p.n_split ? p.part_l2[s_ * rows + row[i]] : -INFINITY;
+                v[i][u] = *reinterpret_cast<const float4*>(p.part_o + (s_ * rows + row[i]) * kD + 4 * d4);
+            }
+#pragma unroll
+        for (int i = 0; i < kRowsEach; i++)
+#pragma unroll
+            for (int u = 0; u < kShares; u++) {
+                if (l2[i][u] == -INFINITY) continue;
+                const float w = __builtin_amdgcn_exp2f(l2[i][u] - M[i]);
+                if (kExact<kD> && w == 0.f) continue;   // a share that has come down to nothing, whatever it holds
+                L[i] += w;
+                o[i].x = fmaf(v[i][u].x, w, o[i].x); o[i].y = fmaf(v[i][u].y, w, o[i].y);
+                o[i].z = fmaf(v[i][u].z, w, o[i].z); o[i].w = fmaf(v[i][u].w, w, o[i].w);
+            }
+    }
+#pragma unroll
+    for (int i = 0; i < kRowsEach; i++) {
+        if (i > 0 && row[i] == row0) break;
+        const float inv = 1.f / L[i];
+        int64_t m, h;
+        const int64_t b = div_index(div_index(row[i], p.Q, m), p.H, h);
+        T* dst = (T*)p.out + b * p.out_stride[0] + h * p.out_stride[1] + m * p.out_stride[2];
+        dst[(4 * d4) * p.out_stride[3]] = Elem<T>::from_float(o[i].x * inv);
+        dst[(4 * d4 + 1) * p.out_stride[3]] = Elem<T>::from_float(o[i].y * inv);
+        dst[(4 * d4 + 2) * p.out_stride[3]] = Elem<T>::from_float(o[i].z * inv);
+        dst[(4 * d4 + 3) * p.out_stride[3]] = Elem<T>::from_float(o[i].w * inv);
+        if (d4 == 0) {
+            const float l2 = M[i] + __builtin_amdgcn_logf(L[i]);  // v_log_f32 is log2
+            p.lse[row[i]] = l2 * 0.6931471805599453f;
+            p.lse2[row[i]] = -l2;
+        }
+    }
+}
+template <typename T, int kD>
+__device__ inline void merge_rows(const FwdParams& p, int64_t block) {
+    switch (merge_batch(p.n_split)) {
+        case 2: return merge_rows_of<T, kD, 2>(p, block);
+        case 4: return merge_rows_of<T, kD, 4>(p, block);
+        default: return merge_rows_of<T, kD, 8>(p, block);
+    }
+}
+
 template <typename T, int kD>
 __global__ void __launch_bounds__(256) fwd_combine_kernel(FwdParams p) {
-    const int64_t rows = p.B * p.H * p.Q;
-    constexpr int kLanes = kD / 4;
-    const int64_t row = (int64_t)blockIdx.x * (256 / kLanes) + threadIdx.x / kLanes;
-    if (row >= rows) return;
-    const int d4 = threadIdx.x % kLanes;
-    // with few rows a thread's loads are the whole kernel: all normalisers first, then the rows, eight on their way at once
-    constexpr int kBatch = 8;
-    float M = -INFINITY;
-    for (int s0 = 0; s0 < p.n_split; s0 += kBatch) {
-        float l2[kBatch];
-#pragma unroll
-        for (int u = 0; u < kBatch; u++) l2[u] = s0 + u < p.n_split ? p.part_l2[(s0 + u) * rows + row] : -INFINITY;
-#pragma unroll
-        for (int u = 0; u < kBatch; u++) M = fmaxf(M, l2[u]);
-    }
-    float L = 0.f;
-    float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int s0 = 0; s0 < p.n_split; s0 += kBatch) {
-        float l2[kBatch];
-        float4 v[kBatch];
-#pragma unroll
-        for (int u = 0; u < kBatch; u++) {
-            const int s_ = s0 + u < p.n_split ? s0 + u : s0;
-            l2[u] = s0 + u < p.n_split ? p.part_l2[s_ * rows + row] : -INFINITY;
-            v[u] = *reinterpret_cast<const float4*>(p.part_o + (s_ * rows + row) * kD + 4 * d4);
-        }
-#pragma unroll
-        for (int u = 0; u < kBatch; u++) {
-            if (l2[u] == -INFINITY) continue;
-            const float w = __builtin_amdgcn_exp2f(l2[u] - M);
-            if (kExact<kD> && w == 0.f) continue;   // a share that has come down to nothing, whatever it holds
-            L += w;
-            o.x = fmaf(v[u].x, w, o.x); o.y = fmaf(v[u].y, w, o.y); o.z = fmaf(v[u].z, w, o.z); o.w = fmaf(v[u].w, w, o.w);
-        }
-    }
-    const float inv = 1.f / L;
-    int64_t m, h;
-    const int64_t b = div_index(div_index(row, p.Q, m), p.H, h);
-    T* dst = (T*)p.out + b * p.out_stride[0] + h * p.out_stride[1] + m * p.out_stride[2];
-    dst[(4 * d4) * p.out_stride[3]] = Elem<T>::from_float(o.x * inv);
-    dst[(4 * d4 + 1) * p.out_stride[3]] = Elem<T>::from_float(o.y * inv);
-    dst[(4 * d4 + 2) * p.out_stride[3]] = Elem<T>::from_float(o.z * inv);
-    dst[(4 * d4 + 3) * p.out_stride[3]] = Elem<T>::from_float(o.w * inv);
-    if (d4 == 0) {
-        const float l2 = M + __builtin_amdgcn_logf(L);  // v_log_f32 is log2
-        p.lse[row] = l2 * 0.6931471805599453f;
-        p.lse2[row] = -l2;
-    }
+    merge_rows<T, kD>(p, blockIdx.x);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1281,7 +1324,12 @@ struct ColsumParams {
     float* part;          // leaves its sums in (row_shares, B*H, N), see colsum_merge_kernel
     int wnew_uniform;     // every entry of w_new has the value wnew_value (beta rounds to one in the tensor dtype)
     float wnew_value;
+    // kMerge: the forward kernel's shares (up to kMergeShares) are still to be merged.  The workgroups behind the first sum_blocks merge
+    // rows, and those work the normalisers of a query tile out from the shares' themselves.
+    int n_split, sum_blocks;
+    FwdParams fwd;
 };
+constexpr int kMergeShares = 8;
 
 constexpr int kQT2 = 128;                     // query rows per LDS tile of the column pass
 constexpr int kCsSub = kQT2 / 32;             // 32-row subtiles of a tile
@@ -1291,10 +1339,17 @@ __host__ __device__ constexpr int cs_stage(int head_dim) { return kQT2 * 2 * hea
 // S = Q K^T).  The (head, query-tile) sequence streams through a double-buffered LDS stage filled
 // by asynchronous copies; lane (col, half) owns key column `col` of each 32-key subtile, so the
 // weighted column sums never leave the lane.
-template <typename T, int kD, bool kShares>
+// kMerge: with the merge of the forward kernel's shares, as an instance of its own: as a branch that is not taken it cost the others 2 %.
+template <typename T, int kD, bool kShares, bool kMerge>
 __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
     extern __shared__ __align__(16) unsigned char smem[];
     constexpr int kKK = kD / 16, kRowBytes = 2 * kD, kCsStage = cs_stage(kD);
+    if constexpr (kMerge) {
+        if ((int)blockIdx.x >= p.sum_blocks) {
+            merge_rows<T, kD>(p.fwd, (int)blockIdx.x - p.sum_blocks);
+            return;
+        }
+    }
     const int Nc = p.n_visible ? *p.n_visible : (int)p.Nc;
     const int N = p.n_visible ? Nc + (int)p.Q : (int)p.N;   // keys somebody can see; those behind get a zero
     float* wnew_lds = reinterpret_cast<float*>(smem + 2 * kCsStage);
@@ -1379,6 +1434,9 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
 #pragma unroll
     for (int kk = 0; kk < kKK; kk++) q_off[kk] = k_lds_off<kD>(col, 2 * kk + half);
     const int64_t head_row0 = (b * p.H + kvh * p.G) * p.Q;
+    // shares' normalisers of a stage's rows, behind the stages and the table of weights
+    const int l2_at = 2 * kCsStage + (p.wnew_uniform ? 0 : (Q * 4 + 15) / 16 * 16);
+    const uint32_t l2_off = (uint32_t)((lane >> 3) < p.n_split ? lane >> 3 : 0) * (uint32_t)(p.B * p.H * p.Q * 4) + (lane & 7) * 16;
     // (head, query tile) of a step are tracked incrementally: integer division per step would
     // cost more scalar instructions than the step's matrix work leaves room for
     auto issue = [&](int g, int mt, int stage) {
@@ -1398,10 +1456,12 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
 #pragma unroll
             for (int j = 0; j < kQBlocks; j++) async_copy16(qt, q_src[j], st + (wave * kQBlocks + j) * 1024);
         }
-        if (wave < 2 && lane < kQT2 / 4) {
+        if (wave < 2 && lane < kQT2 / 4 && (!kMerge || wave)) {
             const char* src = wave ? (const char*)(p.w_ema + mt) : (const char*)(p.lse2 + row0);
             async_copy16(src, lane * 16, st + kQT2 * kRowBytes + wave * (kQT2 * 4));
         }
+        if constexpr (kMerge)   // a wavefront's 32 rows of every share, eight lanes a share
+            async_copy16((const char*)(p.fwd.part_l2 + row0 + wave * 32), l2_off, smem_addr + l2_at + stage * (4 * 1024) + wave * 1024);
     };
 
     auto store = [&](int64_t h, int64_t n, float v) {
@@ -1656,15 +1716,38 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
         }
     };
 
+    // Normalisers of the 32 rows that a wavefront has brought the shares' of: two lanes a row, four shares each.
+    auto merge_norms = [&](int stage) {
+        if constexpr (!kMerge) return;
+        const int r = lane >> 1;
+        const float* l2 = reinterpret_cast<const float*>(smem + l2_at + stage * (4 * 1024) + wave * 1024) + (lane & 1) * (32 * kMergeShares / 2) + r;
+        float v[kMergeShares / 2], M = -INFINITY, L = 0.f;
+#pragma unroll
+        for (int u = 0; u < kMergeShares / 2; u++) {
+            v[u] = (lane & 1) * (kMergeShares / 2) + u < p.n_split ? l2[32 * u] : -INFINITY;
+            M = fmaxf(M, v[u]);
+        }
+        M = fmaxf(M, __shfl_xor(M, 1));
+#pragma unroll
+        for (int u = 0; u < kMergeShares / 2; u++)
+            if (v[u] != -INFINITY) L += __builtin_amdgcn_exp2f(v[u] - M);   // a NaN counts
+        L += __shfl_xor(L, 1);
+        float* lse_lds = reinterpret_cast<float*>(smem + stage * kCsStage + kQT2 * kRowBytes);
+        if ((lane & 1) == 0) lse_lds[wave * 32 + r] = -(M + __builtin_amdgcn_logf(L));
+    };
     // Called by every wavefront once its copies of a step have landed, before the barrier that publishes them.  Rows past
     // the chunk end are copies of its last row, whose normaliser is somebody else's: starting from this value their
     // probability is zero (if the last row is not finite it has spoiled the sums already).  In LDS and not at the
     // accumulators: selects there cost 41 spilled registers, and the whole kernel a quarter of its speed.
     auto hide_rows = [&](int mt, int stage) {
-        if (mt + kQT2 <= Q || wave != 0) return;
+        if (mt + kQT2 <= Q) return;
         float* lse_lds = reinterpret_cast<float*>(smem + stage * kCsStage + kQT2 * kRowBytes);
-        for (int r = lane; r < kQT2; r += 64)
-            if (mt + r >= Q) lse_lds[r] = -3e38f;
+        if constexpr (kMerge) {   // a wavefront its own rows
+            if (lane < 32 && mt + wave * 32 + lane >= Q) lse_lds[wave * 32 + lane] = -3e38f;
+        } else if (wave == 0) {
+            for (int r = lane; r < kQT2; r += 64)
+                if (mt + r >= Q) lse_lds[r] = -3e38f;
+        }
     };
     // two steps per trip: while stage s is consumed the copy of the next step fills stage s^1
     int g_cur = g_first, mt_cur = m_first;    // step being consumed
@@ -1679,6 +1762,7 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
         int g_n = g_cur, mt_n = mt_cur;
         advance(g_n, mt_n);
         __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+        merge_norms(0);
         hide_rows(mt_cur, 0);
         __syncthreads();
         if (step + 1 < n_steps) issue(g_n, mt_n, 1);
@@ -1687,6 +1771,7 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
             int g_n2 = g_n, mt_n2 = mt_n;
             advance(g_n2, mt_n2);
             __builtin_amdgcn_s_waitcnt(0x0F70);
+            merge_norms(1);
             hide_rows(mt_n, 1);
             __syncthreads();
             if (step + 2 < n_steps) issue(g_n2, mt_n2, 0);
@@ -1799,9 +1884,12 @@ int run_mfma(const MfmaProblem& mp, hipStream_t stream) {
         CKV_HIP_TRY(hipGetLastError());
     }
     const int G = (int)(mp.H / mp.KVH);
+    FwdParams fp;
+    const bool scores = mp.colsum || mp.scores;
+    bool merged_by_scores = false;
+    int64_t merging = 0;   // workgroups that merge the forward kernel's shares
     {
         StageScope sc(CKV_STAGE_FWD, stream, true);
-        FwdParams fp;
         fp.qr = mp.qr; fp.kr = mp.kr; fp.vt = mp.vt; fp.tile_vis = mp.tile_vis;
         fp.out = mp.out;
         for (int j = 0; j < 4; j++) fp.out_stride[j] = mp.out_stride[j];
@@ -1826,14 +1914,22 @@ int run_mfma(const MfmaProblem& mp, hipStream_t stream) {
         if (ev0) hipExtLaunchKernelGGL((fwd_pipe_kernel<T, kD>), launch_grid, dim3(512), (uint32_t)lds, stream, ev0, ev1, 0u, fp);
         else hipLaunchKernelGGL((fwd_pipe_kernel<T, kD>), launch_grid, dim3(512), lds, stream, fp);
         CKV_HIP_TRY(hipGetLastError());
-        if (fp.n_split > 1) {
-            const int64_t rows = mp.B * mp.H * mp.Q;
-            constexpr int per = 256 / (kD / 4);
-            hipLaunchKernelGGL((fwd_combine_kernel<T, kD>), dim3((unsigned)((rows + per - 1) / per)), dim3(256), 0, stream, fp);
+        merging = merge_blocks<kD>(mp.B * mp.H * mp.Q, fp.n_split);
+        // The merge may ride in the launch of the score sums: a launch less, and its traffic beside the sums, whose last round leaves
+        // units idle.  But every workgroup of the sums then works the normalisers of its query tiles out for itself, a third of a
+        // microsecond a tile.  Calls, us, apart and together, 32 heads on 8 kv heads (streams x rows x slots): 100 x 1 K 57.6 53.4   300 x
+        // 4 K 94.0 87.2   1000 x 4 K 176.0 166.9   509 x 16 K 278.9 277.4   2 x 500 x 12 K 352.7 350.0   2300 x 8 K 575.9 564.9; where the
+        // estimate says apart: 1000 x 32 K 786.1 786.1   512 x 64 K 836.4 846.6   4 x 44 x 61 K 1003 1040   2 x 1500 x 64 K 4282 4412.
+        // Dense, forward, 64 dims: 8 x 1000 x 500 46.6 42.0   32 x 50 x 1000 34.3 29.9.
+        const int64_t rows = mp.B * mp.H * mp.Q, tiles = (n + 255) / 256 * mp.B * mp.H * ((mp.Q + kQT2 - 1) / kQT2);
+        const double apart_us = 4.0 + (double)(rows * fp.n_split * kD * 4) / 5.5e6, together_us = 0.33 * (double)tiles / (2 * cus);
+        merged_by_scores = scores && fp.n_split <= kMergeShares && together_us < apart_us && rows < (int64_t)1 << 27;   // offsets of 32 bits
+        if (fp.n_split > 1 && !merged_by_scores) {
+            hipLaunchKernelGGL((fwd_combine_kernel<T, kD>), dim3((unsigned)merging), dim3(256), 0, stream, fp);
             CKV_HIP_TRY(hipGetLastError());
         }
     }
-    if (mp.colsum || mp.scores) {
+    if (scores) {
         StageScope sc(CKV_STAGE_SCORES, stream);
         ColsumParams cp;
         cp.qr = mp.qr; cp.kr = mp.kr; cp.tile_vis = mp.tile_vis; cp.lse2 = mp.lse2;
@@ -1876,9 +1972,14 @@ int run_mfma(const MfmaProblem& mp, hipStream_t stream) {
         cp.gsplit = (G % 2 == 0 && G >= 4 && of_two >= 4 * 2 * (int64_t)cus) ? G / 2 : G;
         cp.row_shares = mp.scores && mp.part_scores ? dense_row_shares(mp.B, mp.H, mp.Q, n, cus) : 1;
         cp.part = mp.part_scores;
-        const dim3 grid((unsigned)(cp.nkb * cp.nbkv * cp.gsplit * cp.row_shares));
-        const int lds = 2 * cs_stage(kD) + (cp.wnew_uniform ? 0 : (int)mp.Q * 4);
-        auto kernel = cp.row_shares > 1 ? colsum_mfma_kernel<T, kD, true> : colsum_mfma_kernel<T, kD, false>;
+        cp.n_split = fp.n_split;
+        cp.fwd = fp;
+        cp.sum_blocks = cp.nkb * cp.nbkv * cp.gsplit * cp.row_shares;
+        const bool merge = fp.n_split > 1 && merged_by_scores;
+        const dim3 grid((unsigned)(cp.sum_blocks + (merge ? merging : 0)));
+        const int lds = 2 * cs_stage(kD) + (cp.wnew_uniform ? 0 : ((int)mp.Q * 4 + 15) / 16 * 16) + (merge ? 2 * 4 * 1024 : 0);
+        auto kernel = cp.row_shares > 1 ? (merge ? colsum_mfma_kernel<T, kD, true, true> : colsum_mfma_kernel<T, kD, true, false>)
+                                        : (merge ? colsum_mfma_kernel<T, kD, false, true> : colsum_mfma_kernel<T, kD, false, false>);
         if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(kernel), lds)) return rc;
         hipLaunchKernelGGL(kernel, grid, dim3(256), lds, stream, cp);
         if (cp.row_shares > 1) {

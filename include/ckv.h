@@ -335,7 +335,9 @@ int ckv_linear_rows(const void* x, const void* w, const void* bias, const void* 
  * events on the caller's stream; ckv_profile_read waits for them, ADDS the elapsed milliseconds
  * and launch counts per stage into the caller's arrays (length CKV_STAGE_COUNT) and forgets
  * them.  The plan of a call of several tokens is counted as two (closed forms, walk) also where
- * both are one launch: its time is with the first, the second has none.  Levels 1 and 3 run a
+ * both are one launch: its time is with the first, the second has none.  Where the forward kernel
+ * shares keys out, their merge is with CKV_STAGE_FWD, or with CKV_STAGE_SCORES when it rides in that
+ * launch.  Levels 1 and 3 run a
  * single token's cache update in launches of its own, which ckv_attn_update does otherwise only
  * where it cannot run beside the scores: they show what the stages take one by one, not what
  * such a step takes.  Process-wide and not thread-safe: a measurement aid, off by default.
