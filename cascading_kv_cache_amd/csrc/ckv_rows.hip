@@ -6,11 +6,12 @@
 // of 2 KiB stages in LDS (64 elements of 16 rows: two copies of 1 KiB, whole 128-byte lines, past the caches), several stages ahead
 // and without a barrier.  A group is shared by kParts wavefronts where N alone has too few groups to keep enough of them in flight.
 // One bf16 row, us, torch's operations (product, norm, gate, residual) and this, weights out of memory:
-//   6144 x 4096 norm 20 + 6 -> 12        4096 x 4096 residual 20 + 3 -> 9.5    28672 x 4096 norm, gate 60 + 6 + 4 -> 42.5 (5.5 TB/s)
-//   4096 x 14336 residual 26 + 3 -> 22   128256 x 4096 norm 185 + 6 -> 160 (6.6 TB/s)   3584 x 18944 residual 48 + 3 -> 23.5
-// Ring stages of a lone wavefront's group: 4, 6 and 7 are level (40.4, 40.9 and 40.5 at 28672 x 4096), 4 leaves room for three
-// workgroups; of four parts': 6 and 7 (12 with the norm at 6144 x 4096) leave room for two, 8 do not (14.3).  Copies through the L2
-// 41 -> 45 us and 160 -> 190; workgroups of two wavefronts for lone groups 46.
+//   6144 x 4096 norm 20 + 6 -> 11        4096 x 4096 residual 20 + 3 -> 8.2    28672 x 4096 norm, gate 60 + 6 + 4 -> 41 (5.7 TB/s)
+//   4096 x 14336 residual 26 + 3 -> 22   128256 x 4096 norm 185 + 6 -> 151 (7.0 TB/s)   3584 x 18944 residual 48 + 3 -> 23.5
+// Stretches of W by XCD (rows_kernel): the five products above in turn over four layers and a head of 2.8 GB, 491 -> 477 us.
+// Ring stages of four parts: 6 and 7 are level (12 with the norm at 6144 x 4096) and leave room for two workgroups, 8 do not (14.3);
+// stages of 128 elements are level with two of 64.  Copies through the L2 160 -> 190 us at 128256 x 4096.  How many wavefronts and
+// stages a workgroup gets: run_rows below.
 //
 // The order of a sum is the caller's (kParts, kUnit): part p takes the stretches of kUnit * 64 elements p, p + kParts, ..., one chain
 // of matrix instructions each, and the parts are added up in order.  Another order is as good, but flips the rounding of a few
@@ -51,23 +52,21 @@ __device__ inline f32x4 rows_mma(uint4 a, uint4 b, f32x4 c) {
 
 __host__ __device__ inline int rows_pitch(int K) { return 2 * K + 16; }   // bytes between the rows of x in LDS; the pad spreads the banks
 
-// stages of the ring of a wavefront
+// wavefronts of a workgroup, at most: with one part any number, else one per part
 template <int kParts>
-constexpr int kRing = kParts == 1 ? 4 : kParts == 2 ? 12 : 6;
-template <int kParts>
-constexpr int kRowsWaves = kParts == 2 ? 2 : 4;
+constexpr int kMostWaves = kParts == 1 ? 8 : kParts;
 
 // RMSNorm of the rows in LDS, in place.  The sum of squares is that of 256 threads of four elements at a time, whatever the workgroup:
 // the order (and the bits) of torch's kernel.
-template <typename T, int kWaves>
-__device__ inline void rows_norm(unsigned char* xs, const unsigned char* weights, float (*part)[4], const RowsParams& p) {
+template <typename T>
+__device__ inline void rows_norm(unsigned char* xs, const unsigned char* weights, float (*part)[4], int waves, const RowsParams& p) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int pieces = p.K / 4, pitch = rows_pitch(p.K);
     struct alignas(8) Piece {
         T v[4];
     };
     for (int j = 0; j < p.rows; j++)
-        for (int vw = wave; vw < 4; vw += kWaves) {
+        for (int vw = wave; vw < 4; vw += waves) {
             float s = 0.f;
             for (int i = vw * 64 + lane; i < pieces; i += 256) {
                 const Piece a = *reinterpret_cast<const Piece*>(xs + j * pitch + 8 * i);
@@ -85,7 +84,7 @@ __device__ inline void rows_norm(unsigned char* xs, const unsigned char* weights
     for (int j = 0; j < p.rows; j++) {
         const float sum = (part[j][0] + part[j][2]) + (part[j][1] + part[j][3]);
         const float r = rsqrtf(sum / (float)p.K + p.eps);
-        for (int i = threadIdx.x; i < pieces; i += 64 * kWaves) {
+        for (int i = threadIdx.x; i < pieces; i += 64 * waves) {
             Piece* at = reinterpret_cast<Piece*>(xs + j * pitch + 8 * i);
             const Piece a = *at, w = *reinterpret_cast<const Piece*>(weights + 8 * i);
             Piece o;
@@ -97,28 +96,31 @@ __device__ inline void rows_norm(unsigned char* xs, const unsigned char* weights
     __syncthreads();
 }
 
-template <typename T, int kParts, int kUnit, bool kGated>
-__global__ void __launch_bounds__(64 * kRowsWaves<kParts>) rows_kernel(RowsParams p) {
+template <typename T, int kParts, int kUnit, bool kGated, int kStages>
+__global__ void __launch_bounds__(64 * kMostWaves<kParts>) rows_kernel(RowsParams p) {
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ float norm_part[kMaxRows][4];
-    constexpr int kWaves = kRowsWaves<kParts>, kStages = kRing<kParts>;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int waves = kParts > 1 ? kParts : blockDim.x >> 6;
     const int part = wave % kParts;
     const int groups = p.N / 16;
-    int group = blockIdx.x * (kWaves / kParts) + wave / kParts;
+    // Workgroups go round the eight XCDs: each gets a stretch of W of its own, and meets an eighth of its pages.
+    const int xcd = blockIdx.x % 8, many = gridDim.x / 8, over = gridDim.x % 8;
+    const int block = xcd * many + min(xcd, over) + blockIdx.x / 8;
+    int group = kParts > 1 ? block : block * waves + wave;
     const bool live = group < groups;
     if (!live) group = groups - 1;   // reads what another wavefront does and writes nothing
     const int64_t row_bytes = 2 * (int64_t)p.K;
     unsigned char* ring = smem + wave * (kStages * kStageBytes);
-    unsigned char* xs = smem + kWaves * (kStages * kStageBytes);
+    unsigned char* xs = smem + waves * (kStages * kStageBytes);
     const int pitch = rows_pitch(p.K);
     const uint32_t ring_addr = lds_address(ring), xs_addr = lds_address(xs);
 
     // rows of x, and the norm's weights behind them, go first: 1 KiB a copy, dealt out over the wavefronts
     {
         const int blocks = (p.K + 511) / 512, all = (p.rows + (p.norm ? 1 : 0)) * blocks;
-        for (int i = wave; i < all; i += kWaves) {
+        for (int i = wave; i < all; i += waves) {
             const int j = i / blocks, blk = i - j * blocks;
             const char* src = j < p.rows ? (const char*)p.x + 2 * j * p.x_stride : (const char*)p.norm;
             const int at = blk * 1024 + lane * 16;
@@ -153,7 +155,7 @@ __global__ void __launch_bounds__(64 * kRowsWaves<kParts>) rows_kernel(RowsParam
     for (int i = 0; i < kStages; i++) issue(i < n ? chunk_of(i) : 0, i);
     wait_copies<2 * kStages>();
     __syncthreads();
-    if (p.norm) rows_norm<T, kWaves>(xs, xs + p.rows * pitch, norm_part, p);
+    if (p.norm) rows_norm<T>(xs, xs + p.rows * pitch, norm_part, waves, p);
 
     const int r = lane & 15, q = lane >> 4;
     const int flip = (r & 7) ^ (r >> 3);
@@ -224,19 +226,44 @@ __global__ void __launch_bounds__(64 * kRowsWaves<kParts>) rows_kernel(RowsParam
     }
 }
 
-template <typename T, int kParts, int kUnit, bool kGated>
-int run_rows(const RowsParams& p, hipStream_t stream) {
-    constexpr int kWaves = kRowsWaves<kParts>;
-    const int lds = kWaves * kRing<kParts> * kStageBytes + p.rows * rows_pitch(p.K) + (p.norm ? 2 * p.K : 0);
-    DeviceInfo di;
-    if (int rc = current_device_info(&di)) return rc;
-    if (lds + 256 > di.lds_max) return CKV_ERR_UNSUPPORTED;
-    auto kernel = rows_kernel<T, kParts, kUnit, kGated>;
+template <typename T, int kParts, int kUnit, bool kGated, int kStages>
+int launch_rows(const RowsParams& p, int waves, int lds, hipStream_t stream) {
+    auto kernel = rows_kernel<T, kParts, kUnit, kGated, kStages>;
     if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(kernel), lds)) return rc;
-    const int groups = p.N / 16, per = kWaves / kParts;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)((groups + per - 1) / per)), dim3(64 * kWaves), lds, stream, p);
+    const int groups = p.N / 16, per = waves / kParts;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)((groups + per - 1) / per)), dim3(64 * waves), lds, stream, p);
     CKV_HIP_TRY(hipGetLastError());
     return CKV_OK;
+}
+
+// A launch lasts as long as the compute unit with the most groups, and a workgroup brings the rows and normalises them for itself: with
+// one part a compute unit's even share of the groups is one workgroup of up to eight wavefronts, or a few of the same size (28672 x 4096:
+// 448 workgroups of four lay two on most compute units and one on the others; 256 of seven 43.6 -> 39.4 us, in turn with the other products
+// of a step 43.1 -> 42.0.  37888 x 3584: 44.8 -> 42.0).  Where one workgroup has a compute unit to itself its rings have twice the
+// stages (39.4 -> 38.5, in turn with the others 45 -> 42.0; 10 stages are level).  Two parts: the longer ring where two
+// workgroups still fit (6144 x 4096, norm, a row: 11.6 with 12 stages, 11.9 with 8; four rows, one workgroup on a unit or two: 29.8, 18.0).
+// Four parts: the shorter ring where the longer does not fit.
+template <typename T, int kParts, int kUnit, bool kGated>
+int run_rows(const RowsParams& p, hipStream_t stream) {
+    DeviceInfo di;
+    if (int rc = current_device_info(&di)) return rc;
+    constexpr int kLong = kParts == 1 ? 8 : kParts == 2 ? 12 : 6, kShort = kParts == 2 ? 8 : 4;
+    const int rest = p.rows * rows_pitch(p.K) + (p.norm ? 2 * p.K : 0);
+    auto lds = [&](int waves, int stages) { return waves * stages * kStageBytes + rest; };
+    auto fits = [&](int bytes) { return bytes + 256 <= di.lds_max; };
+    int waves = kParts;
+    bool longer = fits(lds(waves, kLong) * (kParts == 2 ? 2 : 1));
+    if constexpr (kParts == 1) {
+        constexpr int kMany = 4;   // rounds of workgroups: the last one no longer counts, and four wavefronts are the better workgroup
+        const int share = (p.N / 16 + di.cus - 1) / di.cus, most = share > kMany * kMostWaves<1> ? 4 : kMostWaves<1>;
+        const int shares = (share + most - 1) / most;
+        waves = (share + shares - 1) / shares;
+        longer = shares == 1 && fits(lds(waves, kLong));
+        while (waves > 1 && !fits(lds(waves, kShort))) waves--;   // long rows
+    }
+    if (!longer && !fits(lds(waves, kShort))) return CKV_ERR_UNSUPPORTED;
+    return longer ? launch_rows<T, kParts, kUnit, kGated, kLong>(p, waves, lds(waves, kLong), stream)
+                  : launch_rows<T, kParts, kUnit, kGated, kShort>(p, waves, lds(waves, kShort), stream);
 }
 
 template <typename T>

@@ -58,7 +58,7 @@ def gated_silu(gate_up):
 
 def _fits(rows, n, k, order, norm) -> bool:
     """Sizes that ``ckv_linear_rows`` takes: the rows, the norm's weights and a ring of stages share the LDS of a compute unit."""
-    ring = {1: 4 * 4, 2: 2 * 12, 4: 4 * 6}[order[0]] * 2048
+    ring = {1: 4 * 4, 2: 2 * 8, 4: 4 * 4}[order[0]] * 2048
     return 0 < rows <= MAX_ROWS and n % 16 == 0 and k % 64 == 0 and ring + rows * (2 * k + 16) + 2 * k * norm + 256 <= 160 * 1024
 
 

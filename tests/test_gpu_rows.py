@@ -27,7 +27,9 @@ def bound(x, w, dtype):
 # one group and part of a workgroup's, fewer stretches than parts or stages, remainders of both; the largest rows that fit
 @pytest.mark.parametrize("order", rp.ORDERS)
 @pytest.mark.parametrize("rows,n,k", [(1, 16, 64), (2, 48, 128), (16, 80, 192), (3, 16, 576), (1, 4096, 832), (5, 96, 1600), (1, 64, 3584),
-                                      (2, 32, 18944)])
+                                      (2, 32, 18944),
+                                      # several groups a compute unit: one workgroup's, two workgroups', many rounds; rings that just fit
+                                      (2, 16 * 1793, 64), (1, 16 * 2305, 128), (1, 16 * 8449, 64), (16, 16 * 2048, 3584), (4, 32, 14336)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_rows_against_float64(order, rows, n, k, dtype):
     x, w, bias, res, norm = operands(rows, n, k, dtype)
