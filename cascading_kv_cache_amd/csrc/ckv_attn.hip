@@ -24,6 +24,7 @@ struct AttnWorkspace {
     uint32_t* odd_q;
     uint8_t* kmasked;
     float *lse, *lse2, *colsum, *w_ema, *w_new, *part_o, *part_l2;
+    void* before;                   // see KeptScores
     int64_t bytes;
 };
 
@@ -52,6 +53,7 @@ AttnWorkspace carve_attn(void* base, int64_t B, int64_t H, int64_t KVH, int64_t 
     w.part_o = splits > 1 ? (float*)c.take(splits * B * H * Q * D * 4) : nullptr;
     // whole tiles of rows of a share are read by the score kernel
     w.part_l2 = splits > 1 ? (float*)c.take((splits * B * H * Q + kColSlack) * (split ? 8 : 4)) : nullptr;
+    w.before = Q > 1 ? c.take(B * KVH * S * es) : nullptr;
     w.bytes = c.off;
     return w;
 }
@@ -135,6 +137,19 @@ static int run_attn(const ckv_attn_args* args, hipStream_t stream, const ckv_upd
     const bool want_scores = a.cache_s || a.new_scores;
     int rc;
     const bool use_mfma = mfma_supported(a.dtype, a.D, a.H, a.KVH, a.Q) && a.Q > 1 && mfma_fits(N, a.D);
+    const bool split = !use_mfma && f32_split_supported(a.dtype, a.B, a.H, a.KVH, a.Q, N, a.D);
+    KeptScores kept;
+    if (u && (use_mfma || split) && a.S > 0 && a.cache_s && a.new_scores && update_plans_beside_finish(a, *u)) {
+        // the plan's scratch may be the attention's, of which only what the score sums left is still read
+        const char *ws = reinterpret_cast<const char*>(u->workspace), *sums = reinterpret_cast<const char*>(w.colsum);
+        const int64_t need = ckv_update_workspace_bytes(u->N, u->H, u->K, u->max_seq_len, u->cascades);
+        if (ws + need <= sums || ws >= reinterpret_cast<const char*>(a.workspace) + w.bytes) {
+            kept.src = a.cache_s;
+            for (int i = 0; i < 3; i++) kept.stride[i] = a.cache_s_stride[i];
+            kept.dst = w.before;
+            kept.units = a.B * a.KVH; kept.KVH = a.KVH; kept.S = a.S;
+        }
+    }
     if (use_mfma) {
         MfmaProblem mp;
         mp.seg[0] = MfmaSegment{a.sink_k, a.sink_v, {a.sink_stride[0], a.sink_stride[1], a.sink_stride[2], a.sink_stride[3]},
@@ -165,6 +180,7 @@ static int run_attn(const ckv_attn_args* args, hipStream_t stream, const ckv_upd
         mp.w_ema = w.w_ema; mp.w_new = w.w_new;
         mp.beta = a.beta;
         mp.make_weights = want_scores;
+        mp.kept = kept;
         mp.new_mode = 1;
         mp.B = a.B; mp.H = a.H; mp.KVH = a.KVH; mp.Q = a.Q; mp.D = a.D; mp.n = N; mp.n_pad = mfma_n_pad(N);
         mp.scale = a.scale;
@@ -173,7 +189,6 @@ static int run_attn(const ckv_attn_args* args, hipStream_t stream, const ckv_upd
         rc = launch_mfma(mp, stream);
         if (rc) return rc;
     } else {
-        const bool split = f32_split_supported(a.dtype, a.B, a.H, a.KVH, a.Q, N, a.D);
         if (!split) {
             PrepProblem pp{&a, w.qr, w.kr, w.vc, w.kmasked, want_scores ? w.w_ema : nullptr, w.w_new};
             rc = launch_prep_generic(pp, stream);
@@ -201,7 +216,7 @@ static int run_attn(const ckv_attn_args* args, hipStream_t stream, const ckv_upd
                               (uint32_t)(reinterpret_cast<char*>(w.w_new) - reinterpret_cast<char*>(w.w_ema))};
             if (!a.lse) cp.lse = nullptr;
             rc = launch_f32_split(a, cp, f, want_scores ? w.w_ema : nullptr, w.w_new, (float2*)w.lse2, w.part_o,
-                                  (float2*)w.part_l2, stream);
+                                  (float2*)w.part_l2, kept, stream);
         } else {
             rc = launch_core_generic(cp, stream);
         }
@@ -224,7 +239,13 @@ static int run_attn(const ckv_attn_args* args, hipStream_t stream, const ckv_upd
         fp.beta_pow_q = (float)pow(a.beta, (double)a.Q);
         fp.head_reduction = a.head_reduction;
         fp.homogeneous = a.homogeneous_heads;
+        fp.heads = (int)(a.homogeneous_heads ? a.H : a.H / a.KVH);
         fp.dtype = a.dtype;
+        if (kept.src) {
+            fp.before = kept.dst;
+            *updated = true;
+            return launch_finish_and_update(fp, *u, stream);
+        }
         rc = launch_finish(fp, stream);
         if (rc) return rc;
     }

@@ -218,6 +218,8 @@ struct F32Stage {
     uint32_t *vis, *odd_q;
     uint2* odd_kv;
     float *w_ema, *w_new;   // the weights of the score sums, or null
+    int w_items;            // wavefronts with weights; those behind them keep scores
+    KeptScores kept;
     float post_q, post_k;   // what rotated queries and keys are multiplied by
     int nblk, q_tiles;
     int k_items, q_items, v_items, vis_items;   // wavefronts
@@ -374,7 +376,8 @@ __global__ void __launch_bounds__(256) stage_f32_kernel(F32Stage p) {
         return;
     }
     id -= p.vis_items;
-    if (p.w_ema) weights_at<float>(p.w_ema, p.w_new, Q, a.beta, (int64_t)id * 64 + lane);
+    if (id < p.w_items) weights_at<float>(p.w_ema, p.w_new, Q, a.beta, (int64_t)id * 64 + lane);
+    else if (p.kept.src) keep_scores<float, CKV_WAVE>(p.kept, id - p.w_items, lane);
 }
 
 struct F32Fwd {
@@ -926,7 +929,7 @@ __global__ void __launch_bounds__(Col<kGroups>::kWaves* CKV_WAVE, 2) colsum_f32_
 
 template <int D>
 int run(const ckv_attn_args& a, const CoreProblem& p, const F32Planes& f, float* w_ema, float* w_new, float2* norm, float* part_o,
-        float2* part_l, hipStream_t stream) {
+        float2* part_l, const KeptScores& kept, hipStream_t stream) {
     using G_ = Geo<D>;
     const int64_t G = p.H / p.KVH, tiles = (p.Q * G + kRows - 1) / kRows, units = p.B * p.KVH;
     {
@@ -956,7 +959,9 @@ int run(const ckv_attn_args& a, const CoreProblem& p, const F32Planes& f, float*
         };
         st.vec = pieces(a.q_stride, a.q, a.q) && pieces(a.kv_new_stride, a.k_new, a.v_new) &&
                  (a.S == 0 || pieces(a.cache_stride, a.cache_k, a.cache_v)) && (a.num_sink == 0 || pieces(a.sink_stride, a.sink_k, a.sink_v));
-        const int64_t waves = (int64_t)st.k_items + st.q_items + st.v_items + st.vis_items + (w_ema ? (p.Q + kColSlack + 63) / 64 : 0);
+        st.w_items = w_ema ? (int)((p.Q + kColSlack + 63) / 64) : 0;
+        st.kept = kept;
+        const int64_t waves = (int64_t)st.k_items + st.q_items + st.v_items + st.vis_items + st.w_items + kept_pieces(kept, CKV_WAVE);
         hipLaunchKernelGGL(stage_f32_kernel<D>, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, stream, st);
         CKV_HIP_TRY(hipGetLastError());
     }
@@ -1022,9 +1027,9 @@ bool f32_split_supported(int dtype, int64_t B, int64_t H, int64_t KVH, int64_t Q
 int64_t f32_split_plane_bytes(int64_t units, int64_t rows, int64_t D) { return units * ((rows + 31) / 32) * 32 * D * 2 * kPlanes; }
 
 int launch_f32_split(const ckv_attn_args& a, const CoreProblem& p, const F32Planes& f, float* w_ema, float* w_new, float2* norm,
-                     float* part_o, float2* part_l, hipStream_t stream) {
-    return p.D == 64 ? run<64>(a, p, f, w_ema, w_new, norm, part_o, part_l, stream)
-                     : run<128>(a, p, f, w_ema, w_new, norm, part_o, part_l, stream);
+                     float* part_o, float2* part_l, const KeptScores& kept, hipStream_t stream) {
+    return p.D == 64 ? run<64>(a, p, f, w_ema, w_new, norm, part_o, part_l, kept, stream)
+                     : run<128>(a, p, f, w_ema, w_new, norm, part_o, part_l, kept, stream);
 }
 
 }  // namespace ckv

@@ -2,16 +2,12 @@
 // (16-bit and float32) do not take.  Also the small shared stages: score-sum
 // weights, the rotate+gather prologue, and the head-reduction / EMA epilogue.
 #include "ckv_attn_internal.h"
+#include "ckv_finish.h"
 
 #include <algorithm>
 
 namespace ckv {
 namespace {
-
-template <typename T>
-__device__ inline float round_t(float v) {
-    return Elem<T>::to_float(Elem<T>::from_float(v));
-}
 
 template <typename T>
 __global__ void weights_kernel(float* w_ema, float* w_new, int64_t Q, double beta) {
@@ -508,72 +504,18 @@ __global__ void __launch_bounds__(CKV_WAVE) colsum_generic_kernel(CoreProblem p)
 }
 
 // ---------------------------------------------------------------------------------------------
-// epilogue: per-head sums -> dtype -> head reduction -> EMA / new-token scores
-// (cascade_attention.py:231-248, 319-330)
+// epilogue of the scores (ckv_finish.h)
 // ---------------------------------------------------------------------------------------------
-// Eight heads' sums are on their way at a time; they are taken in the order of the heads.  kMedian: the kernel that keeps all
-// of them (in scratch memory, which the launches of the others would pay for).
-constexpr int kHeadsAhead = 8;
-template <typename T, bool kMedian>
-__device__ inline float reduce_heads(const float* colsum, int64_t b, int64_t h0, int nh, int64_t H, int64_t N,
-                                     int64_t n, int mode) {
-    const float* base = colsum + (b * H + h0) * N + n;
-    float r = 0.f;
-    [[maybe_unused]] float vals[kMedian ? 128 : 1];  // lower median (torch.median): element (nh-1)/2 of the sorted values
-    for (int g0 = 0; g0 < nh; g0 += kHeadsAhead) {
-        float x[kHeadsAhead];
-#pragma unroll
-        for (int u = 0; u < kHeadsAhead; u++) x[u] = g0 + u < nh ? base[(g0 + u) * N] : 0.f;
-#pragma unroll
-        for (int u = 0; u < kHeadsAhead; u++) {
-            const int g = g0 + u;
-            if (g >= nh) break;
-            const float v = round_t<T>(x[u]);
-            if constexpr (kMedian) {
-                int i = g;
-                while (i > 0 && vals[i - 1] > v) {
-                    vals[i] = vals[i - 1];
-                    i--;
-                }
-                vals[i] = v;
-            } else if (mode == CKV_REDUCE_MAX) {
-                r = g == 0 ? v : fmaxf(r, v);
-            } else {
-                r = __fadd_rn(r, v);
-            }
-        }
-    }
-    if constexpr (kMedian) return vals[(nh - 1) / 2];
-    return mode == CKV_REDUCE_MAX ? r : round_t<T>(r / (float)nh);
-}
-
 // Grid: slots and new tokens along x, kv heads along y, batch along z.
 // Bound by its trip to memory: with 64-bit divisions of a flat index and the heads' sums read one after the other it took
 // 5.8 us for 8 x 16893 items of 4 heads, now 5.1.
-template <typename T, bool kMedian>
+template <typename T, int kHow>
 __global__ void __launch_bounds__(256) finish_kernel(FinishProblem p) {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= p.S + p.Q) return;
     if (i < p.S ? !p.cache_s : !p.new_scores) return;
-    const int G = (int)p.H / (int)p.KVH, nh = p.homogeneous ? (int)p.H : G;
-    for (int64_t b = blockIdx.z; b < p.B; b += gridDim.z) {
-        for (int64_t kvh = blockIdx.y; kvh < p.KVH; kvh += gridDim.y) {
-            const int64_t h0 = p.homogeneous ? 0 : kvh * G;
-            if (i < p.S) {
-                T* cs = (T*)p.cache_s + b * p.cache_s_stride[0] + kvh * p.cache_s_stride[1] + i * p.cache_s_stride[2];
-                const T old = *cs;
-                const float red = reduce_heads<T, kMedian>(p.colsum, b, h0, nh, p.H, p.N, p.num_sink + i, p.head_reduction);
-                const float decayed = round_t<T>(__fmul_rn(p.beta_pow_q, Elem<T>::to_float(old)));
-                *cs = Elem<T>::from_float(__fadd_rn(decayed, red));
-            } else {
-                const int64_t m = i - p.S;
-                const float red = reduce_heads<T, kMedian>(p.colsum, b, h0, nh, p.H, p.N, p.num_sink + p.S + m, p.head_reduction);
-                T* ns = (T*)p.new_scores + b * p.new_scores_stride[0] + kvh * p.new_scores_stride[1] +
-                        m * p.new_scores_stride[2];
-                *ns = Elem<T>::from_float(red);
-            }
-        }
-    }
+    for (int64_t b = blockIdx.z; b < p.B; b += gridDim.z)
+        for (int64_t kvh = blockIdx.y; kvh < p.KVH; kvh += gridDim.y) finish_score<T, kHow>(p, b, kvh, i);
 }
 
 template <typename T>
@@ -729,11 +671,9 @@ int launch_finish(const FinishProblem& p, hipStream_t stream) {
     StageScope sc(CKV_STAGE_FINISH, stream);
     const dim3 grid((unsigned)((p.S + p.Q + 255) / 256), (unsigned)std::min<int64_t>(p.KVH, 65535), (unsigned)std::min<int64_t>(p.B, 65535));
     const dim3 block(256);
-    const bool median = p.head_reduction != CKV_REDUCE_MAX && p.head_reduction != CKV_REDUCE_MEAN;
     auto launch = [&](auto tag) {
         using T = decltype(tag);
-        if (median) hipLaunchKernelGGL((finish_kernel<T, true>), grid, block, 0, stream, p);
-        else hipLaunchKernelGGL((finish_kernel<T, false>), grid, block, 0, stream, p);
+        with_reduction(p, [&](auto how) { hipLaunchKernelGGL((finish_kernel<T, how.value>), grid, block, 0, stream, p); });
     };
     switch (p.dtype) {
         case CKV_F32: launch(float{}); break;

@@ -5,6 +5,8 @@
 
 namespace ckv {
 
+struct KeptScores;
+
 // max over the two lane halves (lane l and lane l ^ 32) without a trip through LDS
 __device__ inline float half_max(float x) {
     const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
@@ -62,7 +64,7 @@ int64_t f32_split_plane_bytes(int64_t units, int64_t rows, int64_t D);
 // `p`: sizes, out, lse (null: not wanted), colsum and the weights; its operands are not read.  norm: scratch, B*H*Q pairs.  part_o / part_l: f32_split_shares shares of
 // (B*H*Q, D) floats / (B*H*Q) pairs, or null (then the keys of a row tile are not shared out).
 int launch_f32_split(const ckv_attn_args& a, const CoreProblem& p, const F32Planes& f, float* w_ema, float* w_new, float2* norm,
-                     float* part_o, float2* part_l, hipStream_t stream);
+                     float* part_o, float2* part_l, const KeptScores& kept, hipStream_t stream);
 
 // weights of the score sums (cascade_attention.py:270-282, 315-317), rounded like the eager path
 // w_ema gets 64 trailing zeros (slack read by the MFMA column pass)
@@ -97,8 +99,45 @@ struct FinishProblem {
     int64_t B, H, KVH, Q, S, num_sink;
     float beta_pow_q;      // beta^Q rounded to fp32
     int head_reduction, homogeneous, dtype;
+    int heads;             // that are reduced together: H, or H / KVH
+    const void* before = nullptr;  // see KeptScores; null: the update does not share the launch
 };
 int launch_finish(const FinishProblem& p, hipStream_t stream);
+
+// A short chunk's update is planned in the launch that finishes its scores: the plan works the few scores it asks for out by itself,
+// and reads those of the cache as they were before the call, of which the staging launch keeps a copy (the finishing blocks write theirs
+// in place meanwhile).
+struct KeptScores {
+    const void* src = nullptr;   // (units, S); null: nobody asks
+    int64_t stride[3];           // by batch, kv head, slot
+    void* dst;                   // contiguous
+    int64_t units, KVH, S;
+};
+constexpr int kKeptPer = 8;      // slots a thread copies
+inline int64_t kept_pieces(const KeptScores& k, int threads) {
+    return k.src ? k.units * ((k.S + kKeptPer * threads - 1) / (kKeptPer * threads)) : 0;
+}
+template <typename T, int kThreads>
+__device__ inline void keep_scores(const KeptScores& k, int64_t piece, int tid) {
+    const int64_t per = (k.S + kKeptPer * kThreads - 1) / (kKeptPer * kThreads), unit = piece / per;
+    if (unit >= k.units) return;
+    const int64_t b = unit / k.KVH, kvh = unit - b * k.KVH, first = (piece - unit * per) * (kKeptPer * kThreads) + tid;
+    const T* src = (const T*)k.src + b * k.stride[0] + kvh * k.stride[1];
+    T v[kKeptPer];
+#pragma unroll
+    for (int j = 0; j < kKeptPer; j++) {
+        const int64_t i = first + j * kThreads;
+        v[j] = src[(i < k.S ? i : k.S - 1) * k.stride[2]];
+    }
+#pragma unroll
+    for (int j = 0; j < kKeptPer; j++) {
+        const int64_t i = first + j * kThreads;
+        if (i < k.S) ((T*)k.dst)[unit * k.S + i] = v[j];
+    }
+}
+// may the update of a call's tokens be planned in the launch that finishes their scores?  (Both are checked; workspaces apart.)
+bool update_plans_beside_finish(const ckv_attn_args& a, const ckv_update_args& u);
+int launch_finish_and_update(const FinishProblem& p, const ckv_update_args& u, hipStream_t stream);
 
 // rows of slack behind the staged queries, their normalisers and weights: the column pass reads whole
 // tiles of this many query rows
@@ -212,6 +251,7 @@ struct MfmaProblem {
     float* w_new;
     double beta;           // the EMA factor of the weights
     int make_weights = 0;  // the staging launch writes w_ema and w_new too
+    KeptScores kept;       // and keeps these
     int new_mode;
     int64_t B, H, KVH, Q, D, n, n_pad;
     int64_t empty_from = 0, empty_to = 0;  // keys whose slots cannot hold a token yet

@@ -540,6 +540,8 @@ struct StageWeights {
     double beta;
     int* key_order;   // written by the first block where the staging blocks find their keys themselves
     int* n_visible;
+    int blocks;       // with weights; those behind them keep scores
+    KeptScores kept;
 };
 template <typename T, int kD>
 __global__ void __launch_bounds__(256) stage_kernel(StageParams sp, StageQParams sq, StageGrid g, StageWeights sw) {
@@ -552,8 +554,10 @@ __global__ void __launch_bounds__(256) stage_kernel(StageParams sp, StageQParams
         stage_keys_block<T, kD>(sp, id % g.k_bx, id / g.k_bx, g.k_by, lds);
     } else {
         id -= nk;
-        if (id < g.q_bx * g.q_by) stage_q_block<T, kD>(sq, id % g.q_bx, id / g.q_bx, g.q_by, lds);
-        else weights_at<T>(sw.w_ema, sw.w_new, sq.Q, sw.beta, (int64_t)(id - g.q_bx * g.q_by) * 256 + threadIdx.x);
+        const int nq = g.q_bx * g.q_by;
+        if (id < nq) stage_q_block<T, kD>(sq, id % g.q_bx, id / g.q_bx, g.q_by, lds);
+        else if (id < nq + sw.blocks) weights_at<T>(sw.w_ema, sw.w_new, sq.Q, sw.beta, (int64_t)(id - nq) * 256 + threadIdx.x);
+        else keep_scores<T, 256>(sw.kept, id - nq - sw.blocks, threadIdx.x);
     }
 }
 
@@ -1875,9 +1879,9 @@ int run_mfma(const MfmaProblem& mp, hipStream_t stream) {
             if (by < 1) by = 1;
             StageGrid g;
             g.q_bx = (int)bx; g.q_by = (int)by; g.k_bx = (int)(n_pad / kBN); g.k_by = (int)splits;
-            const StageWeights sw{mp.w_ema, mp.w_new, mp.beta, mp.key_order, mp.n_visible};
             const int64_t w_blocks = mp.make_weights ? (mp.Q + kColSlack + 255) / 256 : 0;
-            const int64_t blocks = bx * by + (n_pad / kBN) * splits + w_blocks + (mp.own_order ? 1 : 0);
+            const StageWeights sw{mp.w_ema, mp.w_new, mp.beta, mp.key_order, mp.n_visible, (int)w_blocks, mp.kept};
+            const int64_t blocks = bx * by + (n_pad / kBN) * splits + w_blocks + kept_pieces(mp.kept, 256) + (mp.own_order ? 1 : 0);
             if (blocks > 0x7fffffff) return CKV_ERR_UNSUPPORTED;
             hipLaunchKernelGGL((stage_kernel<T, kD>), dim3((unsigned)blocks), dim3(256), 0, stream, sp, sq, g, sw);
         }

@@ -23,9 +23,10 @@
 // Why this equals the serial loop: within one cascade the n-th insert of a call always lands in
 // ring position (start + stored + n) mod W whatever the scores are; only WHICH arrival owns a
 // slot depends on scores, and that is decided inside the group of arrivals between two inserts.
-#include "ckv_attn_internal.h"
+#include "ckv_finish.h"
 #include "ckv_update_token.h"
 
+#include <algorithm>
 #include <type_traits>
 
 #include <mutex>
@@ -35,7 +36,7 @@ namespace {
 
 constexpr int kMaxCascades = 64;
 constexpr int kPlanMaxTokens = 8192;   // incoming tokens one plan launch takes at most
-constexpr int kRingPer = 8;            // kPlanMaxTokens / 1024 threads, and enough for 256 tokens on 256 threads
+constexpr int kRingPer = 8;            // kPlanMaxTokens / 1024 threads, and enough for kBothLds's tokens on kClosedThreads
 
 constexpr int32_t kPosChange = 1;      // the call put a token into the cascades, so the position ids change
 constexpr int32_t kPlanned = 2;        // the unit has been planned by the steady-state kernel
@@ -156,6 +157,29 @@ __device__ inline bool closed_forms(const ckv_update_args& A, const Unit& u, int
     return __builtin_amdgcn_ballot_w64(ok) == ~0ull;
 }
 
+// The scores that a plan looks at: those that lie in memory, ...
+struct StoredScores {
+    static constexpr int kRing = kRingPer;
+    const ckv_update_args& A;
+    int64_t s_base, cs_base;
+    __device__ StoredScores(const UpdateParams& p, const Unit& u)
+        : A(p.a), s_base(u.n * A.s_stride[0] + u.h * A.s_stride[1] + p.token_offset * A.s_stride[2]),
+          cs_base(u.n * A.cache_s_stride[0] + u.h * A.cache_s_stride[1]) {}
+    __device__ float token(int t) const { return load_as_float(A.s, s_base + (int64_t)t * A.s_stride[2], A.dtype); }
+    __device__ float slot(int64_t i) const { return load_as_float(A.cache_s, cs_base + i * A.cache_s_stride[2], A.dtype); }
+};
+// ... and those that the launch is about to finish (FinishProblem::before).
+template <typename T, int kHow>
+struct FinishingScores {
+    static constexpr int kRing = 3;   // of kClosedThreads: kBothLds's tokens
+    const FinishProblem& f;
+    int64_t b, kvh;
+    __device__ float token(int t) const { return Elem<T>::to_float(token_score<T, kHow>(f, b, kvh, t)); }
+    __device__ float slot(int64_t i) const {
+        return Elem<T>::to_float(slot_score<T, kHow>(f, b, kvh, i, reinterpret_cast<const T*>(f.before)[(b * f.KVH + kvh) * f.S + i]));
+    }
+};
+
 // Workgroup `part` of `parts` plans its share of the inserts of cascade `mine`: a thread per insert folds the arrivals up to the next insert into the group's winner
 // ("later wins iff score >=", cascading_cache.py:699) and writes where every member ends up.  Every chain entry has one
 // writer: cascade i owns the pointers of cascade i's arrivals.  Those are entries of the ring before as it was before the
@@ -167,13 +191,12 @@ __device__ inline bool closed_forms(const ckv_update_args& A, const Unit& u, int
 // inserts 7.1 (16 units x 16 rings of 2048: 15.6; with 256 threads 7.2 and 24.1, with 1024 8.3 and 16.2).  Touched cascades
 // used to be left to the walk, to which a call like 256 tokens on rings of 128 or 4096 on rings of 2048 goes at every other
 // alignment: 14.4 and 77 us there, 6.1 and 15.6 here.  A pass that read its arrivals into registers instead of LDS: level.
+template <typename Scores>
 __device__ inline void plan_closed(const UpdateParams& p, const Unit& u, const ClosedCascade& forms, unsigned long long touched,
-                                   int mine, int part, int parts, unsigned char* smem) {
+                                   int mine, int part, int parts, unsigned char* smem, const Scores& scores_of) {
     const ckv_update_args& A = p.a;
     const int tid = threadIdx.x, T = blockDim.x;
     const int C = A.cascades, W = (int)A.window_size, cap = p.k_sub;
-    const int64_t cs_base = u.n * A.cache_s_stride[0] + u.h * A.cache_s_stride[1];
-    const int64_t s_base = u.n * A.s_stride[0] + u.h * A.s_stride[1] + p.token_offset * A.s_stride[2];
     int32_t* first = p.first + u.bh * A.K + p.token_offset;
     int32_t* next_of = p.next_of + u.bh * A.max_seq_len;
     int32_t* src[2] = {reinterpret_cast<int32_t*>(smem), reinterpret_cast<int32_t*>(smem) + cap};
@@ -184,8 +207,7 @@ __device__ inline void plan_closed(const UpdateParams& p, const Unit& u, const C
         return i * W + (ring >= W ? ring - W : ring);
     };
     auto score_of = [&](int from) -> float {
-        return from < 0 ? load_as_float(A.s, s_base + (int64_t)(-1 - from) * A.s_stride[2], A.dtype)
-                        : load_as_float(A.cache_s, cs_base + (int64_t)from * A.cache_s_stride[2], A.dtype);
+        return from < 0 ? scores_of.token(-1 - from) : scores_of.slot(from);
     };
     auto point = [&](int from, int slot) {  // the arrival that came from `from` ends up in `slot` (-1: nowhere)
         if (from < 0) first[-1 - from] = slot;
@@ -289,7 +311,8 @@ __device__ inline int32_t tracker_word(int32_t stored, int32_t start, int32_t W)
 
 // Workgroups of a unit: one per cascade and extra ones for those with more inserts than threads, as far as they go (with
 // periods that double, cascades of a call of K tokens insert at most 2 K between them).  False: the unit is not planned here.
-__device__ inline bool plan_steady(const UpdateParams& p, const Unit& u, int block, int extra, unsigned char* smem) {
+template <typename Scores>
+__device__ inline bool plan_steady(const UpdateParams& p, const Unit& u, int block, int extra, unsigned char* smem, const Scores& scores_of) {
     const ckv_update_args& A = p.a;
     const int tid = threadIdx.x, lane = tid % CKV_WAVE, T = blockDim.x;
     const int C = A.cascades;
@@ -322,18 +345,20 @@ __device__ inline bool plan_steady(const UpdateParams& p, const Unit& u, int blo
     if (part == 0 && tid == mine) {
         p.trackers[u.bh * C + mine] = (int32_t)(((uint32_t)forms.sx + (uint32_t)forms.E) % (uint32_t)A.window_size);
     }
-    plan_closed(p, u, forms, touched, mine, part, parts, smem);
+    plan_closed(p, u, forms, touched, mine, part, parts, smem, scores_of);
     return true;
 }
 
 __global__ void __launch_bounds__(kClosedThreads) ckv_update_plan_steady_kernel(UpdateParams p) {
     extern __shared__ __align__(16) unsigned char smem[];
     const Unit u(p.a);
-    if (!plan_steady(p, u, (int)blockIdx.x, (int)gridDim.x - p.a.cascades, smem) && blockIdx.x == 0 && threadIdx.x == 0) p.flags[u.bh] = 0;
+    if (!plan_steady(p, u, (int)blockIdx.x, (int)gridDim.x - p.a.cascades, smem, StoredScores(p, u)) && blockIdx.x == 0 && threadIdx.x == 0)
+        p.flags[u.bh] = 0;
 }
 
 // The walk over all arrivals, a workgroup per unit.
-__device__ inline void plan_walk(const UpdateParams& p, const Unit& u, unsigned char* smem) {
+template <typename Scores>
+__device__ inline void plan_walk(const UpdateParams& p, const Unit& u, unsigned char* smem, const Scores& scores_of) {
     const ckv_update_args& A = p.a;
     const int tid = threadIdx.x, T = blockDim.x;
     const int64_t n = u.n, h = u.h, bh = u.bh;
@@ -370,7 +395,6 @@ __device__ inline void plan_walk(const UpdateParams& p, const Unit& u, unsigned 
     const int64_t* g_stored = A.stored_tokens + n * A.tracker_stride[0] + h * A.tracker_stride[1];
     const int64_t* g_start = A.start_indices + n * A.tracker_stride[0] + h * A.tracker_stride[1];
     const int64_t* g_sinks = A.stored_sinks + n * A.stored_sinks_stride[0] + h * A.stored_sinks_stride[1];
-    const int64_t cs_base = n * A.cache_s_stride[0] + h * A.cache_s_stride[1];
     int32_t* first = p.first + bh * A.K + p.token_offset;
     int32_t* next_of = p.next_of + bh * S;
 
@@ -386,9 +410,7 @@ __device__ inline void plan_walk(const UpdateParams& p, const Unit& u, unsigned 
         sx_l[i] = sx;
         per_l[i] = A.do_cache_every_n[i];
         // the plan never writes scores, so the newest slot's score can be read before its cascade's turn
-        lead_l[i] = st > 0 ? load_as_float(A.cache_s, cs_base + ((int64_t)i * W + (sx - 1 + st) % st) * A.cache_s_stride[2],
-                                           A.dtype)
-                           : 0.f;
+        lead_l[i] = st > 0 ? scores_of.slot((int64_t)i * W + (sx - 1 + st) % st) : 0.f;
     }
     // level-0 arrivals: the non-sink tokens of this launch, in order (cascading_cache.py:447-462)
     for (int t = tid; t < cap; t += T) {
@@ -399,8 +421,7 @@ __device__ inline void plan_walk(const UpdateParams& p, const Unit& u, unsigned 
             const int a = t - n_sink_new;
             a_src[0][a] = -1 - t;
             a_trig[0][a] = (uint16_t)t;
-            a_score[0][a] = load_as_float(
-                A.s, n * A.s_stride[0] + h * A.s_stride[1] + (p.token_offset + t) * A.s_stride[2], A.dtype);
+            a_score[0][a] = scores_of.token(t);
         }
     }
     __syncthreads();
@@ -435,13 +456,11 @@ __device__ inline void plan_walk(const UpdateParams& p, const Unit& u, unsigned 
         int n_ring = stored0 + nA - (int)W;
         if (n_ring > stored0 - 1) n_ring = stored0 - 1;
         if (i + 1 >= C) n_ring = 0;
-        float ring_pre[kRingPer];
+        float ring_pre[Scores::kRing];
 #pragma unroll
-        for (int r = 0; r < kRingPer; r++) {
+        for (int r = 0; r < Scores::kRing; r++) {
             const int j = r * T + tid;
-            ring_pre[r] = j < n_ring ? load_as_float(A.cache_s, cs_base + (l + mod_w(start0 + (int64_t)j)) * A.cache_s_stride[2],
-                                                     A.dtype)
-                                     : 0.f;
+            ring_pre[r] = j < n_ring ? scores_of.slot(l + mod_w(start0 + (int64_t)j)) : 0.f;
         }
 
         // ---- pass 1: insert flags (accept, or the first arrival of an empty cascade:
@@ -490,7 +509,7 @@ __device__ inline void plan_walk(const UpdateParams& p, const Unit& u, unsigned 
             w_score[e + 1] = wv;
         }
 #pragma unroll
-        for (int r = 0; r < kRingPer; r++) {
+        for (int r = 0; r < Scores::kRing; r++) {
             const int j = r * T + tid;
             if (j < n_ring) ring_l[j] = ring_pre[r];
         }
@@ -551,7 +570,7 @@ __global__ void ckv_update_plan_kernel(UpdateParams p) {
     extern __shared__ __align__(16) unsigned char smem[];
     const Unit u(p.a);
     if (p.flags[u.bh] & kPlanned) return;  // the steady-state kernel has planned this unit
-    plan_walk(p, u, smem);
+    plan_walk(p, u, smem, StoredScores(p, u));
 }
 
 // Both in one launch: the first workgroup of a unit walks its arrivals if the others, which look at the same trackers (apply commits
@@ -563,7 +582,27 @@ __global__ void __launch_bounds__(kThreads) ckv_update_plan_both_kernel(UpdatePa
     extern __shared__ __align__(16) unsigned char smem[];
     const Unit u(p.a);
     const int block = (int)blockIdx.x - 1;
-    if (!plan_steady(p, u, block, (int)gridDim.x - 1 - p.a.cascades, smem) && block < 0) plan_walk(p, u, smem);
+    const StoredScores scores(p, u);
+    if (!plan_steady(p, u, block, (int)gridDim.x - 1 - p.a.cascades, smem, scores) && block < 0) plan_walk(p, u, smem, scores);
+}
+
+// The same beside the blocks that finish the scores of a chunk: the first `plans` of a unit plan, for which they work the scores they
+// need out for themselves (FinishingScores).  Bound by the plan's chain of trips to memory, no longer than before: the sums of a kv
+// head's query heads are requested together (7.3 us; the two launches 4.9 and 6.6.  With a branch a head it took 11: the code is cold).
+// Calls, us, 28 heads on 4 kv heads, 19 rows x 1 K slots 43.5 -> 40.0; 3 streams, 32 on 8, 163 x 2560 98.0 -> 94.6; 32 on 8, 509 x 16 K
+// 268 -> 264; float32, 256 x 512 70.5 -> 67.8, 74 x 776 60.6 -> 57.8.
+template <typename T, int kHow>
+__global__ void __launch_bounds__(kClosedThreads) ckv_finish_plan_kernel(UpdateParams p, FinishProblem f, int plans) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    const Unit u(p.a);
+    if ((int)blockIdx.x >= plans) {
+        const int64_t i = (int64_t)((int)blockIdx.x - plans) * kClosedThreads + threadIdx.x;
+        if (i < f.S + f.Q) finish_score<T, kHow>(f, u.n, u.h, i);
+        return;
+    }
+    const int block = (int)blockIdx.x - 1;
+    const FinishingScores<T, kHow> scores{f, u.n, u.h};
+    if (!plan_steady(p, u, block, plans - 1 - p.a.cascades, smem, scores) && block < 0) plan_walk(p, u, smem, scores);
 }
 
 // The walk of a single incoming token (the decode step), by one wavefront: lane i fetches what cascade i may need (trackers,
@@ -1165,7 +1204,28 @@ void launch_timed(int stage, Kernel kernel, dim3 grid, dim3 block, size_t lds, h
     else hipLaunchKernelGGL(kernel, grid, block, lds, stream, p);
 }
 
-int run_update(const ckv_update_args& A, void* workspace, int64_t* row, int64_t row_shift, hipStream_t stream) {
+// workgroups of a unit that plan `tokens` tokens, so many threads each: see plan_steady, and one more that may walk
+inline int64_t plan_blocks(int cascades, int64_t tokens, int threads) { return cascades + 2 * tokens / threads + 1; }
+
+int launch_finish_plan(const UpdateParams& p, const FinishProblem& f, size_t lds, hipStream_t stream) {
+    const int plans = (int)plan_blocks(p.a.cascades, p.k_sub, kClosedThreads);
+    const dim3 grid((unsigned)(plans + (f.S + f.Q + kClosedThreads - 1) / kClosedThreads), (unsigned)p.a.H, (unsigned)p.a.N);
+    auto launch = [&](auto kernel) -> int {
+        if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(kernel), (int)lds)) return rc;
+        hipLaunchKernelGGL(kernel, grid, dim3(kClosedThreads), lds, stream, p, f, plans);
+        return CKV_OK;
+    };
+    auto of_type = [&](auto tag) -> int {
+        using T = decltype(tag);
+        return f.head_reduction == CKV_REDUCE_MEDIAN ? launch(ckv_finish_plan_kernel<T, kMedianOfFew>)
+               : f.head_reduction == CKV_REDUCE_MAX  ? launch(ckv_finish_plan_kernel<T, kMaxOfFew>)
+                                                     : launch(ckv_finish_plan_kernel<T, kMeanOfFew>);
+    };
+    return f.dtype == CKV_F32 ? of_type(float{}) : f.dtype == CKV_F16 ? of_type(__half{}) : of_type(__hip_bfloat16{});
+}
+
+// `finish`: the scores that the call's attention has still to finish (update_plans_beside_finish), or null
+int run_update(const ckv_update_args& A, void* workspace, int64_t* row, int64_t row_shift, hipStream_t stream, const FinishProblem* finish = nullptr) {
     const int es = (int)elem_bytes(A.dtype);
     const bool vec = A.kv_stride[3] == 1 && A.cache_stride[3] == 1 && (A.num_sink == 0 || A.sink_stride[3] == 1) &&
                      (A.HID * es) % 16 == 0 && A.HID * es <= 16 * 64 && aligned16(A.k) && aligned16(A.v) &&
@@ -1222,14 +1282,16 @@ int run_update(const ckv_update_args& A, void* workspace, int64_t* row, int64_t 
             auto launch_both = [&](auto threads) -> int {
                 auto kernel = ckv_update_plan_both_kernel<threads.value>;
                 if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(kernel), (int)lds)) return rc;
-                launch_timed(CKV_STAGE_PLAN, kernel, dim3((unsigned)(A.cascades + 2 * ksub / threads.value) + 1, H, N), dim3(threads.value), lds,
+                launch_timed(CKV_STAGE_PLAN, kernel, dim3((unsigned)plan_blocks(A.cascades, ksub, threads.value), H, N), dim3(threads.value), lds,
                              stream, p);
                 prof_empty(CKV_STAGE_PLAN);   // counted as two either way
                 return CKV_OK;
             };
-            if (lds <= kBothLds) {
+            if (finish) {
+                if (int rc = launch_finish_plan(p, *finish, lds, stream)) return rc;
+            } else if (lds <= kBothLds) {
                 if (int rc = launch_both(std::integral_constant<int, kClosedThreads>{})) return rc;
-            } else if ((int64_t)(A.cascades + 2 * ksub / 1024 + 1) * A.N * A.H <= di.cus) {
+            } else if (plan_blocks(A.cascades, ksub, 1024) * A.N * A.H <= di.cus) {
                 if (int rc = launch_both(std::integral_constant<int, 1024>{})) return rc;
             } else {
                 if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(ckv_update_plan_steady_kernel), (int)lds_closed)) return rc;
@@ -1313,6 +1375,26 @@ int check_update(const ckv_update_args* args, bool* empty) {
     const ckv_update_args& A = *args;
     const int64_t need = ckv_update_workspace_bytes(A.N, A.H, A.K, A.max_seq_len, A.cascades);
     return !A.workspace || A.workspace_bytes < need ? CKV_ERR_WORKSPACE : CKV_OK;
+}
+}  // namespace ckv
+
+namespace ckv {
+bool update_plans_beside_finish(const ckv_attn_args& a, const ckv_update_args& u) {
+    auto same = [](const int64_t* x, const int64_t* y, int n) { return std::equal(x, x + n, y); };
+    if (!(u.K == a.Q && a.Q > 1 && u.N == a.B && u.H == a.KVH && u.HID == a.D && u.dtype == a.dtype && u.num_sink == a.num_sink &&
+          u.max_seq_len == a.S && u.cache_s == a.cache_s && same(u.cache_s_stride, a.cache_s_stride, 3) && u.s == a.new_scores && same(u.s_stride, a.new_scores_stride, 3)))
+        return false;
+    if (a.homogeneous_heads || a.H / a.KVH > kFewHeads) return false;
+    DeviceInfo di;
+    if (current_device_info(&di)) return false;
+    // As many tokens as the walk's LDS leaves a compute unit four workgroups for (see kBothLds; the finishing ones reserve it too), and
+    // all in one round of workgroups.
+    return u.K <= kPlanMaxTokens && plan_lds_bytes((int)u.K) <= kBothLds &&
+           (plan_blocks(u.cascades, u.K, kClosedThreads) + (a.S + a.Q + kClosedThreads - 1) / kClosedThreads) * u.N * u.H <= 4 * (int64_t)di.cus;
+}
+
+int launch_finish_and_update(const FinishProblem& f, const ckv_update_args& u, hipStream_t stream) {
+    return run_update(u, u.workspace, nullptr, 0, stream, &f);
 }
 }  // namespace ckv
 

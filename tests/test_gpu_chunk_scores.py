@@ -43,3 +43,38 @@ def test_chunks_whose_keys_are_shared_out_two_tiles_each(H, KVH, D, dtype):
 
     led = run_teacher_forced(1, H, KVH, D, 4, 256, 4, 0, 0, dtype, seed=5, std=0.7, steps=[130, 16, 2, 65, 64, 129, 33, 100, 128, 127, 130, 130])
     assert led.flips <= flip_bound(led), led.summary()
+
+
+# caches that fill (the walk) and full ones (closed forms), periods that do not divide each other, rings shorter than the chunk, the most
+# tokens that share the launch and one more, seven and eight heads per kv head, more workgroups than one round takes
+@pytest.mark.parametrize("B,H,KVH,D,NS,W,C,dtype,func,reduction,q_len,calls", [
+    (1, 8, 2, 128, 4, 33, 4, torch.bfloat16, "pow2", "mean", 17, 24),
+    (2, 14, 2, 128, 0, 64, 3, torch.float16, "pow2", "median", 50, 10),
+    (1, 8, 1, 64, 3, 40, 5, torch.bfloat16, "pow2", "median", 2, 60),
+    (1, 4, 2, 64, 4, 128, 2, torch.float16, "iplus1", "max", 100, 8),
+    (1, 8, 2, 128, 4, 128, 4, torch.float32, "pow2", "max", 256, 6),
+    (3, 6, 2, 64, 1, 96, 1, torch.float32, "pow2", "median", 31, 8),
+    (1, 4, 1, 128, 64, 512, 8, torch.bfloat16, "pow2", "mean", 1092, 6),
+    (1, 4, 1, 128, 64, 512, 8, torch.bfloat16, "pow2", "mean", 1093, 6),
+    (4, 16, 16, 64, 4, 8192, 2, torch.float16, "pow2", "max", 300, 3),
+])
+def test_update_planned_beside_the_finishing_scores_equals_two_calls(B, H, KVH, D, NS, W, C, dtype, func, reduction, q_len, calls):
+    from cascading_kv_cache_amd.cascade_attention import cascade_attention, default_inv_freq
+    from test_gpu_token_step import STATE, bits
+
+    one, two = (make_pair(B, KVH, D, NS, W, C, dtype, func=func, reduction=reduction)[0] for _ in range(2))
+    one.beta = two.beta = 0.99   # scores that change at every call
+    inv_freq = default_inv_freq(D, 5e5, "cuda:0")
+    gen = torch.Generator().manual_seed(7)
+    for call in range(calls):
+        q, k, v = ((torch.randn(B, q_len, h, D, generator=gen) * 0.7).to(dtype).cuda().transpose(1, 2) for h in (H, KVH, KVH))
+        if call % 4 == 2:
+            q = torch.zeros_like(q)   # every visible key weighs the same: ties
+        if call == calls - 1:
+            q[:, 0, q_len // 2] = float("nan")   # and a head's scores that are no numbers
+        out1, new1 = cascade_attention(q, k, v, one, 0, inv_freq)
+        out2, new2 = cascade_attention(q, k, v, two, 0, inv_freq, update_cache=False)
+        two.update_state(k, v, 0, new2)
+        assert torch.equal(bits(out1), bits(out2)) and torch.equal(bits(new1), bits(new2)), call
+        for name in STATE:
+            assert torch.equal(bits(getattr(one, name)[0]), bits(getattr(two, name)[0])), (call, name)
