@@ -56,11 +56,15 @@ def workspace(device: torch.device, nbytes: int, stream: int = 0) -> Tensor:
 
 
 _SAME_DEVICE = contextlib.nullcontext()
+# Its public form first asks whether the device runtime is up, which it is where a tensor lives on a device (0.2 of 0.3 us).  Not public:
+# a torch without it takes that way.
+_current_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)
+_data_ptr = Tensor.data_ptr
 
 
 def on_device(device: torch.device):
     """``torch.cuda.device(device)``, which costs a single-token step 1.4 us of host time, where another device is current."""
-    if device.index is not None and torch.cuda.current_device() == device.index:
+    if device.type == "cuda" and device.index is not None and _current_device() == device.index:
         return _SAME_DEVICE
     return torch.cuda.device(device)
 
@@ -365,10 +369,11 @@ class CascadingKVCache:
         it was described from.  (Object identity would not do: callers may assign a new tensor to
         ``score_cache[l]`` every step, as cascade_attention.py:222-224 does, and a freed object's id is
         handed out again.)"""
-        ts = (self.key_cache[L], self.value_cache[L], self.score_cache[L], self.sink_keys[L], self.sink_values[L],
+        scores = self.score_cache[L]
+        ts = (self.key_cache[L], self.value_cache[L], scores, self.sink_keys[L], self.sink_values[L],
               self.mask[L], self.sink_mask[L], self.pos[L], self.og_pos[L], self.sink_pos[L], self.stored_tokens[L],
               self.start_indices[L], self.stored_sinks[L], self.do_cache_every_n[L], self._seen_dev)
-        return tuple(t.data_ptr() for t in ts) + (self.score_cache[L].stride(), self.score_cache[L].dtype)
+        return (*map(_data_ptr, ts), scores.stride(), scores.dtype)
 
     def update(self, key_states: Tensor, value_states: Tensor, layer_idx: int, score_states: Tensor = None):
         """cascading_cache.py:1297-1348."""
