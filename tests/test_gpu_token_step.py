@@ -136,3 +136,43 @@ def test_a_refused_step_counts_nothing(monkeypatch):
     with pytest.raises(_abi.CkvError):
         cache.update_state(k, k, 0, k[..., 0])
     assert (cache._seen_tokens, cache._seen_host, cache._seen_pending) == before
+
+
+def lower_median(vals):
+    """Of the heads along dim 2: the value that takes place (G - 1) // 2, a NaN behind all others, as counting ranks finds it."""
+    G = vals.size(2)
+    order = torch.where(vals.isnan(), torch.full_like(vals, float("inf")), vals).sort(dim=2).values
+    return order[:, :, (G - 1) // 2]
+
+
+@pytest.mark.parametrize("B,window", [(1, 96), (40, 64)])   # rows, scores and update in one launch; apart
+@pytest.mark.parametrize("G", [1, 2, 4, 7, 8])
+@pytest.mark.parametrize("spoilt", [False, True])
+def test_median_of_a_groups_heads(spoilt, G, B, window):
+    """Scores of a step that starts from zeros, against the median of the same heads' scores as kv heads of their own.  A head of no
+    numbers counts as the largest."""
+    from cascading_kv_cache_amd.cascade_attention import cascade_attention, default_inv_freq
+
+    KVH, gen = 2, torch.Generator().manual_seed(G)
+    inv_freq = default_inv_freq(128, 5e5, "cuda:0")
+    draw = lambda h, n: (torch.randn(B, n, h, 128, generator=gen) * 0.7).bfloat16().cuda().transpose(1, 2)   # noqa: E731
+    steps = [(draw(KVH * G, n), draw(KVH, n), draw(KVH, n)) for n in (2 * window + 4, 1)]
+    if spoilt:
+        steps[-1][0][:, 0] = float("nan")
+    got = []
+    for heads in (KVH, KVH * G):
+        cache = pair(B, heads, 4, window, 2, torch.bfloat16, "pow2", True, "median")[0]
+        for i, (q, k, v) in enumerate(steps):
+            if heads != KVH:
+                k, v = (x.repeat_interleave(G, 1) for x in (k, v))
+            cache.score_cache[0].zero_()
+            new = cascade_attention(q, k, v, cache, 0, inv_freq, update_cache=i == 0)[1]
+        got.append((cache.score_cache[0].float(), new.float()))
+    (scores, new), (each, each_new) = got
+    for mine, every in ((scores, each), (new, each_new)):
+        want = lower_median(every.view(B, KVH, G, -1))
+        if G == 1:
+            want = every
+        assert torch.equal(mine.isnan(), want.isnan())
+        # one rounding to bfloat16 of probabilities that two kernels work out
+        assert torch.allclose(mine, want, rtol=2.0 ** -7, atol=1e-9, equal_nan=True)
