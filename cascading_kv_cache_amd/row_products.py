@@ -67,13 +67,14 @@ def _at(t) -> int:
 
 
 def linear_rows(x, weight, order, bias=None, residual=None, norm=None, eps=0.0, gated=False):
-    """``ckv_linear_rows`` of ``x (B, q, k)``, whose rows lie a fixed stride apart."""
+    """``ckv_linear_rows`` of ``x (B, q, k)``, whose rows lie a fixed stride apart (a single row has none)."""
     n, k = weight.shape
+    rows = x.size(0) * x.size(1)
     out = torch.empty(x.shape[:-1] + (n // 2 if gated else n,), dtype=x.dtype, device=x.device)
-    stride = x.stride(0) if x.size(1) == 1 else x.stride(1)
+    stride = k if rows == 1 else x.stride(0) if x.size(1) == 1 else x.stride(1)
     with on_device(x.device):
         _abi.check(_abi.lib().ckv_linear_rows(x.data_ptr(), weight.data_ptr(), _at(bias), _at(residual), _at(norm), eps, out.data_ptr(),
-                                              x.size(0) * x.size(1), n, k, max(stride, k), int(gated), order[0], order[1],
+                                              rows, n, k, stride, int(gated), order[0], order[1],
                                               _abi.dtype_code(x.dtype), raw_stream(x.device)), "ckv_linear_rows")
     return out
 

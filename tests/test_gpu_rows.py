@@ -63,6 +63,19 @@ def test_rows_a_stride_apart():
         assert not rp._rows_apart(x)
 
 
+@pytest.mark.parametrize("extra", [1, 3, 4, 8])
+def test_one_row_of_a_wider_buffer(extra):
+    """A single row has no distance to a next one, whatever the buffer's rows have; several such rows are torch's to multiply."""
+    w = torch.randn(32, 256, device="cuda").bfloat16()
+    wide = torch.randn(1, 2, 256 + extra, device="cuda").bfloat16()
+    for x in (wide[:, :1, :256], wide[..., :256]):
+        one = x.size(1) == 1
+        assert rp._rows_apart(x) == (one or extra % 8 == 0)
+        with torch.no_grad():
+            got = rp.row_linear(x, w, {1: (1, 1), 2: (1, 1)})
+        assert torch.equal(got, rp.linear_rows(x.contiguous(), w, (1, 1)) if one or extra % 8 == 0 else F.linear(x, w))
+
+
 @pytest.mark.parametrize("preset", ["llama3.1-8b", "qwen2-7b", "tiny"])
 def test_steps_of_a_fused_decoder_have_the_bits_of_torchs_products(preset):
     """One layer's steps by row products where an order is torch's, and by torch's operations: the same bits in the cache, and logits that
