@@ -20,7 +20,7 @@ from torch import nn
 
 from .cascading_cache import CascadingKVCache
 from .latency import ProjectedCascadeAttention
-from .row_products import FAST_ORDER, MAX_ROWS, ROW_TYPES, followed as _followed, gated_silu, library_orders, plain, row_linear
+from .row_products import FAST_ORDER, MAX_ROWS, ROW_TYPES, followed as _followed, gated_silu, library_orders, own_methods, plain, row_linear
 
 
 @dataclass
@@ -86,6 +86,11 @@ class GatedMLP(nn.Module):
         return self.down_proj(gated_silu(nn.functional.linear(x, self._w_gate_up)))
 
 
+own_methods(RMSNorm)
+own_methods(GatedMLP)
+own_methods(ProjectedCascadeAttention, "forward_cascade", "qkv", "attend")
+
+
 class DecoderLayer(nn.Module):
     def __init__(self, cfg, layer_idx, dtype, device):
         super().__init__()
@@ -103,7 +108,7 @@ class DecoderLayer(nn.Module):
         attn, mlp = self.self_attn, self.mlp
         return (self._orders is not None and x.dim() == 3 and x.size(0) * x.size(1) in self._orders["any"] and x.is_cuda and not _followed(x)
                 and not torch.is_autocast_enabled() and isinstance(cache, CascadingKVCache)
-                and plain(attn, ProjectedCascadeAttention, "forward_cascade", "qkv", "attend") and plain(mlp, GatedMLP)
+                and plain(attn, ProjectedCascadeAttention) and plain(mlp, GatedMLP)
                 and attn._w_qkv is not None and mlp._w_gate_up is not None
                 and plain(attn.o_proj, nn.Linear) and plain(mlp.down_proj, nn.Linear)
                 and attn.o_proj.bias is None and mlp.down_proj.bias is None

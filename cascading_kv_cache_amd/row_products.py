@@ -34,13 +34,35 @@ def followed(x) -> bool:
             or torch.jit.is_tracing() or torch.compiler.is_compiling())
 
 
-def plain(module, kind, *methods) -> bool:
-    """Is calling ``module`` nothing but ``kind.forward`` (and the named methods ``kind``'s own): no subclass, no hooks, no method put on
-    the object?"""
+#: kind of module: (name, method) of what calling one runs
+_OWN = {}
+
+
+def own_methods(kind, *names):
+    """Takes down the methods that calling a ``kind`` runs, ``forward`` and the named ones, for :func:`plain` to know them by."""
+    def own(name):
+        method, home = getattr(kind, name), next(c for c in kind.__mro__ if name in vars(c))
+        # torch's classes may have been given another one before
+        original = (method.__module__ == home.__module__ and method.__qualname__.startswith(home.__qualname__ + ".")
+                    and not hasattr(method, "__wrapped__"))
+        return name, method if original else None
+    _OWN[kind] = tuple(map(own, ("__call__", "_call_impl", "forward", *names)))
+
+
+own_methods(nn.Linear)
+
+
+def plain(module, kind) -> bool:
+    """Is calling ``module`` nothing but the methods that :func:`own_methods` has taken down for ``kind``: no subclass, no hooks, no
+    method put on the object or on its class since?"""
     every = nn.modules.module
-    return (type(module) is kind and not module._forward_hooks and not module._forward_pre_hooks
-            and not getattr(every, "_global_forward_hooks", True) and not getattr(every, "_global_forward_pre_hooks", True)
-            and not any(name in module.__dict__ for name in ("forward", *methods)))
+    if not (type(module) is kind and not module._forward_hooks and not module._forward_pre_hooks
+            and not getattr(every, "_global_forward_hooks", True) and not getattr(every, "_global_forward_pre_hooks", True)):
+        return False
+    for name, method in _OWN[kind]:
+        if getattr(kind, name) is not method or name in module.__dict__:
+            return False
+    return True
 
 
 def gated_silu(gate_up):

@@ -1,0 +1,45 @@
+"""When a decoder's step may leave torch's operations for products of a few rows: the parts that need no device."""
+import functools
+
+import pytest
+import torch
+from torch import nn
+
+from cascading_kv_cache_amd import row_products as rp
+from cascading_kv_cache_amd.cascade_attention import CascadeAttention
+from cascading_kv_cache_amd.decoder import PRESETS, GatedMLP, RMSNorm
+from cascading_kv_cache_amd.latency import ProjectedCascadeAttention
+
+MAKE = {nn.Linear: lambda: nn.Linear(4, 4), RMSNorm: lambda: RMSNorm(4, 1e-5, torch.float32, "cpu"),
+        GatedMLP: lambda: GatedMLP(PRESETS["tiny"], torch.float32, "cpu"),
+        ProjectedCascadeAttention: lambda: ProjectedCascadeAttention(64, 2, 1, 32, dtype=torch.float32, device="cpu")}
+
+
+@pytest.mark.parametrize("kind,home,name", [(nn.Linear, nn.Linear, "forward"), (RMSNorm, RMSNorm, "forward"), (GatedMLP, GatedMLP, "forward"),
+                                            (ProjectedCascadeAttention, ProjectedCascadeAttention, "qkv"),
+                                            (ProjectedCascadeAttention, CascadeAttention, "forward"),
+                                            (ProjectedCascadeAttention, CascadeAttention, "forward_cascade"),
+                                            (GatedMLP, nn.Module, "__call__"), (nn.Linear, nn.Module, "_call_impl")])
+def test_methods_put_on_a_class_or_an_object_are_seen(kind, home, name, monkeypatch):
+    module = MAKE[kind]()
+    assert rp.plain(module, kind)
+    own = getattr(home, name)
+
+    @functools.wraps(own)
+    def other(self, *args, **kw):
+        return own(self, *args, **kw)
+
+    monkeypatch.setattr(home, name, other)
+    assert not rp.plain(module, kind)
+    monkeypatch.undo()
+    assert rp.plain(module, kind)
+    object.__setattr__(module, name, other)
+    assert not rp.plain(module, kind)
+
+
+def test_a_method_put_on_torchs_class_before_is_seen(monkeypatch):
+    own = nn.Linear.forward
+    monkeypatch.setattr(nn.Linear, "forward", functools.wraps(own)(lambda self, x: own(self, x)))
+    monkeypatch.setattr(rp, "_OWN", dict(rp._OWN))
+    rp.own_methods(nn.Linear)
+    assert not rp.plain(nn.Linear(4, 4), nn.Linear)
