@@ -92,6 +92,8 @@ own_methods(ProjectedCascadeAttention, "forward_cascade", "qkv", "attend")
 
 
 class DecoderLayer(nn.Module):
+    _orders = None   # of the products of few rows, see CascadeDecoder.fuse_projections; saved layers may have none
+
     def __init__(self, cfg, layer_idx, dtype, device):
         super().__init__()
         self.self_attn = ProjectedCascadeAttention(cfg.hidden_size, cfg.num_heads, cfg.num_kv_heads, cfg.head_dim,
@@ -101,7 +103,6 @@ class DecoderLayer(nn.Module):
         self.mlp = GatedMLP(cfg, dtype, device)
         self.input_layernorm = RMSNorm(cfg.hidden_size, cfg.rms_eps, dtype, device)
         self.post_attention_layernorm = RMSNorm(cfg.hidden_size, cfg.rms_eps, dtype, device)
-        self._orders = None   # of the products of few rows, see CascadeDecoder.fuse_projections
 
     def _as_rows(self, x, cache) -> bool:
         """Are these few rows whose operations nobody follows, and is every module its own?"""

@@ -7,7 +7,7 @@ from torch import nn
 
 from cascading_kv_cache_amd import row_products as rp
 from cascading_kv_cache_amd.cascade_attention import CascadeAttention
-from cascading_kv_cache_amd.decoder import PRESETS, GatedMLP, RMSNorm
+from cascading_kv_cache_amd.decoder import PRESETS, DecoderLayer, GatedMLP, RMSNorm
 from cascading_kv_cache_amd.latency import ProjectedCascadeAttention
 
 MAKE = {nn.Linear: lambda: nn.Linear(4, 4), RMSNorm: lambda: RMSNorm(4, 1e-5, torch.float32, "cpu"),
@@ -43,3 +43,9 @@ def test_a_method_put_on_torchs_class_before_is_seen(monkeypatch):
     monkeypatch.setattr(rp, "_OWN", dict(rp._OWN))
     rp.own_methods(nn.Linear)
     assert not rp.plain(nn.Linear(4, 4), nn.Linear)
+
+
+def test_a_layer_saved_without_orders_keeps_torchs_operations():
+    layer = DecoderLayer(PRESETS["tiny"], 0, torch.float32, "cpu")
+    vars(layer).pop("_orders", None)   # as an object pickled before there were any
+    assert layer._as_rows(torch.zeros(1, 1, 256), None) is False
