@@ -353,10 +353,10 @@ class CascadeAttention(nn.Module):
         query_states, key_states, value_states = self.qkv(
             hidden_states, (bsz, q_len, self.num_heads, self.head_dim),
             (bsz, q_len, self.num_key_value_heads, self.head_dim))
-        out = self.o_proj(self.attend(query_states, key_states, value_states, past_key_value, homogeneous_heads, do_og_pos))
+        out = self.o_proj(self._attend(query_states, key_states, value_states, past_key_value, homogeneous_heads, do_og_pos))
         return out, None, past_key_value
 
-    def attend(self, query_states, key_states, value_states, past_key_value, homogeneous_heads, do_og_pos):
+    def _attend(self, query_states, key_states, value_states, past_key_value, homogeneous_heads, do_og_pos):
         """What lies between the projections: ``(batch, heads, tokens, head_dim)`` in, ``(batch, tokens, hidden)`` out."""
         if not hasattr(self, "_inv_freq") or self._inv_freq.device != query_states.device:
             self._inv_freq = default_inv_freq(self.head_dim, self.rope_theta, query_states.device)

@@ -88,7 +88,7 @@ class GatedMLP(nn.Module):
 
 own_methods(RMSNorm)
 own_methods(GatedMLP)
-own_methods(ProjectedCascadeAttention, "forward_cascade", "qkv", "attend")
+own_methods(ProjectedCascadeAttention, "forward_cascade", "qkv", "_attend", "_split_qkv")
 
 
 class DecoderLayer(nn.Module):
@@ -119,7 +119,7 @@ class DecoderLayer(nn.Module):
         if self._as_rows(x, cache):   # five launches around attention's instead of eleven
             attn, mlp, orders = self.self_attn, self.mlp, self._orders
             qkv = row_linear(x, attn._w_qkv, orders["qkv"], bias=attn._b_qkv, norm=self.input_layernorm)
-            x = row_linear(attn.attend(*attn.split_qkv(qkv), cache, attn.config._homogeneous_heads, attn.config._do_og_pos),
+            x = row_linear(attn._attend(*attn._split_qkv(qkv), cache, attn.config._homogeneous_heads, attn.config._do_og_pos),
                            attn.o_proj.weight, orders["o"], residual=x)
             hidden = row_linear(x, mlp._w_gate_up, orders["gate_up"], norm=self.post_attention_layernorm, gated=True)
             return row_linear(hidden, mlp.down_proj.weight, orders["down"], residual=x)

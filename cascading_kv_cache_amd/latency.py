@@ -62,9 +62,9 @@ class ProjectedCascadeAttention(CascadeAttention):
     def qkv(self, x, size, kv_size):
         if self._w_qkv is None:
             return super().qkv(x, size, kv_size)
-        return self.split_qkv(nn.functional.linear(x, self._w_qkv, self._b_qkv), size, kv_size)
+        return self._split_qkv(nn.functional.linear(x, self._w_qkv, self._b_qkv), size, kv_size)
 
-    def split_qkv(self, rows, size=None, kv_size=None):
+    def _split_qkv(self, rows, size=None, kv_size=None):
         """Rows of ``q | k | v`` as ``qkv`` returns them."""
         size = size or (*rows.shape[:2], self.num_heads, self.head_dim)
         kv_size = kv_size or (*rows.shape[:2], self.num_key_value_heads, self.head_dim)

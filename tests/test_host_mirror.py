@@ -326,3 +326,22 @@ def test_the_gate_stays_with_torch_where_somebody_follows_it(monkeypatch):
         monkeypatch.delattr(torch.autograd.forward_ad, "_current_level")
         assert decoder._followed(x)
         assert torch.equal(decoder.gated_silu(x), torch.nn.functional.silu(x[:, :4]) * x[:, 4:])
+
+
+def test_a_layers_own_helpers_may_have_any_name(monkeypatch):
+    """A layer written against the mixin may call its own methods what it likes."""
+    from cascading_kv_cache_amd import cascade_attention as ca
+    from cascading_kv_cache_amd.latency import ProjectedCascadeAttention
+
+    class Layer(ProjectedCascadeAttention):
+        def attend(self):
+            raise AssertionError("the layer's own")
+
+        split_qkv = attend
+
+    monkeypatch.setattr(ca, "cascade_attention", lambda q, k, v, *args, **kw: (q, None))
+    layer = Layer(64, 2, 1, 32, dtype=torch.float32, device="cpu")
+    for _ in range(2):
+        x = torch.randn(1, 3, 64)
+        assert torch.allclose(layer.forward_cascade(x, past_key_value=None)[0], layer.o_proj(layer.q_proj(x)), atol=1e-5)
+        layer.fuse_projections()
