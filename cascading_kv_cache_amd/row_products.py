@@ -130,37 +130,63 @@ def row_linear(x, weight, orders, bias=None, norm=None, residual=None, gated=Fal
     return y if residual is None else residual + y
 
 
-#: what library_orders has found, by device, type and sizes: facts about torch's products, not about a weight
+# not public: where torch lacks one of them, its public form is slower or there is no such switch
+_SETTINGS = (getattr(torch._C, "_get_blas_preferred_backend", getattr(torch.backends.cuda, "preferred_blas_library", None)),
+             *(getattr(torch._C, name, None) for name in ("_get_cublas_allow_bf16_reduced_precision_reduction",
+                                                          "_get_cublas_allow_fp16_reduced_precision_reduction",
+                                                          "_get_cublas_allow_fp16_accumulation", "_cuda_tunableop_is_enabled")))
+_SETTINGS = tuple(f for f in _SETTINGS if f is not None)
+_tuning = getattr(torch._C, "_cuda_tunableop_is_enabled", lambda: False)
+
+
+def product_settings() -> tuple:
+    """What decides, beside its sizes, which product torch runs (0.5 us)."""
+    return (torch.__version__, *[f() for f in _SETTINGS])
+
+
+#: what library_orders has found, by device, type, sizes and settings: facts about torch's products, not about a weight
 _FOUND = {}
 
 
+def _chains(order, k) -> tuple:
+    """The stretches of 64 elements that each chain of a sum adds up; two orders with the same chains are one."""
+    parts, unit = order
+    chains = (tuple(s for s in range(k // 64) if s // unit % parts == part) for part in range(parts))
+    return tuple(c for c in chains if c)
+
+
 def library_orders(weight, bias=None, most_rows=4):
-    """``{rows: order}`` whose bits are those of ``torch.nn.functional.linear`` for so many rows of 16 bits, found by trying random rows,
-    2 ms a size, once.  Two orders differ in few outputs (4096 x 4096: one of 4000 to 6000), in proportion to the root of the products
-    summed up: enough rows are tried to expect eight differences of a wrong one, twice as many while two are left.  Products so small
-    that this would take more than 64 rows stay with torch."""
-    if weight.device.type != "cuda" or weight.dtype not in ROW_TYPES or not weight.is_contiguous():
+    """``{rows: order}`` whose bits are those of ``torch.nn.functional.linear`` for so many rows of 16 bits, found by trying, 2 ms a
+    size, once.  Rows, weights and bias are drawn, so that what is found hangs on sizes and settings alone and not on a model that is all
+    zeros or has a NaN.  Two orders differ in few outputs (4096 x 4096: one of 4000 to 6000), in proportion to the root of the products
+    summed up: enough rows are tried to expect eight differences of a wrong one, twice as many while two are left, and if two are left
+    then there is none.  Products so small that this would take more than 64 rows stay with torch.  Four rows: the norm of five costs the
+    products behind it more than torch takes (6144 x 4096 with the norm, us, torch's operations and the kernel, by rows  1: 19.6 10.9
+    3: 19.5 18.1  4: 19.6 20.6  5: 19.5 23.0; the four products of that layer  1: 136 84  4: 131 98), and 4 x 14336 is all that fits."""
+    if weight.device.type != "cuda" or weight.dtype not in ROW_TYPES or not weight.is_contiguous() or _tuning():
         return {}
     n, k = weight.shape
     enough = math.ceil(3.5e6 / (n * math.sqrt(k)))
     if enough > 64:
         return {}
-    key = (weight.device, weight.dtype, n, k, bias is not None, most_rows)
+    key = (weight.device, weight.dtype, n, k, bias is not None, most_rows, product_settings())
     if key in _FOUND:
         return _FOUND[key]
     if torch.cuda.is_current_stream_capturing():
         return {}
     orders = {}
-    gen = torch.Generator(device=weight.device).manual_seed(n + k)
-    with torch.no_grad():
+    like = dict(generator=torch.Generator(device=weight.device).manual_seed(n + k), device=weight.device, dtype=weight.dtype)
+    with torch.no_grad(), torch.autocast("cuda", enabled=False):
+        w, b = torch.randn(n, k, **like), None if bias is None else torch.randn(n, **like)
         for rows in range(1, most_rows + 1):
-            left, tried = [o for o in ORDERS if _fits(rows, n, k, o, False)], 0
+            left = {_chains(o, k): o for o in reversed(ORDERS) if _fits(rows, n, k, o, False)}
+            left, tried = list(left.values()), 0
             while left and (tried < enough or (len(left) > 1 and tried < 2 * enough)):
-                x = torch.randn(rows, 1, k, generator=gen, device=weight.device).to(weight.dtype)
-                want = nn.functional.linear(x, weight, bias)
-                left = [o for o in left if torch.equal(linear_rows(x, weight, o, bias), want)]
+                x = torch.randn(rows, 1, k, **like)
+                want = nn.functional.linear(x, w, b)
+                left = [o for o in left if torch.equal(linear_rows(x, w, o, b), want)]
                 tried += rows
-            if left:
+            if len(left) == 1:
                 orders[rows] = left[0]
     _FOUND[key] = orders
     return orders

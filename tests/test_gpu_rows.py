@@ -76,6 +76,47 @@ def test_one_row_of_a_wider_buffer(extra):
         assert torch.equal(got, rp.linear_rows(x.contiguous(), w, (1, 1)) if one or extra % 8 == 0 else F.linear(x, w))
 
 
+def agrees_with_torch(orders, n, k, dtype=torch.bfloat16):
+    w = torch.randn(n, k, device="cuda").to(dtype)
+    return all(torch.equal(rp.linear_rows(x, w, order), F.linear(x, w))
+               for rows, order in orders.items() for x in torch.randn(20, rows, 1, k, device="cuda").to(dtype))
+
+
+@pytest.mark.parametrize("spoil", ["zeros", "nan", "large bias", "autocast"])
+def test_orders_do_not_hang_on_the_weight_that_asks_first(spoil, monkeypatch):
+    n = k = 4096
+    w, b = torch.randn(n, k, device="cuda").bfloat16(), torch.zeros(n, device="cuda").bfloat16()
+    want = rp.library_orders(w), rp.library_orders(w, b)
+    assert want[0] and agrees_with_torch(want[0], n, k)
+    monkeypatch.setattr(rp, "_FOUND", {})
+    if spoil == "zeros":
+        w = torch.zeros_like(w)
+    if spoil == "nan":
+        w[5, 7] = float("nan")
+    if spoil == "large bias":
+        b = b + 1e6
+    with torch.autocast("cuda", torch.float16, enabled=spoil == "autocast"):
+        assert (rp.library_orders(w), rp.library_orders(w, b)) == want
+
+
+def test_orders_are_asked_again_when_torch_is_told_to_take_another_product():
+    n, k = 6144, 4096
+    w = torch.randn(n, k, device="cuda").bfloat16()
+    assert agrees_with_torch(rp.library_orders(w), n, k)
+    blas, flags, seen = torch.backends.cuda.preferred_blas_library, torch.backends.cuda.matmul, {rp.product_settings()}
+    was = blas(), flags.allow_bf16_reduced_precision_reduction
+    try:
+        for library, reduced in (("cublas", True), ("cublas", False), ("cublaslt", False)):
+            blas(library)
+            flags.allow_bf16_reduced_precision_reduction = reduced
+            seen.add(rp.product_settings())
+            assert agrees_with_torch(rp.library_orders(w), n, k), (library, reduced)
+    finally:
+        blas(was[0])
+        flags.allow_bf16_reduced_precision_reduction = was[1]
+    assert len(seen) == 4 and rp.product_settings() in seen
+
+
 @pytest.mark.parametrize("preset", ["llama3.1-8b", "qwen2-7b", "tiny"])
 def test_steps_of_a_fused_decoder_have_the_bits_of_torchs_products(preset):
     """One layer's steps by row products where an order is torch's, and by torch's operations: the same bits in the cache, and logits that

@@ -49,3 +49,11 @@ def test_a_layer_saved_without_orders_keeps_torchs_operations():
     layer = DecoderLayer(PRESETS["tiny"], 0, torch.float32, "cpu")
     vars(layer).pop("_orders", None)   # as an object pickled before there were any
     assert layer._as_rows(torch.zeros(1, 1, 256), None) is False
+
+
+@pytest.mark.parametrize("k,same", [(64, 1), (128, 2), (192, 3), (256, 3), (512, 4), (4096, 4)])
+def test_orders_that_are_one_for_short_rows(k, same):
+    chains = {order: rp._chains(order, k) for order in rp.ORDERS}
+    assert len(set(chains.values())) == same
+    for found in chains.values():
+        assert sorted(s for c in found for s in c) == list(range(k // 64))
