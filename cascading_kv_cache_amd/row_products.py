@@ -163,7 +163,8 @@ def library_orders(weight, bias=None, most_rows=4):
     then there is none.  Products so small that this would take more than 64 rows stay with torch.  Four rows: the norm of five costs the
     products behind it more than torch takes (6144 x 4096 with the norm, us, torch's operations and the kernel, by rows  1: 19.6 10.9
     3: 19.5 18.1  4: 19.6 20.6  5: 19.5 23.0; the four products of that layer  1: 136 84  4: 131 98), and 4 x 14336 is all that fits."""
-    if weight.device.type != "cuda" or weight.dtype not in ROW_TYPES or not weight.is_contiguous() or _tuning():
+    if (type(weight) not in (torch.Tensor, nn.Parameter) or _dispatch_modes() != 0 or _functorch_levels() is not None
+            or weight.device.type != "cuda" or weight.dtype not in ROW_TYPES or not weight.is_contiguous() or _tuning()):
         return {}
     n, k = weight.shape
     enough = math.ceil(3.5e6 / (n * math.sqrt(k)))

@@ -57,3 +57,11 @@ def test_orders_that_are_one_for_short_rows(k, same):
     assert len(set(chains.values())) == same
     for found in chains.values():
         assert sorted(s for c in found for s in c) == list(range(k // 64))
+
+
+def test_nothing_is_tried_on_tensors_without_memory():
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    with FakeTensorMode(allow_non_fake_inputs=True):
+        weight = torch.empty(4096, 4096, dtype=torch.bfloat16, device="cuda")
+        assert rp.library_orders(weight) == {}
