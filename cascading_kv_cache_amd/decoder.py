@@ -160,8 +160,10 @@ class CascadeDecoder(nn.Module):
         self.norm.fused = True
         for layer in self.layers:
             attn, mlp = layer.self_attn, layer.mlp
-            layer._orders = dict(qkv=library_orders(attn._w_qkv, attn._b_qkv), o=library_orders(attn.o_proj.weight),
-                                 gate_up=library_orders(mlp._w_gate_up), down=library_orders(mlp.down_proj.weight))
+            layer._orders = dict(qkv=library_orders(attn._w_qkv, attn._b_qkv, norm=layer.input_layernorm),
+                                 o=library_orders(attn.o_proj.weight),
+                                 gate_up=library_orders(mlp._w_gate_up, norm=layer.post_attention_layernorm),
+                                 down=library_orders(mlp.down_proj.weight))
             layer._orders["any"] = set().union(*layer._orders.values())
         return self
 

@@ -144,7 +144,7 @@ def product_settings() -> tuple:
     return (torch.__version__, *[f() for f in _SETTINGS])
 
 
-#: what library_orders has found, by device, type, sizes and settings: facts about torch's products, not about a weight
+#: what library_orders has found, by device, type, sizes and settings: facts about torch's products and norms, not about a weight
 _FOUND = {}
 
 
@@ -155,9 +155,32 @@ def _chains(order, k) -> tuple:
     return tuple(c for c in chains if c)
 
 
-def library_orders(weight, bias=None, most_rows=4):
-    """``{rows: order}`` whose bits are those of ``torch.nn.functional.linear`` for so many rows of 16 bits, found by trying, 2 ms a
-    size, once.  Rows, weights and bias are drawn, so that what is found hangs on sizes and settings alone and not on a model that is all
+_FRACTION = {torch.bfloat16: 8, torch.float16: 11}   # bits of a value, the leading one included
+
+
+def _norms_like_torch(k, eps, most_rows, like) -> set:
+    """Numbers of rows whose norm in front of a product has the bits of torch's, looked at through a product with the identity.  Another
+    order of the sum of squares moves half the rows' factors by the last bit of a float32, which rounds one element of 65536 of bfloat16
+    (8192 of float16) to another value: enough rows are tried to expect eight."""
+    key = ("norm", like["device"], like["dtype"], k, eps, most_rows, product_settings())
+    if key in _FOUND:
+        return _FOUND[key]
+    left = {rows for rows in range(1, most_rows + 1) if _fits(rows, k, k, (1, 1), True)}
+    enough = math.ceil(8 * 2 ** (25 - _FRACTION[like["dtype"]]) / k)
+    same, w = torch.eye(k, device=like["device"], dtype=like["dtype"]), 1 + 0.1 * torch.randn(k, **like)
+    for rows in sorted(left):
+        differ = torch.zeros((), dtype=torch.int64, device=like["device"])
+        for x in torch.randn(math.ceil(enough / rows), rows, 1, k, **like):
+            differ += (linear_rows(x, same, (1, 1), norm=w, eps=eps) != nn.functional.rms_norm(x, (k,), w, eps)).sum()
+        if differ.item():
+            left.remove(rows)
+    _FOUND[key] = left
+    return left
+
+
+def library_orders(weight, bias=None, most_rows=4, norm=None):
+    """``{rows: order}`` whose bits are those of ``torch.nn.functional.linear`` for so many rows of 16 bits, with a fused RMSNorm module
+    in front or none, found by trying, some ms a size, once.  Rows, weights and bias are drawn, so that what is found hangs on sizes and settings alone and not on a model that is all
     zeros or has a NaN.  Two orders differ in few outputs (4096 x 4096: one of 4000 to 6000), in proportion to the root of the products
     summed up: enough rows are tried to expect eight differences of a wrong one, twice as many while two are left, and if two are left
     then there is none.  Products so small that this would take more than 64 rows stay with torch.  Four rows: the norm of five costs the
@@ -170,7 +193,7 @@ def library_orders(weight, bias=None, most_rows=4):
     enough = math.ceil(3.5e6 / (n * math.sqrt(k)))
     if enough > 64:
         return {}
-    key = (weight.device, weight.dtype, n, k, bias is not None, most_rows, product_settings())
+    key = (weight.device, weight.dtype, n, k, bias is not None, most_rows, None if norm is None else norm.eps, product_settings())
     if key in _FOUND:
         return _FOUND[key]
     if torch.cuda.is_current_stream_capturing():
@@ -179,8 +202,8 @@ def library_orders(weight, bias=None, most_rows=4):
     like = dict(generator=torch.Generator(device=weight.device).manual_seed(n + k), device=weight.device, dtype=weight.dtype)
     with torch.no_grad(), torch.autocast("cuda", enabled=False):
         w, b = torch.randn(n, k, **like), None if bias is None else torch.randn(n, **like)
-        for rows in range(1, most_rows + 1):
-            left = {_chains(o, k): o for o in reversed(ORDERS) if _fits(rows, n, k, o, False)}
+        for rows in range(1, most_rows + 1) if norm is None else _norms_like_torch(k, norm.eps, most_rows, like):
+            left = {_chains(o, k): o for o in reversed(ORDERS) if _fits(rows, n, k, o, norm is not None)}
             left, tried = list(left.values()), 0
             while left and (tried < enough or (len(left) > 1 and tried < 2 * enough)):
                 x = torch.randn(rows, 1, k, **like)

@@ -117,6 +117,24 @@ def test_orders_are_asked_again_when_torch_is_told_to_take_another_product():
     assert len(seen) == 4 and rp.product_settings() in seen
 
 
+@pytest.mark.parametrize("n,k,dtype", [(6144, 4096, torch.bfloat16), (4608, 3584, torch.bfloat16), (6144, 4096, torch.float16)])
+def test_a_norm_in_front_is_tried_too(n, k, dtype, monkeypatch):
+    """Torch's norm with its squares added up in another order: no row count is left."""
+    class Norm:
+        eps = 1e-5
+
+    w = torch.randn(n, k, device="cuda").to(dtype)
+    assert rp.library_orders(w, norm=Norm) == rp.library_orders(w) != {}
+
+    def other(x, shape, weight, eps):
+        factor = torch.rsqrt(x.float().pow(2).flip(-1).cumsum(-1)[..., -1:] / x.size(-1) + eps)
+        return (weight.float() * (factor * x.float())).to(x.dtype)
+
+    monkeypatch.setattr(rp, "_FOUND", {})
+    monkeypatch.setattr(F, "rms_norm", other)
+    assert rp.library_orders(w, norm=Norm) == {} != rp.library_orders(w)
+
+
 @pytest.mark.parametrize("preset", ["llama3.1-8b", "qwen2-7b", "tiny"])
 def test_steps_of_a_fused_decoder_have_the_bits_of_torchs_products(preset):
     """One layer's steps by row products where an order is torch's, and by torch's operations: the same bits in the cache, and logits that
