@@ -20,7 +20,7 @@ from torch import nn
 
 from .cascading_cache import CascadingKVCache
 from .latency import ProjectedCascadeAttention
-from .row_products import FAST_ORDER, MAX_ROWS, ROW_TYPES, followed as _followed, gated_silu, library_orders, own_methods, plain, row_linear
+from .row_products import FAST_ORDER, MAX_ROWS, ROW_TYPES, followed as _followed, gated_silu, library_orders, own_methods, plain, product_settings, row_linear
 
 
 @dataclass
@@ -108,7 +108,7 @@ class DecoderLayer(nn.Module):
         """Are these few rows whose operations nobody follows, and is every module its own?"""
         attn, mlp = self.self_attn, self.mlp
         return (self._orders is not None and x.dim() == 3 and x.size(0) * x.size(1) in self._orders["any"] and x.is_cuda and not _followed(x)
-                and not torch.is_autocast_enabled() and isinstance(cache, CascadingKVCache)
+                and not torch.is_autocast_enabled() and self._orders.get("settings") == product_settings() and isinstance(cache, CascadingKVCache)
                 and plain(attn, ProjectedCascadeAttention) and plain(mlp, GatedMLP)
                 and attn._w_qkv is not None and mlp._w_gate_up is not None
                 and plain(attn.o_proj, nn.Linear) and plain(mlp.down_proj, nn.Linear)
@@ -151,8 +151,9 @@ class CascadeDecoder(nn.Module):
 
     def fuse_projections(self):
         """Fewer, larger launches outside attention (same weights, kept in shared buffers): q/k/v and gate/up
-        projections as one matrix product each, the norms as one kernel.  Off by default: the parity tests compare
-        the plain formulation with the CPU's."""
+        projections as one matrix product each, the norms as one kernel, the products of few rows by the library where they have
+        the bits of torch's (which holds for torch's settings as they are now: under others its products are taken).  Off by
+        default: the parity tests compare the plain formulation with the CPU's."""
         for layer in self.layers:
             layer.self_attn.fuse_projections()
             layer.mlp.fuse_projections()
@@ -165,6 +166,7 @@ class CascadeDecoder(nn.Module):
                                  gate_up=library_orders(mlp._w_gate_up, norm=layer.post_attention_layernorm),
                                  down=library_orders(mlp.down_proj.weight))
             layer._orders["any"] = set().union(*layer._orders.values())
+            layer._orders["settings"] = product_settings() if layer._orders["any"] else None
         return self
 
     def new_cache(self, window, cascades, batch=1, num_sink_tokens=64, **kw):

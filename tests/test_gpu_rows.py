@@ -135,6 +135,23 @@ def test_a_norm_in_front_is_tried_too(n, k, dtype, monkeypatch):
     assert rp.library_orders(w, norm=Norm) == {} != rp.library_orders(w)
 
 
+def test_other_settings_than_a_layer_was_fused_under_keep_torchs_products():
+    from cascading_kv_cache_amd.decoder import PRESETS, CascadeDecoder
+
+    model = CascadeDecoder(replace(PRESETS["llama3.1-8b"], num_layers=1, vocab_size=512), init_on_device=True).fuse_projections()
+    layer, cache, x = model.layers[0], model.new_cache(256, 2, num_sink_tokens=4), torch.randn(1, 1, 4096, device="cuda").bfloat16()
+    flags = torch.backends.cuda.matmul
+    was = flags.allow_bf16_reduced_precision_reduction
+    with torch.no_grad():
+        assert layer._as_rows(x, cache)
+        try:
+            flags.allow_bf16_reduced_precision_reduction = not was
+            assert not layer._as_rows(x, cache)
+        finally:
+            flags.allow_bf16_reduced_precision_reduction = was
+        assert layer._as_rows(x, cache)
+
+
 @pytest.mark.parametrize("preset", ["llama3.1-8b", "qwen2-7b", "tiny"])
 def test_steps_of_a_fused_decoder_have_the_bits_of_torchs_products(preset):
     """One layer's steps by row products where an order is torch's, and by torch's operations: the same bits in the cache, and logits that
