@@ -180,18 +180,22 @@ def _norms_like_torch(k, eps, most_rows, like) -> set:
 
 def library_orders(weight, bias=None, most_rows=4, norm=None):
     """``{rows: order}`` whose bits are those of ``torch.nn.functional.linear`` for so many rows of 16 bits, with a fused RMSNorm module
-    in front or none, found by trying, some ms a size, once.  Rows, weights and bias are drawn, so that what is found hangs on sizes and settings alone and not on a model that is all
-    zeros or has a NaN.  Two orders differ in few outputs (4096 x 4096: one of 4000 to 6000), in proportion to the root of the products
-    summed up: enough rows are tried to expect eight differences of a wrong one, twice as many while two are left, and if two are left
-    then there is none.  Products so small that this would take more than 64 rows stay with torch.  Four rows: the norm of five costs the
-    products behind it more than torch takes (6144 x 4096 with the norm, us, torch's operations and the kernel, by rows  1: 19.6 10.9
-    3: 19.5 18.1  4: 19.6 20.6  5: 19.5 23.0; the four products of that layer  1: 136 84  4: 131 98), and 4 x 14336 is all that fits."""
+    in front or none, found by trying, some 10 ms a size, once.
+
+    Rows, weights and bias are drawn, so that what is found hangs on sizes and settings alone and not on a model that is all zeros or has
+    a NaN.  Two orders differ in few outputs (4096 x 4096: one of 4000 to 6000), in proportion to the root of the products summed up.  A
+    library whose tiles do not come out even on its workgroups cuts the last ones up, and such an order differs from the others' in an
+    output or two a row (152064 x 3584).  So 64 rows are tried, which also expects eight differences of the smallest product that is
+    taken, twice as many while two are left, and if two are left then there is none.
+
+    Four rows: the norm of five costs the products behind it more than torch takes (6144 x 4096 with the norm, us, torch's operations and
+    the kernel, by rows  1: 19.6 10.9  3: 19.5 18.1  4: 19.6 20.6  5: 19.5 23.0; the four products of that layer  1: 136 84  4: 131 98),
+    and 4 x 14336 is all that fits."""
     if (type(weight) not in (torch.Tensor, nn.Parameter) or _dispatch_modes() != 0 or _functorch_levels() is not None
             or weight.device.type != "cuda" or weight.dtype not in ROW_TYPES or not weight.is_contiguous() or _tuning()):
         return {}
     n, k = weight.shape
-    enough = math.ceil(3.5e6 / (n * math.sqrt(k)))
-    if enough > 64:
+    if 3.5e6 / (n * math.sqrt(k)) > 64:   # rows that eight differences take
         return {}
     key = (weight.device, weight.dtype, n, k, bias is not None, most_rows, None if norm is None else norm.eps, product_settings())
     if key in _FOUND:
@@ -202,10 +206,10 @@ def library_orders(weight, bias=None, most_rows=4, norm=None):
     like = dict(generator=torch.Generator(device=weight.device).manual_seed(n + k), device=weight.device, dtype=weight.dtype)
     with torch.no_grad(), torch.autocast("cuda", enabled=False):
         w, b = torch.randn(n, k, **like), None if bias is None else torch.randn(n, **like)
-        for rows in range(1, most_rows + 1) if norm is None else _norms_like_torch(k, norm.eps, most_rows, like):
+        for rows in range(1, most_rows + 1) if norm is None else sorted(_norms_like_torch(k, norm.eps, most_rows, like)):
             left = {_chains(o, k): o for o in reversed(ORDERS) if _fits(rows, n, k, o, norm is not None)}
             left, tried = list(left.values()), 0
-            while left and (tried < enough or (len(left) > 1 and tried < 2 * enough)):
+            while left and (tried < 64 or (len(left) > 1 and tried < 128)):
                 x = torch.randn(rows, 1, k, **like)
                 want = nn.functional.linear(x, w, b)
                 left = [o for o in left if torch.equal(linear_rows(x, w, o, b), want)]
