@@ -16,8 +16,11 @@
 // The order of a sum is the caller's (kParts, kUnit): part p takes the stretches of kUnit * 64 elements p, p + kParts, ..., one chain
 // of matrix instructions each, and the parts are added up in order.  Another order is as good, but flips the rounding of a few
 // outputs in ten thousand, which a decoder of random weights turns into a percent of its logits; so a decoder that has used a library's
-// products before keeps their order (row_products.py finds it).
+// products before keeps their order (row_products.py finds it).  Where the library cuts the sums of some tiles, so does kCut: heads of
+// 128256 x 4096 and 152064 x 3584, norm, a row, 150.5 and 156 us with it, 150.7 and 154 without (torch's operations 190 and 226).
 #include "ckv_common.h"
+
+#include <algorithm>
 
 namespace ckv {
 namespace {
@@ -36,11 +39,14 @@ struct RowsParams {
     float eps;
     int rows, N, K;
     int64_t x_stride;
+    // kCut: tiles of cut_groups groups from tile cut_first on are cut, see cut_of
+    int cut_groups, cut_first, cut_span, cut_length;
 };
 
 constexpr int kChunk = 64;             // elements of a stage
 constexpr int kStageBytes = 2048;      // of 16 rows
 constexpr int kMaxRows = 16;
+constexpr int kMaxRuns = 1024;
 
 template <typename T>
 __device__ inline f32x4 rows_mma(uint4 a, uint4 b, f32x4 c) {
@@ -51,6 +57,16 @@ __device__ inline f32x4 rows_mma(uint4 a, uint4 b, f32x4 c) {
 }
 
 __host__ __device__ inline int rows_pitch(int K) { return 2 * K + 16; }   // bytes between the rows of x in LDS; the pad spreads the banks
+
+// A library that deals its tiles out over a fixed number of workgroups lays the last ones, which do not come out even, end to end and
+// cuts the line of their cut_span stretches into runs of cut_length: a sum whose tile holds the end of a run is two sums, added up.
+// Returns how many stretches of `group` lie before that end, 0 for none.  A run is no shorter than a tile, so there is one end at most.
+__device__ inline int cut_of(const RowsParams& p, int group) {
+    const int tile = group / p.cut_groups - p.cut_first;
+    if (tile < 0) return 0;
+    const int from = tile * p.cut_span, end = (from + p.cut_length - 1) / p.cut_length * p.cut_length;
+    return end < from + p.cut_span ? end - from : 0;
+}
 
 // wavefronts of a workgroup, at most: with one part any number, else one per part
 template <int kParts>
@@ -96,7 +112,7 @@ __device__ inline void rows_norm(unsigned char* xs, const unsigned char* weights
     __syncthreads();
 }
 
-template <typename T, int kParts, int kUnit, bool kGated, int kStages>
+template <typename T, int kParts, int kUnit, bool kGated, bool kCut, int kStages>
 __global__ void __launch_bounds__(64 * kMostWaves<kParts>) rows_kernel(RowsParams p) {
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ float norm_part[kMaxRows][4];
@@ -162,7 +178,15 @@ __global__ void __launch_bounds__(64 * kMostWaves<kParts>) rows_kernel(RowsParam
     const unsigned char* a_at = ring + (r >> 3) * 1024 + (r & 7) * 128;
     const unsigned char* b_at = xs + (r < p.rows ? r : 0) * pitch + q * 16;   // columns that stand for no row repeat the first
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    [[maybe_unused]] f32x4 before = {0.f, 0.f, 0.f, 0.f};   // the sum up to the cut
+    const int cut = kCut ? kUnit * cut_of(p, group) : 0;
     auto step = [&](int i, int slot) {
+        if constexpr (kCut) {
+            if (i == cut) {   // not cut: nothing is in it yet
+                before = acc;
+                acc = f32x4{0.f, 0.f, 0.f, 0.f};
+            }
+        }
         const unsigned char* b = b_at + chunk_of(i) * (2 * kChunk);
         const uint4 a0 = *reinterpret_cast<const uint4*>(a_at + slot * kStageBytes + ((q ^ flip) << 4));
         const uint4 a1 = *reinterpret_cast<const uint4*>(a_at + slot * kStageBytes + (((q + 4) ^ flip) << 4));
@@ -187,14 +211,21 @@ __global__ void __launch_bounds__(64 * kMostWaves<kParts>) rows_kernel(RowsParam
     if constexpr (kParts > 1) {   // the parts in order
         float4* mine = reinterpret_cast<float4*>(ring);
         mine[lane] = make_float4(acc[0], acc[1], acc[2], acc[3]);
+        if constexpr (kCut) mine[CKV_WAVE + lane] = make_float4(before[0], before[1], before[2], before[3]);
         __syncthreads();
         if (part != 0) return;
 #pragma unroll
         for (int w = 1; w < kParts; w++) {
-            const float4 o = reinterpret_cast<const float4*>(ring + w * (kStages * kStageBytes))[lane];
+            const float4* others = reinterpret_cast<const float4*>(ring + w * (kStages * kStageBytes));
+            const float4 o = others[lane];
             acc[0] += o.x; acc[1] += o.y; acc[2] += o.z; acc[3] += o.w;
+            if constexpr (kCut) {
+                const float4 b = others[CKV_WAVE + lane];
+                before[0] += b.x; before[1] += b.y; before[2] += b.z; before[3] += b.w;
+            }
         }
     }
+    if constexpr (kCut) acc += before;
     // lane: row r of x, outputs 4 q + 0..3 of the group
     struct alignas(8) Out {
         T v[4];
@@ -226,9 +257,9 @@ __global__ void __launch_bounds__(64 * kMostWaves<kParts>) rows_kernel(RowsParam
     }
 }
 
-template <typename T, int kParts, int kUnit, bool kGated, int kStages>
+template <typename T, int kParts, int kUnit, bool kGated, bool kCut, int kStages>
 int launch_rows(const RowsParams& p, int waves, int lds, hipStream_t stream) {
-    auto kernel = rows_kernel<T, kParts, kUnit, kGated, kStages>;
+    auto kernel = rows_kernel<T, kParts, kUnit, kGated, kCut, kStages>;
     if (int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(kernel), lds)) return rc;
     const int groups = p.N / 16, per = waves / kParts;
     hipLaunchKernelGGL(kernel, dim3((unsigned)((groups + per - 1) / per)), dim3(64 * waves), lds, stream, p);
@@ -243,7 +274,7 @@ int launch_rows(const RowsParams& p, int waves, int lds, hipStream_t stream) {
 // stages (39.4 -> 38.5, in turn with the others 45 -> 42.0; 10 stages are level).  Two parts: the longer ring where two
 // workgroups still fit (6144 x 4096, norm, a row: 11.6 with 12 stages, 11.9 with 8; four rows, one workgroup on a unit or two: 29.8, 18.0).
 // Four parts: the shorter ring where the longer does not fit.
-template <typename T, int kParts, int kUnit, bool kGated>
+template <typename T, int kParts, int kUnit, bool kGated, bool kCut>
 int run_rows(const RowsParams& p, hipStream_t stream) {
     DeviceInfo di;
     if (int rc = current_device_info(&di)) return rc;
@@ -262,17 +293,33 @@ int run_rows(const RowsParams& p, hipStream_t stream) {
         while (waves > 1 && !fits(lds(waves, kShort))) waves--;   // long rows
     }
     if (!longer && !fits(lds(waves, kShort))) return CKV_ERR_UNSUPPORTED;
-    return longer ? launch_rows<T, kParts, kUnit, kGated, kLong>(p, waves, lds(waves, kLong), stream)
-                  : launch_rows<T, kParts, kUnit, kGated, kShort>(p, waves, lds(waves, kShort), stream);
+    return longer ? launch_rows<T, kParts, kUnit, kGated, kCut, kLong>(p, waves, lds(waves, kLong), stream)
+                  : launch_rows<T, kParts, kUnit, kGated, kCut, kShort>(p, waves, lds(waves, kShort), stream);
+}
+
+// Fills in how sums are cut whose tiles are dealt out over `runs` workgroups: as many whole tiles as come out even, less one round, go
+// first.  Tiles are of 256 rows and 64 elements, or (four parts) of 32 rows and 256 elements.
+inline void cut_into_runs(RowsParams& p, int parts, int runs) {
+    p.cut_groups = parts == 1 ? 16 : 2;
+    p.cut_span = p.K / (kChunk * parts);
+    const int tiles = (p.N / 16 + p.cut_groups - 1) / p.cut_groups, shared = tiles % runs ? tiles % runs + runs : 0;
+    p.cut_first = tiles - shared;   // negative: fewer tiles than runs
+    p.cut_length = std::max(1, (shared * p.cut_span + runs - 1) / runs);
 }
 
 template <typename T>
-int run_rows(const RowsParams& p, bool gated, int parts, int unit, hipStream_t stream) {
-    if (parts == 1) return gated ? run_rows<T, 1, 1, true>(p, stream) : run_rows<T, 1, 1, false>(p, stream);
+int run_rows(RowsParams p, bool gated, int parts, int unit, int runs, hipStream_t stream) {
+    if (runs) {
+        if (gated || unit != 1 || (parts != 1 && parts != 4) || p.K % (kChunk * parts)) return CKV_ERR_UNSUPPORTED;
+        cut_into_runs(p, parts, runs);
+        if (p.cut_first < 0) return CKV_ERR_UNSUPPORTED;
+        return parts == 1 ? run_rows<T, 1, 1, false, true>(p, stream) : run_rows<T, 4, 1, false, true>(p, stream);
+    }
+    if (parts == 1) return gated ? run_rows<T, 1, 1, true, false>(p, stream) : run_rows<T, 1, 1, false, false>(p, stream);
     if (gated) return CKV_ERR_UNSUPPORTED;
-    if (parts == 2 && unit == 2) return run_rows<T, 2, 2, false>(p, stream);
-    if (parts == 4 && unit == 1) return run_rows<T, 4, 1, false>(p, stream);
-    if (parts == 4 && unit == 2) return run_rows<T, 4, 2, false>(p, stream);
+    if (parts == 2 && unit == 2) return run_rows<T, 2, 2, false, false>(p, stream);
+    if (parts == 4 && unit == 1) return run_rows<T, 4, 1, false, false>(p, stream);
+    if (parts == 4 && unit == 2) return run_rows<T, 4, 2, false, false>(p, stream);
     return CKV_ERR_UNSUPPORTED;
 }
 
@@ -287,6 +334,8 @@ extern "C" int ckv_linear_rows(const void* x, const void* w, const void* bias, c
     if (dtype != CKV_F16 && dtype != CKV_BF16) return CKV_ERR_DTYPE;
     if (rows == 0) return CKV_OK;
     if (!x || !w || !out) return CKV_ERR_NULL;
+    const int runs = unit >= 256 ? unit >> 8 : 0;
+    if (runs > kMaxRuns) return CKV_ERR_UNSUPPORTED;
     if (rows > kMaxRows || n % 16 || k % kChunk || n > 0x7fffffff || k > (1 << 20) || (gated && (bias || residual))) return CKV_ERR_UNSUPPORTED;
     // copies and operands are pieces of 16 bytes, outputs of 8
     if (((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(norm)) & 15) || x_stride % 8 ||
@@ -297,6 +346,8 @@ extern "C" int ckv_linear_rows(const void* x, const void* w, const void* bias, c
     p.eps = eps;
     p.rows = (int)rows; p.N = (int)n; p.K = (int)k;
     p.x_stride = x_stride;
+    p.cut_groups = 1; p.cut_first = 0; p.cut_span = 0; p.cut_length = 1;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    return dtype == CKV_F16 ? run_rows<__half>(p, gated != 0, parts, unit, s) : run_rows<__hip_bfloat16>(p, gated != 0, parts, unit, s);
+    if (runs) unit &= 255;
+    return dtype == CKV_F16 ? run_rows<__half>(p, gated != 0, parts, unit, runs, s) : run_rows<__hip_bfloat16>(p, gated != 0, parts, unit, runs, s);
 }

@@ -20,7 +20,7 @@ from torch import nn
 
 from .cascading_cache import CascadingKVCache
 from .latency import ProjectedCascadeAttention
-from .row_products import FAST_ORDER, MAX_ROWS, ROW_TYPES, followed as _followed, gated_silu, library_orders, own_methods, plain, product_settings, row_linear
+from .row_products import followed as _followed, gated_silu, library_orders, own_methods, plain, product_settings, row_linear
 
 
 @dataclass
@@ -129,6 +129,7 @@ class DecoderLayer(nn.Module):
 
 class CascadeDecoder(nn.Module):
     """Decoder-only model whose every layer attends through one :class:`CascadingKVCache`."""
+    _head_orders = None   # of the head's products of few rows, see fuse_projections; saved models may have none
 
     def __init__(self, cfg: DecoderConfig, dtype=torch.bfloat16, device="cuda:0", seed=0, init_on_device=False):
         """Weights are N(0, 0.02) from ``seed``: drawn on the CPU (the same bits whatever the device, what the parity
@@ -167,6 +168,9 @@ class CascadeDecoder(nn.Module):
                                  down=library_orders(mlp.down_proj.weight))
             layer._orders["any"] = set().union(*layer._orders.values())
             layer._orders["settings"] = product_settings() if layer._orders["any"] else None
+        head = self.lm_head
+        orders = library_orders(head.weight, head.bias, norm=self.norm, cut=True)
+        self._head_orders = dict(orders, settings=product_settings() if orders else None)
         return self
 
     def new_cache(self, window, cascades, batch=1, num_sink_tokens=64, **kw):
@@ -189,9 +193,10 @@ class CascadeDecoder(nn.Module):
             x = layer(x, cache)
         if last_only:
             x = x[:, -1:]
-        if (self.norm.fused and x.is_cuda and 0 < x.size(0) * x.size(1) <= MAX_ROWS and not _followed(x) and not torch.is_autocast_enabled()
-                and plain(self.norm, RMSNorm) and plain(self.lm_head, nn.Linear) and x.dtype in ROW_TYPES):
-            return row_linear(x, self.lm_head.weight, {x.size(0) * x.size(1): FAST_ORDER}, bias=self.lm_head.bias, norm=self.norm)
+        orders = self._head_orders
+        if (orders is not None and x.size(0) * x.size(1) in orders and x.is_cuda and not _followed(x) and not torch.is_autocast_enabled()
+                and orders["settings"] == product_settings() and self.norm.fused and plain(self.norm, RMSNorm) and plain(self.lm_head, nn.Linear)):
+            return row_linear(x, self.lm_head.weight, orders, bias=self.lm_head.bias, norm=self.norm)
         return self.lm_head(self.norm(x))
 
 

@@ -16,10 +16,8 @@ from .cascading_cache import on_device, raw_stream
 
 ROW_TYPES = (torch.bfloat16, torch.float16)
 _GATED_TYPES = (torch.bfloat16, torch.float16, torch.float32)
-#: (parts, unit) of ``ckv_linear_rows``
+#: (parts, unit) of ``ckv_linear_rows``, or (parts, unit, runs): see :func:`_cut_orders`
 ORDERS = ((1, 1), (4, 1), (4, 2), (2, 2))
-#: of a product whose roundings nothing is computed from (the head of a decoder): the fastest, 128256 x 4096 in bf16 158 us, (1, 1) 176
-FAST_ORDER = (4, 1)
 MAX_ROWS = 16
 # not public: where torch lacks one of them, somebody may be following
 _function_modes = getattr(torch._C, "_len_torch_function_stack", lambda: 1)
@@ -84,6 +82,14 @@ def _fits(rows, n, k, order, norm) -> bool:
     return 0 < rows <= MAX_ROWS and n % 16 == 0 and k % 64 == 0 and ring + rows * (2 * k + 16) + 2 * k * norm + 256 <= 160 * 1024
 
 
+def _crowded(rows, n, k, order, units) -> bool:
+    """Is a product with the norm in front slower than torch's because one workgroup, of 16 outputs, fills a compute unit's LDS?  Each of
+    them brings and normalises the rows again, which nothing covers then, round after round.  us, torch's operations and the kernel, four
+    parts:  152064 x 3584, by rows  2: 226 163  3: 226 175  4: 227 323   100352 x 4096  2: 182 123  3: 182 197; with few rounds it is
+    level (6144 x 4096  3: 19.5 18.1  4: 19.6 20.6), and one part has more outputs a workgroup (128256 x 4096  4: 190 161)."""
+    return order[0] == 4 and n // 16 > 4 * units and 2 * (6 * 4 * 2048 + rows * (2 * k + 16) + 2 * k + 256) > 160 * 1024
+
+
 def _at(t) -> int:
     return 0 if t is None else t.data_ptr()
 
@@ -96,7 +102,7 @@ def linear_rows(x, weight, order, bias=None, residual=None, norm=None, eps=0.0, 
     stride = k if rows == 1 else x.stride(0) if x.size(1) == 1 else x.stride(1)
     with on_device(x.device):
         _abi.check(_abi.lib().ckv_linear_rows(x.data_ptr(), weight.data_ptr(), _at(bias), _at(residual), _at(norm), eps, out.data_ptr(),
-                                              rows, n, k, stride, int(gated), order[0], order[1],
+                                              rows, n, k, stride, int(gated), order[0], order[1] + 256 * sum(order[2:]),
                                               _abi.dtype_code(x.dtype), raw_stream(x.device)), "ckv_linear_rows")
     return out
 
@@ -155,6 +161,20 @@ def _chains(order, k) -> tuple:
     return tuple(c for c in chains if c)
 
 
+def _cut_orders(n, k, units) -> list:
+    """Orders of a library that lays the tiles which do not come out even on its workgroups (of 256 rows of the weight and 64 elements, or
+    of 32 rows and 256 elements) end to end and cuts the line into runs of one length, whatever tiles they end in: by the number of its
+    workgroups, for which it takes most of a chip of ``units`` compute units.  Of numbers that cut alike the largest."""
+    found = {}
+    for runs in range(units, units * 3 // 4, -1):
+        for parts, height in ((1, 256), (4, 32)):
+            tiles, span = -(-n // height), k // (64 * parts)
+            if k % (64 * parts) == 0 and tiles > runs and tiles % runs:
+                shared = tiles % runs + runs
+                found.setdefault((parts, shared, -(-shared * span // runs)), (parts, 1, runs))
+    return list(found.values())
+
+
 _FRACTION = {torch.bfloat16: 8, torch.float16: 11}   # bits of a value, the leading one included
 
 
@@ -178,9 +198,9 @@ def _norms_like_torch(k, eps, most_rows, like) -> set:
     return left
 
 
-def library_orders(weight, bias=None, most_rows=4, norm=None):
+def library_orders(weight, bias=None, most_rows=4, norm=None, cut=False):
     """``{rows: order}`` whose bits are those of ``torch.nn.functional.linear`` for so many rows of 16 bits, with a fused RMSNorm module
-    in front or none, found by trying, some 10 ms a size, once.
+    in front or none, found by trying, some 10 ms a size, once.  ``cut``: of the orders of :func:`_cut_orders` too.
 
     Rows, weights and bias are drawn, so that what is found hangs on sizes and settings alone and not on a model that is all zeros or has
     a NaN.  Two orders differ in few outputs (4096 x 4096: one of 4000 to 6000), in proportion to the root of the products summed up.  A
@@ -197,7 +217,7 @@ def library_orders(weight, bias=None, most_rows=4, norm=None):
     n, k = weight.shape
     if 3.5e6 / (n * math.sqrt(k)) > 64:   # rows that eight differences take
         return {}
-    key = (weight.device, weight.dtype, n, k, bias is not None, most_rows, None if norm is None else norm.eps, product_settings())
+    key = (weight.device, weight.dtype, n, k, bias is not None, most_rows, None if norm is None else norm.eps, cut, product_settings())
     if key in _FOUND:
         return _FOUND[key]
     if torch.cuda.is_current_stream_capturing():
@@ -206,14 +226,22 @@ def library_orders(weight, bias=None, most_rows=4, norm=None):
     like = dict(generator=torch.Generator(device=weight.device).manual_seed(n + k), device=weight.device, dtype=weight.dtype)
     with torch.no_grad(), torch.autocast("cuda", enabled=False):
         w, b = torch.randn(n, k, **like), None if bias is None else torch.randn(n, **like)
-        for rows in range(1, most_rows + 1) if norm is None else sorted(_norms_like_torch(k, norm.eps, most_rows, like)):
-            left = {_chains(o, k): o for o in reversed(ORDERS) if _fits(rows, n, k, o, norm is not None)}
-            left, tried = list(left.values()), 0
+
+        def agreeing(left, rows):
+            tried = 0
             while left and (tried < 64 or (len(left) > 1 and tried < 128)):
                 x = torch.randn(rows, 1, k, **like)
                 want = nn.functional.linear(x, w, b)
                 left = [o for o in left if torch.equal(linear_rows(x, w, o, b), want)]
                 tried += rows
+            return left
+
+        units = torch.cuda.get_device_properties(weight.device).multi_processor_count
+        for rows in range(1, most_rows + 1) if norm is None else sorted(_norms_like_torch(k, norm.eps, most_rows, like)):
+            fits = [o for o in ORDERS if _fits(rows, n, k, o, norm is not None) and (norm is None or not _crowded(rows, n, k, o, units))]
+            left = agreeing(list({_chains(o, k): o for o in reversed(fits)}.values()), rows)
+            if cut and not left:
+                left = agreeing([o for o in _cut_orders(n, k, units) if o[:2] in fits], rows)
             if len(left) == 1:
                 orders[rows] = left[0]
     _FOUND[key] = orders

@@ -324,7 +324,10 @@ int ckv_gated_silu(const void* gate_up, void* out, int64_t rows, int64_t inter, 
  * in float32; `residual` (rows, n), added to the rounded product; `gated`: W holds n / 2 gate rows and n / 2 up rows, out
  * (rows, n / 2) = silu(gate) * up as ckv_gated_silu has it (no bias or residual then; parts 1).  The float32 sum of an output is made of
  * `parts` chains of matrix instructions, added in order: part p takes stretches p, p + parts, ... of `unit` * 64 elements; (parts, unit)
- * is (1, 1), (2, 2), (4, 1) or (4, 2). */
+ * is (1, 1), (2, 2), (4, 1) or (4, 2).  (1, 1 + 256 runs) and (4, 1 + 256 runs), not gated: as a library sums up that deals tiles of 256
+ * rows of W and 64 elements (four parts: of 32 rows and 256 elements) out over `runs` <= 1024 workgroups, n of at least `runs` tiles,
+ * k % (64 parts) == 0.  What does not come out even, and one round, is laid end to end and cut into `runs` runs of one length; a sum
+ * whose tile holds the end of one is made of two, each as above, added up. */
 int ckv_linear_rows(const void* x, const void* w, const void* bias, const void* residual, const void* norm, float eps, void* out,
                     int64_t rows, int64_t n, int64_t k, int64_t x_stride, int32_t gated, int32_t parts, int32_t unit, int32_t dtype,
                     void* stream);

@@ -164,6 +164,83 @@ def test_other_settings_than_a_layer_was_fused_under_keep_torchs_products():
         assert layer._as_rows(x, cache)
 
 
+@pytest.mark.parametrize("order", [(1, 1), (4, 1)])
+@pytest.mark.parametrize("rows,n,k,runs", [(1, 16 * 16 * 3, 256, 2), (2, 16 * 16 * 5 - 48, 1024, 3), (4, 16 * 77, 1024, 4), (1, 16 * 16 * 7, 4096, 6),
+                                           (3, 16 * 700, 768, 37), (1, 16 * 16 * 4, 256, 2), (2, 16 * 40, 256, 1)])
+def test_sums_cut_where_a_run_of_tiles_ends(rows, n, k, runs, order):
+    """Against the two halves of every cut sum: rows of x that are zero past the cut, or up to it."""
+    x, w, bias, res, norm = operands(rows, n, k, torch.bfloat16)
+    height, span = (256, k // 64) if order[0] == 1 else (32, k // 256)
+    tiles = -(-n // height)
+    shared = tiles % runs + runs if tiles % runs else 0
+    length = -(-shared * span // runs)
+    got = rp.linear_rows(x, w, (*order, runs), residual=res)
+    whole = rp.linear_rows(x, w, order, residual=res)
+    exact = x.double() @ w.double().T + res.double()
+    assert ((got.double() - exact).abs() <= 2 * bound(x, w, torch.bfloat16) + HALF_ULP[torch.bfloat16] * (exact.abs() + res.double().abs())).all()
+    cut_tiles = set()
+    for tile in range(tiles):
+        at = slice(tile * height, min(n, (tile + 1) * height))
+        first = (tile - (tiles - shared)) * span
+        ends = [e for e in range(length, shared * span, length) if first < e < first + span] if shared else []
+        if not ends:
+            assert torch.equal(got[..., at], whole[..., at])
+            continue
+        cut_tiles.add(tile)
+        part = (ends[0] - first) * (k // span)
+        for keep in (slice(0, part), slice(part, k)):
+            y = torch.zeros_like(x)
+            y[..., keep] = x[..., keep]
+            assert torch.equal(rp.linear_rows(y, w, (*order, runs))[..., at], rp.linear_rows(y, w, order)[..., at])
+    assert len(cut_tiles) <= runs and (cut_tiles or not shared or runs == 1)
+
+
+def test_sums_that_cannot_be_cut_are_refused():
+    from cascading_kv_cache_amd import _abi
+
+    x, w, *_ = operands(1, 16 * 32, 256, torch.bfloat16)
+    for order in ((1, 1, 3), (4, 1, 17), (2, 2, 2), (4, 2, 2), (1, 2, 2), (1, 1, 1025)):
+        with pytest.raises(_abi.CkvError):
+            rp.linear_rows(x, w, order)
+    with pytest.raises(_abi.CkvError):
+        rp.linear_rows(x, w, (1, 1, 2), gated=True)
+    with pytest.raises(_abi.CkvError):
+        rp.linear_rows(x[..., :192].contiguous(), w[:, :192].contiguous(), (4, 1, 2))
+
+
+@pytest.mark.parametrize("preset", ["llama3.1-8b", "qwen2-7b"])
+def test_every_product_of_a_step_has_torchs_bits(preset, monkeypatch):
+    """Logits, caches and greedy tokens of a decoder's steps of one to five streams, by row products and by torch's operations."""
+    from cascading_kv_cache_amd.decoder import PRESETS, CascadeDecoder, generate
+
+    cfg = replace(PRESETS[preset], num_layers=2)
+    model = CascadeDecoder(cfg, init_on_device=True).fuse_projections()
+    taken = []
+    monkeypatch.setattr(rp, "linear_rows", lambda *args, run=rp.linear_rows, **kw: taken.append(args[1].shape) or run(*args, **kw))
+    got = []
+    for by_rows in (True, False):
+        if not by_rows:
+            model._head_orders = None
+            for layer in model.layers:
+                layer._orders = None
+        got.append([])
+        gen = torch.Generator().manual_seed(4)
+        with torch.no_grad():
+            for batch in range(1, 6):
+                ids = torch.randint(0, cfg.vocab_size, (batch, 40), generator=gen).cuda()
+                cache = model.new_cache(256, 2, batch=batch, num_sink_tokens=4)
+                logits = [model(cut, cache) for cut in [ids[:, :32]] + [ids[:, i:i + 1] for i in range(32, 40)]]
+                cache_two = model.new_cache(256, 2, batch=batch, num_sink_tokens=4)
+                got[-1].append([*logits, *cache.key_cache, *cache.value_cache, generate(model, ids, cache_two, 32, 12)])
+        if by_rows:   # the layers' four products and the head
+            assert len(set(taken)) == 5, taken
+            taken.clear()
+    assert not taken
+    for batch, (a, b) in enumerate(zip(*got), 1):
+        for x, y in zip(a, b):
+            assert torch.equal(x, y), batch
+
+
 @pytest.mark.parametrize("preset", ["llama3.1-8b", "qwen2-7b", "tiny"])
 def test_steps_of_a_fused_decoder_have_the_bits_of_torchs_products(preset):
     """One layer's steps by row products where an order is torch's, and by torch's operations: the same bits in the cache, and logits that
