@@ -104,6 +104,17 @@ class DecoderLayer(nn.Module):
         self.input_layernorm = RMSNorm(cfg.hidden_size, cfg.rms_eps, dtype, device)
         self.post_attention_layernorm = RMSNorm(cfg.hidden_size, cfg.rms_eps, dtype, device)
 
+    def _find_orders(self):
+        attn, mlp, norm1, norm2 = self.self_attn, self.mlp, self.input_layernorm, self.post_attention_layernorm
+        self._orders = None
+        if not (type(attn) is ProjectedCascadeAttention and type(mlp) is GatedMLP and type(attn.o_proj) is type(mlp.down_proj) is nn.Linear
+                and type(norm1) is type(norm2) is RMSNorm):
+            return   # somebody else's modules, of which nothing is known
+        orders = dict(qkv=library_orders(attn._w_qkv, attn._b_qkv, norm=norm1), o=library_orders(attn.o_proj.weight),
+                      gate_up=library_orders(mlp._w_gate_up, norm=norm2), down=library_orders(mlp.down_proj.weight))
+        any_rows = set().union(*orders.values())
+        self._orders = dict(orders, any=any_rows, settings=product_settings() if any_rows else None)
+
     def _as_rows(self, x, cache) -> bool:
         """Are these few rows whose operations nobody follows, and is every module its own?"""
         attn, mlp = self.self_attn, self.mlp
@@ -161,15 +172,10 @@ class CascadeDecoder(nn.Module):
             layer.input_layernorm.fused = layer.post_attention_layernorm.fused = True
         self.norm.fused = True
         for layer in self.layers:
-            attn, mlp = layer.self_attn, layer.mlp
-            layer._orders = dict(qkv=library_orders(attn._w_qkv, attn._b_qkv, norm=layer.input_layernorm),
-                                 o=library_orders(attn.o_proj.weight),
-                                 gate_up=library_orders(mlp._w_gate_up, norm=layer.post_attention_layernorm),
-                                 down=library_orders(mlp.down_proj.weight))
-            layer._orders["any"] = set().union(*layer._orders.values())
-            layer._orders["settings"] = product_settings() if layer._orders["any"] else None
-        head = self.lm_head
-        orders = library_orders(head.weight, head.bias, norm=self.norm, cut=True)
+            layer._find_orders()
+        head, orders = self.lm_head, {}
+        if type(head) is nn.Linear and type(self.norm) is RMSNorm:
+            orders = library_orders(head.weight, head.bias, norm=self.norm, cut=True)
         self._head_orders = dict(orders, settings=product_settings() if orders else None)
         return self
 

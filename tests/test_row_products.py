@@ -7,7 +7,7 @@ from torch import nn
 
 from cascading_kv_cache_amd import row_products as rp
 from cascading_kv_cache_amd.cascade_attention import CascadeAttention
-from cascading_kv_cache_amd.decoder import PRESETS, DecoderLayer, GatedMLP, RMSNorm
+from cascading_kv_cache_amd.decoder import PRESETS, CascadeDecoder, DecoderLayer, GatedMLP, RMSNorm
 from cascading_kv_cache_amd.latency import ProjectedCascadeAttention
 
 MAKE = {nn.Linear: lambda: nn.Linear(4, 4), RMSNorm: lambda: RMSNorm(4, 1e-5, torch.float32, "cpu"),
@@ -65,3 +65,12 @@ def test_nothing_is_tried_on_tensors_without_memory():
     with FakeTensorMode(allow_non_fake_inputs=True):
         weight = torch.empty(4096, 4096, dtype=torch.bfloat16, device="cuda")
         assert rp.library_orders(weight) == {}
+
+
+@pytest.mark.parametrize("path", ["layers.0.self_attn.o_proj", "layers.0.mlp.down_proj", "lm_head", "layers.0.input_layernorm", "norm"])
+def test_projections_are_fused_beside_modules_of_somebody_elses(path):
+    model = CascadeDecoder(PRESETS["tiny"], torch.float32, "cpu")
+    parent, name = path.rpartition(".")[::2]
+    setattr(model.get_submodule(parent), name, nn.Identity())   # no weight, no eps
+    model.fuse_projections()
+    assert model.layers[0].mlp._w_gate_up is not None and (path.startswith("layers") == (model.layers[0]._orders is None))
