@@ -1720,7 +1720,8 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
         }
     };
 
-    // Normalisers of the 32 rows that a wavefront has brought the shares' of: two lanes a row, four shares each.
+    // Normalisers of the 32 rows that a wavefront has brought the shares' of: two lanes a row, four shares each, added up in the order of
+    // merge_rows_of, so that a score does not hang on which launch has merged the shares.
     auto merge_norms = [&](int stage) {
         if constexpr (!kMerge) return;
         const int r = lane >> 1;
@@ -1732,12 +1733,16 @@ __global__ void __launch_bounds__(256, 2) colsum_mfma_kernel(ColsumParams p) {
             M = fmaxf(M, v[u]);
         }
         M = fmaxf(M, __shfl_xor(M, 1));
+        auto add = [&] {
 #pragma unroll
-        for (int u = 0; u < kMergeShares / 2; u++)
-            if (v[u] != -INFINITY) L += __builtin_amdgcn_exp2f(v[u] - M);   // a NaN counts
-        L += __shfl_xor(L, 1);
+            for (int u = 0; u < kMergeShares / 2; u++)
+                if (v[u] != -INFINITY) L += __builtin_amdgcn_exp2f(v[u] - M);   // a NaN counts
+        };
+        add();
+        L = __shfl_xor(L, 1);   // the second lane goes on from the first one's sum
+        add();
         float* lse_lds = reinterpret_cast<float*>(smem + stage * kCsStage + kQT2 * kRowBytes);
-        if ((lane & 1) == 0) lse_lds[wave * 32 + r] = -(M + __builtin_amdgcn_logf(L));
+        if (lane & 1) lse_lds[wave * 32 + r] = -(M + __builtin_amdgcn_logf(L));
     };
     // Called by every wavefront once its copies of a step have landed, before the barrier that publishes them.  Rows past
     // the chunk end are copies of its last row, whose normaliser is somebody else's: starting from this value their

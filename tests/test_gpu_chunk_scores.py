@@ -78,3 +78,30 @@ def test_update_planned_beside_the_finishing_scores_equals_two_calls(B, H, KVH, 
         assert torch.equal(bits(out1), bits(out2)) and torch.equal(bits(new1), bits(new2)), call
         for name in STATE:
             assert torch.equal(bits(getattr(one, name)[0]), bits(getattr(two, name)[0])), (call, name)
+
+
+@pytest.mark.parametrize("D,dtype", [(128, torch.float16), (128, torch.bfloat16), (64, torch.float16)])
+def test_scores_do_not_hang_on_which_launch_merges_the_shares(D, dtype):
+    """Seven shares of the same 16 K keys, merged in the launch of the score sums (a cache of 16 K slots) and in one of their own (64 K
+    slots, three quarters of them empty)."""
+    from cascading_kv_cache_amd.cascade_attention import cascade_attention, default_inv_freq
+
+    H = KVH = 8
+    tokens, q_len = 16384, 2240
+    inv_freq = default_inv_freq(D, 5e5, "cuda:0")
+    gen = torch.Generator(device="cuda").manual_seed(2)
+    rows = lambda n: torch.randn(1, n, H, D, generator=gen, device="cuda").to(dtype).transpose(1, 2)   # noqa: E731
+    k0, v0, k, v = rows(tokens), rows(tokens), rows(q_len), rows(q_len)
+    caches = []
+    for slots in (tokens, 4 * tokens):
+        cache = make_pair(1, KVH, D, 0, slots, 1, dtype)[0]
+        cache.beta = 0.5   # scores of the last few rows: a normaliser's last bit shows
+        cache.update(k0, v0, 0, torch.zeros(1, KVH, tokens, dtype=dtype, device="cuda"))
+        caches.append(cache)
+    for _ in range(4):
+        q, got = rows(q_len), []
+        for cache in caches:
+            out, new = cascade_attention(q, k, v, cache, 0, inv_freq, update_cache=False)
+            got.append((out, new, cache.score_cache[0][..., :tokens]))
+        for a, b in zip(*got):
+            assert torch.equal(a, b), (a != b).sum()
