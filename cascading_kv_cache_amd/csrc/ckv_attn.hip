@@ -113,6 +113,22 @@ extern "C" int64_t ckv_attn_workspace_bytes(int64_t B, int64_t H, int64_t KVH, i
 }
 
 namespace ckv {
+static bool chunk_uses_mfma(const ckv_attn_args& a) {
+    return mfma_supported(a.dtype, a.D, a.H, a.KVH, a.Q) && a.Q > 1 && mfma_fits(a.num_sink + a.S + a.Q, a.D);
+}
+static bool chunk_uses_f32_split(const ckv_attn_args& a) {
+    return f32_split_supported(a.dtype, a.B, a.H, a.KVH, a.Q, a.num_sink + a.S + a.Q, a.D);
+}
+
+// Is the update `u` planned in the launch that finishes the scores of the chunk `a`?  (Both are checked.)
+static bool plan_rides(const ckv_attn_args& a, const ckv_update_args& u, const AttnWorkspace& w) {
+    if (!(a.S > 0 && a.cache_s && a.new_scores && (chunk_uses_mfma(a) || chunk_uses_f32_split(a)) && update_plans_beside_finish(a, u))) return false;
+    // the plan's scratch may be the attention's, of which only what the score sums left is still read
+    const char *ws = reinterpret_cast<const char*>(u.workspace), *sums = reinterpret_cast<const char*>(w.colsum);
+    const int64_t need = ckv_update_workspace_bytes(u.N, u.H, u.K, u.max_seq_len, u.cascades);
+    return ws + need <= sums || ws >= reinterpret_cast<const char*>(a.workspace) + w.bytes;
+}
+
 // `u`: the cache update that the caller runs next, or null; *updated: it has been launched here
 static int run_attn(const ckv_attn_args* args, hipStream_t stream, const ckv_update_args* u, bool* updated) {
     *updated = false;
@@ -136,19 +152,13 @@ static int run_attn(const ckv_attn_args* args, hipStream_t stream, const ckv_upd
     const int64_t N = a.num_sink + a.S + a.Q;
     const bool want_scores = a.cache_s || a.new_scores;
     int rc;
-    const bool use_mfma = mfma_supported(a.dtype, a.D, a.H, a.KVH, a.Q) && a.Q > 1 && mfma_fits(N, a.D);
-    const bool split = !use_mfma && f32_split_supported(a.dtype, a.B, a.H, a.KVH, a.Q, N, a.D);
+    const bool use_mfma = chunk_uses_mfma(a), split = !use_mfma && chunk_uses_f32_split(a);
     KeptScores kept;
-    if (u && (use_mfma || split) && a.S > 0 && a.cache_s && a.new_scores && update_plans_beside_finish(a, *u)) {
-        // the plan's scratch may be the attention's, of which only what the score sums left is still read
-        const char *ws = reinterpret_cast<const char*>(u->workspace), *sums = reinterpret_cast<const char*>(w.colsum);
-        const int64_t need = ckv_update_workspace_bytes(u->N, u->H, u->K, u->max_seq_len, u->cascades);
-        if (ws + need <= sums || ws >= reinterpret_cast<const char*>(a.workspace) + w.bytes) {
-            kept.src = a.cache_s;
-            for (int i = 0; i < 3; i++) kept.stride[i] = a.cache_s_stride[i];
-            kept.dst = w.before;
-            kept.units = a.B * a.KVH; kept.KVH = a.KVH; kept.S = a.S;
-        }
+    if (u && plan_rides(a, *u, w)) {
+        kept.src = a.cache_s;
+        for (int i = 0; i < 3; i++) kept.stride[i] = a.cache_s_stride[i];
+        kept.dst = w.before;
+        kept.units = a.B * a.KVH; kept.KVH = a.KVH; kept.S = a.S;
     }
     if (use_mfma) {
         MfmaProblem mp;
@@ -265,6 +275,13 @@ extern "C" int ckv_attn_update(const ckv_attn_args* args, const ckv_update_args*
     const bool beside = check_update(update, &empty) == CKV_OK && !empty && !prof_update_apart();
     if (int rc = run_attn(args, reinterpret_cast<hipStream_t>(stream), beside ? update : nullptr, &updated)) return rc;
     return updated ? CKV_OK : ckv_update(update, stream);
+}
+
+// For tests that aim at one way: does ckv_attn_update plan the chunk's update in the launch that finishes its scores (1), or apart (0)?
+extern "C" int ckv_chunk_plan_rides(const ckv_attn_args* args, const ckv_update_args* update) {
+    using namespace ckv;
+    const ckv_attn_args& a = *args;
+    return plan_rides(a, *update, carve_attn(a.workspace, a.B, a.H, a.KVH, a.Q, a.D, a.num_sink, a.S, a.dtype));
 }
 
 namespace ckv {

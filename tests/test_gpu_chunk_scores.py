@@ -1,5 +1,7 @@
 """Score sums of a chunk's own keys: weights that are all alike (the default beta) and weights by distance, wavefronts whose 64 keys are
 all the chunk's and the one in which the chunk starts, lengths around the 32-row subtiles and the 128-row tiles."""
+import ctypes
+
 import pytest
 import torch
 
@@ -47,18 +49,19 @@ def test_chunks_whose_keys_are_shared_out_two_tiles_each(H, KVH, D, dtype):
 
 # caches that fill (the walk) and full ones (closed forms), periods that do not divide each other, rings shorter than the chunk, the most
 # tokens that share the launch and one more, seven and eight heads per kv head, more workgroups than one round takes
-@pytest.mark.parametrize("B,H,KVH,D,NS,W,C,dtype,func,reduction,q_len,calls", [
-    (1, 8, 2, 128, 4, 33, 4, torch.bfloat16, "pow2", "mean", 17, 24),
-    (2, 14, 2, 128, 0, 64, 3, torch.float16, "pow2", "median", 50, 10),
-    (1, 8, 1, 64, 3, 40, 5, torch.bfloat16, "pow2", "median", 2, 60),
-    (1, 4, 2, 64, 4, 128, 2, torch.float16, "iplus1", "max", 100, 8),
-    (1, 8, 2, 128, 4, 128, 4, torch.float32, "pow2", "max", 256, 6),
-    (3, 6, 2, 64, 1, 96, 1, torch.float32, "pow2", "median", 31, 8),
-    (1, 4, 1, 128, 64, 512, 8, torch.bfloat16, "pow2", "mean", 1092, 6),
-    (1, 4, 1, 128, 64, 512, 8, torch.bfloat16, "pow2", "mean", 1093, 6),
-    (4, 16, 16, 64, 4, 8192, 2, torch.float16, "pow2", "max", 300, 3),
+@pytest.mark.parametrize("B,H,KVH,D,NS,W,C,dtype,func,reduction,q_len,calls,rides", [
+    (1, 8, 2, 128, 4, 33, 4, torch.bfloat16, "pow2", "mean", 17, 24, True),
+    (2, 14, 2, 128, 0, 64, 3, torch.float16, "pow2", "median", 50, 10, True),
+    (1, 8, 1, 64, 3, 40, 5, torch.bfloat16, "pow2", "median", 2, 60, True),
+    (1, 4, 2, 64, 4, 128, 2, torch.float16, "iplus1", "max", 100, 8, True),
+    (1, 8, 2, 128, 4, 128, 4, torch.float32, "pow2", "max", 256, 6, True),
+    (3, 6, 2, 64, 1, 96, 1, torch.float32, "pow2", "median", 31, 8, True),
+    (1, 4, 1, 128, 64, 512, 8, torch.bfloat16, "pow2", "mean", 1092, 6, True),
+    (1, 4, 1, 128, 64, 512, 8, torch.bfloat16, "pow2", "mean", 1093, 6, False),
+    (4, 16, 16, 64, 4, 8192, 2, torch.float16, "pow2", "max", 300, 3, False),
 ])
-def test_update_planned_beside_the_finishing_scores_equals_two_calls(B, H, KVH, D, NS, W, C, dtype, func, reduction, q_len, calls):
+def test_update_planned_beside_the_finishing_scores_equals_two_calls(B, H, KVH, D, NS, W, C, dtype, func, reduction, q_len, calls, rides):
+    from cascading_kv_cache_amd import _abi
     from cascading_kv_cache_amd.cascade_attention import cascade_attention, default_inv_freq
     from test_gpu_token_step import STATE, bits
 
@@ -78,6 +81,13 @@ def test_update_planned_beside_the_finishing_scores_equals_two_calls(B, H, KVH, 
         assert torch.equal(bits(out1), bits(out2)) and torch.equal(bits(new1), bits(new2)), call
         for name in STATE:
             assert torch.equal(bits(getattr(one, name)[0]), bits(getattr(two, name)[0])), (call, name)
+    lib = ctypes.CDLL(_abi.LIB_PATH)
+    blocks = [a for a in one._attn_memo.values() if a.Q == q_len and a._update is not None]
+    assert blocks and {bool(lib.ckv_chunk_plan_rides(ctypes.byref(a), ctypes.byref(a._update))) for a in blocks} == {rides}
+    # scratch that would lie over what the finishing blocks still read (asked, not run)
+    a, u = blocks[-1], type(blocks[-1]._update).from_buffer_copy(blocks[-1]._update)
+    u.workspace = a.workspace + _abi.lib().ckv_attn_workspace_bytes(B, H, KVH, q_len, D, NS, W * C, a.dtype) - 512
+    assert not lib.ckv_chunk_plan_rides(ctypes.byref(a), ctypes.byref(u))
 
 
 @pytest.mark.parametrize("D,dtype", [(128, torch.float16), (128, torch.bfloat16), (64, torch.float16)])
