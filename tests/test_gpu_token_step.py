@@ -176,3 +176,32 @@ def test_median_of_a_groups_heads(spoilt, G, B, window):
         assert torch.equal(mine.isnan(), want.isnan())
         # one rounding to bfloat16 of probabilities that two kernels work out
         assert torch.allclose(mine, want, rtol=2.0 ** -7, atol=1e-9, equal_nan=True)
+
+
+@pytest.mark.parametrize("B,window", [(1, 96), (40, 64)])   # rows, scores and update in one launch; apart
+@pytest.mark.parametrize("G", [1, 2, 4, 7, 8])
+@pytest.mark.parametrize("spoilt", [False, True])
+def test_median_of_a_groups_heads_is_one_of_their_values(spoilt, G, B, window):
+    """To the bit: a head's own values come from the same step with its queries in every head's place, where any reduction gives them."""
+    from cascading_kv_cache_amd.cascade_attention import cascade_attention, default_inv_freq
+
+    KVH, gen = 2, torch.Generator().manual_seed(G + 20)
+    inv_freq = default_inv_freq(128, 5e5, "cuda:0")
+    draw = lambda h, n: (torch.randn(B, n, h, 128, generator=gen) * 0.7).bfloat16().cuda().transpose(1, 2)   # noqa: E731
+    (q0, k0, v0), (q, k, v) = ((draw(KVH * G, n), draw(KVH, n), draw(KVH, n)) for n in (2 * window + 4, 1))
+    if spoilt:
+        q[:, 0] = float("nan")
+    cache = pair(B, KVH, 4, window, 2, torch.bfloat16, "pow2", True, "median")[0]
+    cascade_attention(q0, k0, v0, cache, 0, inv_freq)
+
+    def scores(queries):
+        cache.score_cache[0].zero_()
+        new = cascade_attention(queries, k, v, cache, 0, inv_freq, update_cache=False)[1]
+        return torch.cat((cache.score_cache[0], new), dim=-1).float()
+
+    got = scores(q)
+    heads = q.reshape(B, KVH, G, 1, 128)
+    each = torch.stack([scores(heads[:, :, g:g + 1].expand(-1, -1, G, -1, -1).reshape(B, KVH * G, 1, 128)) for g in range(G)], dim=2)
+    want = lower_median(each) if G > 1 else each[:, :, 0]
+    assert torch.equal(got.isnan(), want.isnan()) and got.isnan().any() == (spoilt and G < 2)
+    assert torch.equal(bits(got.nan_to_num()), bits(want.nan_to_num()))
