@@ -2036,8 +2036,10 @@ bool order_by_staging(int64_t n_cached) { return n_cached <= 16384; }
 // order in which a row's sums are added, so a hint about the filled slots would otherwise change results.
 //
 // The launch takes whole rounds of workgroups, a round as long as a workgroup: about 1.6 us per key tile with every unit busy and 16 us
-// to start and finish one (the work list, the first copies, the rows' way out).  Shares cost the merge kernel 6 us and its traffic
-// (float32 rows written and read, 256 rows of 512 bytes per workgroup: 0.058 us).  The cheapest count by that estimate, down to
+// to start and finish one (the work list, the first copies, the rows' way out).  Shares cost a merge kernel, 6 us and its traffic
+// (float32 rows written and read, 256 rows of 512 bytes per workgroup: 0.058 us); that is what a call without scores pays, and one whose
+// merge rides with its score sums (run_mfma) pays less, but the order of a row's sums must not hang on whether scores are asked for.  The
+// cheapest count by that estimate, down to
 // two tiles each: 2300 x 8 K  1: 391  3: 353  8: 416.  (64 dims: 1: 503  3: 398  6: 382; masked keys of the dense operator, which
 // cost nothing, count like the others.)  With no more than a share to 16 tiles of a chunk, and to 8 of the dense operator's, a whole
 // call took, us, 32 heads on 8 kv heads, then and now:  16 rows x 1 K slots 57.8 47.5   33 x 2 K 67.1 55.7   16 x 4 K 76.4 63.7
@@ -2048,8 +2050,9 @@ bool order_by_staging(int64_t n_cached) { return n_cached <= 16384; }
 //
 // Chunks of fewer workgroups than units over caches of 16 K slots and more keep the counts that streams have always had, because a
 // decoder of random weights turns the changed rounding of one hidden state into a percent of its logits: about two workgroups per
-// unit, at most 8 shares; where 8 shares would be of more than 32 tiles, the cheapest count from 8 to 32 by the estimate.  Forward +
-// merge in us, by shares:     509 rows x 16 K  4: 141  8: 155    488 x 16 K, 1000 slots filled  4: 34  8: 47
+// unit, at most 8 shares; where 8 shares would be of more than 32 tiles, the cheapest count from 8 to 32 by the estimate.  The line is
+// drawn by that and not by speed (half the shares would be faster up to 16 K slots), and tiles of the chunk count: a stream over a little
+// less than 16 K slots goes from one count to the other with the length of its chunks.  Forward + merge in us, by shares:     509 rows x 16 K  4: 141  8: 155    488 x 16 K, 1000 slots filled  4: 34  8: 47
 //   128 x 64 K   8: 175  16: 134  32: 160        32 x 64 K  8: 162  16: 95  32: 90      509 x 32 K  4: 237  8: 250
 int mfma_fwd_splits(int64_t B, int64_t H, int64_t KVH, int64_t Q, int64_t n, int cus, bool dense) {
     constexpr double kTileUs = 1.6, kStartUs = 16.0, kMergeUs = 6.0, kMergeWgUs = 0.058;

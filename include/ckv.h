@@ -340,10 +340,12 @@ int ckv_linear_rows(const void* x, const void* w, const void* bias, const void* 
  * them.  The plan of a call of several tokens is counted as two (closed forms, walk) also where
  * both are one launch: its time is with the first, the second has none.  Where the forward kernel
  * shares keys out, their merge is with CKV_STAGE_FWD, or with CKV_STAGE_SCORES when it rides in that
- * launch.  Levels 1 and 3 run a
- * single token's cache update in launches of its own, which ckv_attn_update does otherwise only
- * where it cannot run beside the scores: they show what the stages take one by one, not what
- * such a step takes.  Process-wide and not thread-safe: a measurement aid, off by default.
+ * launch.  Levels 1 and 3 run the cache update of a single token and of a short chunk in
+ * launches of its own.  Otherwise ckv_attn_update runs a single token's beside the scores and
+ * plans a short chunk's in the launch that finishes its scores, wherever it can: the levels show
+ * what the stages take one by one, and their times (CKV_STAGE_FINISH and CKV_STAGE_PLAN among
+ * them) do not add up to what such a call takes.  Process-wide and not thread-safe: a measurement
+ * aid, off by default.
  * ---------------------------------------------------------------------------------------- */
 typedef enum ckv_stage {
     CKV_STAGE_PREP = 0,        /* rotate + gather prologue                      */
