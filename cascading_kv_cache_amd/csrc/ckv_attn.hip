@@ -120,9 +120,10 @@ static bool chunk_uses_f32_split(const ckv_attn_args& a) {
     return f32_split_supported(a.dtype, a.B, a.H, a.KVH, a.Q, a.num_sink + a.S + a.Q, a.D);
 }
 
-// Is the update `u` planned in the launch that finishes the scores of the chunk `a`?  (Both are checked.)
-static bool plan_rides(const ckv_attn_args& a, const ckv_update_args& u, const AttnWorkspace& w) {
-    if (!(a.S > 0 && a.cache_s && a.new_scores && (chunk_uses_mfma(a) || chunk_uses_f32_split(a)) && update_plans_beside_finish(a, u))) return false;
+// Is the update `u` planned in the launch that finishes the scores of the chunk `a`?  (Both are checked.)  matrix: chunk_uses_mfma or
+// chunk_uses_f32_split.
+static bool plan_rides(const ckv_attn_args& a, const ckv_update_args& u, const AttnWorkspace& w, bool matrix) {
+    if (!(matrix && a.S > 0 && a.cache_s && a.new_scores && update_plans_beside_finish(a, u))) return false;
     // the plan's scratch may be the attention's, of which only what the score sums left is still read
     const char *ws = reinterpret_cast<const char*>(u.workspace), *sums = reinterpret_cast<const char*>(w.colsum);
     const int64_t need = ckv_update_workspace_bytes(u.N, u.H, u.K, u.max_seq_len, u.cascades);
@@ -154,7 +155,7 @@ static int run_attn(const ckv_attn_args* args, hipStream_t stream, const ckv_upd
     int rc;
     const bool use_mfma = chunk_uses_mfma(a), split = !use_mfma && chunk_uses_f32_split(a);
     KeptScores kept;
-    if (u && plan_rides(a, *u, w)) {
+    if (u && plan_rides(a, *u, w, use_mfma || split)) {
         kept.src = a.cache_s;
         for (int i = 0; i < 3; i++) kept.stride[i] = a.cache_s_stride[i];
         kept.dst = w.before;
@@ -281,7 +282,8 @@ extern "C" int ckv_attn_update(const ckv_attn_args* args, const ckv_update_args*
 extern "C" int ckv_chunk_plan_rides(const ckv_attn_args* args, const ckv_update_args* update) {
     using namespace ckv;
     const ckv_attn_args& a = *args;
-    return plan_rides(a, *update, carve_attn(a.workspace, a.B, a.H, a.KVH, a.Q, a.D, a.num_sink, a.S, a.dtype));
+    return plan_rides(a, *update, carve_attn(a.workspace, a.B, a.H, a.KVH, a.Q, a.D, a.num_sink, a.S, a.dtype),
+                      chunk_uses_mfma(a) || chunk_uses_f32_split(a));
 }
 
 namespace ckv {
