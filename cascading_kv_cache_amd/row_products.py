@@ -200,7 +200,7 @@ def _norms_like_torch(k, eps, most_rows, like) -> set:
 
 def library_orders(weight, bias=None, most_rows=4, norm=None, cut=False):
     """``{rows: order}`` whose bits are those of ``torch.nn.functional.linear`` for so many rows of 16 bits, with a fused RMSNorm module
-    in front or none, found by trying, some 10 ms a size, once.  ``cut``: of the orders of :func:`_cut_orders` too.
+    in front or none, found by trying, 20 to 60 ms a size, once.  ``cut``: of the orders of :func:`_cut_orders` too (0.2 s).
 
     Rows, weights and bias are drawn, so that what is found hangs on sizes and settings alone and not on a model that is all zeros or has
     a NaN.  Two orders differ in few outputs (4096 x 4096: one of 4000 to 6000), in proportion to the root of the products summed up.  A
