@@ -225,7 +225,10 @@ def library_orders(weight, bias=None, most_rows=4, norm=None, cut=False):
     orders = {}
     like = dict(generator=torch.Generator(device=weight.device).manual_seed(n + k), device=weight.device, dtype=weight.dtype)
     with torch.no_grad(), torch.autocast("cuda", enabled=False):
-        w, b = torch.randn(n, k, **like), None if bias is None else torch.randn(n, **like)
+        try:
+            w, b = torch.randn(n, k, **like), None if bias is None else torch.randn(n, **like)
+        except torch.OutOfMemoryError:   # a model that fills the device: nothing is tried, and nothing taken down
+            return {}
 
         def agreeing(left, rows):
             tried = 0

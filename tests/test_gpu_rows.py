@@ -111,6 +111,17 @@ def test_an_order_that_differs_in_a_few_tiles_is_told_from_torchs(n, k, dtype):
             assert torch.equal(rp.linear_rows(x, w, order), F.linear(x, w)), (rows, order)
 
 
+def test_no_room_to_try_means_no_order(monkeypatch):
+    w = torch.empty(4096, 4096, device="cuda", dtype=torch.bfloat16)
+    monkeypatch.setattr(rp, "_FOUND", {})
+    with monkeypatch.context() as m:
+        def full(*args, **kw):
+            raise torch.OutOfMemoryError("as on a device that a model fills")
+        m.setattr(torch, "randn", full)
+        assert rp.library_orders(w) == {}
+    assert rp.library_orders(w)
+
+
 def test_orders_are_asked_again_when_torch_is_told_to_take_another_product():
     n, k = 6144, 4096
     w = torch.randn(n, k, device="cuda").bfloat16()
@@ -210,7 +221,7 @@ def test_sums_that_cannot_be_cut_are_refused():
 
 @pytest.mark.parametrize("preset", ["llama3.1-8b", "qwen2-7b"])
 def test_every_product_of_a_step_has_torchs_bits(preset, monkeypatch):
-    """Logits, caches and greedy tokens of a decoder's steps of one to five streams, by row products and by torch's operations."""
+    """Logits, caches and greedy tokens of a decoder's steps of one to five streams, and of three tokens at a time, by row products and by torch's operations."""
     from cascading_kv_cache_amd.decoder import PRESETS, CascadeDecoder, generate
 
     cfg = replace(PRESETS[preset], num_layers=2)
@@ -229,7 +240,7 @@ def test_every_product_of_a_step_has_torchs_bits(preset, monkeypatch):
             for batch in range(1, 6):
                 ids = torch.randint(0, cfg.vocab_size, (batch, 40), generator=gen).cuda()
                 cache = model.new_cache(256, 2, batch=batch, num_sink_tokens=4)
-                logits = [model(cut, cache) for cut in [ids[:, :32]] + [ids[:, i:i + 1] for i in range(32, 40)]]
+                logits = [model(cut, cache) for cut in [ids[:, :32], ids[:, 32:35]] + [ids[:, i:i + 1] for i in range(35, 40)]]
                 cache_two = model.new_cache(256, 2, batch=batch, num_sink_tokens=4)
                 got[-1].append([*logits, *cache.key_cache, *cache.value_cache, generate(model, ids, cache_two, 32, 12)])
         if by_rows:   # the layers' four products and the head
