@@ -51,10 +51,11 @@ own_methods(nn.Linear)
 
 
 def plain(module, kind) -> bool:
-    """Is calling ``module`` nothing but the methods that :func:`own_methods` has taken down for ``kind``: no subclass, no hooks, no
-    method put on the object or on its class since?"""
+    """Is calling ``module`` nothing but the methods that :func:`own_methods` has taken down for ``kind``: no subclass, no hooks, not
+    compiled, no method put on the object or on its class since?"""
     every = nn.modules.module
     if not (type(module) is kind and not module._forward_hooks and not module._forward_pre_hooks
+            and getattr(module, "_compiled_call_impl", None) is None
             and not getattr(every, "_global_forward_hooks", True) and not getattr(every, "_global_forward_pre_hooks", True)):
         return False
     for name, method in _OWN[kind]:

@@ -74,3 +74,19 @@ def test_projections_are_fused_beside_modules_of_somebody_elses(path):
     setattr(model.get_submodule(parent), name, nn.Identity())   # no weight, no eps
     model.fuse_projections()
     assert model.layers[0].mlp._w_gate_up is not None and (path.startswith("layers") == (model.layers[0]._orders is None))
+
+
+@pytest.mark.parametrize("kind", list(MAKE))
+def test_a_compiled_module_is_called(kind):
+    module = MAKE[kind]()
+    module._compiled_call_impl = module._call_impl   # what Module.compile() sets
+    assert not rp.plain(module, kind)
+
+
+def test_numbers_of_workgroups_that_cut_alike_are_one():
+    """501 tiles of 256 rows and 64 stretches: runs of 126, whether 256 workgroups share them or 255.  4752 of 32 rows and 14: 250 leave
+    4500 whole ones, and the rest in runs of 15."""
+    assert (1, 1, 256) in rp._cut_orders(128256, 4096, 256) and (1, 1, 255) not in rp._cut_orders(128256, 4096, 256)
+    assert (4, 1, 250) in rp._cut_orders(152064, 3584, 256)
+    assert rp._cut_orders(256 * 32, 4096, 256) == [o for o in rp._cut_orders(256 * 32, 4096, 256) if o[2] < 256]   # one round, nothing to cut
+    assert not any(o[0] == 4 for o in rp._cut_orders(128256, 64 * 3, 256))   # stretches of 256 elements
